@@ -25,7 +25,7 @@
 // together inside one wave; the second wave on the SIMD covers what is left.
 // Scores are in the log2 domain (scale*log2(e) is folded into the Q
 // quantizer), so the exponential is a bare v_exp_f32.
-#include "sage_internal.h"
+#include "sage_attn_common.h"
 
 #include <hip/hip_fp16.h>
 
@@ -43,108 +43,12 @@
 namespace sage {
 constexpr int kLoopPart = SAGE_LOOP_PART;
 
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v8i __attribute__((ext_vector_type(8)));
-typedef int v16i __attribute__((ext_vector_type(16)));
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef _Float16 v2h __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned v2u __attribute__((ext_vector_type(2)));
-
-// Byte offset of 16-byte chunk L of a tile.  Chunks are grouped into 128-byte super-rows
-// (8 chunks); the chunk position inside a super-row is XORed with bits of the index of
-// the PAIR of super-rows it belongs to, so that the 16 lanes the 64-bank LDS serves per
-// cycle (16 consecutive rows, one logical column) land in 16 different 16-byte bank groups.
-__device__ __forceinline__ int swz(int L) { return (((L >> 3) << 3) | ((L & 7) ^ ((L >> 4) & 7))) << 4; }
-
-__device__ __forceinline__ uint16_t f32_to_bf16_rne(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7FFFFFFFu) > 0x7F800000u) return (uint16_t)((u >> 16) | 0x0040u);
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
-}
-
-// 16 bytes per lane from global memory straight into LDS: lane l of the wave lands at
-// lds_base + 16*l.  Written as assembly on purpose: the compiler then keeps no record of
-// an outstanding LDS write and does not put a full vector-memory wait in front of every
-// later LDS read; completion is awaited explicitly (dma_wait) before the workgroup
-// barrier that publishes the tile.
-__device__ __forceinline__ void dma16(const void* gbase_uniform, uint32_t goff, uint32_t lds_base_uniform) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                 :
-                 : "s"(lds_base_uniform), "v"(goff), "s"(gbase_uniform)
-                 : "memory");      // (m0 cannot be named as a clobber: to this compiler it is a reserved register — it
-                                   // warns that "clobbering them may lead to undefined behaviour" — which it never
-                                   // keeps a value in across statements; its own uses set m0 right before the use)
-}
-// Wait until at most N of this wave's copies are still in flight (they complete in order).
-template <int N> __device__ __forceinline__ void dma_wait() {
-    static_assert(N >= 0 && N < 64, "vmcnt is a 6-bit counter");
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
-}
-
-// The int32 score accumulators start at the bit pattern of the float 1/(2*pi) instead of 0.
-// That pattern is 2^-3 * (1 + 2292099 * 2^-23), so adding an integer dot with
-// |dot| < 2292099 (the largest possible |dot| is 128*127*127 = 2064512) changes only the
-// mantissa: a finished accumulator, read as fp32, IS the float 1/(2*pi) + dot * 2^-26.  No
-// int->float conversion is needed and dequantisation, max subtraction and the exponent
-// argument collapse into one FMA per score (the scale carries the factor 2^26).
-constexpr int kMagicI = 0x3E22F983;
-constexpr float kMagicF = 0.15915494309189532f;        // the same 32 bits
-constexpr float kMagicUnit = 67108864.0f;               // 2^26: accumulator-as-float steps per integer
-// With 256 channels |dot| can reach 256*127*127 = 4129024, more than the mantissa of 1/(2*pi) has
-// room for below it.  0.1875 = 2^-3 * (1 + 2^22 * 2^-23) leaves 2^22 = 4194304 either way at the
-// same step of 2^-26.
-constexpr int kMagicWideI = 0x3E400000;
-constexpr float kMagicWideF = 0.1875f;
-// e4m3 variant: a wave whose bias * f can exceed this takes the bias off its accumulators (see exact_bias).
-constexpr float kExactBias = 4096.0f;
-template <int D> struct Magic {
-    static constexpr int I = D > 128 ? kMagicWideI : kMagicI;
-    static constexpr float F = D > 128 ? kMagicWideF : kMagicF;
-};
-
-// First matrix instruction of a score chain: accumulator input = the constant above, held in 16
-// registers for the whole kernel (behind an empty statement, or the compiler re-creates the 16
-// copies for every chain).  The instruction could take 1/(2*pi) as an inline operand, but only
-// written as assembly, and then the compiler does not know that a matrix instruction is writing
-// those registers: it neither keeps the wait states before the first other instruction that
-// touches them — a spill store two instructions later wrote the old contents — nor can it be told.
-template <int D>
-__device__ __forceinline__ v16i magic_splat() {
-    constexpr int M = Magic<D>::I;
-    v16i c = {M, M, M, M, M, M, M, M, M, M, M, M, M, M, M, M};
-    asm volatile("" : "+v"(c));
-    return c;
-}
-
-// A row's reference maximum is only refreshed (and the accumulators rescaled) when a tile
-// exceeds it by more than tau powers of two; until then p = exp2(s - m_used) may reach
-// 2^tau.  fp16 P holds 2^8 without loss.  The e4m3 variant maps p = 2^tau to the format
-// maximum 448, i.e. it stores e4m3(p * 448 / 2^tau); the factor cancels against the
-// normaliser, which sums the same scaled values.  Its reference is always a whole number
-// (the maximum rounded up): a probability's e4m3 significand then depends on the fractional
-// part of its score only, not on which whole number the reference happens to be, so the
-// stored probabilities are those of a softmax taken against ceil(row maximum) up to a power
-// of two, and the rescale factors are exact.
-template <int VARIANT> struct Lazy {
-    static constexpr float tau = VARIANT == 0 ? 8.0f : 1.0f;
-    static constexpr float log2_pscale = VARIANT == 0 ? 0.0f : 7.807354922057604f;     // log2(448 / 2)
-    static constexpr bool integer_ref = VARIANT == 1;
-};
-
 // ADDMASK: an additive score bias (natural-log units, bf16, logical [B,H,Nq,Nkv] through element
 // strides with the key stride 1) is added to the dequantised scores.  That instantiation looks
 // for every tile's maximum on the biased scores (no optimistic tiles) and lets its ordinary
 // global loads share the vector-memory counter with the tile copies, i.e. it waits for all of
 // them at the midpoint: it is bound by the N_q x N_kv bias it has to read, not by the copies.
+
 // Workgroups of the split schedule that gave up on a hand-over (see the kernel's fold-in part).
 static __device__ unsigned int g_split_faults;
 
@@ -198,6 +102,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     __shared__ __attribute__((aligned(1024))) uint8_t lds_v[NSV][V_BYTES];
     __shared__ __attribute__((aligned(16))) float lds_ks[max_keys(D) / 32 + 4];
     __shared__ float lds_qmax[QF ? 8 : 1];              // QF: largest |pre-scaled q| of each wave's 32 rows
+    __shared__ __attribute__((aligned(16))) uint8_t lds_qc[QF && VARIANT == 1 ? NW * 32 * D : 16];      // QF: Q codes on their way into fragments
     static_assert(!QF || (D <= 128 && !STATS && !ADDMASK && !SPLIT), "Q is encoded in the kernel only in the plain forward");
 
     // Work items are (q tile, b*h) pairs, `total_wg` of them; an item takes `ntiles` steps (key
@@ -279,28 +184,23 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         for (int s = 0; s < KSTEPS; s++) qf[s] = *reinterpret_cast<const v4i*>(qp + s * 32);
         sq = qscale[bh * (nq_pad / blkq) + qrow / blkq] * kMagicUnit;
     }
-    // QF: this lane's 16 channels of every 32 (its half of the row), rows past N_q as zeros, and the
-    // channel multipliers that go with them
-    u32x4 rw[QF ? KSTEPS : 1][2];
-    v4f qm[QF ? KSTEPS : 1][4];
+    // QF: the wave's 32 rows, 16 bytes per lane and whole rows per instruction (rows past N_q as zeros), and
+    // the multipliers of the lane's eight channels
+    constexpr int Q_CPR = D / 8, Q_RPI = 64 / Q_CPR, Q_NI = QF ? 32 / Q_RPI : 1;     // chunks per row, rows per load, loads
+    u32x4 rw[Q_NI];
+    float qm[8];
     if constexpr (QF) {
-        {
-            const float* mp = qmul + bh * D + half * 16;
+        const float* mp = qmul + bh * D + (lane % Q_CPR) * 8;
+        const v4f m0 = *reinterpret_cast<const v4f*>(mp), m1 = *reinterpret_cast<const v4f*>(mp + 4);
+        const uint16_t* qp = q_src + b * qsb + h * qsh + (lane % Q_CPR) * 8;
 #pragma unroll
-            for (int s = 0; s < KSTEPS; s++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) qm[s][j] = *reinterpret_cast<const v4f*>(mp + s * 32 + j * 4);
+        for (int i = 0; i < Q_NI; i++) {
+            const int r = wave_row0 + i * Q_RPI + lane / Q_CPR;
+            rw[i] = u32x4{0u, 0u, 0u, 0u};
+            if (r < Nq) rw[i] = *reinterpret_cast<const u32x4*>(qp + (int64_t)r * qsn);
         }
-        {
-            const uint16_t* qp = q_src + b * qsb + h * qsh + (int64_t)qrow * qsn + half * 16;
 #pragma unroll
-            for (int s = 0; s < KSTEPS; s++)
-#pragma unroll
-                for (int j = 0; j < 2; j++) {
-                    rw[s][j] = u32x4{0u, 0u, 0u, 0u};
-                    if (qrow < Nq) rw[s][j] = *reinterpret_cast<const u32x4*>(qp + s * 32 + j * 8);
-                }
-        }
+        for (int e = 0; e < 4; e++) qm[e] = m0[e], qm[4 + e] = m1[e];
         // (the arithmetic follows further down, behind the first tile copies: their latency and this
         // one's then run side by side)
     }
@@ -480,31 +380,20 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         dma_v(min(x, last), x % NSV);
     }
     if constexpr (QF) {
-        // ---- Q of this wave's 32 rows -> int8 codes and scale (quant_i8_block's arithmetic)
-        float x[KSTEPS][16];
+        // ---- Q of this wave's 32 rows -> int8 codes and scale (quant_i8_block's arithmetic).  The codes
+        // turn from the row layout they are loaded in into operand fragments through the wave's own piece
+        // of LDS.  (Fragments loaded as such — a lane's 16 channels of its own row — are 64 separate pieces
+        // per instruction, an address cycle each: 8 row and 16 multiplier loads per wave instead of 8 and 2
+        // took the eight waves 5 us more per workgroup.)
         float am = 0.0f;
-        {
 #pragma unroll
-            for (int s = 0; s < KSTEPS; s++)
+        for (int i = 0; i < Q_NI; i++)
 #pragma unroll
-                for (int j = 0; j < 2; j++) {
-                    const v4f m0 = qm[s][2 * j], m1 = qm[s][2 * j + 1];
-                    const float m[8] = {m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w};
+            for (int e = 0; e < 4; e++)
+                am = fmaxf(fmaxf(am, fabsf(__uint_as_float(rw[i][e] << 16) * qm[2 * e])), fabsf(__uint_as_float(rw[i][e] & 0xFFFF0000u) * qm[2 * e + 1]));
+        // the wave's 32 rows, then the waves that share a scale block
 #pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        x[s][j * 8 + 2 * e] = __uint_as_float(rw[s][j][e] << 16) * m[2 * e];
-                        x[s][j * 8 + 2 * e + 1] = __uint_as_float(rw[s][j][e] & 0xFFFF0000u) * m[2 * e + 1];
-                        am = fmaxf(fmaxf(am, fabsf(x[s][j * 8 + 2 * e])), fabsf(x[s][j * 8 + 2 * e + 1]));
-                    }
-                }
-        }
-        // the row's other half, then the wave's 32 rows, then the waves that share a scale block
-        {
-            const v2u r = __builtin_amdgcn_permlane32_swap(__float_as_uint(am), __float_as_uint(am), false, false);
-            am = fmaxf(__uint_as_float(r.x), __uint_as_float(r.y));
-        }
-#pragma unroll
-        for (int off = 1; off < 32; off <<= 1) am = fmaxf(am, __shfl_xor(am, off, 64));
+        for (int off = 1; off < 64; off <<= 1) am = fmaxf(am, __shfl_xor(am, off, 64));
         if (blkq > 32) {
             if (lane == 0) lds_qmax[wave] = am;
             __syncthreads();
@@ -515,40 +404,23 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         const float sc = am > 0.0f ? am / 127.0f : 1.0f;
         const bool fast = sc >= 0x1p-100f && sc <= 0x1p100f;
         const float rinv = 1.0f / sc;
-        float kRound = 12582912.0f, rv = rinv;             // (see quant_i8_block)
-        asm volatile("" : "+v"(rv), "+v"(kRound));
+        // fp16 variant: the V^T slots that the first copies do not go to; e4m3: a region of its own
+        uint8_t* qs = (VARIANT == 0 ? &lds_v[LEAD][0] : &lds_qc[0]) + wave * 32 * D;
+        static_assert(VARIANT != 0 || !QF || (NSV - LEAD) * V_BYTES >= NW * 32 * D, "Q codes must fit the idle V^T slots");
 #pragma unroll
-        for (int s = 0; s < KSTEPS; s++) {
-            uint32_t tb[16], wd[4];
-            float dm = 0.0f;
+        for (int i = 0; i < Q_NI; i++) {
+            float x[8];
 #pragma unroll
-            for (int e = 0; e < 16; e += 2) {
-                const float t0 = fmaf(x[s][e], rv, kRound), t1 = fmaf(x[s][e + 1], rv, kRound);
-                const float d0 = fmaf(x[s][e], rv, -(t0 - kRound)), d1 = fmaf(x[s][e + 1], rv, -(t1 - kRound));
-                dm = fmaxf(fmaxf(dm, fabsf(d0)), fabsf(d1));
-                tb[e] = __float_as_uint(t0);
-                tb[e + 1] = __float_as_uint(t1);
+            for (int e = 0; e < 4; e++) {
+                x[2 * e] = __uint_as_float(rw[i][e] << 16) * qm[2 * e];
+                x[2 * e + 1] = __uint_as_float(rw[i][e] & 0xFFFF0000u) * qm[2 * e + 1];
             }
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const uint32_t lo = __builtin_amdgcn_perm(tb[4 * j + 1], tb[4 * j], 0x0c0c0400u);
-                const uint32_t hi = __builtin_amdgcn_perm(tb[4 * j + 3], tb[4 * j + 2], 0x0c0c0400u);
-                wd[j] = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
-            }
-            if (__builtin_expect(!fast || __any(!(dm <= 0.5f - 0x1p-16f)), 0)) {
-                asm volatile("" ::: "memory");
-#pragma unroll
-                for (int j = 0; j < 4; j++) wd[j] = 0u;
-#pragma unroll
-                for (int e = 0; e < 16; e++) {
-                    float r = rint_quotient(x[s][e], sc, rinv, fast);
-                    r = r > 127.0f ? 127.0f : r;
-                    r = r < -127.0f ? -127.0f : r;
-                    wd[e >> 2] |= ((uint32_t)((int)r) & 0xFFu) << ((e & 3) * 8);
-                }
-            }
-            qf[s] = v4i{(int)wd[0], (int)wd[1], (int)wd[2], (int)wd[3]};
+            // (16-byte chunks of a row XORed with the row: both sides then touch every bank)
+            const int r = i * Q_RPI + lane / Q_CPR, c = (lane % Q_CPR) >> 1;
+            *reinterpret_cast<u32x2*>(qs + r * D + ((c ^ (r & (D / 16 - 1))) << 4) + (lane & 1) * 8) = encode8_i8(x, sc, rinv, fast);
         }
+#pragma unroll
+        for (int s = 0; s < KSTEPS; s++) qf[s] = *reinterpret_cast<const v4i*>(qs + l32 * D + (((s * 2 + half) ^ (l32 & (D / 16 - 1))) << 4));
         sq = sc * kMagicUnit;
     }
     dma_wait<LEAD*(K_CH + V_CH)>();
@@ -648,17 +520,10 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
 #pragma unroll
                 for (int g = 0; g < 4; g++) {
                     const int key = key0 + kb * 32 + g * 8 + half * 4;
-                    uint32_t w0 = 0u, w1 = 0u;
-                    if (key + 4 <= kv_valid) {
-                        const u32x2 w = *reinterpret_cast<const u32x2*>(mrow + key);
-                        w0 = w.x; w1 = w.y;
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < 4; e++)
-                            if (key + e < kv_valid) (e < 2 ? w0 : w1) |= (uint32_t)mrow[key + e] << ((e & 1) * 16);
-                    }
-                    const float mv[4] = {__uint_as_float(w0 << 16), __uint_as_float(w0 & 0xFFFF0000u),
-                                         __uint_as_float(w1 << 16), __uint_as_float(w1 & 0xFFFF0000u)};
+                    uint32_t w[2] = {0u, 0u};
+                    load_bias4(mrow, key, kv_valid, w);
+                    const float mv[4] = {__uint_as_float(w[0] << 16), __uint_as_float(w[0] & 0xFFFF0000u),
+                                         __uint_as_float(w[1] << 16), __uint_as_float(w[1] & 0xFFFF0000u)};
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
                         const float sdq = (__int_as_float(s[X][kb][g * 4 + e]) - Magic<D>::F) * f[kb];
@@ -993,31 +858,42 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         l_tot = lacc[0];
     }
     const float inv = 1.0f / l_tot + poison;      // l carries pscale, which cancels the pscale in P
-    if (qrow < Nq) {
-        uint16_t* op = o + b * osb + h * osh + (int64_t)qrow * osn;
+    // Through LDS, so that a store instruction writes whole rows (a lane's own 8-byte pieces are 64
+    // separate rows per instruction).  The first half of the waves uses the K ring, the others the V^T ring.
+    __syncthreads();                                // every wave is done with the rings
+    {
+        static_assert(NSK * K_BYTES >= NW / 2 * 64 * D && NSV * V_BYTES >= NW / 2 * 64 * D, "output rows must fit the rings");
+        constexpr int OC = D / 8;                   // 16-byte chunks per output row, XORed with the row
+        uint8_t* os = wave < NW / 2 ? &lds_k[0][0] + wave * 64 * D : &lds_v[0][0] + (wave - NW / 2) * 64 * D;
 #pragma unroll
         for (int d = 0; d < DB; d++)
 #pragma unroll
             for (int g = 0; g < 4; g++) {
-                const int ch = d * 32 + g * 8 + half * 4;
                 float x[4];
 #pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    x[e] = oacc[d][g * 4 + e];
-                    if (VARIANT == 1) x[e] = x[e] * vscale[bh * D + ch + e];
-                    x[e] *= inv;
+                for (int e = 0; e < 4; e++) x[e] = oacc[d][g * 4 + e];
+                if constexpr (VARIANT == 1) {
+                    const v4f vs = *reinterpret_cast<const v4f*>(vscale + bh * D + d * 32 + g * 8 + half * 4);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) x[e] *= vs[e];
                 }
-                u32x2 pk;
-                pk.x = f32_to_bf16_rne(x[0]) | ((uint32_t)f32_to_bf16_rne(x[1]) << 16);
-                pk.y = f32_to_bf16_rne(x[2]) | ((uint32_t)f32_to_bf16_rne(x[3]) << 16);
-                *reinterpret_cast<u32x2*>(op + ch) = pk;
+                *reinterpret_cast<u32x2*>(os + l32 * (D * 2) + (((d * 4 + g) ^ (l32 & (OC - 1))) << 4) + half * 8) =
+                    u32x2{pack_bf16(x[0] * inv, x[1] * inv), pack_bf16(x[2] * inv, x[3] * inv)};
             }
-        if (STATS && half == 0) {
-            // natural-log log-sum-exp of the scaled scores.  With K smoothing every score
-            // of a row was lowered by <q, mean>, which the Q quantizer recorded per row.
-            const float shift = qshift != nullptr ? qshift[bh * nq_pad + qrow] : 0.0f;
-            stats[bh * Nq + qrow] = (m_used + __builtin_amdgcn_logf(l_tot) - Lazy<VARIANT>::log2_pscale + shift) * 0.6931471805599453f;
+        constexpr int RPI = 64 / OC;                // rows per store instruction
+        uint16_t* op = o + b * osb + h * osh + (lane % OC) * 8;
+#pragma unroll
+        for (int i = 0; i < 32 / RPI; i++) {
+            const int r = i * RPI + lane / OC;
+            const u32x4 w = *reinterpret_cast<const u32x4*>(os + r * (D * 2) + (((lane % OC) ^ (r & (OC - 1))) << 4));
+            if (wave_row0 + r < Nq) *reinterpret_cast<u32x4*>(op + (int64_t)(wave_row0 + r) * osn) = w;
         }
+    }
+    if (STATS && qrow < Nq && half == 0) {
+        // natural-log log-sum-exp of the scaled scores.  With K smoothing every score
+        // of a row was lowered by <q, mean>, which the Q quantizer recorded per row.
+        const float shift = qshift != nullptr ? qshift[bh * nq_pad + qrow] : 0.0f;
+        stats[bh * Nq + qrow] = (m_used + __builtin_amdgcn_logf(l_tot) - Lazy<VARIANT>::log2_pscale + shift) * 0.6931471805599453f;
     }
     } while (SPLIT && span_end > span_begin);       // segments
 #ifdef SAGE_CLOCK_PROBE

@@ -1,0 +1,155 @@
+// sage_attn_common.h — what the attention kernels share: vector types, the biased score accumulators, the
+// reference-maximum rule and the bf16 rounding of their outputs.
+#pragma once
+
+#include "sage_internal.h"
+
+namespace sage {
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v8i __attribute__((ext_vector_type(8)));
+typedef int v16i __attribute__((ext_vector_type(16)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned v2u __attribute__((ext_vector_type(2)));
+
+// Byte offset of 16-byte chunk L of a tile.  Chunks are grouped into 128-byte super-rows
+// (8 chunks); the chunk position inside a super-row is XORed with bits of the index of
+// the PAIR of super-rows it belongs to, so that the 16 lanes the 64-bank LDS serves per
+// cycle (16 consecutive rows, one logical column) land in 16 different 16-byte bank groups.
+__device__ __forceinline__ int swz(int L) { return (((L >> 3) << 3) | ((L & 7) ^ ((L >> 4) & 7))) << 4; }
+
+// 16 bytes per lane from global memory straight into LDS: lane l of the wave lands at
+// lds_base + 16*l.  Written as assembly on purpose: the compiler then keeps no record of
+// an outstanding LDS write and does not put a full vector-memory wait in front of every
+// later LDS read; completion is awaited explicitly (dma_wait) before the workgroup
+// barrier that publishes the tile.
+__device__ __forceinline__ void dma16(const void* gbase_uniform, uint32_t goff, uint32_t lds_base_uniform) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :
+                 : "s"(lds_base_uniform), "v"(goff), "s"(gbase_uniform)
+                 : "memory");      // (m0 cannot be named as a clobber: to this compiler it is a reserved register — it
+                                   // warns that "clobbering them may lead to undefined behaviour" — which it never
+                                   // keeps a value in across statements; its own uses set m0 right before the use)
+}
+// Wait until at most N of this wave's copies are still in flight (they complete in order).
+template <int N> __device__ __forceinline__ void dma_wait() {
+    static_assert(N >= 0 && N < 64, "vmcnt is a 6-bit counter");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+__device__ __forceinline__ uint32_t lds_addr(const void* p) {
+    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
+}
+
+// Two floats -> packed bf16, round to nearest even.
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
+    const v2f f = {a, b};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, v2bf));
+}
+
+// The int32 score accumulators start at the bit pattern of the float 1/(2*pi) instead of 0.
+// That pattern is 2^-3 * (1 + 2292099 * 2^-23), so adding an integer dot with
+// |dot| < 2292099 (the largest possible |dot| is 128*127*127 = 2064512) changes only the
+// mantissa: a finished accumulator, read as fp32, IS the float 1/(2*pi) + dot * 2^-26.  No
+// int->float conversion is needed and dequantisation, max subtraction and the exponent
+// argument collapse into one FMA per score (the scale carries the factor 2^26).
+constexpr int kMagicI = 0x3E22F983;
+constexpr float kMagicF = 0.15915494309189532f;        // the same 32 bits
+constexpr float kMagicUnit = 67108864.0f;               // 2^26: accumulator-as-float steps per integer
+// With 256 channels |dot| can reach 256*127*127 = 4129024, more than the mantissa of 1/(2*pi) has
+// room for below it.  0.1875 = 2^-3 * (1 + 2^22 * 2^-23) leaves 2^22 = 4194304 either way at the
+// same step of 2^-26.
+constexpr int kMagicWideI = 0x3E400000;
+constexpr float kMagicWideF = 0.1875f;
+// e4m3 variant: a wave whose bias * f can exceed this takes the bias off its accumulators (see exact_bias).
+constexpr float kExactBias = 4096.0f;
+template <int D> struct Magic {
+    static constexpr int I = D > 128 ? kMagicWideI : kMagicI;
+    static constexpr float F = D > 128 ? kMagicWideF : kMagicF;
+};
+
+// First matrix instruction of a score chain: accumulator input = the constant above, held in 16
+// registers for the whole kernel (behind an empty statement, or the compiler re-creates the 16
+// copies for every chain).  The instruction could take 1/(2*pi) as an inline operand, but only
+// written as assembly, and then the compiler does not know that a matrix instruction is writing
+// those registers: it neither keeps the wait states before the first other instruction that
+// touches them — a spill store two instructions later wrote the old contents — nor can it be told.
+template <int D>
+__device__ __forceinline__ v16i magic_splat() {
+    constexpr int M = Magic<D>::I;
+    v16i c = {M, M, M, M, M, M, M, M, M, M, M, M, M, M, M, M};
+    asm volatile("" : "+v"(c));
+    return c;
+}
+
+// A row's reference maximum is only refreshed (and the accumulators rescaled) when a tile
+// exceeds it by more than tau powers of two; until then p = exp2(s - m_used) may reach
+// 2^tau.  fp16 P holds 2^8 without loss.  The e4m3 variant maps p = 2^tau to the format
+// maximum 448, i.e. it stores e4m3(p * 448 / 2^tau); the factor cancels against the
+// normaliser, which sums the same scaled values.  Its reference is always a whole number
+// (the maximum rounded up): a probability's e4m3 significand then depends on the fractional
+// part of its score only, not on which whole number the reference happens to be, so the
+// stored probabilities are those of a softmax taken against ceil(row maximum) up to a power
+// of two, and the rescale factors are exact.
+template <int VARIANT> struct Lazy {
+    static constexpr float tau = VARIANT == 0 ? 8.0f : 1.0f;
+    static constexpr float log2_pscale = VARIANT == 0 ? 0.0f : 7.807354922057604f;     // log2(448 / 2)
+    static constexpr bool integer_ref = VARIANT == 1;
+};
+
+// Eight scaled values of a row -> int8 codes: the quantizer's arithmetic (quant_i8_block in
+// sage_quant.hip: one fused multiply-add with a magic addend per code, the true quotient where some lane
+// comes close to a rounding tie).  The whole wave calls it.
+__device__ __forceinline__ u32x2 encode8_i8(const float (&x)[8], float sc, float rinv, bool fast) {
+    float kRound = 12582912.0f, rv = rinv;
+    asm volatile("" : "+v"(rv), "+v"(kRound));
+    uint32_t tb[8], wd[2];
+    float dm = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+        const float t0 = fmaf(x[e], rv, kRound), t1 = fmaf(x[e + 1], rv, kRound);
+        const float d0 = fmaf(x[e], rv, -(t0 - kRound)), d1 = fmaf(x[e + 1], rv, -(t1 - kRound));
+        dm = fmaxf(fmaxf(dm, fabsf(d0)), fabsf(d1));
+        tb[e] = __float_as_uint(t0);
+        tb[e + 1] = __float_as_uint(t1);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const uint32_t lo = __builtin_amdgcn_perm(tb[4 * j + 1], tb[4 * j], 0x0c0c0400u);
+        const uint32_t hi = __builtin_amdgcn_perm(tb[4 * j + 3], tb[4 * j + 2], 0x0c0c0400u);
+        wd[j] = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+    }
+    if (__builtin_expect(!fast || __any(!(dm <= 0.5f - 0x1p-16f)), 0)) {
+        asm volatile("" ::: "memory");
+        wd[0] = wd[1] = 0u;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            float r = rint_quotient(x[e], sc, rinv, fast);
+            r = r > 127.0f ? 127.0f : r;
+            r = r < -127.0f ? -127.0f : r;
+            wd[e >> 2] |= ((uint32_t)((int)r) & 0xFFu) << ((e & 3) * 8);
+        }
+    }
+    return u32x2{wd[0], wd[1]};
+}
+
+// Four consecutive bf16 values of a bias row, keys key .. key + 3 (those at and past `n` are left out).
+// Rows start at any even byte address: the access is as wide as the hardware takes it unaligned.
+__device__ __forceinline__ void load_bias4(const uint16_t* row, int key, int n, uint32_t (&w)[2]) {
+    if (key + 4 <= n) {
+        __builtin_memcpy(w, row + key, 8);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            if (key + e < n) w[e >> 1] |= (uint32_t)row[key + e] << ((e & 1) * 16);
+    }
+}
+
+}  // namespace sage
