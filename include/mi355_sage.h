@@ -352,7 +352,9 @@ int mi355_sage_attn_fwd_q16(
     void* O, const int64_t* o_strides, int64_t o_offset_elems, void* stream);
 
 /* Scheduling of the attention kernel (no counterpart in the reference).
- * One workgroup computes 256 query rows of one head against all keys.  A shape whose row tiles
+ * One workgroup computes 256 query rows of one head against all keys.  A problem too small to fill the
+ * chip that way takes 32 or 64 rows per workgroup and splits the keys over the workgroup's waves, which
+ * merge their partial results on the spot.  A shape whose row tiles
  * leave the last round of the 256 compute units at most half full (more than 256 tiles, 16 % or
  * more of the launch idle; fp16 variant, head dim up to 128) is instead cut into equal shares of
  * (row tile, key tile) steps for exactly 256 workgroups, which hand unnormalised partial results to

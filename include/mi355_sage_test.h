@@ -8,7 +8,8 @@
 extern "C" {
 #endif
 
-/* Attention scheduling.  mode 0: by shape and device (default); -1: never split; n > 0 (multiple
+/* Attention scheduling.  mode 0: by shape and device (default); -1: one 256-row workgroup per row tile
+ * whatever the shape (never split, never the short form below); n > 0 (multiple
  * of 8, <= 1024): always split over n workgroups (fp16 variant, head dim up to 128; hand-over slots
  * a caller's workspace does not hold come from a library-owned per-stream buffer).  Returns 0, or -1
  * for a mode outside these. */
@@ -25,6 +26,16 @@ int mi355_sage_set_attn_split_wait(int polls);
 /* Workgroups the split schedule would use for this shape on a device that supports it (256), or 0
  * for one workgroup per row tile: the rule alone, whatever the switch above and the device say. */
 int mi355_sage_attn_split_rule(int B, int H, int N_q, int N_kv, int D, int variant);
+
+/* The short form of the attention kernel (32 or 64 query rows per workgroup, keys split over its
+ * waves).  mode 0: by shape (default); -1: never; 8 or 4: always, with that many key runs per row
+ * block (head dim 256: always 4).  4 and 8 take precedence over the switch above, which otherwise keeps
+ * the short form out when it is set.  Returns 0, or -1 for
+ * a mode outside these. */
+int mi355_sage_set_attn_short(int mode);
+
+/* Key runs the short form would use for this shape by the rule alone, 0 for the 256-row workgroups. */
+int mi355_sage_attn_short_rule(int B, int H, int N_q, int N_kv, int D, int variant);
 
 #ifdef __cplusplus
 }

@@ -988,6 +988,7 @@ static hipError_t launch_attn_dv(const AttnArgs& a, hipStream_t st) {
 static std::atomic<int> g_split_mode{0};       // 0: by shape and device; -1: never; n > 0: always, over n workgroups
 
 void attn_split_override(int mode) { g_split_mode.store(mode); }
+int attn_split_override_mode() { return g_split_mode.load(); }
 
 static bool split_fits(int B, int H, int Nq, int kv_valid, int D, int variant) {
     if (D > 128) return false;                 // four-wave workgroups: one per item
@@ -1063,6 +1064,7 @@ size_t attn_split_bytes(int workgroups, int D) {
 
 hipError_t launch_attn(const AttnArgs& a, hipStream_t st) {
     if (a.nkv_pad > max_keys(a.D)) return hipErrorInvalidValue;      // K scales would not fit the LDS staging
+    if (a.short_kw > 0) return launch_attn_short(a, st);
     if (a.D == 128) return a.variant == 0 ? launch_attn_dv<128, 0>(a, st) : launch_attn_dv<128, 1>(a, st);
     if (a.D == 64) return a.variant == 0 ? launch_attn_dv<64, 0>(a, st) : launch_attn_dv<64, 1>(a, st);
     if (a.D == 256) return a.variant == 0 ? launch_attn_dv<256, 0>(a, st) : launch_attn_dv<256, 1>(a, st);

@@ -1,0 +1,459 @@
+// sage_attn_short.hip — attention on quantized operands for problems too small to fill the chip with
+// 256-row workgroups (gfx950).
+//
+// The main kernel (sage_attn.hip) gives a workgroup 256 query rows and all keys.  At a few hundred
+// tokens that is a few dozen workgroups on 256 compute units, each walking every key tile in turn.
+// Here a workgroup owns 32 or 64 query rows and its waves split the KEYS: wave (r, w) computes rows
+// 32 r .. 32 r + 31 against the w-th of KW equal runs of key steps, and the KW partial results (row
+// maximum, row sum, unnormalised output) meet in LDS at the end — the same online-softmax merge a wave
+// does from step to step, done once across waves.  The matrix layouts are the main kernel's:
+// S^T = K . Q^T, O^T = V^T . P^T, probabilities straight from the score accumulators.
+//
+// No wave shares a key with another, so every wave keeps one step's K and V^T in an LDS region of its own,
+// filled by register-bypassing copies (contiguous runs, swizzled on the source side like the main kernel's
+// tiles): K of the next step as soon as the scores have read theirs, V^T once P.V has.  The waits are the
+// wave's own copy counters; the loop has no barrier.  (Fragments loaded from L2 straight into registers —
+// no LDS at all — were built first: a fragment is 64 separate 16-byte pieces, an address cycle each, and
+// the first step alone took 6.4 us at [1,256,30,128].)  Per key tile a compute unit moves 8 times the main
+// kernel's operand bytes per query row, which is why attn_short_rule stops where the main kernel's
+// workgroups start to fill the chip.
+#include "sage_attn_common.h"
+
+#include <atomic>
+
+namespace sage {
+
+template <int D> constexpr int short_waves() { return D > 128 ? 4 : 8; }      // 256 channels: a wave needs a SIMD's registers
+
+template <int D, int VARIANT, int KW, bool QF, bool ADDMASK>
+__global__ __launch_bounds__(short_waves<D>() * 64) void sage_attn_short_kernel(AttnArgs a, int n_rtiles, int total_wg) {
+    constexpr int NW = short_waves<D>();
+    constexpr int R = NW / KW;                          // 32-row blocks per workgroup
+    constexpr int ROWS = 32 * R;
+    constexpr int KSTEPS = D / 32, DB = D / 32, CPR = D / 8;
+    constexpr int VB = VARIANT == 0 ? 2 : 1;
+    constexpr int SK = VARIANT == 0 ? 32 : 64;          // keys per step (what the P.V matrix instruction divides into)
+    constexpr int SKB = SK / 32;
+    constexpr int NK = KSTEPS * SKB;                    // K fragments per step
+    constexpr int NV = 2 * DB;                          // V^T fragments of 16 bytes per step
+    constexpr int K_BYTES = SK * D, V_BYTES = D * 64;   // one step's K and V^T
+    constexpr int KC = K_BYTES / 1024, VC = V_BYTES / 1024;      // 1 KiB copies of either
+    constexpr int NP = 8 * SKB;                         // pairs of scores per lane and step
+    constexpr int LD = D + 4;                           // floats per row of the exchange buffer (keeps 16-byte alignment, spreads banks)
+    static_assert(NW % KW == 0 && ROWS <= 128, "waves = row blocks x key runs");
+
+    struct Ring { uint8_t k[K_BYTES], v[V_BYTES]; };
+    union Mem {
+        Ring ring[NW];                                  // the loop's operands
+        float acc[NW][32 * LD];                         // the merge's partial outputs
+    };
+    __shared__ __attribute__((aligned(1024))) Mem mem;
+    __shared__ __attribute__((aligned(16))) uint8_t lds_q[QF ? ROWS * D : 16];      // this workgroup's Q codes
+    __shared__ float lds_m[NW][32], lds_l[NW][32];
+    __shared__ float lds_qmax[8];
+
+    // each XCD takes a contiguous range of workgroups, so that those sharing a head share its L2
+    const int bid = blockIdx.x;
+    const int per = total_wg >> 3, extra = total_wg & 7, xcd = bid & 7;
+    const int wg = xcd * per + min(xcd, extra) + (bid >> 3);
+    const int rt = wg % n_rtiles, bh = wg / n_rtiles;
+    const int b = bh / a.H, h = bh % a.H;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, half = lane >> 5;
+    const int kw = wave % KW, rg = wave / KW;
+    const int wg_row0 = rt * ROWS, row0 = wg_row0 + rg * 32, qrow = row0 + l32;
+
+    // causal: keys past the workgroup's last row count as the ragged end
+    const int kv_valid = a.causal ? min(a.kv_valid, wg_row0 + ROWS) : a.kv_valid;
+    const int nsteps = (kv_valid + SK - 1) / SK;
+    const int h0 = nsteps * kw / KW, h1 = nsteps * (kw + 1) / KW;
+
+    // ---- one step's operands: copies into the wave's own LDS region, fragments out of it
+    const uint8_t* kg = reinterpret_cast<const uint8_t*>(a.k8) + (int64_t)bh * a.nkv_pad * D;
+    const uint8_t* vg = static_cast<const uint8_t*>(a.vq) + (int64_t)bh * a.nkv_pad * D * VB;
+    const uint32_t k_lds = lds_addr(&mem.ring[wave].k[0]), v_lds = lds_addr(&mem.ring[wave].v[0]);
+    int vsrc[VC];
+#pragma unroll
+    for (int i = 0; i < VC; i++) {
+        // (fp16: a step is half of a 64-key tile, 64 bytes of every 128-byte channel row)
+        const int L = swz(i * 64 + lane);
+        vsrc[i] = VARIANT == 0 ? (L >> 6) * 128 + (L & 63) : L;
+    }
+    auto copy_k = [&](int hs) {
+        const uint8_t* g = kg + (int64_t)hs * K_BYTES;
+#pragma unroll
+        for (int i = 0; i < KC; i++) dma16(g, swz(i * 64 + lane), __builtin_amdgcn_readfirstlane(k_lds + i * 1024));
+    };
+    auto copy_v = [&](int hs) {
+        const uint8_t* g = VARIANT == 0 ? vg + (int64_t)(hs >> 1) * (D * 128) + (hs & 1) * 64 : vg + (int64_t)hs * V_BYTES;
+#pragma unroll
+        for (int i = 0; i < VC; i++) dma16(g, vsrc[i], __builtin_amdgcn_readfirstlane(v_lds + i * 1024));
+    };
+    typedef const __attribute__((address_space(3))) v4i* lds_v4i_ptr;
+    auto k_frag = [&](int n) -> v4i {
+        return *reinterpret_cast<lds_v4i_ptr>(k_lds + swz(((n / KSTEPS) * 32 + l32) * (D / 16) + (n % KSTEPS) * 2 + half));
+    };
+    // fp16: fragment jj * DB + d = 16 keys, channels 32 d ..; e4m3: fragments 2 d, 2 d + 1 = a lane's 32 keys, channels 32 d ..
+    auto v_frag = [&](int n) -> v4i {
+        const int d = VARIANT == 0 ? n % DB : n >> 1;
+        const int c = VARIANT == 0 ? (n / DB) * 2 + half : half * 2 + (n & 1);
+        return *reinterpret_cast<lds_v4i_ptr>(v_lds + swz((d * 32 + l32) * 4 + c));
+    };
+    // (LDS reads issued before this have delivered: what they read may be overwritten)
+    auto reads_done = [] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
+    if (h0 < h1) {
+        copy_k(h0);
+        copy_v(h0);
+    }
+
+    // ---- Q^T fragments of the wave's 32 rows
+    v4i qf[KSTEPS];
+    float sq;
+    if constexpr (!QF) {
+        const int8_t* qp = a.q8 + ((int64_t)bh * a.nq_pad + qrow) * D + half * 16;
+#pragma unroll
+        for (int s = 0; s < KSTEPS; s++) qf[s] = *reinterpret_cast<const v4i*>(qp + s * 32);
+        sq = a.qscale[(int64_t)bh * (a.nq_pad / a.blkq) + qrow / a.blkq] * kMagicUnit;
+    } else {
+        // Q arrives as bf16: the quantizer's arithmetic, so its codes and scales.  A scale block is wider
+        // than the workgroup's rows as a rule: the waves take the maxima of the whole block, 16 rows at a
+        // time, and the ones that hold this workgroup's rows encode them into LDS for everybody.
+        const uint16_t* qb = a.q_src + b * a.qsb + h * a.qsh;
+        const int cover = a.blkq > ROWS ? a.blkq : ROWS;                 // 32 .. 128 rows: the scale blocks of this workgroup
+        const int cover0 = wg_row0 / cover * cover;
+        constexpr int RPI = 64 / CPR;                                    // rows per load instruction
+        constexpr int NI = 16 / RPI;
+        constexpr int TURNS = 8 / NW;                                    // 16-row pieces of the largest block per wave
+        const int col = (lane % CPR) * 8, rr = lane / CPR;
+        u32x4 w[TURNS][NI];
+#pragma unroll
+        for (int t = 0; t < TURNS; t++)
+#pragma unroll
+            for (int i = 0; i < NI; i++) {
+                const int piece = t * NW + wave, row = cover0 + piece * 16 + i * RPI + rr;
+                w[t][i] = u32x4{0u, 0u, 0u, 0u};
+                if (piece < cover / 16 && row < a.Nq) w[t][i] = *reinterpret_cast<const u32x4*>(qb + (int64_t)row * a.qsn + col);
+            }
+        float m[8];
+        {
+            const float* mp = a.qmul + (int64_t)bh * D + col;
+            const v4f m0 = *reinterpret_cast<const v4f*>(mp), m1 = *reinterpret_cast<const v4f*>(mp + 4);
+#pragma unroll
+            for (int e = 0; e < 4; e++) m[e] = m0[e], m[4 + e] = m1[e];
+        }
+#pragma unroll
+        for (int t = 0; t < TURNS; t++) {
+            float am = 0.0f;
+#pragma unroll
+            for (int i = 0; i < NI; i++)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    am = fmaxf(fmaxf(am, fabsf(__uint_as_float(w[t][i][e] << 16) * m[2 * e])), fabsf(__uint_as_float(w[t][i][e] & 0xFFFF0000u) * m[2 * e + 1]));
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) am = fmaxf(am, __shfl_xor(am, off, 64));
+            if (lane == 0) lds_qmax[t * NW + wave] = am;
+        }
+        __syncthreads();
+        auto block_scale = [&](int row) {                                // of the scale block that holds `row`
+            const int s0 = (row - cover0) / a.blkq * (a.blkq / 16);
+            float am = 0.0f;
+            for (int i = 0; i < a.blkq / 16; i++) am = fmaxf(am, lds_qmax[s0 + i]);
+            return am > 0.0f ? am / 127.0f : 1.0f;
+        };
+#pragma unroll
+        for (int t = 0; t < TURNS; t++) {
+            const int prow = cover0 + (t * NW + wave) * 16 - wg_row0;    // first row of the piece in this workgroup
+            if (prow < 0 || prow >= ROWS) continue;
+            const float sc = block_scale(wg_row0 + prow);
+            const bool fast = sc >= 0x1p-100f && sc <= 0x1p100f;
+            const float rinv = 1.0f / sc;
+#pragma unroll
+            for (int i = 0; i < NI; i++) {
+                float x[8];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    x[2 * e] = __uint_as_float(w[t][i][e] << 16) * m[2 * e];
+                    x[2 * e + 1] = __uint_as_float(w[t][i][e] & 0xFFFF0000u) * m[2 * e + 1];
+                }
+                *reinterpret_cast<u32x2*>(&lds_q[(prow + i * RPI + rr) * D + col]) = encode8_i8(x, sc, rinv, fast);
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < KSTEPS; s++) qf[s] = *reinterpret_cast<const v4i*>(&lds_q[(rg * 32 + l32) * D + s * 32 + half * 16]);
+        sq = block_scale(row0) * kMagicUnit;
+    }
+
+    const float* ksc = a.kscale + (int64_t)bh * (a.nkv_pad / a.blkk);
+    const int ksh = a.blkk == 32 ? 5 : a.blkk == 64 ? 6 : 7;
+    const uint16_t* mrow = ADDMASK ? a.amask + b * a.amb + h * a.amh + (int64_t)min(qrow, a.Nq - 1) * a.amn : nullptr;
+
+    v16f oacc[DB], lacc;
+#pragma unroll
+    for (int d = 0; d < DB; d++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) oacc[d][i] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; i++) lacc[i] = 0.0f;
+    float m_used = -3.0e38f, l_run = 0.0f;              // (finite: a step whose keys are all masked yields p = 0, not NaN)
+    const v16i smagic = magic_splat<D>();
+    const v8i ones8 = {0x38383838, 0x38383838, 0x38383838, 0x38383838, 0x38383838, 0x38383838, 0x38383838, 0x38383838};
+
+    for (int hs = h0; hs < h1; hs++) {
+        v16i s[SKB];
+        dma_wait<VC>();                                 // K of this step has landed (V^T was requested after it)
+        {
+            v4i kf[NK];
+#pragma unroll
+            for (int n = 0; n < NK; n++) kf[n] = k_frag(n);
+#pragma unroll
+            for (int kb = 0; kb < SKB; kb++)
+#pragma unroll
+                for (int st = 0; st < KSTEPS; st++)
+                    s[kb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[kb * KSTEPS + st], qf[st], st == 0 ? smagic : s[kb], 0, 0, 0);
+        }
+        const bool more = hs + 1 < h1;
+        reads_done();
+        if (more) copy_k(hs + 1);
+        const int key0 = hs * SK;
+        float f[SKB];
+#pragma unroll
+        for (int kb = 0; kb < SKB; kb++) f[kb] = sq * ksc[(key0 + kb * 32) >> ksh];
+        if (key0 + SK > kv_valid || (key0 < a.km.hi && key0 + SK > a.km.lo) || (a.causal && key0 + SK - 1 > row0)) {
+#pragma unroll
+            for (int kb = 0; kb < SKB; kb++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    const int key = key0 + kb * 32 + (i >> 2) * 8 + half * 4 + (i & 3);
+                    if (key >= kv_valid || (key >= a.km.lo && key < a.km.hi) || (a.causal && key > qrow)) s[kb][i] = (int)0xFF800000;
+                }
+        }
+        // scores in the log2 domain (the accumulators' bias taken off exactly), or the raw accumulators where
+        // one multiply-add does the rest
+        float x[SKB][16];
+        float mt = -INFINITY;
+        constexpr bool EXACT = ADDMASK || VARIANT == 1;
+#pragma unroll
+        for (int kb = 0; kb < SKB; kb++) {
+            if constexpr (ADDMASK) {
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    const int key = key0 + kb * 32 + g * 8 + half * 4;
+                    uint32_t w[2] = {0u, 0u};
+                    load_bias4(mrow, key, kv_valid, w);
+                    const float mv[4] = {__uint_as_float(w[0] << 16), __uint_as_float(w[0] & 0xFFFF0000u),
+                                         __uint_as_float(w[1] << 16), __uint_as_float(w[1] & 0xFFFF0000u)};
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        x[kb][g * 4 + e] = fmaf(mv[e], 1.4426950408889634f, (__int_as_float(s[kb][g * 4 + e]) - Magic<D>::F) * f[kb]);
+                        mt = fmaxf(mt, x[kb][g * 4 + e]);
+                    }
+                }
+            } else {
+                // the maximum on the raw accumulators (monotone in the score since f > 0)
+                int mi = s[kb][0];
+#pragma unroll
+                for (int i = 1; i < 16; i++) mi = max(mi, s[kb][i]);
+                mt = fmaxf(mt, mi < 0 ? -INFINITY : (float)(mi - Magic<D>::I) * (f[kb] * (1.0f / kMagicUnit)));
+#pragma unroll
+                for (int i = 0; i < 16; i++) x[kb][i] = EXACT ? __int_as_float(s[kb][i]) - Magic<D>::F : __int_as_float(s[kb][i]);
+            }
+        }
+        {
+            const v2u r = __builtin_amdgcn_permlane32_swap(__float_as_uint(mt), __float_as_uint(mt), false, false);
+            mt = fmaxf(__uint_as_float(r.x), __uint_as_float(r.y));
+        }
+        if (__any(mt > m_used + Lazy<VARIANT>::tau)) {
+            const float m_new = Lazy<VARIANT>::integer_ref ? ceilf(fmaxf(m_used, mt)) : fmaxf(m_used, mt);
+            const float corr = __builtin_amdgcn_exp2f(m_used - m_new);
+            m_used = m_new;
+            l_run *= corr;
+            lacc[0] *= corr;
+#pragma unroll
+            for (int d = 0; d < DB; d++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) oacc[d][i] *= corr;
+        }
+        uint32_t p[8];
+#pragma unroll
+        for (int k = 0; k < NP; k++) {
+            const int kb = k >> 3, i = (2 * k) & 15;
+            float e[2];
+#pragma unroll
+            for (int r = 0; r < 2; r++) {
+                float arg;
+                if constexpr (ADDMASK) arg = x[kb][i + r] - (m_used - Lazy<VARIANT>::log2_pscale);
+                else if constexpr (EXACT) arg = fmaf(x[kb][i + r], f[kb], Lazy<VARIANT>::log2_pscale - m_used);
+                else arg = fmaf(x[kb][i + r], f[kb], Lazy<VARIANT>::log2_pscale - fmaf(Magic<D>::F, f[kb], m_used));
+                e[r] = __builtin_amdgcn_exp2f(arg);
+            }
+            if constexpr (VARIANT == 0) {
+                const v2h pr = {(_Float16)e[0], (_Float16)e[1]};
+                p[k] = __builtin_bit_cast(uint32_t, pr);
+                l_run += e[0];
+                l_run += e[1];
+            } else {
+                const int w = k >> 1;
+                if (k & 1) p[w] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(e[0], e[1], (int)p[w], true);
+                else p[w] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(e[0], e[1], 0, false);
+            }
+        }
+        if (more) dma_wait<KC>();                       // V^T of this step (the next step's K was requested after it)
+        else dma_wait<0>();
+        v4i vf[NV];
+#pragma unroll
+        for (int n = 0; n < NV; n++) vf[n] = v_frag(n);
+        if constexpr (VARIANT == 0) {
+#pragma unroll
+            for (int n = 0; n < NV; n++) {
+                const int jj = n / DB, d = n % DB;
+                const v4i pw = {(int)p[jj * 4], (int)p[jj * 4 + 1], (int)p[jj * 4 + 2], (int)p[jj * 4 + 3]};
+                oacc[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, vf[n]), __builtin_bit_cast(v8h, pw), oacc[d], 0, 0, 0);
+            }
+        } else {
+            const v8i pw = {(int)p[0], (int)p[1], (int)p[2], (int)p[3], (int)p[4], (int)p[5], (int)p[6], (int)p[7]};
+#pragma unroll
+            for (int d = 0; d < DB; d++) {
+                const v4i lo = vf[2 * d], hi = vf[2 * d + 1];
+                const v8i v8 = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+                oacc[d] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(v8, pw, oacc[d], 0, 0, 0, 0, 0, 0);
+            }
+            lacc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(ones8, pw, lacc, 0, 0, 0, 0, 0, 0);
+        }
+        reads_done();
+        if (more) copy_v(hs + 1);
+    }
+
+    // ---- merge of the KW partial results, in LDS
+    float l_row = lacc[0];
+    if constexpr (VARIANT == 0) {
+        const v2u r = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_run), __float_as_uint(l_run), false, false);
+        l_row = __uint_as_float(r.x) + __uint_as_float(r.y);
+    }
+    if (half == 0) {
+        lds_m[wave][l32] = m_used;
+        lds_l[wave][l32] = l_row;
+    }
+    __syncthreads();
+    {
+        float mg = lds_m[rg * KW][l32];
+#pragma unroll
+        for (int w = 1; w < KW; w++) mg = fmaxf(mg, lds_m[rg * KW + w][l32]);
+        const float sc = __builtin_amdgcn_exp2f(m_used - mg);
+        float* dst = &mem.acc[wave][l32 * LD + half * 4];
+#pragma unroll
+        for (int d = 0; d < DB; d++)
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+                *reinterpret_cast<v4f*>(dst + d * 32 + g * 8) = v4f{oacc[d][g * 4] * sc, oacc[d][g * 4 + 1] * sc, oacc[d][g * 4 + 2] * sc, oacc[d][g * 4 + 3] * sc};
+    }
+    __syncthreads();
+    // ---- normalise, bf16, caller's strides: eight channels of a row per thread and turn
+    for (int it = tid; it < ROWS * CPR; it += NW * 64) {
+        const int row = it / CPR, ch = (it % CPR) * 8;
+        const int r = row >> 5, rl = row & 31, grow = wg_row0 + row;
+        if (grow >= a.Nq) continue;
+        float mg = lds_m[r * KW][rl];
+#pragma unroll
+        for (int w = 1; w < KW; w++) mg = fmaxf(mg, lds_m[r * KW + w][rl]);
+        float l_tot = 0.0f;
+        v4f x0 = {0.0f, 0.0f, 0.0f, 0.0f}, x1 = x0;
+#pragma unroll
+        for (int w = 0; w < KW; w++) {
+            l_tot += lds_l[r * KW + w][rl] * __builtin_amdgcn_exp2f(lds_m[r * KW + w][rl] - mg);
+            x0 += *reinterpret_cast<const v4f*>(&mem.acc[r * KW + w][rl * LD + ch]);
+            x1 += *reinterpret_cast<const v4f*>(&mem.acc[r * KW + w][rl * LD + ch + 4]);
+        }
+        const float inv = 1.0f / l_tot;
+        if constexpr (VARIANT == 1) {
+            const float* vs = a.vscale + (int64_t)bh * D + ch;
+#pragma unroll
+            for (int e = 0; e < 4; e++) x0[e] *= vs[e], x1[e] *= vs[4 + e];
+        }
+        const u32x4 pk = {pack_bf16(x0[0] * inv, x0[1] * inv), pack_bf16(x0[2] * inv, x0[3] * inv),
+                          pack_bf16(x1[0] * inv, x1[1] * inv), pack_bf16(x1[2] * inv, x1[3] * inv)};
+        *reinterpret_cast<u32x4*>(a.o + b * a.osb + h * a.osh + (int64_t)grow * a.osn + ch) = pk;
+        if (a.stats != nullptr && ch == 0) {
+            const float shift = a.qshift != nullptr ? a.qshift[(int64_t)bh * a.nq_pad + grow] : 0.0f;
+            a.stats[(int64_t)bh * a.Nq + grow] = (mg + __builtin_amdgcn_logf(l_tot) - Lazy<VARIANT>::log2_pscale + shift) * 0.6931471805599453f;
+        }
+    }
+}
+
+template <int D, int VARIANT, int KW>
+static hipError_t launch_short_dvk(const AttnArgs& a, hipStream_t st) {
+    constexpr int NW = short_waves<D>(), ROWS = 32 * (NW / KW);
+    const int n_rtiles = (a.Nq + ROWS - 1) / ROWS;
+    const int64_t total = (int64_t)n_rtiles * a.B * a.H;
+    if (total <= 0 || total > 0x7FFFFFFF) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)total), block(NW * 64);
+    if (a.q_src != nullptr) {
+        if (a.amask != nullptr || a.qmul == nullptr) return hipErrorInvalidValue;
+        hipLaunchKernelGGL((sage_attn_short_kernel<D, VARIANT, KW, true, false>), grid, block, 0, st, a, n_rtiles, (int)total);
+    } else if (a.amask != nullptr) {
+        hipLaunchKernelGGL((sage_attn_short_kernel<D, VARIANT, KW, false, true>), grid, block, 0, st, a, n_rtiles, (int)total);
+    } else {
+        hipLaunchKernelGGL((sage_attn_short_kernel<D, VARIANT, KW, false, false>), grid, block, 0, st, a, n_rtiles, (int)total);
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_attn_short(const AttnArgs& a, hipStream_t st) {
+    if (a.D == 256) return a.variant == 0 ? launch_short_dvk<256, 0, 4>(a, st) : launch_short_dvk<256, 1, 4>(a, st);
+    if (a.D == 128 && a.short_kw == 8) return a.variant == 0 ? launch_short_dvk<128, 0, 8>(a, st) : launch_short_dvk<128, 1, 8>(a, st);
+    if (a.D == 128) return a.variant == 0 ? launch_short_dvk<128, 0, 4>(a, st) : launch_short_dvk<128, 1, 4>(a, st);
+    if (a.D == 64 && a.short_kw == 8) return a.variant == 0 ? launch_short_dvk<64, 0, 8>(a, st) : launch_short_dvk<64, 1, 8>(a, st);
+    if (a.D == 64) return a.variant == 0 ? launch_short_dvk<64, 0, 4>(a, st) : launch_short_dvk<64, 1, 4>(a, st);
+    return hipErrorInvalidValue;
+}
+
+static std::atomic<int> g_short_mode{0};       // 0: by shape; -1: never; 4, 8: always, that many key runs (4 at 256 channels)
+void attn_short_override(int mode) { g_short_mode.store(mode); }
+
+// Which form, from what either costs on an MI355X: time = base + rounds (r + s steps) + fill (f + g steps) in
+// microseconds, with rounds = workgroups / 256 rounded up, fill = workgroups / 256, steps = key tiles (main
+// kernel) or key steps of the longest run (short form).  The coefficients are least-squares fits to 300
+// launches per head dim and variant (4 to 60 heads, 32 to 2048 queries, 32 to 2048 keys), which they
+// meet within 4 to 11 %; picking the form by them came within 0.4 % of always picking the faster one.
+// Measured at [1,256,30,128] 16.7 -> 10.0 us, [1,1024,8,64] 20.2 -> 9.5, [1,1024,8,128] 28.0 -> 13.9,
+// [1,512,24,128] 21.3 -> 12.8; the main kernel's form is back ahead at about 100 workgroups of 256 rows with
+// 128 channels (twice that many with few keys).
+struct FormCost {
+    float base, r, s, f, g;
+    float of(int64_t wgs, int64_t steps) const {
+        const float rounds = (float)((wgs + 255) / 256), fill = (float)wgs / 256.0f, n = (float)steps;
+        return base + rounds * (r + s * n) + fill * (f + g * n);
+    }
+};
+static const FormCost kCost[3][2][3] = {        // [64, 128, 256 channels][variant][main, 4 runs, 8 runs]
+    {{{3.89f, 3.67f, 0.76f, 3.69f, 0.02f}, {5.20f, 1.27f, 0.53f, 1.01f, 0.10f}, {4.59f, 1.68f, 0.57f, 0.39f, 0.10f}},
+     {{3.52f, 4.41f, 0.91f, 3.03f, 0.00f}, {1.72f, 5.65f, 0.79f, 1.02f, 0.11f}, {2.30f, 5.33f, 0.31f, 0.23f, 0.41f}}},
+    {{{4.54f, 5.86f, 0.92f, 6.51f, 0.20f}, {2.76f, 5.78f, 0.77f, 1.97f, 0.52f}, {2.76f, 5.51f, 0.82f, 1.16f, 0.47f}},
+     {{6.95f, 5.91f, 1.08f, 8.20f, 0.00f}, {2.69f, 6.85f, 1.12f, 2.05f, 0.17f}, {2.52f, 6.99f, 0.66f, 1.02f, 0.52f}}},
+    {{{3.16f, 4.72f, 1.40f, 4.64f, 0.00f}, {2.15f, 5.54f, 1.26f, 1.78f, 0.27f}, {}},
+     {{3.08f, 8.00f, 1.09f, 4.97f, 0.00f}, {1.83f, 5.98f, 2.04f, 1.26f, 0.00f}, {}}},
+};
+
+int attn_short_rule(int B, int H, int Nq, int kv_valid, int D, int variant) {
+    const FormCost* c = kCost[D == 64 ? 0 : D == 128 ? 1 : 2][variant == 0 ? 0 : 1];
+    const int64_t bh = (int64_t)B * H;
+    const int64_t tiles = (kv_valid + kTileKV - 1) / kTileKV, steps = variant == 0 ? (kv_valid + 31) / 32 : tiles;
+    const int main_rows = D > 128 ? 128 : 256, rows4 = D > 128 ? 32 : 64;
+    const float t_main = c[0].of(bh * ((Nq + main_rows - 1) / main_rows), tiles);
+    const float t4 = c[1].of(bh * ((Nq + rows4 - 1) / rows4), (steps + 3) / 4);
+    if (D > 128) return t4 < t_main ? 4 : 0;
+    const float t8 = c[2].of(bh * ((Nq + 31) / 32), (steps + 7) / 8);
+    if (t4 < t8) return t4 < t_main ? 4 : 0;
+    return t8 < t_main ? 8 : 0;
+}
+
+int attn_short_runs(int B, int H, int Nq, int kv_valid, int D, int variant) {
+    const int mode = g_short_mode.load();
+    if (mode < 0) return 0;
+    if (mode > 0) return D == 256 ? 4 : mode;
+    if (attn_split_override_mode() != 0) return 0;      // a schedule of the 256-row workgroups was asked for
+    return attn_short_rule(B, H, Nq, kv_valid, D, variant);
+}
+
+}  // namespace sage

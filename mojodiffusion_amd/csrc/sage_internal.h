@@ -135,9 +135,17 @@ struct AttnArgs {
     int64_t qsb, qsh, qsn;
     const float* qmul;
     int split_wgs;           // workgroups of the split schedule (attn_split_workgroups), 0: one workgroup per item
+    int short_kw;            // key runs per row block in the short form (attn_short_runs), 0: the 256-row workgroups
     void* split;             // attn_split_bytes(split_wgs, D) bytes, 256-byte aligned (null when 0)
 };
 hipError_t launch_attn(const AttnArgs& a, hipStream_t st);
+// Shapes too small for 256-row workgroups: 32 or 64 rows per workgroup, keys split over its waves
+// (sage_attn_short.hip).  attn_short_rule: by shape alone, the number of key runs or 0;
+// attn_short_runs: the same, or what the test switch forces.  Takes precedence over the split schedule.
+hipError_t launch_attn_short(const AttnArgs& a, hipStream_t st);
+int attn_short_rule(int B, int H, int Nq, int kv_valid, int D, int variant);
+int attn_short_runs(int B, int H, int Nq, int kv_valid, int D, int variant);
+void attn_short_override(int mode);          // 0: by shape (default); -1: never; 4 or 8: always
 // Shapes whose items do not fill whole rounds of workgroups are spread evenly over a fixed number
 // of workgroups that hand partial results to each other through `split`.
 // attn_split_rule: the number of workgroups (a multiple of 8) the shape alone asks for, or 0 for one
@@ -150,6 +158,7 @@ size_t attn_split_bytes(int workgroups, int D);
 constexpr size_t kSplitFlagBytes = 4096;     // one int per workgroup in front of the state slots
 constexpr int kSplitMaxWorkgroups = 1024;
 void attn_split_override(int mode);          // 0: by shape and device (default); -1: never; n > 0 (multiple of 8): always n
+int attn_split_override_mode();
 void attn_split_wait(int polls);             // bound of the hand-over wait; 0: default; < 0: test mode (no flag is raised)
 int attn_split_faults(int reset);            // workgroups that gave up on the current device since the last reset; < 0: -hipError_t
 
