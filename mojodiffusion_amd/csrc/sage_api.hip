@@ -227,7 +227,7 @@ struct QuantOut {
     float *rowinv_q, *rowinv_k;       // whole-row RMSNorm statistics (only with that pre-op)
 };
 
-// K statistics + Q / K encoders (+ the V passes when vq is given): launches 1-3.
+// K statistics + Q / K encoders (+ the V passes when vq is given): launches 1-3, or one launch.
 int quantize(const View& q, const View& k, const View* v, int B, int H, int Nq, int Nkv, int D, float scale,
              int blkq, int blkk, int k_flags, const KeyMask& km, int kept, const QuantOut& o,
              int variant, void* vq, float* vscale, float* vpart, const Pre& pre_in, hipStream_t st) {
@@ -240,10 +240,32 @@ int quantize(const View& q, const View& k, const View* v, int B, int H, int Nq, 
     const float cmul = cmul_of(scale);
     const int64_t nqp = pad_to(Nq, kTileQ), nkp = pad_to(Nkv, kPadKV);
     const bool kstats = (k_flags & 3) != 0;
+    const bool v_fp8 = v != nullptr && variant != MI355_SAGE_PV_FP16;
+
+    FinalArgs f{};
+    f.total = (int64_t)B * H * D; f.D = D; f.ngroups = (Nkv + kGroup - 1) / kGroup; f.kept = kept;
+    f.flags = k_flags; f.cmul = cmul;
+    f.kpart_sum = kstats ? o.kpart_sum : nullptr; f.kpart_mm = o.kpart_mm;
+    f.kmean = o.kmean; f.qmul = o.qmul; f.kmul = o.kmul;
+    f.vpart = vpart; f.vscale = v_fp8 ? vscale : nullptr;
+
+    QuantArgs a{};
+    a.q = q; a.k = k; a.H = H; a.Nq = Nq; a.Nkv = Nkv; a.nq_pad = nqp; a.nkv_pad = nkp; a.km = km;
+    a.blkq = blkq; a.blkk = blkk; a.cmul = cmul;
+    a.kmean = o.kmean; a.qmul = o.qmul; a.kmul = o.kmul; a.vscale = vscale;
+    a.q8 = o.q8; a.qscale = o.qscale; a.rowdot = o.rowdot; a.k8 = o.k8; a.kscale = o.kscale;
+    if (v_fp8) { a.v = *v; a.v8 = static_cast<uint8_t*>(vq); }
+    else if (v != nullptr) { a.v = *v; a.v16 = static_cast<uint16_t*>(vq); }
+    a.pre_q = pre.q; a.pre_k = pre.k;
+    if (v != nullptr && quant_is_short(a, B, D)) {
+        SAGE_HIP(launch_quant_short(a, f, B, D, st));
+        return 0;
+    }
+
     PrepArgs p{};
     p.k = k; p.H = H; p.Nkv = Nkv; p.nkv_pad = nkp; p.km = km; p.pre_k = pre.k;
     p.vmode = 2;
-    if (v != nullptr && variant != MI355_SAGE_PV_FP16) {
+    if (v_fp8) {
         p.v = *v;
         p.vmode = 1;                       // (the fp16 repack needs no statistics: it goes with launch 3)
         p.vpart = vpart;
@@ -251,23 +273,7 @@ int quantize(const View& q, const View& k, const View* v, int B, int H, int Nq, 
     p.kpart_sum = kstats ? o.kpart_sum : nullptr;
     p.kpart_mm = o.kpart_mm;
     SAGE_HIP(launch_prep(p, B, D, st));
-
-    FinalArgs f{};
-    f.total = (int64_t)B * H * D; f.D = D; f.ngroups = (Nkv + kGroup - 1) / kGroup; f.kept = kept;
-    f.flags = k_flags; f.cmul = cmul;
-    f.kpart_sum = p.kpart_sum; f.kpart_mm = o.kpart_mm;
-    f.kmean = o.kmean; f.qmul = o.qmul; f.kmul = o.kmul;
-    f.vpart = vpart; f.vscale = p.vmode == 1 ? vscale : nullptr;
     SAGE_HIP(launch_stats_final(f, st));
-
-    QuantArgs a{};
-    a.q = q; a.k = k; a.H = H; a.Nq = Nq; a.Nkv = Nkv; a.nq_pad = nqp; a.nkv_pad = nkp; a.km = km;
-    a.blkq = blkq; a.blkk = blkk; a.cmul = cmul;
-    a.kmean = o.kmean; a.qmul = o.qmul; a.kmul = o.kmul; a.vscale = vscale;
-    a.q8 = o.q8; a.qscale = o.qscale; a.rowdot = o.rowdot; a.k8 = o.k8; a.kscale = o.kscale;
-    if (p.vmode == 1) { a.v = *v; a.v8 = static_cast<uint8_t*>(vq); }
-    else if (v != nullptr) { a.v = *v; a.v16 = static_cast<uint16_t*>(vq); }
-    a.pre_q = pre.q; a.pre_k = pre.k;
     SAGE_HIP(launch_quant(a, B, D, st));
     return 0;
 }

@@ -102,6 +102,10 @@ struct QuantArgs {
 };
 hipError_t launch_quant(const QuantArgs& a, int B, int D, hipStream_t st);
 
+// All of it as one launch, for short key sequences (K, V and, with q8, Q; the statistics also go to f's outputs).
+bool quant_is_short(const QuantArgs& a, int B, int D);
+hipError_t launch_quant_short(const QuantArgs& a, const FinalArgs& f, int B, int D, hipStream_t st);
+
 // ---- attention kernel (sage_attn.hip) --------------------------------------
 // rint(x / sc) for |x / sc| <= ~127 without paying a full IEEE divide per element: x * (1/sc)
 // is within 2^-15 of the correctly rounded quotient (both below 128), so whenever it lies at

@@ -1,4 +1,5 @@
-// sage_quant.hip — HBM-bound kernels of the quantized-SDPA path (gfx950), three launches:
+// sage_quant.hip — HBM-bound kernels of the quantized-SDPA path (gfx950), three launches (one for short
+// key sequences, quant_short_kernel):
 //
 //   prep_kernel         per (b,h), workgroup roles:  V repack to tiled fp16  |  V channel
 //                       maxima per 256-token group (e4m3 variant)  |  K channel sums (fp64),
@@ -170,7 +171,7 @@ __device__ __forceinline__ void pre_apply(const PreOp& p, int b, int h, int H, i
 }
 
 // ---------------------------------------------------------------------------
-// Per-block INT8 quantization.  One workgroup (256 threads) per block of BLK tokens of one
+// Per-block INT8 quantization.  NT threads (`tid` counts them) per block of BLK tokens of one
 // (b,h); the BLK x D tile lives in registers between the absmax pass and the encode pass, so
 // HBM sees one read of bf16 and one write of int8.
 // ---------------------------------------------------------------------------
@@ -179,7 +180,7 @@ __device__ __forceinline__ void pre_apply(const PreOp& p, int b, int h, int H, i
 // rowdot (Q only, may be null): <f32(q) * cmul, mean> per row.
 template <int D, int BLK, bool IS_K, bool PRE, int NT>
 __device__ __forceinline__ void quant_i8_block(
-    int t, int h, int b, const uint16_t* __restrict__ x, int64_t sb, int64_t sh, int64_t sn,
+    int t, int h, int b, int tid, const uint16_t* __restrict__ x, int64_t sb, int64_t sh, int64_t sn,
     int N, int H, int64_t n_pad, const KeyMask& km, const float* __restrict__ mean,
     const float* __restrict__ chmul, float cmul,
     int8_t* __restrict__ codes, float* __restrict__ scales, float* __restrict__ rowdot, float* red,
@@ -188,7 +189,6 @@ __device__ __forceinline__ void quant_i8_block(
     constexpr int NCH = BLK * CPR / NT;        // chunks per thread
     static_assert(BLK * CPR % NT == 0, "tile must split evenly over the threads");
     static_assert(NT % CPR == 0, "a thread keeps one column group for all its chunks");
-    const int tid = threadIdx.x;
     const int r0 = t * BLK;
     const int col = (tid % CPR) * 8;
     const int64_t bh = (int64_t)b * H + h;
@@ -336,11 +336,11 @@ struct KGroupSmem {
 
 // D is the number of channels this call covers, starting at channel col0 of a head of DFULL
 // channels (the statistics are per channel, so a 256-channel head is done as two windows of 128).
+// Result in gsum, gmn, gmx of the threads tid < D (channel col0 + tid).
 template <int D, bool PRE, int DFULL = D>
-__device__ __forceinline__ void kstats_group_body(
+__device__ __forceinline__ void kstats_group(
     int g, int h, int b, int tid, const uint16_t* __restrict__ k, int64_t sb, int64_t sh, int64_t sn,
-    int N, int H, int ngroups, const KeyMask& km, double* __restrict__ part_sum, float* __restrict__ part_mm,
-    KGroupSmem<D>& sm, const PreOp& pre, int col0 = 0) {
+    int N, int H, const KeyMask& km, KGroupSmem<D>& sm, const PreOp& pre, int col0, double& gsum, float& gmn, float& gmx) {
     static_assert(!PRE || DFULL == D, "the fused pre-ops need the whole row in one call");
     constexpr int CPR = D / 8;
     const int leaf = tid / CPR, col = (tid % CPR) * 8;
@@ -395,15 +395,27 @@ __device__ __forceinline__ void kstats_group_body(
         sm.leafmax[leaf][col + e] = mx[e];
     }
     __syncthreads();
+    gsum = 0.0;
+    gmn = INFINITY; gmx = -INFINITY;
     if (tid < D && g >= 0) {
-        double gsum = 0.0;
-        float gmn = INFINITY, gmx = -INFINITY;
 #pragma unroll
         for (int u = 0; u < 16; u++) {
             gsum += sm.leafsum[u][tid];
             gmn = fminf(gmn, sm.leafmin[u][tid]);
             gmx = fmaxf(gmx, sm.leafmax[u][tid]);
         }
+    }
+}
+
+template <int D, bool PRE, int DFULL = D>
+__device__ __forceinline__ void kstats_group_body(
+    int g, int h, int b, int tid, const uint16_t* __restrict__ k, int64_t sb, int64_t sh, int64_t sn,
+    int N, int H, int ngroups, const KeyMask& km, double* __restrict__ part_sum, float* __restrict__ part_mm,
+    KGroupSmem<D>& sm, const PreOp& pre, int col0 = 0) {
+    double gsum;
+    float gmn, gmx;
+    kstats_group<D, PRE, DFULL>(g, h, b, tid, k, sb, sh, sn, N, H, km, sm, pre, col0, gsum, gmn, gmx);
+    if (tid < D && g >= 0) {
         const int64_t o = (((int64_t)b * H + h) * ngroups + g) * DFULL + col0 + tid;
         part_sum[o] = gsum;
         part_mm[2 * o] = gmn;
@@ -432,10 +444,9 @@ __device__ __forceinline__ int v_tile_chunk(int slot, int chunk) {
 
 template <int D>
 __device__ __forceinline__ void quant_v_f16_body(
-    int t, int h, int b, const uint16_t* __restrict__ v, int64_t sb, int64_t sh, int64_t sn,
+    int t, int h, int b, int tid, const uint16_t* __restrict__ v, int64_t sb, int64_t sh, int64_t sn,
     int N, int H, int64_t n_pad, const KeyMask& km, uint16_t* __restrict__ out, uint16_t* tile) {
     constexpr int CPR = D / 8;
-    const int tid = threadIdx.x;
     const uint16_t* src = v + b * sb + h * sh;
     u32x4 raw[64 * CPR / 256];
 #pragma unroll
@@ -549,14 +560,13 @@ __device__ __forceinline__ uint32_t f32_to_e4m3(float x) {
 // of this can underflow, or with an all-ones significand, takes the plain formula.
 template <int D, int NT>
 __device__ __forceinline__ void quant_v_fp8_body(
-    int t, int h, int b, const uint16_t* __restrict__ v, int64_t sb, int64_t sh, int64_t sn,
+    int t, int h, int b, int tid, const uint16_t* __restrict__ v, int64_t sb, int64_t sh, int64_t sn,
     int N, int H, int64_t n_pad, const KeyMask& km, const float* __restrict__ vscale,
     uint8_t* __restrict__ out, uint8_t* tile) {
     constexpr int CPR = D / 8;
     constexpr int LD = D + 16;                             // padded row (bytes)
     constexpr int NCH = 64 * CPR / NT;
     static_assert(NT % CPR == 0, "a thread keeps one column group for all its chunks");
-    const int tid = threadIdx.x;
     const int64_t bh = (int64_t)b * H + h;
     const uint16_t* src = v + b * sb + h * sh;
     const int col = (tid % CPR) * 8;
@@ -568,7 +578,7 @@ __device__ __forceinline__ void quant_v_fp8_body(
         if (key_kept(row, N, km)) w[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)row * sn + col);
     }
     float sc[8], y[8];
-    load8(vscale + bh * D + col, sc);
+    load8(vscale + col, sc);
     bool plain = false;
 #pragma unroll
     for (int e = 0; e < 8; e++) {
@@ -647,7 +657,7 @@ __global__ __launch_bounds__(256) void prep_kernel(PrepArgs a) {
     const int b = bh / a.H, h = bh % a.H;
     if (r < a.nv_units) {
         if (a.vmode == 0)
-            quant_v_f16_body<D>(r, h, b, a.v.p, a.v.sb, a.v.sh, a.v.sn, a.Nkv, a.H, a.nkv_pad, a.km, a.v16, sm.tile);
+            quant_v_f16_body<D>(r, h, b, threadIdx.x, a.v.p, a.v.sb, a.v.sh, a.v.sn, a.Nkv, a.H, a.nkv_pad, a.km, a.v16, sm.tile);
         else
             v_absmax_group_body<D>(r, h, b, a.v.p, a.v.sb, a.v.sh, a.v.sn, a.Nkv, a.H, a.ngroups, a.km, a.vpart, sm.red);
     } else if constexpr (D > 128) {
@@ -737,6 +747,16 @@ hipError_t launch_prep(const PrepArgs& a_in, int B, int D, hipStream_t st) {
 //      kmul = 1/s, qmul = cmul*s.
 //   V: vscale = amax/448 (1 when 0).
 // ---------------------------------------------------------------------------
+__device__ __forceinline__ void k_final(double sum, float mn, float mx, int kept, int flags, float& mean, float& s) {
+    mean = 0.0f;
+    s = 1.0f;
+    if (flags & 1) mean = (float)(sum / (double)kept);
+    if (flags & 2) {
+        const float amax = fmaxf(fabsf(mx - mean), fabsf(mn - mean));
+        if (amax > 0.0f) s = sqrtf(amax);
+    }
+}
+
 __global__ __launch_bounds__(64) void stats_final_kernel(FinalArgs a) {
     const int64_t i = (int64_t)blockIdx.x * 64 + threadIdx.x;      // (bh, d)
     if (i >= a.total) return;
@@ -765,11 +785,7 @@ __global__ __launch_bounds__(64) void stats_final_kernel(FinalArgs a) {
                 for (int j = 0; j < NB; j++)
                     if (g0 + j < a.ngroups) { sum += v[j]; mn = fminf(mn, lo[j]); mx = fmaxf(mx, hi[j]); }
             }
-            if (a.flags & 1) mean = (float)(sum / (double)a.kept);
-            if (a.flags & 2) {
-                const float amax = fmaxf(fabsf(mx - mean), fabsf(mn - mean));
-                if (amax > 0.0f) s = sqrtf(amax);
-            }
+            k_final(sum, mn, mx, a.kept, a.flags, mean, s);
         }
         a.kmean[i] = mean;
         a.kmul[i] = 1.0f / s;
@@ -820,7 +836,7 @@ __global__ __launch_bounds__(256) void quant_kernel(QuantArgs a) {
     if (r < a.nq_blk) {
         const float* mul = a.qmul + (int64_t)bh * D;
         const float* mean = a.kmean + (int64_t)bh * D;
-#define SAGE_Q(BLK) quant_i8_block<D, BLK, false, PRE, NT>(r, h, b, a.q.p, a.q.sb, a.q.sh, a.q.sn, a.Nq, a.H, a.nq_pad, none, \
+#define SAGE_Q(BLK) quant_i8_block<D, BLK, false, PRE, NT>(r, h, b, threadIdx.x, a.q.p, a.q.sb, a.q.sh, a.q.sn, a.Nq, a.H, a.nq_pad, none, \
                                                        mean, mul, a.cmul, a.q8, a.qscale, a.rowdot, sm.red, a.pre_q)
         if (a.blkq == 128) SAGE_Q(128);
         else if (a.blkq == 64) SAGE_Q(64);
@@ -830,17 +846,17 @@ __global__ __launch_bounds__(256) void quant_kernel(QuantArgs a) {
         const int t = r - a.nq_blk;
         const float* mul = a.kmul + (int64_t)bh * D;
         const float* mean = a.kmean + (int64_t)bh * D;
-#define SAGE_K(BLK) quant_i8_block<D, BLK, true, PRE, NT>(t, h, b, a.k.p, a.k.sb, a.k.sh, a.k.sn, a.Nkv, a.H, a.nkv_pad, a.km, \
+#define SAGE_K(BLK) quant_i8_block<D, BLK, true, PRE, NT>(t, h, b, threadIdx.x, a.k.p, a.k.sb, a.k.sh, a.k.sn, a.Nkv, a.H, a.nkv_pad, a.km, \
                                                       mean, mul, 0.0f, a.k8, a.kscale, nullptr, sm.red, a.pre_k)
         if (a.blkk == 128) SAGE_K(128);
         else if (a.blkk == 64) SAGE_K(64);
         else SAGE_K(32);
 #undef SAGE_K
     } else if (a.v16 != nullptr) {
-        quant_v_f16_body<D>(r - a.nq_blk - a.nk_blk, h, b, a.v.p, a.v.sb, a.v.sh, a.v.sn, a.Nkv, a.H, a.nkv_pad, a.km, a.v16, sm.tile16);
+        quant_v_f16_body<D>(r - a.nq_blk - a.nk_blk, h, b, threadIdx.x, a.v.p, a.v.sb, a.v.sh, a.v.sn, a.Nkv, a.H, a.nkv_pad, a.km, a.v16, sm.tile16);
     } else {
-        quant_v_fp8_body<D, NT>(r - a.nq_blk - a.nk_blk, h, b, a.v.p, a.v.sb, a.v.sh, a.v.sn, a.Nkv, a.H, a.nkv_pad, a.km,
-                            a.vscale, a.v8, sm.tile8);
+        quant_v_fp8_body<D, NT>(r - a.nq_blk - a.nk_blk, h, b, threadIdx.x, a.v.p, a.v.sb, a.v.sh, a.v.sn, a.Nkv, a.H, a.nkv_pad, a.km,
+                            a.vscale + (int64_t)bh * D, a.v8, sm.tile8);
     }
 }
 
@@ -864,6 +880,172 @@ hipError_t launch_quant(const QuantArgs& a_in, int B, int D, hipStream_t st) {
     else if (D == 256 && !has_pre) SAGE_LAUNCH_QUANT(256, false);
     else return hipErrorInvalidValue;
 #undef SAGE_LAUNCH_QUANT
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// The three launches as one, for short key sequences.  A workgroup of the K and Q roles first computes its
+// head's K statistics by itself — the same leaves, groups and order, so the same bits — and then encodes
+// one block per half of its threads; a V workgroup takes the head's channel maxima (e4m3) the same way.
+// Every workgroup re-reads the head's K (or V) from L2, which is what a short sequence is for: three
+// dependent launches of 4 to 6 us each do almost nothing but start and drain there (see quant_is_short).
+// ---------------------------------------------------------------------------
+constexpr int kShortThreads = 512;
+
+template <int D, bool PRE>
+__global__ __launch_bounds__(kShortThreads) void quant_short_kernel(QuantArgs a, FinalArgs f) {
+    constexpr int DK = D > 128 ? 128 : D;                 // channels per K statistics call
+    constexpr int NWIN = D / DK;                          // windows of DK channels
+    constexpr int TPG = 16 * (DK / 8);                    // threads per K group
+    constexpr int GPW = kShortThreads / TPG;              // groups at a time
+    constexpr int VROWS = kShortThreads / (D / 8);
+    constexpr int UNITS = kShortThreads / 256;            // blocks or tiles per workgroup
+    union Smem {
+        KGroupSmem<DK> kg[GPW];
+        float vred[VROWS][D + 1];
+        float red[UNITS][4];
+        uint8_t tile8[UNITS][64 * (D + 16)];
+        uint16_t tile16[UNITS][64 * D];
+    };
+    __shared__ __attribute__((aligned(16))) Smem sm;
+    __shared__ __attribute__((aligned(16))) float s_mean[D], s_kmul[D], s_qmul[D];
+    __shared__ double s_gsum[GPW][DK];
+    __shared__ float s_gmm[GPW][DK][2];
+    const int bh = blockIdx.x % a.n_bh;
+    int r = blockIdx.x / a.n_bh;
+    const int b = bh / a.H, h = bh % a.H;
+    const int tid = threadIdx.x, unit = tid >> 8, utid = tid & 255;
+    const KeyMask none{0, 0};
+    const int nk_wg = (a.nk_blk + UNITS - 1) / UNITS, nq_wg = (a.nq_blk + UNITS - 1) / UNITS;
+    if (r < nk_wg + nq_wg) {
+        const int sub = tid / TPG, t = tid % TPG;
+#pragma unroll
+        for (int w = 0; w < NWIN; w++) {
+            double sum = 0.0;
+            float mn = INFINITY, mx = -INFINITY;
+            if (f.flags & 3) {
+                for (int g0 = 0; g0 < f.ngroups; g0 += GPW) {
+                    double gsum;
+                    float gmn, gmx;
+                    const int g = g0 + sub;
+                    kstats_group<DK, PRE, D>(g < f.ngroups ? g : -1, h, b, t, a.k.p, a.k.sb, a.k.sh, a.k.sn, a.Nkv, a.H, a.km,
+                                             sm.kg[sub], a.pre_k, w * DK, gsum, gmn, gmx);
+                    if (t < DK) { s_gsum[sub][t] = gsum; s_gmm[sub][t][0] = gmn; s_gmm[sub][t][1] = gmx; }
+                    __syncthreads();
+                    if (tid < DK) {
+#pragma unroll
+                        for (int u = 0; u < GPW; u++)
+                            if (g0 + u < f.ngroups) {
+                                sum += s_gsum[u][tid];
+                                mn = fminf(mn, s_gmm[u][tid][0]);
+                                mx = fmaxf(mx, s_gmm[u][tid][1]);
+                            }
+                    }
+                    __syncthreads();
+                }
+            }
+            if (tid < DK) {
+                float mean, s;
+                k_final(sum, mn, mx, f.kept, f.flags, mean, s);
+                const int d = w * DK + tid;
+                const float kmul = 1.0f / s, qmul = f.cmul * s;
+                s_mean[d] = mean; s_kmul[d] = kmul; s_qmul[d] = qmul;
+                if (r == 0) {
+                    const int64_t i = (int64_t)bh * D + d;
+                    f.kmean[i] = mean; f.kmul[i] = kmul; f.qmul[i] = qmul;
+                }
+            }
+        }
+        __syncthreads();
+        // (an odd count: the last workgroup's halves encode the same block)
+        if (r < nk_wg) {
+            const int blk = min(r * UNITS + unit, a.nk_blk - 1);
+#define SAGE_K(BLK) quant_i8_block<D, BLK, true, PRE, 256>(blk, h, b, utid, a.k.p, a.k.sb, a.k.sh, a.k.sn, a.Nkv, a.H, a.nkv_pad, a.km, \
+                                                       s_mean, s_kmul, 0.0f, a.k8, a.kscale, nullptr, sm.red[unit], a.pre_k)
+            if (a.blkk == 128) SAGE_K(128);
+            else if (a.blkk == 64) SAGE_K(64);
+            else SAGE_K(32);
+#undef SAGE_K
+        } else {
+            const int blk = min((r - nk_wg) * UNITS + unit, a.nq_blk - 1);
+#define SAGE_Q(BLK) quant_i8_block<D, BLK, false, PRE, 256>(blk, h, b, utid, a.q.p, a.q.sb, a.q.sh, a.q.sn, a.Nq, a.H, a.nq_pad, none, \
+                                                        s_mean, s_qmul, a.cmul, a.q8, a.qscale, a.rowdot, sm.red[unit], a.pre_q)
+            if (a.blkq == 128) SAGE_Q(128);
+            else if (a.blkq == 64) SAGE_Q(64);
+            else SAGE_Q(32);
+#undef SAGE_Q
+        }
+        return;
+    }
+    const int t = (r - nk_wg - nq_wg) * UNITS + unit;     // (the key padding makes the tile count even)
+    if (a.v16 != nullptr) {
+        quant_v_f16_body<D>(t, h, b, utid, a.v.p, a.v.sb, a.v.sh, a.v.sn, a.Nkv, a.H, a.nkv_pad, a.km, a.v16, sm.tile16[unit]);
+        return;
+    }
+    {
+        constexpr int CPR = D / 8;
+        const int col = (tid % CPR) * 8, row0 = tid / CPR;
+        const uint16_t* src = a.v.p + b * a.v.sb + h * a.v.sh + col;
+        float m[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll 8
+        for (int row = row0; row < a.Nkv; row += VROWS) {
+            u32x4 w = {0u, 0u, 0u, 0u};
+            if (key_kept(row, a.Nkv, a.km)) w = *reinterpret_cast<const u32x4*>(src + (int64_t)row * a.v.sn);
+            float x[8];
+            unpack8(w, x);
+#pragma unroll
+            for (int e = 0; e < 8; e++) m[e] = fmaxf(m[e], fabsf(x[e]));
+        }
+#pragma unroll
+        for (int e = 0; e < 8; e++) sm.vred[row0][col + e] = m[e];
+        __syncthreads();
+        if (tid < D) {
+            float amax = 0.0f;
+            for (int i = 0; i < VROWS; i++) amax = fmaxf(amax, sm.vred[i][tid]);
+            const float sc = amax > 0.0f ? amax / 448.0f : 1.0f;
+            s_mean[tid] = sc;
+            if (r == nk_wg + nq_wg) f.vscale[(int64_t)bh * D + tid] = sc;
+        }
+        __syncthreads();
+    }
+    quant_v_fp8_body<D, 256>(t, h, b, utid, a.v.p, a.v.sb, a.v.sh, a.v.sn, a.Nkv, a.H, a.nkv_pad, a.km, s_mean, a.v8, sm.tile8[unit]);
+}
+
+static void short_units(QuantArgs& a, int B) {
+    a.nq_blk = a.q8 != nullptr ? (int)(a.nq_pad / a.blkq) : 0;
+    a.nk_blk = (int)(a.nkv_pad / a.blkk);
+    a.nv_tile = (int)(a.nkv_pad / 64);
+    a.n_bh = B * a.H;
+}
+static int64_t short_workgroups(const QuantArgs& a) { return (int64_t)a.n_bh * ((a.nq_blk + 1) / 2 + (a.nk_blk + 1) / 2 + a.nv_tile / 2); }
+
+// One launch where a workgroup gets through its head's statistics in one pass (1024 keys at 64 channels, 512
+// at 128; at 256 channels, where they take two windows, 256) and all workgroups are resident at once (two
+// per compute unit).  Measured over 4 to 60 heads, stage of three launches -> one, us: 11.5-15 -> 7.5-9.5 up
+// to 256 keys, 13-15 -> 9-12.8 at 512 keys of 128 channels, 12-13.4 -> 8.4-10.7 at 1024 keys of 64; a second
+// pass costs 4 us and a second generation of workgroups 7, which is what the two launches less are worth.
+bool quant_is_short(const QuantArgs& a_in, int B, int D) {
+    QuantArgs a = a_in;
+    short_units(a, B);
+    const int groups = (a.Nkv + kGroup - 1) / kGroup;
+    return groups <= (D == 64 ? 4 : D == 128 ? 2 : 1) && short_workgroups(a) <= 512;
+}
+
+hipError_t launch_quant_short(const QuantArgs& a_in, const FinalArgs& f_in, int B, int D, hipStream_t st) {
+    QuantArgs a = a_in;
+    short_units(a, B);
+    if ((a.q8 != nullptr && a.nq_pad % a.blkq != 0) || a.nkv_pad % a.blkk != 0 || a.k8 == nullptr || (a.v8 == nullptr && a.v16 == nullptr))
+        return hipErrorInvalidValue;
+    const int64_t total = short_workgroups(a);
+    if (total <= 0 || total > 0x7FFFFFFF || (a.nv_tile & 1)) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)total), block(kShortThreads);
+    const bool has_pre = a.pre_q.gain != nullptr;
+    if (D == 128 && has_pre) hipLaunchKernelGGL((quant_short_kernel<128, true>), grid, block, 0, st, a, f_in);
+    else if (D == 128) hipLaunchKernelGGL((quant_short_kernel<128, false>), grid, block, 0, st, a, f_in);
+    else if (D == 64 && has_pre) hipLaunchKernelGGL((quant_short_kernel<64, true>), grid, block, 0, st, a, f_in);
+    else if (D == 64) hipLaunchKernelGGL((quant_short_kernel<64, false>), grid, block, 0, st, a, f_in);
+    else if (D == 256 && !has_pre) hipLaunchKernelGGL((quant_short_kernel<256, false>), grid, block, 0, st, a, f_in);
+    else return hipErrorInvalidValue;
     return hipGetLastError();
 }
 
