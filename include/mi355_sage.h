@@ -204,6 +204,20 @@ int mi355_sage_sdpa_bf16_mask(
     void* stream,
     int variant, void* workspace, size_t workspace_bytes);
 
+/* The same for a bias whose rows start anywhere (a contiguous [B,H,N_q,N_kv] tensor of odd N_kv, which the
+ * reference's masked kernels index element by element, serenitymojo/ops/attention.mojo:744-801): key stride
+ * 1, no alignment beyond bf16's own. */
+int mi355_sage_sdpa_bf16_mask_any(
+    const void* Q, const void* K, const void* V, const void* Mask, void* O,
+    int B, int H, int N_q, int N_kv, int D,
+    float scale,
+    const int64_t* q_strides, const int64_t* k_strides,
+    const int64_t* v_strides, const int64_t* mask_strides, const int64_t* o_strides,
+    int64_t q_offset_elems, int64_t k_offset_elems,
+    int64_t v_offset_elems, int64_t mask_offset_elems, int64_t o_offset_elems,
+    void* stream,
+    int variant, void* workspace, size_t workspace_bytes);
+
 /* mi355_sage_sdpa_bf16_train_fwd on the pre-norm projections (default recipe: Q blocks of 128
  * tokens, 32 for the e4m3 variant; K blocks of 64; K smoothing and balancing on), for the blocks that run
  * rms_norm / rope_interleaved in front of sdpa_flash_train_fwd
@@ -407,6 +421,11 @@ int mi355_sage_sdpa_bwd_bf16(
     int64_t dk_offset_elems, int64_t dv_offset_elems,
     int causal, int real_N_q, int real_N_kv, void* stream,
     void* workspace, size_t workspace_bytes);
+
+/* F32 <-> bf16 (round to nearest even) of `count` tensors (1 to 4) in one launch: the casts at the boundary of
+ * callers with F32 activations (serenitymojo/ops/attention_flash.mojo:457-475, :478-535).  n: elements;
+ * to_bf16 != 0: src F32, dst bf16, else the other way; bases 16-byte aligned. */
+int mi355_sage_cast(int count, const void* const* src, void* const* dst, const int64_t* n, int to_bf16, void* stream);
 
 /* Library identification: "mi355_sage <version> gfx950". */
 const char* mi355_sage_version(void);

@@ -1,10 +1,13 @@
-"""ctypes loader for libmi355_sage.so.  There is no fallback: if the library is
+"""ctypes loader for libmi355_sage.so and loader of the native host path _sage_host.so.  There is no fallback: if the library is
 missing, every attention call fails with an error that says how to build it."""
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libmi355_sage.so")
+HOST_PATH = os.path.join(_HERE, "lib", "_sage_host.so")
 
 _i64p = ctypes.POINTER(ctypes.c_int64)
 _vp = ctypes.c_void_p
@@ -26,6 +29,9 @@ SIGNATURES = {
                                      + [_int, _int, _vp, _int, _vp, ctypes.c_size_t]),
     "mi355_sage_sdpa_bf16_mask": (_int, [_vp] * 5 + [_int] * 5 + [ctypes.c_float] + [_i64p] * 5 + [_i64] * 5
                                   + [_vp, _int, _vp, ctypes.c_size_t]),
+    "mi355_sage_sdpa_bf16_mask_any": (_int, [_vp] * 5 + [_int] * 5 + [ctypes.c_float] + [_i64p] * 5 + [_i64] * 5
+                                      + [_vp, _int, _vp, ctypes.c_size_t]),
+    "mi355_sage_cast": (_int, [_int, ctypes.POINTER(_vp), ctypes.POINTER(_vp), _i64p, _int, _vp]),
     "mi355_sage_workspace_bytes": (ctypes.c_size_t, [_int] * 6),
     "mi355_sage_bwd_workspace_bytes": (ctypes.c_size_t, [_int] * 5),
     "mi355_sage_sdpa_bwd_bf16": (_int, [_vp] * 9 + [_int] * 5 + [ctypes.c_float] + [_i64p] * 8 + [_i64] * 9
@@ -69,7 +75,29 @@ ROPE_HALFSPLIT = 1
 ROPE_TABLES_BF16 = 2
 NORM_FULL_ROW = 4
 
+# entry points the native host path calls, in the order of its Api struct (csrc/sage_torch.cpp)
+_HOST_ENTRIES = ("workspace_bytes", "bwd_workspace_bytes", "sdpa_bf16", "sdpa_bf16_train_fwd", "sdpa_bf16_keymask", "sdpa_bf16_mask_any",
+                 "sdpa_bf16_norm_rope", "sdpa_bf16_norm_rope_train_fwd", "sdpa_bwd_bf16", "cast")
+
 _lib = None
+_host = None
+
+
+def host():
+    """The native host path (CPython extension): the common calls without the interpreter in between."""
+    global _host
+    if _host is None:
+        L = lib()
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError(
+                "_sage_host.so is not built (%s). Build it with `make -C mojodiffusion_amd/csrc` "
+                "or `python -c 'import __graft_entry__ as g; g.build()'`; there is no fallback path." % HOST_PATH)
+        loader = importlib.machinery.ExtensionFileLoader("_sage_host", HOST_PATH)
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_sage_host", loader))
+        loader.exec_module(mod)
+        mod.bind(*(ctypes.cast(getattr(L, "mi355_sage_" + n), ctypes.c_void_p).value for n in _HOST_ENTRIES))
+        _host = mod
+    return _host
 
 
 def lib():

@@ -40,21 +40,15 @@ class SdpaFlashFwd:
     stats: torch.Tensor
 
 
-_workspaces = {}
+# Calls that meet every check go through the native host path (_lib.host(), csrc/sage_torch.cpp), which returns
+# None for the others; those continue in the functions below, which state the checks and raise.
+_PLAIN, _TRAIN, _KEYMASK = 0, 1, 2
 
 
-def _workspace(nbytes, device):
-    """Caller-side workspace reuse: one growing buffer per (device, stream), so steady-state
-    calls allocate nothing and calls on different streams never share scratch memory.  A
-    buffer that is replaced stays alive for the work already queued on its stream: torch's
-    allocator hands its memory out again only to that same stream."""
-    stream = torch.cuda.current_stream(device)
-    key = (device.type, device.index, stream.cuda_stream)
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
-        _workspaces[key] = ws
-    return ws
+def _workspace(nbytes, t):
+    """The reusable buffer of t's device and the current stream: grows, never shrinks, shared with the
+    native host path."""
+    return _lib.host().workspace(nbytes, t)
 
 
 def _require_bf16(name, *ts):
@@ -78,7 +72,7 @@ def _call_train_fwd(name, q, k, v, scale, real_q, real_kv, variant, want_stats, 
     o = torch.empty_like(q)
     stats = torch.empty((B, H, Sq, 1), dtype=torch.float32, device=q.device) if want_stats else None
     nbytes = L.mi355_sage_workspace_bytes(B, H, Sq, Skv, Dh, variant)
-    ws = _workspace(max(nbytes, 256), q.device)
+    ws = _workspace(max(nbytes, 256), q)
     qs = _lib.strides_bhnd(Sq, H, Dh)
     ks = _lib.strides_bhnd(Skv, H, Dh)
     stream = torch.cuda.current_stream(q.device).cuda_stream
@@ -116,6 +110,9 @@ def _check_shapes(name, q, k, v, square):
 def sdpa_flash_train_fwd(q, k, v, scale, variant=PV_FP16):
     """Forward on [B,S,H,Dh] BF16 (no mask, non-causal); returns O and the
     log-sum-exp Stats [B,H,S,1].  Fails loudly on any non-zero return code."""
+    r = _lib.host().fwd(q, k, v, scale, variant, _TRAIN, 0, 0, 1)
+    if r is not None:
+        return SdpaFlashFwd(r[0], r[0], q, k, v, r[1])
     _require_bf16("sdpa_flash_train_fwd", q, k, v)
     _check_shapes("sdpa_flash_train_fwd", q, k, v, True)
     _require_cuda("sdpa_flash_train_fwd", q, k, v)
@@ -125,11 +122,27 @@ def sdpa_flash_train_fwd(q, k, v, scale, variant=PV_FP16):
 
 def sdpa_flash_train_fwd_rect(q, k, v, scale, variant=PV_FP16):
     """Rectangular no-mask attention: q [B,Sq,H,Dh], k/v [B,Skv,H,Dh]."""
+    r = _lib.host().fwd(q, k, v, scale, variant, _TRAIN, 0, 0, 0)
+    if r is not None:
+        return SdpaFlashFwd(r[0], r[0], q, k, v, r[1])
     _require_bf16("sdpa_flash_train_fwd_rect", q, k, v)
     _check_shapes("sdpa_flash_train_fwd_rect", q, k, v, False)
     _require_cuda("sdpa_flash_train_fwd_rect", q, k, v)
     o, stats = _call_train_fwd("sdpa_flash_train_fwd_rect", q, k, v, scale, q.shape[1], k.shape[1], variant, True)
     return SdpaFlashFwd(o, o, q, k, v, stats)
+
+
+def sdpa_flash_fwd_o(q, k, v, scale, variant=PV_FP16, rect=False):
+    """O of sdpa_flash_train_fwd (rect: _rect) for callers that do not keep the Stats: the same bits, and
+    the attention kernel then encodes Q itself."""
+    o = _lib.host().fwd(q, k, v, scale, variant, _PLAIN, 0, 0, 0 if rect else 1) if q.dtype == torch.bfloat16 else None
+    if o is not None:
+        return o
+    name = "sdpa_flash_train_fwd_rect" if rect else "sdpa_flash_train_fwd"
+    _require_bf16(name, q, k, v)
+    _check_shapes(name, q, k, v, not rect)
+    _require_cuda(name, q, k, v)
+    return _call_train_fwd(name, q, k, v, scale, q.shape[1], k.shape[1], variant, False)[0]
 
 
 def sdpa_flash_fwd_padmask(q, k, v, real_len, scale, variant=PV_FP16):
@@ -143,6 +156,9 @@ def sdpa_flash_fwd_padmask(q, k, v, real_len, scale, variant=PV_FP16):
         raise Error("sdpa_flash_fwd_padmask: S_BUF must be 128-aligned")
     if real_len < 1 or real_len > s_buf:
         raise Error("sdpa_flash_fwd_padmask: real_len out of [1, S_BUF]")
+    r = _lib.host().fwd(q, k, v, scale, variant, _TRAIN, 0, real_len, 1)
+    if r is not None:
+        return SdpaFlashFwd(r[0], r[0], q, k, v, r[1])
     _require_cuda("sdpa_flash_fwd_padmask", q, k, v)
     o, stats = _call_train_fwd("sdpa_flash_fwd_padmask", q, k, v, scale, real_len, real_len, variant, True)
     return SdpaFlashFwd(o, o, q, k, v, stats)
@@ -164,11 +180,14 @@ class SdpaFlashGrads:
 
 
 def _call_bwd(name, q, k, v, o, d_out, stats, scale, real_q, real_kv):
+    r = _lib.host().bwd(q, k, v, o, d_out, stats, scale, real_q, real_kv)
+    if r is not None:
+        return SdpaFlashGrads(*r)
     B, Sq, H, Dh = q.shape
     Skv = k.shape[1]
     L = _lib.lib()
     d_q, d_k, d_v = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    ws = _workspace(max(L.mi355_sage_bwd_workspace_bytes(B, H, Sq, Skv, Dh), 256), q.device)
+    ws = _workspace(max(L.mi355_sage_bwd_workspace_bytes(B, H, Sq, Skv, Dh), 256), q)
     qs = _lib.strides_bhnd(Sq, H, Dh)
     ks = _lib.strides_bhnd(Skv, H, Dh)
     stream = torch.cuda.current_stream(q.device).cuda_stream
@@ -485,6 +504,9 @@ def record_sdpa(q, k, v, scale, variant=PV_FP16):
     """att = sdpa_nomask(q, k, v, scale) recorded for backpropagation
     (serenitymojo/autograd_v2/ops_record.mojo:329-352): the result carries a node whose backward
     yields d_q, d_k, d_v.  torch's autograd graph stands in for the reference's `Graph`."""
+    att = _lib.host().record(q, k, v, scale, variant)
+    if att is not None:
+        return att
     return _SdpaNode.apply(q, k, v, scale, variant)
 
 
@@ -493,6 +515,9 @@ def sdpa_nomask(q, k, v, scale, variant=PV_FP16):
     every DiT sampler uses.  Output has q's dtype; F32/F16 storage is cast to
     BF16 at the boundary as the reference's per-model dispatchers do
     (models/zimage/lora_block.mojo:99-123)."""
+    o = _lib.host().fwd(q, k, v, scale, variant, _PLAIN, 0, 0, 1)
+    if o is not None:
+        return o
     if q.dtype != k.dtype or q.dtype != v.dtype:
         raise Error("sdpa_nomask: q/k/v dtype mismatch")
     _check_shapes("sdpa_nomask", q, k, v, True)
@@ -506,6 +531,10 @@ def sdpa_nomask(q, k, v, scale, variant=PV_FP16):
 
 
 def _nomask(name, q, k, v, scale, variant, square, mask=None):
+    lo, hi = mask if mask is not None else (0, 0)
+    o = _lib.host().fwd(q, k, v, scale, variant, _PLAIN if mask is None else _KEYMASK, lo, hi, 1 if square else 0)
+    if o is not None:
+        return o
     if q.dtype != k.dtype or q.dtype != v.dtype:
         raise Error("%s: q/k/v dtype mismatch" % name)
     _check_shapes(name, q, k, v, square)
@@ -542,6 +571,9 @@ def sdpa_qwen_keymask(q, k, v, n_txt, real_txt_len, scale, variant=PV_FP16):
 
 def sdpa_cross_nomask(q, k, v, scale, variant=PV_FP16):
     """attention.mojo:1860-1894: rectangular Sq != Skv, no mask."""
+    o = _lib.host().fwd(q, k, v, scale, variant, _PLAIN, 0, 0, 0)
+    if o is not None:
+        return o
     if q.dtype != k.dtype or q.dtype != v.dtype:
         raise Error("sdpa_cross_nomask: q/k/v dtype mismatch")
     _check_shapes("sdpa_cross_nomask", q, k, v, False)
@@ -554,6 +586,9 @@ def sdpa_cross_nomask(q, k, v, scale, variant=PV_FP16):
 
 
 def _masked(name, q, k, v, mask, scale, variant, square):
+    o = _lib.host().bias(q, k, v, mask, scale, variant, 1 if square else 0)
+    if o is not None:
+        return o
     if q.dtype != k.dtype or q.dtype != v.dtype:
         raise Error("%s: q/k/v dtype mismatch" % name)
     if q.dtype != mask.dtype:
@@ -571,20 +606,16 @@ def _masked(name, q, k, v, mask, scale, variant, square):
     out_dtype = q.dtype
     if q.dtype != torch.bfloat16:
         q, k, v, mask = (t.to(torch.bfloat16) for t in (q, k, v, mask))
-    if mask.stride(3) != 1 or any(st % 4 for st in mask.stride()[:3]):
+    if mask.stride(3) != 1:
         mask = mask.contiguous()
-        if Skv % 4:                                   # rows of the bias must start 8-byte aligned
-            padded = torch.zeros((B, H, Sq, (Skv + 3) // 4 * 4), dtype=mask.dtype, device=mask.device)
-            padded[..., :Skv] = mask
-            mask = padded
     L = _lib.lib()
     o = torch.empty_like(q)
-    ws = _workspace(max(L.mi355_sage_workspace_bytes(B, H, Sq, Skv, Dh, variant), 256), q.device)
+    ws = _workspace(max(L.mi355_sage_workspace_bytes(B, H, Sq, Skv, Dh, variant), 256), q)
     qs, ks = _lib.strides_bhnd(Sq, H, Dh), _lib.strides_bhnd(Skv, H, Dh)
     ms = (_lib.ctypes.c_int64 * 4)(*mask.stride())
-    rc = L.mi355_sage_sdpa_bf16_mask(q.data_ptr(), k.data_ptr(), v.data_ptr(), mask.data_ptr(), o.data_ptr(),
-                                     B, H, Sq, Skv, Dh, float(scale), qs, ks, ks, ms, qs, 0, 0, 0, 0, 0,
-                                     torch.cuda.current_stream(q.device).cuda_stream, variant, ws.data_ptr(), ws.numel())
+    rc = L.mi355_sage_sdpa_bf16_mask_any(q.data_ptr(), k.data_ptr(), v.data_ptr(), mask.data_ptr(), o.data_ptr(),
+                                         B, H, Sq, Skv, Dh, float(scale), qs, ks, ks, ms, qs, 0, 0, 0, 0, 0,
+                                         torch.cuda.current_stream(q.device).cuda_stream, variant, ws.data_ptr(), ws.numel())
     if rc != 0:
         raise Error("%s: shim rc=%d (B=%d Sq=%d Skv=%d H=%d Dh=%d)" % (name, rc, B, Sq, Skv, H, Dh))
     return o.to(out_dtype)
@@ -719,15 +750,19 @@ def qk_norm_rope_sdpa_nomask(q_pre, k_pre, v, q_norm, k_norm, eps, cos, sin, sca
     whole inner dim, q_norm/k_norm are [H*Dh] (rms_norm on [S, H*Dh] before the reshape to heads,
     models/ltx2/ltx2_block.mojo:419-432, whose tables are BF16 — also accepted)."""
     name = "qk_norm_rope_sdpa_nomask"
+    if blkq is None:
+        blkq = 32 if variant == PV_FP8 else 128
+    layout = (_lib.ROPE_HALFSPLIT if halfsplit else 0) | (_lib.NORM_FULL_ROW if full_row else 0)
+    o = _lib.host().norm_rope(q_pre, k_pre, v, q_norm, k_norm, eps, cos, sin, scale, variant, blkq, blkk, k_flags, layout, 0)
+    if o is not None:
+        return o
     gq, gk, cos, sin, batch_rows, flags = _norm_rope_args(name, q_pre, k_pre, v, q_norm, k_norm, cos, sin, halfsplit, full_row)
     B, S, H, Dh = q_pre.shape
     L = _lib.lib()
     o = torch.empty_like(q_pre)
     nbytes = L.mi355_sage_workspace_bytes(B, H, S, S, Dh, variant)
-    ws = _workspace(max(nbytes, 256), q_pre.device)
+    ws = _workspace(max(nbytes, 256), q_pre)
     st = _lib.strides_bhnd(S, H, Dh)
-    if blkq is None:
-        blkq = 32 if variant == PV_FP8 else 128
     rc = L.mi355_sage_sdpa_bf16_norm_rope(
         q_pre.data_ptr(), k_pre.data_ptr(), v.data_ptr(), o.data_ptr(), B, H, S, S, Dh, float(scale),
         st, st, st, st, 0, 0, 0, 0, 0, torch.cuda.current_stream(q_pre.device).cuda_stream,
@@ -746,13 +781,17 @@ def qk_norm_rope_sdpa_flash_train_fwd(q_pre, k_pre, v, q_norm, k_norm, eps, cos,
     (serenitymojo/ops/attention_flash.mojo:149-202).  Returns an SdpaFlashFwd whose stats are the
     log-sum-exp of the normalised, rotated Q and K."""
     name = "qk_norm_rope_sdpa_flash_train_fwd"
+    layout = (_lib.ROPE_HALFSPLIT if halfsplit else 0) | (_lib.NORM_FULL_ROW if full_row else 0)
+    r = _lib.host().norm_rope(q_pre, k_pre, v, q_norm, k_norm, eps, cos, sin, scale, variant, 0, 0, 0, layout, 1)
+    if r is not None:
+        return SdpaFlashFwd(r[0], r[0], q_pre, k_pre, v, r[1])
     gq, gk, cos, sin, batch_rows, flags = _norm_rope_args(name, q_pre, k_pre, v, q_norm, k_norm, cos, sin, halfsplit, full_row)
     B, S, H, Dh = q_pre.shape
     L = _lib.lib()
     o = torch.empty_like(q_pre)
     stats = torch.empty((B, H, S, 1), dtype=torch.float32, device=q_pre.device)
     nbytes = L.mi355_sage_workspace_bytes(B, H, S, S, Dh, variant)
-    ws = _workspace(max(nbytes, 256), q_pre.device)
+    ws = _workspace(max(nbytes, 256), q_pre)
     st = _lib.strides_bhnd(S, H, Dh)
     rc = L.mi355_sage_sdpa_bf16_norm_rope_train_fwd(
         q_pre.data_ptr(), k_pre.data_ptr(), v.data_ptr(), o.data_ptr(), stats.data_ptr(), B, H, S, S, Dh, float(scale),

@@ -283,6 +283,7 @@ struct MaskArgs {
     const void* add = nullptr;         // additive bias, bf16, logical [B,H,N_q,N_kv]
     const int64_t* add_strides = nullptr;
     int64_t add_off = 0;
+    bool any_row_start = false;        // rows of the bias may start at any even byte address
 };
 
 int sdpa_impl(const void* Q, const void* K, const void* V, void* O, void* Stats,
@@ -314,7 +315,7 @@ int sdpa_impl(const void* Q, const void* K, const void* V, void* O, void* Stats,
         const int64_t* ms = mask.add_strides;
         if (!ms) return MI355_SAGE_EINVAL;
         const uintptr_t a = reinterpret_cast<uintptr_t>(mask.add) + (uintptr_t)(mask.add_off * 2);
-        if (ms[3] != 1 || (a & 7) || (ms[0] & 3) || (ms[1] & 3) || (ms[2] & 3)) {
+        if (ms[3] != 1 || (!mask.any_row_start && ((a & 7) || (ms[0] & 3) || (ms[1] & 3) || (ms[2] & 3)))) {
             SAGE_LOG("mask: key stride must be 1 and every row 8-byte aligned");
             return MI355_SAGE_EUNSUPPORTED;
         }
@@ -508,18 +509,38 @@ int mi355_sage_sdpa_bf16_keymask(const void* Q, const void* K, const void* V, vo
                      default_blkq(variant), 64, kDefaultFlags, workspace, workspace_bytes, Pre{}, m);
 }
 
+static int sdpa_mask_entry(const void* Q, const void* K, const void* V, const void* Mask, void* O,
+                           int B, int H, int N_q, int N_kv, int D, float scale,
+                           const int64_t* q_strides, const int64_t* k_strides,
+                           const int64_t* v_strides, const int64_t* mask_strides, const int64_t* o_strides,
+                           int64_t q_off, int64_t k_off, int64_t v_off, int64_t mask_off, int64_t o_off,
+                           void* stream, int variant, void* workspace, size_t workspace_bytes, bool any_row_start) {
+    if (!Mask || !mask_strides) return MI355_SAGE_EINVAL;
+    MaskArgs m;
+    m.add = Mask; m.add_strides = mask_strides; m.add_off = mask_off; m.any_row_start = any_row_start;
+    return sdpa_impl(Q, K, V, O, nullptr, B, H, N_q, N_kv, D, scale, q_strides, k_strides, v_strides,
+                     o_strides, q_off, k_off, v_off, o_off, 0, 0, 0, stream, variant,
+                     default_blkq(variant), 64, kDefaultFlags, workspace, workspace_bytes, Pre{}, m);
+}
+
 int mi355_sage_sdpa_bf16_mask(const void* Q, const void* K, const void* V, const void* Mask, void* O,
                               int B, int H, int N_q, int N_kv, int D, float scale,
                               const int64_t* q_strides, const int64_t* k_strides,
                               const int64_t* v_strides, const int64_t* mask_strides, const int64_t* o_strides,
                               int64_t q_off, int64_t k_off, int64_t v_off, int64_t mask_off, int64_t o_off,
                               void* stream, int variant, void* workspace, size_t workspace_bytes) {
-    if (!Mask || !mask_strides) return MI355_SAGE_EINVAL;
-    MaskArgs m;
-    m.add = Mask; m.add_strides = mask_strides; m.add_off = mask_off;
-    return sdpa_impl(Q, K, V, O, nullptr, B, H, N_q, N_kv, D, scale, q_strides, k_strides, v_strides,
-                     o_strides, q_off, k_off, v_off, o_off, 0, 0, 0, stream, variant,
-                     default_blkq(variant), 64, kDefaultFlags, workspace, workspace_bytes, Pre{}, m);
+    return sdpa_mask_entry(Q, K, V, Mask, O, B, H, N_q, N_kv, D, scale, q_strides, k_strides, v_strides, mask_strides, o_strides,
+                           q_off, k_off, v_off, mask_off, o_off, stream, variant, workspace, workspace_bytes, false);
+}
+
+int mi355_sage_sdpa_bf16_mask_any(const void* Q, const void* K, const void* V, const void* Mask, void* O,
+                                  int B, int H, int N_q, int N_kv, int D, float scale,
+                                  const int64_t* q_strides, const int64_t* k_strides,
+                                  const int64_t* v_strides, const int64_t* mask_strides, const int64_t* o_strides,
+                                  int64_t q_off, int64_t k_off, int64_t v_off, int64_t mask_off, int64_t o_off,
+                                  void* stream, int variant, void* workspace, size_t workspace_bytes) {
+    return sdpa_mask_entry(Q, K, V, Mask, O, B, H, N_q, N_kv, D, scale, q_strides, k_strides, v_strides, mask_strides, o_strides,
+                           q_off, k_off, v_off, mask_off, o_off, stream, variant, workspace, workspace_bytes, true);
 }
 
 static int quant_qk_entry(const void* Q, const void* K, int B, int H, int N_q, int N_kv, int D,
@@ -795,6 +816,22 @@ int mi355_sage_attn_short_rule(int B, int H, int N_q, int N_kv, int D, int varia
 int mi355_sage_set_attn_split_wait(int polls) {
     if (polls < -(1 << 24) || polls > (1 << 24)) return MI355_SAGE_EINVAL;
     attn_split_wait(polls);
+    return MI355_SAGE_OK;
+}
+
+int mi355_sage_cast(int count, const void* const* src, void* const* dst, const int64_t* n, int to_bf16, void* stream) {
+    if (count < 1 || count > 4 || !src || !dst || !n) return MI355_SAGE_EINVAL;
+    CastArgs a{};
+    a.count = count;
+    for (int t = 0; t < count; t++) {
+        if (n[t] < 0 || (n[t] > 0 && (!src[t] || !dst[t]))) return MI355_SAGE_EINVAL;
+        if ((reinterpret_cast<uintptr_t>(src[t]) | reinterpret_cast<uintptr_t>(dst[t])) & 15) {
+            SAGE_LOG("cast: tensors must be 16-byte aligned");
+            return MI355_SAGE_EUNSUPPORTED;
+        }
+        a.src[t] = src[t]; a.dst[t] = dst[t]; a.n[t] = n[t];
+    }
+    SAGE_HIP(launch_cast(a, to_bf16 != 0, static_cast<hipStream_t>(stream)));
     return MI355_SAGE_OK;
 }
 

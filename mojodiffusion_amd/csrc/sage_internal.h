@@ -184,6 +184,16 @@ struct BwdArgs {
 };
 hipError_t launch_bwd(const BwdArgs& a, hipStream_t st);
 
+// ---- F32 <-> bf16 at the boundary (sage_cast.hip) ---------------------------
+struct CastArgs {
+    int count;                                   // 1 .. 4 tensors
+    const void* src[4];
+    void* dst[4];
+    int64_t n[4];                                // elements; bases 16-byte aligned
+    unsigned blocks[4];                          // filled by the launcher
+};
+hipError_t launch_cast(const CastArgs& a, bool to_bf16, hipStream_t st);
+
 // Key k of a 64-key tile is stored at this slot of the V tile (host + device).
 __host__ __device__ inline int v_slot_f16(int k) {
     // 16-key groups; inside a group the quads of 4 keys are ordered 0,2,1,3 so that

@@ -1,0 +1,402 @@
+// sage_torch.cpp — the host side of the common calls, native (CPython extension _sage_host).
+//
+// attention_sage.py states the call surface: names, checks, error texts.  This module does the same work for
+// calls that meet every check — allocate the outputs, carve the workspace, call the C ABI on the current
+// stream — without the interpreter in between: 21 us of host time per call from Python and ctypes, of which
+// two launches are 5 us, became 8.  Anything it does not take (another dtype, a shape that must be refused,
+// a non-zero return code) comes back as None, and the Python function goes its own way and raises.
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <ATen/ATen.h>
+#include <c10/hip/HIPStream.h>
+
+#include <cstring>
+#include <map>
+#include <mutex>
+#include <utility>
+
+#include "../../include/mi355_sage.h"
+
+namespace {
+
+// The C ABI's entry points, handed over by the ctypes loader: one library instance whatever its path.
+struct Api {
+    decltype(&mi355_sage_workspace_bytes) workspace_bytes;
+    decltype(&mi355_sage_bwd_workspace_bytes) bwd_workspace_bytes;
+    decltype(&mi355_sage_sdpa_bf16) sdpa;
+    decltype(&mi355_sage_sdpa_bf16_train_fwd) train_fwd;
+    decltype(&mi355_sage_sdpa_bf16_keymask) keymask;
+    decltype(&mi355_sage_sdpa_bf16_mask_any) mask_any;
+    decltype(&mi355_sage_sdpa_bf16_norm_rope) norm_rope;
+    decltype(&mi355_sage_sdpa_bf16_norm_rope_train_fwd) norm_rope_train;
+    decltype(&mi355_sage_sdpa_bwd_bf16) bwd;
+    decltype(&mi355_sage_cast) cast;
+} api;
+constexpr int kApiEntries = sizeof(Api) / sizeof(void*);
+static_assert(sizeof(Api) == kApiEntries * sizeof(void*), "one pointer per entry");
+
+void* stream_of(const at::Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+// One growing buffer per (device, stream): steady-state calls allocate nothing and calls on different streams
+// never share scratch memory.  A replaced buffer stays valid for the work queued on its stream: the
+// allocator hands its memory out again only to that stream.  (Never destroyed: the device may be gone by then.)
+std::mutex g_ws_mutex;
+auto& g_ws = *new std::map<std::pair<int, void*>, at::Tensor>;
+
+at::Tensor workspace(size_t nbytes, const at::Device& dev, void* stream) {
+    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    at::Tensor& ws = g_ws[{dev.index(), stream}];
+    if (!ws.defined() || (size_t)ws.numel() < nbytes)
+        ws = at::empty({(int64_t)nbytes}, at::TensorOptions().dtype(at::kByte).device(dev));
+    return ws;
+}
+size_t at_least(size_t n) { return n < 256 ? 256 : n; }
+
+struct Strides { int64_t s[4]; };
+Strides bshd(const at::Tensor& t) { return Strides{{t.size(1) * t.size(2) * t.size(3), t.size(3), t.size(2) * t.size(3), 1}}; }
+
+bool device_bhsd(const at::Tensor& t) { return t.dim() == 4 && t.is_cuda() && t.is_contiguous(); }
+at::Tensor like(const at::Tensor& t, at::ScalarType dt) { return at::empty(t.sizes(), t.options().dtype(dt).requires_grad(false)); }
+
+bool aligned16(const at::Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; }
+
+// q [B,Sq,H,D], k and v [B,Skv,H,D], contiguous on one device, one dtype.
+bool shapes_ok(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, bool square) {
+    if (!device_bhsd(q) || !device_bhsd(k) || !device_bhsd(v) || k.sizes() != v.sizes()) return false;
+    if (q.scalar_type() != k.scalar_type() || q.scalar_type() != v.scalar_type()) return false;
+    if (q.device() != k.device() || q.device() != v.device()) return false;
+    if (q.size(0) != k.size(0) || q.size(2) != k.size(2) || q.size(3) != k.size(3)) return false;
+    return q.numel() > 0 && k.numel() > 0 && (!square || q.size(1) == k.size(1));
+}
+
+int cast(int n, const at::Tensor* const* src, at::Tensor* dst, bool to_bf16) {
+    const void* s[4];
+    void* d[4];
+    int64_t len[4];
+    for (int i = 0; i < n; i++) {
+        dst[i] = like(*src[i], to_bf16 ? at::kBFloat16 : at::kFloat);
+        s[i] = src[i]->data_ptr(); d[i] = dst[i].data_ptr(); len[i] = src[i]->numel();
+    }
+    return api.cast(n, s, d, len, to_bf16, stream_of(*src[0]));
+}
+
+enum Kind { kPlain = 0, kTrain = 1, kKeyMask = 2 };
+
+// BF16 in, O (and Stats for kTrain) out; lo / hi: the masked key range, or hi = real_N_kv for kTrain.
+int forward(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, double scale, int variant, int kind, int lo, int hi,
+            at::Tensor& o, at::Tensor& stats) {
+    const int B = q.size(0), Sq = q.size(1), H = q.size(2), D = q.size(3), Skv = k.size(1);
+    const size_t need = api.workspace_bytes(B, H, Sq, Skv, D, variant);
+    if (need == 0) return MI355_SAGE_EUNSUPPORTED;
+    void* st = stream_of(q);
+    o = like(q, at::kBFloat16);
+    if (kind == kTrain) stats = at::empty({B, H, Sq, 1}, q.options().dtype(at::kFloat).requires_grad(false));
+    const at::Tensor ws = workspace(at_least(need), q.device(), st);
+    const Strides qs = bshd(q), ks = bshd(k);
+    const void *pq = q.data_ptr(), *pk = k.data_ptr(), *pv = v.data_ptr();
+    void *po = o.data_ptr(), *pw = ws.data_ptr();
+    const size_t nw = (size_t)ws.numel();
+    if (kind == kTrain)
+        return api.train_fwd(pq, pk, pv, po, stats.data_ptr(), B, H, Sq, Skv, D, (float)scale, qs.s, ks.s, ks.s, qs.s, 0, 0, 0, 0, 0, 0,
+                             Sq, hi, st, variant, pw, nw);
+    if (kind == kKeyMask)
+        return api.keymask(pq, pk, pv, po, nullptr, B, H, Sq, Skv, D, (float)scale, qs.s, ks.s, ks.s, qs.s, 0, 0, 0, 0, 0, lo, hi, st,
+                           variant, pw, nw);
+    return api.sdpa(pq, pk, pv, po, B, H, Sq, Skv, D, (float)scale, qs.s, ks.s, ks.s, qs.s, 0, 0, 0, 0, 0, st, variant, pw, nw);
+}
+
+int backward(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& o, const at::Tensor& d_out,
+             const at::Tensor& stats, double scale, int real_q, int real_kv, at::Tensor (&g)[3]) {
+    const int B = q.size(0), Sq = q.size(1), H = q.size(2), D = q.size(3), Skv = k.size(1);
+    const size_t need = api.bwd_workspace_bytes(B, H, Sq, Skv, D);
+    if (need == 0) return MI355_SAGE_EUNSUPPORTED;
+    void* st = stream_of(q);
+    g[0] = like(q, at::kBFloat16); g[1] = like(k, at::kBFloat16); g[2] = like(v, at::kBFloat16);
+    const at::Tensor ws = workspace(at_least(need), q.device(), st);
+    const Strides qs = bshd(q), ks = bshd(k);
+    return api.bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), d_out.data_ptr(), stats.data_ptr(), g[0].data_ptr(),
+                   g[1].data_ptr(), g[2].data_ptr(), B, H, Sq, Skv, D, (float)scale, qs.s, ks.s, ks.s, qs.s, qs.s, qs.s, ks.s, ks.s, 0, 0,
+                   0, 0, 0, 0, 0, 0, 0, 0, real_q, real_kv, st, ws.data_ptr(), (size_t)ws.numel());
+}
+
+// The recorded attention node (attention_sage._SdpaNode): forward set saved, gradients by the flash backward,
+// F32 activations cast at the boundary.
+struct SdpaNode : torch::autograd::Function<SdpaNode> {
+    static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
+                              double scale, int64_t variant) {
+        at::Tensor b[3] = {q, k, v}, o, stats, out;
+        const bool f32 = q.scalar_type() == at::kFloat;
+        if (f32) {
+            const at::Tensor* src[3] = {&q, &k, &v};
+            TORCH_CHECK(cast(3, src, b, true) == 0, "record_sdpa: cast failed");
+        }
+        const int rc = ::forward(b[0], b[1], b[2], scale, (int)variant, kTrain, 0, k.size(1), o, stats);
+        TORCH_CHECK(rc == 0, "sdpa_flash_train_fwd: shim rc=", rc);
+        out = o;
+        if (f32) {
+            const at::Tensor* src[1] = {&o};
+            TORCH_CHECK(cast(1, src, &out, false) == 0, "record_sdpa: cast failed");
+        }
+        ctx->save_for_backward({b[0], b[1], b[2], o, stats});
+        ctx->saved_data["scale"] = scale;
+        return out;
+    }
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
+        const auto saved = ctx->get_saved_variables();
+        const double scale = ctx->saved_data["scale"].toDouble();
+        const at::Tensor& g = grads[0];
+        const at::Tensor& q = saved[0];
+        at::Tensor d = g.is_contiguous() && aligned16(g) ? g : g.clone(at::MemoryFormat::Contiguous), out[3], res[3];
+        if (d.scalar_type() == at::kFloat) {
+            at::Tensor d32 = d;
+            const at::Tensor* src[1] = {&d32};
+            TORCH_CHECK(cast(1, src, &d, true) == 0, "record_sdpa: cast failed");
+        } else {
+            d = d.to(at::kBFloat16);
+        }
+        const int rc = ::backward(q, saved[1], saved[2], saved[3], d, saved[4], scale, q.size(1), saved[1].size(1), out);
+        TORCH_CHECK(rc == 0, "sdpa_flash_backward_raw: shim rc=", rc);
+        if (g.scalar_type() == at::kFloat) {
+            const at::Tensor* src[3] = {&out[0], &out[1], &out[2]};
+            TORCH_CHECK(cast(3, src, res, false) == 0, "record_sdpa: cast failed");
+        } else {
+            for (int i = 0; i < 3; i++) res[i] = out[i].to(g.scalar_type());
+        }
+        return {res[0], res[1], res[2], at::Tensor(), at::Tensor()};
+    }
+};
+
+// ---- argument access -----------------------------------------------------------------------------
+bool tensor_arg(PyObject* o, const at::Tensor*& t) {
+    if (!THPVariable_Check(o)) return false;
+    t = &THPVariable_Unpack(o);
+    return true;
+}
+bool double_arg(PyObject* o, double& x) {
+    x = PyFloat_AsDouble(o);
+    if (x == -1.0 && PyErr_Occurred()) { PyErr_Clear(); return false; }
+    return true;
+}
+bool int_arg(PyObject* o, int& x) {
+    if (!PyLong_Check(o)) return false;
+    const long n = PyLong_AsLong(o);
+    if (n == -1 && PyErr_Occurred()) { PyErr_Clear(); return false; }
+    x = (int)n;
+    return x == n;
+}
+template <class F> int without_gil(F f) {
+    PyThreadState* s = PyEval_SaveThread();
+    int rc;
+    try {
+        rc = f();
+    } catch (...) {
+        PyEval_RestoreThread(s);
+        throw;
+    }
+    PyEval_RestoreThread(s);
+    return rc;
+}
+
+// C++ exceptions (out of memory, HIP errors of the allocator) as Python ones
+template <class F> PyObject* guarded(F f) {
+    try {
+        return f();
+    } catch (const c10::Error& e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace());
+    } catch (const std::exception& e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+    }
+    return nullptr;
+}
+
+// fwd(q, k, v, scale, variant, kind, lo, hi, square) -> o, (o, stats) for kind 1, or None.  BF16; for the kinds
+// without Stats also F32, cast at the boundary.
+PyObject* py_fwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    const at::Tensor *q, *k, *v;
+    double scale;
+    int variant, kind, lo, hi, square;
+    if (n != 9 || !tensor_arg(a[0], q) || !tensor_arg(a[1], k) || !tensor_arg(a[2], v) || !double_arg(a[3], scale) || !int_arg(a[4], variant) ||
+        !int_arg(a[5], kind) || !int_arg(a[6], lo) || !int_arg(a[7], hi) || !int_arg(a[8], square))
+        Py_RETURN_NONE;
+    if (!shapes_ok(*q, *k, *v, square != 0)) Py_RETURN_NONE;
+    const bool f32 = q->scalar_type() == at::kFloat;
+    if (q->scalar_type() != at::kBFloat16 && !(f32 && kind != kTrain)) Py_RETURN_NONE;
+    return guarded([&]() -> PyObject* {
+        at::Tensor o, stats;
+        const int rc = without_gil([&] {
+            if (!f32) return forward(*q, *k, *v, scale, variant, kind, lo, hi, o, stats);
+            at::Tensor b[3], ob;
+            const at::Tensor* src[3] = {q, k, v};
+            int r = cast(3, src, b, true);
+            if (r == 0) r = forward(b[0], b[1], b[2], scale, variant, kind, lo, hi, ob, stats);
+            if (r != 0) return r;
+            const at::Tensor* back[1] = {&ob};
+            return cast(1, back, &o, false);
+        });
+        if (rc != 0) Py_RETURN_NONE;
+        if (kind != kTrain) return THPVariable_Wrap(std::move(o));
+        PyObject* t = PyTuple_New(2);
+        PyTuple_SET_ITEM(t, 0, THPVariable_Wrap(std::move(o)));
+        PyTuple_SET_ITEM(t, 1, THPVariable_Wrap(std::move(stats)));
+        return t;
+    });
+}
+
+// bias(q, k, v, mask, scale, variant, square) -> o or None.  BF16, mask [B,H,Sq,Skv] with contiguous rows.
+PyObject* py_bias(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    const at::Tensor *q, *k, *v, *m;
+    double scale;
+    int variant, square;
+    if (n != 7 || !tensor_arg(a[0], q) || !tensor_arg(a[1], k) || !tensor_arg(a[2], v) || !tensor_arg(a[3], m) || !double_arg(a[4], scale) ||
+        !int_arg(a[5], variant) || !int_arg(a[6], square))
+        Py_RETURN_NONE;
+    if (!shapes_ok(*q, *k, *v, square != 0) || q->scalar_type() != at::kBFloat16 || m->scalar_type() != at::kBFloat16) Py_RETURN_NONE;
+    const int B = q->size(0), Sq = q->size(1), H = q->size(2), D = q->size(3), Skv = k->size(1);
+    if (m->dim() != 4 || m->device() != q->device() || m->size(0) != B || m->size(1) != H || m->size(2) != Sq || m->size(3) != Skv || m->stride(3) != 1)
+        Py_RETURN_NONE;
+    return guarded([&]() -> PyObject* {
+        at::Tensor o;
+        const int rc = without_gil([&] {
+            const size_t need = api.workspace_bytes(B, H, Sq, Skv, D, variant);
+            if (need == 0) return MI355_SAGE_EUNSUPPORTED;
+            void* st = stream_of(*q);
+            o = like(*q, at::kBFloat16);
+            const at::Tensor ws = workspace(at_least(need), q->device(), st);
+            const Strides qs = bshd(*q), ks = bshd(*k), ms{{m->stride(0), m->stride(1), m->stride(2), 1}};
+            return api.mask_any(q->data_ptr(), k->data_ptr(), v->data_ptr(), m->data_ptr(), o.data_ptr(), B, H, Sq, Skv, D, (float)scale, qs.s,
+                                ks.s, ks.s, ms.s, qs.s, 0, 0, 0, 0, 0, st, variant, ws.data_ptr(), (size_t)ws.numel());
+        });
+        if (rc != 0) Py_RETURN_NONE;
+        return THPVariable_Wrap(std::move(o));
+    });
+}
+
+// norm_rope(q, k, v, q_gain, k_gain, eps, cos, sin, scale, variant, blkq, blkk, k_flags, layout, train)
+//   -> o, (o, stats) with train, or None.  BF16 with BF16 gains; layout as in the C ABI, without the table bit.
+PyObject* py_norm_rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    const at::Tensor *q, *k, *v, *gq, *gk, *cs = nullptr, *sn = nullptr;
+    double eps, scale;
+    int variant, blkq, blkk, k_flags, layout, train;
+    if (n != 15 || !tensor_arg(a[0], q) || !tensor_arg(a[1], k) || !tensor_arg(a[2], v) || !tensor_arg(a[3], gq) || !tensor_arg(a[4], gk) ||
+        !double_arg(a[5], eps) || !double_arg(a[8], scale) || !int_arg(a[9], variant) || !int_arg(a[10], blkq) || !int_arg(a[11], blkk) ||
+        !int_arg(a[12], k_flags) || !int_arg(a[13], layout) || !int_arg(a[14], train))
+        Py_RETURN_NONE;
+    if ((a[6] == Py_None) != (a[7] == Py_None)) Py_RETURN_NONE;
+    if (a[6] != Py_None && (!tensor_arg(a[6], cs) || !tensor_arg(a[7], sn))) Py_RETURN_NONE;
+    if (!shapes_ok(*q, *k, *v, true) || q->scalar_type() != at::kBFloat16) Py_RETURN_NONE;
+    const int B = q->size(0), S = q->size(1), H = q->size(2), D = q->size(3);
+    const int64_t cols = (layout & MI355_SAGE_NORM_FULL_ROW) ? (int64_t)H * D : D;
+    for (const at::Tensor* g : {gq, gk})
+        if (g->scalar_type() != at::kBFloat16 || g->device() != q->device() || !g->is_contiguous() || g->numel() != cols) Py_RETURN_NONE;
+    int64_t batch_rows = 0;
+    if (cs) {
+        if (cs->scalar_type() != sn->scalar_type() || (cs->scalar_type() != at::kFloat && cs->scalar_type() != at::kBFloat16)) Py_RETURN_NONE;
+        if (cs->dim() != 2 || cs->sizes() != sn->sizes() || cs->size(1) != D / 2 || !cs->is_contiguous() || !sn->is_contiguous() ||
+            cs->device() != q->device() || sn->device() != q->device())
+            Py_RETURN_NONE;
+        if (cs->scalar_type() == at::kBFloat16) layout |= MI355_SAGE_ROPE_TABLES_BF16;
+        if (cs->size(0) == (int64_t)B * S * H && B > 1) batch_rows = (int64_t)S * H;
+        else if (cs->size(0) != (int64_t)S * H) Py_RETURN_NONE;
+    }
+    return guarded([&]() -> PyObject* {
+        at::Tensor o, stats;
+        const int rc = without_gil([&] {
+            const size_t need = api.workspace_bytes(B, H, S, S, D, variant);
+            if (need == 0) return MI355_SAGE_EUNSUPPORTED;
+            void* st = stream_of(*q);
+            o = like(*q, at::kBFloat16);
+            if (train) stats = at::empty({B, H, S, 1}, q->options().dtype(at::kFloat).requires_grad(false));
+            const at::Tensor ws = workspace(at_least(need), q->device(), st);
+            const Strides s = bshd(*q);
+            const void *pc = cs ? cs->data_ptr() : nullptr, *ps = sn ? sn->data_ptr() : nullptr;
+            if (train)
+                return api.norm_rope_train(q->data_ptr(), k->data_ptr(), v->data_ptr(), o.data_ptr(), stats.data_ptr(), B, H, S, S, D, (float)scale,
+                                           s.s, s.s, s.s, s.s, 0, 0, 0, 0, 0, 0, S, S, st, variant, gq->data_ptr(), gk->data_ptr(), (float)eps, pc,
+                                           ps, batch_rows, layout, ws.data_ptr(), (size_t)ws.numel());
+            return api.norm_rope(q->data_ptr(), k->data_ptr(), v->data_ptr(), o.data_ptr(), B, H, S, S, D, (float)scale, s.s, s.s, s.s, s.s, 0, 0, 0,
+                                 0, 0, st, variant, blkq, blkk, k_flags, gq->data_ptr(), gk->data_ptr(), (float)eps, pc, ps, batch_rows, layout,
+                                 ws.data_ptr(), (size_t)ws.numel());
+        });
+        if (rc != 0) Py_RETURN_NONE;
+        if (!train) return THPVariable_Wrap(std::move(o));
+        PyObject* t = PyTuple_New(2);
+        PyTuple_SET_ITEM(t, 0, THPVariable_Wrap(std::move(o)));
+        PyTuple_SET_ITEM(t, 1, THPVariable_Wrap(std::move(stats)));
+        return t;
+    });
+}
+
+// bwd(q, k, v, o, d_out, stats, scale, real_q, real_kv) -> (d_q, d_k, d_v) or None.  BF16, Stats F32 contiguous.
+PyObject* py_bwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    const at::Tensor *q, *k, *v, *o, *d, *st;
+    double scale;
+    int rq, rk;
+    if (n != 9 || !tensor_arg(a[0], q) || !tensor_arg(a[1], k) || !tensor_arg(a[2], v) || !tensor_arg(a[3], o) || !tensor_arg(a[4], d) ||
+        !tensor_arg(a[5], st) || !double_arg(a[6], scale) || !int_arg(a[7], rq) || !int_arg(a[8], rk))
+        Py_RETURN_NONE;
+    if (!shapes_ok(*q, *k, *v, false) || q->scalar_type() != at::kBFloat16) Py_RETURN_NONE;
+    for (const at::Tensor* t : {o, d})
+        if (t->scalar_type() != at::kBFloat16 || !device_bhsd(*t) || t->sizes() != q->sizes() || t->device() != q->device()) Py_RETURN_NONE;
+    if (st->scalar_type() != at::kFloat || !st->is_cuda() || !st->is_contiguous() || st->device() != q->device() ||
+        st->numel() != q->size(0) * q->size(1) * q->size(2))
+        Py_RETURN_NONE;
+    return guarded([&]() -> PyObject* {
+        at::Tensor g[3];
+        if (without_gil([&] { return backward(*q, *k, *v, *o, *d, *st, scale, rq, rk, g); }) != 0) Py_RETURN_NONE;
+        PyObject* t = PyTuple_New(3);
+        for (int i = 0; i < 3; i++) PyTuple_SET_ITEM(t, i, THPVariable_Wrap(std::move(g[i])));
+        return t;
+    });
+}
+
+// record(q, k, v, scale, variant) -> att with its node, or None.
+PyObject* py_record(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    const at::Tensor *q, *k, *v;
+    double scale;
+    int variant;
+    if (n != 5 || !tensor_arg(a[0], q) || !tensor_arg(a[1], k) || !tensor_arg(a[2], v) || !double_arg(a[3], scale) || !int_arg(a[4], variant))
+        Py_RETURN_NONE;
+    if (!shapes_ok(*q, *k, *v, true) || (q->scalar_type() != at::kBFloat16 && q->scalar_type() != at::kFloat)) Py_RETURN_NONE;
+    // (what the kernels would refuse is left to the Python path, so that nothing can fail inside the node)
+    if ((q->size(3) != 64 && q->size(3) != 128) || (variant != 0 && variant != 1) || !aligned16(*q) || !aligned16(*k) || !aligned16(*v)) Py_RETURN_NONE;
+    return guarded([&]() -> PyObject* {
+        at::Tensor out;
+        without_gil([&] { out = SdpaNode::apply(*q, *k, *v, scale, (int64_t)variant); return 0; });
+        return THPVariable_Wrap(std::move(out));
+    });
+}
+
+// workspace(nbytes, tensor) -> this (device, stream)'s buffer
+PyObject* py_workspace(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    const at::Tensor* t;
+    if (n != 2 || !PyLong_Check(a[0]) || !tensor_arg(a[1], t)) {
+        PyErr_SetString(PyExc_TypeError, "workspace(nbytes, tensor)");
+        return nullptr;
+    }
+    const size_t nbytes = PyLong_AsSize_t(a[0]);
+    if (PyErr_Occurred()) return nullptr;
+    return guarded([&]() -> PyObject* { return THPVariable_Wrap(workspace(nbytes, t->device(), stream_of(*t))); });
+}
+
+// bind(addresses): the C ABI entry points, in the order of Api
+PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != kApiEntries) {
+        PyErr_Format(PyExc_TypeError, "bind: %d addresses expected", kApiEntries);
+        return nullptr;
+    }
+    void* p[kApiEntries];
+    for (int i = 0; i < kApiEntries; i++) {
+        p[i] = PyLong_AsVoidPtr(a[i]);
+        if (PyErr_Occurred()) return nullptr;
+    }
+    std::memcpy(&api, p, sizeof(api));
+    Py_RETURN_NONE;
+}
+
+#define METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(py_##name)), METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {METHOD(fwd), METHOD(bias), METHOD(norm_rope), METHOD(bwd), METHOD(record), METHOD(workspace), METHOD(bind), {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_sage_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__sage_host(void) { return PyModule_Create(&module_def); }

@@ -28,12 +28,11 @@ IDEOGRAM4_SDPA_SAGE = True
 def _product_fwd(name, enabled, q, k, v, scale, variant, rect):
     if not enabled:
         raise Error("%s: the quantized-attention arm is switched off and this package has no other backend" % name)
-    fwd_fn = A.sdpa_flash_train_fwd_rect if rect else A.sdpa_flash_train_fwd
     if q.dtype == torch.bfloat16 and k.dtype == torch.bfloat16 and v.dtype == torch.bfloat16:
         # (the reference clones because its O may be a view into a padded buffer; O here is
         # already an owning, unpadded tensor)
-        return fwd_fn(q, k, v, scale, variant).o
-    out = fwd_fn(q.to(torch.bfloat16), k.to(torch.bfloat16), v.to(torch.bfloat16), scale, variant).o
+        return A.sdpa_flash_fwd_o(q, k, v, scale, variant, rect)
+    out = A.sdpa_flash_fwd_o(q.to(torch.bfloat16), k.to(torch.bfloat16), v.to(torch.bfloat16), scale, variant, rect)
     return out.to(q.dtype)
 
 

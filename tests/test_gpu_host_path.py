@@ -1,0 +1,90 @@
+"""GPU tests of the native host path (csrc/sage_torch.cpp) and of what it calls besides the entry points tested
+elsewhere: the boundary casts, the bias with rows at any start, the recorded node.  The Python path behind it is
+the reference: same kernels, so the same bits."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from mojodiffusion_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("sizes", [(1,), (7, 8, 9), (2047, 2048, 2049, 100003)])
+def test_casts_round_like_torch(sizes):
+    """F32 -> bf16 to nearest even (ties, infinities, subnormals; NaN stays NaN) and back, tensors of any length."""
+    import torch
+    L = _lib.lib()
+    g = torch.Generator(device="cuda")
+    g.manual_seed(3)
+    src = [torch.randn(n, device="cuda", generator=g) * 10.0 ** float(i * 12 - 20) for i, n in enumerate(sizes)]
+    special = torch.tensor([1.00390625, 1.01171875, -1.00390625, float("inf"), -float("inf"), float("nan"), 1e-40, -0.0], device="cuda")
+    src[-1][:min(8, src[-1].numel())] = special[:min(8, src[-1].numel())]
+    dst = [torch.full((t.numel() + 1,), 7.0, device="cuda").bfloat16() for t in src]
+    back = [torch.full((t.numel() + 1,), 7.0, device="cuda") for t in src]
+    n = len(src)
+    ptrs = lambda ts: (ctypes.c_void_p * n)(*(t.data_ptr() for t in ts))
+    lens = (ctypes.c_int64 * n)(*sizes)
+    st = torch.cuda.current_stream().cuda_stream
+    assert L.mi355_sage_cast(n, ptrs(src), ptrs(dst), lens, 1, st) == 0
+    assert L.mi355_sage_cast(n, ptrs(dst), ptrs(back), lens, 0, st) == 0
+    torch.cuda.synchronize()
+    for s, d, b in zip(src, dst, back):
+        want, k = s.bfloat16(), s.numel()
+        assert torch.equal(torch.isnan(d[:k]), torch.isnan(want)) and torch.equal(d[:k].nan_to_num(5.0), want.nan_to_num(5.0))
+        assert torch.equal(b[:k].nan_to_num(5.0), want.float().nan_to_num(5.0))
+        assert float(d[k]) == 7.0 and float(b[k]) == 7.0                    # nothing past the end
+    assert L.mi355_sage_cast(5, ptrs(src), ptrs(dst), lens, 1, st) == -1
+
+
+@pytest.mark.parametrize("variant,Sq,Skv,D", [(0, 70, 77, 128), (1, 33, 129, 64), (0, 600, 1031, 128), (0, 40, 6, 256)])
+def test_bias_rows_at_any_start(variant, Sq, Skv, D):
+    """A contiguous bias of odd key count: the bits of the same bias in rows padded to four keys."""
+    import torch
+    from mojodiffusion_amd import attention_sage as A
+    torch.manual_seed(Sq)
+    q, k, v = (torch.randn((2, n, 3, D), device="cuda").bfloat16() for n in (Sq, Skv, Skv))
+    bias = torch.randn((2, 3, Sq, Skv), device="cuda").bfloat16()
+    got = A.sdpa_cross_masked(q, k, v, bias, D ** -0.5, variant)
+    padded = torch.zeros((2, 3, Sq, (Skv + 3) // 4 * 4), device="cuda").bfloat16()
+    padded[..., :Skv] = bias
+    want = torch.empty_like(q)
+    L = _lib.lib()
+    qs, ks = _lib.strides_bhnd(Sq, 3, D), _lib.strides_bhnd(Skv, 3, D)
+    ms = (ctypes.c_int64 * 4)(*padded.stride())
+    assert L.mi355_sage_sdpa_bf16_mask(q.data_ptr(), k.data_ptr(), v.data_ptr(), padded.data_ptr(), want.data_ptr(), 2, 3, Sq, Skv, D, D ** -0.5,
+                                       qs, ks, ks, ms, qs, 0, 0, 0, 0, 0, torch.cuda.current_stream().cuda_stream, variant, None, 0) == 0
+    torch.cuda.synchronize()
+    assert torch.isfinite(got.float()).all() and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16", "float16"])
+def test_recorded_node_has_the_bits_of_the_python_node(dtype):
+    """record_sdpa through the native node (F32, BF16; F16 falls through) against the Python node: values and gradients."""
+    import torch
+    from mojodiffusion_amd import attention_sage as A
+    torch.manual_seed(1)
+    base = [torch.randn((1, 130, 3, 64), device="cuda").to(getattr(torch, dtype)) for _ in range(4)]
+    runs = []
+    for fn in (A.record_sdpa, lambda q, k, v, s: A._SdpaNode.apply(q, k, v, s, A.PV_FP16)):
+        q, k, v = (t.clone().requires_grad_(True) for t in base[:3])
+        att = fn(q, k, v, 0.125)
+        runs.append((att.detach(),) + torch.autograd.grad(att, (q, k, v), base[3].transpose(1, 2).contiguous().transpose(1, 2)))
+    assert (_lib.host().record(*base[:3], 0.125, 0) is None) == (dtype == "float16")
+    for a, b in zip(*runs):
+        assert a.dtype == b.dtype and torch.equal(a, b)
+
+
+def test_native_path_leaves_what_it_does_not_take():
+    import torch
+    from mojodiffusion_amd import attention_sage as A
+    h = _lib.host()
+    t = torch.zeros((1, 64, 2, 64), device="cuda").bfloat16()
+    assert h.fwd(t, t, t, 0.1, 0, 0, 0, 0, 1) is not None
+    for bad in (t.half(), t.cpu(), t.transpose(1, 2), t[0], None):
+        assert h.fwd(bad, bad, bad, 0.1, 0, 0, 0, 0, 1) is None
+    assert h.fwd(t, t, t, 0.1, 7, 0, 0, 0, 1) is None and h.fwd(t, t[:, :32].contiguous(), t[:, :32].contiguous(), 0.1, 0, 0, 0, 0, 1) is None
+    with pytest.raises(A.Error, match="shim rc=-2"):
+        A.sdpa_nomask(t, t, t, 0.1, 7)
+    assert np.isfinite(A.sdpa_nomask(t.float(), t.float(), t.float(), 0.1).cpu().numpy()).all()
