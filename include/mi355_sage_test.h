@@ -4,6 +4,8 @@
 #ifndef MI355_SAGE_TEST_H
 #define MI355_SAGE_TEST_H
 
+#include <stdint.h>
+
 #ifdef __cplusplus
 extern "C" {
 #endif
@@ -36,6 +38,10 @@ int mi355_sage_set_attn_short(int mode);
 
 /* Key runs the short form would use for this shape by the rule alone, 0 for the 256-row workgroups. */
 int mi355_sage_attn_short_rule(int B, int H, int N_q, int N_kv, int D, int variant);
+
+/* Row tiles (256 rows of a head; 128 at head dim 256) the main kernel would do for this shape on the current
+ * device and under the current switches; the short form does the others. */
+int64_t mi355_sage_attn_main_items(int B, int H, int N_q, int N_kv, int D, int variant);
 
 #ifdef __cplusplus
 }

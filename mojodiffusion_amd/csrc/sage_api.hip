@@ -343,11 +343,10 @@ int sdpa_impl(const void* Q, const void* K, const void* V, void* O, void* Stats,
     }
     // (one decision for carving and launching; slots the caller's workspace was not sized for — a
     // forced schedule of the test switch — come from the library's per-stream buffer)
-    const int short_kw = attn_short_runs(B, H, N_q, kv, D, variant);
-    const int split_wgs = causal || short_kw > 0 ? 0 : attn_split_workgroups(B, H, N_q, kv, D, variant);
+    const AttnPlan plan = attn_plan(B, H, N_q, kv, D, variant, causal != 0);
     // The plain forward leaves Q to the attention kernel, which encodes its own rows (same codes and
     // scales): the quantize stage then neither reads Q nor writes its codes.
-    const bool q_in_kernel = Stats == nullptr && mask.add == nullptr && pre.q.gain == nullptr && (D <= 128 || short_kw > 0) && split_wgs == 0;
+    const bool q_in_kernel = Stats == nullptr && mask.add == nullptr && pre.q.gain == nullptr && (D <= 128 || plan.main_items == 0) && plan.split_wgs == 0;
     QuantOut o{};
     o.q8 = q_in_kernel ? nullptr : reinterpret_cast<int8_t*>(ws + c.q8);
     o.k8 = reinterpret_cast<int8_t*>(ws + c.k8);
@@ -391,8 +390,9 @@ int sdpa_impl(const void* Q, const void* K, const void* V, void* O, void* Stats,
         a.q_src = q.p; a.qsb = q.sb; a.qsh = q.sh; a.qsn = q.sn;
         a.qmul = o.qmul;
     }
-    a.short_kw = short_kw;
-    a.split_wgs = split_wgs;
+    a.main_items = plan.main_items;
+    a.short_kw = plan.short_kw;
+    a.split_wgs = plan.split_wgs;
     if (a.split_wgs > 0) {
         if (attn_split_bytes(a.split_wgs, D) <= attn_split_bytes(attn_split_rule(B, H, N_q, kv, D, variant), D)) a.split = ws + c.split;
         else if ((rc = internal_workspace(g_split_ws, attn_split_bytes(a.split_wgs, D), st, &a.split))) return rc;
@@ -750,8 +750,8 @@ int mi355_sage_attn_fwd(const void* q8, const void* qscale, int blkq, const void
     a.stats = static_cast<float*>(stats);
     // Same scheduling, hence the same bits, as the one-shot calls: shapes that are split over a
     // fixed number of workgroups need hand-over slots, kept per (device, stream) by the library.
-    a.short_kw = attn_short_runs(B, H, N_q, kv_valid, D, variant);
-    a.split_wgs = a.short_kw > 0 ? 0 : attn_split_workgroups(B, H, N_q, kv_valid, D, variant);
+    const AttnPlan plan = attn_plan(B, H, N_q, kv_valid, D, variant, false);
+    a.main_items = plan.main_items; a.short_kw = plan.short_kw; a.split_wgs = plan.split_wgs;
     const size_t split_bytes = attn_split_bytes(a.split_wgs, D);
     if (split_bytes > 0 && (rc = internal_workspace(g_split_ws, split_bytes, static_cast<hipStream_t>(stream), &a.split))) return rc;
     SAGE_HIP(launch_attn(a, static_cast<hipStream_t>(stream)));
@@ -771,10 +771,11 @@ int mi355_sage_attn_fwd_q16(const void* Q, const int64_t* q_strides, int64_t q_o
     int rc;
     if ((rc = check_kv_len(N_kv, blkk, D))) return rc;
     if ((rc = check_view("Q", Q, q_strides, q_off)) || (rc = check_view("O", O, o_strides, o_off))) return rc;
-    // (shapes of the split schedule keep the encoded-Q form: the one-shot calls do the same)
+    // (shapes that qualify for the split schedule keep the encoded-Q form here, whatever the plan)
     AttnArgs a{};
-    a.short_kw = attn_short_runs(B, H, N_q, kv_valid, D, variant);
-    if (a.short_kw == 0 && attn_split_workgroups(B, H, N_q, kv_valid, D, variant) > 0) return MI355_SAGE_EUNSUPPORTED;
+    const AttnPlan plan = attn_plan(B, H, N_q, kv_valid, D, variant, false);
+    if (plan.main_items > 0 && attn_split_workgroups(B, H, N_q, kv_valid, D, variant) > 0) return MI355_SAGE_EUNSUPPORTED;
+    a.main_items = plan.main_items; a.short_kw = plan.short_kw;
     const View q = make_view(Q, q_strides, q_off);
     a.q_src = q.p; a.qsb = q.sb; a.qsh = q.sh; a.qsn = q.sn; a.qmul = static_cast<const float*>(qmul); a.blkq = blkq;
     a.k8 = static_cast<const int8_t*>(k8); a.kscale = static_cast<const float*>(kscale); a.blkk = blkk;
@@ -811,6 +812,11 @@ int mi355_sage_set_attn_short(int mode) {
 int mi355_sage_attn_short_rule(int B, int H, int N_q, int N_kv, int D, int variant) {
     if (B <= 0 || H <= 0 || N_q <= 0 || N_kv <= 0) return 0;
     return attn_short_rule(B, H, N_q, N_kv, D, variant);
+}
+
+int64_t mi355_sage_attn_main_items(int B, int H, int N_q, int N_kv, int D, int variant) {
+    if (B <= 0 || H <= 0 || N_q <= 0 || N_kv <= 0) return 0;
+    return attn_plan(B, H, N_q, N_kv, D, variant, false).main_items;
 }
 
 int mi355_sage_set_attn_split_wait(int polls) {

@@ -923,9 +923,9 @@ __global__ void split_clear_kernel(int* flags, int n) {
 template <int D, int VARIANT>
 static hipError_t launch_attn_dv(const AttnArgs& a, hipStream_t st) {
     constexpr int kThreads = D > 128 ? 256 : 512;             // 32 query rows per wave
-    const int n_qtiles = (int)(a.nq_pad / (kThreads / 2));
-    const int64_t total = (int64_t)n_qtiles * a.B * a.H;
-    if (total <= 0 || total > 0x7FFFFFFF) return hipErrorInvalidValue;
+    const int n_qtiles = (a.Nq + kThreads / 2 - 1) / (kThreads / 2);
+    const int64_t total = a.main_items;
+    if (total <= 0 || total > 0x7FFFFFFF || total > (int64_t)n_qtiles * a.B * a.H) return hipErrorInvalidValue;
     const int split = (D <= 128 && VARIANT == 0 && !a.causal) ? a.split_wgs : 0;
     int* flags = nullptr;
     float* part = nullptr;
@@ -1064,11 +1064,14 @@ size_t attn_split_bytes(int workgroups, int D) {
 
 hipError_t launch_attn(const AttnArgs& a, hipStream_t st) {
     if (a.nkv_pad > max_keys(a.D)) return hipErrorInvalidValue;      // K scales would not fit the LDS staging
-    if (a.short_kw > 0) return launch_attn_short(a, st);
-    if (a.D == 128) return a.variant == 0 ? launch_attn_dv<128, 0>(a, st) : launch_attn_dv<128, 1>(a, st);
-    if (a.D == 64) return a.variant == 0 ? launch_attn_dv<64, 0>(a, st) : launch_attn_dv<64, 1>(a, st);
-    if (a.D == 256) return a.variant == 0 ? launch_attn_dv<256, 0>(a, st) : launch_attn_dv<256, 1>(a, st);
-    return hipErrorInvalidValue;
+    hipError_t e = hipSuccess;
+    if (a.main_items > 0) {
+        if (a.D == 128) e = a.variant == 0 ? launch_attn_dv<128, 0>(a, st) : launch_attn_dv<128, 1>(a, st);
+        else if (a.D == 64) e = a.variant == 0 ? launch_attn_dv<64, 0>(a, st) : launch_attn_dv<64, 1>(a, st);
+        else if (a.D == 256) e = a.variant == 0 ? launch_attn_dv<256, 0>(a, st) : launch_attn_dv<256, 1>(a, st);
+        else e = hipErrorInvalidValue;
+    }
+    return e == hipSuccess && a.short_kw > 0 ? launch_attn_short(a, st) : e;
 }
 
 }  // namespace sage

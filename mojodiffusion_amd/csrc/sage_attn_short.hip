@@ -23,10 +23,11 @@
 
 namespace sage {
 
+template <int D> constexpr int kMainRows = D > 128 ? 128 : 256;               // rows per workgroup of the main kernel
 template <int D> constexpr int short_waves() { return D > 128 ? 4 : 8; }      // 256 channels: a wave needs a SIMD's registers
 
 template <int D, int VARIANT, int KW, bool QF, bool ADDMASK>
-__global__ __launch_bounds__(short_waves<D>() * 64) void sage_attn_short_kernel(AttnArgs a, int n_rtiles, int total_wg) {
+__global__ __launch_bounds__(short_waves<D>() * 64) void sage_attn_short_kernel(AttnArgs a, int n_rtiles, int item0, int total_wg) {
     constexpr int NW = short_waves<D>();
     constexpr int R = NW / KW;                          // 32-row blocks per workgroup
     constexpr int ROWS = 32 * R;
@@ -56,7 +57,12 @@ __global__ __launch_bounds__(short_waves<D>() * 64) void sage_attn_short_kernel(
     const int bid = blockIdx.x;
     const int per = total_wg >> 3, extra = total_wg & 7, xcd = bid & 7;
     const int wg = xcd * per + min(xcd, extra) + (bid >> 3);
-    const int rt = wg % n_rtiles, bh = wg / n_rtiles;
+    // item0 > 0: the main kernel has done the items (row tiles of kMainRows) below it; n_rtiles counts those
+    // tiles then, and consecutive workgroups take the pieces of one
+    constexpr int PIECES = kMainRows<D> / ROWS;
+    const int item = item0 > 0 ? item0 + wg / PIECES : wg;
+    const int rt = item0 > 0 ? item % n_rtiles * PIECES + wg % PIECES : item % n_rtiles, bh = item / n_rtiles;
+    if (rt * ROWS >= a.Nq) return;                      // a piece behind the last row
     const int b = bh / a.H, h = bh % a.H;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -383,18 +389,20 @@ __global__ __launch_bounds__(short_waves<D>() * 64) void sage_attn_short_kernel(
 
 template <int D, int VARIANT, int KW>
 static hipError_t launch_short_dvk(const AttnArgs& a, hipStream_t st) {
-    constexpr int NW = short_waves<D>(), ROWS = 32 * (NW / KW);
-    const int n_rtiles = (a.Nq + ROWS - 1) / ROWS;
-    const int64_t total = (int64_t)n_rtiles * a.B * a.H;
-    if (total <= 0 || total > 0x7FFFFFFF) return hipErrorInvalidValue;
+    constexpr int NW = short_waves<D>(), ROWS = 32 * (NW / KW), PIECES = kMainRows<D> / ROWS;
+    const int64_t bh = (int64_t)a.B * a.H, qtiles = (a.Nq + kMainRows<D> - 1) / kMainRows<D>;
+    const int64_t n_rtiles = a.main_items > 0 ? qtiles : (a.Nq + ROWS - 1) / ROWS;
+    const int64_t total = a.main_items > 0 ? (bh * qtiles - a.main_items) * PIECES : bh * n_rtiles;
+    if (total <= 0 || total > 0x7FFFFFFF || a.main_items > 0x7FFFFFFF) return hipErrorInvalidValue;
     const dim3 grid((unsigned)total), block(NW * 64);
+    const int item0 = (int)a.main_items;
     if (a.q_src != nullptr) {
         if (a.amask != nullptr || a.qmul == nullptr) return hipErrorInvalidValue;
-        hipLaunchKernelGGL((sage_attn_short_kernel<D, VARIANT, KW, true, false>), grid, block, 0, st, a, n_rtiles, (int)total);
+        hipLaunchKernelGGL((sage_attn_short_kernel<D, VARIANT, KW, true, false>), grid, block, 0, st, a, (int)n_rtiles, item0, (int)total);
     } else if (a.amask != nullptr) {
-        hipLaunchKernelGGL((sage_attn_short_kernel<D, VARIANT, KW, false, true>), grid, block, 0, st, a, n_rtiles, (int)total);
+        hipLaunchKernelGGL((sage_attn_short_kernel<D, VARIANT, KW, false, true>), grid, block, 0, st, a, (int)n_rtiles, item0, (int)total);
     } else {
-        hipLaunchKernelGGL((sage_attn_short_kernel<D, VARIANT, KW, false, false>), grid, block, 0, st, a, n_rtiles, (int)total);
+        hipLaunchKernelGGL((sage_attn_short_kernel<D, VARIANT, KW, false, false>), grid, block, 0, st, a, (int)n_rtiles, item0, (int)total);
     }
     return hipGetLastError();
 }
@@ -408,17 +416,19 @@ hipError_t launch_attn_short(const AttnArgs& a, hipStream_t st) {
     return hipErrorInvalidValue;
 }
 
-static std::atomic<int> g_short_mode{0};       // 0: by shape; -1: never; 4, 8: always, that many key runs (4 at 256 channels)
-void attn_short_override(int mode) { g_short_mode.store(mode); }
-
-// Which form, from what either costs on an MI355X: time = base + rounds (r + s steps) + fill (f + g steps) in
+// Which form, from what each costs on an MI355X: time = base + rounds (r + s steps) + fill (f + g steps) in
 // microseconds, with rounds = workgroups / 256 rounded up, fill = workgroups / 256, steps = key tiles (main
-// kernel) or key steps of the longest run (short form).  The coefficients are least-squares fits to 300
-// launches per head dim and variant (4 to 60 heads, 32 to 2048 queries, 32 to 2048 keys), which they
-// meet within 4 to 11 %; picking the form by them came within 0.4 % of always picking the faster one.
-// Measured at [1,256,30,128] 16.7 -> 10.0 us, [1,1024,8,64] 20.2 -> 9.5, [1,1024,8,128] 28.0 -> 13.9,
-// [1,512,24,128] 21.3 -> 12.8; the main kernel's form is back ahead at about 100 workgroups of 256 rows with
-// 128 channels (twice that many with few keys).
+// kernel) or key steps of the longest run (short form); the split schedule: base + per balanced key tile.
+// The coefficients are least-squares fits to about 300 launches per head dim and variant (4 to 480 heads, 32 to
+// 2048 queries, 32 to 4096 keys), which they meet within 4 to 11 %; picking the form by them came within
+// 0.6 % of always picking the faster one.  Measured at [1,256,30,128] 16.7 -> 10.0 us, [1,1024,8,64]
+// 20.2 -> 9.5, [1,1024,8,128] 28.0 -> 13.9, [1,512,24,128] 21.3 -> 12.8; the main kernel's form is back ahead
+// at about 100 workgroups of 256 rows with 128 channels (twice that many with few keys).
+//
+// A problem of some rounds and a bit more takes both: the main kernel does the full rounds and the short
+// form what is left, spread over the whole chip, instead of one more round that is nearly empty (264 items
+// of 32 key tiles, 128 channels: 84 -> 66 us; of 64 channels 61 -> 43).  The split schedule, which balances
+// the same problems by handing partial results over in memory, is left where it is predicted ahead of both.
 struct FormCost {
     float base, r, s, f, g;
     float of(int64_t wgs, int64_t steps) const {
@@ -427,33 +437,61 @@ struct FormCost {
     }
 };
 static const FormCost kCost[3][2][3] = {        // [64, 128, 256 channels][variant][main, 4 runs, 8 runs]
-    {{{3.89f, 3.67f, 0.76f, 3.69f, 0.02f}, {5.20f, 1.27f, 0.53f, 1.01f, 0.10f}, {4.59f, 1.68f, 0.57f, 0.39f, 0.10f}},
+    {{{6.00f, 1.70f, 0.78f, 0.00f, 0.03f}, {4.97f, 1.54f, 0.50f, 0.00f, 0.17f}, {5.18f, 1.19f, 0.41f, 0.14f, 0.27f}},
      {{3.52f, 4.41f, 0.91f, 3.03f, 0.00f}, {1.72f, 5.65f, 0.79f, 1.02f, 0.11f}, {2.30f, 5.33f, 0.31f, 0.23f, 0.41f}}},
-    {{{4.54f, 5.86f, 0.92f, 6.51f, 0.20f}, {2.76f, 5.78f, 0.77f, 1.97f, 0.52f}, {2.76f, 5.51f, 0.82f, 1.16f, 0.47f}},
+    {{{9.36f, 1.64f, 0.89f, 0.08f, 0.51f}, {3.45f, 5.23f, 0.71f, 0.49f, 0.69f}, {4.33f, 4.13f, 0.57f, 0.56f, 0.86f}},
      {{6.95f, 5.91f, 1.08f, 8.20f, 0.00f}, {2.69f, 6.85f, 1.12f, 2.05f, 0.17f}, {2.52f, 6.99f, 0.66f, 1.02f, 0.52f}}},
     {{{3.16f, 4.72f, 1.40f, 4.64f, 0.00f}, {2.15f, 5.54f, 1.26f, 1.78f, 0.27f}, {}},
      {{3.08f, 8.00f, 1.09f, 4.97f, 0.00f}, {1.83f, 5.98f, 2.04f, 1.26f, 0.00f}, {}}},
 };
+static const float kSplitCost[2][2] = {{11.8f, 1.08f}, {30.1f, 1.73f}};       // [64, 128 channels]: base, per key tile
 
-int attn_short_rule(int B, int H, int Nq, int kv_valid, int D, int variant) {
-    const FormCost* c = kCost[D == 64 ? 0 : D == 128 ? 1 : 2][variant == 0 ? 0 : 1];
+namespace {
+struct Short { float t; int kw; };
+Short best_short(const FormCost* c, int64_t rows, int64_t bh, int D, int64_t steps) {
+    const int rows4 = D > 128 ? 32 : 64;
+    const Short four{c[1].of(bh * ((rows + rows4 - 1) / rows4), (steps + 3) / 4), 4};
+    if (D > 128) return four;
+    const Short eight{c[2].of(bh * ((rows + 31) / 32), (steps + 7) / 8), 8};
+    return four.t < eight.t ? four : eight;
+}
+}  // namespace
+
+static AttnPlan plan_by_shape(int B, int H, int Nq, int kv_valid, int D, int variant, bool causal, int split) {
+    const int v = variant == 0 ? 0 : 1, d = D == 64 ? 0 : D == 128 ? 1 : 2;
+    const FormCost* c = kCost[d][v];
     const int64_t bh = (int64_t)B * H;
     const int64_t tiles = (kv_valid + kTileKV - 1) / kTileKV, steps = variant == 0 ? (kv_valid + 31) / 32 : tiles;
-    const int main_rows = D > 128 ? 128 : 256, rows4 = D > 128 ? 32 : 64;
-    const float t_main = c[0].of(bh * ((Nq + main_rows - 1) / main_rows), tiles);
-    const float t4 = c[1].of(bh * ((Nq + rows4 - 1) / rows4), (steps + 3) / 4);
-    if (D > 128) return t4 < t_main ? 4 : 0;
-    const float t8 = c[2].of(bh * ((Nq + 31) / 32), (steps + 7) / 8);
-    if (t4 < t8) return t4 < t_main ? 4 : 0;
-    return t8 < t_main ? 8 : 0;
+    const int rows = D > 128 ? 128 : 256;
+    const int64_t items = bh * ((Nq + rows - 1) / rows), whole = items / 256 * 256;
+    AttnPlan p{items, 0, 0};
+    float best = c[0].of(items, tiles);
+    const Short all = best_short(c, Nq, bh, D, steps);
+    if (all.t < best) { best = all.t; p = AttnPlan{0, all.kw, 0}; }
+    if (!causal && whole > 0 && whole < items) {
+        const Short rest = best_short(c, rows, items - whole, D, steps);
+        const float t = c[0].of(whole, tiles) + rest.t;
+        if (t < best) { best = t; p = AttnPlan{whole, rest.kw, 0}; }
+    }
+    if (!causal && split > 0 && D <= 128 && kSplitCost[d][0] + kSplitCost[d][1] * (float)(items * tiles) / 256.0f < best) p = AttnPlan{items, 0, split};
+    return p;
 }
 
-int attn_short_runs(int B, int H, int Nq, int kv_valid, int D, int variant) {
-    const int mode = g_short_mode.load();
-    if (mode < 0) return 0;
-    if (mode > 0) return D == 256 ? 4 : mode;
-    if (attn_split_override_mode() != 0) return 0;      // a schedule of the 256-row workgroups was asked for
-    return attn_short_rule(B, H, Nq, kv_valid, D, variant);
+static std::atomic<int> g_short_mode{0};       // 0: by shape; -1: never; 4, 8: always, that many key runs (4 at 256 channels)
+void attn_short_override(int mode) { g_short_mode.store(mode); }
+
+int attn_short_rule(int B, int H, int Nq, int kv_valid, int D, int variant) {
+    const AttnPlan p = plan_by_shape(B, H, Nq, kv_valid, D, variant, false, 0);
+    return p.main_items == 0 ? p.short_kw : 0;
+}
+
+AttnPlan attn_plan(int B, int H, int Nq, int kv_valid, int D, int variant, bool causal) {
+    const int mode = g_short_mode.load(), rows = D > 128 ? 128 : 256;
+    if (mode > 0) return AttnPlan{0, D == 256 ? 4 : mode, 0};
+    const int split = causal ? 0 : attn_split_workgroups(B, H, Nq, kv_valid, D, variant);
+    if (mode < 0 || attn_split_override_mode() != 0)      // (a schedule of the main kernel was asked for)
+        return AttnPlan{(int64_t)B * H * ((Nq + rows - 1) / rows), 0, split};
+    return plan_by_shape(B, H, Nq, kv_valid, D, variant, causal, split);
 }
 
 }  // namespace sage

@@ -138,17 +138,22 @@ struct AttnArgs {
     const uint16_t* q_src;   // null: q8 / qscale are read
     int64_t qsb, qsh, qsn;
     const float* qmul;
-    int split_wgs;           // workgroups of the split schedule (attn_split_workgroups), 0: one workgroup per item
-    int short_kw;            // key runs per row block in the short form (attn_short_runs), 0: the 256-row workgroups
+    // the plan (attn_plan): the main kernel does the row tiles below main_items, the short form the rest
+    int64_t main_items;
+    int short_kw;            // key runs per row block in the short form
+    int split_wgs;           // workgroups of the main kernel's split schedule, 0: one workgroup per item
     void* split;             // attn_split_bytes(split_wgs, D) bytes, 256-byte aligned (null when 0)
 };
 hipError_t launch_attn(const AttnArgs& a, hipStream_t st);
-// Shapes too small for 256-row workgroups: 32 or 64 rows per workgroup, keys split over its waves
-// (sage_attn_short.hip).  attn_short_rule: by shape alone, the number of key runs or 0;
-// attn_short_runs: the same, or what the test switch forces.  Takes precedence over the split schedule.
+// Which kernel does what.  Items are row tiles (256 query rows of a head; 128 at 256 channels), head by head.
+struct AttnPlan {
+    int64_t main_items;      // items [0, main_items) by the main kernel, the rest by the short form
+    int short_kw;            // key runs of the short form (32 or 64 rows per workgroup, keys split over its waves)
+    int split_wgs;           // > 0: the main kernel's items in the split schedule (then all of them)
+};
+AttnPlan attn_plan(int B, int H, int Nq, int kv_valid, int D, int variant, bool causal);
 hipError_t launch_attn_short(const AttnArgs& a, hipStream_t st);
-int attn_short_rule(int B, int H, int Nq, int kv_valid, int D, int variant);
-int attn_short_runs(int B, int H, int Nq, int kv_valid, int D, int variant);
+int attn_short_rule(int B, int H, int Nq, int kv_valid, int D, int variant);     // short_kw where the short form does everything by shape, else 0
 void attn_short_override(int mode);          // 0: by shape (default); -1: never; 4 or 8: always
 // Shapes whose items do not fill whole rounds of workgroups are spread evenly over a fixed number
 // of workgroups that hand partial results to each other through `split`.
