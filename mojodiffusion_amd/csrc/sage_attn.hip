@@ -159,7 +159,15 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     // row are masked for every one of its rows — they are treated as the ragged end, so their tiles are
     // never copied — and the steps on a wave's diagonal mask key > row element by element (below).
     const int kv_valid = (!SPLIT && causal) ? min(kv_valid_all, (qt + 1) * ROWS_WG) : kv_valid_all;
-    const int ntiles = SPLIT ? span_end - item_base - t_off : (kv_valid + kTileKV - 1) / kTileKV;
+    // Key tiles that lie in the masked range as a whole are left out: from here on tile t stands for key tile
+    // t, or t + skip from skip_at on.  (An even number of them: the K scales of a trip are read 16 bytes at a time.)
+    int skip_at = 0, skip = 0;
+    if (!SPLIT && !causal && mask_hi > mask_lo) {
+        skip_at = (mask_lo + kTileKV - 1) / kTileKV;
+        skip = max(min(mask_hi, kv_valid) / kTileKV - skip_at, 0) & ~1;
+    }
+    const int ntiles = SPLIT ? span_end - item_base - t_off : (kv_valid + kTileKV - 1) / kTileKV - skip;
+    auto key_tile = [&](int t) -> int { return SPLIT || t < skip_at ? t : t + skip; };
     const bool seg_finishes = !SPLIT || t_off + ntiles == ntiles_item;   // holds the item's last key tile: writes the output
     span_end = item_base + t_off;
     const int64_t bh = (uint32_t)wg / (uint32_t)qtiles_div;
@@ -271,8 +279,8 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
 #pragma unroll
         for (int i = 0; i < V_CH; i++) dma16(g, vsrc[i], __builtin_amdgcn_readfirstlane(vdst[i] + slot * V_BYTES));
     };
-    auto dma_k = [&](int t, int slot) { dma_k_at(kg + (int64_t)t * K_BYTES, slot); };
-    auto dma_v = [&](int t, int slot) { dma_v_at(vg + (int64_t)t * V_BYTES, slot); };
+    auto dma_k = [&](int t, int slot) { dma_k_at(kg + (int64_t)key_tile(t) * K_BYTES, slot); };
+    auto dma_v = [&](int t, int slot) { dma_v_at(vg + (int64_t)key_tile(t) * V_BYTES, slot); };
 
     v16f oacc[DB];
 #pragma unroll
@@ -492,13 +500,14 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         const int slot_vcopy = HT >= 0 ? (HT / SPT + LEAD) & 3 : (t + LEAD) % NSV;
 
         float f[SKB], c0[SKB];
+        const int hk = TRIP ? 0 : (t_off + key_tile(t) - t) * SPT + h;        // the step's keys: hk * SK ..
 #pragma unroll
         for (int kb = 0; kb < SKB; kb++)
-            f[kb] = sq * (TRIP ? kst[((HT + PERIOD - 1) % PERIOD) * SKB + kb] : kscale_of(t_off * 2 + h * SKB + kb));
+            f[kb] = sq * (TRIP ? kst[((HT + PERIOD - 1) % PERIOD) * SKB + kb] : kscale_of(hk * SKB + kb));
         // Steps that hold masked keys (the ragged end, the masked range) are rare: a real branch.
         // A masked score becomes -inf (as an integer: below every real accumulator), which the
         // exponent path below turns into p = 0 without any further test.
-        const int key0 = t_off * kTileKV + h * SK;
+        const int key0 = hk * SK;
         if (!TRIP && __builtin_expect(key0 + SK > kv_valid || (key0 < mask_hi && key0 + SK > mask_lo) ||
                                       (causal && key0 + SK - 1 > wave_row0), 0)) {
             asm volatile("" ::: "memory");
@@ -714,19 +723,28 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     // ones with an additive mask, whose time goes into reading the mask anyway)
     if constexpr (NSK == 4 && NSV == 4 && !SPLIT && !ADDMASK) {
         step(0, X0{}, std::integral_constant<int, 0>{}, T{}, T{});
-        // The main loop takes the steps in front of the first masked key (the ragged end, the masked
-        // range) without looking for masked keys; the steps after that go through the loop below.
-        int clean = (kv_valid - t_off * kTileKV) / SK;
-        if (mask_hi > mask_lo && t_off * kTileKV < mask_hi) clean = min(clean, max(mask_lo - t_off * kTileKV, 0) / SK);
-        if (exact_bias) clean = 0;
+        // The main loop takes the steps whose keys all count without looking for masked keys: those in front
+        // of the masked range or the ragged end, then — the steps that touch the range, at most a few, go
+        // through the general bodies — those between the range and the ragged end.  Either stretch stops
+        // early enough that the copies a trip starts need no clamping and do not cross the left-out tiles.
+        const bool range = mask_hi > mask_lo && t_off * kTileKV < mask_hi;
+        int clean = (kv_valid - t_off * kTileKV) / SK - skip * SPT;
         if (causal) clean = min(clean, (wave_row0 + 1) / SK);       // steps whose every key is <= the wave's first row
-        // (... and in front of the last tiles, so that the copies a trip starts need no clamping)
-        const int trip_end = min(last_step - SPT * (KOFF + LEAD) + (SPT - 1), clean);
+        const int tail_end = exact_bias ? 0 : min(last_step - SPT * (KOFF + LEAD) + (SPT - 1), clean);
+        int trip_end = tail_end, past = 0, resume = 0;
+        if (range) {
+            trip_end = min(trip_end, max(mask_lo - t_off * kTileKV, 0) / SK);
+            if (skip > 0) trip_end = min(trip_end, (skip_at - (KOFF + LEAD)) * SPT - 1 + (SPT - 1));
+            // first step of a trip (1 modulo the period) behind the range
+            resume = (mask_hi - t_off * kTileKV + SK - 1) / SK - skip * SPT;
+            resume = max(resume + (PERIOD - 1), 0) / PERIOD * PERIOD + 1;
+        }
+        for (;;) {
         for (; hs + PERIOD <= trip_end; hs += PERIOD) {
-            kg_trip = kg + (int64_t)(hs / SPT) * K_BYTES;
-            vg_trip = vg + (int64_t)(hs / SPT) * V_BYTES;
+            kg_trip = kg + (int64_t)(hs / SPT + past) * K_BYTES;
+            vg_trip = vg + (int64_t)(hs / SPT + past) * V_BYTES;
             {
-                const v4f* kp = reinterpret_cast<const v4f*>(&lds_ks[KS_OFF + t_off * 2 + hs * SKB]);
+                const v4f* kp = reinterpret_cast<const v4f*>(&lds_ks[KS_OFF + (t_off + past) * 2 + hs * SKB]);
                 const v4f k0 = kp[0], k1 = kp[1];
                 kst[0] = k0.x; kst[1] = k0.y; kst[2] = k0.z; kst[3] = k0.w;
                 kst[4] = k1.x; kst[5] = k1.y; kst[6] = k1.z; kst[7] = k1.w;
@@ -742,13 +760,22 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
                 step(hs + 7, X0{}, std::integral_constant<int, 0>{}, F{}, T{});
             }
         }
+        // the steps up to the next stretch, or to the end: ring slots from the step number (hs is odd here)
+        const bool again = resume > hs && resume + PERIOD <= tail_end;
+        for (const int stop = again ? resume + 1 : last_step; hs + 1 < stop; hs += 2) {
+            step(hs, X1{}, R1{}, F{}, T{});
+            step(hs + 1, X0{}, R0{}, F{}, T{});
+        }
+        if (!again) break;
+        trip_end = tail_end;
+        past = skip;
+        }
     } else {
         step(0, X0{}, R0{}, T{}, T{});
-    }
-    // the remaining steps, ring slots from the step number (hs is odd here)
-    for (; hs + 1 < last_step; hs += 2) {
-        step(hs, X1{}, R1{}, F{}, T{});
-        step(hs + 1, X0{}, R0{}, F{}, T{});
+        for (; hs + 1 < last_step; hs += 2) {
+            step(hs, X1{}, R1{}, F{}, T{});
+            step(hs + 1, X0{}, R0{}, F{}, T{});
+        }
     }
     if (hs == last_step) {
         step(hs, X1{}, R1{}, F{}, F{});

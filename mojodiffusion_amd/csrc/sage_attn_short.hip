@@ -72,7 +72,15 @@ __global__ __launch_bounds__(short_waves<D>() * 64) void sage_attn_short_kernel(
 
     // causal: keys past the workgroup's last row count as the ragged end
     const int kv_valid = a.causal ? min(a.kv_valid, wg_row0 + ROWS) : a.kv_valid;
-    const int nsteps = (kv_valid + SK - 1) / SK;
+    // (steps that lie in the masked range as a whole are left out: step h stands for keys h * SK .., or those
+    // `skip` steps further on from skip_at on)
+    int skip_at = 0, skip = 0;
+    if (!a.causal && a.km.hi > a.km.lo) {
+        skip_at = (a.km.lo + SK - 1) / SK;
+        skip = max(min(a.km.hi, kv_valid) / SK - skip_at, 0);
+    }
+    auto key_step = [&](int h) -> int { return h < skip_at ? h : h + skip; };
+    const int nsteps = (kv_valid + SK - 1) / SK - skip;
     const int h0 = nsteps * kw / KW, h1 = nsteps * (kw + 1) / KW;
 
     // ---- one step's operands: copies into the wave's own LDS region, fragments out of it
@@ -86,12 +94,14 @@ __global__ __launch_bounds__(short_waves<D>() * 64) void sage_attn_short_kernel(
         const int L = swz(i * 64 + lane);
         vsrc[i] = VARIANT == 0 ? (L >> 6) * 128 + (L & 63) : L;
     }
-    auto copy_k = [&](int hs) {
+    auto copy_k = [&](int h) {
+        const int hs = key_step(h);
         const uint8_t* g = kg + (int64_t)hs * K_BYTES;
 #pragma unroll
         for (int i = 0; i < KC; i++) dma16(g, swz(i * 64 + lane), __builtin_amdgcn_readfirstlane(k_lds + i * 1024));
     };
-    auto copy_v = [&](int hs) {
+    auto copy_v = [&](int h) {
+        const int hs = key_step(h);
         const uint8_t* g = VARIANT == 0 ? vg + (int64_t)(hs >> 1) * (D * 128) + (hs & 1) * 64 : vg + (int64_t)hs * V_BYTES;
 #pragma unroll
         for (int i = 0; i < VC; i++) dma16(g, vsrc[i], __builtin_amdgcn_readfirstlane(v_lds + i * 1024));
@@ -222,7 +232,7 @@ __global__ __launch_bounds__(short_waves<D>() * 64) void sage_attn_short_kernel(
         const bool more = hs + 1 < h1;
         reads_done();
         if (more) copy_k(hs + 1);
-        const int key0 = hs * SK;
+        const int key0 = key_step(hs) * SK;
         float f[SKB];
 #pragma unroll
         for (int kb = 0; kb < SKB; kb++) f[kb] = sq * ksc[(key0 + kb * 32) >> ksh];
