@@ -32,16 +32,7 @@
 #include <atomic>
 #include <type_traits>
 
-// Measurement builds only (`make parts`, never part of the library): SAGE_LOOP_PART is a mask of
-// parts of the main loop to leave out, so that what each is worth can be read off the kernel's own
-// clock stamps (bench.py --clock-probe --probe-lib ...).  Results are wrong by design; every kernel
-// still runs to its end (no address and no trip count depends on what is left out).
-//   1 no tile copies in the loop   2 no workgroup barrier in the loop   4 no LDS fragment reads
-#ifndef SAGE_LOOP_PART
-#define SAGE_LOOP_PART 0
-#endif
 namespace sage {
-constexpr int kLoopPart = SAGE_LOOP_PART;
 
 // ADDMASK: an additive score bias (natural-log units, bf16, logical [B,H,Nq,Nkv] through element
 // strides with the key stride 1) is added to the dequantised scores.  That instantiation looks
@@ -348,7 +339,6 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     // e4m3 variant reads both blocks) of the K tile in `kslot` and whose P.V instructions read the
     // steps `sub` of the V^T tile in `vslot`.
     auto fetch = [&](int m, int kslot, int kbq, int vslot, int sub) {
-        if (kLoopPart & 4) { asm volatile("" : "+v"(fr[m][0])); return; }
         if (slot_is_qk(m)) {
             const int n = slot_index(m), st = SKB == 1 ? n : n >> 1, kb = SKB == 1 ? kbq : n & 1;
             fr[m][0] = k_frag(kslot, st, kb);
@@ -646,8 +636,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         // and V(t + LEAD).
         auto midpoint = [&]() {
             dma_wait<ADDMASK ? 0 : (LEAD - 1) * (K_CH + V_CH)>();
-            if (!(kLoopPart & 2)) __syncthreads();
-            if (!(kLoopPart & 1)) {
+            __syncthreads();
             if constexpr (TRIP) {
                 // (the main loop stops early enough that these tiles exist; their addresses are the
                 // trip's base plus a constant)
@@ -657,7 +646,6 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
             } else {
                 dma_k(min(t + KOFF + LEAD, last), slot_kcopy);
                 dma_v(min(t + LEAD, last), slot_vcopy);
-            }
             }
         };
 
