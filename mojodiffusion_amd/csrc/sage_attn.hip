@@ -36,9 +36,9 @@ namespace sage {
 
 // ADDMASK: an additive score bias (natural-log units, bf16, logical [B,H,Nq,Nkv] through element
 // strides with the key stride 1) is added to the dequantised scores.  That instantiation looks
-// for every tile's maximum on the biased scores (no optimistic tiles) and lets its ordinary
-// global loads share the vector-memory counter with the tile copies, i.e. it waits for all of
-// them at the midpoint: it is bound by the N_q x N_kv bias it has to read, not by the copies.
+// for every step's maximum on the biased scores (no optimistic steps).  Its ordinary global loads (the bias
+// of the next step) share the vector-memory counter with the tile copies, so it waits for all of them
+// at the midpoint.
 
 // Workgroups of the split schedule that gave up on a hand-over (see the kernel's fold-in part).
 static __device__ unsigned int g_split_faults;
@@ -59,7 +59,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     float* __restrict__ stats, int n_qtiles, int total_wg,
     const uint16_t* __restrict__ amask, int64_t amb, int64_t amh, int64_t amn,
     int split_groups, float* split_part, int* split_flags, int split_wait) {
-    constexpr int KS_OFF = VARIANT == 0 ? 3 : 2;        // see lds_ks
+    constexpr int KS_OFF = D > 128 ? 0 : VARIANT == 0 ? 3 : 2;        // see lds_ks
     constexpr int VB = (VARIANT == 0) ? 2 : 1;          // bytes per V element
     constexpr int KSTEPS = D / 32;                      // int8 MFMA steps over the head dim
     constexpr int DB = D / 32;                          // 32-channel output blocks
@@ -91,9 +91,11 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
 
     __shared__ __attribute__((aligned(1024))) uint8_t lds_k[NSK][K_BYTES];
     __shared__ __attribute__((aligned(1024))) uint8_t lds_v[NSV][V_BYTES];
-    __shared__ __attribute__((aligned(16))) float lds_ks[max_keys(D) / 32 + 4];
+    __shared__ __attribute__((aligned(16))) float lds_ks[max_keys(D) / 32 + (D > 128 ? 0 : 4)];
+    __shared__ __attribute__((aligned(16))) uint8_t lds_bias[ADDMASK ? NW : 1][ADDMASK ? BiasStage::BYTES : 16];
     __shared__ float lds_qmax[QF ? 8 : 1];              // QF: largest |pre-scaled q| of each wave's 32 rows
     __shared__ __attribute__((aligned(16))) uint8_t lds_qc[QF && VARIANT == 1 ? NW * 32 * D : 16];      // QF: Q codes on their way into fragments
+    static_assert(!(STATS && ADDMASK), "no entry point asks for Stats under an additive mask");
     static_assert(!QF || (D <= 128 && !STATS && !ADDMASK && !SPLIT), "Q is encoded in the kernel only in the plain forward");
 
     // Work items are (q tile, b*h) pairs, `total_wg` of them; an item takes `ntiles` steps (key
@@ -203,8 +205,8 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         // (the arithmetic follows further down, behind the first tile copies: their latency and this
         // one's then run side by side)
     }
-    // this lane's row of the additive bias (padding rows read the last real row; their output is dropped)
-    const uint16_t* mrow = ADDMASK ? amask + b * amb + h * amh + (int64_t)min(qrow, Nq - 1) * amn : nullptr;
+    // the head's additive bias (padding rows read the last real row; their output is dropped)
+    const uint16_t* mhead = ADDMASK ? amask + b * amb + h * amh : nullptr;
 
     // K scales of this head are staged in LDS once: a global load inside the main loop
     // would make the compiler wait for ALL outstanding vector-memory operations, i.e. for the
@@ -447,6 +449,13 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         for (int n = 0; n < NQ; n++) qk_step(0, n, k0[n]);
     }
     const int last_step = ntiles * SPT - 1;
+    auto key_step = [&](int h) -> int { return (t_off + key_tile(h / SPT) - h / SPT) * SPT + h; };       // step h's keys: key_step(h) * SK ..
+    BiasStage bias[SKB];                                // the next step's bias on its way
+    auto bias_load = [&](int h) {
+#pragma unroll
+        for (int kb = 0; kb < SKB; kb++) bias[kb].load(mhead, amn, wave_row0, Nq - 1, key_step(min(h, last_step)) * SK + kb * 32, kv_valid, lane);
+    };
+    if constexpr (ADDMASK) bias_load(0);
 #pragma unroll
     for (int m = PF - 1; m >= 0; m--)
         if (slot_is_qk(m)) fetch(m, (1 / SPT) % NSK, 1 % SPT, 0, 0);
@@ -490,7 +499,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         const int slot_vcopy = HT >= 0 ? (HT / SPT + LEAD) & 3 : (t + LEAD) % NSV;
 
         float f[SKB], c0[SKB];
-        const int hk = TRIP ? 0 : (t_off + key_tile(t) - t) * SPT + h;        // the step's keys: hk * SK ..
+        const int hk = TRIP ? 0 : key_step(h);
 #pragma unroll
         for (int kb = 0; kb < SKB; kb++)
             f[kb] = sq * (TRIP ? kst[((HT + PERIOD - 1) % PERIOD) * SKB + kb] : kscale_of(hk * SKB + kb));
@@ -514,15 +523,12 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         if constexpr (ADDMASK) {
 #pragma unroll
             for (int kb = 0; kb < SKB; kb++) {
+                bias[kb].put(lds_bias[wave], lane);     // (a wave's own LDS accesses keep their order)
                 // (the bias of the accumulators is taken off before the multiplication: exact, where
                 // folding it into the multiply-add's constant would cost the constant's rounding)
 #pragma unroll
                 for (int g = 0; g < 4; g++) {
-                    const int key = key0 + kb * 32 + g * 8 + half * 4;
-                    uint32_t w[2] = {0u, 0u};
-                    load_bias4(mrow, key, kv_valid, w);
-                    const float mv[4] = {__uint_as_float(w[0] << 16), __uint_as_float(w[0] & 0xFFFF0000u),
-                                         __uint_as_float(w[1] << 16), __uint_as_float(w[1] & 0xFFFF0000u)};
+                    const v4f mv = BiasStage::get(lds_bias[wave], l32, half, g);
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
                         const float sdq = (__int_as_float(s[X][kb][g * 4 + e]) - Magic<D>::F) * f[kb];
@@ -530,6 +536,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
                     }
                 }
             }
+            bias_load(h + 1);
         }
         float corr = 1.0f;
         bool refresh = false;
@@ -978,8 +985,8 @@ static hipError_t launch_attn_dv(const AttnArgs& a, hipStream_t st) {
             return hipErrorInvalidValue;
         }
     } else if (a.amask != nullptr) {
-        if (a.stats != nullptr) SAGE_LAUNCH_ATTN(true, true);
-        else SAGE_LAUNCH_ATTN(false, true);
+        if (a.stats != nullptr) return hipErrorInvalidValue;      // (no entry point asks for both)
+        SAGE_LAUNCH_ATTN(false, true);
     } else {
         if (a.stats != nullptr) SAGE_LAUNCH_ATTN(true, false);
         else SAGE_LAUNCH_ATTN(false, false);

@@ -140,16 +140,44 @@ __device__ __forceinline__ u32x2 encode8_i8(const float (&x)[8], float sc, float
     return u32x2{wd[0], wd[1]};
 }
 
-// Four consecutive bf16 values of a bias row, keys key .. key + 3 (those at and past `n` are left out).
-// Rows start at any even byte address: the access is as wide as the hardware takes it unaligned.
-__device__ __forceinline__ void load_bias4(const uint16_t* row, int key, int n, uint32_t (&w)[2]) {
-    if (key + 4 <= n) {
-        __builtin_memcpy(w, row + key, 8);
-    } else {
+// ---- additive bias: 32 rows x 32 keys of a wave ------------------------------------------------------
+// Loaded 16 bytes per lane, whole rows next to each other (a lane's own four keys of its own row, the layout
+// the scores have, are 64 separate pieces per instruction: 4 to 8 of them per step took longer than the
+// step's arithmetic, and twice as long where odd key counts start the rows anywhere), turned into the scores'
+// layout through LDS.  16-byte chunks of a row are XORed with the row, so that both sides touch every bank.
+struct BiasStage {
+    static constexpr int CPR = 4, RPI = 64 / CPR, NI = 32 / RPI;                 // chunks per row, rows per load, loads
+    static constexpr int BYTES = 32 * 64;
+    u32x4 w[NI];
+
+    static __device__ __forceinline__ int at(int row, int chunk) { return row * 64 + ((chunk ^ ((row >> 2) & 3)) << 4); }
+    // keys key0 .. key0 + 31 of rows row0 .. row0 + 31 (rows past the last repeat it; keys at and past n are 0).
+    // Rows start at any even byte address: the access is as wide as the hardware takes it unaligned.
+    __device__ __forceinline__ void load(const uint16_t* head, int64_t row_stride, int row0, int last_row, int key0, int n, int lane) {
+        const int key = key0 + (lane % CPR) * 8;
 #pragma unroll
-        for (int e = 0; e < 4; e++)
-            if (key + e < n) w[e >> 1] |= (uint32_t)row[key + e] << ((e & 1) * 16);
+        for (int i = 0; i < NI; i++) {
+            const uint16_t* p = head + (int64_t)min(row0 + i * RPI + lane / CPR, last_row) * row_stride + key;
+            uint32_t v[4] = {0u, 0u, 0u, 0u};
+            if (key + 8 <= n) {
+                __builtin_memcpy(v, p, 16);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    if (key + e < n) v[e >> 1] |= (uint32_t)p[e] << ((e & 1) * 16);
+            }
+            w[i] = u32x4{v[0], v[1], v[2], v[3]};
+        }
     }
-}
+    __device__ __forceinline__ void put(uint8_t* lds, int lane) const {
+#pragma unroll
+        for (int i = 0; i < NI; i++) *reinterpret_cast<u32x4*>(lds + at(i * RPI + lane / CPR, lane % CPR)) = w[i];
+    }
+    // keys g * 8 + half * 4 .. + 3 of row l32
+    static __device__ __forceinline__ v4f get(const uint8_t* lds, int l32, int half, int g) {
+        const u32x2 v = *reinterpret_cast<const u32x2*>(lds + at(l32, g) + half * 8);
+        return v4f{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xFFFF0000u), __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xFFFF0000u)};
+    }
+};
 
 }  // namespace sage

@@ -43,7 +43,7 @@ __global__ __launch_bounds__(short_waves<D>() * 64) void sage_attn_short_kernel(
     constexpr int LD = D + 4;                           // floats per row of the exchange buffer (keeps 16-byte alignment, spreads banks)
     static_assert(NW % KW == 0 && ROWS <= 128, "waves = row blocks x key runs");
 
-    struct Ring { uint8_t k[K_BYTES], v[V_BYTES]; };
+    struct Ring { uint8_t k[K_BYTES], v[V_BYTES], bias[ADDMASK ? BiasStage::BYTES : 16]; };
     union Mem {
         Ring ring[NW];                                  // the loop's operands
         float acc[NW][32 * LD];                         // the merge's partial outputs
@@ -203,7 +203,15 @@ __global__ __launch_bounds__(short_waves<D>() * 64) void sage_attn_short_kernel(
 
     const float* ksc = a.kscale + (int64_t)bh * (a.nkv_pad / a.blkk);
     const int ksh = a.blkk == 32 ? 5 : a.blkk == 64 ? 6 : 7;
-    const uint16_t* mrow = ADDMASK ? a.amask + b * a.amb + h * a.amh + (int64_t)min(qrow, a.Nq - 1) * a.amn : nullptr;
+    // the bias of a step is loaded while the step before it runs
+    BiasStage bias[SKB];
+    uint8_t* bias_lds = &mem.ring[wave].bias[0];
+    auto bias_load = [&](int hs) {
+#pragma unroll
+        for (int kb = 0; kb < SKB; kb++)
+            bias[kb].load(a.amask + b * a.amb + h * a.amh, a.amn, row0, a.Nq - 1, key_step(min(hs, h1 - 1)) * SK + kb * 32, kv_valid, lane);
+    };
+    if (ADDMASK && h0 < h1) bias_load(h0);
 
     v16f oacc[DB], lacc;
 #pragma unroll
@@ -253,13 +261,10 @@ __global__ __launch_bounds__(short_waves<D>() * 64) void sage_attn_short_kernel(
 #pragma unroll
         for (int kb = 0; kb < SKB; kb++) {
             if constexpr (ADDMASK) {
+                bias[kb].put(bias_lds, lane);
 #pragma unroll
                 for (int g = 0; g < 4; g++) {
-                    const int key = key0 + kb * 32 + g * 8 + half * 4;
-                    uint32_t w[2] = {0u, 0u};
-                    load_bias4(mrow, key, kv_valid, w);
-                    const float mv[4] = {__uint_as_float(w[0] << 16), __uint_as_float(w[0] & 0xFFFF0000u),
-                                         __uint_as_float(w[1] << 16), __uint_as_float(w[1] & 0xFFFF0000u)};
+                    const v4f mv = BiasStage::get(bias_lds, l32, half, g);
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
                         x[kb][g * 4 + e] = fmaf(mv[e], 1.4426950408889634f, (__int_as_float(s[kb][g * 4 + e]) - Magic<D>::F) * f[kb]);
@@ -276,6 +281,7 @@ __global__ __launch_bounds__(short_waves<D>() * 64) void sage_attn_short_kernel(
                 for (int i = 0; i < 16; i++) x[kb][i] = EXACT ? __int_as_float(s[kb][i]) - Magic<D>::F : __int_as_float(s[kb][i]);
             }
         }
+        if constexpr (ADDMASK) bias_load(hs + 1);
         {
             const v2u r = __builtin_amdgcn_permlane32_swap(__float_as_uint(mt), __float_as_uint(mt), false, false);
             mt = fmaxf(__uint_as_float(r.x), __uint_as_float(r.y));
