@@ -842,16 +842,13 @@ int mi355_sage_cast(int count, const void* const* src, void* const* dst, const i
 }
 
 // ---- backward ---------------------------------------------------------------------------------
-struct BwdCarve { size_t kT, qT, doT, lse2, delta, kcen, total; };
-static BwdCarve bwd_carve(int B, int H, int Nq, int Nkv, int D) {
+struct BwdCarve { size_t lse2, delta, kcen, total; };
+static BwdCarve bwd_carve(int B, int H, int Nq, int D) {
     const size_t bh = (size_t)B * H;
-    const size_t nqp = (size_t)pad_to(Nq, 64), nkp = (size_t)pad_to(Nkv, 64);
+    const size_t nqp = (size_t)pad_to(Nq, 64);
     BwdCarve c{};
     size_t off = 0;
     auto take = [&](size_t bytes) { size_t o = off; off += align_up(bytes); return o; };
-    c.kT = take(bh * nkp * D * 2);
-    c.qT = take(bh * nqp * D * 2);
-    c.doT = take(bh * nqp * D * 2);
     c.lse2 = take(bh * nqp * sizeof(float));
     c.delta = take(bh * nqp * sizeof(float));
     c.kcen = take(bh * D * sizeof(float));
@@ -861,7 +858,7 @@ static BwdCarve bwd_carve(int B, int H, int Nq, int Nkv, int D) {
 
 size_t mi355_sage_bwd_workspace_bytes(int B, int H, int N_q, int N_kv, int D) {
     if (B <= 0 || H <= 0 || N_q <= 0 || N_kv <= 0 || !bwd_dims_ok(D)) return 0;
-    return bwd_carve(B, H, N_q, N_kv, D).total;
+    return bwd_carve(B, H, N_q, D).total;
 }
 
 int mi355_sage_sdpa_bwd_bf16(const void* Q, const void* K, const void* V, const void* O, const void* dO,
@@ -900,7 +897,7 @@ int mi355_sage_sdpa_bwd_bf16(const void* Q, const void* K, const void* V, const 
         !span_ok("V", N_kv, v_strides))
         return MI355_SAGE_EUNSUPPORTED;
 
-    const BwdCarve c = bwd_carve(B, H, N_q, N_kv, D);
+    const BwdCarve c = bwd_carve(B, H, N_q, D);
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (workspace == nullptr) {
         if ((rc = internal_workspace(g_ws, c.total, st, &workspace))) return rc;
@@ -923,14 +920,10 @@ int mi355_sage_sdpa_bwd_bf16(const void* Q, const void* K, const void* V, const 
     a.valid_q = real_N_q > 0 && real_N_q < N_q ? real_N_q : N_q;          // cudnn_sdpa_bwd.cpp:362-363
     a.valid_kv = real_N_kv > 0 && real_N_kv < N_kv ? real_N_kv : N_kv;
     a.scale = scale;
-    a.kT = reinterpret_cast<uint16_t*>(ws + c.kT);
-    a.qT = reinterpret_cast<uint16_t*>(ws + c.qT);
-    a.doT = reinterpret_cast<uint16_t*>(ws + c.doT);
     a.lse2 = reinterpret_cast<float*>(ws + c.lse2);
     a.delta = reinterpret_cast<float*>(ws + c.delta);
     a.kcen = reinterpret_cast<float*>(ws + c.kcen);
     a.nq_pad = pad_to(N_q, 64);
-    a.nkv_pad = pad_to(N_kv, 64);
     SAGE_HIP(launch_bwd(a, st));
     return 0;
 }

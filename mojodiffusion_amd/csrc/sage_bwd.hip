@@ -8,24 +8,31 @@
 //
 // Two launches:
 //   1. bwd_prep_kernel     Delta and Stats * log2(e) per query row (padding rows: +inf, so their
-//                          probabilities vanish), and transposed copies K^T, Q^T, dO^T in tiles of
-//                          64 rows whose rows sit in the slot order of the matrix instruction's
-//                          operand layout (v_slot_f16); and a vector c close to the mean key.
+//                          probabilities vanish); and a vector c close to the mean key.
 //   2. bwd_fused_kernel    one grid of two kinds of 8-wave workgroups, the longer kind first:
 //        dQ     owner = 256 query rows, loop over key tiles, as scale * (dS K - rowsum(dS) c)
-//               = scale * dS (K - c)                                          (bwd_pass_body<D,0,8>)
+//               = scale * dS (K - c)                                          (bwd_pass_body<D,0>)
 //        dK,dV  owner = 128 keys, loop over query tiles; pairs of waves share 32 keys, one wave
 //               carrying P and dV, the other dS and dK                        (bwd_dkdv_body)
-//               (head dim 64: 256 keys, every wave both products — bwd_pass_body<D,1,8>)
+//               (head dim 64: 256 keys, every wave both products — bwd_pass_body<D,1>)
 // In both kinds a wave owns 32 rows ("x"), keeps their bf16 row blocks resident as B operands
 // and walks the other side ("y") in tiles of 64 rows staged in LDS by register-bypassing copies,
-// double buffered, one barrier per tile.  A 32x32 block of scores T[y,x] lands in the accumulator
+// a ring of three slots, one barrier per tile.  A 32x32 block of scores T[y,x] lands in the accumulator
 // layout with the owner row as the lane's column, which is exactly the B-operand layout of the
 // products that contract over y — so P and dS go from registers straight into the next matrix
-// instruction, and the only transposed operands (rows = head channel, k = y) are the ones read
-// from the transposed copies of launch 1.
+// instruction.  Those products' A operands are transposed (rows = head channel, k = y); they come from
+// the same row-major tile through the transposing LDS read (ds_read_b64_tr_b16), so every tile is
+// fetched once and nothing is rearranged in memory.
+//
+// What bounds it: a matrix instruction (32 clocks on its SIMD) takes 1 KiB of fragment from LDS (8 clocks of the
+// CU's 128 bytes each), and four SIMDs share the LDS — the two run neck and neck, and every byte the
+// copies write into LDS comes on top.  With pre-transposed copies of K, Q and dO made by launch 1, as the
+// first form had them, each tile was copied twice; owner rows were loaded and results stored as 64 separate
+// pieces per instruction.  Measured, one kernel trace of both, us (before -> now):
+//   [2,1248,30,128]  launch 1 25.8 -> 9.6, launch 2 231 -> 226 (best 218 -> 195)
+//   [1,4608,24,128]  launch 1 31.2 -> 11.8, launch 2 969 -> 884
+//   [1,2304,12,64]   launch 1 8.1 -> 4.8, launch 2 75.9 -> 76.9
 #include "sage_internal.h"
-#include <type_traits>
 
 namespace sage {
 
@@ -45,14 +52,14 @@ namespace {
 constexpr float kLog2e = 1.4426950408889634f;
 
 // ---- LDS layouts -------------------------------------------------------------------------
-// Transposed tile [D rows][64 slots] bf16: 128-byte rows, 8 chunks of 16 bytes per row; chunk
-// position XORed with bits of the pair-of-rows index (same layout as the forward's V^T tile).
-__device__ __forceinline__ int tr_off(int L) { return (((L >> 3) << 3) | ((L & 7) ^ ((L >> 4) & 7))) << 4; }
-// Natural tile [64 rows][D] bf16: CPR chunks per row.  16 consecutive rows reading one logical
-// chunk must land in 16 different 16-byte bank groups.
+// Tile [64 rows][D] bf16 in 16-byte chunks, CPR per row, the chunk position XORed with a function of the row.
+// Two access patterns meet in it:  fragments along the channels (16 consecutive rows, one logical chunk:
+// the 16 lanes must land in 16 different 16-byte bank groups), and transposed fragments (4 consecutive rows
+// times 4 neighbouring chunks per 32 lanes, 8 bytes each: the 16 chunks must be different ones).  With the
+// row's low two bits moved into the chunk's upper bits both are free of conflicts.
 template <int CPR> __device__ __forceinline__ int nat_pos(int row, int c) {
-    if constexpr (CPR == 16) return c ^ (row & 15);
-    else return c ^ ((row >> 1) & 7);
+    if constexpr (CPR == 16) return c ^ (((row & 3) << 2) | ((row >> 2) & 3));
+    else return c ^ ((((row >> 1) & 1) << 2) | ((row >> 2) & 3));       // (row & 1 is the half of the 64 banks)
 }
 template <int CPR> __device__ __forceinline__ int nat_off(int row, int c) { return (row * CPR + nat_pos<CPR>(row, c)) << 4; }
 
@@ -72,131 +79,137 @@ __device__ __forceinline__ void dma4(const void* gbase_uniform, uint32_t goff, u
                  : "s"(lds_base_uniform), "v"(goff), "s"(gbase_uniform)
                  : "memory");
 }
-__device__ __forceinline__ void dma_wait_all() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// Wait until at most N of this wave's copies are still in flight (they complete in order).
+template <int N> __device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
 __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
     const v2f f = {a, b};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, v2bf));       // round to nearest even
 }
 
-// inverse of v_slot_f16: which row of a 64-row tile sits at slot s
-__device__ __forceinline__ int row_of_slot(int s) {
-    const int g = s >> 4, r = s & 15;
-    const int quad = (((r >> 2) & 1) << 1) | (r >> 3);
-    return (g << 4) | (quad << 2) | (r & 3);
+// Transposed fragment of a tile: lane l gets channel (l & 31) of a 32-channel block, rows half * 4 + 0..3 in
+// the first two registers and 8 + half * 4 + 0..3 in the others (half = l >> 5), counted from a 16-row block —
+// the order in which an accumulator lane holds its rows, i.e. the A operand that goes with P and dS.
+// ds_read_b64_tr_b16 works on 16 lanes: lane i names 8 bytes (row i / 4, channels (i % 4) * 4 .. + 3 of a
+// 4 x 16 block) and receives channel i of the four rows.
+typedef short v4s __attribute__((ext_vector_type(4)));
+template <int CPR> __device__ __forceinline__ int tr_frag_off(int lane, int row0, int d) {
+    const int row = row0 + (lane >> 5) * 4 + ((lane & 15) >> 2);
+    const int ch = d * 32 + ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
+    return nat_off<CPR>(row, ch >> 3) + (ch & 7) * 2;
+}
+__device__ __forceinline__ v4i tr_read(const uint8_t* lo, const uint8_t* hi) {
+    using lds_v4s = __attribute__((address_space(3))) v4s;
+    const u32x2 a = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)lo));
+    const u32x2 b = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)hi));
+    return v4i{(int)a.x, (int)a.y, (int)b.x, (int)b.y};
 }
 
 }  // namespace
 
+// ---- the owner rows of a wave, in and out ----------------------------------------------------
+// A lane wants its own row's chunks as operands and ends up with pieces of its own row: as plain loads and
+// stores these are 64 separate pieces per instruction.  Whole rows move instead, through LDS.
+// 32 rows of D bf16 -> LDS at `dst` (64 * D bytes, chunks XORed as in a tile); rows past `last` repeat it.
+template <int D>
+__device__ __forceinline__ void rows_in(const uint16_t* head, int64_t sn, int row0, int last, uint32_t dst, int lane) {
+    constexpr int CPR = D / 8, RPI = 64 / CPR;
+#pragma unroll
+    for (int i = 0; i < 32 / RPI; i++) {
+        const int r = i * RPI + lane / CPR;
+        dma16(head, (uint32_t)min(row0 + r, last) * (uint32_t)(sn * 2) + nat_pos<CPR>(r, lane % CPR) * 16,
+              __builtin_amdgcn_readfirstlane(dst + i * 1024));
+    }
+}
+// channels ch .. ch + 3 (ch = d * 32 + g * 8 + half * 4) of the lane's row -> LDS
+template <int D>
+__device__ __forceinline__ void row_put(uint8_t* os, int l32, int half, int d, int g, u32x2 w) {
+    *reinterpret_cast<u32x2*>(os + nat_off<D / 8>(l32, d * 4 + g) + half * 8) = w;
+}
+// ... and from there to the rows below n of the caller's tensor, 16 bytes per lane
+template <int D>
+__device__ __forceinline__ void rows_out(const uint8_t* os, uint16_t* head, int64_t sn, int row0, int n, int lane) {
+    constexpr int CPR = D / 8, RPI = 64 / CPR;
+    uint16_t* op = head + (lane % CPR) * 8;
+#pragma unroll
+    for (int i = 0; i < 32 / RPI; i++) {
+        const int r = i * RPI + lane / CPR;
+        const u32x4 w = *reinterpret_cast<const u32x4*>(os + nat_off<CPR>(r, lane % CPR));
+        if (row0 + r < n) *reinterpret_cast<u32x4*>(op + (int64_t)(row0 + r) * sn) = w;
+    }
+}
+
 // ---------------------------------------------------------------------------------------------
-// Launch 1.  Roles of one grid, per (b,h): K^T tiles | Q^T tiles | dO^T tiles | row statistics.
+// Launch 1.  Per (b,h): workgroups with the row statistics of 64 query rows each, and one with the
+// mean of 64 keys.
 // ---------------------------------------------------------------------------------------------
 template <int D>
 __global__ __launch_bounds__(256) void bwd_prep_kernel(BwdArgs a) {
-    constexpr int CPR = D / 8;
-    constexpr int LROW = D + 8;                     // LDS row stride in elements (keeps 16-byte alignment, spreads banks)
-    __shared__ __attribute__((aligned(16))) uint16_t tile[64 * LROW];
-    const int ntk = (int)(a.nkv_pad / 64), ntq = (int)(a.nq_pad / 64);
-    const int per_bh = ntk + 3 * ntq;
-    const int bh = blockIdx.x / per_bh;
-    int r = blockIdx.x % per_bh;
+    constexpr int CPR = D / 8, RPP = 256 / CPR;     // threads per row, rows per pass of the workgroup
+    __shared__ float red[RPP * D];
+    const int ntq = (int)(a.nq_pad / 64);
+    const int bh = blockIdx.x / (ntq + 1);
+    const int r = blockIdx.x % (ntq + 1);
     const int b = bh / a.H, h = bh % a.H;
     const int tid = threadIdx.x;
+    const int col = (tid % CPR) * 8;
 
-    if (r >= ntk + 2 * ntq) {
-        // row statistics of 64 query rows: 4 threads per row
-        const int row = (r - ntk - 2 * ntq) * 64 + (tid >> 2);
-        const int part = tid & 3;
-        float sum = 0.0f;
-        if (row < a.valid_q) {
-            const uint16_t* po = a.o.p + b * a.o.sb + h * a.o.sh + (int64_t)row * a.o.sn + part * (D / 4);
-            const uint16_t* pg = a.dout.p + b * a.dout.sb + h * a.dout.sh + (int64_t)row * a.dout.sn + part * (D / 4);
+    if (r < ntq) {
+        const uint16_t* po = a.o.p + b * a.o.sb + h * a.o.sh + col;
+        const uint16_t* pg = a.dout.p + b * a.dout.sb + h * a.dout.sh + col;
+        u32x4 wo[64 / RPP], wg[64 / RPP];
 #pragma unroll
-            for (int c = 0; c < D / 32; c++) {
-                const u32x4 wo = *reinterpret_cast<const u32x4*>(po + c * 8);
-                const u32x4 wg = *reinterpret_cast<const u32x4*>(pg + c * 8);
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    sum = fmaf(__uint_as_float(wo[e] << 16), __uint_as_float(wg[e] << 16), sum);
-                    sum = fmaf(__uint_as_float(wo[e] & 0xFFFF0000u), __uint_as_float(wg[e] & 0xFFFF0000u), sum);
-                }
-            }
+        for (int i = 0; i < 64 / RPP; i++) {
+            const int64_t row = min(r * 64 + i * RPP + tid / CPR, a.valid_q - 1);
+            wo[i] = *reinterpret_cast<const u32x4*>(po + row * a.o.sn);
+            wg[i] = *reinterpret_cast<const u32x4*>(pg + row * a.dout.sn);
         }
-        sum += __shfl_xor(sum, 1);
-        sum += __shfl_xor(sum, 2);
-        if (part == 0) {
-            const int64_t idx = (int64_t)bh * a.nq_pad + row;
-            const bool valid = row < a.valid_q;
-            a.delta[idx] = valid ? sum : 0.0f;
-            a.lse2[idx] = valid ? a.stats[(int64_t)bh * a.Nq + row] * kLog2e : INFINITY;
+#pragma unroll
+        for (int i = 0; i < 64 / RPP; i++) {
+            float sum = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                sum = fmaf(__uint_as_float(wo[i][e] << 16), __uint_as_float(wg[i][e] << 16), sum);
+                sum = fmaf(__uint_as_float(wo[i][e] & 0xFFFF0000u), __uint_as_float(wg[i][e] & 0xFFFF0000u), sum);
+            }
+#pragma unroll
+            for (int m = 1; m < CPR; m <<= 1) sum += __shfl_xor(sum, m);
+            if (tid % CPR == 0) {
+                const int row = r * 64 + i * RPP + tid / CPR;
+                const int64_t idx = (int64_t)bh * a.nq_pad + row;
+                const bool valid = row < a.valid_q;
+                a.delta[idx] = valid ? sum : 0.0f;
+                a.lse2[idx] = valid ? a.stats[(int64_t)bh * a.Nq + row] * kLog2e : INFINITY;
+            }
         }
         return;
     }
 
-    // transposed copy of one 64-row tile
-    View src;
-    uint16_t* dst;
-    int valid, t;
-    int64_t ntiles;
-    const bool is_k = r < ntk;
-    if (r < ntk) { src = a.k; dst = a.kT; valid = a.valid_kv; t = r; ntiles = ntk; }
-    else if (r < ntk + ntq) { src = a.q; dst = a.qT; valid = a.valid_q; t = r - ntk; ntiles = ntq; }
-    else { src = a.dout; dst = a.doT; valid = a.valid_q; t = r - ntk - ntq; ntiles = ntq; }
-    const uint16_t* sp = src.p + b * src.sb + h * src.sh;
     // Rows of dS sum to zero in exact arithmetic, so dS K = dS (K - c) for any vector c; when O and
     // Stats come from a forward of other precision the row sum is small but not zero, and dS K
     // would multiply it by the keys' common offset.  The dQ pass therefore also sums every row of
     // dS (the rounded values the matrix instruction takes) and subtracts rowsum * c at the end,
     // with c close to the mean key: the mean of 64 keys spread evenly over the valid ones, computed
-    // here once per head.  (Centring the K^T copy itself would round K - c to bf16 a second time.)
-    if (is_k && t == 0) {
-        float part[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    // here once per head.  (Centring K itself would round K - c to bf16 a second time.)
+    const uint16_t* sp = a.k.p + b * a.k.sb + h * a.k.sh + col;
+    float part[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-        for (int i = 0; i < 64 * CPR / 256; i++) {
-            const int c = i * 256 + tid;
-            const int smp = c / CPR, col = (c % CPR) * 8;
-            const int64_t key = ((int64_t)smp * valid) >> 6;
-            const u32x4 w = *reinterpret_cast<const u32x4*>(sp + key * src.sn + col);
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                part[2 * e] += __uint_as_float(w[e] << 16);
-                part[2 * e + 1] += __uint_as_float(w[e] & 0xFFFF0000u);
-            }
-        }
-        // thread tid holds samples {tid / CPR + k * (256 / CPR)} of chunk tid % CPR: reduce over tid / CPR
-        float* red = reinterpret_cast<float*>(tile);                 // [256 / CPR][D]
-#pragma unroll
-        for (int e = 0; e < 8; e++) red[(tid / CPR) * D + (tid % CPR) * 8 + e] = part[e];
-        __syncthreads();
-        if (tid < D) {
-            float sum = 0.0f;
-            for (int g = 0; g < 256 / CPR; g++) sum += red[g * D + tid];
-            a.kcen[(int64_t)bh * D + tid] = sum * (1.0f / 64.0f);
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 64 * CPR / 256; i++) {
-        const int c = i * 256 + tid;
-        const int row = c / CPR, col = (c % CPR) * 8;
-        u32x4 w = {0u, 0u, 0u, 0u};
-        if (t * 64 + row < valid) w = *reinterpret_cast<const u32x4*>(sp + (int64_t)(t * 64 + row) * src.sn + col);
-        *reinterpret_cast<u32x4*>(&tile[row * LROW + col]) = w;
-    }
-    __syncthreads();
-    uint16_t* out = dst + ((int64_t)bh * ntiles + t) * (int64_t)(D * 64);
-#pragma unroll
-    for (int i = 0; i < D * 8 / 256; i++) {
-        const int c = i * 256 + tid;
-        const int d = c >> 3, s0 = (c & 7) * 8;
-        uint32_t w[4];
+    for (int i = 0; i < 64 / RPP; i++) {
+        const int64_t key = ((int64_t)(i * RPP + tid / CPR) * a.valid_kv) >> 6;
+        const u32x4 w = *reinterpret_cast<const u32x4*>(sp + key * a.k.sn);
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            const uint32_t lo = tile[row_of_slot(s0 + 2 * e) * LROW + d];
-            const uint32_t hi = tile[row_of_slot(s0 + 2 * e + 1) * LROW + d];
-            w[e] = lo | (hi << 16);
+            part[2 * e] += __uint_as_float(w[e] << 16);
+            part[2 * e + 1] += __uint_as_float(w[e] & 0xFFFF0000u);
         }
-        *reinterpret_cast<u32x4*>(out + d * 64 + s0) = u32x4{w[0], w[1], w[2], w[3]};
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e++) red[(tid / CPR) * D + col + e] = part[e];
+    __syncthreads();
+    if (tid < D) {
+        float sum = 0.0f;
+        for (int g = 0; g < RPP; g++) sum += red[g * D + tid];
+        a.kcen[(int64_t)bh * D + tid] = sum * (1.0f / 64.0f);
     }
 }
 
@@ -206,28 +219,27 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(BwdArgs a) {
 // ---------------------------------------------------------------------------------------------
 template <int D, int PASS>
 struct PassLds {
-    static constexpr int TILE_BYTES = 64 * D * 2;
-    static constexpr int NTR = PASS == 0 ? 1 : 2;
-    uint8_t nat[2][2][TILE_BYTES];
-    uint8_t tr[2][NTR][TILE_BYTES];
-    float row[2][2][64];
+    static constexpr int TILE_BYTES = 64 * D * 2, SLOT = 2 * TILE_BYTES, SLOTS = 3;
+    static constexpr int ROW_BYTES = PASS == 1 ? 2048 : 0;                   // [slot][lse | Delta][64], PASS 1 only
+    // The ring, and during the prologue the owner rows (2 x 32 rows per wave) behind its first slot.
+    static constexpr int OWNER = ROW_BYTES + SLOT;
+    static constexpr int BYTES = OWNER + 8 * 2 * 64 * D;
+    static_assert(BYTES >= ROW_BYTES + SLOTS * SLOT, "the ring must fit");
 };
 
-template <int D, int PASS, int NW>
-__device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, PassLds<D, PASS>& L, int block) {
+template <int D, int PASS>
+__device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, uint8_t* smem, int block) {
+    using L = PassLds<D, PASS>;
+    constexpr int NW = 8;
     constexpr int XROWS = NW * 32;                  // owner rows per workgroup
-    constexpr int CPR = D / 8;                      // 16-byte chunks per natural row
-    constexpr int TILE_BYTES = 64 * D * 2;          // natural and transposed tiles have the same size
+    constexpr int CPR = D / 8;                      // 16-byte chunks per row
+    constexpr int TILE_BYTES = L::TILE_BYTES;
     constexpr int RUNS = TILE_BYTES / 1024;         // 1 KiB copies per tile
     constexpr int RPW = RUNS / NW;                  // per wave
     constexpr int KS = D / 16;                      // matrix-instruction steps over the head dim
     constexpr int DB = D / 32;                      // 32-channel output blocks
     constexpr int NTR = PASS == 0 ? 1 : 2;          // transposed operands per tile
     static_assert(RUNS % NW == 0, "tile copies must divide over the waves");
-
-    auto& lds_nat = L.nat;
-    auto& lds_tr = L.tr;
-    auto& lds_row = L.row;
 
     const int Nx = PASS == 0 ? a.Nq : a.Nkv;
     const int valid_x = PASS == 0 ? a.valid_q : a.valid_kv;
@@ -239,24 +251,55 @@ __device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, PassLds<D, PASS>
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, half = lane >> 5;
-    const int x = xt * XROWS + wave * 32 + l32;
+    const int x0 = xt * XROWS + wave * 32;          // this wave's first row
+    const int x = x0 + l32;
+
+    // y side
+    const View& yv1 = PASS == 0 ? a.k : a.q;
+    const View& yv2 = PASS == 0 ? a.v : a.dout;
+    const uint8_t* y1 = reinterpret_cast<const uint8_t*>(yv1.p + b * yv1.sb + h * yv1.sh);
+    const uint8_t* y2 = reinterpret_cast<const uint8_t*>(yv2.p + b * yv2.sb + h * yv2.sh);
+    const uint8_t* rows_l = reinterpret_cast<const uint8_t*>(a.lse2 + (int64_t)bh * a.nq_pad);
+    const uint8_t* rows_d = reinterpret_cast<const uint8_t*>(a.delta + (int64_t)bh * a.nq_pad);
+    // owners that are all padding have nothing to compute: they only store zeros
+    const int ntiles = xt * XROWS < valid_x ? (valid_y + 63) / 64 : 0;
+
+    // per-lane pieces of the copy addresses: run i of this wave covers physical chunks
+    // (i*8 + wave)*64 + lane of a tile
+    int nat_row[RPW], nat_col[RPW];
+#pragma unroll
+    for (int i = 0; i < RPW; i++) {
+        const int P = (i * NW + wave) * 64 + lane;
+        nat_row[i] = P / CPR;
+        nat_col[i] = nat_pos<CPR>(P / CPR, P % CPR) * 16;          // the XOR is its own inverse
+    }
+    const uint32_t row_base = lds_addr(smem), nat_base = row_base + L::ROW_BYTES;
+    const uint32_t ys1 = (uint32_t)(yv1.sn * 2), ys2 = (uint32_t)(yv2.sn * 2);
+    auto copy_tile = [&](int t, int slot) {
+        if constexpr (PASS == 1) {                  // (first, so that a wait for the 2 * RPW copies below covers it)
+            if (wave == 0) dma4(rows_l + (int64_t)t * 256, lane * 4, __builtin_amdgcn_readfirstlane(row_base + (slot * 2 + 0) * 256));
+            if (wave == 1) dma4(rows_d + (int64_t)t * 256, lane * 4, __builtin_amdgcn_readfirstlane(row_base + (slot * 2 + 1) * 256));
+        }
+#pragma unroll
+        for (int i = 0; i < RPW; i++) {
+            const uint32_t row = (uint32_t)min(t * 64 + nat_row[i], valid_y - 1);      // padding repeats the last valid row
+            const uint32_t dst = (uint32_t)((i * NW + wave) * 1024) + nat_base + slot * L::SLOT;
+            dma16(y1, row * ys1 + nat_col[i], __builtin_amdgcn_readfirstlane(dst));
+            dma16(y2, row * ys2 + nat_col[i], __builtin_amdgcn_readfirstlane(dst + TILE_BYTES));
+        }
+    };
+
+    // owner side: two resident row blocks (B operands: column = owner row, k = head channel).
     // (rows past the valid length are never read: what the caller keeps there — NaNs included — must
     // not reach a valid row's gradient through a product with a zero probability)
-    const int xc = min(x, max(valid_x, 1) - 1);
-
-    // owner side: two resident row blocks (B operands: column = owner row, k = head channel)
     const View& xv1 = PASS == 0 ? a.q : a.k;
     const View& xv2 = PASS == 0 ? a.dout : a.v;
     v4i b1[KS], b2[KS];
-    {
-        const uint16_t* p1 = xv1.p + b * xv1.sb + h * xv1.sh + (int64_t)xc * xv1.sn + half * 8;
-        const uint16_t* p2 = xv2.p + b * xv2.sb + h * xv2.sh + (int64_t)xc * xv2.sn + half * 8;
-#pragma unroll
-        for (int s = 0; s < KS; s++) {
-            b1[s] = *reinterpret_cast<const v4i*>(p1 + s * 16);
-            b2[s] = *reinterpret_cast<const v4i*>(p2 + s * 16);
-        }
-    }
+    const int last_x = max(valid_x, 1) - 1;
+    const uint32_t own = L::OWNER + wave * 2 * 64 * D;
+    rows_in<D>(xv1.p + b * xv1.sb + h * xv1.sh, xv1.sn, x0, last_x, row_base + own, lane);
+    rows_in<D>(xv2.p + b * xv2.sb + h * xv2.sh, xv2.sn, x0, last_x, row_base + own + 64 * D, lane);
+    if (ntiles > 0) copy_tile(0, 0);
     float lse_x = 0.0f, delta_x = 0.0f;
     float ds_rowsum = 0.0f;                         // dQ pass: sum over the keys of this lane's dS values
     if constexpr (PASS == 0) {
@@ -268,65 +311,25 @@ __device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, PassLds<D, PASS>
     // first use of its result, and such a wait inside the loop would also wait for the tile copies
     // that are meant to stay in flight (they share the counter).  Using the values here puts the
     // waits here.
+    dma_wait<0>();
+#pragma unroll
+    for (int s = 0; s < KS; s++) {
+        b1[s] = *reinterpret_cast<const v4i*>(smem + own + nat_off<CPR>(l32, s * 2 + half));
+        b2[s] = *reinterpret_cast<const v4i*>(smem + own + 64 * D + nat_off<CPR>(l32, s * 2 + half));
+    }
 #pragma unroll
     for (int s = 0; s < KS; s++) asm volatile("" : "+v"(b1[s]), "+v"(b2[s]));
     asm volatile("" : "+v"(lse_x), "+v"(delta_x));
-    dma_wait_all();
-
-    // y side
-    const View& yv1 = PASS == 0 ? a.k : a.q;
-    const View& yv2 = PASS == 0 ? a.v : a.dout;
-    const uint8_t* y1 = reinterpret_cast<const uint8_t*>(yv1.p + b * yv1.sb + h * yv1.sh);
-    const uint8_t* y2 = reinterpret_cast<const uint8_t*>(yv2.p + b * yv2.sb + h * yv2.sh);
-    const int64_t ny_pad = PASS == 0 ? a.nkv_pad : a.nq_pad;
-    const uint8_t* t1 = reinterpret_cast<const uint8_t*>(PASS == 0 ? a.kT : a.qT) + (int64_t)bh * ny_pad * D * 2;
-    const uint8_t* t2 = reinterpret_cast<const uint8_t*>(a.doT) + (int64_t)bh * ny_pad * D * 2;
-    const uint8_t* rows_l = reinterpret_cast<const uint8_t*>(a.lse2 + (int64_t)bh * a.nq_pad);
-    const uint8_t* rows_d = reinterpret_cast<const uint8_t*>(a.delta + (int64_t)bh * a.nq_pad);
-    // owners that are all padding have nothing to compute: they only store zeros
-    const int ntiles = xt * XROWS < valid_x ? (valid_y + 63) / 64 : 0;
-
-    // per-lane pieces of the copy addresses: run i of this wave covers physical chunks
-    // (i*4 + wave)*64 + lane of a tile
-    int nat_row[RPW], nat_col[RPW];
-    uint32_t tr_src[RPW];
-#pragma unroll
-    for (int i = 0; i < RPW; i++) {
-        const int P = (i * NW + wave) * 64 + lane;
-        const int row = P / CPR, pos = P % CPR;
-        nat_row[i] = row;
-        nat_col[i] = nat_pos<CPR>(row, pos) * 16;          // the XOR is its own inverse
-        tr_src[i] = (uint32_t)tr_off(P);
-    }
-    const uint32_t nat_base = lds_addr(&lds_nat[0][0][0]), tr_base = lds_addr(&lds_tr[0][0][0]);
-    const uint32_t row_base = lds_addr(&lds_row[0][0][0]);
-    const uint32_t ys1 = (uint32_t)(yv1.sn * 2), ys2 = (uint32_t)(yv2.sn * 2);
-    auto copy_tile = [&](int t, int stage) {
-#pragma unroll
-        for (int i = 0; i < RPW; i++) {
-            const uint32_t row = (uint32_t)min(t * 64 + nat_row[i], valid_y - 1);      // padding repeats the last valid row
-            const uint32_t dst = (uint32_t)((i * NW + wave) * 1024);
-            dma16(y1, row * ys1 + nat_col[i], __builtin_amdgcn_readfirstlane(nat_base + (stage * 2 + 0) * TILE_BYTES + dst));
-            dma16(y2, row * ys2 + nat_col[i], __builtin_amdgcn_readfirstlane(nat_base + (stage * 2 + 1) * TILE_BYTES + dst));
-            dma16(t1 + (int64_t)t * TILE_BYTES, tr_src[i], __builtin_amdgcn_readfirstlane(tr_base + (stage * NTR + 0) * TILE_BYTES + dst));
-            if constexpr (PASS == 1)
-                dma16(t2 + (int64_t)t * TILE_BYTES, tr_src[i], __builtin_amdgcn_readfirstlane(tr_base + (stage * NTR + 1) * TILE_BYTES + dst));
-        }
-        if constexpr (PASS == 1) {
-            if (wave == 0) dma4(rows_l + (int64_t)t * 256, lane * 4, __builtin_amdgcn_readfirstlane(row_base + (stage * 2 + 0) * 256));
-            if (wave == 1) dma4(rows_d + (int64_t)t * 256, lane * 4, __builtin_amdgcn_readfirstlane(row_base + (stage * 2 + 1) * 256));
-        }
-    };
+    __syncthreads();                     // the owner rows' LDS becomes the ring's second and third slot
+    if (ntiles > 1) copy_tile(1, 1);
 
     // fragment offsets inside a tile
-    int nat_frag[2][KS];                 // [32-row block][k-step]
+    int nat_frag[KS];                    // [k-step]; 32-row blocks are + 64 * D bytes
 #pragma unroll
-    for (int blk = 0; blk < 2; blk++)
+    for (int s = 0; s < KS; s++) nat_frag[s] = nat_off<CPR>(l32, s * 2 + half);
+    int tr_frag[DB][2];                  // [32-channel block][rows 0-7 | 8-15]; 16-row blocks are + 32 * D bytes
 #pragma unroll
-        for (int s = 0; s < KS; s++) nat_frag[blk][s] = nat_off<CPR>(blk * 32 + l32, s * 2 + half);
-    int tr_frag[4];                      // [k-step over the 64 slots]; 32-channel blocks are +32*128 bytes
-#pragma unroll
-    for (int j = 0; j < 4; j++) tr_frag[j] = tr_off(l32 * 8 + j * 2 + half);
+    for (int d = 0; d < DB; d++) tr_frag[d][0] = tr_frag_off<CPR>(lane, 0, d), tr_frag[d][1] = tr_frag_off<CPR>(lane, 8, d);
 
     v16f acc1[DB], acc2[PASS == 1 ? DB : 1];
 #pragma unroll
@@ -338,16 +341,10 @@ __device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, PassLds<D, PASS>
         }
     const float c = a.scale * kLog2e;
 
-    if (ntiles > 0) copy_tile(0, 0);
-    for (int t = 0; t < ntiles; t++) {
-        const int stage = t & 1;
-        dma_wait_all();
-        __syncthreads();                 // tile t is visible; every wave is done with the other stage
-        if (t + 1 < ntiles) copy_tile(t + 1, stage ^ 1);
-        const uint8_t* n1 = &lds_nat[stage][0][0];
-        const uint8_t* n2 = &lds_nat[stage][1][0];
-        const uint8_t* r1 = &lds_tr[stage][0][0];
-        const uint8_t* r2 = &lds_tr[stage][NTR - 1][0];
+    auto tile = [&](int t, int slot) {
+        const uint8_t* n1 = smem + L::ROW_BYTES + slot * L::SLOT;
+        const uint8_t* n2 = n1 + TILE_BYTES;
+        const uint8_t* rows = smem + slot * 512;
         // Two 32-row blocks per tile, software-pipelined so that the vector work of one block is
         // issued between the matrix instructions of the other:
         //   scores(0) | scores(1) + exponentials(0) | products(0) + exponentials(1) | products(1)
@@ -362,8 +359,8 @@ __device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, PassLds<D, PASS>
         // fragments of step ks + 1 are requested before the products of step ks are issued.
         v4i f1[2], f2[2];
         auto scores_load = [&](int blk, int ks) {
-            f1[ks & 1] = *reinterpret_cast<const v4i*>(n1 + nat_frag[blk][ks]);
-            f2[ks & 1] = *reinterpret_cast<const v4i*>(n2 + nat_frag[blk][ks]);
+            f1[ks & 1] = *reinterpret_cast<const v4i*>(n1 + nat_frag[ks] + blk * 64 * D);
+            f2[ks & 1] = *reinterpret_cast<const v4i*>(n2 + nat_frag[ks] + blk * 64 * D);
         };
         auto scores_step = [&](int blk, int ks) {
             if (ks + 1 < KS) scores_load(blk, ks + 1);
@@ -378,8 +375,8 @@ __device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, PassLds<D, PASS>
 #pragma unroll
                     for (int e = 0; e < 4; e++) lse[e] = lse_x, dl[e] = delta_x;
                 } else {
-                    const v4f vl = *reinterpret_cast<const v4f*>(&lds_row[stage][0][blk * 32 + g * 8 + half * 4]);
-                    const v4f vd = *reinterpret_cast<const v4f*>(&lds_row[stage][1][blk * 32 + g * 8 + half * 4]);
+                    const v4f vl = *reinterpret_cast<const v4f*>(rows + (blk * 32 + g * 8 + half * 4) * 4);
+                    const v4f vd = *reinterpret_cast<const v4f*>(rows + 256 + (blk * 32 + g * 8 + half * 4) * 4);
 #pragma unroll
                     for (int e = 0; e < 4; e++) lse[e] = vl[e], dl[e] = vd[e];
                 }
@@ -406,14 +403,14 @@ __device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, PassLds<D, PASS>
         constexpr int ACC_M = 2 * DB * NTR;
         auto acc_step = [&](int blk, int m) {
             const int which = m / (2 * DB), j2 = (m / DB) & 1, d = m % DB;
-            const int j = blk * 2 + j2;
+            const int rows16 = (blk * 2 + j2) * 32 * D;
             if (which == 0) {
                 const v4i sb = {(int)sp[blk][j2 * 4], (int)sp[blk][j2 * 4 + 1], (int)sp[blk][j2 * 4 + 2], (int)sp[blk][j2 * 4 + 3]};
-                const v4i fa = *reinterpret_cast<const v4i*>(r1 + tr_frag[j] + d * 32 * 128);
+                const v4i fa = tr_read(n1 + tr_frag[d][0] + rows16, n1 + tr_frag[d][1] + rows16);
                 acc1[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, fa), __builtin_bit_cast(v8bf, sb), acc1[d], 0, 0, 0);
             } else if constexpr (PASS == 1) {
                 const v4i pb = {(int)pp[blk][j2 * 4], (int)pp[blk][j2 * 4 + 1], (int)pp[blk][j2 * 4 + 2], (int)pp[blk][j2 * 4 + 3]};
-                const v4i fa = *reinterpret_cast<const v4i*>(r2 + tr_frag[j] + d * 32 * 128);
+                const v4i fa = tr_read(n2 + tr_frag[d][0] + rows16, n2 + tr_frag[d][1] + rows16);
                 acc2[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, fa), __builtin_bit_cast(v8bf, pb), acc2[d], 0, 0, 0);
             }
         };
@@ -442,49 +439,57 @@ __device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, PassLds<D, PASS>
         }
 #pragma unroll
         for (int m = 0; m < ACC_M; m++) acc_step(1, m);
+    };
+
+    // Tile t sits in slot t % 3 and was requested two iterations earlier: the wait at the top leaves the
+    // copies of tile t + 1 in flight.
+    int slot = 0;
+    for (int t = 0; t < ntiles; t++) {
+        if (t + 1 < ntiles) dma_wait<2 * RPW>();
+        else dma_wait<0>();
+        __syncthreads();                 // tile t is visible; every wave is done with the slot of tile t - 1
+        if (t + 2 < ntiles) copy_tile(t + 2, slot == 0 ? 2 : slot - 1);
+        tile(t, slot);
+        slot = slot == 2 ? 0 : slot + 1;
     }
 
     // ---- epilogue: rows of valid owners get their gradient, padding rows zeros -----------------
-    if (x < Nx) {
-        const bool live = x < valid_x;
-        uint16_t* o1 = (PASS == 0 ? a.dq : a.dk) + b * (PASS == 0 ? a.dq_sb : a.dk_sb) + h * (PASS == 0 ? a.dq_sh : a.dk_sh) +
-                       (int64_t)x * (PASS == 0 ? a.dq_sn : a.dk_sn);
-        uint16_t* o2 = PASS == 1 ? a.dv + b * a.dv_sb + h * a.dv_sh + (int64_t)x * a.dv_sn : nullptr;
-        // dQ = scale * (dS K - rowsum(dS) c): the two half-waves hold different keys of the same query
-        float rs = 0.0f;
-        if constexpr (PASS == 0) {
-            const v2u r = __builtin_amdgcn_permlane32_swap(__float_as_uint(ds_rowsum), __float_as_uint(ds_rowsum), false, false);
-            rs = __uint_as_float(r.x) + __uint_as_float(r.y);
+    // `slot` and the one after it have no readers any more (the last tile sits in the one before).
+    if (ntiles == 0) __syncthreads();    // (the owner rows of the other waves are still on their way then)
+    uint8_t* os = smem + L::ROW_BYTES + (slot + (wave >> 2) >= 3 ? 0 : slot + (wave >> 2)) * L::SLOT + (wave & 3) * 64 * D;
+    const bool live = x < valid_x;
+    // dQ = scale * (dS K - rowsum(dS) c): the two half-waves hold different keys of the same query
+    float rs = 0.0f;
+    if constexpr (PASS == 0) {
+        const v2u r = __builtin_amdgcn_permlane32_swap(__float_as_uint(ds_rowsum), __float_as_uint(ds_rowsum), false, false);
+        rs = __uint_as_float(r.x) + __uint_as_float(r.y);
+    }
+    const float* cen = a.kcen + (int64_t)bh * D;
+#pragma unroll
+    for (int d = 0; d < DB; d++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            float y[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) y[e] = acc1[d][g * 4 + e];
+            if constexpr (PASS == 0) {
+                const v4f c4 = *reinterpret_cast<const v4f*>(cen + d * 32 + g * 8 + half * 4);
+#pragma unroll
+                for (int e = 0; e < 4; e++) y[e] -= rs * c4[e];
+            }
+            const u32x2 w = {pack_bf16(y[0] * a.scale, y[1] * a.scale), pack_bf16(y[2] * a.scale, y[3] * a.scale)};
+            row_put<D>(os, l32, half, d, g, live ? w : u32x2{0u, 0u});
         }
-        const float* cen = a.kcen + (int64_t)bh * D;
+    rows_out<D>(os, PASS == 0 ? a.dq + b * a.dq_sb + h * a.dq_sh : a.dk + b * a.dk_sb + h * a.dk_sh, PASS == 0 ? a.dq_sn : a.dk_sn, x0, Nx, lane);
+    if constexpr (PASS == 1) {
 #pragma unroll
         for (int d = 0; d < DB; d++)
 #pragma unroll
             for (int g = 0; g < 4; g++) {
-                const int ch = d * 32 + g * 8 + half * 4;
-                u32x2 w = {0u, 0u};
-                if (live) {
-                    float y[4];
-#pragma unroll
-                    for (int e = 0; e < 4; e++) y[e] = acc1[d][g * 4 + e];
-                    if constexpr (PASS == 0) {
-                        const v4f c4 = *reinterpret_cast<const v4f*>(cen + ch);
-#pragma unroll
-                        for (int e = 0; e < 4; e++) y[e] -= rs * c4[e];
-                    }
-                    w.x = pack_bf16(y[0] * a.scale, y[1] * a.scale);
-                    w.y = pack_bf16(y[2] * a.scale, y[3] * a.scale);
-                }
-                *reinterpret_cast<u32x2*>(o1 + ch) = w;
-                if constexpr (PASS == 1) {
-                    u32x2 u = {0u, 0u};
-                    if (live) {
-                        u.x = pack_bf16(acc2[d][g * 4], acc2[d][g * 4 + 1]);
-                        u.y = pack_bf16(acc2[d][g * 4 + 2], acc2[d][g * 4 + 3]);
-                    }
-                    *reinterpret_cast<u32x2*>(o2 + ch) = u;
-                }
+                const u32x2 u = {pack_bf16(acc2[d][g * 4], acc2[d][g * 4 + 1]), pack_bf16(acc2[d][g * 4 + 2], acc2[d][g * 4 + 3])};
+                row_put<D>(os, l32, half, d, g, live ? u : u32x2{0u, 0u});
             }
+        rows_out<D>(os, a.dv + b * a.dv_sb + h * a.dv_sh, a.dv_sn, x0, Nx, lane);
     }
 }
 
@@ -494,31 +499,31 @@ __device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, PassLds<D, PASS>
 // shares 32 keys:
 //   the P wave keeps the keys' K rows and the dV accumulators:  T = Q K^T -> P = exp2(cT - lse) -> dV += P^T dO
 //   the S wave keeps the keys' V rows and the dK accumulators:  G = dO V^T, dS = P (G - Delta)  -> dK += dS^T Q
-// No product is computed twice and every fragment is read from LDS once.  P goes from the P wave
+// No product is computed twice.  P goes from the P wave
 // to the S wave through LDS, in the lane layout of the accumulator, which both waves share — as
 // fp16 (11 significant bits, truncated): dS is P times a difference and is itself rounded to bf16,
-// and a bf16 P underneath would add a second error of the same size to every term of dK.  The S wave runs one query tile behind the P wave, so the hand-over is ordered by the
-// workgroup barrier that every tile has anyway; the tiles the S wave reads (dO, Q^T, Delta) are
-// copied one iteration later than the P wave's (Q, dO^T, lse), which keeps every ring at two slots.
-// There is room for one hand-over slot only (160 KiB of LDS): before the P wave overwrites it, it
-// checks a per-pair counter that the S wave advances as soon as it holds the previous tile's P in
-// registers — at the top of the iteration, half a tile before the P wave gets there.
+// and a bf16 P underneath would add a second error of the same size to every term of dK.  The S wave
+// runs one query tile behind the P wave, so the hand-over is ordered by the
+// workgroup barrier that every tile has anyway: two slots of P, three of tiles (tile t is copied in
+// iteration t - 1, read by the P waves in t and by the S waves in t + 1).
 // ---------------------------------------------------------------------------------------------
 template <int D>
 struct DkDvLds {
-    static constexpr int TILE_BYTES = 64 * D * 2;
-    uint8_t nat[2][2][TILE_BYTES];                  // [stage][0: Q | 1: dO], natural rows
-    uint8_t tr[2][2][TILE_BYTES];                   // [stage][0: Q^T | 1: dO^T]
-    u32x4 p[4][2][2][64];                           // [pair][32-row block][values 0-7 | 8-15][lane], fp16 pairs
-    float row[2][2][64];                            // [stage][0: lse | 1: Delta]
-    int taken[4];                                   // per pair: the S wave holds P of every tile below this
+    static constexpr int TILE_BYTES = 64 * D * 2, SLOT = 2 * TILE_BYTES, SLOTS = 3;
+    static constexpr int ROW_BYTES = 2048;          // [slot][lse | Delta][64]
+    static constexpr int P_BYTES = 4 * 2 * 2 * 64 * 16;      // [pair][32-row block][values 0-7 | 8-15][lane], fp16 pairs
+    static constexpr int RING = ROW_BYTES + 2 * P_BYTES;
+    static constexpr int OWNER = RING + SLOT;       // during the prologue: 32 owner rows per wave
+    static constexpr int BYTES = RING + SLOTS * SLOT;
+    static_assert(8 * 64 * D <= 2 * SLOT, "the owner rows must fit behind the first slot");
 };
 
 template <int D, int ROLE>
-__device__ __forceinline__ void dkdv_role(const BwdArgs& a, DkDvLds<D>& L, int bh, int xt, int wave, int lane) {
+__device__ __forceinline__ void dkdv_role(const BwdArgs& a, uint8_t* smem, int bh, int xt, int wave, int lane) {
+    using L = DkDvLds<D>;
     constexpr int NW = 8;
     constexpr int CPR = D / 8;
-    constexpr int TILE_BYTES = 64 * D * 2;
+    constexpr int TILE_BYTES = L::TILE_BYTES;
     constexpr int RUNS = TILE_BYTES / 1024;
     constexpr int RPW = RUNS / NW;
     constexpr int KS = D / 16;
@@ -527,73 +532,53 @@ __device__ __forceinline__ void dkdv_role(const BwdArgs& a, DkDvLds<D>& L, int b
     const int b = bh / a.H, h = bh % a.H;
     const int pair = wave & 3;
     const int l32 = lane & 31, half = lane >> 5;
-    const int x = xt * 128 + pair * 32 + l32;
-    const int xc = min(x, max(a.valid_kv, 1) - 1);
-
-    // owner side: the P wave keeps K rows, the S wave V rows (B operands: column = key, k = head channel)
-    const View& xv = ROLE == 0 ? a.k : a.v;
-    v4i bx[KS];
-    {
-        const uint16_t* px = xv.p + b * xv.sb + h * xv.sh + (int64_t)xc * xv.sn + half * 8;
-#pragma unroll
-        for (int s = 0; s < KS; s++) bx[s] = *reinterpret_cast<const v4i*>(px + s * 16);
-    }
-#pragma unroll
-    for (int s = 0; s < KS; s++) asm volatile("" : "+v"(bx[s]));     // the wait for these loads stays out of the loop
-    dma_wait_all();
+    const int x0 = xt * 128 + pair * 32, x = x0 + l32;
 
     const uint8_t* yq = reinterpret_cast<const uint8_t*>(a.q.p + b * a.q.sb + h * a.q.sh);
     const uint8_t* yg = reinterpret_cast<const uint8_t*>(a.dout.p + b * a.dout.sb + h * a.dout.sh);
-    const uint8_t* tq = reinterpret_cast<const uint8_t*>(a.qT) + (int64_t)bh * a.nq_pad * D * 2;
-    const uint8_t* tg = reinterpret_cast<const uint8_t*>(a.doT) + (int64_t)bh * a.nq_pad * D * 2;
     const uint8_t* rows_l = reinterpret_cast<const uint8_t*>(a.lse2 + (int64_t)bh * a.nq_pad);
     const uint8_t* rows_d = reinterpret_cast<const uint8_t*>(a.delta + (int64_t)bh * a.nq_pad);
     const int ntiles = xt * 128 < a.valid_kv ? (a.valid_q + 63) / 64 : 0;
 
     int nat_row[RPW], nat_col[RPW];
-    uint32_t tr_src[RPW];
 #pragma unroll
     for (int i = 0; i < RPW; i++) {
         const int P = (i * NW + wave) * 64 + lane;
-        const int row = P / CPR, pos = P % CPR;
-        nat_row[i] = row;
-        nat_col[i] = nat_pos<CPR>(row, pos) * 16;
-        tr_src[i] = (uint32_t)tr_off(P);
+        nat_row[i] = P / CPR;
+        nat_col[i] = nat_pos<CPR>(P / CPR, P % CPR) * 16;
     }
-    const uint32_t nat_base = lds_addr(&L.nat[0][0][0]), tr_base = lds_addr(&L.tr[0][0][0]);
-    const uint32_t row_base = lds_addr(&L.row[0][0][0]);
+    const uint32_t row_base = lds_addr(smem), nat_base = row_base + L::RING;
     const uint32_t sq = (uint32_t)(a.q.sn * 2), sg = (uint32_t)(a.dout.sn * 2);
-    // what the P wave reads of query tile t: Q rows, dO^T, lse
-    auto copy_for_p = [&](int t, int stage) {
+    auto copy_tile = [&](int t, int slot) {
 #pragma unroll
         for (int i = 0; i < RPW; i++) {
             const uint32_t row = (uint32_t)min(t * 64 + nat_row[i], a.valid_q - 1);
-            const uint32_t dst = (uint32_t)((i * NW + wave) * 1024);
-            dma16(yq, row * sq + nat_col[i], __builtin_amdgcn_readfirstlane(nat_base + (stage * 2 + 0) * TILE_BYTES + dst));
-            dma16(tg + (int64_t)t * TILE_BYTES, tr_src[i], __builtin_amdgcn_readfirstlane(tr_base + (stage * 2 + 1) * TILE_BYTES + dst));
+            const uint32_t dst = (uint32_t)((i * NW + wave) * 1024) + nat_base + slot * L::SLOT;
+            dma16(yq, row * sq + nat_col[i], __builtin_amdgcn_readfirstlane(dst));
+            dma16(yg, row * sg + nat_col[i], __builtin_amdgcn_readfirstlane(dst + TILE_BYTES));
         }
-        if (wave == 0) dma4(rows_l + (int64_t)t * 256, lane * 4, __builtin_amdgcn_readfirstlane(row_base + (stage * 2 + 0) * 256));
-    };
-    // what the S wave reads of query tile t: dO rows, Q^T, Delta
-    auto copy_for_s = [&](int t, int stage) {
-#pragma unroll
-        for (int i = 0; i < RPW; i++) {
-            const uint32_t row = (uint32_t)min(t * 64 + nat_row[i], a.valid_q - 1);
-            const uint32_t dst = (uint32_t)((i * NW + wave) * 1024);
-            dma16(yg, row * sg + nat_col[i], __builtin_amdgcn_readfirstlane(nat_base + (stage * 2 + 1) * TILE_BYTES + dst));
-            dma16(tq + (int64_t)t * TILE_BYTES, tr_src[i], __builtin_amdgcn_readfirstlane(tr_base + (stage * 2 + 0) * TILE_BYTES + dst));
-        }
-        if (wave == 1) dma4(rows_d + (int64_t)t * 256, lane * 4, __builtin_amdgcn_readfirstlane(row_base + (stage * 2 + 1) * 256));
+        if (wave == 0) dma4(rows_l + (int64_t)t * 256, lane * 4, __builtin_amdgcn_readfirstlane(row_base + (slot * 2 + 0) * 256));
+        if (wave == 1) dma4(rows_d + (int64_t)t * 256, lane * 4, __builtin_amdgcn_readfirstlane(row_base + (slot * 2 + 1) * 256));
     };
 
-    int nat_frag[2][KS];
+    // owner side: the P wave keeps K rows, the S wave V rows (B operands: column = key, k = head channel)
+    const View& xv = ROLE == 0 ? a.k : a.v;
+    v4i bx[KS];
+    const uint32_t own = L::OWNER + wave * 64 * D;
+    rows_in<D>(xv.p + b * xv.sb + h * xv.sh, xv.sn, x0, max(a.valid_kv, 1) - 1, row_base + own, lane);
+    if (ntiles > 0) copy_tile(0, 0);
+    dma_wait<0>();
 #pragma unroll
-    for (int blk = 0; blk < 2; blk++)
+    for (int s = 0; s < KS; s++) bx[s] = *reinterpret_cast<const v4i*>(smem + own + nat_off<CPR>(l32, s * 2 + half));
 #pragma unroll
-        for (int s = 0; s < KS; s++) nat_frag[blk][s] = nat_off<CPR>(blk * 32 + l32, s * 2 + half);
-    int tr_frag[4];
+    for (int s = 0; s < KS; s++) asm volatile("" : "+v"(bx[s]));     // the wait for these stays out of the loop
+
+    int nat_frag[KS];
 #pragma unroll
-    for (int j = 0; j < 4; j++) tr_frag[j] = tr_off(l32 * 8 + j * 2 + half);
+    for (int s = 0; s < KS; s++) nat_frag[s] = nat_off<CPR>(l32, s * 2 + half);
+    int tr_frag[DB][2];
+#pragma unroll
+    for (int d = 0; d < DB; d++) tr_frag[d][0] = tr_frag_off<CPR>(lane, 0, d), tr_frag[d][1] = tr_frag_off<CPR>(lane, 8, d);
 
     v16f acc[DB];
 #pragma unroll
@@ -601,39 +586,33 @@ __device__ __forceinline__ void dkdv_role(const BwdArgs& a, DkDvLds<D>& L, int b
 #pragma unroll
         for (int i = 0; i < 16; i++) acc[d][i] = 0.0f;
     const float c = a.scale * kLog2e;
-    // (an LDS pointer by type: through a generic one the accesses become flat instructions, whose waits
-    // also wait for the tile copies in flight)
-    volatile __attribute__((address_space(3))) int* taken = (volatile __attribute__((address_space(3))) int*)&L.taken[pair];
+    // this wave's part of the two hand-over slots
+    u32x4* hand = reinterpret_cast<u32x4*>(smem + L::ROW_BYTES) + pair * 256 + lane;
 
-    if (ntiles > 0) copy_for_p(0, 0);
     // iteration `it`: the P wave works on query tile it, the S wave on tile it - 1
+    int slot = 0;                        // it % 3
     for (int it = 0; ntiles > 0 && it <= ntiles; it++) {
-        const int stage = it & 1;
-        dma_wait_all();
-        __syncthreads();                 // this iteration's tiles and the previous one's P are visible; the other stage is free
-        if (it + 1 < ntiles) copy_for_p(it + 1, stage ^ 1);
-        if (it < ntiles) copy_for_s(it, stage ^ 1);
+        dma_wait<0>();
+        __syncthreads();                 // this iteration's tile and the previous one's P are visible; the slot of tile it - 2 is free
+        const int next = slot == 2 ? 0 : slot + 1;
+        const int mine = ROLE == 0 ? slot : slot == 0 ? 2 : slot - 1;
+        slot = next;
+        if (it + 1 < ntiles) copy_tile(it + 1, next);
         if (ROLE == 0 ? it >= ntiles : it == 0) continue;
 
-        const uint8_t* nt = &L.nat[stage][ROLE][0];
-        const uint8_t* rt = &L.tr[stage][1 - ROLE][0];
-        const float* rowv = &L.row[stage][ROLE][0];
+        const uint8_t* nt = smem + L::RING + mine * L::SLOT + ROLE * TILE_BYTES;
+        const uint8_t* rt = smem + L::RING + mine * L::SLOT + (1 - ROLE) * TILE_BYTES;
+        const uint8_t* rowv = smem + (mine * 2 + ROLE) * 256;
         uint32_t hp[2][8];               // S wave: the P wave's probabilities of this tile
         if constexpr (ROLE == 1) {
 #pragma unroll
             for (int blk = 0; blk < 2; blk++)
 #pragma unroll
                 for (int j = 0; j < 2; j++) {
-                    const u32x4 w = L.p[pair][blk][j][lane];
+                    const u32x4 w = hand[((it - 1) & 1) * (L::P_BYTES / 16) + (blk * 2 + j) * 64];
 #pragma unroll
                     for (int e = 0; e < 4; e++) hp[blk][j * 4 + e] = w[e];
                 }
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-            for (int blk = 0; blk < 2; blk++)
-#pragma unroll
-                for (int e = 0; e < 8; e++) asm volatile("" : "+v"(hp[blk][e]));
-            if (lane == 0) *taken = it;
         }
         v16f sacc[2];
         uint32_t pk[2][8];               // P (P wave) or dS (S wave), packed bf16 pairs: the next product's B operand
@@ -644,7 +623,7 @@ __device__ __forceinline__ void dkdv_role(const BwdArgs& a, DkDvLds<D>& L, int b
 #pragma unroll
             for (int i = 0; i < 16; i++) sacc[blk][i] = 0.0f;
         v4i f[2];
-        auto scores_load = [&](int blk, int ks) { f[ks & 1] = *reinterpret_cast<const v4i*>(nt + nat_frag[blk][ks]); };
+        auto scores_load = [&](int blk, int ks) { f[ks & 1] = *reinterpret_cast<const v4i*>(nt + nat_frag[ks] + blk * 64 * D); };
         auto scores_step = [&](int blk, int ks) {
             if (ks + 1 < KS) scores_load(blk, ks + 1);
             sacc[blk] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, f[ks & 1]), __builtin_bit_cast(v8bf, bx[ks]), sacc[blk], 0, 0, 0);
@@ -653,7 +632,7 @@ __device__ __forceinline__ void dkdv_role(const BwdArgs& a, DkDvLds<D>& L, int b
         auto value_pair = [&](int blk, int i) {
             const int g = i >> 2;
             if ((i & 3) == 0) {
-                const v4f vr = *reinterpret_cast<const v4f*>(rowv + blk * 32 + g * 8 + half * 4);
+                const v4f vr = *reinterpret_cast<const v4f*>(rowv + (blk * 32 + g * 8 + half * 4) * 4);
 #pragma unroll
                 for (int e = 0; e < 4; e++) rv[e] = vr[e];
             }
@@ -672,16 +651,16 @@ __device__ __forceinline__ void dkdv_role(const BwdArgs& a, DkDvLds<D>& L, int b
         constexpr int ACC_M = 2 * DB;
         auto acc_step = [&](int blk, int m) {
             const int j2 = m / DB, d = m % DB;
-            const int j = blk * 2 + j2;
+            const int rows16 = (blk * 2 + j2) * 32 * D;
             const v4i sb = {(int)pk[blk][j2 * 4], (int)pk[blk][j2 * 4 + 1], (int)pk[blk][j2 * 4 + 2], (int)pk[blk][j2 * 4 + 3]};
-            const v4i fa = *reinterpret_cast<const v4i*>(rt + tr_frag[j] + d * 32 * 128);
+            const v4i fa = tr_read(rt + tr_frag[d][0] + rows16, rt + tr_frag[d][1] + rows16);
             acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, fa), __builtin_bit_cast(v8bf, sb), acc[d], 0, 0, 0);
         };
         auto hand_over = [&](int blk) {
             if constexpr (ROLE == 0) {
 #pragma unroll
                 for (int j = 0; j < 2; j++)
-                    L.p[pair][blk][j][lane] = u32x4{ph[blk][j * 4], ph[blk][j * 4 + 1], ph[blk][j * 4 + 2], ph[blk][j * 4 + 3]};
+                    hand[(it & 1) * (L::P_BYTES / 16) + (blk * 2 + j) * 64] = u32x4{ph[blk][j * 4], ph[blk][j * 4 + 1], ph[blk][j * 4 + 2], ph[blk][j * 4 + 3]};
             }
         };
         scores_load(0, 0);
@@ -693,11 +672,6 @@ __device__ __forceinline__ void dkdv_role(const BwdArgs& a, DkDvLds<D>& L, int b
             scores_step(1, ks);
 #pragma unroll
             for (int q = 0; q < 8 / KS; q++) value_pair(0, (ks * (8 / KS) + q) * 2);
-        }
-        if constexpr (ROLE == 0) {
-            // the slot still holds the previous tile's P until the S wave has it in registers
-            while (__builtin_amdgcn_readfirstlane(*taken) < it) __builtin_amdgcn_s_sleep(1);
-            asm volatile("" ::: "memory");
         }
         hand_over(0);
 #pragma unroll
@@ -711,34 +685,33 @@ __device__ __forceinline__ void dkdv_role(const BwdArgs& a, DkDvLds<D>& L, int b
         for (int m = 0; m < ACC_M; m++) acc_step(1, m);
     }
 
-    if (x < a.Nkv) {
-        const bool live = x < a.valid_kv;
-        uint16_t* o = ROLE == 0 ? a.dv + b * a.dv_sb + h * a.dv_sh + (int64_t)x * a.dv_sn
-                                : a.dk + b * a.dk_sb + h * a.dk_sh + (int64_t)x * a.dk_sn;
-        const float mul = ROLE == 0 ? 1.0f : a.scale;
+    // The loop ends with the last tile in the slot two before `slot` (slot = (ntiles + 1) % 3), which the S
+    // waves may still be reading; the P waves' output rows go through the one before `slot`, the S waves'
+    // through `slot`: their last readers were one barrier ago.
+    if (ntiles == 0) __syncthreads();    // (the owner rows of the other waves are still on their way then)
+    uint8_t* os = smem + L::RING + (ROLE == 1 ? slot : slot == 0 ? 2 : slot - 1) * L::SLOT + pair * 64 * D;
+    const bool live = x < a.valid_kv;
+    const float mul = ROLE == 0 ? 1.0f : a.scale;
 #pragma unroll
-        for (int d = 0; d < DB; d++)
+    for (int d = 0; d < DB; d++)
 #pragma unroll
-            for (int g = 0; g < 4; g++) {
-                u32x2 w = {0u, 0u};
-                if (live) {
-                    w.x = pack_bf16(acc[d][g * 4] * mul, acc[d][g * 4 + 1] * mul);
-                    w.y = pack_bf16(acc[d][g * 4 + 2] * mul, acc[d][g * 4 + 3] * mul);
-                }
-                *reinterpret_cast<u32x2*>(o + d * 32 + g * 8 + half * 4) = w;
-            }
-    }
+        for (int g = 0; g < 4; g++) {
+            const u32x2 w = {pack_bf16(acc[d][g * 4] * mul, acc[d][g * 4 + 1] * mul),
+                             pack_bf16(acc[d][g * 4 + 2] * mul, acc[d][g * 4 + 3] * mul)};
+            row_put<D>(os, l32, half, d, g, live ? w : u32x2{0u, 0u});
+        }
+    if constexpr (ROLE == 0) rows_out<D>(os, a.dv + b * a.dv_sb + h * a.dv_sh, a.dv_sn, x0, a.Nkv, lane);
+    else rows_out<D>(os, a.dk + b * a.dk_sb + h * a.dk_sh, a.dk_sn, x0, a.Nkv, lane);
 }
 
 template <int D>
-__device__ __forceinline__ void bwd_dkdv_body(const BwdArgs& a, DkDvLds<D>& L, int block) {
+__device__ __forceinline__ void bwd_dkdv_body(const BwdArgs& a, uint8_t* smem, int block) {
     const int x_tiles = (a.Nkv + 127) / 128;
     const int xt = block % x_tiles, bh = block / x_tiles;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    if (tid < 4) L.taken[tid] = 0;                  // ordered before the first use by the loop's first barrier
-    if (wave < 4) dkdv_role<D, 0>(a, L, bh, xt, wave, lane);
-    else dkdv_role<D, 1>(a, L, bh, xt, wave, lane);
+    if (wave < 4) dkdv_role<D, 0>(a, smem, bh, xt, wave, lane);
+    else dkdv_role<D, 1>(a, smem, bh, xt, wave, lane);
 }
 
 // One grid for both: the first n_dq workgroups are the dQ pass (the longer ones first), the rest
@@ -747,19 +720,19 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdArgs& a, DkDvLds<D>& L, i
 template <int D>
 __global__ __launch_bounds__(512, 2) void bwd_fused_kernel(BwdArgs a, int n_dq) {
     constexpr bool PAIRED = D > 64;                 // below, the single-wave form already fits two waves per SIMD
-    using KvLds = std::conditional_t<PAIRED, DkDvLds<D>, PassLds<D, 1>>;
-    constexpr size_t BYTES = sizeof(KvLds) > sizeof(PassLds<D, 0>) ? sizeof(KvLds) : sizeof(PassLds<D, 0>);
+    constexpr int KV_BYTES = PAIRED ? DkDvLds<D>::BYTES : PassLds<D, 1>::BYTES;
+    constexpr int BYTES = KV_BYTES > PassLds<D, 0>::BYTES ? KV_BYTES : PassLds<D, 0>::BYTES;
     __shared__ __attribute__((aligned(1024))) uint8_t smem[BYTES];
     const int block = (int)blockIdx.x;
-    if (block < n_dq) bwd_pass_body<D, 0, 8>(a, *reinterpret_cast<PassLds<D, 0>*>(smem), block);
-    else if constexpr (PAIRED) bwd_dkdv_body<D>(a, *reinterpret_cast<DkDvLds<D>*>(smem), block - n_dq);
-    else bwd_pass_body<D, 1, 8>(a, *reinterpret_cast<PassLds<D, 1>*>(smem), block - n_dq);
+    if (block < n_dq) bwd_pass_body<D, 0>(a, smem, block);
+    else if constexpr (PAIRED) bwd_dkdv_body<D>(a, smem, block - n_dq);
+    else bwd_pass_body<D, 1>(a, smem, block - n_dq);
 }
 
 template <int D>
 static hipError_t launch_bwd_d(const BwdArgs& a, hipStream_t st) {
     const int64_t bh = (int64_t)a.B * a.H;
-    const int64_t prep = bh * (a.nkv_pad / 64 + 3 * (a.nq_pad / 64));
+    const int64_t prep = bh * (a.nq_pad / 64 + 1);
     // dQ: 256 query rows per workgroup; dK, dV: 128 keys (wave pairs) or 256 keys (single-wave form)
     constexpr int KEYS_WG = D > 64 ? 128 : 256;
     const int64_t gq = bh * ((a.Nq + 255) / 256), gk = bh * ((a.Nkv + KEYS_WG - 1) / KEYS_WG);
