@@ -55,19 +55,18 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
-__device__ __forceinline__ uint32_t f32_to_bf16_rne(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7FFFFFFFu) > 0x7F800000u) return (u >> 16) | 0x0040u;
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return u >> 16;
-}
-__device__ __forceinline__ float round_to_bf16(float f) { return __uint_as_float(f32_to_bf16_rne(f) << 16); }
-
 __device__ __forceinline__ bool key_kept(int s, int N, const KeyMask& m) { return s < N && !(s >= m.lo && s < m.hi); }
 
-// RMSNorm (+ RoPE) of one row, spread over the D/8 consecutive lanes that hold its 16-byte
-// chunks: x[0..7] are channels col..col+7.  Every lane of the group must call this (it
-// exchanges partial sums); `valid` false = a padding row, which stays zero.
+// A lane exchange inside rows of 16 lanes that goes with the vector instruction, not through the LDS pipe.
+template <int CTRL> __device__ __forceinline__ float dpp(float x) {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(x), CTRL, 0xF, 0xF, false));
+}
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppXor3 = 0x1B, kDppXor7 = 0x141, kDppRor = 0x120;      // quad_perm, row_half_mirror, row_ror
+__device__ __forceinline__ float xor4(float x) { return dpp<kDppXor7>(dpp<kDppXor3>(x)); }
+__device__ __forceinline__ float xor8(float x) { return dpp<kDppRor + 8>(x); }
+
+// RMSNorm (+ RoPE) of rows spread over the D/8 consecutive lanes that hold their 16-byte chunks: x[0..7] are
+// channels col..col+7.  Every lane of the group must call these (they exchange partial sums).
 // Arithmetic, step for step (all fp32, no fused multiply-add):
 //   the squares are added in the order of serenitymojo/ops/norm.mojo:56-72 — a 256-slot array
 //   folded in halves, far pairs first: channel t with t+64 (D = 128), then strides 32, 16 and
@@ -75,91 +74,159 @@ __device__ __forceinline__ bool key_kept(int s, int N, const KeyMask& m) { retur
 //   inv = 1/sqrt(sum/D + eps); y = bf16((x*inv)*gain); rotation of (y[2i], y[2i+1]) by
 //   the table angle with both products rounded before the subtract / add; result bf16.
 //   (p.halfsplit: the pairs are (y[i], y[i + D/2]) instead.)
+// What bounds the kernels that use them is vector instructions, so: the exchanges are DPP modifiers of the adds
+// (as LDS permutes they were 32 of them per 16-byte chunk), a row's square root and reciprocal are taken by one
+// lane of its group instead of by all (row_inverses), and both roundings are the conversion instruction
+// (half an operation per element instead of six).  Behind that it is latency: table entries are requested ahead
+// (see RopeTab).  [2,4352,30,128], us: K statistics 89 -> 47, encoders (with the V repack) 174 -> 111.  Dealing the
+// workgroups so that Q, K and the batch items share table rows in an XCD's L2 measured slower (K statistics 69).
 template <int D>
-__device__ __forceinline__ void pre_apply(const PreOp& p, int b, int h, int H, int row, int col, bool valid, float* x) {
+__device__ __forceinline__ float row_square_sum(const float* x) {
     constexpr int CPR = D / 8;
+    static_assert(CPR == 8 || CPR == 16, "rows of 8 or 16 lanes");
     float sq[8];
 #pragma unroll
     for (int e = 0; e < 8; e++) sq[e] = x[e] * x[e];
+    if constexpr (CPR == 16) {
+        // (after the first step lanes l and l + 8 agree, after the second l and l + 4, ...: a rotation then
+        // reaches the same value as the exclusive-or)
 #pragma unroll
-    for (int off = CPR / 2; off > 0; off >>= 1)
+        for (int e = 0; e < 8; e++) sq[e] = sq[e] + xor8(sq[e]);
 #pragma unroll
-        for (int e = 0; e < 8; e++) sq[e] = sq[e] + __shfl_xor(sq[e], off, 64);
+        for (int e = 0; e < 8; e++) sq[e] = sq[e] + dpp<kDppRor + 4>(sq[e]);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; e++) sq[e] = sq[e] + xor4(sq[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e++) sq[e] = sq[e] + dpp<kDppXor2>(sq[e]);
+#pragma unroll
+    for (int e = 0; e < 8; e++) sq[e] = sq[e] + dpp<kDppXor1>(sq[e]);
 #pragma unroll
     for (int e = 0; e < 4; e++) sq[e] = sq[e] + sq[e + 4];
     sq[0] = sq[0] + sq[2];
     sq[1] = sq[1] + sq[3];
-    const float a = sq[0] + sq[1];
-    const float mean = a / (float)D;
-    float inv = 1.0f / sqrtf(mean + p.eps);
-    const uint16_t* gain = p.gain;
-    if (p.row_inv != nullptr) {
-        // the statistic of the whole token (all heads), computed by launch 0; gain of H*D entries
-        inv = valid ? p.row_inv[(int64_t)b * p.row_n + row] : 0.0f;
-        gain += h * D;
+    return sq[0] + sq[1];
+}
+
+// inv[i] = 1/sqrt(mean square of row i + eps) for the N rows of a lane group whose chunks are w[0..N-1]: lane j
+// of the group takes the root of row j.
+template <int D, int N>
+__device__ __forceinline__ void row_inverses(float eps, const u32x4 (&w)[N], float (&inv)[N]) {
+    constexpr int CPR = D / 8;
+    const int lane = threadIdx.x & 63, j = lane % CPR;
+#pragma unroll
+    for (int i0 = 0; i0 < N; i0 += CPR) {
+        float mine = 0.0f;
+#pragma unroll
+        for (int i = 0; i < CPR && i0 + i < N; i++) {
+            float x[8];
+            unpack8(w[i0 + i], x);
+            const float sum = row_square_sum<D>(x);
+            mine = j == i ? sum : mine;
+            asm volatile("" : "+v"(mine));          // (or the compiler gathers the sums in an array in memory and indexes it)
+        }
+        const float mean = mine / (float)D;
+        const float r = 1.0f / sqrtf(mean + eps);
+#pragma unroll
+        for (int i = 0; i < CPR && i0 + i < N; i++) inv[i0 + i] = __shfl(r, (lane & ~(CPR - 1)) + i, 64);
     }
-    const u32x4 gw = *reinterpret_cast<const u32x4*>(gain + col);
-    float g[8];
-    unpack8(gw, g);
+}
+
+__device__ __forceinline__ void round8_to_bf16(float* x) {
+    typedef float v2f __attribute__((ext_vector_type(2)));
+    typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+        const v2f f = {x[e], x[e + 1]};
+        const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(f, v2bf));     // round to nearest even
+        x[e] = bf16_lo(w);
+        x[e + 1] = bf16_hi(w);
+    }
+}
+
+// gains of the thread's channels (with a statistic of the whole token: H*D of them)
+__device__ __forceinline__ void pre_gains(const PreOp& p, int h, int D, int col, float* g) {
+    unpack8(*reinterpret_cast<const u32x4*>(p.gain + (p.row_inv != nullptr ? h * D : 0) + col), g);
+}
+
+// Table entries of one chunk, requested AHEAD chunks ahead.  PRE 1: 16 bytes of cosines and of sines, whatever
+// the layout (bf16 tables of interleaved pairs: the 16 bytes around the 8 that are needed; no tables: the
+// gains, which are not looked at) — the same loads in every case, because behind a branch around a load the compiler
+// has to wait for every load in flight.  PRE 2: half-split pairs with fp32 tables, 32 bytes of each.
+template <int PRE> struct RopeTab { u32x4 c[PRE > 0 ? PRE : 1], s[PRE > 0 ? PRE : 1]; };
+struct RopeAt { const uint8_t *c, *s; int64_t row_bytes; };
+template <int D>
+__device__ __forceinline__ RopeAt rope_at(const PreOp& p, int b, int h, int H, int col) {
+    const uint8_t* gain = reinterpret_cast<const uint8_t*>(p.gain + col);
+    if (p.cos == nullptr) return RopeAt{gain, gain, 0};
+    const int esz = p.tables_bf16 ? 2 : 4;
+    const int at = ((p.halfsplit ? col & (D / 2 - 1) : col / 2) * esz) & ~15;
+    const int64_t off = ((int64_t)b * p.batch_rows + h) * (D / 2) * esz + at;
+    return RopeAt{reinterpret_cast<const uint8_t*>(p.cos) + off, reinterpret_cast<const uint8_t*>(p.sin) + off, (int64_t)H * (D / 2) * esz};
+}
+template <int PRE>
+__device__ __forceinline__ void rope_load(const RopeAt& r, int row, RopeTab<PRE>& t) {
+#pragma unroll
+    for (int i = 0; i < PRE; i++) {
+        t.c[i] = *reinterpret_cast<const u32x4*>(r.c + (int64_t)row * r.row_bytes + i * 16);
+        t.s[i] = *reinterpret_cast<const u32x4*>(r.s + (int64_t)row * r.row_bytes + i * 16);
+    }
+}
+
+// The rest of the pre-op for one row: normalise with `inv`, rotate; `valid` false = a padding row, which stays zero.
+template <int D, int PRE>
+__device__ __forceinline__ void pre_apply(const PreOp& p, int col, bool valid, float inv, const float* g, const RopeTab<PRE>& tab, float* x) {
+    constexpr int CPR = D / 8;
     float y[8];
 #pragma unroll
     for (int e = 0; e < 8; e++) {
         const float t = x[e] * inv;
-        y[e] = round_to_bf16(t * g[e]);
+        y[e] = t * g[e];
     }
-    if (p.cos != nullptr && p.halfsplit) {
+    round8_to_bf16(y);
+    if (PRE == 2 || (p.cos != nullptr && p.halfsplit)) {
         // pairs (i, i + D/2): the partner channel sits in the lane CPR/2 further on (or back) among
         // the CPR lanes of this row; both lanes of a pair use table entries (col mod D/2) .. +7
         float yp[8];
 #pragma unroll
-        for (int e = 0; e < 8; e++) yp[e] = __shfl_xor(y[e], CPR / 2, 64);
+        for (int e = 0; e < 8; e++) yp[e] = CPR == 16 ? xor8(y[e]) : xor4(y[e]);
         const bool upper = col >= D / 2;
         float cv[8], sv[8];
+        if constexpr (PRE == 2) {
 #pragma unroll
-        for (int e = 0; e < 8; e++) cv[e] = 1.0f, sv[e] = 0.0f;
-        if (valid) {
-            const int64_t trow = (int64_t)b * p.batch_rows + (int64_t)row * H + h;
-            const int64_t ti = trow * (D / 2) + (col & (D / 2 - 1));
-            if (p.tables_bf16) {
-                unpack8(*reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(p.cos) + ti), cv);
-                unpack8(*reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(p.sin) + ti), sv);
-            } else {
-                const float* pc = p.cos + ti;
-                const float* ps = p.sin + ti;
-                const float4 c0 = *reinterpret_cast<const float4*>(pc), c1 = *reinterpret_cast<const float4*>(pc + 4);
-                const float4 s0 = *reinterpret_cast<const float4*>(ps), s1 = *reinterpret_cast<const float4*>(ps + 4);
-                cv[0] = c0.x; cv[1] = c0.y; cv[2] = c0.z; cv[3] = c0.w; cv[4] = c1.x; cv[5] = c1.y; cv[6] = c1.z; cv[7] = c1.w;
-                sv[0] = s0.x; sv[1] = s0.y; sv[2] = s0.z; sv[3] = s0.w; sv[4] = s1.x; sv[5] = s1.y; sv[6] = s1.z; sv[7] = s1.w;
-            }
+            for (int e = 0; e < 8; e++) cv[e] = __uint_as_float(tab.c[e >> 2][e & 3]), sv[e] = __uint_as_float(tab.s[e >> 2][e & 3]);
+        } else {
+            unpack8(tab.c[0], cv);
+            unpack8(tab.s[0], sv);
         }
 #pragma unroll
         for (int e = 0; e < 8; e++) {
             // lower half: x0*c - x1*s with x0 = own, x1 = partner; upper half: x1*c + x0*s with x1 = own
             const float own = y[e] * cv[e], oth = yp[e] * sv[e];
-            x[e] = round_to_bf16(upper ? own + oth : own - oth);
+            x[e] = upper ? own + oth : own - oth;
         }
+        round8_to_bf16(x);
     } else if (p.cos != nullptr) {
-        float4 c4 = {1.f, 1.f, 1.f, 1.f}, s4 = {0.f, 0.f, 0.f, 0.f};
-        if (valid) {
-            const int64_t trow = (int64_t)b * p.batch_rows + (int64_t)row * H + h;
-            if (p.tables_bf16) {
-                const u32x2 cw = *reinterpret_cast<const u32x2*>(reinterpret_cast<const uint16_t*>(p.cos) + trow * (D / 2) + col / 2);
-                const u32x2 sw = *reinterpret_cast<const u32x2*>(reinterpret_cast<const uint16_t*>(p.sin) + trow * (D / 2) + col / 2);
-                c4 = float4{__uint_as_float(cw.x << 16), __uint_as_float(cw.x & 0xFFFF0000u), __uint_as_float(cw.y << 16), __uint_as_float(cw.y & 0xFFFF0000u)};
-                s4 = float4{__uint_as_float(sw.x << 16), __uint_as_float(sw.x & 0xFFFF0000u), __uint_as_float(sw.y << 16), __uint_as_float(sw.y & 0xFFFF0000u)};
-            } else {
-                c4 = *reinterpret_cast<const float4*>(p.cos + trow * (D / 2) + col / 2);
-                s4 = *reinterpret_cast<const float4*>(p.sin + trow * (D / 2) + col / 2);
-            }
+        float cv[4], sv[4];
+        if (p.tables_bf16) {
+            const bool hi = (col >> 3) & 1;
+            const u32x2 c = hi ? u32x2{tab.c[0].z, tab.c[0].w} : u32x2{tab.c[0].x, tab.c[0].y};
+            const u32x2 s = hi ? u32x2{tab.s[0].z, tab.s[0].w} : u32x2{tab.s[0].x, tab.s[0].y};
+            cv[0] = bf16_lo(c.x); cv[1] = bf16_hi(c.x); cv[2] = bf16_lo(c.y); cv[3] = bf16_hi(c.y);
+            sv[0] = bf16_lo(s.x); sv[1] = bf16_hi(s.x); sv[2] = bf16_lo(s.y); sv[3] = bf16_hi(s.y);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++) cv[i] = __uint_as_float(tab.c[0][i]), sv[i] = __uint_as_float(tab.s[0][i]);
         }
-        const float cv[4] = {c4.x, c4.y, c4.z, c4.w}, sv[4] = {s4.x, s4.y, s4.z, s4.w};
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const float y0 = y[2 * i], y1 = y[2 * i + 1];
             const float p00 = y0 * cv[i], p11 = y1 * sv[i], p01 = y0 * sv[i], p10 = y1 * cv[i];
-            x[2 * i] = round_to_bf16(p00 - p11);
-            x[2 * i + 1] = round_to_bf16(p01 + p10);
+            x[2 * i] = p00 - p11;
+            x[2 * i + 1] = p01 + p10;
         }
+        round8_to_bf16(x);
     } else {
 #pragma unroll
         for (int e = 0; e < 8; e++) x[e] = y[e];
@@ -178,7 +245,7 @@ __device__ __forceinline__ void pre_apply(const PreOp& p, int b, int h, int H, i
 // Q (IS_K false): x = f32(q) * chmul[d].  K (IS_K true): x = (f32(k) - mean[d]) * chmul[d];
 // tokens that are masked or beyond N count for nothing and get code 0.
 // rowdot (Q only, may be null): <f32(q) * cmul, mean> per row.
-template <int D, int BLK, bool IS_K, bool PRE, int NT>
+template <int D, int BLK, bool IS_K, int PRE, int NT>
 __device__ __forceinline__ void quant_i8_block(
     int t, int h, int b, int tid, const uint16_t* __restrict__ x, int64_t sb, int64_t sh, int64_t sn,
     int N, int H, int64_t n_pad, const KeyMask& km, const float* __restrict__ mean,
@@ -207,11 +274,31 @@ __device__ __forceinline__ void quant_i8_block(
 
     float v[NCH][8];
     float amax = 0.0f;
+    float inv[NCH], gain[8];
+    constexpr int AHEAD = 2;                   // (four take the kernel from three waves per SIMD to two)
+    RopeTab<PRE> tab[AHEAD];
+    auto clamped = [&](int i) { return min(r0 + (i * NT + tid) / CPR, N - 1); };
+    RopeAt rope{};
+    if constexpr (PRE) {
+        rope = rope_at<D>(pre, b, h, H, col);
+#pragma unroll
+        for (int i = 0; i < AHEAD && i < NCH; i++) rope_load<PRE>(rope, clamped(i), tab[i]);
+        pre_gains(pre, h, D, col, gain);
+        if (pre.row_inv == nullptr) {
+            row_inverses<D, NCH>(pre.eps, raw, inv);
+        } else {
+#pragma unroll
+            for (int i = 0; i < NCH; i++) inv[i] = pre.row_inv[(int64_t)b * pre.row_n + clamped(i)];
+        }
+    }
 #pragma unroll
     for (int i = 0; i < NCH; i++) {
         const int row = r0 + (i * NT + tid) / CPR;
         unpack8(raw[i], v[i]);
-        if constexpr (PRE) pre_apply<D>(pre, b, h, H, row, col, row < N, v[i]);
+        if constexpr (PRE) {
+            pre_apply<D, PRE>(pre, col, row < N, inv[i], gain, tab[i % AHEAD], v[i]);
+            if (i + AHEAD < NCH) rope_load<PRE>(rope, clamped(i + AHEAD), tab[i % AHEAD]);
+        }
         bool counts;
         if (IS_K) {
             counts = key_kept(row, N, km);
@@ -255,8 +342,8 @@ __device__ __forceinline__ void quant_i8_block(
 
     uint32_t pk[NCH][2];
     float far[NCH] = {};        // per 16-byte chunk: how close the thread's products come to a rounding tie
-    bool all_careful = PRE || !fast;
-    if constexpr (!PRE) {
+    const bool all_careful = !fast;
+    {
         // The common case, three operations per element and no test: t = x * rinv + 1.5 * 2^23 in one
         // fused step IS rint of the exact product p, as an integer in the low bits of t (its lowest
         // byte is the code: |p| <= 127 (1 + 2^-22) for every token that counts, so nothing needs
@@ -337,7 +424,7 @@ struct KGroupSmem {
 // D is the number of channels this call covers, starting at channel col0 of a head of DFULL
 // channels (the statistics are per channel, so a 256-channel head is done as two windows of 128).
 // Result in gsum, gmn, gmx of the threads tid < D (channel col0 + tid).
-template <int D, bool PRE, int DFULL = D>
+template <int D, int PRE, int DFULL = D>
 __device__ __forceinline__ void kstats_group(
     int g, int h, int b, int tid, const uint16_t* __restrict__ k, int64_t sb, int64_t sh, int64_t sn,
     int N, int H, const KeyMask& km, KGroupSmem<D>& sm, const PreOp& pre, int col0, double& gsum, float& gmn, float& gmx) {
@@ -357,6 +444,23 @@ __device__ __forceinline__ void kstats_group(
     float mn[8], mx[8], xprev[8];
 #pragma unroll
     for (int e = 0; e < 8; e++) { mn[e] = INFINITY; mx[e] = -INFINITY; xprev[e] = 0.0f; }
+    float inv[kLeaf], gain[8];
+    constexpr int AHEAD = PRE == 2 ? 2 : 4;
+    RopeTab<PRE> tab[AHEAD];
+    auto clamped = [&](int i) { return min(max(s0, 0) + i, N - 1); };
+    RopeAt rope{};
+    if constexpr (PRE) {
+        rope = rope_at<D>(pre, b, h, H, col);
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++) rope_load<PRE>(rope, clamped(i), tab[i]);
+        pre_gains(pre, h, D, col, gain);
+        if (pre.row_inv == nullptr) {
+            row_inverses<D, kLeaf>(pre.eps, w, inv);
+        } else {
+#pragma unroll
+            for (int i = 0; i < kLeaf; i++) inv[i] = pre.row_inv[(int64_t)b * pre.row_n + clamped(i)];
+        }
+    }
     // every token of this leaf counts (no ragged end, no masked range inside it)
     const bool all_kept = g >= 0 && s0 + kLeaf <= N && !(s0 < km.hi && s0 + kLeaf > km.lo);
     static_assert(kLeaf % 2 == 0, "tokens are taken in pairs");
@@ -365,7 +469,10 @@ __device__ __forceinline__ void kstats_group(
         float x[8];
         unpack8(w[i], x);
         const bool kept = g >= 0 && key_kept(s0 + i, N, km);
-        if constexpr (PRE) pre_apply<D>(pre, b, h, H, s0 + i, col, kept, x);
+        if constexpr (PRE) {
+            pre_apply<D, PRE>(pre, col, kept, inv[i], gain, tab[i % AHEAD], x);
+            if (i + AHEAD < kLeaf) rope_load<PRE>(rope, clamped(i + AHEAD), tab[i % AHEAD]);
+        }
         // tokens that do not count are +0.0 here, which leaves a double sum unchanged
 #pragma unroll
         for (int e = 0; e < 8; e++) acc[e] += (double)x[e];
@@ -407,7 +514,7 @@ __device__ __forceinline__ void kstats_group(
     }
 }
 
-template <int D, bool PRE, int DFULL = D>
+template <int D, int PRE, int DFULL = D>
 __device__ __forceinline__ void kstats_group_body(
     int g, int h, int b, int tid, const uint16_t* __restrict__ k, int64_t sb, int64_t sh, int64_t sn,
     int N, int H, int ngroups, const KeyMask& km, double* __restrict__ part_sum, float* __restrict__ part_mm,
@@ -636,7 +743,7 @@ __device__ __forceinline__ void quant_v_fp8_body(
 // Launch 1: independent passes over V and K as workgroup roles of one grid (one launch fills
 // the chip where each pass alone is too short to).
 // ---------------------------------------------------------------------------
-template <int D, bool PRE>
+template <int D, int PRE>
 __global__ __launch_bounds__(256) void prep_kernel(PrepArgs a) {
     constexpr int DK = D > 128 ? 128 : D;                 // channels per K statistics call
     constexpr int GPW = 256 / (16 * (DK / 8));            // K groups per workgroup (D = 256: one group, one half of the channels)
@@ -662,7 +769,7 @@ __global__ __launch_bounds__(256) void prep_kernel(PrepArgs a) {
             v_absmax_group_body<D>(r, h, b, a.v.p, a.v.sb, a.v.sh, a.v.sn, a.Nkv, a.H, a.ngroups, a.km, a.vpart, sm.red);
     } else if constexpr (D > 128) {
         const int u = r - a.nv_units;                     // (group, channel half)
-        kstats_group_body<DK, false, D>(u >> 1, h, b, threadIdx.x, a.k.p, a.k.sb, a.k.sh, a.k.sn, a.Nkv, a.H, a.ngroups,
+        kstats_group_body<DK, 0, D>(u >> 1, h, b, threadIdx.x, a.k.p, a.k.sb, a.k.sh, a.k.sn, a.Nkv, a.H, a.ngroups,
                                         a.km, a.kpart_sum, a.kpart_mm, sm.kg[0], a.pre_k, (u & 1) * DK);
     } else {
         const int sub = threadIdx.x / (16 * (D / 8));
@@ -718,6 +825,9 @@ hipError_t launch_row_inv(const View& q, const View& k, int B, int H, int Nq, in
     return hipGetLastError();
 }
 
+// Which instantiation the pre-ops take (see RopeTab).
+static int pre_kind(const PreOp& p) { return p.gain == nullptr ? 0 : p.cos != nullptr && p.halfsplit && !p.tables_bf16 ? 2 : 1; }
+
 hipError_t launch_prep(const PrepArgs& a_in, int B, int D, hipStream_t st) {
     PrepArgs a = a_in;
     a.ngroups = (a.Nkv + kGroup - 1) / kGroup;
@@ -725,16 +835,18 @@ hipError_t launch_prep(const PrepArgs& a_in, int B, int D, hipStream_t st) {
     a.nk_wg = a.kpart_sum == nullptr ? 0 : D == 256 ? a.ngroups * 2 : D == 128 ? a.ngroups : (a.ngroups + 1) / 2;
     a.nv_units = a.vmode == 0 ? (int)(a.nkv_pad / 64) : (a.vmode == 1 ? a.ngroups : 0);
     a.n_bh = B * a.H;
+    const int has_pre = pre_kind(a.pre_k);
     const int64_t total = (int64_t)B * a.H * (a.nv_units + a.nk_wg);
     if (total == 0) return hipSuccess;
     if (total > 0x7FFFFFFF) return hipErrorInvalidValue;
     dim3 grid((unsigned)total), block(256);
-    const bool has_pre = a.pre_k.gain != nullptr;
-    if (D == 128 && has_pre) hipLaunchKernelGGL((prep_kernel<128, true>), grid, block, 0, st, a);
-    else if (D == 128) hipLaunchKernelGGL((prep_kernel<128, false>), grid, block, 0, st, a);
-    else if (D == 64 && has_pre) hipLaunchKernelGGL((prep_kernel<64, true>), grid, block, 0, st, a);
-    else if (D == 64) hipLaunchKernelGGL((prep_kernel<64, false>), grid, block, 0, st, a);
-    else if (D == 256 && !has_pre) hipLaunchKernelGGL((prep_kernel<256, false>), grid, block, 0, st, a);
+    if (D == 128 && has_pre == 2) hipLaunchKernelGGL((prep_kernel<128, 2>), grid, block, 0, st, a);
+    else if (D == 128 && has_pre) hipLaunchKernelGGL((prep_kernel<128, 1>), grid, block, 0, st, a);
+    else if (D == 128) hipLaunchKernelGGL((prep_kernel<128, 0>), grid, block, 0, st, a);
+    else if (D == 64 && has_pre == 2) hipLaunchKernelGGL((prep_kernel<64, 2>), grid, block, 0, st, a);
+    else if (D == 64 && has_pre) hipLaunchKernelGGL((prep_kernel<64, 1>), grid, block, 0, st, a);
+    else if (D == 64) hipLaunchKernelGGL((prep_kernel<64, 0>), grid, block, 0, st, a);
+    else if (D == 256 && !has_pre) hipLaunchKernelGGL((prep_kernel<256, 0>), grid, block, 0, st, a);
     else return hipErrorInvalidValue;
     return hipGetLastError();
 }
@@ -817,9 +929,9 @@ hipError_t launch_stats_final(const FinalArgs& a, hipStream_t st) {
 // Launch 3: Q blocks, K blocks and (e4m3 variant) V tiles as workgroup roles.
 // ---------------------------------------------------------------------------
 // Threads per workgroup (512 at 128 channels, i.e. fewer registers and more waves per SIMD, measured slower).
-template <int D, bool PRE> constexpr int quant_threads() { return 256; }
+template <int D, int PRE> constexpr int quant_threads() { return 256; }
 
-template <int D, bool PRE>
+template <int D, int PRE>
 __global__ __launch_bounds__(256) void quant_kernel(QuantArgs a) {
     constexpr int NT = quant_threads<D, PRE>();
     union Smem {
@@ -868,16 +980,18 @@ hipError_t launch_quant(const QuantArgs& a_in, int B, int D, hipStream_t st) {
     if (a.q8 != nullptr && a.nq_pad % a.blkq != 0) return hipErrorInvalidValue;
     if (a.k8 != nullptr && a.nkv_pad % a.blkk != 0) return hipErrorInvalidValue;
     a.n_bh = B * a.H;
+    const int has_pre = pre_kind(a.pre_q);
     const int64_t total = (int64_t)B * a.H * (a.nq_blk + a.nk_blk + a.nv_tile);
     if (total <= 0 || total > 0x7FFFFFFF) return hipErrorInvalidValue;
     dim3 grid((unsigned)total);
-    const bool has_pre = a.pre_q.gain != nullptr;
 #define SAGE_LAUNCH_QUANT(DD, PP) hipLaunchKernelGGL((quant_kernel<DD, PP>), grid, dim3((quant_threads<DD, PP>())), 0, st, a)
-    if (D == 128 && has_pre) SAGE_LAUNCH_QUANT(128, true);
-    else if (D == 128) SAGE_LAUNCH_QUANT(128, false);
-    else if (D == 64 && has_pre) SAGE_LAUNCH_QUANT(64, true);
-    else if (D == 64) SAGE_LAUNCH_QUANT(64, false);
-    else if (D == 256 && !has_pre) SAGE_LAUNCH_QUANT(256, false);
+    if (D == 128 && has_pre == 2) SAGE_LAUNCH_QUANT(128, 2);
+    else if (D == 128 && has_pre) SAGE_LAUNCH_QUANT(128, 1);
+    else if (D == 128) SAGE_LAUNCH_QUANT(128, 0);
+    else if (D == 64 && has_pre == 2) SAGE_LAUNCH_QUANT(64, 2);
+    else if (D == 64 && has_pre) SAGE_LAUNCH_QUANT(64, 1);
+    else if (D == 64) SAGE_LAUNCH_QUANT(64, 0);
+    else if (D == 256 && !has_pre) SAGE_LAUNCH_QUANT(256, 0);
     else return hipErrorInvalidValue;
 #undef SAGE_LAUNCH_QUANT
     return hipGetLastError();
@@ -892,7 +1006,7 @@ hipError_t launch_quant(const QuantArgs& a_in, int B, int D, hipStream_t st) {
 // ---------------------------------------------------------------------------
 constexpr int kShortThreads = 512;
 
-template <int D, bool PRE>
+template <int D, int PRE>
 __global__ __launch_bounds__(kShortThreads) void quant_short_kernel(QuantArgs a, FinalArgs f) {
     constexpr int DK = D > 128 ? 128 : D;                 // channels per K statistics call
     constexpr int NWIN = D / DK;                          // windows of DK channels
@@ -1039,12 +1153,14 @@ hipError_t launch_quant_short(const QuantArgs& a_in, const FinalArgs& f_in, int 
     const int64_t total = short_workgroups(a);
     if (total <= 0 || total > 0x7FFFFFFF || (a.nv_tile & 1)) return hipErrorInvalidValue;
     const dim3 grid((unsigned)total), block(kShortThreads);
-    const bool has_pre = a.pre_q.gain != nullptr;
-    if (D == 128 && has_pre) hipLaunchKernelGGL((quant_short_kernel<128, true>), grid, block, 0, st, a, f_in);
-    else if (D == 128) hipLaunchKernelGGL((quant_short_kernel<128, false>), grid, block, 0, st, a, f_in);
-    else if (D == 64 && has_pre) hipLaunchKernelGGL((quant_short_kernel<64, true>), grid, block, 0, st, a, f_in);
-    else if (D == 64) hipLaunchKernelGGL((quant_short_kernel<64, false>), grid, block, 0, st, a, f_in);
-    else if (D == 256 && !has_pre) hipLaunchKernelGGL((quant_short_kernel<256, false>), grid, block, 0, st, a, f_in);
+    const int has_pre = pre_kind(a.pre_q);
+    if (D == 128 && has_pre == 2) hipLaunchKernelGGL((quant_short_kernel<128, 2>), grid, block, 0, st, a, f_in);
+    else if (D == 128 && has_pre) hipLaunchKernelGGL((quant_short_kernel<128, 1>), grid, block, 0, st, a, f_in);
+    else if (D == 128) hipLaunchKernelGGL((quant_short_kernel<128, 0>), grid, block, 0, st, a, f_in);
+    else if (D == 64 && has_pre == 2) hipLaunchKernelGGL((quant_short_kernel<64, 2>), grid, block, 0, st, a, f_in);
+    else if (D == 64 && has_pre) hipLaunchKernelGGL((quant_short_kernel<64, 1>), grid, block, 0, st, a, f_in);
+    else if (D == 64) hipLaunchKernelGGL((quant_short_kernel<64, 0>), grid, block, 0, st, a, f_in);
+    else if (D == 256 && !has_pre) hipLaunchKernelGGL((quant_short_kernel<256, 0>), grid, block, 0, st, a, f_in);
     else return hipErrorInvalidValue;
     return hipGetLastError();
 }
