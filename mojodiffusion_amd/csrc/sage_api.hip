@@ -921,7 +921,7 @@ int mi355_sage_sdpa_bwd_bf16(const void* Q, const void* K, const void* V, const 
     a.valid_kv = real_N_kv > 0 && real_N_kv < N_kv ? real_N_kv : N_kv;
     a.scale = scale;
     a.lse2 = reinterpret_cast<float*>(ws + c.lse2);
-    a.delta = reinterpret_cast<float*>(ws + c.delta);
+    a.ndelta = reinterpret_cast<float*>(ws + c.delta);
     a.kcen = reinterpret_cast<float*>(ws + c.kcen);
     a.nq_pad = pad_to(N_q, 64);
     SAGE_HIP(launch_bwd(a, st));

@@ -7,7 +7,7 @@
 // with v_mfma_f32_32x32x16_bf16, fp32 accumulation, P and dS rounded to bf16 as matrix operands.
 //
 // Two launches:
-//   1. bwd_prep_kernel     Delta and Stats * log2(e) per query row (padding rows: +inf, so their
+//   1. bwd_prep_kernel     -Delta and Stats * log2(e) per query row (padding rows: +inf, so their
 //                          probabilities vanish); and a vector c close to the mean key.
 //   2. bwd_fused_kernel    one grid of two kinds of 8-wave workgroups, the longer kind first:
 //        dQ     owner = 256 query rows, loop over key tiles, as scale * (dS K - rowsum(dS) c)
@@ -33,6 +33,7 @@
 //   [1,4608,24,128]  launch 1 31.2 -> 11.8, launch 2 969 -> 884
 //   [1,2304,12,64]   launch 1 8.1 -> 4.8, launch 2 75.9 -> 76.9
 #include "sage_internal.h"
+#include <type_traits>
 
 namespace sage {
 
@@ -178,7 +179,7 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(BwdArgs a) {
                 const int row = r * 64 + i * RPP + tid / CPR;
                 const int64_t idx = (int64_t)bh * a.nq_pad + row;
                 const bool valid = row < a.valid_q;
-                a.delta[idx] = valid ? sum : 0.0f;
+                a.ndelta[idx] = valid ? -sum : 0.0f;
                 a.lse2[idx] = valid ? a.stats[(int64_t)bh * a.Nq + row] * kLog2e : INFINITY;
             }
         }
@@ -220,7 +221,7 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(BwdArgs a) {
 template <int D, int PASS>
 struct PassLds {
     static constexpr int TILE_BYTES = 64 * D * 2, SLOT = 2 * TILE_BYTES, SLOTS = 3;
-    static constexpr int ROW_BYTES = PASS == 1 ? 2048 : 0;                   // [slot][lse | Delta][64], PASS 1 only
+    static constexpr int ROW_BYTES = PASS == 1 ? 2048 : 0;                   // [slot][lse | -Delta][64], PASS 1 only
     // The ring, and during the prologue the owner rows (2 x 32 rows per wave) behind its first slot.
     static constexpr int OWNER = ROW_BYTES + SLOT;
     static constexpr int BYTES = OWNER + 8 * 2 * 64 * D;
@@ -260,7 +261,7 @@ __device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, uint8_t* smem, i
     const uint8_t* y1 = reinterpret_cast<const uint8_t*>(yv1.p + b * yv1.sb + h * yv1.sh);
     const uint8_t* y2 = reinterpret_cast<const uint8_t*>(yv2.p + b * yv2.sb + h * yv2.sh);
     const uint8_t* rows_l = reinterpret_cast<const uint8_t*>(a.lse2 + (int64_t)bh * a.nq_pad);
-    const uint8_t* rows_d = reinterpret_cast<const uint8_t*>(a.delta + (int64_t)bh * a.nq_pad);
+    const uint8_t* rows_d = reinterpret_cast<const uint8_t*>(a.ndelta + (int64_t)bh * a.nq_pad);
     // owners that are all padding have nothing to compute: they only store zeros
     const int ntiles = xt * XROWS < valid_x ? (valid_y + 63) / 64 : 0;
 
@@ -300,12 +301,12 @@ __device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, uint8_t* smem, i
     rows_in<D>(xv1.p + b * xv1.sb + h * xv1.sh, xv1.sn, x0, last_x, row_base + own, lane);
     rows_in<D>(xv2.p + b * xv2.sb + h * xv2.sh, xv2.sn, x0, last_x, row_base + own + 64 * D, lane);
     if (ntiles > 0) copy_tile(0, 0);
-    float lse_x = 0.0f, delta_x = 0.0f;
+    float lse_x = 0.0f, ndelta_x = 0.0f;
     float ds_rowsum = 0.0f;                         // dQ pass: sum over the keys of this lane's dS values
     if constexpr (PASS == 0) {
         const int64_t idx = (int64_t)bh * a.nq_pad + min((int64_t)x, a.nq_pad - 1);
         lse_x = a.lse2[idx];
-        delta_x = a.delta[idx];
+        ndelta_x = a.ndelta[idx];
     }
     // The plain loads above must have landed before the loop: the compiler waits for a load at the
     // first use of its result, and such a wait inside the loop would also wait for the tile copies
@@ -319,7 +320,7 @@ __device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, uint8_t* smem, i
     }
 #pragma unroll
     for (int s = 0; s < KS; s++) asm volatile("" : "+v"(b1[s]), "+v"(b2[s]));
-    asm volatile("" : "+v"(lse_x), "+v"(delta_x));
+    asm volatile("" : "+v"(lse_x), "+v"(ndelta_x));
     __syncthreads();                     // the owner rows' LDS becomes the ring's second and third slot
     if (ntiles > 1) copy_tile(1, 1);
 
@@ -340,8 +341,15 @@ __device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, uint8_t* smem, i
             if constexpr (PASS == 1) acc2[d][i] = 0.0f;
         }
     const float c = a.scale * kLog2e;
+    v16f nd_splat;
+    if constexpr (PASS == 0 && D == 64) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) nd_splat[i] = ndelta_x;
+        asm volatile("" : "+v"(nd_splat));          // (16 registers for the whole loop, not 16 copies per use)
+    }
 
-    auto tile = [&](int t, int slot) {
+    auto tile = [&](auto ragged_tag, int t, int slot) {
+        constexpr bool RAGGED = decltype(ragged_tag)::value;             // dQ pass: the tile's last keys are padding
         const uint8_t* n1 = smem + L::ROW_BYTES + slot * L::SLOT;
         const uint8_t* n2 = n1 + TILE_BYTES;
         const uint8_t* rows = smem + slot * 512;
@@ -350,11 +358,23 @@ __device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, uint8_t* smem, i
         //   scores(0) | scores(1) + exponentials(0) | products(0) + exponentials(1) | products(1)
         v16f tacc[2], gacc[2];
         uint32_t pp[2][8], sp[2][8];
-        float lse[4], dl[4];
+        float lse[4];
+        // G starts from -Delta wherever that saves the subtraction: read into the accumulators where the rows run
+        // along them (PASS 1); in the dQ pass it is one value per lane, whose 16 copies there are registers for
+        // at 64 channels only.
+        constexpr bool G_FROM_DELTA = PASS == 1 || D == 64;
 #pragma unroll
         for (int blk = 0; blk < 2; blk++)
 #pragma unroll
-            for (int i = 0; i < 16; i++) tacc[blk][i] = 0.0f, gacc[blk][i] = 0.0f;
+            for (int g = 0; g < 4; g++) {
+                v4f nd = {0.0f, 0.0f, 0.0f, 0.0f};
+                if constexpr (PASS == 1) nd = *reinterpret_cast<const v4f*>(rows + 256 + (blk * 32 + g * 8 + half * 4) * 4);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    tacc[blk][g * 4 + e] = 0.0f;
+                    gacc[blk][g * 4 + e] = PASS == 1 ? nd[e] : G_FROM_DELTA ? nd_splat[g * 4 + e] : 0.0f;
+                }
+            }
         // one k-step of the two score products of a block: T += Y1 . X1^T, G += Y2 . X2^T.  The
         // fragments of step ks + 1 are requested before the products of step ks are issued.
         v4i f1[2], f2[2];
@@ -373,24 +393,22 @@ __device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, uint8_t* smem, i
             if ((i & 3) == 0) {
                 if constexpr (PASS == 0) {
 #pragma unroll
-                    for (int e = 0; e < 4; e++) lse[e] = lse_x, dl[e] = delta_x;
+                    for (int e = 0; e < 4; e++) lse[e] = lse_x;
                 } else {
                     const v4f vl = *reinterpret_cast<const v4f*>(rows + (blk * 32 + g * 8 + half * 4) * 4);
-                    const v4f vd = *reinterpret_cast<const v4f*>(rows + 256 + (blk * 32 + g * 8 + half * 4) * 4);
 #pragma unroll
-                    for (int e = 0; e < 4; e++) lse[e] = vl[e], dl[e] = vd[e];
+                    for (int e = 0; e < 4; e++) lse[e] = vl[e];
                 }
             }
             float pr[2], ds[2];
 #pragma unroll
             for (int e = 0; e < 2; e++) {
                 float arg = fmaf(tacc[blk][i + e], c, -lse[(i & 3) + e]);
-                if constexpr (PASS == 0) {
-                    // keys past the valid length (only possible in the last tile)
+                if constexpr (RAGGED) {
                     if (t * 64 + blk * 32 + g * 8 + half * 4 + (i & 3) + e >= valid_y) arg = -INFINITY;
                 }
                 pr[e] = __builtin_amdgcn_exp2f(arg);
-                ds[e] = pr[e] * (gacc[blk][i + e] - dl[(i & 3) + e]);
+                ds[e] = pr[e] * (G_FROM_DELTA ? gacc[blk][i + e] : gacc[blk][i + e] + ndelta_x);
             }
             sp[blk][i >> 1] = pack_bf16(ds[0], ds[1]);
             // dQ pass: this lane's share of the row sum of dS, over the rounded values
@@ -444,12 +462,21 @@ __device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, uint8_t* smem, i
     // Tile t sits in slot t % 3 and was requested two iterations earlier: the wait at the top leaves the
     // copies of tile t + 1 in flight.
     int slot = 0;
-    for (int t = 0; t < ntiles; t++) {
+    auto next_tile = [&](int t) {
         if (t + 1 < ntiles) dma_wait<2 * RPW>();
         else dma_wait<0>();
         __syncthreads();                 // tile t is visible; every wave is done with the slot of tile t - 1
         if (t + 2 < ntiles) copy_tile(t + 2, slot == 0 ? 2 : slot - 1);
-        tile(t, slot);
+    };
+    const int clean = PASS == 0 && (valid_y & 63) && ntiles > 0 ? ntiles - 1 : ntiles;
+    for (int t = 0; t < clean; t++) {
+        next_tile(t);
+        tile(std::false_type{}, t, slot);
+        slot = slot == 2 ? 0 : slot + 1;
+    }
+    if (PASS == 0 && clean < ntiles) {   // (a copy of the loop body: tested per element it was 64 of 273 vector instructions of every tile)
+        next_tile(clean);
+        tile(std::true_type{}, clean, slot);
         slot = slot == 2 ? 0 : slot + 1;
     }
 
@@ -510,7 +537,7 @@ __device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, uint8_t* smem, i
 template <int D>
 struct DkDvLds {
     static constexpr int TILE_BYTES = 64 * D * 2, SLOT = 2 * TILE_BYTES, SLOTS = 3;
-    static constexpr int ROW_BYTES = 2048;          // [slot][lse | Delta][64]
+    static constexpr int ROW_BYTES = 2048;          // [slot][lse | -Delta][64]
     static constexpr int P_BYTES = 4 * 2 * 2 * 64 * 16;      // [pair][32-row block][values 0-7 | 8-15][lane], fp16 pairs
     static constexpr int RING = ROW_BYTES + 2 * P_BYTES;
     static constexpr int OWNER = RING + SLOT;       // during the prologue: 32 owner rows per wave
@@ -537,7 +564,7 @@ __device__ __forceinline__ void dkdv_role(const BwdArgs& a, uint8_t* smem, int b
     const uint8_t* yq = reinterpret_cast<const uint8_t*>(a.q.p + b * a.q.sb + h * a.q.sh);
     const uint8_t* yg = reinterpret_cast<const uint8_t*>(a.dout.p + b * a.dout.sb + h * a.dout.sh);
     const uint8_t* rows_l = reinterpret_cast<const uint8_t*>(a.lse2 + (int64_t)bh * a.nq_pad);
-    const uint8_t* rows_d = reinterpret_cast<const uint8_t*>(a.delta + (int64_t)bh * a.nq_pad);
+    const uint8_t* rows_d = reinterpret_cast<const uint8_t*>(a.ndelta + (int64_t)bh * a.nq_pad);
     const int ntiles = xt * 128 < a.valid_kv ? (a.valid_q + 63) / 64 : 0;
 
     int nat_row[RPW], nat_col[RPW];
@@ -614,14 +641,19 @@ __device__ __forceinline__ void dkdv_role(const BwdArgs& a, uint8_t* smem, int b
                     for (int e = 0; e < 4; e++) hp[blk][j * 4 + e] = w[e];
                 }
         }
-        v16f sacc[2];
+        v16f sacc[2];                    // (the S wave's start from -Delta)
         uint32_t pk[2][8];               // P (P wave) or dS (S wave), packed bf16 pairs: the next product's B operand
         uint32_t ph[2][8];               // P wave: the same P as fp16 pairs, for the S wave
-        float rv[4];
+        float rv[4];                     // P wave: lse
 #pragma unroll
         for (int blk = 0; blk < 2; blk++)
 #pragma unroll
-            for (int i = 0; i < 16; i++) sacc[blk][i] = 0.0f;
+            for (int g = 0; g < 4; g++) {
+                v4f nd = {0.0f, 0.0f, 0.0f, 0.0f};
+                if constexpr (ROLE == 1) nd = *reinterpret_cast<const v4f*>(rowv + (blk * 32 + g * 8 + half * 4) * 4);
+#pragma unroll
+                for (int e = 0; e < 4; e++) sacc[blk][g * 4 + e] = nd[e];
+            }
         v4i f[2];
         auto scores_load = [&](int blk, int ks) { f[ks & 1] = *reinterpret_cast<const v4i*>(nt + nat_frag[ks] + blk * 64 * D); };
         auto scores_step = [&](int blk, int ks) {
@@ -631,7 +663,7 @@ __device__ __forceinline__ void dkdv_role(const BwdArgs& a, uint8_t* smem, int b
         // elements i, i+1 of a block (i even): query rows (i>>2)*8 + half*4 + (i&3) (+1), column = key
         auto value_pair = [&](int blk, int i) {
             const int g = i >> 2;
-            if ((i & 3) == 0) {
+            if (ROLE == 0 && (i & 3) == 0) {
                 const v4f vr = *reinterpret_cast<const v4f*>(rowv + (blk * 32 + g * 8 + half * 4) * 4);
 #pragma unroll
                 for (int e = 0; e < 4; e++) rv[e] = vr[e];
@@ -643,8 +675,9 @@ __device__ __forceinline__ void dkdv_role(const BwdArgs& a, uint8_t* smem, int b
                 ph[blk][i >> 1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(y[0], y[1]));
             } else {
                 const v2h w = __builtin_bit_cast(v2h, hp[blk][i >> 1]);
-                y[0] = (float)w[0] * (sacc[blk][i] - rv[i & 3]);
-                y[1] = (float)w[1] * (sacc[blk][i + 1] - rv[(i & 3) + 1]);
+                // (as a multiply-add: one instruction with the fp16 operand's conversion in it)
+                y[0] = fmaf((float)w[0], sacc[blk][i], 0.0f);
+                y[1] = fmaf((float)w[1], sacc[blk][i + 1], 0.0f);
             }
             pk[blk][i >> 1] = pack_bf16(y[0], y[1]);
         };

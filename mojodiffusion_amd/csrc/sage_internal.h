@@ -182,7 +182,7 @@ struct BwdArgs {
     int valid_q, valid_kv;                       // rows / keys past these are padding
     float scale;
     // workspace
-    float *lse2, *delta;                         // [B,H,nq_pad]: Stats*log2(e) (+inf past valid), rowsum(dO*O)
+    float *lse2, *ndelta;                        // [B,H,nq_pad]: Stats*log2(e) (+inf past valid), -rowsum(dO*O)
     float* kcen;                                 // [B,H,D]: a vector close to the mean key (see sage_bwd.hip)
     int64_t nq_pad;                              // Nq rounded up to a multiple of 64
 };
