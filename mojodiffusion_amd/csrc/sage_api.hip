@@ -273,8 +273,9 @@ int quantize(const View& q, const View& k, const View* v, int B, int H, int Nq, 
     p.kpart_sum = kstats ? o.kpart_sum : nullptr;
     p.kpart_mm = o.kpart_mm;
     SAGE_HIP(launch_prep(p, B, D, st));
-    SAGE_HIP(launch_stats_final(f, st));
-    SAGE_HIP(launch_quant(a, B, D, st));
+    const bool adds_up = f.kmean != nullptr && quant_adds_up(a);
+    if (!adds_up) SAGE_HIP(launch_stats_final(f, st));
+    SAGE_HIP(launch_quant(a, adds_up ? &f : nullptr, B, D, st));
     return 0;
 }
 
@@ -720,7 +721,7 @@ int mi355_sage_quant_v_fp8(const void* V, int B, int H, int N_kv, int D, const i
     QuantArgs a{};
     a.v = p.v; a.H = H; a.Nkv = N_kv; a.nkv_pad = p.nkv_pad; a.km = p.km; a.blkq = 32; a.blkk = 32;
     a.vscale = f.vscale; a.v8 = static_cast<uint8_t*>(v8);
-    SAGE_HIP(launch_quant(a, B, D, st));
+    SAGE_HIP(launch_quant(a, nullptr, B, D, st));
     return MI355_SAGE_OK;
 }
 

@@ -100,7 +100,10 @@ struct QuantArgs {
     PreOp pre_q, pre_k;
     int nq_blk, nk_blk, nv_tile, n_bh;     // filled by the launcher
 };
-hipError_t launch_quant(const QuantArgs& a, int B, int D, hipStream_t st);
+// f given: launch 2 is left out, the encoders add up the group results themselves and leave them in f's outputs
+// (quant_adds_up: where that pays; needs k8, and v8 where f has vscale).
+bool quant_adds_up(const QuantArgs& a);
+hipError_t launch_quant(const QuantArgs& a, const FinalArgs* f, int B, int D, hipStream_t st);
 
 // All of it as one launch, for short key sequences (K, V and, with q8, Q; the statistics also go to f's outputs).
 bool quant_is_short(const QuantArgs& a, int B, int D);

@@ -1,5 +1,5 @@
 // sage_quant.hip — HBM-bound kernels of the quantized-SDPA path (gfx950), three launches (one for short
-// key sequences, quant_short_kernel):
+// key sequences, quant_short_kernel; two for the next longer ones, quant_adds_up):
 //
 //   prep_kernel         per (b,h), workgroup roles:  V repack to tiled fp16  |  V channel
 //                       maxima per 256-token group (e4m3 variant)  |  K channel sums (fp64),
@@ -869,54 +869,60 @@ __device__ __forceinline__ void k_final(double sum, float mn, float mx, int kept
     }
 }
 
+// Groups added up, strictly in group order; the loads go NB groups at a time (taken one by one, each waits
+// out a memory latency).
+template <int NB>
+__device__ __forceinline__ void k_totals(const FinalArgs& a, int64_t bh, int d, float& mean, float& s) {
+    mean = 0.0f;
+    s = 1.0f;
+    if (a.kpart_sum == nullptr) return;
+    const double* p = a.kpart_sum + bh * a.ngroups * a.D + d;
+    const float* q = a.kpart_mm + 2 * (bh * a.ngroups * a.D + d);
+    double sum = 0.0;
+    float mn = INFINITY, mx = -INFINITY;
+    for (int g0 = 0; g0 < a.ngroups; g0 += NB) {
+        double v[NB];
+        float lo[NB], hi[NB];
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            const int64_t g = g0 + j < a.ngroups ? g0 + j : a.ngroups - 1;
+            v[j] = p[g * a.D];
+            lo[j] = q[2 * g * a.D];
+            hi[j] = q[2 * g * a.D + 1];
+        }
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+            if (g0 + j < a.ngroups) { sum += v[j]; mn = fminf(mn, lo[j]); mx = fmaxf(mx, hi[j]); }
+    }
+    k_final(sum, mn, mx, a.kept, a.flags, mean, s);
+}
+template <int NB>
+__device__ __forceinline__ float v_total(const FinalArgs& a, int64_t bh, int d) {
+    const float* p = a.vpart + bh * a.ngroups * a.D + d;
+    float amax = 0.0f;
+    for (int g0 = 0; g0 < a.ngroups; g0 += NB) {
+        float v[NB];
+#pragma unroll
+        for (int j = 0; j < NB; j++) v[j] = p[(int64_t)(g0 + j < a.ngroups ? g0 + j : a.ngroups - 1) * a.D];
+#pragma unroll
+        for (int j = 0; j < NB; j++) amax = fmaxf(amax, v[j]);
+    }
+    return amax > 0.0f ? amax / 448.0f : 1.0f;
+}
+
 __global__ __launch_bounds__(64) void stats_final_kernel(FinalArgs a) {
     const int64_t i = (int64_t)blockIdx.x * 64 + threadIdx.x;      // (bh, d)
     if (i >= a.total) return;
     const int64_t bh = i / a.D;
     const int d = (int)(i % a.D);
     if (a.kmean != nullptr) {
-        float mean = 0.0f, s = 1.0f;
-        if (a.kpart_sum != nullptr) {
-            const double* p = a.kpart_sum + bh * a.ngroups * a.D + d;
-            const float* q = a.kpart_mm + 2 * (bh * a.ngroups * a.D + d);
-            double sum = 0.0;
-            float mn = INFINITY, mx = -INFINITY;
-            // loads 32 groups at a time (all independent, in flight together); sums strictly in group order
-            constexpr int NB = 32;
-            for (int g0 = 0; g0 < a.ngroups; g0 += NB) {
-                double v[NB];
-                float lo[NB], hi[NB];
-#pragma unroll
-                for (int j = 0; j < NB; j++) {
-                    const int64_t g = g0 + j < a.ngroups ? g0 + j : a.ngroups - 1;
-                    v[j] = p[g * a.D];
-                    lo[j] = q[2 * g * a.D];
-                    hi[j] = q[2 * g * a.D + 1];
-                }
-#pragma unroll
-                for (int j = 0; j < NB; j++)
-                    if (g0 + j < a.ngroups) { sum += v[j]; mn = fminf(mn, lo[j]); mx = fmaxf(mx, hi[j]); }
-            }
-            k_final(sum, mn, mx, a.kept, a.flags, mean, s);
-        }
+        float mean, s;
+        k_totals<32>(a, bh, d, mean, s);
         a.kmean[i] = mean;
         a.kmul[i] = 1.0f / s;
         a.qmul[i] = a.cmul * s;
     }
-    if (a.vscale != nullptr) {
-        const float* p = a.vpart + bh * a.ngroups * a.D + d;
-        float amax = 0.0f;
-        // (32 loads in flight at a time: taken one by one, each waits out a memory latency)
-        constexpr int NB = 32;
-        for (int g0 = 0; g0 < a.ngroups; g0 += NB) {
-            float v[NB];
-#pragma unroll
-            for (int j = 0; j < NB; j++) v[j] = p[(int64_t)(g0 + j < a.ngroups ? g0 + j : a.ngroups - 1) * a.D];
-#pragma unroll
-            for (int j = 0; j < NB; j++) amax = fmaxf(amax, v[j]);
-        }
-        a.vscale[i] = amax > 0.0f ? amax / 448.0f : 1.0f;
-    }
+    if (a.vscale != nullptr) a.vscale[i] = v_total<32>(a, bh, d);
 }
 
 hipError_t launch_stats_final(const FinalArgs& a, hipStream_t st) {
@@ -931,8 +937,10 @@ hipError_t launch_stats_final(const FinalArgs& a, hipStream_t st) {
 // Threads per workgroup (512 at 128 channels, i.e. fewer registers and more waves per SIMD, measured slower).
 template <int D, int PRE> constexpr int quant_threads() { return 256; }
 
-template <int D, int PRE>
-__global__ __launch_bounds__(256) void quant_kernel(QuantArgs a) {
+// FIN: launch 2 is left out — every workgroup adds up the group results it needs for itself (the same additions,
+// so the same bits), the first of a head's K and V workgroups also leave them for later launches.
+template <int D, int PRE, bool FIN>
+__global__ __launch_bounds__(256) void quant_kernel(QuantArgs a, FinalArgs f) {
     constexpr int NT = quant_threads<D, PRE>();
     union Smem {
         float red[NT / 64];
@@ -945,9 +953,29 @@ __global__ __launch_bounds__(256) void quant_kernel(QuantArgs a) {
     const int bh = blockIdx.x % a.n_bh, r = blockIdx.x / a.n_bh;
     const int b = bh / a.H, h = bh % a.H;
     const KeyMask none{0, 0};
+    __shared__ __attribute__((aligned(16))) float s_fin[FIN ? 3 : 1][FIN ? D : 4];      // mean, kmul, qmul; or vscale
+    if constexpr (FIN) {
+        const bool is_v = r >= a.nq_blk + a.nk_blk;
+        if (threadIdx.x < D && !(is_v && a.v16 != nullptr)) {
+            const int d = threadIdx.x;
+            const int64_t i = (int64_t)bh * D + d;
+            if (is_v) {
+                const float sc = v_total<8>(f, bh, d);
+                s_fin[0][d] = sc;
+                if (r == a.nq_blk + a.nk_blk) f.vscale[i] = sc;
+            } else {
+                float mean, s;
+                k_totals<8>(f, bh, d, mean, s);
+                const float kmul = 1.0f / s, qmul = f.cmul * s;
+                s_fin[0][d] = mean; s_fin[1][d] = kmul; s_fin[2][d] = qmul;
+                if (r == a.nq_blk) { f.kmean[i] = mean; f.kmul[i] = kmul; f.qmul[i] = qmul; }
+            }
+        }
+        __syncthreads();
+    }
     if (r < a.nq_blk) {
-        const float* mul = a.qmul + (int64_t)bh * D;
-        const float* mean = a.kmean + (int64_t)bh * D;
+        const float* mul = FIN ? s_fin[FIN ? 2 : 0] : a.qmul + (int64_t)bh * D;
+        const float* mean = FIN ? s_fin[0] : a.kmean + (int64_t)bh * D;
 #define SAGE_Q(BLK) quant_i8_block<D, BLK, false, PRE, NT>(r, h, b, threadIdx.x, a.q.p, a.q.sb, a.q.sh, a.q.sn, a.Nq, a.H, a.nq_pad, none, \
                                                        mean, mul, a.cmul, a.q8, a.qscale, a.rowdot, sm.red, a.pre_q)
         if (a.blkq == 128) SAGE_Q(128);
@@ -956,8 +984,8 @@ __global__ __launch_bounds__(256) void quant_kernel(QuantArgs a) {
 #undef SAGE_Q
     } else if (r < a.nq_blk + a.nk_blk) {
         const int t = r - a.nq_blk;
-        const float* mul = a.kmul + (int64_t)bh * D;
-        const float* mean = a.kmean + (int64_t)bh * D;
+        const float* mul = FIN ? s_fin[FIN ? 1 : 0] : a.kmul + (int64_t)bh * D;
+        const float* mean = FIN ? s_fin[0] : a.kmean + (int64_t)bh * D;
 #define SAGE_K(BLK) quant_i8_block<D, BLK, true, PRE, NT>(t, h, b, threadIdx.x, a.k.p, a.k.sb, a.k.sh, a.k.sn, a.Nkv, a.H, a.nkv_pad, a.km, \
                                                       mean, mul, 0.0f, a.k8, a.kscale, nullptr, sm.red, a.pre_k)
         if (a.blkk == 128) SAGE_K(128);
@@ -968,11 +996,22 @@ __global__ __launch_bounds__(256) void quant_kernel(QuantArgs a) {
         quant_v_f16_body<D>(r - a.nq_blk - a.nk_blk, h, b, threadIdx.x, a.v.p, a.v.sb, a.v.sh, a.v.sn, a.Nkv, a.H, a.nkv_pad, a.km, a.v16, sm.tile16);
     } else {
         quant_v_fp8_body<D, NT>(r - a.nq_blk - a.nk_blk, h, b, threadIdx.x, a.v.p, a.v.sb, a.v.sh, a.v.sn, a.Nkv, a.H, a.nkv_pad, a.km,
-                            a.vscale + (int64_t)bh * D, a.v8, sm.tile8);
+                            FIN ? s_fin[0] : a.vscale + (int64_t)bh * D, a.v8, sm.tile8);
     }
 }
 
-hipError_t launch_quant(const QuantArgs& a_in, int B, int D, hipStream_t st) {
+// Where launch 2 is left out.  It costs 3 us, the start and end of a kernel that does next to nothing; adding up
+// costs every workgroup the group results of its head from L2, 16 bytes per group and channel next to the 128 (Q:
+// 256) bytes per channel it encodes.  Stage of K and V, us, three launches -> two: [1,1153,24,128] 15.7 -> 12.7,
+// [2,1248,30,128] 24.5 -> 22.5, [1,2304,24,128] (9 groups) 19.8 -> 17.1, [1,3000,24,128] (12) 24.0 -> 22.9,
+// [1,4608,24,128] (18) 28.4 -> 30.2, [1,1153,18,256] 20.4 -> 16.9.  e4m3, with 32-row Q blocks: [1,1800,24,128] (8)
+// 24.9 -> 23.2, [1,2304,24,128] (9) 27.1 -> 28.1.
+bool quant_adds_up(const QuantArgs& a) {
+    const int groups = (a.Nkv + kGroup - 1) / kGroup;
+    return a.k8 != nullptr && groups <= (a.v8 != nullptr ? 8 : 10);
+}
+
+hipError_t launch_quant(const QuantArgs& a_in, const FinalArgs* f, int B, int D, hipStream_t st) {
     QuantArgs a = a_in;
     a.nq_blk = a.q8 != nullptr ? (int)(a.nq_pad / a.blkq) : 0;
     a.nk_blk = a.k8 != nullptr ? (int)(a.nkv_pad / a.blkk) : 0;
@@ -984,7 +1023,11 @@ hipError_t launch_quant(const QuantArgs& a_in, int B, int D, hipStream_t st) {
     const int64_t total = (int64_t)B * a.H * (a.nq_blk + a.nk_blk + a.nv_tile);
     if (total <= 0 || total > 0x7FFFFFFF) return hipErrorInvalidValue;
     dim3 grid((unsigned)total);
-#define SAGE_LAUNCH_QUANT(DD, PP) hipLaunchKernelGGL((quant_kernel<DD, PP>), grid, dim3((quant_threads<DD, PP>())), 0, st, a)
+#define SAGE_LAUNCH_QUANT(DD, PP)                                                                                              \
+    do {                                                                                                                       \
+        if (f != nullptr) hipLaunchKernelGGL((quant_kernel<DD, PP, true>), grid, dim3((quant_threads<DD, PP>())), 0, st, a, *f); \
+        else hipLaunchKernelGGL((quant_kernel<DD, PP, false>), grid, dim3((quant_threads<DD, PP>())), 0, st, a, FinalArgs{});    \
+    } while (0)
     if (D == 128 && has_pre == 2) SAGE_LAUNCH_QUANT(128, 2);
     else if (D == 128 && has_pre) SAGE_LAUNCH_QUANT(128, 1);
     else if (D == 128) SAGE_LAUNCH_QUANT(128, 0);
