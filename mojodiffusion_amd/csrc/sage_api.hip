@@ -257,7 +257,7 @@ int quantize(const View& q, const View& k, const View* v, int B, int H, int Nq, 
     if (v_fp8) { a.v = *v; a.v8 = static_cast<uint8_t*>(vq); }
     else if (v != nullptr) { a.v = *v; a.v16 = static_cast<uint16_t*>(vq); }
     a.pre_q = pre.q; a.pre_k = pre.k;
-    if (v != nullptr && quant_is_short(a, B, D)) {
+    if (v != nullptr && quant_short_workgroups(a, B, D) > 0) {
         SAGE_HIP(launch_quant_short(a, f, B, D, st));
         return 0;
     }
@@ -347,7 +347,29 @@ int sdpa_impl(const void* Q, const void* K, const void* V, void* O, void* Stats,
     const AttnPlan plan = attn_plan(B, H, N_q, kv, D, variant, causal != 0);
     // The plain forward leaves Q to the attention kernel, which encodes its own rows (same codes and
     // scales): the quantize stage then neither reads Q nor writes its codes.
-    const bool q_in_kernel = Stats == nullptr && mask.add == nullptr && pre.q.gain == nullptr && (D <= 128 || plan.main_items == 0) && plan.split_wgs == 0;
+    // Not where the encoders have room for it and a prologue is on the path of the whole call — the main kernel does
+    // everything in one round that leaves compute units without a workgroup (us with Q in the kernel -> in the
+    // encoders: [1,700,24,128] 36.7 -> 34.3, [1,1153,24,128] 46.6 -> 43.8; but [1,2304,24,128], two rounds, 72.9 ->
+    // 75.4) — nor with e4m3 P.V, whose scale blocks are single waves' and whose prologue costs more
+    // ([1,256,30,128] 18.9 -> 16.8, [1,1153,24,128] 49.8 -> 46.6, [1,4608,24,128] 220.7 -> 216.3; level at 16896, at 64
+    // channels level at 4608 and 383 -> 388 at 8192).  Many queries on few keys keep it ([1,3840 x 333,32,128] fp16
+    // 50.1 -> 52.0, e4m3 57.5 -> 64.0), and so does a K that takes one launch alone and three, or more than a
+    // workgroup per compute unit, with Q ([1,2048 x 512,32,64] 23.7 -> 30.4, e4m3 [1,512,24,128] 21.5 -> 25.6).
+    auto one_launch = [&](bool with_q) {
+        QuantArgs t{};
+        t.H = H; t.Nkv = kv; t.blkq = blkq; t.blkk = blkk;
+        t.nq_pad = pad_to(N_q, kTileQ); t.nkv_pad = pad_to(kv, kPadKV);
+        t.q8 = with_q ? reinterpret_cast<int8_t*>(ws) : nullptr;
+        return quant_short_workgroups(t, B, D);
+    };
+    const bool one_round = plan.main_items > 0 && plan.short_kw == 0 && plan.main_items < 256;
+    bool q_in_encoders = (one_round || (variant == MI355_SAGE_PV_FP8 && (int64_t)N_q * 64 <= (int64_t)4096 * D)) && N_q <= 2 * N_kv;
+    if (q_in_encoders && one_launch(false) > 0) {
+        const int64_t wgs = one_launch(true);
+        q_in_encoders = wgs > 0 && wgs <= 256;
+    }
+    const bool q_in_kernel = Stats == nullptr && mask.add == nullptr && pre.q.gain == nullptr && (D <= 128 || plan.main_items == 0) &&
+                             plan.split_wgs == 0 && !q_in_encoders;
     QuantOut o{};
     o.q8 = q_in_kernel ? nullptr : reinterpret_cast<int8_t*>(ws + c.q8);
     o.k8 = reinterpret_cast<int8_t*>(ws + c.k8);

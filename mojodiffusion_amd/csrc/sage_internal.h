@@ -106,7 +106,7 @@ bool quant_adds_up(const QuantArgs& a);
 hipError_t launch_quant(const QuantArgs& a, const FinalArgs* f, int B, int D, hipStream_t st);
 
 // All of it as one launch, for short key sequences (K, V and, with q8, Q; the statistics also go to f's outputs).
-bool quant_is_short(const QuantArgs& a, int B, int D);
+int64_t quant_short_workgroups(const QuantArgs& a, int B, int D);     // 0: not this form
 hipError_t launch_quant_short(const QuantArgs& a, const FinalArgs& f, int B, int D, hipStream_t st);
 
 // ---- attention kernel (sage_attn.hip) --------------------------------------

@@ -1045,7 +1045,7 @@ hipError_t launch_quant(const QuantArgs& a_in, const FinalArgs* f, int B, int D,
 // head's K statistics by itself — the same leaves, groups and order, so the same bits — and then encodes
 // one block per half of its threads; a V workgroup takes the head's channel maxima (e4m3) the same way.
 // Every workgroup re-reads the head's K (or V) from L2, which is what a short sequence is for: three
-// dependent launches of 4 to 6 us each do almost nothing but start and drain there (see quant_is_short).
+// dependent launches of 4 to 6 us each do almost nothing but start and drain there (see quant_short_workgroups).
 // ---------------------------------------------------------------------------
 constexpr int kShortThreads = 512;
 
@@ -1181,11 +1181,12 @@ static int64_t short_workgroups(const QuantArgs& a) { return (int64_t)a.n_bh * (
 // per compute unit).  Measured over 4 to 60 heads, stage of three launches -> one, us: 11.5-15 -> 7.5-9.5 up
 // to 256 keys, 13-15 -> 9-12.8 at 512 keys of 128 channels, 12-13.4 -> 8.4-10.7 at 1024 keys of 64; a second
 // pass costs 4 us and a second generation of workgroups 7, which is what the two launches less are worth.
-bool quant_is_short(const QuantArgs& a_in, int B, int D) {
+int64_t quant_short_workgroups(const QuantArgs& a_in, int B, int D) {
     QuantArgs a = a_in;
     short_units(a, B);
     const int groups = (a.Nkv + kGroup - 1) / kGroup;
-    return groups <= (D == 64 ? 4 : D == 128 ? 2 : 1) && short_workgroups(a) <= 512;
+    const int64_t wgs = short_workgroups(a);
+    return groups <= (D == 64 ? 4 : D == 128 ? 2 : 1) && wgs <= 512 ? wgs : 0;
 }
 
 hipError_t launch_quant_short(const QuantArgs& a_in, const FinalArgs& f_in, int B, int D, hipStream_t st) {
