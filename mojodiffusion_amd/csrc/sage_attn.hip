@@ -882,7 +882,11 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     const float inv = 1.0f / l_tot + poison;      // l carries pscale, which cancels the pscale in P
     // Through LDS, so that a store instruction writes whole rows (a lane's own 8-byte pieces are 64
     // separate rows per instruction).  The first half of the waves uses the K ring, the others the V^T ring.
-    __syncthreads();                                // every wave is done with the rings
+    // The last midpoints' copies of the clamped last tile go to slots of those rings and may still be on their
+    // way (the barrier does not wait for them, and the compiler does not know of them): every wave lets its own
+    // land before it says that it is done.
+    dma_wait<0>();
+    __syncthreads();                                // every wave is done with the rings, its copies included
     {
         static_assert(NSK * K_BYTES >= NW / 2 * 64 * D && NSV * V_BYTES >= NW / 2 * 64 * D, "output rows must fit the rings");
         constexpr int OC = D / 8;                   // 16-byte chunks per output row, XORed with the row
