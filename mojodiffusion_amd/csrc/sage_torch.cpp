@@ -3,8 +3,10 @@
 // attention_sage.py states the call surface: names, checks, error texts.  This module does the same work for
 // calls that meet every check — allocate the outputs, carve the workspace, call the C ABI on the current
 // stream — without the interpreter in between: 21 us of host time per call from Python and ctypes, of which
-// two launches are 5 us, became 8.  Anything it does not take (another dtype, a shape that must be refused,
-// a non-zero return code) comes back as None, and the Python function goes its own way and raises.
+// two launches are 5 us, became 8.  Anything it does not take (another dtype, a shape that must be refused, a
+// tensor of a subclass, a tracer or a transform, a non-zero return code) comes back as None, and the Python
+// function goes its own way and raises.
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <ATen/ATen.h>
@@ -45,6 +47,8 @@ auto& g_ws = *new std::map<std::pair<int, void*>, at::Tensor>;
 
 at::Tensor workspace(size_t nbytes, const at::Device& dev, void* stream) {
     std::lock_guard<std::mutex> lock(g_ws_mutex);
+    // (plain memory also when a mode is on for this thread: the buffer outlives it)
+    c10::impl::ForceDispatchKeyGuard no_modes(c10::default_included_set, c10::default_excluded_set);
     at::Tensor& ws = g_ws[{dev.index(), stream}];
     if (!ws.defined() || (size_t)ws.numel() < nbytes)
         ws = at::empty({(int64_t)nbytes}, at::TensorOptions().dtype(at::kByte).device(dev));
@@ -167,10 +171,23 @@ struct SdpaNode : torch::autograd::Function<SdpaNode> {
 };
 
 // ---- argument access -----------------------------------------------------------------------------
+// Dense device memory and nothing else.  Every other kind of tensor — fake, functional, batched or wrapped by a
+// transform, dual — carries a dispatch key or a tangent of its own; its sizes may be symbolic and it may have no
+// memory to point to.
+bool plain(const at::Tensor& t) {
+    static const uint64_t keys = c10::DispatchKeySet({c10::DispatchKey::CUDA, c10::DispatchKey::AutogradCUDA, c10::DispatchKey::AutocastCUDA,
+                                                      c10::DispatchKey::ADInplaceOrView}).raw_repr();
+    return t.defined() && (t.key_set().raw_repr() & ~keys) == 0 && !t._fw_grad(0).defined();
+}
+// Taken: a plain torch.Tensor or Parameter (a subclass's results are of its type: left to the Python path).
 bool tensor_arg(PyObject* o, const at::Tensor*& t) {
-    if (!THPVariable_Check(o)) return false;
+    if (!THPVariable_CheckExact(o)) return false;
     t = &THPVariable_Unpack(o);
-    return true;
+    return plain(*t);
+}
+// A mode or transform is on for this thread (its allocations would not be plain tensors either).
+bool intercepted() {
+    return (c10::impl::tls_local_dispatch_key_set().included_.raw_repr() & ~c10::default_included_set.raw_repr()) != 0;
 }
 bool double_arg(PyObject* o, double& x) {
     x = PyFloat_AsDouble(o);
@@ -197,87 +214,82 @@ template <class F> int without_gil(F f) {
     return rc;
 }
 
-// C++ exceptions (out of memory, HIP errors of the allocator) as Python ones
-template <class F> PyObject* guarded(F f) {
+// What the interpreter calls: no C++ exception crosses its frames.  Out of memory, errors of the device and
+// exceptions of Python hooks arrive as the Python exceptions torch raises for them.
+template <PyObject* (*F)(PyObject* const*, Py_ssize_t)> PyObject* entry(PyObject*, PyObject* const* a, Py_ssize_t n) {
     try {
-        return f();
-    } catch (const c10::Error& e) {
-        PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace());
-    } catch (const std::exception& e) {
-        PyErr_SetString(PyExc_RuntimeError, e.what());
+        return F(a, n);
+    } catch (...) {
+        torch::translate_exception_to_python(std::current_exception());
+        return nullptr;
     }
-    return nullptr;
 }
 
 // fwd(q, k, v, scale, variant, kind, lo, hi, square) -> o, (o, stats) for kind 1, or None.  BF16; for the kinds
 // without Stats also F32, cast at the boundary.
-PyObject* py_fwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
+PyObject* py_fwd(PyObject* const* a, Py_ssize_t n) {
     const at::Tensor *q, *k, *v;
     double scale;
     int variant, kind, lo, hi, square;
-    if (n != 9 || !tensor_arg(a[0], q) || !tensor_arg(a[1], k) || !tensor_arg(a[2], v) || !double_arg(a[3], scale) || !int_arg(a[4], variant) ||
+    if (intercepted() || n != 9 || !tensor_arg(a[0], q) || !tensor_arg(a[1], k) || !tensor_arg(a[2], v) || !double_arg(a[3], scale) || !int_arg(a[4], variant) ||
         !int_arg(a[5], kind) || !int_arg(a[6], lo) || !int_arg(a[7], hi) || !int_arg(a[8], square))
         Py_RETURN_NONE;
     if (!shapes_ok(*q, *k, *v, square != 0)) Py_RETURN_NONE;
     const bool f32 = q->scalar_type() == at::kFloat;
     if (q->scalar_type() != at::kBFloat16 && !(f32 && kind != kTrain)) Py_RETURN_NONE;
-    return guarded([&]() -> PyObject* {
-        at::Tensor o, stats;
-        const int rc = without_gil([&] {
-            if (!f32) return forward(*q, *k, *v, scale, variant, kind, lo, hi, o, stats);
-            at::Tensor b[3], ob;
-            const at::Tensor* src[3] = {q, k, v};
-            int r = cast(3, src, b, true);
-            if (r == 0) r = forward(b[0], b[1], b[2], scale, variant, kind, lo, hi, ob, stats);
-            if (r != 0) return r;
-            const at::Tensor* back[1] = {&ob};
-            return cast(1, back, &o, false);
-        });
-        if (rc != 0) Py_RETURN_NONE;
-        if (kind != kTrain) return THPVariable_Wrap(std::move(o));
-        PyObject* t = PyTuple_New(2);
-        PyTuple_SET_ITEM(t, 0, THPVariable_Wrap(std::move(o)));
-        PyTuple_SET_ITEM(t, 1, THPVariable_Wrap(std::move(stats)));
-        return t;
+    at::Tensor o, stats;
+    const int rc = without_gil([&] {
+        if (!f32) return forward(*q, *k, *v, scale, variant, kind, lo, hi, o, stats);
+        at::Tensor b[3], ob;
+        const at::Tensor* src[3] = {q, k, v};
+        int r = cast(3, src, b, true);
+        if (r == 0) r = forward(b[0], b[1], b[2], scale, variant, kind, lo, hi, ob, stats);
+        if (r != 0) return r;
+        const at::Tensor* back[1] = {&ob};
+        return cast(1, back, &o, false);
     });
+    if (rc != 0) Py_RETURN_NONE;
+    if (kind != kTrain) return THPVariable_Wrap(std::move(o));
+    PyObject* t = PyTuple_New(2);
+    PyTuple_SET_ITEM(t, 0, THPVariable_Wrap(std::move(o)));
+    PyTuple_SET_ITEM(t, 1, THPVariable_Wrap(std::move(stats)));
+    return t;
 }
 
 // bias(q, k, v, mask, scale, variant, square) -> o or None.  BF16, mask [B,H,Sq,Skv] with contiguous rows.
-PyObject* py_bias(PyObject*, PyObject* const* a, Py_ssize_t n) {
+PyObject* py_bias(PyObject* const* a, Py_ssize_t n) {
     const at::Tensor *q, *k, *v, *m;
     double scale;
     int variant, square;
-    if (n != 7 || !tensor_arg(a[0], q) || !tensor_arg(a[1], k) || !tensor_arg(a[2], v) || !tensor_arg(a[3], m) || !double_arg(a[4], scale) ||
+    if (intercepted() || n != 7 || !tensor_arg(a[0], q) || !tensor_arg(a[1], k) || !tensor_arg(a[2], v) || !tensor_arg(a[3], m) || !double_arg(a[4], scale) ||
         !int_arg(a[5], variant) || !int_arg(a[6], square))
         Py_RETURN_NONE;
     if (!shapes_ok(*q, *k, *v, square != 0) || q->scalar_type() != at::kBFloat16 || m->scalar_type() != at::kBFloat16) Py_RETURN_NONE;
     const int B = q->size(0), Sq = q->size(1), H = q->size(2), D = q->size(3), Skv = k->size(1);
     if (m->dim() != 4 || m->device() != q->device() || m->size(0) != B || m->size(1) != H || m->size(2) != Sq || m->size(3) != Skv || m->stride(3) != 1)
         Py_RETURN_NONE;
-    return guarded([&]() -> PyObject* {
-        at::Tensor o;
-        const int rc = without_gil([&] {
-            const size_t need = api.workspace_bytes(B, H, Sq, Skv, D, variant);
-            if (need == 0) return MI355_SAGE_EUNSUPPORTED;
-            void* st = stream_of(*q);
-            o = like(*q, at::kBFloat16);
-            const at::Tensor ws = workspace(at_least(need), q->device(), st);
-            const Strides qs = bshd(*q), ks = bshd(*k), ms{{m->stride(0), m->stride(1), m->stride(2), 1}};
-            return api.mask_any(q->data_ptr(), k->data_ptr(), v->data_ptr(), m->data_ptr(), o.data_ptr(), B, H, Sq, Skv, D, (float)scale, qs.s,
-                                ks.s, ks.s, ms.s, qs.s, 0, 0, 0, 0, 0, st, variant, ws.data_ptr(), (size_t)ws.numel());
-        });
-        if (rc != 0) Py_RETURN_NONE;
-        return THPVariable_Wrap(std::move(o));
+    at::Tensor o;
+    const int rc = without_gil([&] {
+        const size_t need = api.workspace_bytes(B, H, Sq, Skv, D, variant);
+        if (need == 0) return MI355_SAGE_EUNSUPPORTED;
+        void* st = stream_of(*q);
+        o = like(*q, at::kBFloat16);
+        const at::Tensor ws = workspace(at_least(need), q->device(), st);
+        const Strides qs = bshd(*q), ks = bshd(*k), ms{{m->stride(0), m->stride(1), m->stride(2), 1}};
+        return api.mask_any(q->data_ptr(), k->data_ptr(), v->data_ptr(), m->data_ptr(), o.data_ptr(), B, H, Sq, Skv, D, (float)scale, qs.s,
+                            ks.s, ks.s, ms.s, qs.s, 0, 0, 0, 0, 0, st, variant, ws.data_ptr(), (size_t)ws.numel());
     });
+    if (rc != 0) Py_RETURN_NONE;
+    return THPVariable_Wrap(std::move(o));
 }
 
 // norm_rope(q, k, v, q_gain, k_gain, eps, cos, sin, scale, variant, blkq, blkk, k_flags, layout, train)
 //   -> o, (o, stats) with train, or None.  BF16 with BF16 gains; layout as in the C ABI, without the table bit.
-PyObject* py_norm_rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
+PyObject* py_norm_rope(PyObject* const* a, Py_ssize_t n) {
     const at::Tensor *q, *k, *v, *gq, *gk, *cs = nullptr, *sn = nullptr;
     double eps, scale;
     int variant, blkq, blkk, k_flags, layout, train;
-    if (n != 15 || !tensor_arg(a[0], q) || !tensor_arg(a[1], k) || !tensor_arg(a[2], v) || !tensor_arg(a[3], gq) || !tensor_arg(a[4], gk) ||
+    if (intercepted() || n != 15 || !tensor_arg(a[0], q) || !tensor_arg(a[1], k) || !tensor_arg(a[2], v) || !tensor_arg(a[3], gq) || !tensor_arg(a[4], gk) ||
         !double_arg(a[5], eps) || !double_arg(a[8], scale) || !int_arg(a[9], variant) || !int_arg(a[10], blkq) || !int_arg(a[11], blkk) ||
         !int_arg(a[12], k_flags) || !int_arg(a[13], layout) || !int_arg(a[14], train))
         Py_RETURN_NONE;
@@ -298,40 +310,38 @@ PyObject* py_norm_rope(PyObject*, PyObject* const* a, Py_ssize_t n) {
         if (cs->size(0) == (int64_t)B * S * H && B > 1) batch_rows = (int64_t)S * H;
         else if (cs->size(0) != (int64_t)S * H) Py_RETURN_NONE;
     }
-    return guarded([&]() -> PyObject* {
-        at::Tensor o, stats;
-        const int rc = without_gil([&] {
-            const size_t need = api.workspace_bytes(B, H, S, S, D, variant);
-            if (need == 0) return MI355_SAGE_EUNSUPPORTED;
-            void* st = stream_of(*q);
-            o = like(*q, at::kBFloat16);
-            if (train) stats = at::empty({B, H, S, 1}, q->options().dtype(at::kFloat).requires_grad(false));
-            const at::Tensor ws = workspace(at_least(need), q->device(), st);
-            const Strides s = bshd(*q);
-            const void *pc = cs ? cs->data_ptr() : nullptr, *ps = sn ? sn->data_ptr() : nullptr;
-            if (train)
-                return api.norm_rope_train(q->data_ptr(), k->data_ptr(), v->data_ptr(), o.data_ptr(), stats.data_ptr(), B, H, S, S, D, (float)scale,
-                                           s.s, s.s, s.s, s.s, 0, 0, 0, 0, 0, 0, S, S, st, variant, gq->data_ptr(), gk->data_ptr(), (float)eps, pc,
-                                           ps, batch_rows, layout, ws.data_ptr(), (size_t)ws.numel());
-            return api.norm_rope(q->data_ptr(), k->data_ptr(), v->data_ptr(), o.data_ptr(), B, H, S, S, D, (float)scale, s.s, s.s, s.s, s.s, 0, 0, 0,
-                                 0, 0, st, variant, blkq, blkk, k_flags, gq->data_ptr(), gk->data_ptr(), (float)eps, pc, ps, batch_rows, layout,
-                                 ws.data_ptr(), (size_t)ws.numel());
-        });
-        if (rc != 0) Py_RETURN_NONE;
-        if (!train) return THPVariable_Wrap(std::move(o));
-        PyObject* t = PyTuple_New(2);
-        PyTuple_SET_ITEM(t, 0, THPVariable_Wrap(std::move(o)));
-        PyTuple_SET_ITEM(t, 1, THPVariable_Wrap(std::move(stats)));
-        return t;
+    at::Tensor o, stats;
+    const int rc = without_gil([&] {
+        const size_t need = api.workspace_bytes(B, H, S, S, D, variant);
+        if (need == 0) return MI355_SAGE_EUNSUPPORTED;
+        void* st = stream_of(*q);
+        o = like(*q, at::kBFloat16);
+        if (train) stats = at::empty({B, H, S, 1}, q->options().dtype(at::kFloat).requires_grad(false));
+        const at::Tensor ws = workspace(at_least(need), q->device(), st);
+        const Strides s = bshd(*q);
+        const void *pc = cs ? cs->data_ptr() : nullptr, *ps = sn ? sn->data_ptr() : nullptr;
+        if (train)
+            return api.norm_rope_train(q->data_ptr(), k->data_ptr(), v->data_ptr(), o.data_ptr(), stats.data_ptr(), B, H, S, S, D, (float)scale,
+                                       s.s, s.s, s.s, s.s, 0, 0, 0, 0, 0, 0, S, S, st, variant, gq->data_ptr(), gk->data_ptr(), (float)eps, pc,
+                                       ps, batch_rows, layout, ws.data_ptr(), (size_t)ws.numel());
+        return api.norm_rope(q->data_ptr(), k->data_ptr(), v->data_ptr(), o.data_ptr(), B, H, S, S, D, (float)scale, s.s, s.s, s.s, s.s, 0, 0, 0,
+                             0, 0, st, variant, blkq, blkk, k_flags, gq->data_ptr(), gk->data_ptr(), (float)eps, pc, ps, batch_rows, layout,
+                             ws.data_ptr(), (size_t)ws.numel());
     });
+    if (rc != 0) Py_RETURN_NONE;
+    if (!train) return THPVariable_Wrap(std::move(o));
+    PyObject* t = PyTuple_New(2);
+    PyTuple_SET_ITEM(t, 0, THPVariable_Wrap(std::move(o)));
+    PyTuple_SET_ITEM(t, 1, THPVariable_Wrap(std::move(stats)));
+    return t;
 }
 
 // bwd(q, k, v, o, d_out, stats, scale, real_q, real_kv) -> (d_q, d_k, d_v) or None.  BF16, Stats F32 contiguous.
-PyObject* py_bwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
+PyObject* py_bwd(PyObject* const* a, Py_ssize_t n) {
     const at::Tensor *q, *k, *v, *o, *d, *st;
     double scale;
     int rq, rk;
-    if (n != 9 || !tensor_arg(a[0], q) || !tensor_arg(a[1], k) || !tensor_arg(a[2], v) || !tensor_arg(a[3], o) || !tensor_arg(a[4], d) ||
+    if (intercepted() || n != 9 || !tensor_arg(a[0], q) || !tensor_arg(a[1], k) || !tensor_arg(a[2], v) || !tensor_arg(a[3], o) || !tensor_arg(a[4], d) ||
         !tensor_arg(a[5], st) || !double_arg(a[6], scale) || !int_arg(a[7], rq) || !int_arg(a[8], rk))
         Py_RETURN_NONE;
     if (!shapes_ok(*q, *k, *v, false) || q->scalar_type() != at::kBFloat16) Py_RETURN_NONE;
@@ -340,46 +350,43 @@ PyObject* py_bwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (st->scalar_type() != at::kFloat || !st->is_cuda() || !st->is_contiguous() || st->device() != q->device() ||
         st->numel() != q->size(0) * q->size(1) * q->size(2))
         Py_RETURN_NONE;
-    return guarded([&]() -> PyObject* {
-        at::Tensor g[3];
-        if (without_gil([&] { return backward(*q, *k, *v, *o, *d, *st, scale, rq, rk, g); }) != 0) Py_RETURN_NONE;
-        PyObject* t = PyTuple_New(3);
-        for (int i = 0; i < 3; i++) PyTuple_SET_ITEM(t, i, THPVariable_Wrap(std::move(g[i])));
-        return t;
-    });
+    at::Tensor g[3];
+    if (without_gil([&] { return backward(*q, *k, *v, *o, *d, *st, scale, rq, rk, g); }) != 0) Py_RETURN_NONE;
+    PyObject* t = PyTuple_New(3);
+    for (int i = 0; i < 3; i++) PyTuple_SET_ITEM(t, i, THPVariable_Wrap(std::move(g[i])));
+    return t;
 }
 
 // record(q, k, v, scale, variant) -> att with its node, or None.
-PyObject* py_record(PyObject*, PyObject* const* a, Py_ssize_t n) {
+PyObject* py_record(PyObject* const* a, Py_ssize_t n) {
     const at::Tensor *q, *k, *v;
     double scale;
     int variant;
-    if (n != 5 || !tensor_arg(a[0], q) || !tensor_arg(a[1], k) || !tensor_arg(a[2], v) || !double_arg(a[3], scale) || !int_arg(a[4], variant))
+    if (intercepted() || n != 5 || !tensor_arg(a[0], q) || !tensor_arg(a[1], k) || !tensor_arg(a[2], v) || !double_arg(a[3], scale) || !int_arg(a[4], variant))
         Py_RETURN_NONE;
     if (!shapes_ok(*q, *k, *v, true) || (q->scalar_type() != at::kBFloat16 && q->scalar_type() != at::kFloat)) Py_RETURN_NONE;
     // (what the kernels would refuse is left to the Python path, so that nothing can fail inside the node)
     if ((q->size(3) != 64 && q->size(3) != 128) || (variant != 0 && variant != 1) || !aligned16(*q) || !aligned16(*k) || !aligned16(*v)) Py_RETURN_NONE;
-    return guarded([&]() -> PyObject* {
-        at::Tensor out;
-        without_gil([&] { out = SdpaNode::apply(*q, *k, *v, scale, (int64_t)variant); return 0; });
-        return THPVariable_Wrap(std::move(out));
-    });
+    at::Tensor out;
+    without_gil([&] { out = SdpaNode::apply(*q, *k, *v, scale, (int64_t)variant); return 0; });
+    return THPVariable_Wrap(std::move(out));
 }
 
 // workspace(nbytes, tensor) -> this (device, stream)'s buffer
-PyObject* py_workspace(PyObject*, PyObject* const* a, Py_ssize_t n) {
-    const at::Tensor* t;
-    if (n != 2 || !PyLong_Check(a[0]) || !tensor_arg(a[1], t)) {
+PyObject* py_workspace(PyObject* const* a, Py_ssize_t n) {
+    if (n != 2 || !PyLong_Check(a[0]) || !THPVariable_Check(a[1])) {
         PyErr_SetString(PyExc_TypeError, "workspace(nbytes, tensor)");
         return nullptr;
     }
+    const at::Tensor* t = &THPVariable_Unpack(a[1]);
+    TORCH_CHECK(plain(*t), "workspace: not a tensor with device memory");
     const size_t nbytes = PyLong_AsSize_t(a[0]);
     if (PyErr_Occurred()) return nullptr;
-    return guarded([&]() -> PyObject* { return THPVariable_Wrap(workspace(nbytes, t->device(), stream_of(*t))); });
+    return THPVariable_Wrap(workspace(nbytes, t->device(), stream_of(*t)));
 }
 
 // bind(addresses): the C ABI entry points, in the order of Api
-PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
+PyObject* py_bind(PyObject* const* a, Py_ssize_t n) {
     if (n != kApiEntries) {
         PyErr_Format(PyExc_TypeError, "bind: %d addresses expected", kApiEntries);
         return nullptr;
@@ -393,7 +400,7 @@ PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Py_RETURN_NONE;
 }
 
-#define METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(py_##name)), METH_FASTCALL, nullptr}
+#define METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(entry<py_##name>)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {METHOD(fwd), METHOD(bias), METHOD(norm_rope), METHOD(bwd), METHOD(record), METHOD(workspace), METHOD(bind), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_sage_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -88,3 +88,42 @@ def test_native_path_leaves_what_it_does_not_take():
     with pytest.raises(A.Error, match="shim rc=-2"):
         A.sdpa_nomask(t, t, t, 0.1, 7)
     assert np.isfinite(A.sdpa_nomask(t.float(), t.float(), t.float(), 0.1).cpu().numpy()).all()
+
+
+def test_subclasses_modes_and_exception_types():
+    """A subclass's result is of its type, a mode sees plain tensors and leaves the shared workspace plain, running out of
+    memory is torch's own exception: each as the Python path has it, with the native path's bits."""
+    import torch
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from mojodiffusion_amd import attention_sage as A
+
+    class Sub(torch.Tensor):
+        pass
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    torch.manual_seed(2)
+    t = torch.randn((1, 130, 2, 64), device="cuda").bfloat16()
+    want = A.sdpa_nomask(t, t, t, 0.125)
+    s = t.clone().as_subclass(Sub)
+    got = A.sdpa_nomask(s, s, s, 0.125)
+    assert type(got) is Sub and torch.equal(got.as_subclass(torch.Tensor), want)
+    p = torch.nn.Parameter(t)
+    assert type(A.sdpa_nomask(p, p, p, 0.125)) is torch.Tensor
+    with Mode():
+        assert _lib.host().fwd(t, t, t, 0.125, 0, 0, 0, 0, 1) is None
+        assert torch.equal(A.sdpa_nomask(t, t, t, 0.125), want)
+    with torch.cuda.stream(torch.cuda.Stream()):                # a stream without a workspace yet
+        with FakeTensorMode() as fake:
+            f = fake.from_tensor(t)
+            with pytest.raises(RuntimeError):
+                A.sdpa_nomask(f, f, f, 0.125)
+        torch.cuda.synchronize()
+        assert torch.equal(A.sdpa_nomask(t, t, t, 0.125), want)
+    with pytest.raises(torch.OutOfMemoryError):
+        _lib.host().workspace(1 << 50, t)
+    torch.cuda.synchronize()
+    assert torch.equal(A.sdpa_nomask(t, t, t, 0.125), want)
