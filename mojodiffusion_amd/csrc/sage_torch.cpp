@@ -42,16 +42,21 @@ void* stream_of(const at::Tensor& t) { return c10::hip::getCurrentHIPStream(t.de
 // One growing buffer per (device, stream): steady-state calls allocate nothing and calls on different streams
 // never share scratch memory.  A replaced buffer stays valid for the work queued on its stream: the
 // allocator hands its memory out again only to that stream.  (Never destroyed: the device may be gone by then.)
+// Order of locks: g_ws_mutex is taken without the interpreter's lock, because what happens under it — an
+// allocation, the end of a tensor that Python has seen — may wait for that one.
 std::mutex g_ws_mutex;
 auto& g_ws = *new std::map<std::pair<int, void*>, at::Tensor>;
 
 at::Tensor workspace(size_t nbytes, const at::Device& dev, void* stream) {
+    at::Tensor replaced;                // (dies after the lock is released)
     std::lock_guard<std::mutex> lock(g_ws_mutex);
     // (plain memory also when a mode is on for this thread: the buffer outlives it)
     c10::impl::ForceDispatchKeyGuard no_modes(c10::default_included_set, c10::default_excluded_set);
     at::Tensor& ws = g_ws[{dev.index(), stream}];
-    if (!ws.defined() || (size_t)ws.numel() < nbytes)
-        ws = at::empty({(int64_t)nbytes}, at::TensorOptions().dtype(at::kByte).device(dev));
+    if (!ws.defined() || (size_t)ws.numel() < nbytes) {
+        at::Tensor grown = at::empty({(int64_t)nbytes}, at::TensorOptions().dtype(at::kByte).device(dev));
+        replaced = std::exchange(ws, std::move(grown));
+    }
     return ws;
 }
 size_t at_least(size_t n) { return n < 256 ? 256 : n; }
@@ -382,7 +387,9 @@ PyObject* py_workspace(PyObject* const* a, Py_ssize_t n) {
     TORCH_CHECK(plain(*t), "workspace: not a tensor with device memory");
     const size_t nbytes = PyLong_AsSize_t(a[0]);
     if (PyErr_Occurred()) return nullptr;
-    return THPVariable_Wrap(workspace(nbytes, t->device(), stream_of(*t)));
+    at::Tensor ws;
+    without_gil([&] { ws = workspace(nbytes, t->device(), stream_of(*t)); return 0; });
+    return THPVariable_Wrap(std::move(ws));
 }
 
 // bind(addresses): the C ABI entry points, in the order of Api

@@ -127,3 +127,34 @@ def test_subclasses_modes_and_exception_types():
         _lib.host().workspace(1 << 50, t)
     torch.cuda.synchronize()
     assert torch.equal(A.sdpa_nomask(t, t, t, 0.125), want)
+
+
+def test_threads_that_grow_workspaces_python_has_seen():
+    """F16 storage takes the Python path, which sees the stream's workspace; the larger BF16 call behind it replaces that
+    buffer natively.  Several threads at once, a stream each, finish with the results of one thread alone."""
+    import threading
+    import torch
+    from mojodiffusion_amd import attention_sage as A
+    torch.manual_seed(4)
+    sizes = list(range(64, 1600, 96))
+    x = [torch.randn((1, n, 2, 64), device="cuda") for n in sizes]
+    call = lambda t: (A.sdpa_nomask(t.half(), t.half(), t.half(), 0.125), A.sdpa_nomask(t.bfloat16(), t.bfloat16(), t.bfloat16(), 0.125))
+    want = [call(t) for t in x]
+    torch.cuda.synchronize()
+    got = {}
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            r = [call(t) for t in x]
+            torch.cuda.current_stream().synchronize()
+        got[i] = r
+
+    threads = [threading.Thread(target=work, args=(i,), daemon=True) for i in range(6)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+        assert not t.is_alive(), "the threads wait for each other"
+    for i in range(6):
+        for a, b in zip(got[i], want):
+            assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
