@@ -163,6 +163,14 @@ int internal_workspace(std::vector<StreamWs>& registry, size_t need, hipStream_t
     return 0;
 }
 
+// A call's launches go out together: threads that call on one stream share its workspace (the library's own, or the
+// host path's), which is safe in stream order only if no other call's launches fall between them.  One mutex per
+// stream, by hash (streams that share one wait for each other's few microseconds of submission); uncontended ~20 ns.
+std::mutex& launch_mutex(hipStream_t stream) {
+    static std::mutex m[64];
+    return m[(reinterpret_cast<uintptr_t>(stream) * 0x9E3779B97F4A7C15ull) >> 58];
+}
+
 // The optional ops in front of the quantizers (RMSNorm + interleaved RoPE of Q and of K).
 struct Pre {
     PreOp q{}, k{};
@@ -329,6 +337,7 @@ int sdpa_impl(const void* Q, const void* K, const void* V, void* O, void* Stats,
     if (kept <= 0) { SAGE_LOG("every key is masked"); return MI355_SAGE_EINVAL; }
 
     hipStream_t st = static_cast<hipStream_t>(stream);
+    std::lock_guard<std::mutex> together(launch_mutex(st));
     const Carve c = carve(B, H, N_q, kv, D, variant);
     uint8_t* ws = static_cast<uint8_t*>(workspace);
     if (ws) {
@@ -775,6 +784,7 @@ int mi355_sage_attn_fwd(const void* q8, const void* qscale, int blkq, const void
     // fixed number of workgroups need hand-over slots, kept per (device, stream) by the library.
     const AttnPlan plan = attn_plan(B, H, N_q, kv_valid, D, variant, false);
     a.main_items = plan.main_items; a.short_kw = plan.short_kw; a.split_wgs = plan.split_wgs;
+    std::lock_guard<std::mutex> together(launch_mutex(static_cast<hipStream_t>(stream)));
     const size_t split_bytes = attn_split_bytes(a.split_wgs, D);
     if (split_bytes > 0 && (rc = internal_workspace(g_split_ws, split_bytes, static_cast<hipStream_t>(stream), &a.split))) return rc;
     SAGE_HIP(launch_attn(a, static_cast<hipStream_t>(stream)));
@@ -922,6 +932,7 @@ int mi355_sage_sdpa_bwd_bf16(const void* Q, const void* K, const void* V, const 
 
     const BwdCarve c = bwd_carve(B, H, N_q, D);
     hipStream_t st = static_cast<hipStream_t>(stream);
+    std::lock_guard<std::mutex> together(launch_mutex(st));
     if (workspace == nullptr) {
         if ((rc = internal_workspace(g_ws, c.total, st, &workspace))) return rc;
     } else if (workspace_bytes < c.total || (reinterpret_cast<uintptr_t>(workspace) & (kAlign - 1))) {

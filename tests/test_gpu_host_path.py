@@ -158,3 +158,45 @@ def test_threads_that_grow_workspaces_python_has_seen():
     for i in range(6):
         for a, b in zip(got[i], want):
             assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+
+
+@pytest.mark.parametrize("entry", ["native", "python", "no_workspace"])
+def test_threads_on_one_stream_share_its_workspace(entry):
+    """Calls of several threads on one stream use one workspace: each has the bits of the call alone, forward, training
+    forward and backward, through the native path, the Python path (F16 storage) and the library's own buffers."""
+    import threading
+    import torch
+    from mojodiffusion_amd import attention_sage as A
+    L = _lib.lib()
+    torch.manual_seed(5)
+    x = [[torch.randn((1, 700, 4, 64), device="cuda").bfloat16() for _ in range(2)] for _ in range(6)]
+    qs = _lib.strides_bhnd(700, 4, 64)
+
+    def call(t, g):
+        if entry == "native":
+            f = A.sdpa_flash_train_fwd(t, t, t, 0.125)
+            b = A.sdpa_flash_backward(f, g, 0.125)
+            return A.sdpa_nomask(t, t, t, 0.125), f.o, f.stats, b.d_q, b.d_k, b.d_v
+        if entry == "python":
+            return (A.sdpa_nomask(t.half(), t.half(), t.half(), 0.125),)
+        o = torch.empty_like(t)
+        assert L.mi355_sage_sdpa_bf16(t.data_ptr(), t.data_ptr(), t.data_ptr(), o.data_ptr(), 1, 4, 700, 700, 64, 0.125, qs, qs, qs, qs, 0, 0, 0, 0, 0,
+                                      torch.cuda.current_stream().cuda_stream, 0, None, 0) == 0
+        return (o,)
+
+    want = [call(*p) for p in x]
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work(i):
+        for rep in range(30):
+            if not all(torch.equal(a, b) for a, b in zip(call(*x[i]), want[i])):
+                wrong.append((i, rep))
+
+    threads = [threading.Thread(target=work, args=(i,), daemon=True) for i in range(6)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+        assert not t.is_alive()
+    assert not wrong, wrong
