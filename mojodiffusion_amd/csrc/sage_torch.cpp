@@ -61,6 +61,15 @@ at::Tensor workspace(size_t nbytes, const at::Device& dev, void* stream) {
 }
 size_t at_least(size_t n) { return n < 256 ? 256 : n; }
 
+// Dense device memory and nothing else.  Every other kind of tensor — fake, functional, batched or wrapped by a
+// transform, dual — carries a dispatch key or a tangent of its own; its sizes may be symbolic and it may have no
+// memory to point to.
+bool plain(const at::Tensor& t) {
+    static const uint64_t keys = c10::DispatchKeySet({c10::DispatchKey::CUDA, c10::DispatchKey::AutogradCUDA, c10::DispatchKey::AutocastCUDA,
+                                                      c10::DispatchKey::ADInplaceOrView}).raw_repr();
+    return t.defined() && (t.key_set().raw_repr() & ~keys) == 0 && !t._fw_grad(0).defined();
+}
+
 struct Strides { int64_t s[4]; };
 Strides bshd(const at::Tensor& t) { return Strides{{t.size(1) * t.size(2) * t.size(3), t.size(3), t.size(2) * t.size(3), 1}}; }
 
@@ -114,6 +123,15 @@ int forward(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, doubl
     return api.sdpa(pq, pk, pv, po, B, H, Sq, Skv, D, (float)scale, qs.s, ks.s, ks.s, qs.s, 0, 0, 0, 0, 0, st, variant, pw, nw);
 }
 
+// What the backward kernels read: shapes, types and devices of the saved set and the upstream gradient.
+bool bwd_set_ok(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& o, const at::Tensor& d, const at::Tensor& st) {
+    if (!shapes_ok(q, k, v, false) || q.scalar_type() != at::kBFloat16) return false;
+    for (const at::Tensor* t : {&o, &d})
+        if (t->scalar_type() != at::kBFloat16 || !device_bhsd(*t) || t->sizes() != q.sizes() || t->device() != q.device()) return false;
+    return st.scalar_type() == at::kFloat && st.is_cuda() && st.is_contiguous() && st.device() == q.device() &&
+           st.numel() == q.size(0) * q.size(1) * q.size(2);
+}
+
 int backward(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& o, const at::Tensor& d_out,
              const at::Tensor& stats, double scale, int real_q, int real_kv, at::Tensor (&g)[3]) {
     const int B = q.size(0), Sq = q.size(1), H = q.size(2), D = q.size(3), Skv = k.size(1);
@@ -163,6 +181,10 @@ struct SdpaNode : torch::autograd::Function<SdpaNode> {
         } else {
             d = d.to(at::kBFloat16);
         }
+        // (saved-tensor hooks may hand back anything)
+        for (const at::Tensor& t : saved) TORCH_CHECK(plain(t), "sdpa_flash_backward_raw: a saved tensor came back without device memory");
+        TORCH_CHECK(bwd_set_ok(q, saved[1], saved[2], saved[3], d, saved[4]),
+                    "sdpa_flash_backward_raw: a saved tensor came back with another shape, type, layout or device");
         const int rc = ::backward(q, saved[1], saved[2], saved[3], d, saved[4], scale, q.size(1), saved[1].size(1), out);
         TORCH_CHECK(rc == 0, "sdpa_flash_backward_raw: shim rc=", rc);
         if (g.scalar_type() == at::kFloat) {
@@ -176,14 +198,6 @@ struct SdpaNode : torch::autograd::Function<SdpaNode> {
 };
 
 // ---- argument access -----------------------------------------------------------------------------
-// Dense device memory and nothing else.  Every other kind of tensor — fake, functional, batched or wrapped by a
-// transform, dual — carries a dispatch key or a tangent of its own; its sizes may be symbolic and it may have no
-// memory to point to.
-bool plain(const at::Tensor& t) {
-    static const uint64_t keys = c10::DispatchKeySet({c10::DispatchKey::CUDA, c10::DispatchKey::AutogradCUDA, c10::DispatchKey::AutocastCUDA,
-                                                      c10::DispatchKey::ADInplaceOrView}).raw_repr();
-    return t.defined() && (t.key_set().raw_repr() & ~keys) == 0 && !t._fw_grad(0).defined();
-}
 // Taken: a plain torch.Tensor or Parameter (a subclass's results are of its type: left to the Python path).
 bool tensor_arg(PyObject* o, const at::Tensor*& t) {
     if (!THPVariable_CheckExact(o)) return false;
@@ -349,12 +363,7 @@ PyObject* py_bwd(PyObject* const* a, Py_ssize_t n) {
     if (intercepted() || n != 9 || !tensor_arg(a[0], q) || !tensor_arg(a[1], k) || !tensor_arg(a[2], v) || !tensor_arg(a[3], o) || !tensor_arg(a[4], d) ||
         !tensor_arg(a[5], st) || !double_arg(a[6], scale) || !int_arg(a[7], rq) || !int_arg(a[8], rk))
         Py_RETURN_NONE;
-    if (!shapes_ok(*q, *k, *v, false) || q->scalar_type() != at::kBFloat16) Py_RETURN_NONE;
-    for (const at::Tensor* t : {o, d})
-        if (t->scalar_type() != at::kBFloat16 || !device_bhsd(*t) || t->sizes() != q->sizes() || t->device() != q->device()) Py_RETURN_NONE;
-    if (st->scalar_type() != at::kFloat || !st->is_cuda() || !st->is_contiguous() || st->device() != q->device() ||
-        st->numel() != q->size(0) * q->size(1) * q->size(2))
-        Py_RETURN_NONE;
+    if (!bwd_set_ok(*q, *k, *v, *o, *d, *st)) Py_RETURN_NONE;
     at::Tensor g[3];
     if (without_gil([&] { return backward(*q, *k, *v, *o, *d, *st, scale, rq, rk, g); }) != 0) Py_RETURN_NONE;
     PyObject* t = PyTuple_New(3);

@@ -200,3 +200,36 @@ def test_threads_on_one_stream_share_its_workspace(entry):
         t.join(60)
         assert not t.is_alive()
     assert not wrong, wrong
+
+
+def test_recorded_node_under_saved_tensor_hooks():
+    """The node saves through torch's hooks: a set that comes back as it was (from host memory, too) gives the same
+    gradients; one that comes back as something else is refused before a kernel reads it."""
+    import torch
+    from mojodiffusion_amd import attention_sage as A
+    torch.manual_seed(6)
+    base = [torch.randn((1, 130, 3, 64), device="cuda").bfloat16() for _ in range(4)]
+
+    def grads(pack, unpack):
+        q, k, v = (t.clone().requires_grad_(True) for t in base[:3])
+        with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+            att = A.record_sdpa(q, k, v, 0.125)
+        return torch.autograd.grad(att, (q, k, v), base[3])
+
+    same = lambda t: t
+    want = grads(same, same)
+    for a, b in zip(grads(lambda t: t.cpu(), lambda t: t.cuda()), want):
+        assert torch.equal(a, b)
+    for unpack in (lambda t: t.cpu(), lambda t: t.half(), lambda t: t[:, :1], lambda t: t.transpose(1, 2), lambda t: t.float().contiguous()):
+        with pytest.raises(RuntimeError):
+            grads(same, unpack)
+
+    class Mark(Exception):
+        pass
+
+    def fail(t):
+        raise Mark("from the hook")
+    with pytest.raises(Mark, match="from the hook"):
+        grads(fail, same)
+    for a, b in zip(grads(same, same), want):
+        assert torch.equal(a, b)
