@@ -183,7 +183,14 @@ def _call_bwd(name, q, k, v, o, d_out, stats, scale, real_q, real_kv):
     r = _lib.host().bwd(q, k, v, o, d_out, stats, scale, real_q, real_kv)
     if r is not None:
         return SdpaFlashGrads(*r)
+    _check_shapes(name, q, k, v, False)
+    if o.shape != q.shape or d_out.shape != q.shape:
+        raise Error("%s: o/d_out shape does not match q [B,S,H,Dh]" % name)
     B, Sq, H, Dh = q.shape
+    if stats.dtype != torch.float32 or stats.numel() != B * H * Sq:
+        raise Error("%s: stats must be F32 [B,H,S,1]" % name)
+    if any(t.device != q.device for t in (k, v, o, d_out, stats)):
+        raise Error("%s: tensors must live on one device" % name)
     Skv = k.shape[1]
     L = _lib.lib()
     d_q, d_k, d_v = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)

@@ -97,3 +97,16 @@ print("done", case, flush=True)
 def test_left_to_the_python_path(case):
     r = subprocess.run([sys.executable, "-c", CHILD, case], capture_output=True, text=True, timeout=300, cwd=_lib.os.path.dirname(_lib._HERE))
     assert r.returncode == 0 and r.stdout.split() == ["done", case], (r.returncode, r.stdout[-500:], r.stderr[-1500:])
+
+
+def test_backward_refuses_a_set_of_another_shape():
+    """The kernels take every extent from q and k: a smaller o, d_out, stats or v is refused before its pointer is used."""
+    import torch
+    from mojodiffusion_amd import attention_sage as A
+    q = torch.zeros((1, 64, 2, 64), dtype=torch.bfloat16)
+    st = torch.zeros((1, 2, 64, 1))
+    half = q[:, :32].contiguous()
+    for bad in ({"o": half}, {"d_out": half}, {"v": half}, {"stats": st[:, :, :32]}, {"stats": st.bfloat16()}, {"stats": st.to("meta")}):
+        a = {"q": q, "k": q, "v": q, "o": q, "d_out": q, "stats": st, **bad}
+        with pytest.raises(A.Error, match="shape|stats|device"):
+            A._call_bwd("bwd", *(a[n] for n in ("q", "k", "v", "o", "d_out", "stats")), 0.1, 64, 64)
