@@ -731,6 +731,8 @@ def _norm_rope_args(name, q_pre, k_pre, v, q_norm, k_norm, cos, sin, halfsplit=F
             flags |= _lib.ROPE_TABLES_BF16
         if cos.shape != sin.shape or cos.dim() != 2 or cos.shape[1] != Dh // 2:
             raise Error("%s: cos/sin must be [rows, D/2]" % name)
+        if cos.device != q_pre.device or sin.device != q_pre.device:
+            raise Error("%s: cos/sin must live on the device of q" % name)
         if cos.shape[0] == B * S * H and B > 1:
             batch_rows = S * H
         elif cos.shape[0] != S * H:

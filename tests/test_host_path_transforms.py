@@ -110,3 +110,18 @@ def test_backward_refuses_a_set_of_another_shape():
         a = {"q": q, "k": q, "v": q, "o": q, "d_out": q, "stats": st, **bad}
         with pytest.raises(A.Error, match="shape|stats|device"):
             A._call_bwd("bwd", *(a[n] for n in ("q", "k", "v", "o", "d_out", "stats")), 0.1, 64, 64)
+
+
+def test_tables_on_the_host_are_refused():
+    """RoPE tables in host memory: an error, not a host pointer in a kernel."""
+    import torch
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from mojodiffusion_amd import attention_sage as A
+    with FakeTensorMode():
+        q = torch.empty((1, 64, 2, 64), device="cuda", dtype=torch.bfloat16)
+        gain = torch.empty((64,), device="cuda", dtype=torch.bfloat16)
+        dev, host = (torch.empty((128, 32), device=d) for d in ("cuda", "cpu"))
+        A._norm_rope_args("f", q, q, q, gain, gain, dev, dev)
+        for cos, sin in ((host, host), (dev, host), (host, dev)):
+            with pytest.raises(A.Error, match="device of q"):
+                A._norm_rope_args("f", q, q, q, gain, gain, cos, sin)
