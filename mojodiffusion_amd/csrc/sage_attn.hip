@@ -434,9 +434,14 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     // both are multiples of 2^-26 below 2^-2), and its constant is the reference alone.
     bool exact_bias = false;
     if constexpr (VARIANT == 1 && !ADDMASK) {
+        // Only rows and keys that count are asked: a scale block without any has scale 1 (rows past N_q, the second half
+        // of the last 128 keys, a masked range), which would send whole waves outside the main loop, and the others
+        // of the workgroup meet them at every tile's barrier ([1,16000,4,128] 389 -> 328 us, [1,5000,12,128] 163 ->
+        // 147, [1,8001,24,128] 599 -> 530, [1,8000,8,64] 163 -> 137).
         float ks_max = 0.0f;
-        for (int i = lane; i < (int)(nkv_pad / 32); i += 64) ks_max = fmaxf(ks_max, lds_ks[KS_OFF + i]);
-        exact_bias = __any(Magic<D>::F * sq * ks_max > kExactBias);
+        for (int i = lane; i * 32 < kv_valid_all; i += 64)
+            if (i * 32 < mask_lo || i * 32 + 32 > mask_hi) ks_max = fmaxf(ks_max, lds_ks[KS_OFF + i]);
+        exact_bias = __any(qrow < Nq && Magic<D>::F * sq * ks_max > kExactBias);
     }
     {
         v4i k0[NQ];
