@@ -453,7 +453,11 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
 #pragma unroll
         for (int n = 0; n < NQ; n++) qk_step(0, n, k0[n]);
     }
-    const int last_step = ntiles * SPT - 1;
+    // Steps come in pairs: an odd number of 64-key steps is followed by one whose keys are all past the end (its copies are
+    // the clamped last tile's, its scores are masked).  Bodies that end an odd number as such had no registers left:
+    // their spills, written and read back by every wave, cost a round of workgroups up to 50 us (e4m3, cross
+    // [1,3840 x 192,32,128] 90.1 -> 42.6 us, [1,4000,16,128] 133.9 -> 116.2, [1,2304,18,256] 193.6 -> 187.1).
+    const int last_step = (ntiles * SPT + 1) / 2 * 2 - 1;
     auto key_step = [&](int h) -> int { return (t_off + key_tile(h / SPT) - h / SPT) * SPT + h; };       // step h's keys: key_step(h) * SK ..
     BiasStage bias[SKB];                                // the next step's bias on its way
     auto bias_load = [&](int h) {
@@ -505,9 +509,10 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
 
         float f[SKB], c0[SKB];
         const int hk = TRIP ? 0 : key_step(h);
+        const int hks = SPT == 1 ? min(hk, (kv_valid_all - 1) / SK) : hk;      // (nothing past the last key is read)
 #pragma unroll
         for (int kb = 0; kb < SKB; kb++)
-            f[kb] = sq * (TRIP ? kst[((HT + PERIOD - 1) % PERIOD) * SKB + kb] : kscale_of(hk * SKB + kb));
+            f[kb] = sq * (TRIP ? kst[((HT + PERIOD - 1) % PERIOD) * SKB + kb] : kscale_of(hks * SKB + kb));
         // Steps that hold masked keys (the ragged end, the masked range) are rare: a real branch.
         // A masked score becomes -inf (as an integer: below every real accumulator), which the
         // exponent path below turns into p = 0 without any further test.
@@ -716,8 +721,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     using X1 = std::integral_constant<int, 1>;
     using R0 = std::integral_constant<int, -1>;                         // ring slots from h at run time; first step of a tile
     using R1 = std::integral_constant<int, SPT == 2 ? -2 : -1>;         // ... the step of odd h
-    // The last step computes no further scores.  (With a single step the first one is also the last;
-    // it computes the scores of the clamped copy and nobody reads them.)
+    // The last step computes no further scores.
     int hs = 1;
     // (the split instantiations sit at the register limit and keep their slots in registers; so do the
     // ones with an additive mask, whose time goes into reading the mask anyway)
@@ -730,7 +734,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         const bool range = mask_hi > mask_lo && t_off * kTileKV < mask_hi;
         int clean = (kv_valid - t_off * kTileKV) / SK - skip * SPT;
         if (causal) clean = min(clean, (wave_row0 + 1) / SK);       // steps whose every key is <= the wave's first row
-        const int tail_end = exact_bias ? 0 : min(last_step - SPT * (KOFF + LEAD) + (SPT - 1), clean);
+        const int tail_end = exact_bias ? 0 : min((ntiles - KOFF - LEAD) * SPT - 1 + (SPT - 1), clean);
         int trip_end = tail_end, past = 0, resume = 0;
         if (range) {
             trip_end = min(trip_end, max(mask_lo - t_off * kTileKV, 0) / SK);
@@ -777,34 +781,26 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
             step(hs + 1, X0{}, R0{}, F{}, T{});
         }
     }
-    if (hs == last_step) {
-        step(hs, X1{}, R1{}, F{}, F{});
-    } else if constexpr (SPT == 1) {                    // (with two steps per tile the last step is an odd one)
-        if (hs + 1 == last_step) {
-            step(hs, X1{}, R1{}, F{}, T{});
-            step(hs + 1, X0{}, R0{}, F{}, F{});
-        }
-    }
+    // (always so; without the question the loop in front of it is compiled with its addresses kept across it: 20 % slower
+    // at 256 channels)
+    if (hs == last_step) step(hs, X1{}, R1{}, F{}, F{});
     // ---- drain: P.V of the last step ------------------------------------------------------
-    auto drain = [&](auto x_tag) {
-        constexpr int X = decltype(x_tag)::value;
+    {
         v4i vd[NPV][FPU];
         auto read_vd = [&](int u) {
             const int j = VARIANT == 0 ? 2 * (SPT - 1) + u / DB : 0, d = u % DB;
 #pragma unroll
             for (int x = 0; x < FPU; x++)
-                vd[u][x] = v_frag(last % NSV, j * FPU + x, d);
+                vd[u][x] = v_frag((SPT == 2 ? last : last_step) % NSV, j * FPU + x, d);
         };
 #pragma unroll
         for (int u = 0; u < PD && u < NPV; u++) read_vd(u);
 #pragma unroll
         for (int u = 0; u < NPV; u++) {
             if (u + PD < NPV) read_vd(u + PD);
-            pv_unit(X, u, vd[u]);
+            pv_unit(1, u, vd[u]);
         }
-    };
-    if (SPT == 2 || (last_step & 1)) drain(X1{});
-    else drain(X0{});
+    }
 
     // Hand-over between workgroups of ONE XCD goes through that XCD's L2, which every compute unit
     // of the XCD reads and writes: the producer only has to wait until its stores have left the

@@ -35,3 +35,40 @@ def test_scales_of_padding_do_not_matter(variant, wid, Sq, Skv, mask):
         L.mi355_sage_set_attn_split(0)
     assert torch.isfinite(torch.from_numpy(out[0].astype(np.int32) << 16).view(torch.float32)).all()
     np.testing.assert_array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("variant,D", [(1, 64), (1, 128), (1, 256), (0, 128)])
+@pytest.mark.parametrize("kv_valid", [1, 64, 100, 128, 150, 300, 449, 577])
+def test_nothing_past_the_last_key_matters(oracle, variant, D, kv_valid):
+    """One to ten key tiles, odd and even, of operands that go on behind them: V of the tiles behind as NaN, their scales as
+    NaN.  The main kernel's bits are those of operands that end there; both meet the checker's bar."""
+    import torch
+    import gpu_harness as H
+    from mojodiffusion_amd import _lib
+    from mojodiffusion_amd.workloads import bf16_bits_to_f32
+    w = WORKLOADS[2].scaled(B=1, H=2, S=640)
+    Sq, blkq = 300, 128 if variant == 0 else 32
+    rng = np.random.default_rng(kv_valid + D)
+    q, k, v = (np.ascontiguousarray((rng.standard_normal((1, n, 2, D)).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16))
+               for n in (Sq, kv_valid, kv_valid))
+    scale = D ** -0.5
+    g = H.quant_qk(q, k, scale, blkq, 64, True)["dev"]
+    gv = H.quant_v(v, variant)["dev"]
+    n = (kv_valid + 63) // 64                                       # key tiles that hold a key
+    k8 = torch.full((1, 2, 640, D), 99, dtype=torch.int8, device="cuda")
+    k8[:, :, :n * 64] = g["k8"][:, :, :n * 64]
+    ks = torch.full((1, 2, 10), float("nan"), device="cuda")
+    ks[..., :n] = g["kscale"][..., :n]
+    vq = torch.full((1, 2, 10, D, 64), 0x7E00 if variant == 0 else 0x7F, dtype=gv["vq"].dtype, device="cuda")
+    vq[:, :, :n] = gv["vq"].view(1, 2, -1, D, 64)[:, :, :n]
+    L = _lib.lib()
+    assert L.mi355_sage_set_attn_split(-1) == 0                     # the main kernel, whatever the size
+    try:
+        want, ws = H.attn_fwd(g["q8"], g["qscale"], blkq, g["k8"], g["kscale"], 64, gv["vq"], gv.get("vscale"), variant, Sq, kv_valid, want_stats=True)
+        got, gs = H.attn_fwd(g["q8"], g["qscale"], blkq, k8, ks, 64, vq, gv.get("vscale"), variant, Sq, 640, kv_valid=kv_valid, want_stats=True)
+    finally:
+        L.mi355_sage_set_attn_split(0)
+    np.testing.assert_array_equal(got, want)
+    np.testing.assert_array_equal(gs, ws)
+    _, ref = oracle.sdpa_bf16(q, k, v, scale, variant=variant, blkq=blkq, blkk=64)
+    assert np.isfinite(bf16_bits_to_f32(got)).all() and np.abs(bf16_bits_to_f32(got) - ref).max() <= 2e-2
