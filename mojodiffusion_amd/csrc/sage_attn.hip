@@ -47,7 +47,12 @@ static __device__ unsigned int g_split_faults;
 // wave in the prologue — the quantize stage's arithmetic (quant_i8_block), so the codes and scales
 // are the ones that stage would have written — which saves the stage a read of Q and a write and
 // this kernel's read of the codes.
-template <int D, int VARIANT, bool STATS, bool ADDMASK, bool SPLIT, bool QF = false>
+//
+// RANGE: the call masks a range of keys.  Instantiations of their own, because what leaves tiles out and goes on behind
+// the range costs the ones that have none registers and addresses in their last steps (one-shot call, us with it -> without,
+// no range masked: e4m3 [1,2304,18,256] 187.0 -> 179.6, cross [1,3840 x 333,32,128] 50.4 -> 47.9; fp16 [2,4352,30,128] 476.2
+// -> 473.9, [1,2304,18,256] 165.0 -> 162.8).
+template <int D, int VARIANT, bool STATS, bool ADDMASK, bool SPLIT, bool RANGE = false, bool QF = false>
 __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     const int8_t* __restrict__ q8, const float* __restrict__ qscale, int blkq,
     const uint16_t* __restrict__ q_src, int64_t qsb, int64_t qsh, int64_t qsn, const float* __restrict__ qmul,
@@ -96,6 +101,8 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     __shared__ float lds_qmax[QF ? 8 : 1];              // QF: largest |pre-scaled q| of each wave's 32 rows
     __shared__ __attribute__((aligned(16))) uint8_t lds_qc[QF && VARIANT == 1 ? NW * 32 * D : 16];      // QF: Q codes on their way into fragments
     static_assert(!(STATS && ADDMASK), "no entry point asks for Stats under an additive mask");
+    static_assert(!RANGE || (!ADDMASK && !SPLIT), "no entry point masks a range under an additive mask; the split schedule tests every step");
+    constexpr bool MASKED = RANGE || SPLIT;             // mask_lo .. mask_hi may hold keys (otherwise the launcher has seen that it does not)
     static_assert(!QF || (D <= 128 && !STATS && !ADDMASK && !SPLIT), "Q is encoded in the kernel only in the plain forward");
 
     // Work items are (q tile, b*h) pairs, `total_wg` of them; an item takes `ntiles` steps (key
@@ -155,12 +162,12 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     // Key tiles that lie in the masked range as a whole are left out: from here on tile t stands for key tile
     // t, or t + skip from skip_at on.  (An even number of them: the K scales of a trip are read 16 bytes at a time.)
     int skip_at = 0, skip = 0;
-    if (!SPLIT && !causal && mask_hi > mask_lo) {
+    if (RANGE && !causal) {
         skip_at = (mask_lo + kTileKV - 1) / kTileKV;
         skip = max(min(mask_hi, kv_valid) / kTileKV - skip_at, 0) & ~1;
     }
     const int ntiles = SPLIT ? span_end - item_base - t_off : (kv_valid + kTileKV - 1) / kTileKV - skip;
-    auto key_tile = [&](int t) -> int { return SPLIT || t < skip_at ? t : t + skip; };
+    auto key_tile = [&](int t) -> int { return !RANGE || t < skip_at ? t : t + skip; };
     const bool seg_finishes = !SPLIT || t_off + ntiles == ntiles_item;   // holds the item's last key tile: writes the output
     span_end = item_base + t_off;
     const int64_t bh = (uint32_t)wg / (uint32_t)qtiles_div;
@@ -440,7 +447,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         // 147, [1,8001,24,128] 599 -> 530, [1,8000,8,64] 163 -> 137).
         float ks_max = 0.0f;
         for (int i = lane; i * 32 < kv_valid_all; i += 64)
-            if (i * 32 < mask_lo || i * 32 + 32 > mask_hi) ks_max = fmaxf(ks_max, lds_ks[KS_OFF + i]);
+            if (!MASKED || i * 32 < mask_lo || i * 32 + 32 > mask_hi) ks_max = fmaxf(ks_max, lds_ks[KS_OFF + i]);
         exact_bias = __any(qrow < Nq && Magic<D>::F * sq * ks_max > kExactBias);
     }
     {
@@ -517,7 +524,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         // A masked score becomes -inf (as an integer: below every real accumulator), which the
         // exponent path below turns into p = 0 without any further test.
         const int key0 = hk * SK;
-        if (!TRIP && __builtin_expect(key0 + SK > kv_valid || (key0 < mask_hi && key0 + SK > mask_lo) ||
+        if (!TRIP && __builtin_expect(key0 + SK > kv_valid || (MASKED && key0 < mask_hi && key0 + SK > mask_lo) ||
                                       (causal && key0 + SK - 1 > wave_row0), 0)) {
             asm volatile("" ::: "memory");
 #pragma unroll
@@ -525,7 +532,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
 #pragma unroll
                 for (int i = 0; i < 16; i++) {
                     const int key = key0 + kb * 32 + (i >> 2) * 8 + half * 4 + (i & 3);
-                    if (key >= kv_valid || (key >= mask_lo && key < mask_hi) || (causal && key > qrow)) s[X][kb][i] = (int)0xFF800000;
+                    if (key >= kv_valid || (MASKED && key >= mask_lo && key < mask_hi) || (causal && key > qrow)) s[X][kb][i] = (int)0xFF800000;
                 }
         }
         // biased scores in the log2 domain, without the reference maximum (ADDMASK only)
@@ -731,7 +738,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         // of the masked range or the ragged end, then — the steps that touch the range, at most a few, go
         // through the general bodies — those between the range and the ragged end.  Either stretch stops
         // early enough that the copies a trip starts need no clamping and do not cross the left-out tiles.
-        const bool range = mask_hi > mask_lo && t_off * kTileKV < mask_hi;
+        const bool range = RANGE && t_off * kTileKV < mask_hi;
         int clean = (kv_valid - t_off * kTileKV) / SK - skip * SPT;
         if (causal) clean = min(clean, (wave_row0 + 1) / SK);       // steps whose every key is <= the wave's first row
         const int tail_end = exact_bias ? 0 : min((ntiles - KOFF - LEAD) * SPT - 1 + (SPT - 1), clean);
@@ -765,7 +772,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
             }
         }
         // the steps up to the next stretch, or to the end: ring slots from the step number (hs is odd here)
-        const bool again = resume > hs && resume + PERIOD <= tail_end;
+        const bool again = RANGE && resume > hs && resume + PERIOD <= tail_end;
         for (const int stop = again ? resume + 1 : last_step; hs + 1 < stop; hs += 2) {
             step(hs, X1{}, R1{}, F{}, T{});
             step(hs + 1, X0{}, R0{}, F{}, T{});
@@ -964,33 +971,39 @@ static hipError_t launch_attn_dv(const AttnArgs& a, hipStream_t st) {
         hipLaunchKernelGGL(split_clear_kernel, dim3(1), dim3(256), 0, st, flags, split);
     }
     dim3 grid((unsigned)(split > 0 ? split : total)), block(kThreads);
-#define SAGE_LAUNCH_ATTN2(STATS, ADDMASK, SPLIT)                                                                         \
-    hipLaunchKernelGGL((sage_attn_kernel<D, VARIANT, STATS, ADDMASK, SPLIT>), grid, block, 0, st, a.q8, a.qscale, a.blkq, \
+    const bool range = a.km.hi > a.km.lo;
+#define SAGE_LAUNCH_ATTN2(STATS, ADDMASK, SPLIT, RANGE)                                                                  \
+    hipLaunchKernelGGL((sage_attn_kernel<D, VARIANT, STATS, ADDMASK, SPLIT, RANGE>), grid, block, 0, st, a.q8, a.qscale, a.blkq, \
                        a.q_src, a.qsb, a.qsh, a.qsn, a.qmul, a.k8, a.kscale, a.blkk, (const uint8_t*)a.vq, a.vscale, a.qshift, a.H, a.Nq, a.kv_valid,          \
                        a.km.lo, a.km.hi, a.causal, a.nq_pad, a.nkv_pad, a.o, a.osb, a.osh, a.osn, a.stats, n_qtiles,               \
                        (int)total, a.amask, a.amb, a.amh, a.amn, split >> 3, part, flags, g_split_wait.load())
-#define SAGE_LAUNCH_ATTN(STATS, ADDMASK)                                  \
-    do {                                                                  \
-        if constexpr (D <= 128 && VARIANT == 0) {                         \
-            if (split > 0) SAGE_LAUNCH_ATTN2(STATS, ADDMASK, true);       \
-            else SAGE_LAUNCH_ATTN2(STATS, ADDMASK, false);                \
-        } else {                                                          \
-            SAGE_LAUNCH_ATTN2(STATS, ADDMASK, false);                     \
-        }                                                                 \
+#define SAGE_LAUNCH_ATTN(STATS, ADDMASK)                                               \
+    do {                                                                               \
+        if constexpr (D <= 128 && VARIANT == 0) {                                      \
+            if (split > 0) { SAGE_LAUNCH_ATTN2(STATS, ADDMASK, true, false); break; }  \
+        }                                                                              \
+        if constexpr (!ADDMASK) {                                                      \
+            if (range) { SAGE_LAUNCH_ATTN2(STATS, ADDMASK, false, true); break; }      \
+        }                                                                              \
+        SAGE_LAUNCH_ATTN2(STATS, ADDMASK, false, false);                               \
     } while (0)
     if (a.q_src != nullptr) {
         // Q encoded by the kernel: the plain forward only
         if constexpr (D <= 128) {
             if (a.amask != nullptr || a.stats != nullptr || split > 0 || a.qmul == nullptr) return hipErrorInvalidValue;
-            hipLaunchKernelGGL((sage_attn_kernel<D, VARIANT, false, false, false, true>), grid, block, 0, st, nullptr, nullptr, a.blkq,
-                               a.q_src, a.qsb, a.qsh, a.qsn, a.qmul, a.k8, a.kscale, a.blkk, (const uint8_t*)a.vq, a.vscale, nullptr,
-                               a.H, a.Nq, a.kv_valid, a.km.lo, a.km.hi, a.causal, a.nq_pad, a.nkv_pad, a.o, a.osb, a.osh, a.osn, nullptr,
-                               n_qtiles, (int)total, nullptr, 0, 0, 0, 0, nullptr, nullptr, g_split_wait.load());
+#define SAGE_LAUNCH_ATTN_QF(RANGE)                                                                                              \
+    hipLaunchKernelGGL((sage_attn_kernel<D, VARIANT, false, false, false, RANGE, true>), grid, block, 0, st, nullptr, nullptr, a.blkq, \
+                       a.q_src, a.qsb, a.qsh, a.qsn, a.qmul, a.k8, a.kscale, a.blkk, (const uint8_t*)a.vq, a.vscale, nullptr,  \
+                       a.H, a.Nq, a.kv_valid, a.km.lo, a.km.hi, a.causal, a.nq_pad, a.nkv_pad, a.o, a.osb, a.osh, a.osn, nullptr, \
+                       n_qtiles, (int)total, nullptr, 0, 0, 0, 0, nullptr, nullptr, g_split_wait.load())
+            if (range) SAGE_LAUNCH_ATTN_QF(true);
+            else SAGE_LAUNCH_ATTN_QF(false);
+#undef SAGE_LAUNCH_ATTN_QF
         } else {
             return hipErrorInvalidValue;
         }
     } else if (a.amask != nullptr) {
-        if (a.stats != nullptr) return hipErrorInvalidValue;      // (no entry point asks for both)
+        if (a.stats != nullptr || range) return hipErrorInvalidValue;      // (no entry point asks for both)
         SAGE_LAUNCH_ATTN(false, true);
     } else {
         if (a.stats != nullptr) SAGE_LAUNCH_ATTN(true, false);
