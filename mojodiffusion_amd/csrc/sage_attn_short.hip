@@ -435,16 +435,19 @@ hipError_t launch_attn_short(const AttnArgs& a, hipStream_t st) {
 // Which form, from what each costs on an MI355X: time = base + rounds (r + s steps) + fill (f + g steps) in
 // microseconds, with rounds = workgroups / 256 rounded up, fill = workgroups / 256, steps = key tiles (main
 // kernel) or key steps of the longest run (short form); the split schedule: base + per balanced key tile.
-// The coefficients are least-squares fits to about 300 launches per head dim and variant (4 to 480 heads, 32 to
-// 2048 queries, 32 to 4096 keys), which they meet within 4 to 11 %; picking the form by them came within
-// 0.6 % of always picking the faster one.  Measured at [1,256,30,128] 16.7 -> 10.0 us, [1,1024,8,64]
-// 20.2 -> 9.5, [1,1024,8,128] 28.0 -> 13.9, [1,512,24,128] 21.3 -> 12.8; the main kernel's form is back ahead
-// at about 100 workgroups of 256 rows with 128 channels (twice that many with few keys).
+// The coefficients are fitted to 350 to 400 launches of the kernel and 230 one-shot calls per head dim and variant
+// (2 to 480 heads, 32 to 16384 queries, 16 to 32768 keys): choosing by them costs 0.05 to 0.9 % over always choosing
+// right.  (A fit that ended at 4096 keys, carried on to longer ones, gave whole problems of 64 channels with e4m3 P.V
+// to the short form, which moves 8 times the operand bytes: [1,16384,12,64] 970 us, now 700.)  Measured at
+// [1,256,30,128] 16.7 -> 10.0 us, [1,1024,8,64] 20.2 -> 9.5, [1,1024,8,128] 28.0 -> 13.9, [1,512,24,128] 21.3 -> 12.8;
+// whatever the key count, the main kernel's form is back ahead at 75 (128 channels, fp16) to 190 (64, e4m3) workgroups
+// of 256 rows, 110 to 140 of 128 rows at 256 channels.
 //
 // A problem of some rounds and a bit more takes both: the main kernel does the full rounds and the short
 // form what is left, spread over the whole chip, instead of one more round that is nearly empty (264 items
-// of 32 key tiles, 128 channels: 84 -> 66 us; of 64 channels 61 -> 43).  The split schedule, which balances
-// the same problems by handing partial results over in memory, is left where it is predicted ahead of both.
+// of 32 key tiles, 128 channels: 84 -> 66 us; of 64 channels 61 -> 43).
+// The split schedule, which balances the same problems by handing partial results over in memory, is left where it is
+// predicted ahead of both.
 struct FormCost {
     float base, r, s, f, g;
     float of(int64_t wgs, int64_t steps) const {
@@ -454,12 +457,14 @@ struct FormCost {
 };
 static const FormCost kCost[3][2][3] = {        // [64, 128, 256 channels][variant][main, 4 runs, 8 runs]
     {{{6.00f, 1.70f, 0.78f, 0.00f, 0.03f}, {4.97f, 1.54f, 0.50f, 0.00f, 0.17f}, {5.18f, 1.19f, 0.41f, 0.14f, 0.27f}},
-     {{3.52f, 4.41f, 0.91f, 3.03f, 0.00f}, {1.72f, 5.65f, 0.79f, 1.02f, 0.11f}, {2.30f, 5.33f, 0.31f, 0.23f, 0.41f}}},
-    {{{9.36f, 1.64f, 0.89f, 0.08f, 0.51f}, {3.45f, 5.23f, 0.71f, 0.49f, 0.69f}, {4.33f, 4.13f, 0.57f, 0.56f, 0.86f}},
-     {{6.95f, 5.91f, 1.08f, 8.20f, 0.00f}, {2.69f, 6.85f, 1.12f, 2.05f, 0.17f}, {2.52f, 6.99f, 0.66f, 1.02f, 0.52f}}},
-    {{{3.16f, 4.72f, 1.40f, 4.64f, 0.00f}, {2.15f, 5.54f, 1.26f, 1.78f, 0.27f}, {}},
-     {{3.08f, 8.00f, 1.09f, 4.97f, 0.00f}, {1.83f, 5.98f, 2.04f, 1.26f, 0.00f}, {}}},
+     {{1.91f, 3.27f, 0.76f, 1.13f, 0.06f}, {3.02f, 1.61f, 1.08f, 1.28f, 0.00f}, {2.55f, 1.40f, 1.20f, 1.06f, 0.00f}}},
+    {{{1.29f, 3.84f, 0.75f, 0.88f, 0.54f}, {2.68f, 3.27f, 0.92f, 0.05f, 0.42f}, {2.56f, 3.24f, 0.95f, 0.04f, 0.36f}},
+     {{2.15f, 4.92f, 0.95f, 1.71f, 0.11f}, {2.52f, 4.17f, 1.20f, 0.18f, 0.30f}, {2.54f, 3.25f, 1.40f, 0.75f, 0.14f}}},
+    {{{1.44f, 4.16f, 1.36f, 2.31f, 0.26f}, {2.87f, 6.05f, 1.29f, 0.20f, 0.25f}, {}},
+     {{3.61f, 4.01f, 1.64f, 2.79f, 0.00f}, {1.45f, 5.06f, 2.57f, 1.45f, 0.00f}, {}}},
 };
+// (fp16 at 64 channels past 3072 keys: no one set meets both ends there)
+static const FormCost kCost64Long[3] = {{1.81f, 2.54f, 0.66f, 0.34f, 0.16f}, {3.60f, 0.70f, 0.78f, 0.00f, 0.06f}, {3.72f, 0.77f, 0.55f, 0.03f, 0.18f}};
 static const float kSplitCost[2][2] = {{11.8f, 1.08f}, {30.1f, 1.73f}};       // [64, 128 channels]: base, per key tile
 
 namespace {
@@ -475,9 +480,9 @@ Short best_short(const FormCost* c, int64_t rows, int64_t bh, int D, int64_t ste
 
 static AttnPlan plan_by_shape(int B, int H, int Nq, int kv_valid, int D, int variant, bool causal, int split) {
     const int v = variant == 0 ? 0 : 1, d = D == 64 ? 0 : D == 128 ? 1 : 2;
-    const FormCost* c = kCost[d][v];
     const int64_t bh = (int64_t)B * H;
     const int64_t tiles = (kv_valid + kTileKV - 1) / kTileKV, steps = variant == 0 ? (kv_valid + 31) / 32 : tiles;
+    const FormCost* c = D == 64 && v == 0 && tiles > 48 ? kCost64Long : kCost[d][v];
     const int rows = D > 128 ? 128 : 256;
     const int64_t items = bh * ((Nq + rows - 1) / rows), whole = items / 256 * 256;
     AttnPlan p{items, 0, 0};

@@ -73,6 +73,18 @@ def test_split_schedule_is_a_function_of_the_shape():
         assert L.mi355_sage_set_attn_split(bad) == -1
 
 
+def test_form_of_the_attention_kernel_by_shape():
+    """The short form (the keys split over a workgroup's waves) is for problems that do not fill the chip, whatever the
+    length: timed on an MI355X, it is behind the 256-row workgroups from about 75 (128 channels, fp16) to 190 (64
+    channels, e4m3) of them on, and ahead below half of that."""
+    rule = _lib.lib().mi355_sage_attn_short_rule
+    for B, H, S, D, variant in [(1, 12, 16384, 64, 1), (1, 4, 16384, 64, 1), (2, 24, 16384, 64, 1), (1, 30, 12288, 64, 1), (1, 4, 12288, 128, 1),
+                                (1, 8, 12288, 64, 0), (1, 12, 8192, 64, 0), (1, 8, 10240, 128, 0), (1, 24, 4608, 128, 0), (1, 40, 2304, 64, 0)]:
+        assert rule(B, H, S, S, D, variant) == 0, (B, H, S, D, variant)
+    for B, H, S, D, variant in [(1, 4, 2048, 64, 1), (1, 4, 2048, 128, 0), (1, 2, 8192, 64, 1), (1, 1, 8192, 128, 1), (1, 8, 1024, 64, 0), (1, 30, 256, 128, 0)]:
+        assert rule(B, H, S, S, D, variant) in (4, 8), (B, H, S, D, variant)
+
+
 def test_argument_validation_without_device():
     """Order and codes of serenitymojo/ops/cshim/cudnn_sdpa.cpp:391-393: null
     pointers, non-positive dims, null strides -> -1 before anything touches a GPU.
