@@ -26,7 +26,8 @@ int mi355_sage_set_attn_split(int mode);
 int mi355_sage_set_attn_split_wait(int polls);
 
 /* Workgroups the split schedule would use for this shape on a device that supports it (256), or 0
- * for one workgroup per row tile: the rule alone, whatever the switch above and the device say. */
+ * where it is not considered: the rule that sizes the workspace, whatever the switch above and the
+ * device say.  Whether it is taken is decided by the predicted costs of the forms. */
 int mi355_sage_attn_split_rule(int B, int H, int N_q, int N_kv, int D, int variant);
 
 /* The short form of the attention kernel (32 or 64 query rows per workgroup, keys split over its

@@ -1014,17 +1014,18 @@ static hipError_t launch_attn_dv(const AttnArgs& a, hipStream_t st) {
     return hipGetLastError();
 }
 
-// ---- split scheduling: when, and over how many workgroups -------------------------------------
+// ---- split scheduling: for which shapes, and over how many workgroups ---------------------------
 // One workgroup per item runs in ceil(items / 256) rounds on the 256 compute units (a workgroup
-// fills one).  When the last round is at most half full and leaves 16 % or more of the launch's
-// compute-unit time idle, the steps are spread over exactly 256 workgroups instead.  Measured on
-// an MI355X (one-shot call, D = 128): 323 items -13 %, 576 items -11 %, 640 items -5 %, 320 items
-// of 32 steps -6 %; under 3 % either way at 400, 432 and 864 items (last round 56 %, 69 %, 38 %
+// fills one).  Where the last round is at most half full and leaves 16 % or more of the launch's
+// compute-unit time idle, spreading the steps over exactly 256 workgroups instead can be worth its
+// hand-overs — a second prologue and 132 KB each way.  The rule below says for which shapes it is
+// considered, and sizes the hand-over slots; attn_plan takes it where its cost is predicted below the
+// main kernel's and below main kernel + short form (sage_attn_short.hip, which has the figures).
+// Outside the rule it was under 3 % either way at 400, 432 and 864 items (last round 56 %, 69 %, 38 %
 // full) and at 1584 items (seven rounds): a partly filled round runs at a higher clock — the chip
-// is power-limited under this kernel — and every hand-over costs a second prologue and 132 KB
-// each way.  Twice as many workgroups (two per compute unit, one after the other) were slower
-// everywhere but at 1584 items.  The decision depends on the shape only, so every entry point
-// produces the same bits for the same problem.
+// is power-limited under this kernel.  Twice as many workgroups (two per compute unit, one after the
+// other) were slower everywhere but at 1584 items.  The decision depends on the shape only, so every
+// entry point produces the same bits for the same problem.
 static std::atomic<int> g_split_mode{0};       // 0: by shape and device; -1: never; n > 0: always, over n workgroups
 
 void attn_split_override(int mode) { g_split_mode.store(mode); }

@@ -438,7 +438,7 @@ hipError_t launch_attn_short(const AttnArgs& a, hipStream_t st) {
 // The coefficients are fitted to 350 to 400 launches of the kernel and 230 one-shot calls per head dim and variant
 // (2 to 480 heads, 32 to 16384 queries, 16 to 32768 keys): choosing by them costs 0.05 to 0.9 % over always choosing
 // right.  (A fit that ended at 4096 keys, carried on to longer ones, gave whole problems of 64 channels with e4m3 P.V
-// to the short form, which moves 8 times the operand bytes: [1,16384,12,64] 970 us, now 700.)  Measured at
+// to the short form, which moves 8 times the operand bytes: [1,16384,12,64] 970 us, now 708.)  Measured at
 // [1,256,30,128] 16.7 -> 10.0 us, [1,1024,8,64] 20.2 -> 9.5, [1,1024,8,128] 28.0 -> 13.9, [1,512,24,128] 21.3 -> 12.8;
 // whatever the key count, the main kernel's form is back ahead at 75 (128 channels, fp16) to 190 (64, e4m3) workgroups
 // of 256 rows, 110 to 140 of 128 rows at 256 channels.
@@ -446,8 +446,11 @@ hipError_t launch_attn_short(const AttnArgs& a, hipStream_t st) {
 // A problem of some rounds and a bit more takes both: the main kernel does the full rounds and the short
 // form what is left, spread over the whole chip, instead of one more round that is nearly empty (264 items
 // of 32 key tiles, 128 channels: 84 -> 66 us; of 64 channels 61 -> 43).
-// The split schedule, which balances the same problems by handing partial results over in memory, is left where it is
-// predicted ahead of both.
+// The split schedule, which balances the same problems by handing partial results over in memory, is ahead of both where
+// the second of few rounds is a quarter to a half full and the key sequence is long: a sixth (64 channels) and a
+// thirteenth (128) of the 788 shapes of its rule that were timed, among them one-shot [1,4352 x 8192,19,128] 344 -> 315 us
+// and [1,4352 x 8192,19,64] 225 -> 205 (323 row tiles), [1,12288,7,128] 477 -> 444; where it is taken it never cost
+// more than 0.5 %.
 struct FormCost {
     float base, r, s, f, g;
     float of(int64_t wgs, int64_t steps) const {
@@ -465,7 +468,7 @@ static const FormCost kCost[3][2][3] = {        // [64, 128, 256 channels][varia
 };
 // (fp16 at 64 channels past 3072 keys: no one set meets both ends there)
 static const FormCost kCost64Long[3] = {{1.81f, 2.54f, 0.66f, 0.34f, 0.16f}, {3.60f, 0.70f, 0.78f, 0.00f, 0.06f}, {3.72f, 0.77f, 0.55f, 0.03f, 0.18f}};
-static const float kSplitCost[2][2] = {{11.8f, 1.08f}, {30.1f, 1.73f}};       // [64, 128 channels]: base, per key tile
+static const float kSplitCost[2][2] = {{17.0f, 0.96f}, {25.0f, 1.53f}};       // [64, 128 channels]: base, per key tile
 
 namespace {
 struct Short { float t; int kw; };

@@ -43,7 +43,7 @@ def test_no_gpu_helpers():
 
 def test_split_schedule_is_a_function_of_the_shape():
     """Hand-over slots (256 workgroups x (D/32*16 + 2) x 512 floats + 4 KiB of flags) are part of the
-    workspace exactly for the shapes that split: fp16 variant, more than 256 row tiles, last round of
+    workspace exactly for the shapes the split schedule is considered for: fp16 variant, more than 256 row tiles, last round of
     256 at most half full, 16 % or more of the launch idle, spans of 16 steps or more.  The size is a
     function of the shape alone: the test switch that forces a schedule does not move it."""
     L = _lib.lib()

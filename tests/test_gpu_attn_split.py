@@ -97,23 +97,29 @@ def test_forced_split_stats_masks_and_rectangular(oracle, split, variant):
     np.testing.assert_allclose(got[1][..., 0], want_stats, atol=2e-3 if variant == 0 else 1e-2)
 
 
+# 336 row tiles of 192 key tiles on 256 compute units: a second round less than a third full, and long
+SPLITS = dict(B=1, H=7, S=12288)
+
+
 def test_shape_that_splits_by_itself(split):
-    """264 row tiles on 256 compute units would run in two rounds, the second almost empty: the
-    library splits such a shape without being told.  The one-shot call and the stage pipeline take
-    the same decision (same bits); the result agrees with the plain schedule and the fp32 referee."""
+    """The library splits such a shape without being told: the bits are those of the schedule forced over 256 workgroups.
+    The one-shot call and the stage pipeline take the same decision (same bits); the result agrees with the plain
+    schedule and the fp32 referee."""
     import torch
     import gpu_harness as H
     from test_gpu_attn import _one_shot
     L = _lib.lib()
-    w = WORKLOADS[1].scaled(B=1, H=33, S=2048)
+    w = WORKLOADS[2].scaled(**SPLITS)
     assert L.mi355_sage_workspace_bytes(w.B, w.H, w.S, w.S, w.D, 0) > \
-        L.mi355_sage_workspace_bytes(w.B, 32, w.S, w.S, w.D, 0) * 33 // 32 + (1 << 20)   # hand-over slots included
+        L.mi355_sage_workspace_bytes(w.B, 5, w.S, w.S, w.D, 0) * 7 // 5 + (1 << 20)   # hand-over slots included
     q, k, v = make_inputs(w)
     got = _one_shot(q, k, v, w.scale, 0)
     g = H.quant_qk(q, k, w.scale, 128, 64, True)["dev"]
     gv = H.quant_v(v, 0)["dev"]
     staged, _ = H.attn_fwd(g["q8"], g["qscale"], 128, g["k8"], g["kscale"], 64, gv["vq"], None, 0, w.S, w.S)
     np.testing.assert_array_equal(got, staged)
+    split(256)
+    np.testing.assert_array_equal(_one_shot(q, k, v, w.scale, 0), got)
     split(-1)
     plain = _one_shot(q, k, v, w.scale, 0)
     assert not np.array_equal(got, plain)                  # it really was another schedule
@@ -130,7 +136,7 @@ def test_split_call_in_a_hip_graph(split):
     import gpu_harness as H
     L = _lib.lib()
     split(0)
-    w = WORKLOADS[1].scaled(B=1, H=33, S=2048)             # 264 row tiles: splits by itself, slots in the caller's workspace
+    w = WORKLOADS[2].scaled(**SPLITS)                      # splits by itself (the test above), slots in the caller's workspace
     assert L.mi355_sage_attn_split_rule(w.B, w.H, w.S, w.S, w.D, 0) == 256
     q0, k0, v0 = (H.dev_bf16(x) for x in make_inputs(w))
     q, k, v = q0.clone(), k0.clone(), v0.clone()
