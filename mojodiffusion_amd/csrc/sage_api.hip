@@ -359,9 +359,11 @@ int sdpa_impl(const void* Q, const void* K, const void* V, void* O, void* Stats,
     // Not where the encoders have room for it and a prologue is on the path of the whole call — the main kernel does
     // everything in one round that leaves compute units without a workgroup (us with Q in the kernel -> in the
     // encoders: [1,700,24,128] 36.7 -> 34.3, [1,1153,24,128] 46.6 -> 43.8; but [1,2304,24,128], two rounds, 72.9 ->
-    // 75.4) — nor with e4m3 P.V, whose scale blocks are single waves' and whose prologue costs more
-    // ([1,256,30,128] 18.9 -> 16.8, [1,1153,24,128] 49.8 -> 46.6, [1,4608,24,128] 220.7 -> 216.3; level at 16896, at 64
-    // channels level at 4608 and 383 -> 388 at 8192).  Many queries on few keys keep it ([1,3840 x 333,32,128] fp16
+    // 75.4) — nor, with e4m3 P.V, whose scale blocks are single waves' and whose prologue costs more, where the short form
+    // does all or part of it ([1,256,30,128] 18.9 -> 16.8, [1,1153,24,128] 49.8 -> 46.6, [1,3072,30,128] 153.2 -> 151.1) or the
+    // main kernel has up to 160 workgroups ([2,320,32,128], 128 of them, 33.2 -> 31.4; but 240, [1,1497,40,128], 62.9 -> 66.7,
+    // 256, [2,1995,16,128], 73.9 -> 78.0, 960, [2,2822,40,128], 308.6 -> 315.9), up to 8192 tokens of 128 channels, 4096 of 64
+    // (level at 16896).  Many queries on few keys keep it ([1,3840 x 333,32,128] fp16
     // 50.1 -> 52.0, e4m3 57.5 -> 64.0), and so does a K that takes one launch alone and three, or more than a
     // workgroup per compute unit, with Q ([1,2048 x 512,32,64] 23.7 -> 30.4, e4m3 [1,512,24,128] 21.5 -> 25.6).
     auto one_launch = [&](bool with_q) {
@@ -371,8 +373,9 @@ int sdpa_impl(const void* Q, const void* K, const void* V, void* O, void* Stats,
         t.q8 = with_q ? reinterpret_cast<int8_t*>(ws) : nullptr;
         return quant_short_workgroups(t, B, D);
     };
-    const bool one_round = plan.main_items > 0 && plan.short_kw == 0 && plan.main_items < 256;
-    bool q_in_encoders = (one_round || (variant == MI355_SAGE_PV_FP8 && (int64_t)N_q * 64 <= (int64_t)4096 * D)) && N_q <= 2 * N_kv;
+    const bool room = variant == MI355_SAGE_PV_FP8 ? (plan.short_kw > 0 || plan.main_items <= 160) && (int64_t)N_q * 64 <= (int64_t)4096 * D
+                                                   : plan.main_items > 0 && plan.short_kw == 0 && plan.main_items < 256;
+    bool q_in_encoders = room && N_q <= 2 * N_kv;
     if (q_in_encoders && one_launch(false) > 0) {
         const int64_t wgs = one_launch(true);
         q_in_encoders = wgs > 0 && wgs <= 256;
