@@ -44,6 +44,9 @@ int mi355_sage_attn_short_rule(int B, int H, int N_q, int N_kv, int D, int varia
  * device and under the current switches; the short form does the others. */
 int64_t mi355_sage_attn_main_items(int B, int H, int N_q, int N_kv, int D, int variant);
 
+/* The same by the shape alone, on a device of that many compute units and without the split schedule. */
+int64_t mi355_sage_attn_main_items_on(int units, int B, int H, int N_q, int N_kv, int D, int variant);
+
 #ifdef __cplusplus
 }
 #endif

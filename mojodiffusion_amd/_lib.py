@@ -65,6 +65,7 @@ SIGNATURES = {
     "mi355_sage_set_attn_short": (_int, [_int]),
     "mi355_sage_attn_short_rule": (_int, [_int] * 6),
     "mi355_sage_attn_main_items": (_i64, [_int] * 6),
+    "mi355_sage_attn_main_items_on": (_i64, [_int] * 7),
     "mi355_sage_set_attn_split_wait": (_int, [_int]),
     "mi355_sage_version": (ctypes.c_char_p, []),
 }

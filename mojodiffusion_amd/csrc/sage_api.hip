@@ -361,7 +361,7 @@ int sdpa_impl(const void* Q, const void* K, const void* V, void* O, void* Stats,
     // encoders: [1,700,24,128] 36.7 -> 34.3, [1,1153,24,128] 46.6 -> 43.8; but [1,2304,24,128], two rounds, 72.9 ->
     // 75.4) — nor, with e4m3 P.V, whose scale blocks are single waves' and whose prologue costs more, where the short form
     // does all or part of it ([1,256,30,128] 18.9 -> 16.8, [1,1153,24,128] 49.8 -> 46.6, [1,3072,30,128] 153.2 -> 151.1) or the
-    // main kernel has up to 160 workgroups ([2,320,32,128], 128 of them, 33.2 -> 31.4; but 240, [1,1497,40,128], 62.9 -> 66.7,
+    // main kernel fills at most five eighths of the chip ([2,320,32,128], 128 of them, 33.2 -> 31.4; but 240, [1,1497,40,128], 62.9 -> 66.7,
     // 256, [2,1995,16,128], 73.9 -> 78.0, 960, [2,2822,40,128], 308.6 -> 315.9), up to 8192 tokens of 128 channels, 4096 of 64
     // (level at 16896).  Many queries on few keys keep it ([1,3840 x 333,32,128] fp16
     // 50.1 -> 52.0, e4m3 57.5 -> 64.0), and so does a K that takes one launch alone and three, or more than a
@@ -373,12 +373,13 @@ int sdpa_impl(const void* Q, const void* K, const void* V, void* O, void* Stats,
         t.q8 = with_q ? reinterpret_cast<int8_t*>(ws) : nullptr;
         return quant_short_workgroups(t, B, D);
     };
-    const bool room = variant == MI355_SAGE_PV_FP8 ? (plan.short_kw > 0 || plan.main_items <= 160) && (int64_t)N_q * 64 <= (int64_t)4096 * D
-                                                   : plan.main_items > 0 && plan.short_kw == 0 && plan.main_items < 256;
+    const int units = compute_units();
+    const bool room = variant == MI355_SAGE_PV_FP8 ? (plan.short_kw > 0 || plan.main_items * 8 <= units * 5) && (int64_t)N_q * 64 <= (int64_t)4096 * D
+                                                   : plan.main_items > 0 && plan.short_kw == 0 && plan.main_items < units;
     bool q_in_encoders = room && N_q <= 2 * N_kv;
     if (q_in_encoders && one_launch(false) > 0) {
         const int64_t wgs = one_launch(true);
-        q_in_encoders = wgs > 0 && wgs <= 256;
+        q_in_encoders = wgs > 0 && wgs <= units;
     }
     const bool q_in_kernel = Stats == nullptr && mask.add == nullptr && pre.q.gain == nullptr && (D <= 128 || plan.main_items == 0) &&
                              plan.split_wgs == 0 && !q_in_encoders;
@@ -853,6 +854,11 @@ int mi355_sage_attn_short_rule(int B, int H, int N_q, int N_kv, int D, int varia
 int64_t mi355_sage_attn_main_items(int B, int H, int N_q, int N_kv, int D, int variant) {
     if (B <= 0 || H <= 0 || N_q <= 0 || N_kv <= 0) return 0;
     return attn_plan(B, H, N_q, N_kv, D, variant, false).main_items;
+}
+
+int64_t mi355_sage_attn_main_items_on(int units, int B, int H, int N_q, int N_kv, int D, int variant) {
+    if (units <= 0 || B <= 0 || H <= 0 || N_q <= 0 || N_kv <= 0 || !dims_ok(D)) return 0;
+    return attn_main_items_on(units, B, H, N_q, N_kv, D, variant);
 }
 
 int mi355_sage_set_attn_split_wait(int polls) {

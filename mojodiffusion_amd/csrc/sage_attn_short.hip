@@ -433,7 +433,7 @@ hipError_t launch_attn_short(const AttnArgs& a, hipStream_t st) {
 }
 
 // Which form, from what each costs on an MI355X: time = base + rounds (r + s steps) + fill (f + g steps) in
-// microseconds, with rounds = workgroups / 256 rounded up, fill = workgroups / 256, steps = key tiles (main
+// microseconds, with rounds = workgroups / compute units rounded up, fill = workgroups / compute units, steps = key tiles (main
 // kernel) or key steps of the longest run (short form); the split schedule: base + per balanced key tile.
 // The coefficients are fitted to 350 to 400 launches of the kernel and 230 one-shot calls per head dim and variant
 // (2 to 480 heads, 32 to 16384 queries, 16 to 32768 keys): choosing by them costs 0.05 to 0.9 % over always choosing
@@ -453,8 +453,8 @@ hipError_t launch_attn_short(const AttnArgs& a, hipStream_t st) {
 // more than 0.5 %.
 struct FormCost {
     float base, r, s, f, g;
-    float of(int64_t wgs, int64_t steps) const {
-        const float rounds = (float)((wgs + 255) / 256), fill = (float)wgs / 256.0f, n = (float)steps;
+    float of(int64_t wgs, int64_t steps, int units) const {
+        const float rounds = (float)((wgs + units - 1) / units), fill = (float)wgs / (float)units, n = (float)steps;
         return base + rounds * (r + s * n) + fill * (f + g * n);
     }
 };
@@ -472,29 +472,29 @@ static const float kSplitCost[2][2] = {{17.0f, 0.96f}, {25.0f, 1.53f}};       //
 
 namespace {
 struct Short { float t; int kw; };
-Short best_short(const FormCost* c, int64_t rows, int64_t bh, int D, int64_t steps) {
+Short best_short(const FormCost* c, int64_t rows, int64_t bh, int D, int64_t steps, int units) {
     const int rows4 = D > 128 ? 32 : 64;
-    const Short four{c[1].of(bh * ((rows + rows4 - 1) / rows4), (steps + 3) / 4), 4};
+    const Short four{c[1].of(bh * ((rows + rows4 - 1) / rows4), (steps + 3) / 4, units), 4};
     if (D > 128) return four;
-    const Short eight{c[2].of(bh * ((rows + 31) / 32), (steps + 7) / 8), 8};
+    const Short eight{c[2].of(bh * ((rows + 31) / 32), (steps + 7) / 8, units), 8};
     return four.t < eight.t ? four : eight;
 }
 }  // namespace
 
-static AttnPlan plan_by_shape(int B, int H, int Nq, int kv_valid, int D, int variant, bool causal, int split) {
+static AttnPlan plan_by_shape(int units, int B, int H, int Nq, int kv_valid, int D, int variant, bool causal, int split) {
     const int v = variant == 0 ? 0 : 1, d = D == 64 ? 0 : D == 128 ? 1 : 2;
     const int64_t bh = (int64_t)B * H;
     const int64_t tiles = (kv_valid + kTileKV - 1) / kTileKV, steps = variant == 0 ? (kv_valid + 31) / 32 : tiles;
     const FormCost* c = D == 64 && v == 0 && tiles > 48 ? kCost64Long : kCost[d][v];
     const int rows = D > 128 ? 128 : 256;
-    const int64_t items = bh * ((Nq + rows - 1) / rows), whole = items / 256 * 256;
+    const int64_t items = bh * ((Nq + rows - 1) / rows), whole = items / units * units;
     AttnPlan p{items, 0, 0};
-    float best = c[0].of(items, tiles);
-    const Short all = best_short(c, Nq, bh, D, steps);
+    float best = c[0].of(items, tiles, units);
+    const Short all = best_short(c, Nq, bh, D, steps, units);
     if (all.t < best) { best = all.t; p = AttnPlan{0, all.kw, 0}; }
     if (!causal && whole > 0 && whole < items) {
-        const Short rest = best_short(c, rows, items - whole, D, steps);
-        const float t = c[0].of(whole, tiles) + rest.t;
+        const Short rest = best_short(c, rows, items - whole, D, steps, units);
+        const float t = c[0].of(whole, tiles, units) + rest.t;
         if (t < best) { best = t; p = AttnPlan{whole, rest.kw, 0}; }
     }
     if (!causal && split > 0 && D <= 128 && kSplitCost[d][0] + kSplitCost[d][1] * (float)(items * tiles) / 256.0f < best) p = AttnPlan{items, 0, split};
@@ -505,8 +505,25 @@ static std::atomic<int> g_short_mode{0};       // 0: by shape; -1: never; 4, 8: 
 void attn_short_override(int mode) { g_short_mode.store(mode); }
 
 int attn_short_rule(int B, int H, int Nq, int kv_valid, int D, int variant) {
-    const AttnPlan p = plan_by_shape(B, H, Nq, kv_valid, D, variant, false, 0);
+    const AttnPlan p = plan_by_shape(256, B, H, Nq, kv_valid, D, variant, false, 0);
     return p.main_items == 0 ? p.short_kw : 0;
+}
+
+int64_t attn_main_items_on(int units, int B, int H, int Nq, int kv_valid, int D, int variant) {
+    return plan_by_shape(units, B, H, Nq, kv_valid, D, variant, false, 0).main_items;
+}
+
+// Asked of the device once.  (256 where there is none to ask.)
+int compute_units() {
+    static std::atomic<int> known[64];
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+    int n = known[dev].load();
+    if (n == 0) {
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+        known[dev].store(n);
+    }
+    return n;
 }
 
 AttnPlan attn_plan(int B, int H, int Nq, int kv_valid, int D, int variant, bool causal) {
@@ -515,7 +532,7 @@ AttnPlan attn_plan(int B, int H, int Nq, int kv_valid, int D, int variant, bool 
     const int split = causal ? 0 : attn_split_workgroups(B, H, Nq, kv_valid, D, variant);
     if (mode < 0 || attn_split_override_mode() != 0)      // (a schedule of the main kernel was asked for)
         return AttnPlan{(int64_t)B * H * ((Nq + rows - 1) / rows), 0, split};
-    return plan_by_shape(B, H, Nq, kv_valid, D, variant, causal, split);
+    return plan_by_shape(compute_units(), B, H, Nq, kv_valid, D, variant, causal, split);
 }
 
 }  // namespace sage

@@ -155,6 +155,8 @@ struct AttnPlan {
     int split_wgs;           // > 0: the main kernel's items in the split schedule (then all of them)
 };
 AttnPlan attn_plan(int B, int H, int Nq, int kv_valid, int D, int variant, bool causal);
+int compute_units();        // of the current device
+int64_t attn_main_items_on(int units, int B, int H, int Nq, int kv_valid, int D, int variant);       // the plan by shape on that many compute units
 hipError_t launch_attn_short(const AttnArgs& a, hipStream_t st);
 int attn_short_rule(int B, int H, int Nq, int kv_valid, int D, int variant);     // short_kw where the short form does everything by shape, else 0
 void attn_short_override(int mode);          // 0: by shape (default); -1: never; 4 or 8: always

@@ -85,6 +85,17 @@ def test_form_of_the_attention_kernel_by_shape():
         assert rule(B, H, S, S, D, variant) in (4, 8), (B, H, S, D, variant)
 
 
+def test_forms_scale_with_the_compute_units():
+    """A partition of the chip with an eighth of its compute units fills up with an eighth of the workgroups, and its last
+    round is another one: eight times the heads on the whole chip take the same form as the heads on the partition."""
+    items = _lib.lib().mi355_sage_attn_main_items_on
+    for S, D, variant in [(256, 128, 0), (1024, 64, 0), (1153, 128, 1), (2048, 128, 0), (4608, 128, 0), (1024, 256, 0)]:
+        for heads in (1, 2, 3, 4, 5, 8):
+            assert items(256, 1, 8 * heads, S, S, D, variant) == 8 * items(32, 1, heads, S, S, D, variant), (S, D, variant, heads)
+    assert items(256, 1, 4, 2048, 2048, 128, 0) == 0            # 32 row tiles: the short form on 256 compute units,
+    assert items(32, 1, 4, 2048, 2048, 128, 0) == 32            # one full round on 32
+
+
 def test_argument_validation_without_device():
     """Order and codes of serenitymojo/ops/cshim/cudnn_sdpa.cpp:391-393: null
     pointers, non-positive dims, null strides -> -1 before anything touches a GPU.
