@@ -528,12 +528,14 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
                                       (causal && key0 + SK - 1 > wave_row0), 0)) {
             asm volatile("" ::: "memory");
 #pragma unroll
-            for (int kb = 0; kb < SKB; kb++)
+            for (int kb = 0; kb < SKB; kb++) {
+                f[kb] = masked_scale(f[kb]);
 #pragma unroll
                 for (int i = 0; i < 16; i++) {
                     const int key = key0 + kb * 32 + (i >> 2) * 8 + half * 4 + (i & 3);
                     if (key >= kv_valid || (MASKED && key >= mask_lo && key < mask_hi) || (causal && key > qrow)) s[X][kb][i] = (int)0xFF800000;
                 }
+            }
         }
         // biased scores in the log2 domain, without the reference maximum (ADDMASK only)
         float xs[SKB][ADDMASK ? 16 : 1];

@@ -75,6 +75,11 @@ template <int D> struct Magic {
     static constexpr float F = D > 128 ? kMagicWideF : kMagicF;
 };
 
+// The score scale of a step that holds masked scores: at least the smallest normal number, because -inf times a scale
+// that has underflowed to zero is NaN.  (A real score times a scale below it is 0 in the exponent either way; a NaN
+// scale stays one.)
+static __device__ __forceinline__ float masked_scale(float f) { return f < 0x1p-126f ? 0x1p-126f : f; }
+
 // First matrix instruction of a score chain: accumulator input = the constant above, held in 16
 // registers for the whole kernel (behind an empty statement, or the compiler re-creates the 16
 // copies for every chain).  The instruction could take 1/(2*pi) as an inline operand, but only

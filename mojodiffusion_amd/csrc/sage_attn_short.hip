@@ -246,12 +246,14 @@ __global__ __launch_bounds__(short_waves<D>() * 64) void sage_attn_short_kernel(
         for (int kb = 0; kb < SKB; kb++) f[kb] = sq * ksc[(key0 + kb * 32) >> ksh];
         if (key0 + SK > kv_valid || (key0 < a.km.hi && key0 + SK > a.km.lo) || (a.causal && key0 + SK - 1 > row0)) {
 #pragma unroll
-            for (int kb = 0; kb < SKB; kb++)
+            for (int kb = 0; kb < SKB; kb++) {
+                f[kb] = masked_scale(f[kb]);
 #pragma unroll
                 for (int i = 0; i < 16; i++) {
                     const int key = key0 + kb * 32 + (i >> 2) * 8 + half * 4 + (i & 3);
                     if (key >= kv_valid || (key >= a.km.lo && key < a.km.hi) || (a.causal && key > qrow)) s[kb][i] = (int)0xFF800000;
                 }
+            }
         }
         // scores in the log2 domain (the accumulators' bias taken off exactly), or the raw accumulators where
         // one multiply-add does the rest

@@ -72,3 +72,27 @@ def test_nothing_past_the_last_key_matters(oracle, variant, D, kv_valid):
     np.testing.assert_array_equal(gs, ws)
     _, ref = oracle.sdpa_bf16(q, k, v, scale, variant=variant, blkq=blkq, blkk=64)
     assert np.isfinite(bf16_bits_to_f32(got)).all() and np.abs(bf16_bits_to_f32(got) - ref).max() <= 2e-2
+
+
+@pytest.mark.parametrize("form", ["main", "short"])
+@pytest.mark.parametrize("variant,D", [(0, 64), (0, 128), (1, 64), (1, 128), (1, 256)])
+@pytest.mark.parametrize("Skv", [192, 256, 300])
+def test_score_scales_that_underflow_to_zero(form, variant, D, Skv):
+    """Inputs so small that the score scale is zero in F32: every key counts alike, and a masked score (-inf) times that
+    scale must not become NaN.  The result is the mean of V over the keys; V is within 1, so 2e-2 bounds its
+    storage (e4m3: 2^-4 relative, averaged) and the rounding of O."""
+    import torch
+    from mojodiffusion_amd import _lib, model_dispatch as M
+    g = torch.Generator().manual_seed(Skv + D)
+    q, k = (1e-25 * torch.randn((1, n, 2, D), generator=g) for n in (300, Skv))
+    v = torch.rand((1, Skv, 2, D), generator=g).bfloat16()
+    L = _lib.lib()
+    assert L.mi355_sage_set_attn_split(-1 if form == "main" else 0) == 0
+    assert L.mi355_sage_set_attn_short(0 if form == "main" else 4) == 0
+    try:
+        o = M.ltx2_sdpa_product_fwd_rect(q.bfloat16().cuda(), k.bfloat16().cuda(), v.cuda(), D ** -0.5, variant)
+    finally:
+        L.mi355_sage_set_attn_split(0)
+        L.mi355_sage_set_attn_short(0)
+    want = v.double().mean(dim=1, keepdim=True)
+    assert float((o.cpu().double() - want).abs().max()) <= 2e-2
