@@ -241,19 +241,17 @@ __global__ __launch_bounds__(short_waves<D>() * 64) void sage_attn_short_kernel(
         reads_done();
         if (more) copy_k(hs + 1);
         const int key0 = key_step(hs) * SK;
-        float f[SKB];
+        float f[SKB];           // (taken at least so large in every step: in the branch below it was 1 % slower at 256 channels)
 #pragma unroll
-        for (int kb = 0; kb < SKB; kb++) f[kb] = sq * ksc[(key0 + kb * 32) >> ksh];
+        for (int kb = 0; kb < SKB; kb++) f[kb] = masked_scale(sq * ksc[(key0 + kb * 32) >> ksh]);
         if (key0 + SK > kv_valid || (key0 < a.km.hi && key0 + SK > a.km.lo) || (a.causal && key0 + SK - 1 > row0)) {
 #pragma unroll
-            for (int kb = 0; kb < SKB; kb++) {
-                f[kb] = masked_scale(f[kb]);
+            for (int kb = 0; kb < SKB; kb++)
 #pragma unroll
                 for (int i = 0; i < 16; i++) {
                     const int key = key0 + kb * 32 + (i >> 2) * 8 + half * 4 + (i & 3);
                     if (key >= kv_valid || (key >= a.km.lo && key < a.km.hi) || (a.causal && key > qrow)) s[kb][i] = (int)0xFF800000;
                 }
-            }
         }
         // scores in the log2 domain (the accumulators' bias taken off exactly), or the raw accumulators where
         // one multiply-add does the rest
