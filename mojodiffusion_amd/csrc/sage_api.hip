@@ -366,13 +366,7 @@ int sdpa_impl(const void* Q, const void* K, const void* V, void* O, void* Stats,
     // (level at 16896).  Many queries on few keys keep it ([1,3840 x 333,32,128] fp16
     // 50.1 -> 52.0, e4m3 57.5 -> 64.0), and so does a K that takes one launch alone and three, or more than a
     // workgroup per compute unit, with Q ([1,2048 x 512,32,64] 23.7 -> 30.4, e4m3 [1,512,24,128] 21.5 -> 25.6).
-    auto one_launch = [&](bool with_q) {
-        QuantArgs t{};
-        t.H = H; t.Nkv = kv; t.blkq = blkq; t.blkk = blkk;
-        t.nq_pad = pad_to(N_q, kTileQ); t.nkv_pad = pad_to(kv, kPadKV);
-        t.q8 = with_q ? reinterpret_cast<int8_t*>(ws) : nullptr;
-        return quant_short_workgroups(t, B, D);
-    };
+    auto one_launch = [&](bool with_q) { return quant_short_workgroups(B, H, N_q, kv, D, blkq, blkk, with_q); };
     const int units = compute_units();
     const bool room = variant == MI355_SAGE_PV_FP8 ? (plan.short_kw > 0 || plan.main_items * 8 <= units * 5) && (int64_t)N_q * 64 <= (int64_t)4096 * D
                                                    : plan.main_items > 0 && plan.short_kw == 0 && plan.main_items < units;

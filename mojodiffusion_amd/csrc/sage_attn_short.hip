@@ -19,6 +19,7 @@
 // workgroups start to fill the chip.
 #include "sage_attn_common.h"
 
+#include <algorithm>
 #include <atomic>
 
 namespace sage {
@@ -470,6 +471,13 @@ static const FormCost kCost[3][2][3] = {        // [64, 128, 256 channels][varia
 static const FormCost kCost64Long[3] = {{1.81f, 2.54f, 0.66f, 0.34f, 0.16f}, {3.60f, 0.70f, 0.78f, 0.00f, 0.06f}, {3.72f, 0.77f, 0.55f, 0.03f, 0.18f}};
 static const float kSplitCost[2][2] = {{17.0f, 0.96f}, {25.0f, 1.53f}};       // [64, 128 channels]: base, per key tile
 
+// Microseconds a call takes more with the main kernel where its Q cannot go to the encoders for next to nothing:
+// many queries on few keys, which keep Q in the kernel's prologue, and a K that takes one launch alone but not with Q.
+// One-shot, main kernel against short form: [1,510 x 139,24,128] 22.2 against 20.4, [1,256 x 292,40,128] 26.2 against 23.7,
+// e4m3 [2,71 x 45,32,256] 38.2 against 31.6; with as many keys as queries the main kernel is ahead, [1,64,24,128] 16.1
+// against 17.6.  (64 channels: nothing to gain, or the second kind's fit is as good without.)
+static const float kQCost[3][2][2] = {{{0.0f, 0.0f}, {0.8f, 0.0f}}, {{1.4f, 1.4f}, {0.0f, 0.0f}}, {{0.0f, 2.0f}, {0.0f, 2.0f}}};
+
 namespace {
 struct Short { float t; int kw; };
 Short best_short(const FormCost* c, int64_t rows, int64_t bh, int D, int64_t steps, int units) {
@@ -489,12 +497,16 @@ static AttnPlan plan_by_shape(int units, int B, int H, int Nq, int kv_valid, int
     const int rows = D > 128 ? 128 : 256;
     const int64_t items = bh * ((Nq + rows - 1) / rows), whole = items / units * units;
     AttnPlan p{items, 0, 0};
-    float best = c[0].of(items, tiles, units);
+    const int blkq = variant == 0 ? 128 : 32;
+    const int64_t alone = quant_short_workgroups(B, H, Nq, kv_valid, D, blkq, 64, false);
+    const int64_t with_q = alone > 0 ? quant_short_workgroups(B, H, Nq, kv_valid, D, blkq, 64, true) : 0;
+    const float q_cost = std::max(Nq > 2 * kv_valid ? kQCost[d][v][0] : 0.0f, alone > 0 && (with_q == 0 || with_q > units) ? kQCost[d][v][1] : 0.0f);
+    float best = c[0].of(items, tiles, units) + q_cost;
     const Short all = best_short(c, Nq, bh, D, steps, units);
     if (all.t < best) { best = all.t; p = AttnPlan{0, all.kw, 0}; }
     if (!causal && whole > 0 && whole < items) {
         const Short rest = best_short(c, rows, items - whole, D, steps, units);
-        const float t = c[0].of(whole, tiles, units) + rest.t;
+        const float t = c[0].of(whole, tiles, units) + q_cost + rest.t;
         if (t < best) { best = t; p = AttnPlan{whole, rest.kw, 0}; }
     }
     if (!causal && split > 0 && D <= 128 && kSplitCost[d][0] + kSplitCost[d][1] * (float)(items * tiles) / 256.0f < best) p = AttnPlan{items, 0, split};

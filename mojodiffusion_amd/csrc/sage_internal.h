@@ -107,6 +107,7 @@ hipError_t launch_quant(const QuantArgs& a, const FinalArgs* f, int B, int D, hi
 
 // All of it as one launch, for short key sequences (K, V and, with q8, Q; the statistics also go to f's outputs).
 int64_t quant_short_workgroups(const QuantArgs& a, int B, int D);     // 0: not this form
+int64_t quant_short_workgroups(int B, int H, int Nq, int Nkv, int D, int blkq, int blkk, bool with_q);      // the same by the shape
 hipError_t launch_quant_short(const QuantArgs& a, const FinalArgs& f, int B, int D, hipStream_t st);
 
 // ---- attention kernel (sage_attn.hip) --------------------------------------

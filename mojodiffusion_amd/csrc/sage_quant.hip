@@ -1168,8 +1168,8 @@ __global__ __launch_bounds__(kShortThreads) void quant_short_kernel(QuantArgs a,
     quant_v_fp8_body<D, 256>(t, h, b, utid, a.v.p, a.v.sb, a.v.sh, a.v.sn, a.Nkv, a.H, a.nkv_pad, a.km, s_mean, a.v8, sm.tile8[unit]);
 }
 
-static void short_units(QuantArgs& a, int B) {
-    a.nq_blk = a.q8 != nullptr ? (int)(a.nq_pad / a.blkq) : 0;
+static void short_units(QuantArgs& a, int B, bool with_q) {
+    a.nq_blk = with_q ? (int)(a.nq_pad / a.blkq) : 0;
     a.nk_blk = (int)(a.nkv_pad / a.blkk);
     a.nv_tile = (int)(a.nkv_pad / 64);
     a.n_bh = B * a.H;
@@ -1181,17 +1181,27 @@ static int64_t short_workgroups(const QuantArgs& a) { return (int64_t)a.n_bh * (
 // per compute unit).  Measured over 4 to 60 heads, stage of three launches -> one, us: 11.5-15 -> 7.5-9.5 up
 // to 256 keys, 13-15 -> 9-12.8 at 512 keys of 128 channels, 12-13.4 -> 8.4-10.7 at 1024 keys of 64; a second
 // pass costs 4 us and a second generation of workgroups 7, which is what the two launches less are worth.
-int64_t quant_short_workgroups(const QuantArgs& a_in, int B, int D) {
-    QuantArgs a = a_in;
-    short_units(a, B);
+static int64_t short_rule(const QuantArgs& a, int D) {
     const int groups = (a.Nkv + kGroup - 1) / kGroup;
     const int64_t wgs = short_workgroups(a);
     return groups <= (D == 64 ? 4 : D == 128 ? 2 : 1) && wgs <= 512 ? wgs : 0;
 }
+int64_t quant_short_workgroups(const QuantArgs& a_in, int B, int D) {
+    QuantArgs a = a_in;
+    short_units(a, B, a.q8 != nullptr);
+    return short_rule(a, D);
+}
+int64_t quant_short_workgroups(int B, int H, int Nq, int Nkv, int D, int blkq, int blkk, bool with_q) {
+    QuantArgs a{};
+    a.H = H; a.Nkv = Nkv; a.blkq = blkq; a.blkk = blkk;
+    a.nq_pad = pad_to(Nq, kTileQ); a.nkv_pad = pad_to(Nkv, kPadKV);
+    short_units(a, B, with_q);
+    return short_rule(a, D);
+}
 
 hipError_t launch_quant_short(const QuantArgs& a_in, const FinalArgs& f_in, int B, int D, hipStream_t st) {
     QuantArgs a = a_in;
-    short_units(a, B);
+    short_units(a, B, a.q8 != nullptr);
     if ((a.q8 != nullptr && a.nq_pad % a.blkq != 0) || a.nkv_pad % a.blkk != 0 || a.k8 == nullptr || (a.v8 == nullptr && a.v16 == nullptr))
         return hipErrorInvalidValue;
     const int64_t total = short_workgroups(a);

@@ -83,6 +83,9 @@ def test_form_of_the_attention_kernel_by_shape():
         assert rule(B, H, S, S, D, variant) == 0, (B, H, S, D, variant)
     for B, H, S, D, variant in [(1, 4, 2048, 64, 1), (1, 4, 2048, 128, 0), (1, 2, 8192, 64, 1), (1, 1, 8192, 128, 1), (1, 8, 1024, 64, 0), (1, 30, 256, 128, 0)]:
         assert rule(B, H, S, S, D, variant) in (4, 8), (B, H, S, D, variant)
+    # where Q stays in the main kernel's prologue: many queries on few keys, or K and V take one launch but not with Q
+    assert rule(1, 24, 510, 139, 128, 0) == rule(1, 40, 256, 292, 128, 0) == rule(2, 32, 71, 45, 256, 1) == rule(2, 30, 128, 26, 256, 1) == 4
+    assert rule(1, 24, 64, 64, 128, 0) == rule(1, 24, 64, 49, 128, 0) == 0
 
 
 def test_forms_scale_with_the_compute_units():
