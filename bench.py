@@ -139,6 +139,7 @@ def clock_probe(args, L, w, qd, kd, vd, o, st, stream):
     P = ctypes.CDLL(args.probe_lib or os.path.join(os.path.dirname(_lib.LIB_PATH), "libmi355_sage_probe.so"))
     for name in ("mi355_sage_quant_qk_bf16", "mi355_sage_quant_v_f16", "mi355_sage_quant_v_fp8", "mi355_sage_attn_fwd"):
         getattr(P, name).restype, getattr(P, name).argtypes = _lib.SIGNATURES[name]
+    assert P.mi355_sage_set_attn_split(-1) == 0     # the main kernel, which stamps, for the whole problem (the short form does not)
     B, S, H, D = w.B, w.S, w.H, w.D
     dev = qd.device
     nqp, nkp = L.mi355_sage_pad_q(S), L.mi355_sage_pad_kv(S)

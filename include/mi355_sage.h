@@ -369,17 +369,17 @@ int mi355_sage_attn_fwd_q16(
 /* Scheduling of the attention kernel (no counterpart in the reference).
  * One workgroup computes 256 query rows of one head against all keys.  A problem too small to fill the
  * chip that way takes 32 or 64 rows per workgroup and splits the keys over the workgroup's waves, which
- * merge their partial results on the spot.  A shape whose row tiles
- * leave the last round of the 256 compute units at most half full (more than 256 tiles, 16 % or
- * more of the launch idle; fp16 variant, head dim up to 128) is instead cut into equal shares of
- * (row tile, key tile) steps for exactly 256 workgroups, which hand unnormalised partial results to
- * each other inside the launch.  The choice depends on the shape only, so all entry points give the
- * same bits for the same problem; outputs of the two schedules differ by rounding (the probabilities
- * of a row are rounded against a different running maximum).  The hand-over relies on workgroup ids
- * being dealt round-robin to 8 XCDs of 32 compute units, so the schedule is used only on a device
- * that reports exactly that (hipDeviceAttributeNumberOfXccs == 8, 256 compute units); on any other
- * partitioning every shape takes one workgroup per row tile.  Its hand-over slots are part of
- * mi355_sage_workspace_bytes for the shapes that qualify (whatever the device); mi355_sage_attn_fwd,
+ * merge their partial results on the spot; a problem of some full rounds of workgroups and a bit more takes
+ * both, the second form for what is left.  Where the last of few rounds is at most half full (more than 256
+ * row tiles, 16 % or more of the launch idle; fp16 variant, head dim up to 128) the row tiles can instead be
+ * cut into equal shares of (row tile, key tile) steps for exactly 256 workgroups, which hand unnormalised
+ * partial results to each other inside the launch; that is taken for the few of these shapes, of many keys, where
+ * it is predicted ahead of the other two.  The choice follows from the shape and the device's compute units, so
+ * all entry points give the same bits for the same problem; outputs of the forms differ by rounding (the
+ * probabilities of a row are rounded against a different running maximum).  The hand-over relies on workgroup
+ * ids being dealt round-robin to 8 XCDs of 32 compute units, so the schedule is used only on a device
+ * that reports exactly that (hipDeviceAttributeNumberOfXccs == 8, 256 compute units).  Its hand-over
+ * slots are part of mi355_sage_workspace_bytes for every shape that qualifies (whatever is chosen); mi355_sage_attn_fwd,
  * which takes no workspace, keeps its slots in a library-owned per-stream buffer (allocated on the
  * first such call of a stream, never while that stream is being captured).
  *

@@ -29,9 +29,9 @@
 // copies write into LDS comes on top.  With pre-transposed copies of K, Q and dO made by launch 1, as the
 // first form had them, each tile was copied twice; owner rows were loaded and results stored as 64 separate
 // pieces per instruction.  Measured, one kernel trace of both, us (before -> now):
-//   [2,1248,30,128]  launch 1 25.8 -> 9.6, launch 2 231 -> 226 (best 218 -> 195)
-//   [1,4608,24,128]  launch 1 31.2 -> 11.8, launch 2 969 -> 884
-//   [1,2304,12,64]   launch 1 8.1 -> 4.8, launch 2 75.9 -> 76.9
+//   [2,1248,30,128]  launch 1 25.8 -> 9.6, launch 2 231 -> 204 (best 218 -> 185)
+//   [1,4608,24,128]  launch 1 31.2 -> 11.7, launch 2 969 -> 864
+//   [1,2304,12,64]   launch 1 8.1 -> 4.9, launch 2 75.9 -> 72.5
 #include "sage_internal.h"
 #include <type_traits>
 

@@ -2,10 +2,10 @@
 //
 // attention_sage.py states the call surface: names, checks, error texts.  This module does the same work for
 // calls that meet every check — allocate the outputs, carve the workspace, call the C ABI on the current
-// stream — without the interpreter in between: 21 us of host time per call from Python and ctypes, of which
-// two launches are 5 us, became 8.  Anything it does not take (another dtype, a shape that must be refused, a
-// tensor of a subclass, a tracer or a transform, a non-zero return code) comes back as None, and the Python
-// function goes its own way and raises.
+// stream — without the interpreter in between: a call of [1,64,4,64] takes 16.4 us of host time from Python and
+// ctypes and 8.4 here, of which two launches are 5.  Anything it does not take (another dtype, a shape that must be
+// refused, a tensor of a subclass, a tracer or a transform, a non-zero return code) comes back as None, and the
+// Python function goes its own way and raises.
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
