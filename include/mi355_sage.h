@@ -357,7 +357,7 @@ int mi355_sage_attn_fwd(
  * are on their way — the same codes and scales mi355_sage_quant_qkv_bf16 writes, so O has the
  * same bits as mi355_sage_attn_fwd on that stage's q8 / qscale.  mi355_sage_quant_qkv_bf16 with
  * q8 == qscale == NULL is the quantize stage that goes with it (K and V only, qmul still written).
- * Head dims 64 and 128; a shape that the split schedule takes returns -2 (use mi355_sage_attn_fwd).
+ * Head dims 64 and 128; a shape that qualifies for the split schedule returns -2 (use mi355_sage_attn_fwd).
  * The rest of the arguments as in mi355_sage_attn_fwd.  (A stage of this library's own; the
  * reference's boundary is the one-shot call, serenitymojo/ops/cshim/cudnn_sdpa.cpp:370-393.) */
 int mi355_sage_attn_fwd_q16(

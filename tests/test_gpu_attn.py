@@ -136,6 +136,25 @@ def test_attention_stage_that_encodes_q_itself(variant, blkq, D, S):
         assert rc == -2, rc
 
 
+@pytest.mark.parametrize("B,H,Sq,Skv,D,variant", [
+    (2, 32, 320, 320, 128, 1), (3, 32, 320, 320, 128, 1),      # e4m3: up to five eighths of a round in the encoders, more in the kernel
+    (1, 30, 256, 256, 128, 1), (1, 8, 4097, 300, 64, 1),       # the short form; many queries on few keys
+    (1, 3, 8193, 129, 128, 1), (1, 2, 4160, 4097, 64, 1),      # past the lengths that the rule is asked for
+    (2, 32, 700, 700, 128, 0), (1, 33, 2040, 333, 64, 0),      # fp16: a round with room, more than a round
+    (1, 24, 510, 139, 128, 0), (1, 24, 64, 64, 128, 0), (1, 40, 256, 292, 128, 0), (2, 32, 71, 45, 256, 1)])
+def test_one_shot_gives_the_stages_bits_wherever_q_is_encoded(B, H, Sq, Skv, D, variant):
+    """Whether the encoders or the attention kernel turn Q into codes is a rule on the shape: the one-shot call has the bits
+    of the stage calls, which always take the encoders, on either side of it."""
+    import gpu_harness as G
+    rng = np.random.default_rng(Sq + Skv)
+    q, k, v = ((rng.standard_normal((B, n, H, D)).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16) for n in (Sq, Skv, Skv))
+    blkq = 128 if variant == 0 else 32
+    g = G.quant_qk(q, k, D ** -0.5, blkq, 64, True)["dev"]
+    gv = G.quant_v(v, variant)["dev"]
+    staged, _ = G.attn_fwd(g["q8"], g["qscale"], blkq, g["k8"], g["kscale"], 64, gv["vq"], gv.get("vscale"), variant, Sq, Skv)
+    np.testing.assert_array_equal(_one_shot(q, k, v, D ** -0.5, variant, blkq, 64), staged)
+
+
 def test_default_recipe_entry_point(oracle):
     """mi355_sage_sdpa_bf16 without the recipe arguments: blkq 128 / blkk 64 / smoothing and balancing on."""
     import gpu_harness as H
