@@ -273,11 +273,11 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     }
     auto dma_k_at = [&](const uint8_t* g, int slot) {
 #pragma unroll
-        for (int i = 0; i < K_CH; i++) dma16(g, ksrc[i], __builtin_amdgcn_readfirstlane(kdst[i] + slot * K_BYTES));
+        for (int i = 0; i < K_CH; i++) dma16(g, ksrc[i], kdst[i] + slot * K_BYTES);
     };
     auto dma_v_at = [&](const uint8_t* g, int slot) {
 #pragma unroll
-        for (int i = 0; i < V_CH; i++) dma16(g, vsrc[i], __builtin_amdgcn_readfirstlane(vdst[i] + slot * V_BYTES));
+        for (int i = 0; i < V_CH; i++) dma16(g, vsrc[i], vdst[i] + slot * V_BYTES);
     };
     auto dma_k = [&](int t, int slot) { dma_k_at(kg + (int64_t)key_tile(t) * K_BYTES, slot); };
     auto dma_v = [&](int t, int slot) { dma_v_at(vg + (int64_t)key_tile(t) * V_BYTES, slot); };
@@ -292,13 +292,13 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     float m_used = -3.0e38f;
     float l_run = 0.0f;            // fp16 variant: this lane's share of the row sum
     // e4m3 variant: the row sum is taken over the ROUNDED probabilities, on the matrix pipe — one
-    // more product per tile against a tile of ones (e4m3 1.0 = 0x38) gives every lane the sum over
-    // all 64 keys of its query, in every accumulator element; element 0 is the one that is kept
-    // to scale.  It is rescaled together with the output accumulators.
+    // more product per tile against a tile of ones (as e2m1, where 1.0 = 0x2 and a tile takes four registers
+    // instead of eight) gives every lane the sum over all 64 keys of its query, in every accumulator element;
+    // element 0 is the one that is kept to scale.  It is rescaled together with the output accumulators.
     v16f lacc;
 #pragma unroll
     for (int i = 0; i < 16; i++) lacc[i] = 0.0f;
-    const v8i ones8 = {0x38383838, 0x38383838, 0x38383838, 0x38383838, 0x38383838, 0x38383838, 0x38383838, 0x38383838};
+    const v8i ones4 = {0x22222222, 0x22222222, 0x22222222, 0x22222222, 0, 0, 0, 0};
 
     // The main loop advances in STEPS of SK keys: 32 for the fp16 variant (one P.V matrix
     // instruction covers 16 keys), 64 for the e4m3 variant (its matrix instruction covers 64).  A
@@ -343,6 +343,10 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     v16i s[2][SKB];
     const v16i smagic = magic_splat<D>();
     uint32_t p[2][PWS];
+    if constexpr (VARIANT == 1) {
+#pragma unroll
+        for (int w = 0; w < PWS; w++) p[0][w] = p[1][w] = 0;
+    }
 
     // Operands of slot m of a step whose score instructions read key block `kbq` (fp16 variant; the
     // e4m3 variant reads both blocks) of the K tile in `kslot` and whose P.V instructions read the
@@ -373,7 +377,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
             const v8i pw = {(int)p[pb][0], (int)p[pb][1], (int)p[pb][2], (int)p[pb][3],
                             (int)p[pb][4], (int)p[pb][5], (int)p[pb][6], (int)p[pb][7]};
             oacc[d] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a8, pw, oacc[d], 0, 0, 0, 0, 0, 0);
-            if (u == NPV - 1) lacc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(ones8, pw, lacc, 0, 0, 0, 0, 0, 0);
+            if (u == NPV - 1) lacc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(ones4, pw, lacc, 4, 0, 0, 0, 0, 0);
         }
     };
 
@@ -497,8 +501,8 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         constexpr int HT = decltype(h_tag)::value;
         constexpr bool FIRST = decltype(first_tag)::value;
         constexpr bool DOQK = decltype(qk_tag)::value;       // false in the last step
-        constexpr bool OPT = VARIANT == 0 && !FIRST && !ADDMASK;
         constexpr bool TRIP = HT >= 0 && !FIRST;             // a step of the main loop: no masked keys, scales in kst
+        constexpr bool OPT = VARIANT == 0 && !FIRST && !ADDMASK;
         static_assert(HT < 0 || (NSK == 4 && NSV == 4), "constant slots need four-slot rings");
         constexpr int SUB = HT >= 0 ? HT % SPT : -1 - HT;    // step within its tile
         static_assert(SUB >= 0 && SUB < SPT, "position in the tile");
@@ -559,7 +563,18 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         }
         float corr = 1.0f;
         bool refresh = false;
-        // the step's maximum on the raw accumulators (monotone in the score since f > 0), refresh decision
+        // largest raw accumulator of a key block (monotone in the score since f > 0)
+        auto block_max = [&](int kb) -> int {
+            int ma = max(max(s[X][kb][0], s[X][kb][1]), s[X][kb][2]);
+            int mb = max(max(s[X][kb][3], s[X][kb][4]), s[X][kb][5]);
+#pragma unroll
+            for (int i = 6; i < 14; i += 4) {
+                ma = max(max(ma, s[X][kb][i]), s[X][kb][i + 1]);
+                mb = max(max(mb, s[X][kb][i + 2]), s[X][kb][i + 3]);
+            }
+            return max(max(ma, mb), max(s[X][kb][14], s[X][kb][15]));
+        };
+        // the step's maximum, refresh decision
         auto decide = [&](float tau) {
             float mt = -INFINITY;
             if constexpr (ADDMASK) {
@@ -570,14 +585,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
             } else
 #pragma unroll
             for (int kb = 0; kb < SKB; kb++) {
-                int ma = max(max(s[X][kb][0], s[X][kb][1]), s[X][kb][2]);
-                int mb = max(max(s[X][kb][3], s[X][kb][4]), s[X][kb][5]);
-#pragma unroll
-                for (int i = 6; i < 14; i += 4) {
-                    ma = max(max(ma, s[X][kb][i]), s[X][kb][i + 1]);
-                    mb = max(max(mb, s[X][kb][i + 2]), s[X][kb][i + 3]);
-                }
-                const int mi = max(max(ma, mb), max(s[X][kb][14], s[X][kb][15]));
+                const int mi = block_max(kb);
                 const float mk = mi < 0 ? -INFINITY : (float)(mi - Magic<D>::I) * (f[kb] * (1.0f / kMagicUnit));
                 mt = fmaxf(mt, mk);
             }
@@ -590,11 +598,12 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
             m_used = m_new;
             l_run *= corr;             // already includes step h-1's probabilities
         };
-        if (!OPT) decide(Lazy<VARIANT>::tau);
+        auto constants = [&] {
 #pragma unroll
-        for (int kb = 0; kb < SKB; kb++) {
-            c0[kb] = Lazy<VARIANT>::log2_pscale - fmaf(Magic<D>::F, f[kb], m_used);
-        }
+            for (int kb = 0; kb < SKB; kb++) c0[kb] = Lazy<VARIANT>::log2_pscale - fmaf(Magic<D>::F, f[kb], m_used);
+        };
+        if (!OPT) decide(Lazy<VARIANT>::tau);
+        constants();
         // (e4m3 variant, score scales beyond anything the workloads show: see `exact_bias`; such a wave
         // takes none of its steps through the main loop)
         if constexpr (VARIANT == 1 && !ADDMASK && !TRIP) {
@@ -649,7 +658,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
                 } else {
                     const int w = k >> 1;
                     if (k & 1) p[X][w] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(ea[k][0], ea[k][1], (int)p[X][w], true);
-                    else p[X][w] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(ea[k][0], ea[k][1], 0, false);
+                    else p[X][w] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(ea[k][0], ea[k][1], ADDMASK ? 0 : (int)p[X][w], false);      // (either half is written before the word is read)
                     asm volatile("" : "+v"(p[X][w]));
                 }
             } else {
@@ -660,16 +669,14 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         // At the barrier every wave has finished the previous tile's steps completely, so the ring
         // slots they read are free: publish K(t + KOFF) / V(t), start the copies of K(t + KOFF + LEAD)
         // and V(t + LEAD).
+        // The barrier alone: LDS reads that are on their way across it are for slots this step and the next read, and the
+        // slots the copies go to were last read for matrix instructions that have been issued (__syncthreads would drain
+        // the reads: 1 % of the e4m3 loop's clocks).
+        constexpr int dt = TRIP ? ((HT + PERIOD - 1) % PERIOD + 1 % SPT) / SPT : 0;        // tiles since the trip's first step
         auto midpoint = [&]() {
             dma_wait<ADDMASK ? 0 : (LEAD - 1) * (K_CH + V_CH)>();
-            __syncthreads();
-            if constexpr (TRIP) {
-                // (the main loop stops early enough that these tiles exist; their addresses are the
-                // trip's base plus a constant)
-                constexpr int dt = ((HT + PERIOD - 1) % PERIOD + 1 % SPT) / SPT;       // tiles since the trip's first step
-                dma_k_at(kg_trip + (dt + KOFF + LEAD) * K_BYTES, slot_kcopy);
-                dma_v_at(vg_trip + (dt + LEAD) * V_BYTES, slot_vcopy);
-            } else {
+            asm volatile("s_barrier" ::: "memory");
+            if constexpr (!TRIP) {
                 dma_k(min(t + KOFF + LEAD, last), slot_kcopy);
                 dma_v(min(t + LEAD, last), slot_vcopy);
             }
@@ -699,6 +706,25 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
 #pragma unroll
             for (int n = m * NV / NM; n < (m + 1) * NV / NM; n++) vop(n);
             if (SUB == 0 && m == NM / 2 - 1) midpoint();
+            // (the main loop stops early enough that these tiles exist; their addresses are the trip's base plus a
+            // constant.  Behind the barrier by two and five slots: all waves' copies at once right behind it wait for
+            // each other at the vector memory path, and a wave that waits there issues nothing else)
+            if constexpr (TRIP && SUB == 0) {
+                if (m == NM / 2 + 1) dma_k_at(kg_trip + (dt + KOFF + LEAD) * K_BYTES, slot_kcopy);
+                if (m == NM - 2) dma_v_at(vg_trip + (dt + LEAD) * V_BYTES, slot_vcopy);
+            }
+            // A SIMD issues from its older wave first, which then stands at the barrier while the other has its SIMD's
+            // latencies to itself.  The further a wave is on its way to the next barrier, the lower its priority: the
+            // two then arrive together.  (Clocks per 64-key tile, e4m3 / fp16 at 128 channels: 2330 / 2250 with all copies
+            // behind the barrier and no priorities; 2226 / 2171 with the priorities; 2076 / 2087 with the copies moved, too;
+            // 1950 / 2120 without any barrier.  Two levels, or one for the P.V instructions: 2215, 2227.  The chip gives a
+            // part back as a lower clock: one-shot [1,16896,24,128] e4m3 2098 -> 1975 us, [1,4608,24,64] e4m3 162 -> 143,
+            // [1,4608,24,128] fp16 225 -> 221, [2,4352,30,128] fp16 473 -> 464.)
+            if constexpr (NW == 8) {
+                constexpr int SLOTS = NM * SPT;             // from one barrier to the next
+                const int past = (SUB * NM + m - (NM / 2 - 1) + SLOTS) % SLOTS, level = 3 - past * 4 / SLOTS;
+                if (past == 0 || level != 3 - (past - 1) * 4 / SLOTS) wave_priority(level);
+            }
             __builtin_amdgcn_sched_barrier(0);
         }
         if (OPT) {
@@ -706,8 +732,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
             if (__builtin_expect(__any(!(l_run - l_before <= 4096.0f)), 0)) {
                 l_run = l_before;
                 decide(0.0f);
-#pragma unroll
-                for (int kb = 0; kb < SKB; kb++) c0[kb] = Lazy<VARIANT>::log2_pscale - fmaf(Magic<D>::F, f[kb], m_used);
+                constants();
 #pragma unroll
                 for (int n = 0; n < NV; n++) vop(n);
             }
