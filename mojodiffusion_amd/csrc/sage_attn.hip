@@ -35,10 +35,13 @@
 namespace sage {
 
 // ADDMASK: an additive score bias (natural-log units, bf16, logical [B,H,Nq,Nkv] through element
-// strides with the key stride 1) is added to the dequantised scores.  That instantiation looks
-// for every step's maximum on the biased scores (no optimistic steps).  Its ordinary global loads (the bias
-// of the next step) share the vector-memory counter with the tile copies, so it waits for all of them
-// at the midpoint.
+// strides with the key stride 1) is added to the dequantised scores.  What bounds it is the way of the bias: from HBM
+// (two steps of 32 keys ahead of its use), through LDS into the scores' layout (half a step ahead), so that neither
+// latency stands in front of a step.  The fp16 variant takes its steps optimistically, like the plain forward; the
+// e4m3 variant looks for every step's maximum on the biased scores.  The bias's ordinary loads share the vector-memory
+// counter with the tile copies; that makes the waits at the midpoint longer, never shorter.  (One-shot, us, one step
+// ahead, turned and searched for its maximum in front of each step -> now: [1,1153,24,128] 68.8 -> 61.2,
+// [1,2304,24,128] 109.5 -> 99.5, [1,1700,24,128] 92.4 -> 82.7, [1,700,24,64] 33.6 -> 30.6.  Four steps ahead: 67.)
 
 // Workgroups of the split schedule that gave up on a hand-over (see the kernel's fold-in part).
 static __device__ unsigned int g_split_faults;
@@ -92,6 +95,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     constexpr int FPU = VARIANT == 0 ? 1 : 2;           // 16-byte V fragments per PV instruction
     constexpr int PD = VARIANT == 0 ? 2 : 1;            // V fragment prefetch distance (units)
     constexpr int PW = VARIANT == 0 ? 16 : 8;           // dwords of packed P per tile
+    constexpr bool BPIPE = ADDMASK && VARIANT == 0 && D <= 128 && !SPLIT;      // see ADDMASK
     static_assert(32 % NUNIT == 0 && (EPU % 2 == 0 || EPU == 1), "unit split");
 
     __shared__ __attribute__((aligned(1024))) uint8_t lds_k[NSK][K_BYTES];
@@ -470,12 +474,33 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     // [1,3840 x 192,32,128] 90.1 -> 42.6 us, [1,4000,16,128] 133.9 -> 116.2, [1,2304,18,256] 193.6 -> 187.1).
     const int last_step = (ntiles * SPT + 1) / 2 * 2 - 1;
     auto key_step = [&](int h) -> int { return (t_off + key_tile(h / SPT) - h / SPT) * SPT + h; };       // step h's keys: key_step(h) * SK ..
-    BiasStage bias[SKB];                                // the next step's bias on its way
-    auto bias_load = [&](int h) {
+    // The bias of the next two steps on its way (of one where two do not fit the registers), and (BPIPE) in the
+    // scores' layout that of this step and the next, by parity of the step: dword k = scores 2k, 2k + 1 of the lane.
+    constexpr int NBIAS = (VARIANT == 1 && D == 128) || D > 128 || SPLIT ? 1 : 2;
+    BiasStage bias[NBIAS][SKB];
+    uint32_t mv[2][BPIPE ? 8 : 1];
+    BiasStage::Rows brows{};
+    if constexpr (ADDMASK) brows = BiasStage::rows(mhead, amn, wave_row0, Nq - 1, lane);
+    auto bias_load = [&](int h, BiasStage (&to)[SKB]) {
 #pragma unroll
-        for (int kb = 0; kb < SKB; kb++) bias[kb].load(mhead, amn, wave_row0, Nq - 1, key_step(min(h, last_step)) * SK + kb * 32, kv_valid, lane);
+        for (int kb = 0; kb < SKB; kb++) to[kb].load(brows, key_step(min(h, last_step)) * SK + kb * 32, kv_valid, lane);
     };
-    if constexpr (ADDMASK) bias_load(0);
+    auto bias_turn = [&](int h, const BiasStage& from, uint32_t (&to)[BPIPE ? 8 : 1]) {
+        from.put(lds_bias[wave], lane, key_step(min(h, last_step)) * SK, kv_valid);             // (a wave's own LDS accesses keep their order)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const u32x2 w = BiasStage::get_packed(lds_bias[wave], l32, half, g);
+            if constexpr (BPIPE) to[2 * g] = w.x, to[2 * g + 1] = w.y;
+        }
+    };
+    if constexpr (ADDMASK) {
+#pragma unroll
+        for (int i = 0; i < NBIAS; i++) bias_load(i, bias[i]);
+        if constexpr (BPIPE) {
+            bias_turn(0, bias[0][0], mv[0]);
+            bias_load(NBIAS, bias[0]);
+        }
+    }
 #pragma unroll
     for (int m = PF - 1; m >= 0; m--)
         if (slot_is_qk(m)) fetch(m, (1 / SPT) % NSK, 1 % SPT, 0, 0);
@@ -502,7 +527,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         constexpr bool FIRST = decltype(first_tag)::value;
         constexpr bool DOQK = decltype(qk_tag)::value;       // false in the last step
         constexpr bool TRIP = HT >= 0 && !FIRST;             // a step of the main loop: no masked keys, scales in kst
-        constexpr bool OPT = VARIANT == 0 && !FIRST && !ADDMASK;
+        constexpr bool OPT = VARIANT == 0 && !FIRST && (!ADDMASK || BPIPE);
         static_assert(HT < 0 || (NSK == 4 && NSV == 4), "constant slots need four-slot rings");
         constexpr int SUB = HT >= 0 ? HT % SPT : -1 - HT;    // step within its tile
         static_assert(SUB >= 0 && SUB < SPT, "position in the tile");
@@ -541,25 +566,27 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
                 }
             }
         }
-        // biased scores in the log2 domain, without the reference maximum (ADDMASK only)
-        float xs[SKB][ADDMASK ? 16 : 1];
-        if constexpr (ADDMASK) {
+        // Biased scores in the log2 domain, without the reference maximum.  (The bias of the accumulators is taken off
+        // before the multiplication: exact, where folding it into the multiply-add's constant would cost the constant's
+        // rounding.)
+        auto biased = [&](int kb, int i, float m) -> float {
+            return fmaf(__int_as_float(s[X][kb][i]) - Magic<D>::F, f[kb], m);
+        };
+        auto mv_at = [&](int i) -> float { return __uint_as_float(i & 1 ? mv[X][i >> 1] & 0xFFFF0000u : mv[X][i >> 1] << 16); };
+        constexpr float kLog2e = 1.4426950408889634f;
+        float xs[SKB][ADDMASK && !BPIPE ? 16 : 1];
+        if constexpr (ADDMASK && !BPIPE) {
 #pragma unroll
             for (int kb = 0; kb < SKB; kb++) {
-                bias[kb].put(lds_bias[wave], lane);     // (a wave's own LDS accesses keep their order)
-                // (the bias of the accumulators is taken off before the multiplication: exact, where
-                // folding it into the multiply-add's constant would cost the constant's rounding)
+                bias[X % NBIAS][kb].put(lds_bias[wave], lane, hk * SK + kb * 32, kv_valid);     // (a wave's own LDS accesses keep their order)
 #pragma unroll
                 for (int g = 0; g < 4; g++) {
-                    const v4f mv = BiasStage::get(lds_bias[wave], l32, half, g);
+                    const v4f w = BiasStage::get(lds_bias[wave], l32, half, g);
 #pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        const float sdq = (__int_as_float(s[X][kb][g * 4 + e]) - Magic<D>::F) * f[kb];
-                        xs[kb][g * 4 + e] = fmaf(mv[e], 1.4426950408889634f, sdq);
-                    }
+                    for (int e = 0; e < 4; e++) xs[kb][g * 4 + e] = fmaf(w[e], kLog2e, biased(kb, g * 4 + e, 0.0f));
                 }
             }
-            bias_load(h + 1);
+            bias_load(h + NBIAS, bias[X % NBIAS]);
         }
         float corr = 1.0f;
         bool refresh = false;
@@ -581,7 +608,10 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
 #pragma unroll
                 for (int kb = 0; kb < SKB; kb++)
 #pragma unroll
-                    for (int i = 0; i < 16; i++) mt = fmaxf(mt, xs[kb][i]);
+                    for (int i = 0; i < 16; i++) {
+                        if constexpr (BPIPE) mt = fmaxf(mt, fmaf(mv_at(i), kLog2e, biased(kb, i, 0.0f)));
+                        else mt = fmaxf(mt, xs[kb][i]);
+                    }
             } else
 #pragma unroll
             for (int kb = 0; kb < SKB; kb++) {
@@ -661,7 +691,8 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
             }
             const int kb = k >> 3, i = (2 * k) & 15;
             if (r < 2) {
-                if constexpr (ADDMASK) ea[k][r] = xs[kb][i + r] - (m_used - Lazy<VARIANT>::log2_pscale);
+                if constexpr (BPIPE) ea[k][r] = fmaf(mv_at(i + r), kLog2e, biased(kb, i + r, -m_used));
+                else if constexpr (ADDMASK) ea[k][r] = xs[kb][i + r] - (m_used - Lazy<VARIANT>::log2_pscale);
                 else ea[k][r] = fmaf(__int_as_float(s[X][kb][i + r]), f[kb], c0[kb]);
             } else if (r < 4) {
                 ea[k][r - 2] = __builtin_amdgcn_exp2f(ea[k][r - 2]);
@@ -691,7 +722,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         // the reads: 1 % of the e4m3 loop's clocks).
         constexpr int dt = TRIP ? ((HT + PERIOD - 1) % PERIOD + 1 % SPT) / SPT : 0;        // tiles since the trip's first step
         auto midpoint = [&]() {
-            dma_wait<ADDMASK ? 0 : (LEAD - 1) * (K_CH + V_CH)>();
+            dma_wait<(LEAD - 1) * (K_CH + V_CH)>();         // (younger loads of the bias only make it wait for more)
             asm volatile("s_barrier" ::: "memory");
             if constexpr (!TRIP) {
                 dma_k(min(t + KOFF + LEAD, last), slot_kcopy);
@@ -723,6 +754,13 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
 #pragma unroll
             for (int n = m * NV / NM; n < (m + 1) * NV / NM; n++) vop(n);
             if (SUB == 0 && m == NM / 2 - 1) midpoint();
+            if constexpr (BPIPE) {
+                if (m == NM / 2) {
+                    constexpr int NEXT = (X ^ 1) % NBIAS;
+                    bias_turn(h + 1, bias[NEXT][0], mv[X ^ 1]);
+                    bias_load(h + 1 + NBIAS, bias[NEXT]);
+                }
+            }
             // (the main loop stops early enough that these tiles exist; their addresses are the trip's base plus a
             // constant.  Behind the barrier by two and five slots: all waves' copies at once right behind it wait for
             // each other at the vector memory path, and a wave that waits there issues nothing else)

@@ -164,31 +164,56 @@ struct BiasStage {
     u32x4 w[NI];
 
     static __device__ __forceinline__ int at(int row, int chunk) { return row * 64 + ((chunk ^ ((row >> 2) & 3)) << 4); }
-    // keys key0 .. key0 + 31 of rows row0 .. row0 + 31 (rows past the last repeat it; keys at and past n are 0).
-    // Rows start at any even byte address: the access is as wide as the hardware takes it unaligned.
-    __device__ __forceinline__ void load(const uint16_t* head, int64_t row_stride, int row0, int last_row, int key0, int n, int lane) {
-        const int key = key0 + (lane % CPR) * 8;
+    // the lane's rows of row0 .. row0 + 31 (rows past the last repeat it)
+    struct Rows { const uint16_t* p[NI]; };
+    static __device__ __forceinline__ Rows rows(const uint16_t* head, int64_t row_stride, int row0, int last_row, int lane) {
+        Rows r;
 #pragma unroll
-        for (int i = 0; i < NI; i++) {
-            const uint16_t* p = head + (int64_t)min(row0 + i * RPI + lane / CPR, last_row) * row_stride + key;
-            uint32_t v[4] = {0u, 0u, 0u, 0u};
-            if (key + 8 <= n) {
-                __builtin_memcpy(v, p, 16);
-            } else {
+        for (int i = 0; i < NI; i++) r.p[i] = head + (int64_t)min(row0 + i * RPI + lane / CPR, last_row) * row_stride;
+        return r;
+    }
+    // Keys key0 .. key0 + 31 of those rows, n of which there are.  Rows start at any even byte address: the access is as
+    // wide as the hardware takes it unaligned.  A chunk that reaches past its row's end is loaded as the row's last eight
+    // keys and shifted on its way to LDS: one load for all lanes, nothing past a row's end is read.  (Rows of fewer than
+    // eight keys are taken key by key.)
+    __device__ __forceinline__ void load(const Rows& r, int key0, int n, int lane) {
+        const int key = key0 + (lane % CPR) * 8;
+        if (__builtin_expect(n >= 8, 1)) {
+#pragma unroll
+            for (int i = 0; i < NI; i++) __builtin_memcpy(&w[i], r.p[i] + min(key, n - 8), 16);
+        } else {
+#pragma unroll
+            for (int i = 0; i < NI; i++) {
+                uint32_t v[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
                 for (int e = 0; e < 8; e++)
-                    if (key + e < n) v[e >> 1] |= (uint32_t)p[e] << ((e & 1) * 16);
+                    if (key + e < n) v[e >> 1] |= (uint32_t)r.p[i][key + e] << ((e & 1) * 16);
+                w[i] = u32x4{v[0], v[1], v[2], v[3]};
             }
-            w[i] = u32x4{v[0], v[1], v[2], v[3]};
         }
     }
-    __device__ __forceinline__ void put(uint8_t* lds, int lane) const {
+    // (keys at and past n are 0)
+    __device__ __forceinline__ void put(uint8_t* lds, int lane, int key0, int n) const {
 #pragma unroll
-        for (int i = 0; i < NI; i++) *reinterpret_cast<u32x4*>(lds + at(i * RPI + lane / CPR, lane % CPR)) = w[i];
+        for (int i = 0; i < NI; i++) {
+            u32x4 x = w[i];
+            if (__builtin_expect(key0 + 32 > n && n >= 8, 0)) {
+                const int d = key0 + (lane % CPR) * 8 - (n - 8);        // keys to shift out
+                if (d & 4) x = u32x4{x.z, x.w, 0u, 0u};
+                if (d & 2) x = u32x4{x.y, x.z, x.w, 0u};
+                if (d & 1) x = u32x4{(x.x >> 16) | (x.y << 16), (x.y >> 16) | (x.z << 16), (x.z >> 16) | (x.w << 16), x.w >> 16};
+                if (d >= 8) x = u32x4{0u, 0u, 0u, 0u};
+                if (d <= 0) x = w[i];
+            }
+            *reinterpret_cast<u32x4*>(lds + at(i * RPI + lane / CPR, lane % CPR)) = x;
+        }
     }
     // keys g * 8 + half * 4 .. + 3 of row l32
+    static __device__ __forceinline__ u32x2 get_packed(const uint8_t* lds, int l32, int half, int g) {
+        return *reinterpret_cast<const u32x2*>(lds + at(l32, g) + half * 8);
+    }
     static __device__ __forceinline__ v4f get(const uint8_t* lds, int l32, int half, int g) {
-        const u32x2 v = *reinterpret_cast<const u32x2*>(lds + at(l32, g) + half * 8);
+        const u32x2 v = get_packed(lds, l32, half, g);
         return v4f{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xFFFF0000u), __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xFFFF0000u)};
     }
 };

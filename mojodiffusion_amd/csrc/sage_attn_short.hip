@@ -27,8 +27,9 @@ namespace sage {
 template <int D> constexpr int kMainRows = D > 128 ? 128 : 256;               // rows per workgroup of the main kernel
 template <int D> constexpr int short_waves() { return D > 128 ? 4 : 8; }      // 256 channels: a wave needs a SIMD's registers
 
+// (64 channels, fp16: two workgroups share a compute unit, which takes 128 registers at most)
 template <int D, int VARIANT, int KW, bool QF, bool ADDMASK>
-__global__ __launch_bounds__(short_waves<D>() * 64) void sage_attn_short_kernel(AttnArgs a, int n_rtiles, int item0, int total_wg) {
+__global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 : 1) void sage_attn_short_kernel(AttnArgs a, int n_rtiles, int item0, int total_wg) {
     constexpr int NW = short_waves<D>();
     constexpr int R = NW / KW;                          // 32-row blocks per workgroup
     constexpr int ROWS = 32 * R;
@@ -207,10 +208,12 @@ __global__ __launch_bounds__(short_waves<D>() * 64) void sage_attn_short_kernel(
     // the bias of a step is loaded while the step before it runs
     BiasStage bias[SKB];
     uint8_t* bias_lds = &mem.ring[wave].bias[0];
+    BiasStage::Rows brows{};
+    if (ADDMASK) brows = BiasStage::rows(a.amask + b * a.amb + h * a.amh, a.amn, row0, a.Nq - 1, lane);
     auto bias_load = [&](int hs) {
 #pragma unroll
         for (int kb = 0; kb < SKB; kb++)
-            bias[kb].load(a.amask + b * a.amb + h * a.amh, a.amn, row0, a.Nq - 1, key_step(min(hs, h1 - 1)) * SK + kb * 32, kv_valid, lane);
+            bias[kb].load(brows, key_step(min(hs, h1 - 1)) * SK + kb * 32, kv_valid, lane);
     };
     if (ADDMASK && h0 < h1) bias_load(h0);
 
@@ -262,7 +265,7 @@ __global__ __launch_bounds__(short_waves<D>() * 64) void sage_attn_short_kernel(
 #pragma unroll
         for (int kb = 0; kb < SKB; kb++) {
             if constexpr (ADDMASK) {
-                bias[kb].put(bias_lds, lane);
+                bias[kb].put(bias_lds, lane, key0 + kb * 32, kv_valid);
 #pragma unroll
                 for (int g = 0; g < 4; g++) {
                     const v4f mv = BiasStage::get(bias_lds, l32, half, g);
