@@ -747,6 +747,15 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdArgs& a, uint8_t* smem, i
     else dkdv_role<D, 1>(a, smem, bh, xt, wave, lane);
 }
 
+// Workgroup j of n of a kind -> the block it works on: consecutive ids go to the 8 XCDs in turn, and each XCD takes a
+// contiguous range of blocks, so that the blocks of a head, which all walk the same rows, share one L2.  (Launch 1 + 2,
+// us, blocks in the order of ids -> so: [2,1248,30,128] 196.7 -> 191.8, [2,2001,40,64] 310.8 -> 304.6, level where a
+// few heads are all there is.)
+__device__ __forceinline__ int xcd_block(int j, int n) {
+    const int per = n >> 3, extra = n & 7, xcd = j & 7;
+    return xcd * per + min(xcd, extra) + (j >> 3);
+}
+
 // One grid for both: the first n_dq workgroups are the dQ pass (the longer ones first), the rest
 // the dK/dV pass.  Both take a whole CU (8 waves, most of the LDS); in one grid the second
 // kind starts on a CU as soon as the first kind runs out, instead of after its last workgroup.
@@ -757,9 +766,10 @@ __global__ __launch_bounds__(512, 2) void bwd_fused_kernel(BwdArgs a, int n_dq) 
     constexpr int BYTES = KV_BYTES > PassLds<D, 0>::BYTES ? KV_BYTES : PassLds<D, 0>::BYTES;
     __shared__ __attribute__((aligned(1024))) uint8_t smem[BYTES];
     const int block = (int)blockIdx.x;
-    if (block < n_dq) bwd_pass_body<D, 0>(a, smem, block);
-    else if constexpr (PAIRED) bwd_dkdv_body<D>(a, smem, block - n_dq);
-    else bwd_pass_body<D, 1>(a, smem, block - n_dq);
+    const int n_kv = (int)gridDim.x - n_dq;
+    if (block < n_dq) bwd_pass_body<D, 0>(a, smem, xcd_block(block, n_dq));
+    else if constexpr (PAIRED) bwd_dkdv_body<D>(a, smem, xcd_block(block - n_dq, n_kv));
+    else bwd_pass_body<D, 1>(a, smem, xcd_block(block - n_dq, n_kv));
 }
 
 template <int D>
