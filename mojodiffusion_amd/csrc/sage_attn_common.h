@@ -44,14 +44,6 @@ template <int N> __device__ __forceinline__ void dma_wait() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// Issue priority of this wave among those of its SIMD, 0 .. 3 (the instruction takes a constant only).
-__device__ __forceinline__ void wave_priority(int level) {
-    if (level == 0) __builtin_amdgcn_s_setprio(0);
-    else if (level == 1) __builtin_amdgcn_s_setprio(1);
-    else if (level == 2) __builtin_amdgcn_s_setprio(2);
-    else __builtin_amdgcn_s_setprio(3);
-}
-
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
 }

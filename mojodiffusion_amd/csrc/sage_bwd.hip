@@ -432,9 +432,13 @@ __device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, uint8_t* smem, i
                 acc2[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, fa), __builtin_bit_cast(v8bf, pb), acc2[d], 0, 0, 0);
             }
         };
+        // (the further a wave is on its way to the next tile's barrier, the lower its priority: the two waves of a SIMD,
+        // which issues from the older one first, arrive there together.  Head dim 64: 1.5 % of launch 2)
+        wave_priority(3);
         scores_load(0, 0);
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) scores_step(0, ks);
+        wave_priority(2);
         // scores of block 1 with the exponentials of block 0: 8 pairs over KS k-steps
         scores_load(1, 0);
 #pragma unroll
@@ -443,6 +447,7 @@ __device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, uint8_t* smem, i
 #pragma unroll
             for (int q = 0; q < 8 / KS; q++) softmax_pair(0, (ks * (8 / KS) + q) * 2);
         }
+        wave_priority(1);
         // accumulation of block 0 with the exponentials of block 1: 8 pairs over ACC_M instructions
         // (ACC_M is 4, 8 or 16; with 16 a pair goes with every second instruction)
 #pragma unroll
@@ -455,6 +460,7 @@ __device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, uint8_t* smem, i
                 if (m & 1) softmax_pair(1, (m >> 1) * 2);
             }
         }
+        wave_priority(0);
 #pragma unroll
         for (int m = 0; m < ACC_M; m++) acc_step(1, m);
     };
@@ -624,8 +630,10 @@ __device__ __forceinline__ void dkdv_role(const BwdArgs& a, uint8_t* smem, int b
         const int next = slot == 2 ? 0 : slot + 1;
         const int mine = ROLE == 0 ? slot : slot == 0 ? 2 : slot - 1;
         slot = next;
-        if (it + 1 < ntiles) copy_tile(it + 1, next);
-        if (ROLE == 0 ? it >= ntiles : it == 0) continue;
+        if (ROLE == 0 ? it >= ntiles : it == 0) {
+            if (it + 1 < ntiles) copy_tile(it + 1, next);
+            continue;
+        }
 
         const uint8_t* nt = smem + L::RING + mine * L::SLOT + ROLE * TILE_BYTES;
         const uint8_t* rt = smem + L::RING + mine * L::SLOT + (1 - ROLE) * TILE_BYTES;
@@ -699,6 +707,10 @@ __device__ __forceinline__ void dkdv_role(const BwdArgs& a, uint8_t* smem, int b
         scores_load(0, 0);
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) scores_step(0, ks);
+        // The next tile's copies: behind the first block's scores, so that the wave's matrix instructions run while it
+        // stands at the vector memory path, where all eight waves' copies meet (in front of them the launch took, us:
+        // [2,1248,30,128] 185.6, here 181.9; [1,3000,16,128] 268.9, 257.9; behind the second block's scores 184.3, 265.8).
+        if (it + 1 < ntiles) copy_tile(it + 1, next);
         scores_load(1, 0);
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {

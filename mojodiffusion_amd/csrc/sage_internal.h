@@ -123,6 +123,14 @@ __device__ __forceinline__ float rint_quotient(float x, float sc, float rinv, bo
     return n;
 }
 
+// Issue priority of this wave among those of its SIMD, 0 .. 3 (the instruction takes a constant only).
+__device__ __forceinline__ void wave_priority(int level) {
+    if (level == 0) __builtin_amdgcn_s_setprio(0);
+    else if (level == 1) __builtin_amdgcn_s_setprio(1);
+    else if (level == 2) __builtin_amdgcn_s_setprio(2);
+    else __builtin_amdgcn_s_setprio(3);
+}
+
 struct AttnArgs {
     const int8_t* q8;  const float* qscale;  int blkq;
     const int8_t* k8;  const float* kscale;  int blkk;
