@@ -46,14 +46,17 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
     static_assert(NW % KW == 0 && ROWS <= 128, "waves = row blocks x key runs");
 
     struct Ring { uint8_t k[K_BYTES], v[V_BYTES], bias[ADDMASK ? BiasStage::BYTES : 16]; };
+    // A wave's loop operands, then its partial output for the merge, in the same place: a wave that is done with its
+    // keys leaves its output without waiting for the others.
     union Mem {
-        Ring ring[NW];                                  // the loop's operands
-        float acc[NW][32 * LD];                         // the merge's partial outputs
+        Ring ring;
+        float acc[32 * LD];
+        uint8_t stride[((sizeof(Ring) > 32 * LD * 4 ? sizeof(Ring) : 32 * LD * 4) + 255) / 256 * 256];
     };
-    __shared__ __attribute__((aligned(1024))) Mem mem;
+    __shared__ __attribute__((aligned(1024))) Mem mem[NW];
     __shared__ __attribute__((aligned(16))) uint8_t lds_q[QF ? ROWS * D : 16];      // this workgroup's Q codes
     __shared__ float lds_m[NW][32], lds_l[NW][32];
-    __shared__ float lds_qmax[8];
+    __shared__ __attribute__((aligned(16))) float lds_qmax[8];
 
     // each XCD takes a contiguous range of workgroups, so that those sharing a head share its L2
     const int bid = blockIdx.x;
@@ -88,7 +91,7 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
     // ---- one step's operands: copies into the wave's own LDS region, fragments out of it
     const uint8_t* kg = reinterpret_cast<const uint8_t*>(a.k8) + (int64_t)bh * a.nkv_pad * D;
     const uint8_t* vg = static_cast<const uint8_t*>(a.vq) + (int64_t)bh * a.nkv_pad * D * VB;
-    const uint32_t k_lds = lds_addr(&mem.ring[wave].k[0]), v_lds = lds_addr(&mem.ring[wave].v[0]);
+    const uint32_t k_lds = lds_addr(&mem[wave].ring.k[0]), v_lds = lds_addr(&mem[wave].ring.v[0]);
     int vsrc[VC];
 #pragma unroll
     for (int i = 0; i < VC; i++) {
@@ -120,10 +123,12 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
     };
     // (LDS reads issued before this have delivered: what they read may be overwritten)
     auto reads_done = [] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
-    if (h0 < h1) {
-        copy_k(h0);
-        copy_v(h0);
-    }
+    auto first_copies = [&] {
+        if (h0 < h1) {
+            copy_k(h0);
+            copy_v(h0);
+        }
+    };
 
     // ---- Q^T fragments of the wave's 32 rows
     v4i qf[KSTEPS];
@@ -133,10 +138,12 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
 #pragma unroll
         for (int s = 0; s < KSTEPS; s++) qf[s] = *reinterpret_cast<const v4i*>(qp + s * 32);
         sq = a.qscale[(int64_t)bh * (a.nq_pad / a.blkq) + qrow / a.blkq] * kMagicUnit;
+        first_copies();
     } else {
         // Q arrives as bf16: the quantizer's arithmetic, so its codes and scales.  A scale block is wider
         // than the workgroup's rows as a rule: the waves take the maxima of the whole block, 16 rows at a
-        // time, and the ones that hold this workgroup's rows encode them into LDS for everybody.
+        // time, and then all of them encode this workgroup's rows into LDS, a chunk or two of eight channels per
+        // thread.  (By the waves that had taken those rows' maxima, two of eight, it took 0.7 us instead of 0.2.)
         const uint16_t* qb = a.q_src + b * a.qsb + h * a.qsh;
         const int cover = a.blkq > ROWS ? a.blkq : ROWS;                 // 32 .. 128 rows: the scale blocks of this workgroup
         const int cover0 = wg_row0 / cover * cover;
@@ -153,6 +160,15 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
                 w[t][i] = u32x4{0u, 0u, 0u, 0u};
                 if (piece < cover / 16 && row < a.Nq) w[t][i] = *reinterpret_cast<const u32x4*>(qb + (int64_t)row * a.qsn + col);
             }
+        constexpr int OWN = (ROWS * CPR + NW * 64 - 1) / (NW * 64);      // this thread's chunks of the workgroup's rows
+        static_assert(ROWS * CPR % 64 == 0 && (NW * 64) % CPR == 0, "whole waves of chunks, one column per thread");
+        u32x4 own[OWN];
+#pragma unroll
+        for (int i = 0; i < OWN; i++) {
+            const int row = wg_row0 + i * (NW * 64 / CPR) + tid / CPR;
+            own[i] = u32x4{0u, 0u, 0u, 0u};
+            if (row < a.Nq) own[i] = *reinterpret_cast<const u32x4*>(qb + (int64_t)row * a.qsn + col);
+        }
         float m[8];
         {
             const float* mp = a.qmul + (int64_t)bh * D + col;
@@ -160,6 +176,7 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
 #pragma unroll
             for (int e = 0; e < 4; e++) m[e] = m0[e], m[4 + e] = m1[e];
         }
+        first_copies();
 #pragma unroll
         for (int t = 0; t < TURNS; t++) {
             float am = 0.0f;
@@ -173,41 +190,44 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
             if (lane == 0) lds_qmax[t * NW + wave] = am;
         }
         __syncthreads();
+        // (all eight maxima in two reads and the block's picked: as a loop over them, one after the other, this was half a
+        // microsecond each time it was asked)
+        const int blk16 = a.blkq >> 4, blksh = a.blkq == 32 ? 5 : a.blkq == 64 ? 6 : 7;
+        const v4f qm0 = *reinterpret_cast<const v4f*>(&lds_qmax[0]), qm1 = *reinterpret_cast<const v4f*>(&lds_qmax[4]);
         auto block_scale = [&](int row) {                                // of the scale block that holds `row`
-            const int s0 = (row - cover0) / a.blkq * (a.blkq / 16);
+            const int s0 = ((row - cover0) >> blksh) * blk16;
             float am = 0.0f;
-            for (int i = 0; i < a.blkq / 16; i++) am = fmaxf(am, lds_qmax[s0 + i]);
+#pragma unroll
+            for (int i = 0; i < 8; i++) am = i >= s0 && i < s0 + blk16 ? fmaxf(am, i < 4 ? qm0[i & 3] : qm1[i & 3]) : am;
             return am > 0.0f ? am / 127.0f : 1.0f;
         };
+        sq = block_scale(row0) * kMagicUnit;
 #pragma unroll
-        for (int t = 0; t < TURNS; t++) {
-            const int prow = cover0 + (t * NW + wave) * 16 - wg_row0;    // first row of the piece in this workgroup
-            if (prow < 0 || prow >= ROWS) continue;
-            const float sc = block_scale(wg_row0 + prow);
+        for (int i = 0; i < OWN; i++) {
+            // (a wave's rows lie in one scale block: it holds 2 to 8 of them, from a multiple of that on)
+            const int row = i * (NW * 64 / CPR) + tid / CPR;
+            if (ROWS * CPR < NW * 64 && row >= ROWS) break;
+            const float sc = block_scale(wg_row0 + row);
             const bool fast = sc >= 0x1p-100f && sc <= 0x1p100f;
             const float rinv = 1.0f / sc;
+            float x[8];
 #pragma unroll
-            for (int i = 0; i < NI; i++) {
-                float x[8];
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    x[2 * e] = __uint_as_float(w[t][i][e] << 16) * m[2 * e];
-                    x[2 * e + 1] = __uint_as_float(w[t][i][e] & 0xFFFF0000u) * m[2 * e + 1];
-                }
-                *reinterpret_cast<u32x2*>(&lds_q[(prow + i * RPI + rr) * D + col]) = encode8_i8(x, sc, rinv, fast);
+            for (int e = 0; e < 4; e++) {
+                x[2 * e] = __uint_as_float(own[i][e] << 16) * m[2 * e];
+                x[2 * e + 1] = __uint_as_float(own[i][e] & 0xFFFF0000u) * m[2 * e + 1];
             }
+            *reinterpret_cast<u32x2*>(&lds_q[row * D + col]) = encode8_i8(x, sc, rinv, fast);
         }
         __syncthreads();
 #pragma unroll
         for (int s = 0; s < KSTEPS; s++) qf[s] = *reinterpret_cast<const v4i*>(&lds_q[(rg * 32 + l32) * D + s * 32 + half * 16]);
-        sq = block_scale(row0) * kMagicUnit;
     }
 
     const float* ksc = a.kscale + (int64_t)bh * (a.nkv_pad / a.blkk);
     const int ksh = a.blkk == 32 ? 5 : a.blkk == 64 ? 6 : 7;
     // the bias of a step is loaded while the step before it runs
     BiasStage bias[SKB];
-    uint8_t* bias_lds = &mem.ring[wave].bias[0];
+    uint8_t* bias_lds = &mem[wave].ring.bias[0];
     BiasStage::Rows brows{};
     if (ADDMASK) brows = BiasStage::rows(a.amask + b * a.amb + h * a.amh, a.amn, row0, a.Nq - 1, lane);
     auto bias_load = [&](int hs) {
@@ -361,18 +381,13 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
         lds_m[wave][l32] = m_used;
         lds_l[wave][l32] = l_row;
     }
-    __syncthreads();
     {
-        float mg = lds_m[rg * KW][l32];
-#pragma unroll
-        for (int w = 1; w < KW; w++) mg = fmaxf(mg, lds_m[rg * KW + w][l32]);
-        const float sc = __builtin_amdgcn_exp2f(m_used - mg);
-        float* dst = &mem.acc[wave][l32 * LD + half * 4];
+        float* dst = &mem[wave].acc[l32 * LD + half * 4];
 #pragma unroll
         for (int d = 0; d < DB; d++)
 #pragma unroll
             for (int g = 0; g < 4; g++)
-                *reinterpret_cast<v4f*>(dst + d * 32 + g * 8) = v4f{oacc[d][g * 4] * sc, oacc[d][g * 4 + 1] * sc, oacc[d][g * 4 + 2] * sc, oacc[d][g * 4 + 3] * sc};
+                *reinterpret_cast<v4f*>(dst + d * 32 + g * 8) = v4f{oacc[d][g * 4], oacc[d][g * 4 + 1], oacc[d][g * 4 + 2], oacc[d][g * 4 + 3]};
     }
     __syncthreads();
     // ---- normalise, bf16, caller's strides: eight channels of a row per thread and turn
@@ -387,9 +402,11 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
         v4f x0 = {0.0f, 0.0f, 0.0f, 0.0f}, x1 = x0;
 #pragma unroll
         for (int w = 0; w < KW; w++) {
-            l_tot += lds_l[r * KW + w][rl] * __builtin_amdgcn_exp2f(lds_m[r * KW + w][rl] - mg);
-            x0 += *reinterpret_cast<const v4f*>(&mem.acc[r * KW + w][rl * LD + ch]);
-            x1 += *reinterpret_cast<const v4f*>(&mem.acc[r * KW + w][rl * LD + ch + 4]);
+            const float sc = __builtin_amdgcn_exp2f(lds_m[r * KW + w][rl] - mg);
+            const v4f y0 = *reinterpret_cast<const v4f*>(&mem[r * KW + w].acc[rl * LD + ch]), y1 = *reinterpret_cast<const v4f*>(&mem[r * KW + w].acc[rl * LD + ch + 4]);
+            l_tot = fmaf(lds_l[r * KW + w][rl], sc, l_tot);
+#pragma unroll
+            for (int e = 0; e < 4; e++) x0[e] = fmaf(y0[e], sc, x0[e]), x1[e] = fmaf(y1[e], sc, x1[e]);
         }
         const float inv = 1.0f / l_tot;
         if constexpr (VARIANT == 1) {
