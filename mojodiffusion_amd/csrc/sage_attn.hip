@@ -407,8 +407,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
             for (int e = 0; e < 4; e++)
                 am = fmaxf(fmaxf(am, fabsf(__uint_as_float(rw[i][e] << 16) * qm[2 * e])), fabsf(__uint_as_float(rw[i][e] & 0xFFFF0000u) * qm[2 * e + 1]));
         // the wave's 32 rows, then the waves that share a scale block
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) am = fmaxf(am, __shfl_xor(am, off, 64));
+        am = wave_max(am);
         if (blkq > 32) {
             if (lane == 0) lds_qmax[wave] = am;
             __syncthreads();

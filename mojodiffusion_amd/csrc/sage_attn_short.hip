@@ -185,8 +185,7 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
 #pragma unroll
                 for (int e = 0; e < 4; e++)
                     am = fmaxf(fmaxf(am, fabsf(__uint_as_float(w[t][i][e] << 16) * m[2 * e])), fabsf(__uint_as_float(w[t][i][e] & 0xFFFF0000u) * m[2 * e + 1]));
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) am = fmaxf(am, __shfl_xor(am, off, 64));
+            am = wave_max(am);
             if (lane == 0) lds_qmax[t * NW + wave] = am;
         }
         __syncthreads();

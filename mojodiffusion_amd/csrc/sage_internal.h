@@ -131,6 +131,22 @@ __device__ __forceinline__ void wave_priority(int level) {
     else __builtin_amdgcn_s_setprio(3);
 }
 
+// The wave's maximum, in every lane, without the LDS pipe: four exchanges as modifiers of the instruction inside rows of
+// 16 lanes, two swaps across them (as LDS permutes the six steps are 0.25 us one after the other).
+__device__ __forceinline__ float wave_max(float v) {
+    typedef unsigned v2u __attribute__((ext_vector_type(2)));
+#define SAGE_DPP_MAX(CTRL) v = fmaxf(v, __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), CTRL, 0xF, 0xF, false)))
+    SAGE_DPP_MAX(0xB1);         // quad_perm: lanes xor 1
+    SAGE_DPP_MAX(0x4E);         // lanes xor 2
+    SAGE_DPP_MAX(0x141);        // row_half_mirror: the other quad of eight
+    SAGE_DPP_MAX(0x140);        // row_mirror: the other eight of sixteen
+#undef SAGE_DPP_MAX
+    const v2u a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(a.x), __uint_as_float(a.y));
+    const v2u b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(b.x), __uint_as_float(b.y));
+}
+
 struct AttnArgs {
     const int8_t* q8;  const float* qscale;  int blkq;
     const int8_t* k8;  const float* kscale;  int blkk;

@@ -49,12 +49,6 @@ __device__ __forceinline__ void load8(const float* p, float* x) {
     x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
 }
 
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-    return v;
-}
-
 __device__ __forceinline__ bool key_kept(int s, int N, const KeyMask& m) { return s < N && !(s >= m.lo && s < m.hi); }
 
 // A lane exchange inside rows of 16 lanes that goes with the vector instruction, not through the LDS pipe.
@@ -245,13 +239,14 @@ __device__ __forceinline__ void pre_apply(const PreOp& p, int col, bool valid, f
 // Q (IS_K false): x = f32(q) * chmul[d].  K (IS_K true): x = (f32(k) - mean[d]) * chmul[d];
 // tokens that are masked or beyond N count for nothing and get code 0.
 // rowdot (Q only, may be null): <f32(q) * cmul, mean> per row.
-template <int D, int BLK, bool IS_K, int PRE, int NT>
+// HAVE: the threads have requested the block's rows before (have: as the loop below loads them).
+template <int D, int BLK, bool IS_K, int PRE, int NT, bool HAVE = false>
 __device__ __forceinline__ void quant_i8_block(
     int t, int h, int b, int tid, const uint16_t* __restrict__ x, int64_t sb, int64_t sh, int64_t sn,
     int N, int H, int64_t n_pad, const KeyMask& km, const float* __restrict__ mean,
     const float* __restrict__ chmul, float cmul,
     int8_t* __restrict__ codes, float* __restrict__ scales, float* __restrict__ rowdot, float* red,
-    const PreOp& pre) {
+    const PreOp& pre, const u32x4* have = nullptr) {
     constexpr int CPR = D / 8;                 // 16-byte chunks per row
     constexpr int NCH = BLK * CPR / NT;        // chunks per thread
     static_assert(BLK * CPR % NT == 0, "tile must split evenly over the threads");
@@ -264,9 +259,13 @@ __device__ __forceinline__ void quant_i8_block(
     u32x4 raw[NCH];
 #pragma unroll
     for (int i = 0; i < NCH; i++) {
-        const int row = r0 + (i * NT + tid) / CPR;
-        raw[i] = u32x4{0u, 0u, 0u, 0u};
-        if (row < N) raw[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)row * sn + col);
+        if constexpr (HAVE) {
+            raw[i] = have[i];
+        } else {
+            const int row = r0 + (i * NT + tid) / CPR;
+            raw[i] = u32x4{0u, 0u, 0u, 0u};
+            if (row < N) raw[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)row * sn + col);
+        }
     }
     float mul[8], mu[8];
     load8(chmul + col, mul);
@@ -441,9 +440,11 @@ __device__ __forceinline__ void kstats_group(
     const uint16_t* src = k + b * sb + h * sh + col0 + col;
     const int s0 = g * kGroup + leaf * kLeaf;
 
+    // (a group past the end: its waves only meet the barrier.  Whole waves are idle or not)
+    if (g >= 0) {
     u32x4 w[kLeaf];
     // every token of this leaf counts (no ragged end, no masked range inside it)
-    const bool all_kept = g >= 0 && s0 + kLeaf <= N && !(s0 < km.hi && s0 + kLeaf > km.lo);
+    const bool all_kept = s0 + kLeaf <= N && !(s0 < km.hi && s0 + kLeaf > km.lo);
     if (__all(all_kept)) {
 #pragma unroll
         for (int i = 0; i < kLeaf; i++) w[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)(s0 + i) * sn);
@@ -451,7 +452,7 @@ __device__ __forceinline__ void kstats_group(
 #pragma unroll
         for (int i = 0; i < kLeaf; i++) {
             w[i] = u32x4{0u, 0u, 0u, 0u};
-            if (g >= 0 && key_kept(s0 + i, N, km)) w[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)(s0 + i) * sn);
+            if (key_kept(s0 + i, N, km)) w[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)(s0 + i) * sn);
         }
     }
     double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -461,7 +462,7 @@ __device__ __forceinline__ void kstats_group(
     float inv[kLeaf], gain[8];
     constexpr int AHEAD = PRE == 2 ? 2 : 4;
     RopeTab<PRE> tab[AHEAD];
-    auto clamped = [&](int i) { return min(max(s0, 0) + i, N - 1); };
+    auto clamped = [&](int i) { return min(s0 + i, N - 1); };
     RopeAt rope{};
     if constexpr (PRE) {
         rope = rope_at<D>(pre, b, h, H, col);
@@ -480,7 +481,7 @@ __device__ __forceinline__ void kstats_group(
     for (int i = 0; i < kLeaf; i++) {
         float x[8];
         unpack8(w[i], x);
-        const bool kept = g >= 0 && key_kept(s0 + i, N, km);
+        const bool kept = key_kept(s0 + i, N, km);
         if constexpr (PRE) {
             pre_apply<D, PRE>(pre, col, kept, inv[i], gain, tab[i % AHEAD], x);
             if (i + AHEAD < kLeaf) rope_load<PRE>(rope, clamped(i + AHEAD), tab[i % AHEAD]);
@@ -513,6 +514,7 @@ __device__ __forceinline__ void kstats_group(
         sm.leafsum[leaf][at] = acc[e];
         sm.leafmin[leaf][at] = mn[e];
         sm.leafmax[leaf][at] = mx[e];
+    }
     }
     __syncthreads();
     gsum = 0.0;
@@ -1090,6 +1092,24 @@ __global__ __launch_bounds__(kShortThreads) void quant_short_kernel(QuantArgs a,
     const int nk_wg = (a.nk_blk + UNITS - 1) / UNITS, nq_wg = (a.nq_blk + UNITS - 1) / UNITS;
     if (r < nk_wg + nq_wg) {
         const int sub = tid / TPG, t = tid % TPG;
+        // (an odd count: the last workgroup's halves encode the same block)
+        const bool is_k = r < nk_wg;
+        const int blk = is_k ? min(r * UNITS + unit, a.nk_blk - 1) : min((r - nk_wg) * UNITS + unit, a.nq_blk - 1);
+        // The block's rows are requested ahead of the statistics where it has the size the one-shot call gives it.
+        constexpr int CPR = D / 8, RPC = 256 / CPR;           // rows per chunk of the half's threads
+        u32x4 rows[128 / RPC];
+        const int ahead = PRE == 0 && D <= 128 ? (is_k ? (a.blkk == 64 ? 64 : 0) : (a.blkq == 128 ? 128 : 0)) : 0;
+        if constexpr (PRE == 0 && D <= 128) {
+            const View& x = is_k ? a.k : a.q;
+            const int n = is_k ? a.Nkv : a.Nq;
+            const uint16_t* src = x.p + b * x.sb + h * x.sh + (utid % CPR) * 8;
+#pragma unroll
+            for (int i = 0; i < 128 / RPC; i++) {
+                const int row = blk * ahead + i * RPC + utid / CPR;
+                rows[i] = u32x4{0u, 0u, 0u, 0u};
+                if (i * RPC < ahead && row < n) rows[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)row * x.sn);
+            }
+        }
 #pragma unroll
         for (int w = 0; w < NWIN; w++) {
             double sum = 0.0;
@@ -1101,6 +1121,11 @@ __global__ __launch_bounds__(kShortThreads) void quant_short_kernel(QuantArgs a,
                     const int g = g0 + sub;
                     kstats_group<DK, PRE, D>(g < f.ngroups ? g : -1, h, b, t, a.k.p, a.k.sb, a.k.sh, a.k.sn, a.Nkv, a.H, a.km,
                                              sm.kg[sub], a.pre_k, w * DK, gsum, gmn, gmx);
+                    if (f.ngroups == 1) {                   // (nothing to exchange)
+                        if (tid < DK) { sum += gsum; mn = fminf(mn, gmn); mx = fmaxf(mx, gmx); }
+                        if (NWIN > 1) __syncthreads();      // (the next window's leaves)
+                        break;
+                    }
                     if (t < DK) { s_gsum[sub][t] = gsum; s_gmm[sub][t][0] = gmn; s_gmm[sub][t][1] = gmx; }
                     __syncthreads();
                     if (tid < DK) {
@@ -1128,24 +1153,22 @@ __global__ __launch_bounds__(kShortThreads) void quant_short_kernel(QuantArgs a,
             }
         }
         __syncthreads();
-        // (an odd count: the last workgroup's halves encode the same block)
-        if (r < nk_wg) {
-            const int blk = min(r * UNITS + unit, a.nk_blk - 1);
-#define SAGE_K(BLK) quant_i8_block<D, BLK, true, PRE, 256>(blk, h, b, utid, a.k.p, a.k.sb, a.k.sh, a.k.sn, a.Nkv, a.H, a.nkv_pad, a.km, \
-                                                       s_mean, s_kmul, 0.0f, a.k8, a.kscale, nullptr, sm.red[unit], a.pre_k)
-            if (a.blkk == 128) SAGE_K(128);
-            else if (a.blkk == 64) SAGE_K(64);
-            else SAGE_K(32);
-#undef SAGE_K
+#define SAGE_K(BLK, HAVE) quant_i8_block<D, BLK, true, PRE, 256, HAVE>(blk, h, b, utid, a.k.p, a.k.sb, a.k.sh, a.k.sn, a.Nkv, a.H, a.nkv_pad, a.km, \
+                                                       s_mean, s_kmul, 0.0f, a.k8, a.kscale, nullptr, sm.red[unit], a.pre_k, rows)
+#define SAGE_Q(BLK, HAVE) quant_i8_block<D, BLK, false, PRE, 256, HAVE>(blk, h, b, utid, a.q.p, a.q.sb, a.q.sh, a.q.sn, a.Nq, a.H, a.nq_pad, none, \
+                                                        s_mean, s_qmul, a.cmul, a.q8, a.qscale, a.rowdot, sm.red[unit], a.pre_q, rows)
+        constexpr bool HAVE = PRE == 0 && D <= 128;
+        if (is_k) {
+            if (a.blkk == 128) SAGE_K(128, false);
+            else if (a.blkk == 64) SAGE_K(64, HAVE);
+            else SAGE_K(32, false);
         } else {
-            const int blk = min((r - nk_wg) * UNITS + unit, a.nq_blk - 1);
-#define SAGE_Q(BLK) quant_i8_block<D, BLK, false, PRE, 256>(blk, h, b, utid, a.q.p, a.q.sb, a.q.sh, a.q.sn, a.Nq, a.H, a.nq_pad, none, \
-                                                        s_mean, s_qmul, a.cmul, a.q8, a.qscale, a.rowdot, sm.red[unit], a.pre_q)
-            if (a.blkq == 128) SAGE_Q(128);
-            else if (a.blkq == 64) SAGE_Q(64);
-            else SAGE_Q(32);
-#undef SAGE_Q
+            if (a.blkq == 128) SAGE_Q(128, HAVE);
+            else if (a.blkq == 64) SAGE_Q(64, false);
+            else SAGE_Q(32, false);
         }
+#undef SAGE_Q
+#undef SAGE_K
         return;
     }
     const int t = (r - nk_wg - nq_wg) * UNITS + unit;     // (the key padding makes the tile count even)
