@@ -568,11 +568,11 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         // Biased scores in the log2 domain, without the reference maximum.  (The bias of the accumulators is taken off
         // before the multiplication: exact, where folding it into the multiply-add's constant would cost the constant's
         // rounding.)
-        auto biased = [&](int kb, int i, float m) -> float {
-            return fmaf(__int_as_float(s[X][kb][i]) - Magic<D>::F, f[kb], m);
+        constexpr float kLog2e = 1.4426950408889634f;
+        auto biased = [&](int kb, int i, float bias_nat) -> float {
+            return fmaf(bias_nat, kLog2e, (__int_as_float(s[X][kb][i]) - Magic<D>::F) * f[kb]);
         };
         auto mv_at = [&](int i) -> float { return __uint_as_float(i & 1 ? mv[X][i >> 1] & 0xFFFF0000u : mv[X][i >> 1] << 16); };
-        constexpr float kLog2e = 1.4426950408889634f;
         float xs[SKB][ADDMASK && !BPIPE ? 16 : 1];
         if constexpr (ADDMASK && !BPIPE) {
 #pragma unroll
@@ -582,7 +582,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
                 for (int g = 0; g < 4; g++) {
                     const v4f w = BiasStage::get(lds_bias[wave], l32, half, g);
 #pragma unroll
-                    for (int e = 0; e < 4; e++) xs[kb][g * 4 + e] = fmaf(w[e], kLog2e, biased(kb, g * 4 + e, 0.0f));
+                    for (int e = 0; e < 4; e++) xs[kb][g * 4 + e] = biased(kb, g * 4 + e, w[e]);
                 }
             }
             bias_load(h + NBIAS, bias[X % NBIAS]);
@@ -608,7 +608,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
                 for (int kb = 0; kb < SKB; kb++)
 #pragma unroll
                     for (int i = 0; i < 16; i++) {
-                        if constexpr (BPIPE) mt = fmaxf(mt, fmaf(mv_at(i), kLog2e, biased(kb, i, 0.0f)));
+                        if constexpr (BPIPE) mt = fmaxf(mt, biased(kb, i, mv_at(i)));
                         else mt = fmaxf(mt, xs[kb][i]);
                     }
             } else
@@ -690,7 +690,9 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
             }
             const int kb = k >> 3, i = (2 * k) & 15;
             if (r < 2) {
-                if constexpr (BPIPE) ea[k][r] = fmaf(mv_at(i + r), kLog2e, biased(kb, i + r, -m_used));
+                // (the reference is taken off the rounded sum, which its maximum was taken of: with a bias of -1e9 the sum's
+                // rounding is 64, and an argument that has it not is past what fp16 holds)
+                if constexpr (BPIPE) ea[k][r] = biased(kb, i + r, mv_at(i + r)) - (m_used - Lazy<VARIANT>::log2_pscale);
                 else if constexpr (ADDMASK) ea[k][r] = xs[kb][i + r] - (m_used - Lazy<VARIANT>::log2_pscale);
                 else ea[k][r] = fmaf(__int_as_float(s[X][kb][i + r]), f[kb], c0[kb]);
             } else if (r < 4) {

@@ -48,3 +48,37 @@ def test_bias_rows(oracle, form, variant, D, Sq, Skv, gap):
     assert np.isfinite(got).all()
     cos, mx = G.cos_maxabs(got, want)
     assert mx <= 2e-2 and cos >= 0.9999, (cos, mx)            # (the bars of every O test: one bf16 step at |O| ~ 4)
+
+
+@pytest.mark.parametrize("form", [-1, 4])
+@pytest.mark.parametrize("variant,D,value", [(0, 128, -1e9), (0, 128, -2e38), (0, 64, -1e9), (0, 64, -1e30), (0, 256, -1e9), (1, 128, -1e9), (1, 64, -1e30)])
+def test_bias_beyond_the_scores_precision(oracle, form, variant, D, value):
+    """Whole steps of keys, and whole rows, at a bias whose rounding is larger than any score: such keys weigh nothing
+    where a row has others, and are alike where it has none."""
+    import torch
+    import gpu_harness as G
+    S = 290
+    w = WORKLOADS[1 if D == 64 else 2].scaled(B=1, H=2, S=S, D=D)
+    q, k, v = make_inputs(w)
+    bias = np.zeros((w.B, w.H, S, S), np.float32)
+    bias[:, 0, :, :130] = value                              # the first steps
+    bias[:, 1, :, 70:] = value                               # the later ones
+    bias[:, :, 40:75] = value                                # rows with nothing else
+    bias = f32_to_bf16_bits(bias)
+    qd, kd, vd, md = (G.dev_bf16(x) for x in (q, k, v, bias))
+    o = torch.zeros_like(qd)
+    L = _lib.lib()
+    qs, ms = _lib.strides_bhnd(S, w.H, D), (ctypes.c_int64 * 4)(w.H * S * S, S * S, S, 1)
+    assert L.mi355_sage_set_attn_short(form) == 0
+    try:
+        rc = L.mi355_sage_sdpa_bf16_mask_any(qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), md.data_ptr(), o.data_ptr(), w.B, w.H, S, S, D,
+                                             w.scale, qs, qs, qs, ms, qs, 0, 0, 0, 0, 0, G.stream(), variant, None, 0)
+        torch.cuda.synchronize()
+    finally:
+        L.mi355_sage_set_attn_short(0)
+    assert rc == 0, rc
+    _, want = oracle.sdpa_bf16(q, k, v, w.scale, variant=variant, blkq=128 if variant == 0 else 32, blkk=64, addmask=bf16_bits_to_f32(bias))
+    got = o.float().cpu().numpy()
+    assert np.isfinite(got).all()
+    cos, mx = G.cos_maxabs(got, want)
+    assert mx <= 2e-2 and cos >= 0.9999, (cos, mx)            # (the bars of every O test: one bf16 step at |O| ~ 4)
