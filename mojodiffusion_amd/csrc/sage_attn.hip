@@ -773,7 +773,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
             // latencies to itself.  The further a wave is on its way to the next barrier, the lower its priority: the
             // two then arrive together.  (Clocks per 64-key tile, e4m3 / fp16 at 128 channels: 2330 / 2250 with all copies
             // behind the barrier and no priorities; 2226 / 2171 with the priorities; 2076 / 2087 with the copies moved, too;
-            // 1950 / 2120 without any barrier.  Two levels, or one for the P.V instructions: 2215, 2227.  The chip gives a
+            // 1950 / 2120 without any barrier; 1843 for e4m3 with the shorter search for a maximum above.  Two levels, or one for the P.V instructions: 2215, 2227.  The chip gives a
             // part back as a lower clock: one-shot [1,16896,24,128] e4m3 2098 -> 1975 us, [1,4608,24,64] e4m3 162 -> 143,
             // [1,4608,24,128] fp16 225 -> 221, [2,4352,30,128] fp16 473 -> 464.)
             if constexpr (NW == 8) {
