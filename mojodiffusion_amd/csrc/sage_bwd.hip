@@ -32,6 +32,7 @@
 //   [2,1248,30,128]  launch 1 25.8 -> 9.6, launch 2 231 -> 204 (best 218 -> 185)
 //   [1,4608,24,128]  launch 1 31.2 -> 11.7, launch 2 969 -> 864
 //   [1,2304,12,64]   launch 1 8.1 -> 4.9, launch 2 75.9 -> 72.5
+#include "sage_grid.h"
 #include "sage_internal.h"
 #include <type_traits>
 
@@ -229,7 +230,7 @@ struct PassLds {
 };
 
 template <int D, int PASS>
-__device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, uint8_t* smem, int block) {
+__device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, uint8_t* smem, int bh, int xt) {
     using L = PassLds<D, PASS>;
     constexpr int NW = 8;
     constexpr int XROWS = NW * 32;                  // owner rows per workgroup
@@ -245,9 +246,6 @@ __device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, uint8_t* smem, i
     const int Nx = PASS == 0 ? a.Nq : a.Nkv;
     const int valid_x = PASS == 0 ? a.valid_q : a.valid_kv;
     const int valid_y = PASS == 0 ? a.valid_kv : a.valid_q;
-    const int x_tiles = (Nx + XROWS - 1) / XROWS;
-    const int xt = block % x_tiles;
-    const int bh = block / x_tiles;
     const int b = bh / a.H, h = bh % a.H;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -750,50 +748,41 @@ __device__ __forceinline__ void dkdv_role(const BwdArgs& a, uint8_t* smem, int b
 }
 
 template <int D>
-__device__ __forceinline__ void bwd_dkdv_body(const BwdArgs& a, uint8_t* smem, int block) {
-    const int x_tiles = (a.Nkv + 127) / 128;
-    const int xt = block % x_tiles, bh = block / x_tiles;
+__device__ __forceinline__ void bwd_dkdv_body(const BwdArgs& a, uint8_t* smem, int bh, int xt) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     if (wave < 4) dkdv_role<D, 0>(a, smem, bh, xt, wave, lane);
     else dkdv_role<D, 1>(a, smem, bh, xt, wave, lane);
 }
 
-// Workgroup j of n of a kind -> the block it works on: consecutive ids go to the 8 XCDs in turn, and each XCD takes a
-// contiguous range of blocks, so that the blocks of a head, which all walk the same rows, share one L2.  (Launch 1 + 2,
-// us, blocks in the order of ids -> so: [2,1248,30,128] 196.7 -> 191.8, [2,2001,40,64] 310.8 -> 304.6, level where a
-// few heads are all there is.)
-__device__ __forceinline__ int xcd_block(int j, int n) {
-    const int per = n >> 3, extra = n & 7, xcd = j & 7;
-    return xcd * per + min(xcd, extra) + (j >> 3);
-}
+// keys of a dK/dV workgroup: 128 (wave pairs) or 256 (single-wave form, which fits two waves per SIMD at 64 channels)
+template <int D> constexpr int kKeysWg = D > 64 ? 128 : 256;
 
-// One grid for both: the first n_dq workgroups are the dQ pass (the longer ones first), the rest
-// the dK/dV pass.  Both take a whole CU (8 waves, most of the LDS); in one grid the second
-// kind starts on a CU as soon as the first kind runs out, instead of after its last workgroup.
+// One grid for both: first the dQ pass (the longer ones first), then the dK/dV pass.  Both take a whole CU (8 waves,
+// most of the LDS); in one grid the second kind starts on a CU as soon as the first kind runs out, instead of after its
+// last workgroup.  (Which block a workgroup takes: bwd_block.  Launch 1 + 2, us, blocks in the order of ids -> in ranges
+// over the XCDs: [2,1248,30,128] 196.7 -> 191.8, [2,2001,40,64] 310.8 -> 304.6, level where a few heads are all there is.)
 template <int D>
-__global__ __launch_bounds__(512, 2) void bwd_fused_kernel(BwdArgs a, int n_dq) {
-    constexpr bool PAIRED = D > 64;                 // below, the single-wave form already fits two waves per SIMD
+__global__ __launch_bounds__(512, 2) void bwd_fused_kernel(BwdArgs a) {
+    constexpr bool PAIRED = D > 64;
     constexpr int KV_BYTES = PAIRED ? DkDvLds<D>::BYTES : PassLds<D, 1>::BYTES;
     constexpr int BYTES = KV_BYTES > PassLds<D, 0>::BYTES ? KV_BYTES : PassLds<D, 0>::BYTES;
     __shared__ __attribute__((aligned(1024))) uint8_t smem[BYTES];
-    const int block = (int)blockIdx.x;
-    const int n_kv = (int)gridDim.x - n_dq;
-    if (block < n_dq) bwd_pass_body<D, 0>(a, smem, xcd_block(block, n_dq));
-    else if constexpr (PAIRED) bwd_dkdv_body<D>(a, smem, xcd_block(block - n_dq, n_kv));
-    else bwd_pass_body<D, 1>(a, smem, xcd_block(block - n_dq, n_kv));
+    constexpr int KW = kKeysWg<D>;
+    const BwdBlock w = bwd_block((int)blockIdx.x, a.B * a.H, (a.Nq + 255) / 256, (a.valid_q + 255) / 256, (a.Nkv + KW - 1) / KW, (a.valid_kv + KW - 1) / KW);
+    if (!w.dkdv) bwd_pass_body<D, 0>(a, smem, w.head, w.tile);
+    else if constexpr (PAIRED) bwd_dkdv_body<D>(a, smem, w.head, w.tile);
+    else bwd_pass_body<D, 1>(a, smem, w.head, w.tile);
 }
 
 template <int D>
 static hipError_t launch_bwd_d(const BwdArgs& a, hipStream_t st) {
     const int64_t bh = (int64_t)a.B * a.H;
     const int64_t prep = bh * (a.nq_pad / 64 + 1);
-    // dQ: 256 query rows per workgroup; dK, dV: 128 keys (wave pairs) or 256 keys (single-wave form)
-    constexpr int KEYS_WG = D > 64 ? 128 : 256;
-    const int64_t gq = bh * ((a.Nq + 255) / 256), gk = bh * ((a.Nkv + KEYS_WG - 1) / KEYS_WG);
+    const int64_t gq = bh * ((a.Nq + 255) / 256), gk = bh * ((a.Nkv + kKeysWg<D> - 1) / kKeysWg<D>);
     if (prep > 0x7FFFFFFF || gq + gk > 0x7FFFFFFF) return hipErrorInvalidValue;
     hipLaunchKernelGGL((bwd_prep_kernel<D>), dim3((unsigned)prep), dim3(256), 0, st, a);
-    hipLaunchKernelGGL((bwd_fused_kernel<D>), dim3((unsigned)(gq + gk)), dim3(512), 0, st, a, (int)gq);
+    hipLaunchKernelGGL((bwd_fused_kernel<D>), dim3((unsigned)(gq + gk)), dim3(512), 0, st, a);
     return hipGetLastError();
 }
 

@@ -497,3 +497,13 @@ def test_recorded_sdpa_node_backpropagates():
     assert qb.grad.dtype == torch.bfloat16 and vb.grad.shape == vb.shape
     with pytest.raises(A.Error, match="sdpa_nomask: q/k/v dtype mismatch"):
         A.record_sdpa(qb, kb.float(), vb, scale)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("H,Sq,Skv,rq,rk", [(3, 700, 900, 200, 130), (8, 600, 520, 256, 1), (5, 257, 1100, 257, 600), (1, 520, 257, 1, 256)])
+def test_bwd_whole_blocks_of_padding(oracle, H, Sq, Skv, rq, rk, D):
+    """Workgroups whose rows are all padding, with heads that do and do not divide over the 8 XCDs: every block is taken."""
+    outs, want = _run_case(oracle, 1, Sq, Skv, H, D, float(1.0 / np.sqrt(D)), seed=300 + Sq, real_q=rq, real_kv=rk)
+    for name, got, ref, n in zip(("dQ", "dK", "dV"), outs, want, (rq, rk, rk)):
+        _check(name, got, ref)
+        assert not got[:, n:].float().abs().sum().item(), name
