@@ -132,6 +132,7 @@ __device__ __forceinline__ void row_put(uint8_t* os, int l32, int half, int d, i
 template <int D>
 __device__ __forceinline__ void rows_out(const uint8_t* os, uint16_t* head, int64_t sn, int row0, int n, int lane) {
     constexpr int CPR = D / 8, RPI = 64 / CPR;
+    asm volatile("" : "+v"(lane));      // (the row numbers of rows_in are formed again, not kept across the loop in between)
     uint16_t* op = head + (lane % CPR) * 8;
 #pragma unroll
     for (int i = 0; i < 32 / RPI; i++) {
