@@ -18,6 +18,7 @@
 // kernel's operand bytes per query row, which is why attn_short_rule stops where the main kernel's
 // workgroups start to fill the chip.
 #include "sage_attn_common.h"
+#include "sage_grid.h"
 
 #include <algorithm>
 #include <atomic>
@@ -27,7 +28,8 @@ namespace sage {
 template <int D> constexpr int kMainRows = D > 128 ? 128 : 256;               // rows per workgroup of the main kernel
 template <int D> constexpr int short_waves() { return D > 128 ? 4 : 8; }      // 256 channels: a wave needs a SIMD's registers
 
-// (64 channels, fp16: two workgroups share a compute unit, which takes 128 registers at most)
+// (64 channels, fp16: two workgroups share a compute unit, which takes 128 registers at most.  Under a bias that is 10 %
+// of a call whose workgroups are more than the compute units: [1,700,24,64] 31.1 us at 146 registers, 27.7 at 128.)
 template <int D, int VARIANT, int KW, bool QF, bool ADDMASK>
 __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 : 1) void sage_attn_short_kernel(AttnArgs a, int n_rtiles, int item0, int total_wg) {
     constexpr int NW = short_waves<D>();
@@ -59,9 +61,7 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
     __shared__ __attribute__((aligned(16))) float lds_qmax[8];
 
     // each XCD takes a contiguous range of workgroups, so that those sharing a head share its L2
-    const int bid = blockIdx.x;
-    const int per = total_wg >> 3, extra = total_wg & 7, xcd = bid & 7;
-    const int wg = xcd * per + min(xcd, extra) + (bid >> 3);
+    const int wg = xcd_item((int)blockIdx.x, total_wg);
     // item0 > 0: the main kernel has done the items (row tiles of kMainRows) below it; n_rtiles counts those
     // tiles then, and consecutive workgroups take the pieces of one
     constexpr int PIECES = kMainRows<D> / ROWS;
@@ -230,9 +230,17 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
     BiasStage::Rows brows{};
     if (ADDMASK) brows = BiasStage::rows(a.amask + b * a.amb + h * a.amh, a.amn, row0, a.Nq - 1, lane);
     auto bias_load = [&](int hs) {
+        BiasStage::Rows rows = brows;
+        if constexpr (D == 64 && VARIANT == 0) {
+            // (one pointer of the two is formed for each step, behind an empty statement: both, kept over the loop, are one
+            // register too many)
+            int first = row0;
+            asm volatile("" : "+s"(first));
+            rows.p[1] = BiasStage::rows(a.amask + b * a.amb + h * a.amh, a.amn, first, a.Nq - 1, lane).p[1];
+        }
 #pragma unroll
         for (int kb = 0; kb < SKB; kb++)
-            bias[kb].load(brows, key_step(min(hs, h1 - 1)) * SK + kb * 32, kv_valid, lane);
+            bias[kb].load(rows, key_step(min(hs, h1 - 1)) * SK + kb * 32, kv_valid, lane);
     };
     if (ADDMASK && h0 < h1) bias_load(h0);
 
