@@ -35,13 +35,24 @@
 namespace sage {
 
 // ADDMASK: an additive score bias (natural-log units, bf16, logical [B,H,Nq,Nkv] through element
-// strides with the key stride 1) is added to the dequantised scores.  What bounds it is the way of the bias: from HBM
-// (two steps of 32 keys ahead of its use), through LDS into the scores' layout (half a step ahead), so that neither
-// latency stands in front of a step.  The fp16 variant takes its steps optimistically, like the plain forward; the
-// e4m3 variant looks for every step's maximum on the biased scores.  The bias's ordinary loads share the vector-memory
-// counter with the tile copies; that makes the waits at the midpoint longer, never shorter.  (One-shot, us, one step
-// ahead, turned and searched for its maximum in front of each step -> now: [1,1153,24,128] 68.8 -> 61.2,
-// [1,2304,24,128] 109.5 -> 99.5, [1,1700,24,128] 92.4 -> 82.7, [1,700,24,64] 33.6 -> 30.6.  Four steps ahead: 67.)
+// strides with the key stride 1) is added to the dequantised scores.  What bounds it is the way of the bias, from HBM and
+// through LDS into the scores' layout.
+//
+// fp16 variant up to 128 channels, one workgroup per item (BPIPE): the bias is requested two steps of 32 keys ahead and
+// turned half a step ahead, so that neither latency stands in front of a step, and the steps are taken optimistically, like
+// the plain forward's.  (One-shot, us, one step ahead, turned and searched for its maximum in front of each step -> so:
+// [1,1153,24,128] 68.8 -> 61.2, [1,2304,24,128] 109.5 -> 99.5, [1,1700,24,128] 92.4 -> 82.7, [1,700,24,64] 33.6 -> 30.6.
+// Four steps ahead: 67.)  That rests on a row's biased scores not rising by more than 2^12 within 32 keys as a rule.  Where
+// they do, the softmax of the step is done twice: [1,2304,24,128] with a bias of -0.5 per key of distance 117 -> 133,
+// -0.1 per key 116 -> 119, heads with slopes of 2^(-8 h / H) 120 -> 135, 0.5 N(0, 1) 120 -> 107, a third of the keys at
+// -1e4 112 -> 103.  (Looking first behind a step that was done twice: 126, 134, 134, 108, 105.)
+//
+// The other instantiations turn the bias and look for the maximum on the biased scores in front of every step: e4m3 in
+// steps of 64 keys, requested two steps ahead at 64 channels and one at 128; 256 channels and the split schedule in steps
+// of their variant, one ahead.
+//
+// The bias's ordinary loads share the vector-memory counter with the tile copies; that makes the waits at the midpoint
+// longer, never shorter.
 
 // Workgroups of the split schedule that gave up on a hand-over (see the kernel's fold-in part).
 static __device__ unsigned int g_split_faults;
@@ -297,7 +308,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     float l_run = 0.0f;            // fp16 variant: this lane's share of the row sum
     // e4m3 variant: the row sum is taken over the ROUNDED probabilities, on the matrix pipe — one
     // more product per tile against a tile of ones (as e2m1, where 1.0 = 0x2 and a tile takes four registers
-    // instead of eight) gives every lane the sum over all 64 keys of its query, in every accumulator element;
+    // instead of eight, which with the words of p that are written in place takes ten moves per tile out) gives every lane the sum over all 64 keys of its query, in every accumulator element;
     // element 0 is the one that is kept to scale.  It is rescaled together with the output accumulators.
     v16f lacc;
 #pragma unroll
@@ -633,10 +644,12 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         };
         if constexpr (VARIANT == 1 && TRIP && !ADDMASK) {
             // The main loop asks the largest exponent argument against the reference as it stands, without the other half's
-            // maximum and without the arithmetic of a new reference: 20 vector instructions less of 148 (one of them an
-            // exponential) in most steps.  (No look at all, and a look at the packed codes for one that is full, took 16
-            // more and was slower: a wave has some row in 32 that rises in a good part of the steps, and the step again
-            // costs all its exponentials.  [1,4608,24,128] 200 -> 217 us, [1,4608,24,64] 143 -> 166.)
+            // maximum and without the arithmetic of a new reference: 110 vector instructions instead of 129 in the trip's
+            // code, one of them an exponential, in most steps.  (No look at all, and a look at the packed codes for one that
+            // is full, took 16 more out and was slower: a wave has some row in 32 that rises in a good part of the steps, and
+            // the step again costs all its exponentials.  [1,4608,24,128] 200 -> 217 us, [1,4608,24,64] 143 -> 166.)  The
+            // argument that is compared is the rounded one that is used; next to the limit that can decide otherwise than the
+            // comparison of maximum and reference in `decide`, so a probability can be rounded against another reference.
             constants();
             float top = fmaf(__int_as_float(block_max(0)), f[0], c0[0]);
 #pragma unroll
@@ -763,8 +776,10 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
                 }
             }
             // (the main loop stops early enough that these tiles exist; their addresses are the trip's base plus a
-            // constant.  Behind the barrier by two and five slots: all waves' copies at once right behind it wait for
-            // each other at the vector memory path, and a wave that waits there issues nothing else)
+            // constant.  Behind the barrier, K by two slots and V^T by five at 128 channels, both by two at 64, which has six
+            // slots in all: all waves' copies at once right behind it wait for each other at the vector memory path, and a
+            // wave that waits there issues nothing else)
+            static_assert(NM / 2 - 1 < NM / 2 + 1 && NM / 2 + 1 <= NM - 2, "copies go out behind the barrier of their tile");
             if constexpr (TRIP && SUB == 0) {
                 if (m == NM / 2 + 1) dma_k_at(kg_trip + (dt + KOFF + LEAD) * K_BYTES, slot_kcopy);
                 if (m == NM - 2) dma_v_at(vg_trip + (dt + LEAD) * V_BYTES, slot_vcopy);
@@ -773,9 +788,10 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
             // latencies to itself.  The further a wave is on its way to the next barrier, the lower its priority: the
             // two then arrive together.  (Clocks per 64-key tile, e4m3 / fp16 at 128 channels: 2330 / 2250 with all copies
             // behind the barrier and no priorities; 2226 / 2171 with the priorities; 2076 / 2087 with the copies moved, too;
-            // 1950 / 2120 without any barrier; 1843 for e4m3 with the shorter search for a maximum above.  Two levels, or one for the P.V instructions: 2215, 2227.  The chip gives a
-            // part back as a lower clock: one-shot [1,16896,24,128] e4m3 2098 -> 1975 us, [1,4608,24,64] e4m3 162 -> 143,
-            // [1,4608,24,128] fp16 225 -> 221, [2,4352,30,128] fp16 473 -> 464.)
+            // 1950 / 2120 without any barrier; 1843 for e4m3 with the shorter search for a maximum above.  Two levels, or
+            // one for the P.V instructions: 2215, 2227.  The chip gives a part back as a lower clock: one-shot
+            // [1,16896,24,128] e4m3 2098 -> 1975 us, [1,4608,24,64] e4m3 162 -> 143, [1,4608,24,128] fp16 225 -> 221,
+            // [2,4352,30,128] fp16 473 -> 464.)
             if constexpr (NW == 8) {
                 constexpr int SLOTS = NM * SPT;             // from one barrier to the next
                 const int past = (SUB * NM + m - (NM / 2 - 1) + SLOTS) % SLOTS, level = 3 - past * 4 / SLOTS;

@@ -253,6 +253,7 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
     for (int i = 0; i < 16; i++) lacc[i] = 0.0f;
     float m_used = -3.0e38f, l_run = 0.0f;              // (finite: a step whose keys are all masked yields p = 0, not NaN)
     const v16i smagic = magic_splat<D>();
+    // (e4m3 1.0 = 0x38.  As e2m1, like the main kernel's, they would take four registers less; that was measured there only.)
     const v8i ones8 = {0x38383838, 0x38383838, 0x38383838, 0x38383838, 0x38383838, 0x38383838, 0x38383838, 0x38383838};
 
     for (int hs = h0; hs < h1; hs++) {
@@ -463,22 +464,26 @@ hipError_t launch_attn_short(const AttnArgs& a, hipStream_t st) {
 // Which form, from what each costs on an MI355X: time = base + rounds (r + s steps) + fill (f + g steps) in
 // microseconds, with rounds = workgroups / compute units rounded up, fill = workgroups / compute units, steps = key tiles (main
 // kernel) or key steps of the longest run (short form); the split schedule: base + per balanced key tile.
-// The coefficients are fitted to 350 to 400 launches of the kernel and 230 one-shot calls per head dim and variant
-// (2 to 480 heads, 32 to 16384 queries, 16 to 32768 keys): choosing by them costs 0.05 to 0.9 % over always choosing
-// right.  (A fit that ended at 4096 keys, carried on to longer ones, gave whole problems of 64 channels with e4m3 P.V
-// to the short form, which moves 8 times the operand bytes: [1,16384,12,64] 970 us, now 708.)  Measured at
-// [1,256,30,128] 16.7 -> 10.0 us, [1,1024,8,64] 20.2 -> 9.5, [1,1024,8,128] 28.0 -> 13.9, [1,512,24,128] 21.3 -> 12.8;
-// whatever the key count, the main kernel's form is back ahead at 75 (128 channels, fp16) to 190 (64, e4m3) workgroups
-// of 256 rows, 110 to 140 of 128 rows at 256 channels.
+// The coefficients were fitted to 350 to 400 launches of the kernel and 230 one-shot calls per head dim and variant
+// (2 to 480 heads, 32 to 16384 queries, 16 to 32768 keys), of earlier forms of both kernels, of which both have become
+// faster since.  With the kernels as they are, choosing by them costs 0.2 to 0.9 % on average over the best of the forms
+// taken for everything (70 one-shot calls drawn per head dim and variant, 2 to 240 heads, 64 to 4096 queries): 20 of 420
+// over 2 %, the worst 10 %, [1,75,22,128] 17.5 us instead of 15.9.  There is no term for a bias: with one 0.2 to 2.5 % (30
+// calls each), the worst 22 % ([1,73,35,128] 19.5 instead of 16.1).  (A fit that ended at 4096 keys, carried on to longer
+// ones, gave whole problems of 64 channels with e4m3 P.V to the short form, which moves 8 times the operand bytes:
+// [1,16384,12,64] 929 us, the main kernel 614.)  One-shot, main kernel -> short form: [1,256,30,128] 19.2 -> 17.1 us,
+// [1,1024,8,64] 24.6 -> 17.2, [1,1024,8,128] 30.6 -> 22.2, [1,512,24,128] 24.1 -> 22.3.  The main kernel is back ahead
+// between 64 and 75 workgroups of 256 rows (128 rows at 256 channels) with fp16 P.V, at 64 channels and 2048 keys between 90
+// and 110; with e4m3 the two are level from 75 on at 512 keys, and it is back ahead between 125 and 140 at 2048.
 //
 // A problem of some rounds and a bit more takes both: the main kernel does the full rounds and the short
 // form what is left, spread over the whole chip, instead of one more round that is nearly empty (264 items
-// of 32 key tiles, 128 channels: 84 -> 66 us; of 64 channels 61 -> 43).
+// of 32 key tiles, 128 channels: 84 -> 66 us; of 64 channels 61 -> 43; by earlier forms of both).
 // The split schedule, which balances the same problems by handing partial results over in memory, is ahead of both where
 // the second of few rounds is a quarter to a half full and the key sequence is long: a sixth (64 channels) and a
-// thirteenth (128) of the 788 shapes of its rule that were timed, among them one-shot [1,4352 x 8192,19,128] 344 -> 315 us
-// and [1,4352 x 8192,19,64] 225 -> 205 (323 row tiles), [1,12288,7,128] 477 -> 444; where it is taken it never cost
-// more than 0.5 %.
+// thirteenth (128) of the 788 shapes of its rule that were timed (with earlier forms of the kernels, where it was taken it
+// never cost more than 0.5 %); one-shot, main kernel alone -> split: [1,4352 x 8192,19,128] 335 -> 312 us and
+// [1,4352 x 8192,19,64] 230 -> 196 (323 row tiles), [1,12288,7,128] 457 -> 433.
 struct FormCost {
     float base, r, s, f, g;
     float of(int64_t wgs, int64_t steps, int units) const {
@@ -500,9 +505,9 @@ static const float kSplitCost[2][2] = {{17.0f, 0.96f}, {25.0f, 1.53f}};       //
 
 // Microseconds a call takes more with the main kernel where its Q cannot go to the encoders for next to nothing:
 // many queries on few keys, which keep Q in the kernel's prologue, and a K that takes one launch alone but not with Q.
-// One-shot, main kernel against short form: [1,510 x 139,24,128] 22.2 against 20.4, [1,256 x 292,40,128] 26.2 against 23.7,
-// e4m3 [2,71 x 45,32,256] 38.2 against 31.6; with as many keys as queries the main kernel is ahead, [1,64,24,128] 16.1
-// against 17.6.  (64 channels: nothing to gain, or the second kind's fit is as good without.)
+// One-shot, main kernel against short form: [1,510 x 139,24,128] 20.8 against 19.0, [1,256 x 292,40,128] 25.0 against 22.3,
+// e4m3 [2,71 x 45,32,256] 36.3 against 28.8; with as many keys as queries they are level, [1,64,24,128] 15.2 against 15.2
+// to 16.0.  (64 channels: nothing to gain, or the second kind's fit is as good without.)
 static const float kQCost[3][2][2] = {{{0.0f, 0.0f}, {0.8f, 0.0f}}, {{1.4f, 1.4f}, {0.0f, 0.0f}}, {{0.0f, 2.0f}, {0.0f, 2.0f}}};
 
 namespace {
