@@ -230,6 +230,8 @@ def test_reference_maximum_keeps_rising(oracle, variant):
     than the kernel's lazy-refresh margin: every path that repairs a stale reference
     maximum (refresh + accumulator rescale, redo of an optimistic tile) is exercised, in
     interior tiles, repeatedly.  The second case puts one huge key in the middle.
+    (At this size the short form takes the call, and an e4m3 wave of the main kernel would take none of these steps
+    through its main loop; tests/test_gpu_attn_rising.py has that loop.)
 
     Nearly every row here is dominated by one or two keys, and the scores are ~25 times larger
     than on real inputs.  Both variants stay inside the 2e-2 bar on every element: for the e4m3
