@@ -1,7 +1,7 @@
 """Rows whose maximum rises along the keys, in the main kernel's main loop (test_reference_maximum_keeps_rising has rises
 so steep, on a problem so short, that the short form and the loop's careful bodies take it): the optimistic steps that
 are done again (fp16), the reference that is raised inside a trip (e4m3), and the rescaled accumulators, sums and Stats.
-What the inputs make happen is counted on the host, from the checker's own codes and scales."""
+What the inputs make happen is counted on the host, from the oracle's codes and scales."""
 import numpy as np
 import pytest
 
