@@ -78,7 +78,6 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     float* __restrict__ stats, int n_qtiles, int total_wg,
     const uint16_t* __restrict__ amask, int64_t amb, int64_t amh, int64_t amn,
     int split_groups, float* split_part, int* split_flags, int split_wait) {
-    constexpr int KS_OFF = D > 128 ? 0 : VARIANT == 0 ? 3 : 2;        // see lds_ks
     constexpr int VB = (VARIANT == 0) ? 2 : 1;          // bytes per V element
     constexpr int KSTEPS = D / 32;                      // int8 MFMA steps over the head dim
     constexpr int DB = D / 32;                          // 32-channel output blocks
@@ -92,11 +91,12 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     constexpr int K_NCH = K_BYTES / 1024, V_NCH = V_BYTES / 1024;      // 1 KiB copies per tile
     constexpr int K_CH = (K_NCH + NW - 1) / NW;         // copies per wave (short tiles: some waves repeat a copy)
     constexpr int V_CH = (V_NCH + NW - 1) / NW;
-    constexpr int LEAD = D > 128 ? 1 : 2;               // tile copies run this many iterations ahead (LDS: 160 KiB)
+    // Tile copies run this many iterations ahead (LDS: 160 KiB, of which a tile of 256 channels takes 48 with fp16 V).
+    constexpr int LEAD = D > 128 && VARIANT == 0 ? 1 : 2;
     // ring depths: the tile in use, LEAD tiles published or in flight, and the slot the next copy
     // goes to — for K the tile whose scores are being computed is t+1, for V^T the tile in use is t-1.
-    // (Up to 128 channels that is four slots each, so slot numbers are a mask away.)
     constexpr int NSK = LEAD + 2, NSV = LEAD + 2;
+    constexpr int KS_OFF = D > 128 && ADDMASK ? 0 : LEAD == 1 ? 1 : VARIANT == 0 ? 3 : 2;      // see lds_ks
     constexpr int K_CPR = D / 16;                       // chunks per K row
     constexpr int V_CPR = kTileKV * VB / 16;            // chunks per V^T row
     constexpr int VROW = kTileKV * VB;                  // bytes per V^T row
@@ -111,7 +111,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
 
     __shared__ __attribute__((aligned(1024))) uint8_t lds_k[NSK][K_BYTES];
     __shared__ __attribute__((aligned(1024))) uint8_t lds_v[NSV][V_BYTES];
-    __shared__ __attribute__((aligned(16))) float lds_ks[max_keys(D) / 32 + (D > 128 ? 0 : 4)];
+    __shared__ __attribute__((aligned(16))) float lds_ks[max_keys(D) / 32 + (KS_OFF > 0 ? 4 : 0)];
     __shared__ __attribute__((aligned(16))) uint8_t lds_bias[ADDMASK ? NW : 1][ADDMASK ? BiasStage::BYTES : 16];
     __shared__ float lds_qmax[QF ? 8 : 1];              // QF: largest |pre-scaled q| of each wave's 32 rows
     __shared__ __attribute__((aligned(16))) uint8_t lds_qc[QF && VARIANT == 1 ? NW * 32 * D : 16];      // QF: Q codes on their way into fragments
@@ -207,6 +207,13 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         for (int s = 0; s < KSTEPS; s++) qf[s] = *reinterpret_cast<const v4i*>(qp + s * 32);
         sq = qscale[bh * (nq_pad / blkq) + qrow / blkq] * kMagicUnit;
     }
+    if constexpr (D > 128) {
+        // 300 registers are in use, of which vector instructions reach 256: the rest (accumulation registers) is for what
+        // only matrix instructions read.  Left to the compiler it was scores and addresses, 53 moves per tile of 64 keys,
+        // now 5 ([1,4608,18,256] 358 -> 347 us).
+#pragma unroll
+        for (int s = 0; s < KSTEPS; s++) asm volatile("" : "+a"(qf[s]));
+    }
     // QF: the wave's 32 rows, 16 bytes per lane and whole rows per instruction (rows past N_q as zeros), and
     // the multipliers of the lane's eight channels
     constexpr int Q_CPR = D / 8, Q_RPI = 64 / Q_CPR, Q_NI = QF ? 32 / Q_RPI : 1;     // chunks per row, rows per load, loads
@@ -236,7 +243,8 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     const float* ksc = kscale + bh * (nkv_pad / blkk);
     const int ush = blkk == 32 ? 0 : (blkk == 64 ? 1 : 2);      // log2(32-key blocks per scale block)
     // (staged per 32-key block, KS_OFF entries in: the main loop fetches the eight entries of one trip
-    // with two 16-byte reads, and its first entry then sits on a 16-byte boundary)
+    // with two 16-byte reads, the six of a trip over three slots with three of 8, and its first entry then sits
+    // on such a boundary)
     for (int i = tid; i < (int)(nkv_pad / 32); i += THREADS) lds_ks[KS_OFF + i] = ksc[i >> ush];
     auto kscale_of = [&](int u32blk) -> float { return lds_ks[KS_OFF + u32blk]; };
 
@@ -315,6 +323,11 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     for (int i = 0; i < 16; i++) lacc[i] = 0.0f;
     const v8i ones4 = {0x22222222, 0x22222222, 0x22222222, 0x22222222, 0, 0, 0, 0};
 
+    // At 256 channels the wave has its SIMD to itself, and what bounds it is the number of instructions it issues, 4.4
+    // clocks each with nobody to fill in: 743 per tile of 64 keys before it took the trips with constant slots below, 299
+    // now.  One-shot, us, fp16 / e4m3: [1,4608,18,256] 419 -> 347 / 403 -> 317, [1,1153,18,256] 60.3 -> 52.6 / 80.3 -> 68.7.
+    // (Two waves per SIMD, each with half of the output channels and all scores: 404 / 420 and 55.0 / 74.3.)
+    //
     // The main loop advances in STEPS of SK keys: 32 for the fp16 variant (one P.V matrix
     // instruction covers 16 keys), 64 for the e4m3 variant (its matrix instruction covers 64).  A
     // 64-key tile in LDS holds SPT = 64 / SK steps.  Step h is NM matrix-instruction slots: the
@@ -338,7 +351,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     constexpr int PWS = PW / SPT;                       // dwords of packed P per step
     constexpr int PDS = 2;      // operand fragments are requested this many slots ahead
     constexpr int KOFF = SPT == 1 ? 2 : 1;              // the barrier of tile t publishes K(t + KOFF) and V(t)
-    constexpr int PERIOD = 4 * SPT;                     // steps after which ring slots and parity repeat
+    constexpr int PERIOD = NSK * SPT;                   // steps after which ring slots and parity repeat
     // GRP == 3: the operands of three slots are requested together, three to five slots ahead and in
     // reverse order, so that the first of the three matrix instructions waits for the request made
     // last — LDS answers in order — and the other two need no wait instruction at all.
@@ -529,7 +542,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     // HT >= 0: h modulo 4 * SPT as a compile-time number (both rings have four slots then), so that
     // every ring slot and key block below is a constant and the LDS addresses are register + immediate.
     // HT < 0: h is known at run time only, but for its position in the tile, -1 - HT.
-    float kst[8];       // K scales of the eight 32-key blocks of one trip of the main loop
+    float kst[PERIOD * SKB];        // K scales of the 32-key blocks of one trip of the main loop
     const uint8_t *kg_trip = kg, *vg_trip = vg;          // K and V^T tile of the trip's first step
     auto step = [&](int h, auto x_tag, auto h_tag, auto first_tag, auto qk_tag) {
         constexpr int X = decltype(x_tag)::value;            // h & 1: selects the score / probability buffers
@@ -538,7 +551,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         constexpr bool DOQK = decltype(qk_tag)::value;       // false in the last step
         constexpr bool TRIP = HT >= 0 && !FIRST;             // a step of the main loop: no masked keys, scales in kst
         constexpr bool OPT = VARIANT == 0 && !FIRST && (!ADDMASK || BPIPE);
-        static_assert(HT < 0 || (NSK == 4 && NSV == 4), "constant slots need four-slot rings");
+        static_assert(HT < 0 || (NSK == NSV && PERIOD % 2 == 0), "constant slots need rings of one depth");
         constexpr int SUB = HT >= 0 ? HT % SPT : -1 - HT;    // step within its tile
         static_assert(SUB >= 0 && SUB < SPT, "position in the tile");
         static_assert((SPT == 1 || X == SUB) && (HT < 0 || X == (HT & 1)), "parity of the step");
@@ -546,12 +559,12 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         // tiles: score operands of step h+1, and of step h+2 (requested at the end of this step);
         // V^T of step h-1, and of step h
         const int tq = (h + 1) / SPT, tq2 = (h + 2) / SPT, tv = (h + SPT - 1) / SPT - 1, tv2 = h / SPT;
-        const int slot_kq = HT >= 0 ? ((HT + 1) / SPT) & 3 : tq % NSK, slot_kq2 = HT >= 0 ? ((HT + 2) / SPT) & 3 : tq2 % NSK;
-        const int slot_vp = HT >= 0 ? ((HT + 4 * SPT - 1) / SPT) & 3 : (tv + NSV) % NSV, slot_vp2 = HT >= 0 ? (HT / SPT) & 3 : tv2 % NSV;
+        const int slot_kq = HT >= 0 ? ((HT + 1) / SPT) % NSK : tq % NSK, slot_kq2 = HT >= 0 ? ((HT + 2) / SPT) % NSK : tq2 % NSK;
+        const int slot_vp = HT >= 0 ? ((HT + NSV * SPT - 1) / SPT) % NSV : (tv + NSV) % NSV, slot_vp2 = HT >= 0 ? (HT / SPT) % NSV : tv2 % NSV;
         constexpr int kbq = (SUB + 1) % SPT, kbq2 = SUB % SPT;            // key block of the scores (fp16 variant)
         constexpr int subv = (SUB + SPT - 1) % SPT, subv2 = SUB;          // step of the V^T tile
-        const int slot_kcopy = HT >= 0 ? (HT / SPT + KOFF + LEAD) & 3 : (t + KOFF + LEAD) % NSK;
-        const int slot_vcopy = HT >= 0 ? (HT / SPT + LEAD) & 3 : (t + LEAD) % NSV;
+        const int slot_kcopy = HT >= 0 ? (HT / SPT + KOFF + LEAD) % NSK : (t + KOFF + LEAD) % NSK;
+        const int slot_vcopy = HT >= 0 ? (HT / SPT + LEAD) % NSV : (t + LEAD) % NSV;
 
         float f[SKB], c0[SKB];
         const int hk = TRIP ? 0 : key_step(h);
@@ -831,7 +844,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     int hs = 1;
     // (the split instantiations sit at the register limit and keep their slots in registers; so do the
     // ones with an additive mask, whose time goes into reading the mask anyway)
-    if constexpr (NSK == 4 && NSV == 4 && !SPLIT && !ADDMASK) {
+    if constexpr (!SPLIT && !ADDMASK) {
         step(0, X0{}, std::integral_constant<int, 0>{}, T{}, T{});
         // The main loop takes the steps whose keys all count without looking for masked keys: those in front
         // of the masked range or the ragged end, then — the steps that touch the range, at most a few, go
@@ -854,18 +867,26 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
             kg_trip = kg + (int64_t)(hs / SPT + past) * K_BYTES;
             vg_trip = vg + (int64_t)(hs / SPT + past) * V_BYTES;
             {
-                const v4f* kp = reinterpret_cast<const v4f*>(&lds_ks[KS_OFF + (t_off + past) * 2 + hs * SKB]);
-                const v4f k0 = kp[0], k1 = kp[1];
-                kst[0] = k0.x; kst[1] = k0.y; kst[2] = k0.z; kst[3] = k0.w;
-                kst[4] = k1.x; kst[5] = k1.y; kst[6] = k1.z; kst[7] = k1.w;
+                typedef float kvec __attribute__((ext_vector_type(PERIOD * SKB == 8 ? 4 : 2)));
+                constexpr int KV = sizeof(kvec) / sizeof(float);
+                const kvec* kp = reinterpret_cast<const kvec*>(&lds_ks[KS_OFF + (t_off + past) * 2 + hs * SKB]);
+#pragma unroll
+                for (int i = 0; i < PERIOD * SKB; i += KV) {
+                    const kvec k = kp[i / KV];
+#pragma unroll
+                    for (int e = 0; e < KV; e++) kst[i + e] = k[e];
+                }
             }
             step(hs, X1{}, std::integral_constant<int, 1 % PERIOD>{}, F{}, T{});
             step(hs + 1, X0{}, std::integral_constant<int, 2 % PERIOD>{}, F{}, T{});
             step(hs + 2, X1{}, std::integral_constant<int, 3 % PERIOD>{}, F{}, T{});
             step(hs + 3, X0{}, std::integral_constant<int, 4 % PERIOD>{}, F{}, T{});
-            if constexpr (PERIOD == 8) {
+            static_assert(PERIOD == 4 || PERIOD == 6 || PERIOD == 8, "steps of a trip");
+            if constexpr (PERIOD >= 6) {
                 step(hs + 4, X1{}, std::integral_constant<int, 5>{}, F{}, T{});
-                step(hs + 5, X0{}, std::integral_constant<int, 6>{}, F{}, T{});
+                step(hs + 5, X0{}, std::integral_constant<int, 6 % PERIOD>{}, F{}, T{});
+            }
+            if constexpr (PERIOD == 8) {
                 step(hs + 6, X1{}, std::integral_constant<int, 7>{}, F{}, T{});
                 step(hs + 7, X0{}, std::integral_constant<int, 0>{}, F{}, T{});
             }

@@ -466,7 +466,7 @@ hipError_t launch_attn_short(const AttnArgs& a, hipStream_t st) {
 // kernel) or key steps of the longest run (short form); the split schedule: base + per balanced key tile.
 // The coefficients were fitted to 350 to 400 launches of the kernel and 230 one-shot calls per head dim and variant
 // (2 to 480 heads, 32 to 16384 queries, 16 to 32768 keys), of earlier forms of both kernels, of which both have become
-// faster since.  With the kernels as they are, choosing by them costs 0.2 to 0.9 % on average over the best of the forms
+// faster since (the main kernel's cost per tile at 256 channels is of the present one).  With the kernels as they are, choosing by them costs 0.2 to 0.9 % on average over the best of the forms
 // taken for everything (70 one-shot calls drawn per head dim and variant, 2 to 240 heads, 64 to 4096 queries): 20 of 420
 // over 2 %, the worst 10 %, [1,75,22,128] 17.5 us instead of 15.9.  There is no term for a bias: with one 0.2 to 2.5 % (30
 // calls each), the worst 22 % ([1,73,35,128] 19.5 instead of 16.1).  (A fit that ended at 4096 keys, carried on to longer
@@ -496,8 +496,8 @@ static const FormCost kCost[3][2][3] = {        // [64, 128, 256 channels][varia
      {{1.91f, 3.27f, 0.76f, 1.13f, 0.06f}, {3.02f, 1.61f, 1.08f, 1.28f, 0.00f}, {2.55f, 1.40f, 1.20f, 1.06f, 0.00f}}},
     {{{1.29f, 3.84f, 0.75f, 0.88f, 0.54f}, {2.68f, 3.27f, 0.92f, 0.05f, 0.42f}, {2.56f, 3.24f, 0.95f, 0.04f, 0.36f}},
      {{2.15f, 4.92f, 0.95f, 1.71f, 0.11f}, {2.52f, 4.17f, 1.20f, 0.18f, 0.30f}, {2.54f, 3.25f, 1.40f, 0.75f, 0.14f}}},
-    {{{1.44f, 4.16f, 1.36f, 2.31f, 0.26f}, {2.87f, 6.05f, 1.29f, 0.20f, 0.25f}, {}},
-     {{3.61f, 4.01f, 1.64f, 2.79f, 0.00f}, {1.45f, 5.06f, 2.57f, 1.45f, 0.00f}, {}}},
+    {{{1.44f, 4.16f, 0.90f, 2.31f, 0.44f}, {2.87f, 6.05f, 1.29f, 0.20f, 0.25f}, {}},
+     {{3.61f, 4.01f, 1.09f, 2.79f, 0.10f}, {1.45f, 5.06f, 2.57f, 1.45f, 0.00f}, {}}},
 };
 // (fp16 at 64 channels past 3072 keys: no one set meets both ends there)
 static const FormCost kCost64Long[3] = {{1.81f, 2.54f, 0.66f, 0.34f, 0.16f}, {3.60f, 0.70f, 0.78f, 0.00f, 0.06f}, {3.72f, 0.77f, 0.55f, 0.03f, 0.18f}};
