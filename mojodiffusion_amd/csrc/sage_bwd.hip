@@ -9,12 +9,12 @@
 // Two launches:
 //   1. bwd_prep_kernel     -Delta and Stats * log2(e) per query row (padding rows: +inf, so their
 //                          probabilities vanish); and a vector c close to the mean key.
-//   2. bwd_fused_kernel    one grid of two kinds of 8-wave workgroups, the longer kind first:
-//        dQ     owner = 256 query rows, loop over key tiles, as scale * (dS K - rowsum(dS) c)
+//   2. bwd_fused_kernel    one grid of two kinds of 8-wave workgroups (4-wave at head dim 64), the longer kind first:
+//        dQ     owner = 256 (128) query rows, loop over key tiles, as scale * (dS K - rowsum(dS) c)
 //               = scale * dS (K - c)                                          (bwd_pass_body<D,0>)
 //        dK,dV  owner = 128 keys, loop over query tiles; pairs of waves share 32 keys, one wave
 //               carrying P and dV, the other dS and dK                        (bwd_dkdv_body)
-//               (head dim 64: 256 keys, every wave both products — bwd_pass_body<D,1>)
+//               (head dim 64: every wave both products of 32 keys — bwd_pass_body<D,1>)
 // In both kinds a wave owns 32 rows ("x"), keeps their bf16 row blocks resident as B operands
 // and walks the other side ("y") in tiles of 64 rows staged in LDS by register-bypassing copies,
 // a ring of three slots, one barrier per tile.  A 32x32 block of scores T[y,x] lands in the accumulator
@@ -220,20 +220,28 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(BwdArgs a) {
 // Launch 2, the form in which one wave carries every product of its 32 owner rows: the dQ
 // workgroups (PASS 0), and the dK/dV workgroups at head dim 64 (PASS 1).
 // ---------------------------------------------------------------------------------------------
+// Waves per workgroup.  At 64 channels four waves' ring is 50 KiB and two workgroups share a compute unit: the waves of a
+// SIMD then meet no common barrier, so that one's matrix instructions run beside the other's exponentials, and a
+// grid that does not fill the chip leaves less of it idle.  Both launches, us, eight waves -> four: [2,1248,30,64] 86.5 ->
+// 78.2, [1,2304,12,64] 74.4 -> 71.6, [1,4608,24,64] 459 -> 454, [1,700,16,64] 19.6 -> 15.2.  (At 128 channels that form
+// takes tiles of 32 rows and twice the copies: 11 % fewer clocks at [2,1248,30,128], which the chip, at its power limit,
+// turns into a lower clock: 176.4 us against 174.4.)
+template <int D> constexpr int kBwdWaves = D > 64 ? 8 : 4;
+
 template <int D, int PASS>
 struct PassLds {
     static constexpr int TILE_BYTES = 64 * D * 2, SLOT = 2 * TILE_BYTES, SLOTS = 3;
     static constexpr int ROW_BYTES = PASS == 1 ? 2048 : 0;                   // [slot][lse | -Delta][64], PASS 1 only
     // The ring, and during the prologue the owner rows (2 x 32 rows per wave) behind its first slot.
     static constexpr int OWNER = ROW_BYTES + SLOT;
-    static constexpr int BYTES = OWNER + 8 * 2 * 64 * D;
-    static_assert(BYTES >= ROW_BYTES + SLOTS * SLOT, "the ring must fit");
+    static constexpr int RING_END = ROW_BYTES + SLOTS * SLOT, OWNER_END = OWNER + kBwdWaves<D> * 2 * 64 * D;
+    static constexpr int BYTES = RING_END > OWNER_END ? RING_END : OWNER_END;
 };
 
 template <int D, int PASS>
 __device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, uint8_t* smem, int bh, int xt) {
     using L = PassLds<D, PASS>;
-    constexpr int NW = 8;
+    constexpr int NW = kBwdWaves<D>;
     constexpr int XROWS = NW * 32;                  // owner rows per workgroup
     constexpr int CPR = D / 8;                      // 16-byte chunks per row
     constexpr int TILE_BYTES = L::TILE_BYTES;
@@ -756,21 +764,22 @@ __device__ __forceinline__ void bwd_dkdv_body(const BwdArgs& a, uint8_t* smem, i
     else dkdv_role<D, 1>(a, smem, bh, xt, wave, lane);
 }
 
-// keys of a dK/dV workgroup: 128 (wave pairs) or 256 (single-wave form, which fits two waves per SIMD at 64 channels)
-template <int D> constexpr int kKeysWg = D > 64 ? 128 : 256;
+// keys of a dK/dV workgroup (wave pairs at 128 channels, every wave 32 keys of its own at 64), rows of a dQ workgroup
+constexpr int kKeysWg = 128;
+template <int D> constexpr int kRowsWg = kBwdWaves<D> * 32;
+static_assert(kBwdWaves<128> * 16 == kKeysWg && kBwdWaves<64> * 32 == kKeysWg, "keys of the waves");
 
-// One grid for both: first the dQ pass (the longer ones first), then the dK/dV pass.  Both take a whole CU (8 waves,
-// most of the LDS); in one grid the second kind starts on a CU as soon as the first kind runs out, instead of after its
-// last workgroup.  (Which block a workgroup takes: bwd_block.  Launch 1 + 2, us, blocks in the order of ids -> in ranges
+// One grid for both: first the dQ pass (the longer ones first), then the dK/dV pass.  In one grid the second kind starts
+// on a CU as soon as the first kind runs out, instead of after its last workgroup.  (Which block a workgroup takes: bwd_block.  Launch 1 + 2, us, blocks in the order of ids -> in ranges
 // over the XCDs: [2,1248,30,128] 196.7 -> 191.8, [2,2001,40,64] 310.8 -> 304.6, level where a few heads are all there is.)
 template <int D>
-__global__ __launch_bounds__(512, 2) void bwd_fused_kernel(BwdArgs a) {
+__global__ __launch_bounds__(kBwdWaves<D> * 64, 2) void bwd_fused_kernel(BwdArgs a) {
     constexpr bool PAIRED = D > 64;
     constexpr int KV_BYTES = PAIRED ? DkDvLds<D>::BYTES : PassLds<D, 1>::BYTES;
     constexpr int BYTES = KV_BYTES > PassLds<D, 0>::BYTES ? KV_BYTES : PassLds<D, 0>::BYTES;
     __shared__ __attribute__((aligned(1024))) uint8_t smem[BYTES];
-    constexpr int KW = kKeysWg<D>;
-    const BwdBlock w = bwd_block((int)blockIdx.x, a.B * a.H, (a.Nq + 255) / 256, (a.valid_q + 255) / 256, (a.Nkv + KW - 1) / KW, (a.valid_kv + KW - 1) / KW);
+    constexpr int RW = kRowsWg<D>, KW = kKeysWg;
+    const BwdBlock w = bwd_block((int)blockIdx.x, a.B * a.H, (a.Nq + RW - 1) / RW, (a.valid_q + RW - 1) / RW, (a.Nkv + KW - 1) / KW, (a.valid_kv + KW - 1) / KW);
     if (!w.dkdv) bwd_pass_body<D, 0>(a, smem, w.head, w.tile);
     else if constexpr (PAIRED) bwd_dkdv_body<D>(a, smem, w.head, w.tile);
     else bwd_pass_body<D, 1>(a, smem, w.head, w.tile);
@@ -780,10 +789,10 @@ template <int D>
 static hipError_t launch_bwd_d(const BwdArgs& a, hipStream_t st) {
     const int64_t bh = (int64_t)a.B * a.H;
     const int64_t prep = bh * (a.nq_pad / 64 + 1);
-    const int64_t gq = bh * ((a.Nq + 255) / 256), gk = bh * ((a.Nkv + kKeysWg<D> - 1) / kKeysWg<D>);
+    const int64_t gq = bh * ((a.Nq + kRowsWg<D> - 1) / kRowsWg<D>), gk = bh * ((a.Nkv + kKeysWg - 1) / kKeysWg);
     if (prep > 0x7FFFFFFF || gq + gk > 0x7FFFFFFF) return hipErrorInvalidValue;
     hipLaunchKernelGGL((bwd_prep_kernel<D>), dim3((unsigned)prep), dim3(256), 0, st, a);
-    hipLaunchKernelGGL((bwd_fused_kernel<D>), dim3((unsigned)(gq + gk)), dim3(512), 0, st, a);
+    hipLaunchKernelGGL((bwd_fused_kernel<D>), dim3((unsigned)(gq + gk)), dim3(kBwdWaves<D> * 64), 0, st, a);
     return hipGetLastError();
 }
 
