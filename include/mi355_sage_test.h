@@ -32,12 +32,14 @@ int mi355_sage_attn_split_rule(int B, int H, int N_q, int N_kv, int D, int varia
 
 /* The short form of the attention kernel (32 or 64 query rows per workgroup, keys split over its
  * waves).  mode 0: by shape (default); -1: never; 8 or 4: always, with that many key runs per row
- * block (head dim 256: always 4).  4 and 8 take precedence over the switch above, which otherwise keeps
- * the short form out when it is set.  Returns 0, or -1 for
+ * block (head dim 256: always 4); 2: the two-run form of the main kernel instead (128 rows, the keys split over two halves
+ * of the waves), where it exists (not at head dim 256, under a bias with e4m3, or past 32768 keys).  2, 4 and 8 take
+ * precedence over the switch above, which otherwise keeps the short and the two-run form out when it is set.  Returns 0, or -1 for
  * a mode outside these. */
 int mi355_sage_set_attn_short(int mode);
 
-/* Key runs the short form would use for this shape by the rule alone, 0 for the 256-row workgroups. */
+/* Key runs the short form would use for this shape where the choice is between it and the 256-row workgroups alone, 0 for
+ * the latter. */
 int mi355_sage_attn_short_rule(int B, int H, int N_q, int N_kv, int D, int variant);
 
 /* Row tiles (256 rows of a head; 128 at head dim 256) the main kernel would do for this shape on the current

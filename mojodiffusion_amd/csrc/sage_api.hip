@@ -353,7 +353,7 @@ int sdpa_impl(const void* Q, const void* K, const void* V, void* O, void* Stats,
     }
     // (one decision for carving and launching; slots the caller's workspace was not sized for — a
     // forced schedule of the test switch — come from the library's per-stream buffer)
-    const AttnPlan plan = attn_plan(B, H, N_q, kv, D, variant, causal != 0);
+    const AttnPlan plan = attn_plan(B, H, N_q, kv, D, variant, causal != 0, mask.add != nullptr);
     // The plain forward leaves Q to the attention kernel, which encodes its own rows (same codes and
     // scales): the quantize stage then neither reads Q nor writes its codes.
     // Not where the encoders have room for it and a prologue is on the path of the whole call — the main kernel does
@@ -368,8 +368,10 @@ int sdpa_impl(const void* Q, const void* K, const void* V, void* O, void* Stats,
     // workgroup per compute unit, with Q ([1,2048 x 512,32,64] 23.7 -> 30.4, e4m3 [1,512,24,128] 21.5 -> 25.6).
     auto one_launch = [&](bool with_q) { return quant_short_workgroups(B, H, N_q, kv, D, blkq, blkk, with_q); };
     const int units = compute_units();
-    const bool room = variant == MI355_SAGE_PV_FP8 ? (plan.short_kw > 0 || plan.main_items * 8 <= units * 5) && (int64_t)N_q * 64 <= (int64_t)4096 * D
-                                                   : plan.main_items > 0 && plan.short_kw == 0 && plan.main_items < units;
+    // (row tiles of the main kernel's loop in one round or less; of both its forms together where it takes more)
+    const int64_t loop_items = plan.two_runs && plan.main_items == 0 ? (int64_t)B * H * ((N_q + kTileQ - 1) / kTileQ) : plan.main_items;
+    const bool room = variant == MI355_SAGE_PV_FP8 ? (plan.short_kw > 0 || loop_items * 8 <= units * 5) && (int64_t)N_q * 64 <= (int64_t)4096 * D
+                                                   : loop_items > 0 && plan.short_kw == 0 && loop_items < units;
     bool q_in_encoders = room && N_q <= 2 * N_kv;
     if (q_in_encoders && one_launch(false) > 0) {
         const int64_t wgs = one_launch(true);
@@ -422,6 +424,7 @@ int sdpa_impl(const void* Q, const void* K, const void* V, void* O, void* Stats,
     }
     a.main_items = plan.main_items;
     a.short_kw = plan.short_kw;
+    a.two_runs = plan.two_runs;
     a.split_wgs = plan.split_wgs;
     if (a.split_wgs > 0) {
         if (attn_split_bytes(a.split_wgs, D) <= attn_split_bytes(attn_split_rule(B, H, N_q, kv, D, variant), D)) a.split = ws + c.split;
@@ -781,7 +784,7 @@ int mi355_sage_attn_fwd(const void* q8, const void* qscale, int blkq, const void
     // Same scheduling, hence the same bits, as the one-shot calls: shapes that are split over a
     // fixed number of workgroups need hand-over slots, kept per (device, stream) by the library.
     const AttnPlan plan = attn_plan(B, H, N_q, kv_valid, D, variant, false);
-    a.main_items = plan.main_items; a.short_kw = plan.short_kw; a.split_wgs = plan.split_wgs;
+    a.main_items = plan.main_items; a.short_kw = plan.short_kw; a.split_wgs = plan.split_wgs; a.two_runs = plan.two_runs;
     std::lock_guard<std::mutex> together(launch_mutex(static_cast<hipStream_t>(stream)));
     const size_t split_bytes = attn_split_bytes(a.split_wgs, D);
     if (split_bytes > 0 && (rc = internal_workspace(g_split_ws, split_bytes, static_cast<hipStream_t>(stream), &a.split))) return rc;
@@ -806,7 +809,7 @@ int mi355_sage_attn_fwd_q16(const void* Q, const int64_t* q_strides, int64_t q_o
     AttnArgs a{};
     const AttnPlan plan = attn_plan(B, H, N_q, kv_valid, D, variant, false);
     if (plan.main_items > 0 && attn_split_workgroups(B, H, N_q, kv_valid, D, variant) > 0) return MI355_SAGE_EUNSUPPORTED;
-    a.main_items = plan.main_items; a.short_kw = plan.short_kw;
+    a.main_items = plan.main_items; a.short_kw = plan.short_kw; a.two_runs = plan.two_runs;
     const View q = make_view(Q, q_strides, q_off);
     a.q_src = q.p; a.qsb = q.sb; a.qsh = q.sh; a.qsn = q.sn; a.qmul = static_cast<const float*>(qmul); a.blkq = blkq;
     a.k8 = static_cast<const int8_t*>(k8); a.kscale = static_cast<const float*>(kscale); a.blkk = blkk;
@@ -835,7 +838,7 @@ int mi355_sage_set_attn_split(int mode) {
 }
 
 int mi355_sage_set_attn_short(int mode) {
-    if (mode != -1 && mode != 0 && mode != 4 && mode != 8) return MI355_SAGE_EINVAL;
+    if (mode != -1 && mode != 0 && mode != 2 && mode != 4 && mode != 8) return MI355_SAGE_EINVAL;
     attn_short_override(mode);
     return MI355_SAGE_OK;
 }

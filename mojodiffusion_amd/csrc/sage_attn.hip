@@ -66,7 +66,9 @@ static __device__ unsigned int g_split_faults;
 // the range costs the ones that have none registers and addresses in their last steps (one-shot call, us with it -> without,
 // no range masked: e4m3 [1,2304,18,256] 187.0 -> 179.6, cross [1,3840 x 333,32,128] 50.4 -> 47.9; fp16 [2,4352,30,128] 476.2
 // -> 473.9, [1,2304,18,256] 165.0 -> 162.8).
-template <int D, int VARIANT, bool STATS, bool ADDMASK, bool SPLIT, bool RANGE = false, bool QF = false>
+// KW 2: the two halves of a workgroup's waves split the KEYS of 128 query rows and merge their results at the end (the
+// two-run form, see attn_plan).
+template <int D, int VARIANT, bool STATS, bool ADDMASK, bool SPLIT, bool RANGE = false, bool QF = false, int KW = 1>
 __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     const int8_t* __restrict__ q8, const float* __restrict__ qscale, int blkq,
     const uint16_t* __restrict__ q_src, int64_t qsb, int64_t qsh, int64_t qsn, const float* __restrict__ qmul,
@@ -75,19 +77,24 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     const float* __restrict__ qshift,
     int H, int Nq, int kv_valid_all, int mask_lo, int mask_hi, int causal, int64_t nq_pad, int64_t nkv_pad,
     uint16_t* __restrict__ o, int64_t osb, int64_t osh, int64_t osn,
-    float* __restrict__ stats, int n_qtiles, int total_wg,
+    float* __restrict__ stats, int n_qtiles, int first_item, int total_wg,
     const uint16_t* __restrict__ amask, int64_t amb, int64_t amh, int64_t amn,
     int split_groups, float* split_part, int* split_flags, int split_wait) {
     constexpr int VB = (VARIANT == 0) ? 2 : 1;          // bytes per V element
     constexpr int KSTEPS = D / 32;                      // int8 MFMA steps over the head dim
     constexpr int DB = D / 32;                          // 32-channel output blocks
-    constexpr int K_BYTES = kTileKV * D;                // K tile
-    constexpr int V_BYTES = D * kTileKV * VB;           // V^T tile
+    constexpr int SK = VARIANT == 0 ? 32 : 64;          // keys per step (see below)
+    // Keys of a tile: 64, and with two runs as many as the waves take in one step, wave group kw the part from kw * SK on.
+    constexpr int TK = KW == 1 ? kTileKV : KW * SK;
+    static_assert(KW == 1 || (KW == 2 && D <= 128 && !SPLIT), "two runs: whole items, up to 128 channels");
+    constexpr int K_BYTES = TK * D;                     // K tile
+    constexpr int V_BYTES = D * TK * VB;                // V^T tile (two runs of e4m3: two tiles of the layout, one behind the other)
     // 256 channels: the output accumulators alone take 128 registers per lane, so a wave gets a SIMD
     // to itself (up to 512 registers) and a workgroup is 4 waves = 128 query rows.
     constexpr int NW = D > 128 ? 4 : 8;                 // waves per workgroup
     constexpr int THREADS = NW * 64;
-    constexpr int ROWS_WG = NW * 32;                    // query rows per workgroup
+    constexpr int RG = NW / KW;                         // 32-row groups of a workgroup
+    constexpr int ROWS_WG = RG * 32;                    // query rows per workgroup
     constexpr int K_NCH = K_BYTES / 1024, V_NCH = V_BYTES / 1024;      // 1 KiB copies per tile
     constexpr int K_CH = (K_NCH + NW - 1) / NW;         // copies per wave (short tiles: some waves repeat a copy)
     constexpr int V_CH = (V_NCH + NW - 1) / NW;
@@ -100,21 +107,21 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     constexpr int K_CPR = D / 16;                       // chunks per K row
     constexpr int V_CPR = kTileKV * VB / 16;            // chunks per V^T row
     constexpr int VROW = kTileKV * VB;                  // bytes per V^T row
-    constexpr int JS = VARIANT == 0 ? 4 : 1;            // PV steps over the 64 keys of a tile
-    constexpr int NUNIT = JS * DB;                      // PV matrix instructions per tile
+    constexpr int JS = VARIANT == 0 ? 4 / KW : 1;       // PV steps over a wave's keys of a tile
+    constexpr int NUNIT = JS * DB;                      // PV matrix instructions per tile and wave
     constexpr int EPU = 32 / NUNIT;                     // scores exponentiated per PV instruction
     constexpr int FPU = VARIANT == 0 ? 1 : 2;           // 16-byte V fragments per PV instruction
     constexpr int PD = VARIANT == 0 ? 2 : 1;            // V fragment prefetch distance (units)
-    constexpr int PW = VARIANT == 0 ? 16 : 8;           // dwords of packed P per tile
+    constexpr int PW = VARIANT == 0 ? 16 / KW : 8;      // dwords of packed P per tile and wave
     constexpr bool BPIPE = ADDMASK && VARIANT == 0 && D <= 128 && !SPLIT;      // see ADDMASK
     static_assert(32 % NUNIT == 0 && (EPU % 2 == 0 || EPU == 1), "unit split");
 
     __shared__ __attribute__((aligned(1024))) uint8_t lds_k[NSK][K_BYTES];
     __shared__ __attribute__((aligned(1024))) uint8_t lds_v[NSV][V_BYTES];
-    __shared__ __attribute__((aligned(16))) float lds_ks[max_keys(D) / 32 + (KS_OFF > 0 ? 4 : 0)];
+    __shared__ __attribute__((aligned(16))) float lds_ks[(KW == 1 ? max_keys(D) : kTwoRunKeys) / 32 + (KS_OFF > 0 ? 4 : 0)];
     __shared__ __attribute__((aligned(16))) uint8_t lds_bias[ADDMASK ? NW : 1][ADDMASK ? BiasStage::BYTES : 16];
     __shared__ float lds_qmax[QF ? 8 : 1];              // QF: largest |pre-scaled q| of each wave's 32 rows
-    __shared__ __attribute__((aligned(16))) uint8_t lds_qc[QF && VARIANT == 1 ? NW * 32 * D : 16];      // QF: Q codes on their way into fragments
+    __shared__ __attribute__((aligned(16))) uint8_t lds_qc[QF && VARIANT == 1 ? RG * 32 * D : 16];      // QF: Q codes on their way into fragments
     static_assert(!(STATS && ADDMASK), "no entry point asks for Stats under an additive mask");
     static_assert(!RANGE || (!ADDMASK && !SPLIT), "no entry point masks a range under an additive mask; the split schedule tests every step");
     constexpr bool MASKED = RANGE || SPLIT;             // mask_lo .. mask_hi may hold keys (otherwise the launcher has seen that it does not)
@@ -139,7 +146,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     const int xcd_full = total_wg - (items_per - 1) * 8;        // XCDs that own `items_per` items (1..8)
     const int n_items = xcd < xcd_full ? items_per : items_per - 1;
     const int item0 = xcd < xcd_full ? xcd * items_per : xcd_full * items_per + (xcd - xcd_full) * (items_per - 1);
-    const int ntiles_item = (kv_valid_all + kTileKV - 1) / kTileKV;
+    const int ntiles_item = (kv_valid_all + TK - 1) / TK;
     // (the launcher has checked that steps x workgroups stays inside 32 bits)
     const uint32_t xcd_steps = (uint32_t)n_items * (uint32_t)ntiles_item;
     auto span_lo = [&](int j) -> int {
@@ -168,8 +175,9 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     const int item_local = SPLIT ? (int)((uint32_t)(span_end - 1) / (uint32_t)ntiles_div) : wg_j;
     const int item_base = item_local * ntiles_item;
     const int t_off = SPLIT ? max(span_begin, item_base) - item_base : 0;
-    const int wg = item0 + item_local;
+    const int wg = first_item + item0 + item_local;
     const int qt = (int)((uint32_t)wg % (uint32_t)qtiles_div);
+    if (KW > 1 && qt * ROWS_WG >= Nq) return;           // (behind the main kernel's row tiles: the second half of a short last one)
     // Causal (query i sees keys j <= i, cuDNN's top-left alignment): the keys past this workgroup's last
     // row are masked for every one of its rows — they are treated as the ragged end, so their tiles are
     // never copied — and the steps on a wave's diagonal mask key > row element by element (below).
@@ -178,10 +186,10 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     // t, or t + skip from skip_at on.  (An even number of them: the K scales of a trip are read 16 bytes at a time.)
     int skip_at = 0, skip = 0;
     if (RANGE && !causal) {
-        skip_at = (mask_lo + kTileKV - 1) / kTileKV;
-        skip = max(min(mask_hi, kv_valid) / kTileKV - skip_at, 0) & ~1;
+        skip_at = (mask_lo + TK - 1) / TK;
+        skip = max(min(mask_hi, kv_valid) / TK - skip_at, 0) & ~1;
     }
-    const int ntiles = SPLIT ? span_end - item_base - t_off : (kv_valid + kTileKV - 1) / kTileKV - skip;
+    const int ntiles = SPLIT ? span_end - item_base - t_off : (kv_valid + TK - 1) / TK - skip;
     auto key_tile = [&](int t) -> int { return !RANGE || t < skip_at ? t : t + skip; };
     const bool seg_finishes = !SPLIT || t_off + ntiles == ntiles_item;   // holds the item's last key tile: writes the output
     span_end = item_base + t_off;
@@ -193,9 +201,9 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     int lane = tid & 63;
     if constexpr (SPLIT) asm volatile("" : "+v"(lane));
     const int l32 = lane & 31, half = lane >> 5;
-    const int row_in_tile = wave * 32 + l32;
-    const int qrow = qt * ROWS_WG + row_in_tile;        // this lane's query (padded index)
-    const int wave_row0 = qt * ROWS_WG + wave * 32;     // the wave's first query (the same for all its lanes)
+    const int rg = KW == 1 ? wave : wave % RG, kw = KW == 1 ? 0 : wave / RG;       // row group, key run
+    const int wave_row0 = qt * ROWS_WG + rg * 32;       // the wave's first query (the same for all its lanes)
+    const int qrow = wave_row0 + l32;                   // this lane's query (padded index)
     if constexpr (SPLIT) __syncthreads();               // every wave has left the previous segment's LDS
 
     // Q^T fragments: 16 bytes of the head dim per step, resident for the whole kernel.
@@ -260,13 +268,13 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     // where the compiler, left to fold the bases itself, re-forms addresses past 65 535 in the loop)
     uint32_t koff[KSTEPS], voff[JS * FPU];
 #pragma unroll
-    for (int s = 0; s < KSTEPS; s++) koff[s] = lds_addr(&lds_k[0][0]) + swz(l32 * K_CPR + s * 2 + half);
+    for (int s = 0; s < KSTEPS; s++) koff[s] = lds_addr(&lds_k[0][0]) + swz((kw * SK + l32) * K_CPR + s * 2 + half);
     if constexpr (VARIANT == 0) {
 #pragma unroll
-        for (int j = 0; j < JS; j++) voff[j] = lds_addr(&lds_v[0][0]) + swz(l32 * V_CPR + j * 2 + half);
+        for (int j = 0; j < JS; j++) voff[j] = lds_addr(&lds_v[0][0]) + swz(l32 * V_CPR + (kw * JS + j) * 2 + half);
     } else {
-        voff[0] = lds_addr(&lds_v[0][0]) + swz(l32 * V_CPR + half * 2);
-        voff[1] = lds_addr(&lds_v[0][0]) + swz(l32 * V_CPR + half * 2 + 1);
+        voff[0] = lds_addr(&lds_v[0][0]) + kw * D * VROW + swz(l32 * V_CPR + half * 2);
+        voff[1] = lds_addr(&lds_v[0][0]) + kw * D * VROW + swz(l32 * V_CPR + half * 2 + 1);
     }
 #pragma unroll
     for (int s = 0; s < KSTEPS; s++) asm volatile("" : "+v"(koff[s]));
@@ -339,9 +347,9 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     // 2060 clocks per 64 keys with the score instructions in a block of their own, 1680 dealt
     // out like this).  Three steps are in flight per wave, yet the scores (two buffers of SK keys)
     // and the packed probabilities (two buffers) take no more registers than one 64-key tile did.
-    constexpr int SK = VARIANT == 0 ? 32 : 64;          // keys per step
     constexpr int SKB = SK / 32;                        // 32-key blocks per step
-    constexpr int SPT = kTileKV / SK;                   // steps per tile
+    constexpr int SPT = TK / (SK * KW);                 // steps per tile
+    constexpr int GK = SK * KW;                         // keys that a step takes off all runs together
     constexpr int NQ = KSTEPS * SKB;                    // score matrix instructions per step
     constexpr int NPV = NUNIT / SPT;                    // P.V matrix instructions per step
     constexpr int NM = NQ + NPV;                        // slots per step
@@ -433,9 +441,9 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         // the wave's 32 rows, then the waves that share a scale block
         am = wave_max(am);
         if (blkq > 32) {
-            if (lane == 0) lds_qmax[wave] = am;
+            if (lane == 0) lds_qmax[rg] = am;       // (the waves of both runs encode the same rows for themselves)
             __syncthreads();
-            const int nwv = blkq >> 5, w0 = wave & ~(nwv - 1);
+            const int nwv = blkq >> 5, w0 = rg & ~(nwv - 1);
             am = lds_qmax[w0];
             for (int w = 1; w < nwv; w++) am = fmaxf(am, lds_qmax[w0 + w]);
         }
@@ -443,7 +451,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         const bool fast = sc >= 0x1p-100f && sc <= 0x1p100f;
         const float rinv = 1.0f / sc;
         // fp16 variant: the V^T slots that the first copies do not go to; e4m3: a region of its own
-        uint8_t* qs = (VARIANT == 0 ? &lds_v[LEAD][0] : &lds_qc[0]) + wave * 32 * D;
+        uint8_t* qs = VARIANT == 0 ? &lds_v[LEAD][0] + wave * 32 * D : &lds_qc[0] + rg * 32 * D;
         static_assert(VARIANT != 0 || !QF || (NSV - LEAD) * V_BYTES >= NW * 32 * D, "Q codes must fit the idle V^T slots");
 #pragma unroll
         for (int i = 0; i < Q_NI; i++) {
@@ -496,7 +504,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     // their spills, written and read back by every wave, cost a round of workgroups up to 50 us (e4m3, cross
     // [1,3840 x 192,32,128] 90.1 -> 42.6 us, [1,4000,16,128] 133.9 -> 116.2, [1,2304,18,256] 193.6 -> 187.1).
     const int last_step = (ntiles * SPT + 1) / 2 * 2 - 1;
-    auto key_step = [&](int h) -> int { return (t_off + key_tile(h / SPT) - h / SPT) * SPT + h; };       // step h's keys: key_step(h) * SK ..
+    auto key_step = [&](int h) -> int { return ((t_off + key_tile(h / SPT) - h / SPT) * SPT + h) * KW + kw; };       // step h's keys: key_step(h) * SK ..
     // The bias of the next two steps on its way (of one where two do not fit the registers), and (BPIPE) in the
     // scores' layout that of this step and the next, by parity of the step: dword k = scores 2k, 2k + 1 of the lane.
     constexpr int NBIAS = (VARIANT == 1 && D == 128) || D > 128 || SPLIT ? 1 : 2;
@@ -850,16 +858,16 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         // of the masked range or the ragged end, then — the steps that touch the range, at most a few, go
         // through the general bodies — those between the range and the ragged end.  Either stretch stops
         // early enough that the copies a trip starts need no clamping and do not cross the left-out tiles.
-        const bool range = RANGE && t_off * kTileKV < mask_hi;
-        int clean = (kv_valid - t_off * kTileKV) / SK - skip * SPT;
-        if (causal) clean = min(clean, (wave_row0 + 1) / SK);       // steps whose every key is <= the wave's first row
+        const bool range = RANGE && t_off * TK < mask_hi;
+        int clean = (kv_valid - t_off * TK) / GK - skip * SPT;
+        if (causal) clean = min(clean, (wave_row0 + 1) / GK);       // steps whose every key is <= the wave's first row
         const int tail_end = exact_bias ? 0 : min((ntiles - KOFF - LEAD) * SPT - 1 + (SPT - 1), clean);
         int trip_end = tail_end, past = 0, resume = 0;
         if (range) {
-            trip_end = min(trip_end, max(mask_lo - t_off * kTileKV, 0) / SK);
+            trip_end = min(trip_end, max(mask_lo - t_off * TK, 0) / GK);
             if (skip > 0) trip_end = min(trip_end, (skip_at - (KOFF + LEAD)) * SPT - 1 + (SPT - 1));
             // first step of a trip (1 modulo the period) behind the range
-            resume = (mask_hi - t_off * kTileKV + SK - 1) / SK - skip * SPT;
+            resume = (mask_hi - t_off * TK + GK - 1) / GK - skip * SPT;
             resume = max(resume + (PERIOD - 1), 0) / PERIOD * PERIOD + 1;
         }
         for (;;) {
@@ -867,12 +875,12 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
             kg_trip = kg + (int64_t)(hs / SPT + past) * K_BYTES;
             vg_trip = vg + (int64_t)(hs / SPT + past) * V_BYTES;
             {
-                typedef float kvec __attribute__((ext_vector_type(PERIOD * SKB == 8 ? 4 : 2)));
+                typedef float kvec __attribute__((ext_vector_type(KW > 1 ? SKB : PERIOD * SKB == 8 ? 4 : 2)));
                 constexpr int KV = sizeof(kvec) / sizeof(float);
-                const kvec* kp = reinterpret_cast<const kvec*>(&lds_ks[KS_OFF + (t_off + past) * 2 + hs * SKB]);
+                const kvec* kp = reinterpret_cast<const kvec*>(&lds_ks[KS_OFF + (t_off + past) * (TK / 32) + (hs * KW + kw) * SKB]);
 #pragma unroll
                 for (int i = 0; i < PERIOD * SKB; i += KV) {
-                    const kvec k = kp[i / KV];
+                    const kvec k = kp[i / KV * KW];
 #pragma unroll
                     for (int e = 0; e < KV; e++) kst[i + e] = k[e];
                 }
@@ -999,6 +1007,43 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         }
     }
 
+    constexpr int DW = D / KW, DWB = DW / 32;           // channels that a wave writes out, from kw * DW on
+    if constexpr (KW > 1) {
+        // ---- the partner wave's keys: each of the two takes half of the channels, and leaves its own results of the other
+        // half in LDS, lane by lane (both hold the same rows and channels in the same lanes)
+        dma_wait<0>();                                  // (copies of the clamped last tile, see the epilogue)
+        __syncthreads();
+        static_assert(NSV * V_BYTES >= NW * DWB * 16 * 64 * 4 && kTwoRunKeys / 32 >= NW * 128, "hand-over regions");
+        v4f* give = reinterpret_cast<v4f*>(&lds_v[0][0]) + wave * (DWB * 4 * 64) + lane;
+        const v4f* take = reinterpret_cast<const v4f*>(&lds_v[0][0]) + (wave ^ RG) * (DWB * 4 * 64) + lane;
+#pragma unroll
+        for (int d = 0; d < DWB; d++)
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                v4f x;
+#pragma unroll
+                for (int e = 0; e < 4; e++) x[e] = kw == 0 ? oacc[DWB + d][g * 4 + e] : oacc[d][g * 4 + e];
+                give[(d * 4 + g) * 64] = x;
+            }
+        lds_ks[wave * 128 + lane] = m_used;
+        lds_ks[wave * 128 + 64 + lane] = VARIANT == 0 ? l_run : lacc[0];
+        __syncthreads();
+        const float m_p = lds_ks[(wave ^ RG) * 128 + lane], l_p = lds_ks[(wave ^ RG) * 128 + 64 + lane];
+        const float m_new = fmaxf(m_used, m_p);
+        const float ca = __builtin_amdgcn_exp2f(m_used - m_new), cb = __builtin_amdgcn_exp2f(m_p - m_new);
+        if constexpr (VARIANT == 0) l_run = l_run * ca + l_p * cb;
+        else lacc[0] = lacc[0] * ca + l_p * cb;
+#pragma unroll
+        for (int d = 0; d < DWB; d++)
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const v4f x = take[(d * 4 + g) * 64];
+#pragma unroll
+                for (int e = 0; e < 4; e++) oacc[d][g * 4 + e] = (kw == 0 ? oacc[d][g * 4 + e] : oacc[DWB + d][g * 4 + e]) * ca + x[e] * cb;
+            }
+        m_used = m_new;
+    }
+
     // ---- epilogue: normalise, bf16 round-to-nearest-even, caller's strides ---------
     float l_tot;
     if constexpr (VARIANT == 0) {
@@ -1013,37 +1058,39 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     // The last midpoints' copies of the clamped last tile go to slots of those rings and may still be on their
     // way (the barrier does not wait for them, and the compiler does not know of them): every wave lets its own
     // land before it says that it is done.
-    dma_wait<0>();
-    __syncthreads();                                // every wave is done with the rings, its copies included
+    if constexpr (KW == 1) {
+        dma_wait<0>();
+        __syncthreads();                            // every wave is done with the rings, its copies included
+    }
     {
-        static_assert(NSK * K_BYTES >= NW / 2 * 64 * D && NSV * V_BYTES >= NW / 2 * 64 * D, "output rows must fit the rings");
-        constexpr int OC = D / 8;                   // 16-byte chunks per output row, XORed with the row
-        uint8_t* os = wave < NW / 2 ? &lds_k[0][0] + wave * 64 * D : &lds_v[0][0] + (wave - NW / 2) * 64 * D;
+        static_assert(KW == 1 ? NSK * K_BYTES >= NW / 2 * 64 * D && NSV * V_BYTES >= NW / 2 * 64 * D : NSK * K_BYTES >= NW * 64 * DW, "output rows must fit the rings");
+        constexpr int OC = DW / 8;                  // 16-byte chunks per output row, XORed with the row
+        uint8_t* os = KW > 1 || wave < NW / 2 ? &lds_k[0][0] + wave * 64 * DW : &lds_v[0][0] + (wave - NW / 2) * 64 * DW;
 #pragma unroll
-        for (int d = 0; d < DB; d++)
+        for (int d = 0; d < DWB; d++)
 #pragma unroll
             for (int g = 0; g < 4; g++) {
                 float x[4];
 #pragma unroll
                 for (int e = 0; e < 4; e++) x[e] = oacc[d][g * 4 + e];
                 if constexpr (VARIANT == 1) {
-                    const v4f vs = *reinterpret_cast<const v4f*>(vscale + bh * D + d * 32 + g * 8 + half * 4);
+                    const v4f vs = *reinterpret_cast<const v4f*>(vscale + bh * D + kw * DW + d * 32 + g * 8 + half * 4);
 #pragma unroll
                     for (int e = 0; e < 4; e++) x[e] *= vs[e];
                 }
-                *reinterpret_cast<u32x2*>(os + l32 * (D * 2) + (((d * 4 + g) ^ (l32 & (OC - 1))) << 4) + half * 8) =
+                *reinterpret_cast<u32x2*>(os + l32 * (DW * 2) + (((d * 4 + g) ^ (l32 & (OC - 1))) << 4) + half * 8) =
                     u32x2{pack_bf16(x[0] * inv, x[1] * inv), pack_bf16(x[2] * inv, x[3] * inv)};
             }
         constexpr int RPI = 64 / OC;                // rows per store instruction
-        uint16_t* op = o + b * osb + h * osh + (lane % OC) * 8;
+        uint16_t* op = o + b * osb + h * osh + kw * DW + (lane % OC) * 8;
 #pragma unroll
         for (int i = 0; i < 32 / RPI; i++) {
             const int r = i * RPI + lane / OC;
-            const u32x4 w = *reinterpret_cast<const u32x4*>(os + r * (D * 2) + (((lane % OC) ^ (r & (OC - 1))) << 4));
+            const u32x4 w = *reinterpret_cast<const u32x4*>(os + r * (DW * 2) + (((lane % OC) ^ (r & (OC - 1))) << 4));
             if (wave_row0 + r < Nq) *reinterpret_cast<u32x4*>(op + (int64_t)(wave_row0 + r) * osn) = w;
         }
     }
-    if (STATS && qrow < Nq && half == 0) {
+    if (STATS && kw == 0 && qrow < Nq && half == 0) {
         // natural-log log-sum-exp of the scaled scores.  With K smoothing every score
         // of a row was lowered by <q, mean>, which the Q quantizer recorded per row.
         const float shift = qshift != nullptr ? qshift[bh * nq_pad + qrow] : 0.0f;
@@ -1074,12 +1121,17 @@ __global__ void split_clear_kernel(int* flags, int n) {
     for (int i = threadIdx.x; i < n; i += blockDim.x) flags[i] = 0;
 }
 
+// two_runs: the row tiles from a.main_items on, in the two-run form; otherwise those below it.
 template <int D, int VARIANT>
-static hipError_t launch_attn_dv(const AttnArgs& a, hipStream_t st) {
+static hipError_t launch_attn_dv(const AttnArgs& a, bool two_runs, hipStream_t st) {
     constexpr int kThreads = D > 128 ? 256 : 512;             // 32 query rows per wave
-    const int n_qtiles = (a.Nq + kThreads / 2 - 1) / (kThreads / 2);
-    const int64_t total = a.main_items;
-    if (total <= 0 || total > 0x7FFFFFFF || total > (int64_t)n_qtiles * a.B * a.H) return hipErrorInvalidValue;
+    const int rows = kThreads / 2 / (two_runs ? 2 : 1);
+    // (behind row tiles of the main kernel: two pieces to each of them, the last of which may be empty)
+    const int n_qtiles = two_runs && a.main_items > 0 ? 2 * ((a.Nq + kThreads / 2 - 1) / (kThreads / 2)) : (a.Nq + rows - 1) / rows;
+    const int64_t first = two_runs ? 2 * a.main_items : 0;
+    const int64_t total = two_runs ? (int64_t)n_qtiles * a.B * a.H - first : a.main_items;
+    if (total <= 0 || first + total > 0x7FFFFFFF || first + total > (int64_t)n_qtiles * a.B * a.H) return hipErrorInvalidValue;
+    if (two_runs && (D > 128 || a.short_kw > 0 || a.split_wgs > 0 || a.nkv_pad > kTwoRunKeys || (VARIANT == 1 && a.amask != nullptr))) return hipErrorInvalidValue;
     const int split = (D <= 128 && VARIANT == 0 && !a.causal) ? a.split_wgs : 0;
     int* flags = nullptr;
     float* part = nullptr;
@@ -1092,32 +1144,41 @@ static hipError_t launch_attn_dv(const AttnArgs& a, hipStream_t st) {
     }
     dim3 grid((unsigned)(split > 0 ? split : total)), block(kThreads);
     const bool range = a.km.hi > a.km.lo;
-#define SAGE_LAUNCH_ATTN2(STATS, ADDMASK, SPLIT, RANGE)                                                                  \
-    hipLaunchKernelGGL((sage_attn_kernel<D, VARIANT, STATS, ADDMASK, SPLIT, RANGE>), grid, block, 0, st, a.q8, a.qscale, a.blkq, \
+#define SAGE_LAUNCH_ATTN2(STATS, ADDMASK, SPLIT, RANGE, KW)                                                              \
+    hipLaunchKernelGGL((sage_attn_kernel<D, VARIANT, STATS, ADDMASK, SPLIT, RANGE, false, KW>), grid, block, 0, st, a.q8, a.qscale, a.blkq, \
                        a.q_src, a.qsb, a.qsh, a.qsn, a.qmul, a.k8, a.kscale, a.blkk, (const uint8_t*)a.vq, a.vscale, a.qshift, a.H, a.Nq, a.kv_valid,          \
-                       a.km.lo, a.km.hi, a.causal, a.nq_pad, a.nkv_pad, a.o, a.osb, a.osh, a.osn, a.stats, n_qtiles,               \
+                       a.km.lo, a.km.hi, a.causal, a.nq_pad, a.nkv_pad, a.o, a.osb, a.osh, a.osn, a.stats, n_qtiles, (int)first,   \
                        (int)total, a.amask, a.amb, a.amh, a.amn, split >> 3, part, flags, g_split_wait.load())
 #define SAGE_LAUNCH_ATTN(STATS, ADDMASK)                                               \
     do {                                                                               \
         if constexpr (D <= 128 && VARIANT == 0) {                                      \
-            if (split > 0) { SAGE_LAUNCH_ATTN2(STATS, ADDMASK, true, false); break; }  \
+            if (split > 0) { SAGE_LAUNCH_ATTN2(STATS, ADDMASK, true, false, 1); break; }  \
+        }                                                                              \
+        if constexpr (D <= 128 && !(ADDMASK && VARIANT == 1)) {                        \
+            if constexpr (!ADDMASK) {                                                  \
+                if (range && two_runs) { SAGE_LAUNCH_ATTN2(STATS, ADDMASK, false, true, 2); break; }      \
+            }                                                                          \
+            if (two_runs) { SAGE_LAUNCH_ATTN2(STATS, ADDMASK, false, false, 2); break; }       \
         }                                                                              \
         if constexpr (!ADDMASK) {                                                      \
-            if (range) { SAGE_LAUNCH_ATTN2(STATS, ADDMASK, false, true); break; }      \
+            if (range) { SAGE_LAUNCH_ATTN2(STATS, ADDMASK, false, true, 1); break; }      \
         }                                                                              \
-        SAGE_LAUNCH_ATTN2(STATS, ADDMASK, false, false);                               \
+        SAGE_LAUNCH_ATTN2(STATS, ADDMASK, false, false, 1);                            \
     } while (0)
     if (a.q_src != nullptr) {
         // Q encoded by the kernel: the plain forward only
         if constexpr (D <= 128) {
             if (a.amask != nullptr || a.stats != nullptr || split > 0 || a.qmul == nullptr) return hipErrorInvalidValue;
-#define SAGE_LAUNCH_ATTN_QF(RANGE)                                                                                              \
-    hipLaunchKernelGGL((sage_attn_kernel<D, VARIANT, false, false, false, RANGE, true>), grid, block, 0, st, nullptr, nullptr, a.blkq, \
+#define SAGE_LAUNCH_ATTN_QF(RANGE, KW)                                                                                          \
+    hipLaunchKernelGGL((sage_attn_kernel<D, VARIANT, false, false, false, RANGE, true, KW>), grid, block, 0, st, nullptr, nullptr, a.blkq, \
                        a.q_src, a.qsb, a.qsh, a.qsn, a.qmul, a.k8, a.kscale, a.blkk, (const uint8_t*)a.vq, a.vscale, nullptr,  \
                        a.H, a.Nq, a.kv_valid, a.km.lo, a.km.hi, a.causal, a.nq_pad, a.nkv_pad, a.o, a.osb, a.osh, a.osn, nullptr, \
-                       n_qtiles, (int)total, nullptr, 0, 0, 0, 0, nullptr, nullptr, g_split_wait.load())
-            if (range) SAGE_LAUNCH_ATTN_QF(true);
-            else SAGE_LAUNCH_ATTN_QF(false);
+                       n_qtiles, (int)first, (int)total, nullptr, 0, 0, 0, 0, nullptr, nullptr, g_split_wait.load())
+            if (range) {
+                if (two_runs) SAGE_LAUNCH_ATTN_QF(true, 2);
+                else SAGE_LAUNCH_ATTN_QF(true, 1);
+            } else if (two_runs) SAGE_LAUNCH_ATTN_QF(false, 2);
+            else SAGE_LAUNCH_ATTN_QF(false, 1);
 #undef SAGE_LAUNCH_ATTN_QF
         } else {
             return hipErrorInvalidValue;
@@ -1225,13 +1286,15 @@ size_t attn_split_bytes(int workgroups, int D) {
 
 hipError_t launch_attn(const AttnArgs& a, hipStream_t st) {
     if (a.nkv_pad > max_keys(a.D)) return hipErrorInvalidValue;      // K scales would not fit the LDS staging
+    auto main = [&](bool two_runs) -> hipError_t {
+        if (a.D == 128) return a.variant == 0 ? launch_attn_dv<128, 0>(a, two_runs, st) : launch_attn_dv<128, 1>(a, two_runs, st);
+        if (a.D == 64) return a.variant == 0 ? launch_attn_dv<64, 0>(a, two_runs, st) : launch_attn_dv<64, 1>(a, two_runs, st);
+        if (a.D == 256) return a.variant == 0 ? launch_attn_dv<256, 0>(a, two_runs, st) : launch_attn_dv<256, 1>(a, two_runs, st);
+        return hipErrorInvalidValue;
+    };
     hipError_t e = hipSuccess;
-    if (a.main_items > 0) {
-        if (a.D == 128) e = a.variant == 0 ? launch_attn_dv<128, 0>(a, st) : launch_attn_dv<128, 1>(a, st);
-        else if (a.D == 64) e = a.variant == 0 ? launch_attn_dv<64, 0>(a, st) : launch_attn_dv<64, 1>(a, st);
-        else if (a.D == 256) e = a.variant == 0 ? launch_attn_dv<256, 0>(a, st) : launch_attn_dv<256, 1>(a, st);
-        else e = hipErrorInvalidValue;
-    }
+    if (a.main_items > 0) e = main(false);
+    if (e == hipSuccess && a.two_runs) return main(true);
     return e == hipSuccess && a.short_kw > 0 ? launch_attn_short(a, st) : e;
 }
 

@@ -462,23 +462,19 @@ hipError_t launch_attn_short(const AttnArgs& a, hipStream_t st) {
 }
 
 // Which form, from what each costs on an MI355X: time = base + rounds (r + s steps) + fill (f + g steps) in
-// microseconds, with rounds = workgroups / compute units rounded up, fill = workgroups / compute units, steps = key tiles (main
-// kernel) or key steps of the longest run (short form); the split schedule: base + per balanced key tile.
-// The coefficients were fitted to 350 to 400 launches of the kernel and 230 one-shot calls per head dim and variant
-// (2 to 480 heads, 32 to 16384 queries, 16 to 32768 keys), of earlier forms of both kernels, of which both have become
-// faster since (the main kernel's cost per tile at 256 channels is of the present one).  With the kernels as they are, choosing by them costs 0.2 to 0.9 % on average over the best of the forms
-// taken for everything (70 one-shot calls drawn per head dim and variant, 2 to 240 heads, 64 to 4096 queries): 20 of 420
-// over 2 %, the worst 10 %, [1,75,22,128] 17.5 us instead of 15.9.  There is no term for a bias: with one 0.2 to 2.5 % (30
-// calls each), the worst 22 % ([1,73,35,128] 19.5 instead of 16.1).  (A fit that ended at 4096 keys, carried on to longer
-// ones, gave whole problems of 64 channels with e4m3 P.V to the short form, which moves 8 times the operand bytes:
-// [1,16384,12,64] 929 us, the main kernel 614.)  One-shot, main kernel -> short form: [1,256,30,128] 19.2 -> 17.1 us,
-// [1,1024,8,64] 24.6 -> 17.2, [1,1024,8,128] 30.6 -> 22.2, [1,512,24,128] 24.1 -> 22.3.  The main kernel is back ahead
-// between 64 and 75 workgroups of 256 rows (128 rows at 256 channels) with fp16 P.V, at 64 channels and 2048 keys between 90
-// and 110; with e4m3 the two are level from 75 on at 512 keys, and it is back ahead between 125 and 140 at 2048.
+// microseconds, with rounds = workgroups / compute units rounded up, fill = workgroups / compute units, steps = key tiles of
+// 64 (main kernel, two-run form) or key steps of the longest run (short form); the split schedule: base + per balanced key
+// tile.  Four forms: the main kernel, 256 query rows and all keys per workgroup; its loop with 128 rows, the keys split
+// over two halves of the waves (two runs: the same tiles, a step of them per wave, results merged in LDS at the end); and the
+// short form with 64 rows in four runs or 32 in eight.  What splits the keys is for grids that do not fill the chip: a
+// step takes a wave about as long with the chip half empty.  One-shot, us, without the two-run form -> with it: [1,1127,19,128] 39.0 ->
+// 32.5, [1,1091,16,128] 36.4 -> 29.2, e4m3 [2,615,16,128] 34.1 -> 31.1, [1,1127,19,64] 30.6 -> 25.7, with a bias
+// [1,1153,24,128] 55.0 -> 45.0.  Past about 128 row tiles its workgroups take a second round and the main kernel is ahead
+// ([1,1322,30,128] 47 against 58); below 40 to 60 the short form is (eight runs: [1,256,30,128] 16.6 against 18.4).
 //
-// A problem of some rounds and a bit more takes both: the main kernel does the full rounds and the short
-// form what is left, spread over the whole chip, instead of one more round that is nearly empty (264 items
-// of 32 key tiles, 128 channels: 84 -> 66 us; of 64 channels 61 -> 43; by earlier forms of both).
+// A problem of some rounds and a bit more takes two: the main kernel does the full rounds and another form what is left,
+// spread over the whole chip, instead of one more round that is nearly empty (short form, 264 items of 32 key tiles, 128
+// channels: 84 -> 66 us; of 64 channels 61 -> 43; by earlier forms of both).
 // The split schedule, which balances the same problems by handing partial results over in memory, is ahead of both where
 // the second of few rounds is a quarter to a half full and the key sequence is long: a sixth (64 channels) and a
 // thirteenth (128) of the 788 shapes of its rule that were timed (with earlier forms of the kernels, where it was taken it
@@ -491,70 +487,105 @@ struct FormCost {
         return base + rounds * (r + s * n) + fill * (f + g * n);
     }
 };
-static const FormCost kCost[3][2][3] = {        // [64, 128, 256 channels][variant][main, 4 runs, 8 runs]
-    {{{6.00f, 1.70f, 0.78f, 0.00f, 0.03f}, {4.97f, 1.54f, 0.50f, 0.00f, 0.17f}, {5.18f, 1.19f, 0.41f, 0.14f, 0.27f}},
-     {{1.91f, 3.27f, 0.76f, 1.13f, 0.06f}, {3.02f, 1.61f, 1.08f, 1.28f, 0.00f}, {2.55f, 1.40f, 1.20f, 1.06f, 0.00f}}},
-    {{{1.29f, 3.84f, 0.75f, 0.88f, 0.54f}, {2.68f, 3.27f, 0.92f, 0.05f, 0.42f}, {2.56f, 3.24f, 0.95f, 0.04f, 0.36f}},
-     {{2.15f, 4.92f, 0.95f, 1.71f, 0.11f}, {2.52f, 4.17f, 1.20f, 0.18f, 0.30f}, {2.54f, 3.25f, 1.40f, 0.75f, 0.14f}}},
-    {{{1.44f, 4.16f, 0.90f, 2.31f, 0.44f}, {2.87f, 6.05f, 1.29f, 0.20f, 0.25f}, {}},
-     {{3.61f, 4.01f, 1.09f, 2.79f, 0.10f}, {1.45f, 5.06f, 2.57f, 1.45f, 0.00f}, {}}},
+enum Form { MAIN = 0, TWO_RUNS = 1, RUNS4 = 2, RUNS8 = 3, FORMS = 4 };
+constexpr FormCost kNoForm{1e9f, 0.0f, 0.0f, 0.0f, 0.0f};
+// Up to 3072 keys, 64 and 128 channels.  Fitted to the differences between the forms of 225 one-shot calls each (120 of 500 to
+// 3000 tokens, 65 cross, 40 of 64 to 4096, all forms timed), Q where sdpa_impl puts it; what all forms have in common is not
+// in them.  Over those calls the choice costs 0.1 % on average over the best single form, the worst 11 %; without the two-run
+// form it cost 3 to 6 % on average.
+static const FormCost kCost[2][2][FORMS] = {
+    {{{6.00f, 1.70f, 0.70f, 0.00f, 0.03f}, {5.94f, 2.18f, 0.46f, 0.56f, 0.02f}, {4.97f, 2.18f, 0.53f, 0.18f, 0.26f}, {5.18f, 1.40f, 0.40f, 0.00f, 0.25f}},
+     {{0.00f, 5.53f, 0.57f, 3.88f, 0.00f}, {1.57f, 5.08f, 0.26f, 0.81f, 0.08f}, {0.45f, 5.44f, 0.72f, 0.00f, 0.07f}, {1.33f, 4.41f, 0.58f, 0.00f, 0.12f}}},
+    {{{0.00f, 8.33f, 0.68f, 10.04f, 0.00f}, {3.91f, 5.03f, 0.35f, 5.68f, 0.02f}, {3.16f, 6.96f, 0.32f, 0.00f, 0.70f}, {3.24f, 5.57f, 0.44f, 0.00f, 0.61f}},
+     {{0.00f, 6.65f, 0.72f, 9.30f, 0.00f}, {1.82f, 6.43f, 0.35f, 3.58f, 0.05f}, {0.40f, 6.76f, 0.88f, 0.21f, 0.34f}, {0.80f, 5.48f, 1.06f, 0.00f, 0.17f}}},
+};
+// Under an additive bias, fp16 P.V (50 calls of 128 to 2304 tokens at 64 channels, 110 at 128: 0.1 % and nothing).
+static const FormCost kCostBias[2][FORMS] = {
+    {{0.00f, 7.38f, 1.37f, 19.88f, 0.04f}, {4.24f, 3.73f, 0.78f, 11.53f, 0.00f}, {8.78f, 0.70f, 0.52f, 5.33f, 0.71f}, {7.37f, 1.30f, 0.00f, 2.40f, 1.24f}},
+    {{0.00f, 14.94f, 1.53f, 14.28f, 0.06f}, {11.61f, 3.82f, 0.90f, 9.82f, 0.00f}, {10.61f, 5.30f, 0.78f, 3.42f, 0.85f}, {10.33f, 5.25f, 0.32f, 1.00f, 1.35f}},
+};
+// All lengths, by launches and calls of up to 32 768 keys of earlier forms of the kernels (the two-run form against the
+// main kernel's figures here): longer key sequences, 256 channels, and what the split schedule is compared with.
+static const FormCost kCostLong[3][2][FORMS] = {        // [64, 128, 256 channels]
+    {{{6.00f, 1.70f, 0.78f, 0.00f, 0.03f}, {5.94f, 2.48f, 0.46f, 0.56f, 0.02f}, {4.97f, 1.54f, 0.50f, 0.00f, 0.17f}, {5.18f, 1.19f, 0.41f, 0.14f, 0.27f}},
+     {{1.91f, 3.27f, 0.76f, 1.13f, 0.06f}, {1.52f, 3.29f, 0.43f, 1.86f, 0.00f}, {3.02f, 1.61f, 1.08f, 1.28f, 0.00f}, {2.55f, 1.40f, 1.20f, 1.06f, 0.00f}}},
+    {{{1.29f, 3.84f, 0.75f, 0.88f, 0.54f}, {1.85f, 4.15f, 0.35f, 0.79f, 0.35f}, {2.68f, 3.27f, 0.92f, 0.05f, 0.42f}, {2.56f, 3.24f, 0.95f, 0.04f, 0.36f}},
+     {{2.15f, 4.92f, 0.95f, 1.71f, 0.11f}, {2.88f, 3.94f, 0.57f, 2.66f, 0.00f}, {2.52f, 4.17f, 1.20f, 0.18f, 0.30f}, {2.54f, 3.25f, 1.40f, 0.75f, 0.14f}}},
+    {{{1.44f, 4.16f, 0.90f, 2.31f, 0.44f}, kNoForm, {2.87f, 6.05f, 1.29f, 0.20f, 0.25f}, kNoForm},
+     {{3.61f, 4.01f, 1.09f, 2.79f, 0.10f}, kNoForm, {1.45f, 5.06f, 2.57f, 1.45f, 0.00f}, kNoForm}},
 };
 // (fp16 at 64 channels past 3072 keys: no one set meets both ends there)
-static const FormCost kCost64Long[3] = {{1.81f, 2.54f, 0.66f, 0.34f, 0.16f}, {3.60f, 0.70f, 0.78f, 0.00f, 0.06f}, {3.72f, 0.77f, 0.55f, 0.03f, 0.18f}};
+static const FormCost kCost64Long[FORMS] = {{1.81f, 2.54f, 0.66f, 0.34f, 0.16f}, {1.75f, 3.32f, 0.34f, 0.90f, 0.15f}, {3.60f, 0.70f, 0.78f, 0.00f, 0.06f}, {3.72f, 0.77f, 0.55f, 0.03f, 0.18f}};
 static const float kSplitCost[2][2] = {{17.0f, 0.96f}, {25.0f, 1.53f}};       // [64, 128 channels]: base, per key tile
 
 // Microseconds a call takes more with the main kernel where its Q cannot go to the encoders for next to nothing:
 // many queries on few keys, which keep Q in the kernel's prologue, and a K that takes one launch alone but not with Q.
 // One-shot, main kernel against short form: [1,510 x 139,24,128] 20.8 against 19.0, [1,256 x 292,40,128] 25.0 against 22.3,
 // e4m3 [2,71 x 45,32,256] 36.3 against 28.8; with as many keys as queries they are level, [1,64,24,128] 15.2 against 15.2
-// to 16.0.  (64 channels: nothing to gain, or the second kind's fit is as good without.)
+// to 16.0.  (64 channels: nothing to gain, or the second kind's fit is as good without; kCost has it in its figures.)
 static const float kQCost[3][2][2] = {{{0.0f, 0.0f}, {0.8f, 0.0f}}, {{1.4f, 1.4f}, {0.0f, 0.0f}}, {{0.0f, 2.0f}, {0.0f, 2.0f}}};
 
 namespace {
-struct Short { float t; int kw; };
-Short best_short(const FormCost* c, int64_t rows, int64_t bh, int D, int64_t steps, int units) {
-    const int rows4 = D > 128 ? 32 : 64;
-    const Short four{c[1].of(bh * ((rows + rows4 - 1) / rows4), (steps + 3) / 4, units), 4};
-    if (D > 128) return four;
-    const Short eight{c[2].of(bh * ((rows + 31) / 32), (steps + 7) / 8, units), 8};
-    return four.t < eight.t ? four : eight;
+struct Choice { float t; AttnPlan p; };
+// `rows` query rows of each of bh heads by the form that is predicted fastest, the main kernel's left out
+Choice best_small(const FormCost* c, int64_t rows, int64_t bh, int D, int variant, int64_t kv, int units, bool two_runs) {
+    const int64_t tiles = (kv + kTileKV - 1) / kTileKV, steps = variant == 0 ? (kv + 31) / 32 : tiles;
+    auto wgs = [&](int per) { return bh * ((rows + per - 1) / per); };
+    Choice best{1e30f, AttnPlan{0, 4, 0}};
+    auto offer = [&](float t, const AttnPlan& p) { if (t < best.t) best = Choice{t, p}; };
+    if (two_runs) offer(c[TWO_RUNS].of(wgs(128), variant == 0 ? tiles : (tiles + 1) / 2 * 2, units), AttnPlan{0, 0, 0, true});
+    offer(c[RUNS4].of(wgs(D > 128 ? 32 : 64), (steps + 3) / 4, units), AttnPlan{0, 4, 0});
+    if (D <= 128) offer(c[RUNS8].of(wgs(32), (steps + 7) / 8, units), AttnPlan{0, 8, 0});
+    return best;
 }
 }  // namespace
 
-static AttnPlan plan_by_shape(int units, int B, int H, int Nq, int kv_valid, int D, int variant, bool causal, int split) {
+// short_or_main: what the figures for all lengths say of those two alone.
+static AttnPlan plan_by_shape(int units, int B, int H, int Nq, int kv_valid, int D, int variant, bool causal, bool bias, int split, bool short_or_main = false) {
     const int v = variant == 0 ? 0 : 1, d = D == 64 ? 0 : D == 128 ? 1 : 2;
-    const int64_t bh = (int64_t)B * H;
-    const int64_t tiles = (kv_valid + kTileKV - 1) / kTileKV, steps = variant == 0 ? (kv_valid + 31) / 32 : tiles;
-    const FormCost* c = D == 64 && v == 0 && tiles > 48 ? kCost64Long : kCost[d][v];
+    const int64_t bh = (int64_t)B * H, tiles = (kv_valid + kTileKV - 1) / kTileKV;
     const int rows = D > 128 ? 128 : 256;
     const int64_t items = bh * ((Nq + rows - 1) / rows), whole = items / units * units;
-    AttnPlan p{items, 0, 0};
+    const FormCost* by_length = D == 64 && v == 0 && tiles > 48 ? kCost64Long : kCostLong[d][v];
     const int blkq = variant == 0 ? 128 : 32;
     const int64_t alone = quant_short_workgroups(B, H, Nq, kv_valid, D, blkq, 64, false);
     const int64_t with_q = alone > 0 ? quant_short_workgroups(B, H, Nq, kv_valid, D, blkq, 64, true) : 0;
     const float q_cost = std::max(Nq > 2 * kv_valid ? kQCost[d][v][0] : 0.0f, alone > 0 && (with_q == 0 || with_q > units) ? kQCost[d][v][1] : 0.0f);
-    float best = c[0].of(items, tiles, units) + q_cost;
-    const Short all = best_short(c, Nq, bh, D, steps, units);
-    if (all.t < best) { best = all.t; p = AttnPlan{0, all.kw, 0}; }
-    if (!causal && whole > 0 && whole < items) {
-        const Short rest = best_short(c, rows, items - whole, D, steps, units);
-        const float t = c[0].of(whole, tiles, units) + q_cost + rest.t;
-        if (t < best) { best = t; p = AttnPlan{whole, rest.kw, 0}; }
-    }
-    if (!causal && split > 0 && D <= 128 && kSplitCost[d][0] + kSplitCost[d][1] * (float)(items * tiles) / 256.0f < best) p = AttnPlan{items, 0, split};
-    return p;
+    auto choose = [&](const FormCost* c, float q_main, float launch, bool two_runs) -> Choice {
+        // (past a round of row tiles the two-run form does what the main kernel's whole rounds leave: that is ahead of
+        // it doing everything, or level)
+        Choice best = best_small(c, Nq, bh, D, variant, kv_valid, units, two_runs && (causal || whole == 0 || whole == items));
+        const float main = c[MAIN].of(items, tiles, units) + q_main;
+        if (main <= best.t) best = Choice{main, AttnPlan{items, 0, 0}};
+        if (!causal && whole > 0 && whole < items) {
+            const Choice rest = best_small(c, rows, items - whole, D, variant, kv_valid, units, two_runs);
+            const float t = c[MAIN].of(whole, tiles, units) + q_main + launch + rest.t;
+            if (t < best.t) best = Choice{t, AttnPlan{whole, rest.p.short_kw, 0, rest.p.two_runs}};
+        }
+        return best;
+    };
+    if (!causal && split > 0 && D <= 128 &&
+        kSplitCost[d][0] + kSplitCost[d][1] * (float)(items * tiles) / 256.0f < choose(by_length, q_cost, 0.0f, false).t)
+        return AttnPlan{items, 0, split};
+    if (short_or_main) return choose(by_length, q_cost, 0.0f, false).p;
+    // (figures that were fitted to differences have not got what a second launch costs)
+    const float launch = d == 0 && v == 0 ? 0.0f : 3.0f;
+    const bool two_runs = D <= 128 && pad_to(kv_valid, kPadKV) <= kTwoRunKeys && !(bias && v == 1);
+    if (D <= 128 && bias && v == 0) return choose(kCostBias[d], 0.0f, 3.0f, two_runs).p;
+    if (D <= 128 && !bias && tiles <= 48) return choose(kCost[d][v], 0.0f, launch, two_runs).p;
+    return choose(by_length, q_cost, 0.0f, two_runs).p;
 }
 
 static std::atomic<int> g_short_mode{0};       // 0: by shape; -1: never; 4, 8: always, that many key runs (4 at 256 channels)
 void attn_short_override(int mode) { g_short_mode.store(mode); }
 
 int attn_short_rule(int B, int H, int Nq, int kv_valid, int D, int variant) {
-    const AttnPlan p = plan_by_shape(256, B, H, Nq, kv_valid, D, variant, false, 0);
+    const AttnPlan p = plan_by_shape(256, B, H, Nq, kv_valid, D, variant, false, false, 0, true);
     return p.main_items == 0 ? p.short_kw : 0;
 }
 
 int64_t attn_main_items_on(int units, int B, int H, int Nq, int kv_valid, int D, int variant) {
-    return plan_by_shape(units, B, H, Nq, kv_valid, D, variant, false, 0).main_items;
+    return plan_by_shape(units, B, H, Nq, kv_valid, D, variant, false, false, 0).main_items;
 }
 
 // Asked of the device once.  (256 where there is none to ask.)
@@ -570,13 +601,16 @@ int compute_units() {
     return n;
 }
 
-AttnPlan attn_plan(int B, int H, int Nq, int kv_valid, int D, int variant, bool causal) {
+AttnPlan attn_plan(int B, int H, int Nq, int kv_valid, int D, int variant, bool causal, bool bias) {
     const int mode = g_short_mode.load(), rows = D > 128 ? 128 : 256;
+    const bool two_runs_fit = D <= 128 && pad_to(kv_valid, kPadKV) <= kTwoRunKeys && !(bias && variant != 0);
+    if (mode == 2 && two_runs_fit) return AttnPlan{0, 0, 0, true};
+    if (mode == 2) return AttnPlan{(int64_t)B * H * ((Nq + rows - 1) / rows), 0, 0};
     if (mode > 0) return AttnPlan{0, D == 256 ? 4 : mode, 0};
     const int split = causal ? 0 : attn_split_workgroups(B, H, Nq, kv_valid, D, variant);
     if (mode < 0 || attn_split_override_mode() != 0)      // (a schedule of the main kernel was asked for)
         return AttnPlan{(int64_t)B * H * ((Nq + rows - 1) / rows), 0, split};
-    return plan_by_shape(compute_units(), B, H, Nq, kv_valid, D, variant, causal, split);
+    return plan_by_shape(compute_units(), B, H, Nq, kv_valid, D, variant, causal, bias, split);
 }
 
 }  // namespace sage

@@ -16,6 +16,7 @@ constexpr int kGroup  = 256;   // tokens per group (16 leaves)
 // The attention kernel stages one head's K scales in LDS, one entry per 32 keys: keys per head it takes
 // (256 channels: the tile rings leave room for a quarter as many entries).
 __host__ __device__ constexpr int max_keys(int D) { return (D > 128 ? 2048 : 8192) * 32; }
+constexpr int kTwoRunKeys = 32768;       // ... in the two-run form
 
 inline int64_t pad_to(int64_t n, int64_t m) { return (n + m - 1) / m * m; }
 
@@ -166,20 +167,22 @@ struct AttnArgs {
     const uint16_t* q_src;   // null: q8 / qscale are read
     int64_t qsb, qsh, qsn;
     const float* qmul;
-    // the plan (attn_plan): the main kernel does the row tiles below main_items, the short form the rest
+    // the plan (attn_plan): the main kernel does the row tiles below main_items, the short or the two-run form the rest
     int64_t main_items;
     int short_kw;            // key runs per row block in the short form
+    bool two_runs;           // the rest in the main kernel's two-run form
     int split_wgs;           // workgroups of the main kernel's split schedule, 0: one workgroup per item
     void* split;             // attn_split_bytes(split_wgs, D) bytes, 256-byte aligned (null when 0)
 };
 hipError_t launch_attn(const AttnArgs& a, hipStream_t st);
 // Which kernel does what.  Items are row tiles (256 query rows of a head; 128 at 256 channels), head by head.
 struct AttnPlan {
-    int64_t main_items;      // items [0, main_items) by the main kernel, the rest by the short form
+    int64_t main_items;      // items [0, main_items) by the main kernel, the rest by the short or the two-run form
     int short_kw;            // key runs of the short form (32 or 64 rows per workgroup, keys split over its waves)
     int split_wgs;           // > 0: the main kernel's items in the split schedule (then all of them)
+    bool two_runs = false;   // the two-run form: the main kernel's loop, 128 rows per workgroup, two key runs over its waves
 };
-AttnPlan attn_plan(int B, int H, int Nq, int kv_valid, int D, int variant, bool causal);
+AttnPlan attn_plan(int B, int H, int Nq, int kv_valid, int D, int variant, bool causal, bool bias = false);
 int compute_units();        // of the current device
 int64_t attn_main_items_on(int units, int B, int H, int Nq, int kv_valid, int D, int variant);       // the plan by shape on that many compute units
 hipError_t launch_attn_short(const AttnArgs& a, hipStream_t st);
