@@ -564,24 +564,24 @@ __device__ __forceinline__ int v_tile_chunk(int slot, int chunk) {
     return D == 256 ? (chunk ^ (((slot >> 3) & 7) << 2)) : D == 128 ? (chunk ^ (((slot >> 3) & 7) << 1)) : (chunk ^ ((slot >> 3) & 7));
 }
 
-template <int D>
+template <int D, int NT = 256>
 __device__ __forceinline__ void quant_v_f16_body(
     int t, int h, int b, int tid, const uint16_t* __restrict__ v, int64_t sb, int64_t sh, int64_t sn,
     int N, int H, int64_t n_pad, const KeyMask& km, uint16_t* __restrict__ out, uint16_t* tile) {
     constexpr int CPR = D / 8;
     const uint16_t* src = v + b * sb + h * sh;
-    u32x4 raw[64 * CPR / 256];
+    u32x4 raw[64 * CPR / NT];
 #pragma unroll
-    for (int i = 0; i < 64 * CPR / 256; i++) {
-        const int c = i * 256 + tid;
+    for (int i = 0; i < 64 * CPR / NT; i++) {
+        const int c = i * NT + tid;
         const int key = c / CPR, col = (c % CPR) * 8;
         const int row = t * 64 + key;
         raw[i] = u32x4{0u, 0u, 0u, 0u};
         if (key_kept(row, N, km)) raw[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)row * sn + col);
     }
 #pragma unroll
-    for (int i = 0; i < 64 * CPR / 256; i++) {
-        const int c = i * 256 + tid;
+    for (int i = 0; i < 64 * CPR / NT; i++) {
+        const int c = i * NT + tid;
         const int key = c / CPR, chunk = c % CPR;
         float x[8];
         unpack8(raw[i], x);
@@ -598,8 +598,8 @@ __device__ __forceinline__ void quant_v_f16_body(
     // work item = (channel pair, 8 consecutive slots): eight dword reads, two 16-byte stores
     const uint32_t* tile32 = reinterpret_cast<const uint32_t*>(tile);
 #pragma unroll
-    for (int i = 0; i < (D / 2) * 8 / 256; i++) {
-        const int c = i * 256 + tid;
+    for (int i = 0; i < (D / 2) * 8 / NT; i++) {
+        const int c = i * NT + tid;
         const int dp = c >> 3, s0 = (c & 7) * 8;            // channels 2*dp, 2*dp+1
         uint32_t w[8];
 #pragma unroll
@@ -950,13 +950,16 @@ hipError_t launch_stats_final(const FinalArgs& a, hipStream_t st) {
 // ---------------------------------------------------------------------------
 // Launch 3: Q blocks, K blocks and (e4m3 variant) V tiles as workgroup roles.
 // ---------------------------------------------------------------------------
-// Threads per workgroup (512 at 128 channels, i.e. fewer registers and more waves per SIMD, measured slower).
-template <int D, int PRE> constexpr int quant_threads() { return 256; }
+// Threads per workgroup.  At 256 channels a Q block of 128 rows is 128 elements to each of 256 threads, twice what it is at
+// 128, and its chain is what the launch lasts; with 512 the call takes, us, [1,1153,18,256] 52.2 -> 49.3, e4m3 69.0 -> 65.8,
+// [1,4608,18,256] 346 -> 337, [2,300,30,256] 39.5 -> 36.7.  (512 at 128 channels, i.e. fewer registers and more waves per
+// SIMD, measured slower; so did rows requested ahead of FIN's sums, whose registers halve the waves: [1,1153,24,128] 36.1 -> 41.6.)
+template <int D, int PRE> constexpr int quant_threads() { return D > 128 ? 512 : 256; }
 
 // FIN: launch 2 is left out — every workgroup adds up the group results it needs for itself (the same additions,
 // so the same bits), the first of a head's K and V workgroups also leave them for later launches.
 template <int D, int PRE, bool FIN>
-__global__ __launch_bounds__(256) void quant_kernel(QuantArgs a, FinalArgs f) {
+__global__ __launch_bounds__((quant_threads<D, PRE>())) void quant_kernel(QuantArgs a, FinalArgs f) {
     constexpr int NT = quant_threads<D, PRE>();
     union Smem {
         float red[NT / 64];
@@ -1009,7 +1012,7 @@ __global__ __launch_bounds__(256) void quant_kernel(QuantArgs a, FinalArgs f) {
         else SAGE_K(32);
 #undef SAGE_K
     } else if (a.v16 != nullptr) {
-        quant_v_f16_body<D>(r - a.nq_blk - a.nk_blk, h, b, threadIdx.x, a.v.p, a.v.sb, a.v.sh, a.v.sn, a.Nkv, a.H, a.nkv_pad, a.km, a.v16, sm.tile16);
+        quant_v_f16_body<D, NT>(r - a.nq_blk - a.nk_blk, h, b, threadIdx.x, a.v.p, a.v.sb, a.v.sh, a.v.sn, a.Nkv, a.H, a.nkv_pad, a.km, a.v16, sm.tile16);
     } else {
         quant_v_fp8_body<D, NT>(r - a.nq_blk - a.nk_blk, h, b, threadIdx.x, a.v.p, a.v.sb, a.v.sh, a.v.sn, a.Nkv, a.H, a.nkv_pad, a.km,
                             FIN ? s_fin[0] : a.vscale + (int64_t)bh * D, a.v8, sm.tile8);
