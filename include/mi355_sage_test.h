@@ -33,7 +33,8 @@ int mi355_sage_attn_split_rule(int B, int H, int N_q, int N_kv, int D, int varia
 /* The short form of the attention kernel (32 or 64 query rows per workgroup, keys split over its
  * waves).  mode 0: by shape (default); -1: never; 8 or 4: always, with that many key runs per row
  * block (head dim 256: always 4); 2: the two-run form of the main kernel instead (128 rows, the keys split over two halves
- * of the waves), where it exists (not at head dim 256, under a bias with e4m3, or past 32768 keys).  2, 4 and 8 take
+ * of the waves), where it exists (not at head dim 256, under a bias with e4m3, or past 32768 keys); 3: the main kernel in
+ * workgroups of four waves, where they exist (not under any bias either).  2, 3, 4 and 8 take
  * precedence over the switch above, which otherwise keeps the short and the two-run form out when it is set.  Returns 0, or -1 for
  * a mode outside these. */
 int mi355_sage_set_attn_short(int mode);

@@ -424,7 +424,7 @@ int sdpa_impl(const void* Q, const void* K, const void* V, void* O, void* Stats,
     }
     a.main_items = plan.main_items;
     a.short_kw = plan.short_kw;
-    a.two_runs = plan.two_runs;
+    a.two_runs = plan.two_runs; a.four_waves = plan.four_waves;
     a.split_wgs = plan.split_wgs;
     if (a.split_wgs > 0) {
         if (attn_split_bytes(a.split_wgs, D) <= attn_split_bytes(attn_split_rule(B, H, N_q, kv, D, variant), D)) a.split = ws + c.split;
@@ -784,7 +784,7 @@ int mi355_sage_attn_fwd(const void* q8, const void* qscale, int blkq, const void
     // Same scheduling, hence the same bits, as the one-shot calls: shapes that are split over a
     // fixed number of workgroups need hand-over slots, kept per (device, stream) by the library.
     const AttnPlan plan = attn_plan(B, H, N_q, kv_valid, D, variant, false);
-    a.main_items = plan.main_items; a.short_kw = plan.short_kw; a.split_wgs = plan.split_wgs; a.two_runs = plan.two_runs;
+    a.main_items = plan.main_items; a.short_kw = plan.short_kw; a.split_wgs = plan.split_wgs; a.two_runs = plan.two_runs; a.four_waves = plan.four_waves;
     std::lock_guard<std::mutex> together(launch_mutex(static_cast<hipStream_t>(stream)));
     const size_t split_bytes = attn_split_bytes(a.split_wgs, D);
     if (split_bytes > 0 && (rc = internal_workspace(g_split_ws, split_bytes, static_cast<hipStream_t>(stream), &a.split))) return rc;
@@ -809,7 +809,7 @@ int mi355_sage_attn_fwd_q16(const void* Q, const int64_t* q_strides, int64_t q_o
     AttnArgs a{};
     const AttnPlan plan = attn_plan(B, H, N_q, kv_valid, D, variant, false);
     if (plan.main_items > 0 && attn_split_workgroups(B, H, N_q, kv_valid, D, variant) > 0) return MI355_SAGE_EUNSUPPORTED;
-    a.main_items = plan.main_items; a.short_kw = plan.short_kw; a.two_runs = plan.two_runs;
+    a.main_items = plan.main_items; a.short_kw = plan.short_kw; a.two_runs = plan.two_runs; a.four_waves = plan.four_waves;
     const View q = make_view(Q, q_strides, q_off);
     a.q_src = q.p; a.qsb = q.sb; a.qsh = q.sh; a.qsn = q.sn; a.qmul = static_cast<const float*>(qmul); a.blkq = blkq;
     a.k8 = static_cast<const int8_t*>(k8); a.kscale = static_cast<const float*>(kscale); a.blkk = blkk;
@@ -838,7 +838,7 @@ int mi355_sage_set_attn_split(int mode) {
 }
 
 int mi355_sage_set_attn_short(int mode) {
-    if (mode != -1 && mode != 0 && mode != 2 && mode != 4 && mode != 8) return MI355_SAGE_EINVAL;
+    if (mode != -1 && mode != 0 && mode != 2 && mode != 3 && mode != 4 && mode != 8) return MI355_SAGE_EINVAL;
     attn_short_override(mode);
     return MI355_SAGE_OK;
 }

@@ -68,8 +68,9 @@ static __device__ unsigned int g_split_faults;
 // -> 473.9, [1,2304,18,256] 165.0 -> 162.8).
 // KW 2: the two halves of a workgroup's waves split the KEYS of 128 query rows and merge their results at the end (the
 // two-run form, see attn_plan).
-template <int D, int VARIANT, bool STATS, bool ADDMASK, bool SPLIT, bool RANGE = false, bool QF = false, int KW = 1>
-__global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
+// WAVES 4: workgroups of four waves, 128 query rows, two to a compute unit (see attn_plan).
+template <int D, int VARIANT, bool STATS, bool ADDMASK, bool SPLIT, bool RANGE = false, bool QF = false, int KW = 1, int WAVES = (D > 128 ? 4 : 8)>
+__global__ __launch_bounds__(WAVES * 64, D <= 128 ? 2 : 1) void sage_attn_kernel(
     const int8_t* __restrict__ q8, const float* __restrict__ qscale, int blkq,
     const uint16_t* __restrict__ q_src, int64_t qsb, int64_t qsh, int64_t qsn, const float* __restrict__ qmul,
     const int8_t* __restrict__ k8, const float* __restrict__ kscale, int blkk,
@@ -91,7 +92,9 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     constexpr int V_BYTES = D * TK * VB;                // V^T tile (two runs of e4m3: two tiles of the layout, one behind the other)
     // 256 channels: the output accumulators alone take 128 registers per lane, so a wave gets a SIMD
     // to itself (up to 512 registers) and a workgroup is 4 waves = 128 query rows.
-    constexpr int NW = D > 128 ? 4 : 8;                 // waves per workgroup
+    constexpr int NW = WAVES;                           // waves per workgroup
+    constexpr bool PAIRED = D <= 128 && WAVES == 4;     // half of a compute unit's LDS
+    static_assert(!PAIRED || (KW == 1 && !ADDMASK && !SPLIT), "four waves: whole items");
     constexpr int THREADS = NW * 64;
     constexpr int RG = NW / KW;                         // 32-row groups of a workgroup
     constexpr int ROWS_WG = RG * 32;                    // query rows per workgroup
@@ -99,7 +102,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
     constexpr int K_CH = (K_NCH + NW - 1) / NW;         // copies per wave (short tiles: some waves repeat a copy)
     constexpr int V_CH = (V_NCH + NW - 1) / NW;
     // Tile copies run this many iterations ahead (LDS: 160 KiB, of which a tile of 256 channels takes 48 with fp16 V).
-    constexpr int LEAD = D > 128 && VARIANT == 0 ? 1 : 2;
+    constexpr int LEAD = (D > 128 || (PAIRED && D == 128)) && VARIANT == 0 ? 1 : 2;
     // ring depths: the tile in use, LEAD tiles published or in flight, and the slot the next copy
     // goes to — for K the tile whose scores are being computed is t+1, for V^T the tile in use is t-1.
     constexpr int NSK = LEAD + 2, NSV = LEAD + 2;
@@ -118,10 +121,13 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
 
     __shared__ __attribute__((aligned(1024))) uint8_t lds_k[NSK][K_BYTES];
     __shared__ __attribute__((aligned(1024))) uint8_t lds_v[NSV][V_BYTES];
-    __shared__ __attribute__((aligned(16))) float lds_ks[(KW == 1 ? max_keys(D) : kTwoRunKeys) / 32 + (KS_OFF > 0 ? 4 : 0)];
+    __shared__ __attribute__((aligned(16))) float lds_ks[(KW == 1 && !PAIRED ? max_keys(D) : kTwoRunKeys) / 32 + (KS_OFF > 0 ? 4 : 0)];
     __shared__ __attribute__((aligned(16))) uint8_t lds_bias[ADDMASK ? NW : 1][ADDMASK ? BiasStage::BYTES : 16];
+    // QF: the codes turn into fragments in the V^T slots that the first copies do not go to, or where those do not hold
+    // them in a region of their own
+    constexpr bool Q_IN_V = (NSV - LEAD) * V_BYTES >= NW * 32 * D;
     __shared__ float lds_qmax[QF ? 8 : 1];              // QF: largest |pre-scaled q| of each wave's 32 rows
-    __shared__ __attribute__((aligned(16))) uint8_t lds_qc[QF && VARIANT == 1 ? RG * 32 * D : 16];      // QF: Q codes on their way into fragments
+    __shared__ __attribute__((aligned(16))) uint8_t lds_qc[QF && !Q_IN_V ? RG * 32 * D : 16];      // QF: Q codes on their way into fragments
     static_assert(!(STATS && ADDMASK), "no entry point asks for Stats under an additive mask");
     static_assert(!RANGE || (!ADDMASK && !SPLIT), "no entry point masks a range under an additive mask; the split schedule tests every step");
     constexpr bool MASKED = RANGE || SPLIT;             // mask_lo .. mask_hi may hold keys (otherwise the launcher has seen that it does not)
@@ -450,9 +456,7 @@ __global__ __launch_bounds__(D > 128 ? 256 : 512) void sage_attn_kernel(
         const float sc = am > 0.0f ? am / 127.0f : 1.0f;
         const bool fast = sc >= 0x1p-100f && sc <= 0x1p100f;
         const float rinv = 1.0f / sc;
-        // fp16 variant: the V^T slots that the first copies do not go to; e4m3: a region of its own
-        uint8_t* qs = VARIANT == 0 ? &lds_v[LEAD][0] + wave * 32 * D : &lds_qc[0] + rg * 32 * D;
-        static_assert(VARIANT != 0 || !QF || (NSV - LEAD) * V_BYTES >= NW * 32 * D, "Q codes must fit the idle V^T slots");
+        uint8_t* qs = Q_IN_V ? &lds_v[LEAD][0] + wave * 32 * D : &lds_qc[0] + rg * 32 * D;
 #pragma unroll
         for (int i = 0; i < Q_NI; i++) {
             float x[8];
@@ -1125,13 +1129,15 @@ __global__ void split_clear_kernel(int* flags, int n) {
 template <int D, int VARIANT>
 static hipError_t launch_attn_dv(const AttnArgs& a, bool two_runs, hipStream_t st) {
     constexpr int kThreads = D > 128 ? 256 : 512;             // 32 query rows per wave
-    const int rows = kThreads / 2 / (two_runs ? 2 : 1);
+    const bool four = D <= 128 && a.four_waves && !two_runs;
+    const int rows = kThreads / 2 / (two_runs || four ? 2 : 1);
     // (behind row tiles of the main kernel: two pieces to each of them, the last of which may be empty)
     const int n_qtiles = two_runs && a.main_items > 0 ? 2 * ((a.Nq + kThreads / 2 - 1) / (kThreads / 2)) : (a.Nq + rows - 1) / rows;
     const int64_t first = two_runs ? 2 * a.main_items : 0;
-    const int64_t total = two_runs ? (int64_t)n_qtiles * a.B * a.H - first : a.main_items;
+    const int64_t total = two_runs || four ? (int64_t)n_qtiles * a.B * a.H - first : a.main_items;
     if (total <= 0 || first + total > 0x7FFFFFFF || first + total > (int64_t)n_qtiles * a.B * a.H) return hipErrorInvalidValue;
     if (two_runs && (D > 128 || a.short_kw > 0 || a.split_wgs > 0 || a.nkv_pad > kTwoRunKeys || (VARIANT == 1 && a.amask != nullptr))) return hipErrorInvalidValue;
+    if (four && (a.amask != nullptr || a.two_runs || a.short_kw > 0 || a.split_wgs > 0 || a.nkv_pad > kTwoRunKeys)) return hipErrorInvalidValue;
     const int split = (D <= 128 && VARIANT == 0 && !a.causal) ? a.split_wgs : 0;
     int* flags = nullptr;
     float* part = nullptr;
@@ -1142,10 +1148,10 @@ static hipError_t launch_attn_dv(const AttnArgs& a, bool two_runs, hipStream_t s
         // (a kernel, not a memset: the call may be recorded into a graph)
         hipLaunchKernelGGL(split_clear_kernel, dim3(1), dim3(256), 0, st, flags, split);
     }
-    dim3 grid((unsigned)(split > 0 ? split : total)), block(kThreads);
+    dim3 grid((unsigned)(split > 0 ? split : total)), block(four ? 256 : kThreads);
     const bool range = a.km.hi > a.km.lo;
-#define SAGE_LAUNCH_ATTN2(STATS, ADDMASK, SPLIT, RANGE, KW)                                                              \
-    hipLaunchKernelGGL((sage_attn_kernel<D, VARIANT, STATS, ADDMASK, SPLIT, RANGE, false, KW>), grid, block, 0, st, a.q8, a.qscale, a.blkq, \
+#define SAGE_LAUNCH_ATTN2(STATS, ADDMASK, SPLIT, RANGE, ...)                                                             \
+    hipLaunchKernelGGL((sage_attn_kernel<D, VARIANT, STATS, ADDMASK, SPLIT, RANGE, false, __VA_ARGS__>), grid, block, 0, st, a.q8, a.qscale, a.blkq, \
                        a.q_src, a.qsb, a.qsh, a.qsn, a.qmul, a.k8, a.kscale, a.blkk, (const uint8_t*)a.vq, a.vscale, a.qshift, a.H, a.Nq, a.kv_valid,          \
                        a.km.lo, a.km.hi, a.causal, a.nq_pad, a.nkv_pad, a.o, a.osb, a.osh, a.osn, a.stats, n_qtiles, (int)first,   \
                        (int)total, a.amask, a.amb, a.amh, a.amn, split >> 3, part, flags, g_split_wait.load())
@@ -1161,6 +1167,10 @@ static hipError_t launch_attn_dv(const AttnArgs& a, bool two_runs, hipStream_t s
             if (two_runs) { SAGE_LAUNCH_ATTN2(STATS, ADDMASK, false, false, 2); break; }       \
         }                                                                              \
         if constexpr (!ADDMASK) {                                                      \
+            if constexpr (D <= 128) {                                                  \
+                if (range && four) { SAGE_LAUNCH_ATTN2(STATS, ADDMASK, false, true, 1, 4); break; }      \
+                if (four) { SAGE_LAUNCH_ATTN2(STATS, ADDMASK, false, false, 1, 4); break; }      \
+            }                                                                          \
             if (range) { SAGE_LAUNCH_ATTN2(STATS, ADDMASK, false, true, 1); break; }      \
         }                                                                              \
         SAGE_LAUNCH_ATTN2(STATS, ADDMASK, false, false, 1);                            \
@@ -1169,16 +1179,20 @@ static hipError_t launch_attn_dv(const AttnArgs& a, bool two_runs, hipStream_t s
         // Q encoded by the kernel: the plain forward only
         if constexpr (D <= 128) {
             if (a.amask != nullptr || a.stats != nullptr || split > 0 || a.qmul == nullptr) return hipErrorInvalidValue;
-#define SAGE_LAUNCH_ATTN_QF(RANGE, KW)                                                                                          \
-    hipLaunchKernelGGL((sage_attn_kernel<D, VARIANT, false, false, false, RANGE, true, KW>), grid, block, 0, st, nullptr, nullptr, a.blkq, \
+#define SAGE_LAUNCH_ATTN_QF(RANGE, ...)                                                                                         \
+    hipLaunchKernelGGL((sage_attn_kernel<D, VARIANT, false, false, false, RANGE, true, __VA_ARGS__>), grid, block, 0, st, nullptr, nullptr, a.blkq, \
                        a.q_src, a.qsb, a.qsh, a.qsn, a.qmul, a.k8, a.kscale, a.blkk, (const uint8_t*)a.vq, a.vscale, nullptr,  \
                        a.H, a.Nq, a.kv_valid, a.km.lo, a.km.hi, a.causal, a.nq_pad, a.nkv_pad, a.o, a.osb, a.osh, a.osn, nullptr, \
                        n_qtiles, (int)first, (int)total, nullptr, 0, 0, 0, 0, nullptr, nullptr, g_split_wait.load())
             if (range) {
                 if (two_runs) SAGE_LAUNCH_ATTN_QF(true, 2);
+                else if (four) SAGE_LAUNCH_ATTN_QF(true, 1, 4);
                 else SAGE_LAUNCH_ATTN_QF(true, 1);
-            } else if (two_runs) SAGE_LAUNCH_ATTN_QF(false, 2);
-            else SAGE_LAUNCH_ATTN_QF(false, 1);
+            } else {
+                if (two_runs) SAGE_LAUNCH_ATTN_QF(false, 2);
+                else if (four) SAGE_LAUNCH_ATTN_QF(false, 1, 4);
+                else SAGE_LAUNCH_ATTN_QF(false, 1);
+            }
 #undef SAGE_LAUNCH_ATTN_QF
         } else {
             return hipErrorInvalidValue;

@@ -472,6 +472,11 @@ hipError_t launch_attn_short(const AttnArgs& a, hipStream_t st) {
 // [1,1153,24,128] 55.0 -> 45.0.  Past about 128 row tiles its workgroups take a second round and the main kernel is ahead
 // ([1,1322,30,128] 47 against 58); below 40 to 60 the short form is (eight runs: [1,256,30,128] 16.6 against 18.4).
 //
+// The same with workgroups of four waves, 128 rows and half of a compute unit's LDS: two share a unit, one's rows in and
+// out run beside the other's products, and a last round is nearer full.  The waves copy every tile twice per unit, which is
+// what keeps it out of one round and out of long key sequences ([1,4608,24,128] 215 -> 231 us).  [1,3792 x 341,40,128] 56.7 ->
+// 49.1, [2,6224 x 63,30,64] 44.6 -> 36.2, [2,775,40,64] 46.2 -> 38.3, [1,2379,40,128] 123.8 -> 118.9; same bits.
+//
 // A problem of some rounds and a bit more takes two: the main kernel does the full rounds and another form what is left,
 // spread over the whole chip, instead of one more round that is nearly empty (short form, 264 items of 32 key tiles, 128
 // channels: 84 -> 66 us; of 64 channels 61 -> 43; by earlier forms of both).
@@ -495,10 +500,14 @@ constexpr FormCost kNoForm{1e9f, 0.0f, 0.0f, 0.0f, 0.0f};
 // form it cost 3 to 6 % on average.
 static const FormCost kCost[2][2][FORMS] = {
     {{{6.00f, 1.70f, 0.70f, 0.00f, 0.03f}, {5.94f, 2.18f, 0.46f, 0.56f, 0.02f}, {4.97f, 2.18f, 0.53f, 0.18f, 0.26f}, {5.18f, 1.40f, 0.40f, 0.00f, 0.25f}},
-     {{0.00f, 5.53f, 0.57f, 3.88f, 0.00f}, {1.57f, 5.08f, 0.26f, 0.81f, 0.08f}, {0.45f, 5.44f, 0.72f, 0.00f, 0.07f}, {1.33f, 4.41f, 0.58f, 0.00f, 0.12f}}},
+     {{0.30f, 5.53f, 0.57f, 3.88f, 0.00f}, {1.87f, 5.08f, 0.26f, 0.81f, 0.08f}, {0.45f, 5.44f, 0.72f, 0.00f, 0.07f}, {1.33f, 4.41f, 0.58f, 0.00f, 0.12f}}},
     {{{0.00f, 8.33f, 0.68f, 10.04f, 0.00f}, {3.91f, 5.03f, 0.35f, 5.68f, 0.02f}, {3.16f, 6.96f, 0.32f, 0.00f, 0.70f}, {3.24f, 5.57f, 0.44f, 0.00f, 0.61f}},
      {{0.00f, 6.65f, 0.72f, 9.30f, 0.00f}, {1.82f, 6.43f, 0.35f, 3.58f, 0.05f}, {0.40f, 6.76f, 0.88f, 0.21f, 0.34f}, {0.80f, 5.48f, 1.06f, 0.00f, 0.17f}}},
 };
+// The main kernel in workgroups of four waves, two to a compute unit (rounds and fill count two of them per unit), against
+// the figures above, up to 3072 keys: 120 calls each, chosen where it is ahead it takes 1.2 to 2.5 % off them on average.
+static const FormCost kCostFour[2][2] = {{{6.06f, 1.67f, 0.53f, 0.00f, 0.00f}, {1.26f, 4.06f, 0.37f, 1.06f, 0.60f}},
+                                         {{1.29f, 7.39f, 0.73f, 7.76f, 0.17f}, {2.29f, 4.29f, 0.72f, 6.77f, 0.25f}}};
 // Under an additive bias, fp16 P.V (50 calls of 128 to 2304 tokens at 64 channels, 110 at 128: 0.1 % and nothing).
 static const FormCost kCostBias[2][FORMS] = {
     {{0.00f, 7.38f, 1.37f, 19.88f, 0.04f}, {4.24f, 3.73f, 0.78f, 11.53f, 0.00f}, {8.78f, 0.70f, 0.52f, 5.33f, 0.71f}, {7.37f, 1.30f, 0.00f, 2.40f, 1.24f}},
@@ -572,7 +581,13 @@ static AttnPlan plan_by_shape(int units, int B, int H, int Nq, int kv_valid, int
     const float launch = d == 0 && v == 0 ? 0.0f : 3.0f;
     const bool two_runs = D <= 128 && pad_to(kv_valid, kPadKV) <= kTwoRunKeys && !(bias && v == 1);
     if (D <= 128 && bias && v == 0) return choose(kCostBias[d], 0.0f, 3.0f, two_runs).p;
-    if (D <= 128 && !bias && tiles <= 48) return choose(kCost[d][v], 0.0f, launch, two_runs).p;
+    if (D <= 128 && !bias && tiles <= 48) {
+        const Choice best = choose(kCost[d][v], 0.0f, launch, two_runs);
+        // Four waves: past a round of row tiles, but for the few that a second launch takes better (16 in 256).
+        const bool over = items > units && (tiles <= 4 || (items - whole) * 16 > units || items == whole);
+        const float four = kCostFour[d][v].of(bh * ((Nq + 127) / 128), tiles, 2 * units);
+        return over && four < best.t ? AttnPlan{items, 0, 0, false, true} : best.p;
+    }
     return choose(by_length, q_cost, 0.0f, two_runs).p;
 }
 
@@ -605,7 +620,8 @@ AttnPlan attn_plan(int B, int H, int Nq, int kv_valid, int D, int variant, bool 
     const int mode = g_short_mode.load(), rows = D > 128 ? 128 : 256;
     const bool two_runs_fit = D <= 128 && pad_to(kv_valid, kPadKV) <= kTwoRunKeys && !(bias && variant != 0);
     if (mode == 2 && two_runs_fit) return AttnPlan{0, 0, 0, true};
-    if (mode == 2) return AttnPlan{(int64_t)B * H * ((Nq + rows - 1) / rows), 0, 0};
+    if (mode == 3 && two_runs_fit && !bias) return AttnPlan{(int64_t)B * H * ((Nq + rows - 1) / rows), 0, 0, false, true};
+    if (mode == 2 || mode == 3) return AttnPlan{(int64_t)B * H * ((Nq + rows - 1) / rows), 0, 0};
     if (mode > 0) return AttnPlan{0, D == 256 ? 4 : mode, 0};
     const int split = causal ? 0 : attn_split_workgroups(B, H, Nq, kv_valid, D, variant);
     if (mode < 0 || attn_split_override_mode() != 0)      // (a schedule of the main kernel was asked for)

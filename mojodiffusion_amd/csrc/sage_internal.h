@@ -171,6 +171,7 @@ struct AttnArgs {
     int64_t main_items;
     int short_kw;            // key runs per row block in the short form
     bool two_runs;           // the rest in the main kernel's two-run form
+    bool four_waves;         // the main kernel with workgroups of four waves (everything)
     int split_wgs;           // workgroups of the main kernel's split schedule, 0: one workgroup per item
     void* split;             // attn_split_bytes(split_wgs, D) bytes, 256-byte aligned (null when 0)
 };
@@ -181,6 +182,7 @@ struct AttnPlan {
     int short_kw;            // key runs of the short form (32 or 64 rows per workgroup, keys split over its waves)
     int split_wgs;           // > 0: the main kernel's items in the split schedule (then all of them)
     bool two_runs = false;   // the two-run form: the main kernel's loop, 128 rows per workgroup, two key runs over its waves
+    bool four_waves = false; // the main kernel's items (then all of them) in workgroups of four waves, two to a compute unit
 };
 AttnPlan attn_plan(int B, int H, int Nq, int kv_valid, int D, int variant, bool causal, bool bias = false);
 int compute_units();        // of the current device
