@@ -379,6 +379,24 @@ int sdpa_impl(const void* Q, const void* K, const void* V, void* O, void* Stats,
     }
     const bool q_in_kernel = Stats == nullptr && mask.add == nullptr && pre.q.gain == nullptr && (D <= 128 || plan.main_items == 0) &&
                              plan.split_wgs == 0 && !q_in_encoders;
+    if (pre.q.gain == nullptr && attn_fused_rule(plan, B, H, N_q, kv, D, variant, blkq, blkk)) {
+        const View q = make_view(Q, qs, q_off);
+        AttnArgs a{};
+        a.blkq = blkq; a.blkk = blkk; a.variant = variant; a.km = km;
+        a.B = B; a.H = H; a.Nq = N_q; a.Nkv = kv; a.kv_valid = kv; a.D = D;
+        a.causal = causal ? 1 : 0;
+        a.nq_pad = pad_to(N_q, kTileQ); a.nkv_pad = pad_to(kv, kPadKV);
+        a.o = static_cast<uint16_t*>(O) + o_off; a.osb = os[0]; a.osh = os[1]; a.osn = os[2];
+        a.stats = Stats ? static_cast<float*>(Stats) + stats_off : nullptr;
+        if (mask.add != nullptr) {
+            a.amask = static_cast<const uint16_t*>(mask.add) + mask.add_off;
+            a.amb = mask.add_strides[0]; a.amh = mask.add_strides[1]; a.amn = mask.add_strides[2];
+        }
+        a.q_src = q.p; a.qsb = q.sb; a.qsh = q.sh; a.qsn = q.sn;
+        a.short_kw = plan.short_kw;
+        SAGE_HIP(launch_attn_fused(a, FuseArgs{make_view(K, ks, k_off), make_view(V, vs, v_off), kept, k_flags, cmul_of(scale)}, st));
+        return MI355_SAGE_OK;
+    }
     QuantOut o{};
     o.q8 = q_in_kernel ? nullptr : reinterpret_cast<int8_t*>(ws + c.q8);
     o.k8 = reinterpret_cast<int8_t*>(ws + c.k8);

@@ -19,20 +19,207 @@
 // workgroups start to fill the chip.
 #include "sage_attn_common.h"
 #include "sage_grid.h"
+#include "sage_quant_common.h"
 
 #include <algorithm>
 #include <atomic>
 
 namespace sage {
 
+static std::atomic<int> g_short_mode{0};       // see attn_short_override
 template <int D> constexpr int kMainRows = D > 128 ? 128 : 256;               // rows per workgroup of the main kernel
 template <int D> constexpr int short_waves() { return D > 128 ? 4 : 8; }      // 256 channels: a wave needs a SIMD's registers
 
-// (64 channels, fp16: two workgroups share a compute unit, which takes 128 registers at most.  Under a bias that is 10 %
-// of a call whose workgroups are more than the compute units: [1,700,24,64] 31.1 us at 146 registers, 27.7 at 128.)
-template <int D, int VARIANT, int KW, bool QF, bool ADDMASK>
-__global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 : 1) void sage_attn_short_kernel(AttnArgs a, int n_rtiles, int item0, int total_wg) {
+// ---- the whole call in one launch -----------------------------------------------------------------
+// At 256 keys (512 of 64 channels) the quantizers' launch and this one last 7 to 9 us each, of which 2.5 are its start and
+// end, the rest latencies of loads and barriers and a chain of little work per wave.  Here every workgroup quantizes
+// its head's keys and values for itself, into LDS, where the form above keeps the pieces its waves copy in: the
+// statistics by the same leaves, groups and order, the codes by the same arithmetic, so the same bits.  All eight waves
+// share either: K as sixteen tokens of four channels to a thread, which holds them from the sums to the codes; V as four neighbouring
+// keys of eight channels to a thread, one write per channel in the slots' order.  (K by four of the waves and V by the
+// others was 14.3 us at [1,256,30,128], 13.4 so.)  One-shot, two launches -> one, us: [1,256,30,128] 16.5 -> 13.4, [1,64,4,128]
+// 13.9 -> 11.2, [1,512,8,64] 13.7 -> 12.7, with Stats [1,256,30,128] 19.0 -> 13.6, with a bias 17.6 -> 14.0.
+// (fp16 P.V only: with the e4m3 maxima and quotients in it the same was 16.0 us against 14.8 in two launches.)
+template <int D> struct FuseLds {
+    static constexpr int KEYS = fused_keys(D), CPR = D / 8, LD = D + CPR;
+    static constexpr int K8 = KEYS * D, V = KEYS * D * 2;
+    static constexpr int LEAVES = KEYS / 16, LEAF = K8 + V, LEAF_BYTES = LEAVES * LD * 16;       // sums (double), minima, maxima
+    static constexpr int BYTES = LEAF + LEAF_BYTES;
+    static_assert(LEAVES * (D / 4) == 512 && KEYS / 4 * CPR == 2 * 512, "K: a leaf of four channels to a thread; V: two quads of keys");
+};
+template <int D> struct FuseStats { float mean[D], kmul[D], qmul[D], ks[fused_keys(D) / 64], kmax[8]; };
+
+template <int D>
+struct FuseQuant {
+    using L = FuseLds<D>;
+    static constexpr int CPR = L::CPR, LD = L::LD, WL = D == 128 ? 2 : 1;      // waves that share four leaves (one scale block)
+    float v[kLeaf][4];                                  // the K values of this thread's leaf
+    bool live;                                          // (waves whose 64 tokens are past the end only leave empty leaves: no step reads their codes)
+    // this thread's leaf and first of four channels (K); first quad of keys and first of eight channels (V)
+    __device__ static __forceinline__ int leaf(int tid) { return (tid >> 6) / WL * 4 + ((tid & 63) >> 4); }
+    __device__ static __forceinline__ int kcol(int tid) { return ((tid >> 6) % WL * 16 + (tid & 15)) * 4; }
+    __device__ static __forceinline__ int quad(int tid, int i) { return tid / CPR + i * (512 / CPR); }
+    __device__ static __forceinline__ int vcol(int tid) { return tid % CPR * 8; }
+
+    // Statistics, V^T, K values and their largest per wave.  (Meets two barriers.)
+    __device__ __forceinline__ void values(const FuseArgs& f, int b, int h, int N, const KeyMask& km, int tid, uint8_t* raw, FuseStats<D>& st) {
+        double* leafsum = reinterpret_cast<double*>(raw + L::LEAF);
+        float* leafmin = reinterpret_cast<float*>(raw + L::LEAF + L::LEAVES * LD * 8);
+        float* leafmax = leafmin + L::LEAVES * LD;
+        const int s0 = leaf(tid) * kLeaf, c4 = kcol(tid), c8 = vcol(tid);
+        // (every token of the wave's leaves counts: the common case)
+        live = __any(s0 < N);
+        const bool all_kept = __all(s0 + kLeaf <= N && !(s0 < km.hi && s0 + kLeaf > km.lo));
+        u32x2 w[kLeaf];
+        u32x4 wv[2][4];                                 // [item][key of the quad]
+        {
+            // (tokens past the end repeat the last; what does not count becomes zero)
+            const uint16_t* src = f.k.p + b * f.k.sb + h * f.k.sh + c4;
+#pragma unroll
+            for (int i = 0; i < kLeaf; i++) w[i] = *reinterpret_cast<const u32x2*>(src + (int64_t)min(s0 + i, N - 1) * f.k.sn);
+            const uint16_t* vsrc = f.v.p + b * f.v.sb + h * f.v.sh + c8;
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) wv[i][r] = *reinterpret_cast<const u32x4*>(vsrc + (int64_t)min(quad(tid, i) * 4 + r, N - 1) * f.v.sn);
+            if (!all_kept) {
+#pragma unroll
+                for (int i = 0; i < kLeaf; i++)
+                    if (!key_kept(s0 + i, N, km)) w[i] = u32x2{0u, 0u};
+            }
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (!key_kept(quad(tid, i) * 4 + r, N, km)) wv[i][r] = u32x4{0u, 0u, 0u, 0u};
+        }
+        double acc[4] = {0, 0, 0, 0};
+        float mn[4], mx[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) { mn[e] = INFINITY; mx[e] = -INFINITY; }
+        if (live) {
+#pragma unroll
+        for (int i = 0; i < kLeaf; i++) {
+            v[i][0] = bf16_lo(w[i].x); v[i][1] = bf16_hi(w[i].x);
+            v[i][2] = bf16_lo(w[i].y); v[i][3] = bf16_hi(w[i].y);
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[e] += (double)v[i][e];           // (tokens that do not count are +0.0)
+        }
+#pragma unroll
+        for (int i = 0; i < kLeaf; i += 2) {
+            float x[2][4];
+#pragma unroll
+            for (int r = 0; r < 2; r++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) x[r][e] = v[i + r][e];
+            if (!all_kept) {
+                // (a NaN takes no part in a minimum or maximum)
+#pragma unroll
+                for (int r = 0; r < 2; r++)
+                    if (!key_kept(s0 + i + r, N, km))
+#pragma unroll
+                        for (int e = 0; e < 4; e++) x[r][e] = __builtin_nanf("");
+            }
+            // (as instructions: fminf and fmaxf of values out of bit operations are several each, see kstats_group)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                asm("v_min3_f32 %0, %0, %1, %2" : "+v"(mn[e]) : "v"(x[0][e]), "v"(x[1][e]));
+                asm("v_max3_f32 %0, %0, %1, %2" : "+v"(mx[e]) : "v"(x[0][e]), "v"(x[1][e]));
+            }
+        }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            // (channel 8 c + e at e * D/8 + c, as in KGroupSmem)
+            const int at = leaf(tid) * LD + ((c4 + e) & 7) * CPR + (c4 >> 3);
+            leafsum[at] = acc[e];
+            leafmin[at] = mn[e];
+            leafmax[at] = mx[e];
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int key = quad(tid, i) * 4, slot = v_slot_f16(key & 31);
+            if (!__any((key & ~31) < N)) continue;      // (no step reads it)
+            uint8_t* step = raw + L::K8 + (key >> 5) * (D * 64);
+            float x[4][8];
+#pragma unroll
+            for (int r = 0; r < 4; r++) unpack8(wv[i][r], x[r]);
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const u32x2 o = {f16_pair_sat(x[0][e], x[1][e]), f16_pair_sat(x[2][e], x[3][e])};
+                *reinterpret_cast<u32x2*>(step + swz((c8 + e) * 4 + (slot >> 3)) + (slot & 7) * 2) = o;
+            }
+        }
+        __syncthreads();
+        if (tid < D) {
+            double sum = 0.0;
+            float lo = INFINITY, hi = -INFINITY;
+            for (int g = 0; g * kGroup < N; g++) {
+                double gsum = 0.0;
+#pragma unroll
+                for (int u = 0; u < 16; u++) {
+                    gsum += leafsum[(g * 16 + u) * LD + tid];
+                    lo = fminf(lo, leafmin[(g * 16 + u) * LD + tid]);
+                    hi = fmaxf(hi, leafmax[(g * 16 + u) * LD + tid]);
+                }
+                sum += gsum;
+            }
+            float mean, sd;
+            k_final(sum, lo, hi, f.kept, f.flags, mean, sd);
+            const int d = leaf_channel<D>(tid);
+            st.mean[d] = mean; st.kmul[d] = 1.0f / sd; st.qmul[d] = f.cmul * sd;
+        }
+        __syncthreads();
+        if (!live) return;
+        const v4f mu = *reinterpret_cast<const v4f*>(&st.mean[c4]), mul = *reinterpret_cast<const v4f*>(&st.kmul[c4]);
+        float am = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kLeaf; i++) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float d = v[i][e] - mu[e];
+                v[i][e] = d * mul[e];
+            }
+            if (!all_kept && !key_kept(s0 + i, N, km)) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[i][e] = 0.0f;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; e += 2) am = fmaxf(fmaxf(am, fabsf(v[i][e])), fabsf(v[i][e + 1]));
+        }
+        am = wave_max(am);
+        if ((tid & 63) == 0) st.kmax[tid >> 6] = am;
+    }
+
+    // Codes and scales.  (Behind a barrier that publishes kmax; another one publishes them.)
+    __device__ __forceinline__ void codes(int tid, uint8_t* raw, FuseStats<D>& st) {
+        if (!live) return;
+        const int s0 = leaf(tid) * kLeaf, c4 = kcol(tid), wave = tid >> 6;
+        float am = st.kmax[wave];
+        if constexpr (WL == 2) am = fmaxf(am, st.kmax[wave ^ 1]);
+        const float sc = am > 0.0f ? am / 127.0f : 1.0f;
+        if ((tid & (64 * WL - 1)) == 0) st.ks[s0 >> 6] = sc;
+        const bool fast = sc >= 0x1p-100f && sc <= 0x1p100f;
+        const float rinv = 1.0f / sc;
+#pragma unroll
+        for (int i = 0; i < kLeaf; i += 2) {
+            // (two tokens of four channels as one encoder call of eight values)
+            const float x[8] = {v[i][0], v[i][1], v[i][2], v[i][3], v[i + 1][0], v[i + 1][1], v[i + 1][2], v[i + 1][3]};
+            const u32x2 o = encode8_i8(x, sc, rinv, fast);
+#pragma unroll
+            for (int r = 0; r < 2; r++) {
+                const int key = s0 + i + r;
+                *reinterpret_cast<uint32_t*>(raw + (key >> 5) * (32 * D) + swz((key & 31) * (D / 16) + (c4 >> 4)) + (c4 & 15)) = r ? o.y : o.x;
+            }
+        }
+    }
+};
+
+// FUSE: K and V are quantized here (fz), the fields of `a` that name their codes, scales and multipliers are not read.
+template <int D, int VARIANT, int KW, bool QF, bool ADDMASK, bool FUSE>
+__device__ __forceinline__ void short_body(const AttnArgs& a, const FuseArgs& fz, int n_rtiles, int item0, int total_wg) {
     constexpr int NW = short_waves<D>();
+    static_assert(!FUSE || (QF && D <= 128 && VARIANT == 0), "one launch: Q is encoded here too");
     constexpr int R = NW / KW;                          // 32-row blocks per workgroup
     constexpr int ROWS = 32 * R;
     constexpr int KSTEPS = D / 32, DB = D / 32, CPR = D / 8;
@@ -55,7 +242,13 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
         float acc[32 * LD];
         uint8_t stride[((sizeof(Ring) > 32 * LD * 4 ? sizeof(Ring) : 32 * LD * 4) + 255) / 256 * 256];
     };
-    __shared__ __attribute__((aligned(1024))) Mem mem[NW];
+    using L = FuseLds<FUSE ? D : 128>;
+    constexpr int ACC_BYTES = NW * 32 * LD * 4, RAW = L::BYTES > ACC_BYTES ? L::BYTES : ACC_BYTES;
+    __shared__ __attribute__((aligned(1024))) Mem mem[FUSE ? 1 : NW];
+    __shared__ __attribute__((aligned(1024))) uint8_t raw[FUSE ? RAW : 16];         // FUSE: K, V^T and the statistics' leaves, then the partial outputs
+    __shared__ __attribute__((aligned(16))) FuseStats<FUSE ? D : 64> fstat;
+    __shared__ float lds_shift[FUSE ? ROWS : 1];
+    auto acc_of = [&](int w) -> float* { return FUSE ? reinterpret_cast<float*>(raw) + w * (32 * LD) : mem[FUSE ? 0 : w].acc; };
     __shared__ __attribute__((aligned(16))) uint8_t lds_q[QF ? ROWS * D : 16];      // this workgroup's Q codes
     __shared__ float lds_m[NW][32], lds_l[NW][32];
     __shared__ __attribute__((aligned(16))) float lds_qmax[8];
@@ -91,7 +284,8 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
     // ---- one step's operands: copies into the wave's own LDS region, fragments out of it
     const uint8_t* kg = reinterpret_cast<const uint8_t*>(a.k8) + (int64_t)bh * a.nkv_pad * D;
     const uint8_t* vg = static_cast<const uint8_t*>(a.vq) + (int64_t)bh * a.nkv_pad * D * VB;
-    const uint32_t k_lds = lds_addr(&mem[wave].ring.k[0]), v_lds = lds_addr(&mem[wave].ring.v[0]);
+    const uint32_t k_lds = FUSE ? lds_addr(&raw[0]) : lds_addr(&mem[FUSE ? 0 : wave].ring.k[0]);
+    const uint32_t v_lds = FUSE ? lds_addr(&raw[L::K8]) : lds_addr(&mem[FUSE ? 0 : wave].ring.v[0]);
     int vsrc[VC];
 #pragma unroll
     for (int i = 0; i < VC; i++) {
@@ -112,19 +306,19 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
         for (int i = 0; i < VC; i++) dma16(g, vsrc[i], __builtin_amdgcn_readfirstlane(v_lds + i * 1024));
     };
     typedef const __attribute__((address_space(3))) v4i* lds_v4i_ptr;
-    auto k_frag = [&](int n) -> v4i {
-        return *reinterpret_cast<lds_v4i_ptr>(k_lds + swz(((n / KSTEPS) * 32 + l32) * (D / 16) + (n % KSTEPS) * 2 + half));
+    auto k_frag = [&](int n, int hs) -> v4i {
+        return *reinterpret_cast<lds_v4i_ptr>(k_lds + (FUSE ? key_step(hs) * K_BYTES : 0) + swz(((n / KSTEPS) * 32 + l32) * (D / 16) + (n % KSTEPS) * 2 + half));
     };
     // fp16: fragment jj * DB + d = 16 keys, channels 32 d ..; e4m3: fragments 2 d, 2 d + 1 = a lane's 32 keys, channels 32 d ..
-    auto v_frag = [&](int n) -> v4i {
+    auto v_frag = [&](int n, int hs) -> v4i {
         const int d = VARIANT == 0 ? n % DB : n >> 1;
         const int c = VARIANT == 0 ? (n / DB) * 2 + half : half * 2 + (n & 1);
-        return *reinterpret_cast<lds_v4i_ptr>(v_lds + swz((d * 32 + l32) * 4 + c));
+        return *reinterpret_cast<lds_v4i_ptr>(v_lds + (FUSE ? key_step(hs) * V_BYTES : 0) + swz((d * 32 + l32) * 4 + c));
     };
     // (LDS reads issued before this have delivered: what they read may be overwritten)
     auto reads_done = [] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
     auto first_copies = [&] {
-        if (h0 < h1) {
+        if (!FUSE && h0 < h1) {
             copy_k(h0);
             copy_v(h0);
         }
@@ -169,9 +363,11 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
             own[i] = u32x4{0u, 0u, 0u, 0u};
             if (row < a.Nq) own[i] = *reinterpret_cast<const u32x4*>(qb + (int64_t)row * a.qsn + col);
         }
+        FuseQuant<FUSE ? D : 128> fq;
+        if constexpr (FUSE) fq.values(fz, b, h, a.kv_valid, a.km, tid, raw, fstat);
         float m[8];
         {
-            const float* mp = a.qmul + (int64_t)bh * D + col;
+            const float* mp = FUSE ? &fstat.qmul[col] : a.qmul + (int64_t)bh * D + col;
             const v4f m0 = *reinterpret_cast<const v4f*>(mp), m1 = *reinterpret_cast<const v4f*>(mp + 4);
 #pragma unroll
             for (int e = 0; e < 4; e++) m[e] = m0[e], m[4 + e] = m1[e];
@@ -189,6 +385,7 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
             if (lane == 0) lds_qmax[t * NW + wave] = am;
         }
         __syncthreads();
+        if constexpr (FUSE) fq.codes(tid, raw, fstat);
         // (all eight maxima in two reads and the block's picked: as a loop over them, one after the other, this was half a
         // microsecond each time it was asked)
         const int blk16 = a.blkq >> 4, blksh = a.blkq == 32 ? 5 : a.blkq == 64 ? 6 : 7;
@@ -216,17 +413,30 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
                 x[2 * e + 1] = __uint_as_float(own[i][e] & 0xFFFF0000u) * m[2 * e + 1];
             }
             *reinterpret_cast<u32x2*>(&lds_q[row * D + col]) = encode8_i8(x, sc, rinv, fast);
+            if (FUSE && a.stats != nullptr) {
+                // <pre-scaled query row, K mean>, as the Q encoder takes it: what K smoothing lowers the row's scores by
+                float dot = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    const float q = e & 1 ? __uint_as_float(own[i][e >> 1] & 0xFFFF0000u) : __uint_as_float(own[i][e >> 1] << 16);
+                    dot += (q * fz.cmul) * fstat.mean[col + e];
+                }
+#pragma unroll
+                for (int off = CPR / 2; off > 0; off >>= 1) dot += __shfl_xor(dot, off, 64);
+                if (tid % CPR == 0) lds_shift[row] = dot;
+            }
         }
         __syncthreads();
 #pragma unroll
         for (int s = 0; s < KSTEPS; s++) qf[s] = *reinterpret_cast<const v4i*>(&lds_q[(rg * 32 + l32) * D + s * 32 + half * 16]);
     }
 
-    const float* ksc = a.kscale + (int64_t)bh * (a.nkv_pad / a.blkk);
+    const float* ksc = FUSE ? &fstat.ks[0] : a.kscale + (int64_t)bh * (a.nkv_pad / a.blkk);
     const int ksh = a.blkk == 32 ? 5 : a.blkk == 64 ? 6 : 7;
     // the bias of a step is loaded while the step before it runs
     BiasStage bias[SKB];
-    uint8_t* bias_lds = &mem[wave].ring.bias[0];
+    uint8_t* bias_lds = FUSE ? &raw[L::LEAF + (ADDMASK ? wave * BiasStage::BYTES : 0)] : &mem[FUSE ? 0 : wave].ring.bias[0];
+    static_assert(!FUSE || NW * BiasStage::BYTES <= L::LEAF_BYTES, "the bias takes the leaves' place");
     BiasStage::Rows brows{};
     if (ADDMASK) brows = BiasStage::rows(a.amask + b * a.amb + h * a.amh, a.amn, row0, a.Nq - 1, lane);
     auto bias_load = [&](int hs) {
@@ -258,11 +468,11 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
 
     for (int hs = h0; hs < h1; hs++) {
         v16i s[SKB];
-        dma_wait<VC>();                                 // K of this step has landed (V^T was requested after it)
+        if constexpr (!FUSE) dma_wait<VC>();            // K of this step has landed (V^T was requested after it)
         {
             v4i kf[NK];
 #pragma unroll
-            for (int n = 0; n < NK; n++) kf[n] = k_frag(n);
+            for (int n = 0; n < NK; n++) kf[n] = k_frag(n, hs);
 #pragma unroll
             for (int kb = 0; kb < SKB; kb++)
 #pragma unroll
@@ -270,8 +480,10 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
                     s[kb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[kb * KSTEPS + st], qf[st], st == 0 ? smagic : s[kb], 0, 0, 0);
         }
         const bool more = hs + 1 < h1;
-        reads_done();
-        if (more) copy_k(hs + 1);
+        if constexpr (!FUSE) {
+            reads_done();
+            if (more) copy_k(hs + 1);
+        }
         const int key0 = key_step(hs) * SK;
         float f[SKB];           // (taken at least so large in every step: in the branch below it was 1 % slower at 256 channels)
 #pragma unroll
@@ -353,11 +565,13 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
                 else p[w] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(e[0], e[1], 0, false);
             }
         }
-        if (more) dma_wait<KC>();                       // V^T of this step (the next step's K was requested after it)
-        else dma_wait<0>();
+        if constexpr (!FUSE) {
+            if (more) dma_wait<KC>();                   // V^T of this step (the next step's K was requested after it)
+            else dma_wait<0>();
+        }
         v4i vf[NV];
 #pragma unroll
-        for (int n = 0; n < NV; n++) vf[n] = v_frag(n);
+        for (int n = 0; n < NV; n++) vf[n] = v_frag(n, hs);
         if constexpr (VARIANT == 0) {
 #pragma unroll
             for (int n = 0; n < NV; n++) {
@@ -375,8 +589,10 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
             }
             lacc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(ones8, pw, lacc, 0, 0, 0, 0, 0, 0);
         }
-        reads_done();
-        if (more) copy_v(hs + 1);
+        if constexpr (!FUSE) {
+            reads_done();
+            if (more) copy_v(hs + 1);
+        }
     }
 
     // ---- merge of the KW partial results, in LDS
@@ -389,8 +605,9 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
         lds_m[wave][l32] = m_used;
         lds_l[wave][l32] = l_row;
     }
+    if constexpr (FUSE) __syncthreads();                // (no wave reads K, V^T or the bias any more)
     {
-        float* dst = &mem[wave].acc[l32 * LD + half * 4];
+        float* dst = acc_of(wave) + l32 * LD + half * 4;
 #pragma unroll
         for (int d = 0; d < DB; d++)
 #pragma unroll
@@ -411,7 +628,8 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
 #pragma unroll
         for (int w = 0; w < KW; w++) {
             const float sc = __builtin_amdgcn_exp2f(lds_m[r * KW + w][rl] - mg);
-            const v4f y0 = *reinterpret_cast<const v4f*>(&mem[r * KW + w].acc[rl * LD + ch]), y1 = *reinterpret_cast<const v4f*>(&mem[r * KW + w].acc[rl * LD + ch + 4]);
+            const float* part = acc_of(r * KW + w) + rl * LD + ch;
+            const v4f y0 = *reinterpret_cast<const v4f*>(part), y1 = *reinterpret_cast<const v4f*>(part + 4);
             l_tot = fmaf(lds_l[r * KW + w][rl], sc, l_tot);
 #pragma unroll
             for (int e = 0; e < 4; e++) x0[e] = fmaf(y0[e], sc, x0[e]), x1[e] = fmaf(y1[e], sc, x1[e]);
@@ -426,10 +644,51 @@ __global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 
                           pack_bf16(x1[0] * inv, x1[1] * inv), pack_bf16(x1[2] * inv, x1[3] * inv)};
         *reinterpret_cast<u32x4*>(a.o + b * a.osb + h * a.osh + (int64_t)grow * a.osn + ch) = pk;
         if (a.stats != nullptr && ch == 0) {
-            const float shift = a.qshift != nullptr ? a.qshift[(int64_t)bh * a.nq_pad + grow] : 0.0f;
+            const float shift = FUSE ? lds_shift[row] : a.qshift != nullptr ? a.qshift[(int64_t)bh * a.nq_pad + grow] : 0.0f;
             a.stats[(int64_t)bh * a.Nq + grow] = (mg + __builtin_amdgcn_logf(l_tot) - Lazy<VARIANT>::log2_pscale + shift) * 0.6931471805599453f;
         }
     }
+}
+
+// (64 channels, fp16: two workgroups share a compute unit, which takes 128 registers at most.  Under a bias that is 10 %
+// of a call whose workgroups are more than the compute units: [1,700,24,64] 31.1 us at 146 registers, 27.7 at 128.)
+template <int D, int VARIANT, int KW, bool QF, bool ADDMASK>
+__global__ __launch_bounds__(short_waves<D>() * 64, D == 64 && VARIANT == 0 ? 4 : 1) void sage_attn_short_kernel(AttnArgs a, int n_rtiles, int item0, int total_wg) {
+    short_body<D, VARIANT, KW, QF, ADDMASK, false>(a, FuseArgs{}, n_rtiles, item0, total_wg);
+}
+
+template <int D, int KW, bool ADDMASK>
+__global__ __launch_bounds__(512) void sage_attn_fused_kernel(AttnArgs a, FuseArgs f, int n_rtiles, int total_wg) {
+    short_body<D, 0, KW, true, ADDMASK, true>(a, f, n_rtiles, 0, total_wg);
+}
+
+template <int D, int KW>
+static hipError_t launch_fused_dk(const AttnArgs& a, const FuseArgs& f, hipStream_t st) {
+    constexpr int ROWS = 32 * (8 / KW);
+    const int64_t n_rtiles = (a.Nq + ROWS - 1) / ROWS, total = (int64_t)a.B * a.H * n_rtiles;
+    if (total <= 0 || total > 0x7FFFFFFF || a.q_src == nullptr || a.blkk != 64 || a.variant != 0 || a.kv_valid > fused_keys(D)) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)total), block(512);
+    if (a.amask != nullptr) hipLaunchKernelGGL((sage_attn_fused_kernel<D, KW, true>), grid, block, 0, st, a, f, (int)n_rtiles, (int)total);
+    else hipLaunchKernelGGL((sage_attn_fused_kernel<D, KW, false>), grid, block, 0, st, a, f, (int)n_rtiles, (int)total);
+    return hipGetLastError();
+}
+
+hipError_t launch_attn_fused(const AttnArgs& a, const FuseArgs& f, hipStream_t st) {
+    if (a.D == 128) return a.short_kw == 8 ? launch_fused_dk<128, 8>(a, f, st) : launch_fused_dk<128, 4>(a, f, st);
+    if (a.D == 64) return a.short_kw == 8 ? launch_fused_dk<64, 8>(a, f, st) : launch_fused_dk<64, 4>(a, f, st);
+    return hipErrorInvalidValue;
+}
+
+// Where the workgroups are at most one per compute unit: each of them quantizes its head's keys again.
+static int fused_runs(int units, int B, int H, int Nq, int kv_valid, int D, int variant) {
+    if (variant != 0 || D > 128 || kv_valid > fused_keys(D)) return 0;
+    const int64_t bh = (int64_t)B * H;
+    return bh * ((Nq + 31) / 32) <= units ? 8 : bh * ((Nq + 63) / 64) <= units ? 4 : 0;
+}
+
+bool attn_fused_rule(const AttnPlan& p, int B, int H, int Nq, int kv_valid, int D, int variant, int blkq, int blkk) {
+    if (p.main_items > 0 || p.short_kw == 0 || blkk != 64 || blkq != 128 || g_short_mode.load() != 0) return false;
+    return fused_runs(compute_units(), B, H, Nq, kv_valid, D, variant) == p.short_kw;
 }
 
 template <int D, int VARIANT, int KW>
@@ -577,6 +836,7 @@ static AttnPlan plan_by_shape(int units, int B, int H, int Nq, int kv_valid, int
         kSplitCost[d][0] + kSplitCost[d][1] * (float)(items * tiles) / 256.0f < choose(by_length, q_cost, 0.0f, false).t)
         return AttnPlan{items, 0, split};
     if (short_or_main) return choose(by_length, q_cost, 0.0f, false).p;
+    if (const int runs = fused_runs(units, B, H, Nq, kv_valid, D, variant)) return AttnPlan{0, runs, 0};
     // (figures that were fitted to differences have not got what a second launch costs)
     const float launch = d == 0 && v == 0 ? 0.0f : 3.0f;
     const bool two_runs = D <= 128 && pad_to(kv_valid, kPadKV) <= kTwoRunKeys && !(bias && v == 1);
@@ -591,7 +851,7 @@ static AttnPlan plan_by_shape(int units, int B, int H, int Nq, int kv_valid, int
     return choose(by_length, q_cost, 0.0f, two_runs).p;
 }
 
-static std::atomic<int> g_short_mode{0};       // 0: by shape; -1: never; 4, 8: always, that many key runs (4 at 256 channels)
+// 0: by shape; -1: never; 4, 8: always, that many key runs (4 at 256 channels)
 void attn_short_override(int mode) { g_short_mode.store(mode); }
 
 int attn_short_rule(int B, int H, int Nq, int kv_valid, int D, int variant) {

@@ -188,6 +188,16 @@ AttnPlan attn_plan(int B, int H, int Nq, int kv_valid, int D, int variant, bool 
 int compute_units();        // of the current device
 int64_t attn_main_items_on(int units, int B, int H, int Nq, int kv_valid, int D, int variant);       // the plan by shape on that many compute units
 hipError_t launch_attn_short(const AttnArgs& a, hipStream_t st);
+// The short form with the quantizers of K and V in it: the whole call in one launch, up to this many keys (their codes stay
+// in LDS).
+__host__ __device__ constexpr int fused_keys(int D) { return D == 64 ? 512 : 256; }
+struct FuseArgs {
+    View k, v;
+    int kept, flags;         // as in FinalArgs
+    float cmul;
+};
+hipError_t launch_attn_fused(const AttnArgs& a, const FuseArgs& f, hipStream_t st);
+bool attn_fused_rule(const AttnPlan& p, int B, int H, int Nq, int kv_valid, int D, int variant, int blkq, int blkk);
 int attn_short_rule(int B, int H, int Nq, int kv_valid, int D, int variant);     // short_kw where the short form does everything by shape, else 0
 void attn_short_override(int mode);          // 0: by shape (default); -1: never; 4 or 8: always
 // Shapes whose items do not fill whole rounds of workgroups are spread evenly over a fixed number

@@ -13,43 +13,9 @@
 // round-half-to-even) and every reduction either has a fixed order (the fp64 sums) or is
 // order-free (max / min), so codes, scales and statistics are reproducible bit for bit.
 // All kernels read bf16 rows with 16-byte loads (8 channels per lane).
-#include "sage_internal.h"
-
-#include <hip/hip_fp16.h>
+#include "sage_quant_common.h"
 
 namespace sage {
-
-typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
-
-// Running maximum of the magnitudes of bf16 pairs, as 16-bit integers: of one order with the values
-// themselves, infinities and NaNs on top (>= 0x7F80).  One packed instruction per pair.
-__device__ __forceinline__ uint32_t bf16_mag_max(uint32_t acc, uint32_t pair) {
-    const u16x2 m = __builtin_elementwise_max(__builtin_bit_cast(u16x2, acc), __builtin_bit_cast(u16x2, pair & 0x7FFF7FFFu));
-    return __builtin_bit_cast(uint32_t, m);
-}
-__device__ __forceinline__ bool bf16_mag_finite(uint32_t acc) { return (acc & 0xFFFFu) < 0x7F80u && (acc >> 16) < 0x7F80u; }
-
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }
-__device__ __forceinline__ float bf16_hi(uint32_t w) { return __uint_as_float(w & 0xFFFF0000u); }
-
-__device__ __forceinline__ void unpack8(const u32x4& w, float* x) {
-    x[0] = bf16_lo(w.x); x[1] = bf16_hi(w.x);
-    x[2] = bf16_lo(w.y); x[3] = bf16_hi(w.y);
-    x[4] = bf16_lo(w.z); x[5] = bf16_hi(w.z);
-    x[6] = bf16_lo(w.w); x[7] = bf16_hi(w.w);
-}
-
-__device__ __forceinline__ void load8(const float* p, float* x) {
-    const float4 a = *reinterpret_cast<const float4*>(p);
-    const float4 b = *reinterpret_cast<const float4*>(p + 4);
-    x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
-    x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
-}
-
-__device__ __forceinline__ bool key_kept(int s, int N, const KeyMask& m) { return s < N && !(s >= m.lo && s < m.hi); }
 
 // A lane exchange inside rows of 16 lanes that goes with the vector instruction, not through the LDS pipe.
 template <int CTRL> __device__ __forceinline__ float dpp(float x) {
@@ -424,9 +390,6 @@ struct KGroupSmem {
     float leafmin[16][LD];
     float leafmax[16][LD];
 };
-// the channel whose results thread t < D adds up
-template <int D> __device__ __forceinline__ int leaf_channel(int t) { return t % (D / 8) * 8 + t / (D / 8); }
-
 // D is the number of channels this call covers, starting at channel col0 of a head of DFULL
 // channels (the statistics are per channel, so a 256-channel head is done as two windows of 128).
 // Result in gsum, gmn, gmx of the threads tid < D (channel col0 + leaf_channel(tid)).
@@ -550,11 +513,6 @@ __device__ __forceinline__ void kstats_group_body(
 // v_slot_f16(k).  One workgroup per (tile, h, b): rows are read coalesced, staged in LDS and
 // written back channel-major in 16-byte runs.  Rows that are masked or beyond N become 0.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ uint16_t f32_to_f16_sat(float x) {
-    x = fminf(fmaxf(x, -65504.0f), 65504.0f);
-    return __half_as_ushort(__float2half_rn(x));
-}
-
 // LDS tile: 64 slots x D halves, unpadded; the 16-byte chunk index of a row is XORed with
 // 2*(slot/8) so that both the row-wise 16-byte writes and the column-wise dword reads below
 // touch every bank once (D = 128: 16 chunks; D = 64: 8 chunks, XOR with slot/8 instead).
@@ -586,10 +544,10 @@ __device__ __forceinline__ void quant_v_f16_body(
         float x[8];
         unpack8(raw[i], x);
         u32x4 o;
-        o.x = f32_to_f16_sat(x[0]) | ((uint32_t)f32_to_f16_sat(x[1]) << 16);
-        o.y = f32_to_f16_sat(x[2]) | ((uint32_t)f32_to_f16_sat(x[3]) << 16);
-        o.z = f32_to_f16_sat(x[4]) | ((uint32_t)f32_to_f16_sat(x[5]) << 16);
-        o.w = f32_to_f16_sat(x[6]) | ((uint32_t)f32_to_f16_sat(x[7]) << 16);
+        o.x = f16_pair_sat(x[0], x[1]);
+        o.y = f16_pair_sat(x[2], x[3]);
+        o.z = f16_pair_sat(x[4], x[5]);
+        o.w = f16_pair_sat(x[6], x[7]);
         const int slot = v_slot_f16(key);
         *reinterpret_cast<u32x4*>(&tile[slot * D + v_tile_chunk<D>(slot, chunk) * 8]) = o;
     }
@@ -648,27 +606,6 @@ __device__ __forceinline__ void v_absmax_group_body(
         for (int i = 0; i < ROWS; i++) mm = fmaxf(mm, red[i][tid]);
         part[(((int64_t)b * H + h) * ngroups + g) * D + leaf_channel<D>(tid)] = mm;
     }
-}
-
-// fp32 -> e4m3fn, round-to-nearest-even, saturating at +-448, NaN -> +-0.
-__device__ __forceinline__ uint32_t f32_to_e4m3(float x) {
-    const uint32_t u = __float_as_uint(x);
-    const uint32_t sign = (u >> 24) & 0x80u;
-    float a = fabsf(x);
-    if (!(a == a)) return sign;
-    a = fminf(a, 448.0f);
-    uint32_t byte;
-    if (a < 0.015625f) {                                   // below 2^-6: quantum 2^-9
-        byte = (uint32_t)(int)rintf(a * 512.0f);           // 0..8; 8 is exactly code 0x08
-    } else {
-        const uint32_t au = __float_as_uint(a);
-        // keep 3 mantissa bits, round half to even on the 20 dropped bits
-        uint32_t r = au + 0x7FFFFu + ((au >> 20) & 1u);
-        r >>= 20;                                          // (biased exp << 3) | mant3, carry included
-        byte = r - ((127u - 7u) << 3);
-        if (byte > 0x7Eu) byte = 0x7Eu;
-    }
-    return byte | sign;
 }
 
 // V tile -> e4m3 with the per-channel scales, tiled layout (slot order v_slot_fp8).
@@ -875,16 +812,6 @@ hipError_t launch_prep(const PrepArgs& a_in, int B, int D, hipStream_t st) {
 //      kmul = 1/s, qmul = cmul*s.
 //   V: vscale = amax/448 (1 when 0).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void k_final(double sum, float mn, float mx, int kept, int flags, float& mean, float& s) {
-    mean = 0.0f;
-    s = 1.0f;
-    if (flags & 1) mean = (float)(sum / (double)kept);
-    if (flags & 2) {
-        const float amax = fmaxf(fabsf(mx - mean), fabsf(mn - mean));
-        if (amax > 0.0f) s = sqrtf(amax);
-    }
-}
-
 // Groups added up, strictly in group order; the loads go NB groups at a time (taken one by one, each waits
 // out a memory latency).
 template <int NB>
