@@ -35,4 +35,18 @@ __host__ __device__ inline BwdBlock bwd_block(int id, int heads, int tq, int lq,
     return j < pq ? BwdBlock{false, j / (tq - lq), lq + j % (tq - lq)} : BwdBlock{true, (j - pq) / (tk - lk), lk + (j - pq) % (tk - lk)};
 }
 
+// The encoders' grid where rows are rotated by tables.  What reads the same table rows — the Q and K blocks of one run of
+// rows of one head, in every batch that shares the tables — is a set; its `members` go to one XCD, one soon after the other,
+// so that the rows come from its L2 after the first.  Sets run over the heads first and are taken 32 at a time, member by
+// member: consecutive ids read neighbours in memory, as everywhere in the quantizers.
+constexpr int kSetGroup = 32;                    // (a multiple of the XCDs)
+struct SetMember { int set, member; };
+__host__ __device__ inline SetMember set_member(int id, int members) {
+    const int at = id % (kSetGroup * members);
+    return SetMember{id / (kSetGroup * members) * kSetGroup + at % kSetGroup, at / kSetGroup};
+}
+__host__ __device__ inline long long set_grid(long long sets, int members) {
+    return (sets + kSetGroup - 1) / kSetGroup * kSetGroup * members;
+}
+
 }  // namespace sage

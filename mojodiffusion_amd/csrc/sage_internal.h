@@ -100,6 +100,7 @@ struct QuantArgs {
     uint16_t* v16;                   // fp16 V tiles (the repack needs no statistics; it rides here so that launch 1 is short)
     PreOp pre_q, pre_k;
     int nq_blk, nk_blk, nv_tile, n_bh;     // filled by the launcher
+    int n_sets, members, batches, q_per, k_per;    // likewise: workgroups dealt by set_member (sage_grid.h), and what they are
 };
 // f given: launch 2 is left out, the encoders add up the group results themselves and leave them in f's outputs
 // (quant_adds_up: where that pays; needs k8, and v8 where f has vscale).

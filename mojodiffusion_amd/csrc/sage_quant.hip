@@ -13,6 +13,7 @@
 // round-half-to-even) and every reduction either has a fixed order (the fp64 sums) or is
 // order-free (max / min), so codes, scales and statistics are reproducible bit for bit.
 // All kernels read bf16 rows with 16-byte loads (8 channels per lane).
+#include "sage_grid.h"
 #include "sage_quant_common.h"
 
 namespace sage {
@@ -885,7 +886,8 @@ template <int D, int PRE> constexpr int quant_threads() { return D > 128 ? 512 :
 
 // FIN: launch 2 is left out — every workgroup adds up the group results it needs for itself (the same additions,
 // so the same bits), the first of a head's K and V workgroups also leave them for later launches.
-template <int D, int PRE, bool FIN>
+// SETS: Q and K blocks are dealt by set_member (sage_grid.h; where: launch_quant).
+template <int D, int PRE, bool FIN, bool SETS>
 __global__ __launch_bounds__((quant_threads<D, PRE>())) void quant_kernel(QuantArgs a, FinalArgs f) {
     constexpr int NT = quant_threads<D, PRE>();
     union Smem {
@@ -896,7 +898,22 @@ __global__ __launch_bounds__((quant_threads<D, PRE>())) void quant_kernel(QuantA
     __shared__ __attribute__((aligned(16))) Smem sm;
     // consecutive workgroups take the same rows of consecutive heads: in [.., N, H, D] memory those
     // are neighbours, so the workgroups in flight together read whole DRAM pages between them
-    const int bh = blockIdx.x % a.n_bh, r = blockIdx.x / a.n_bh;
+    int bh = blockIdx.x % a.n_bh, r = blockIdx.x / a.n_bh;
+    if constexpr (SETS) {
+        const int id = blockIdx.x;
+        if (id < a.n_sets) {
+            const SetMember m = set_member(id, a.members);
+            const int heads = a.n_bh / a.batches, run = m.set / heads, which = m.member / a.batches;
+            const bool is_k = which >= a.q_per;
+            const int t = is_k ? run * a.k_per + which - a.q_per : run * a.q_per + which;
+            if (t >= (is_k ? a.nk_blk : a.nq_blk)) return;           // (also the sets past the last one)
+            bh = m.member % a.batches * heads + m.set % heads;
+            r = is_k ? a.nq_blk + t : t;
+        } else {
+            bh = (id - a.n_sets) % a.n_bh;
+            r = a.nq_blk + a.nk_blk + (id - a.n_sets) / a.n_bh;
+        }
+    }
     const int b = bh / a.H, h = bh % a.H;
     const KeyMask none{0, 0};
     __shared__ __attribute__((aligned(16))) float s_fin[FIN ? 3 : 1][FIN ? D : 4];      // mean, kmul, qmul; or vscale
@@ -966,21 +983,43 @@ hipError_t launch_quant(const QuantArgs& a_in, const FinalArgs* f, int B, int D,
     if (a.k8 != nullptr && a.nkv_pad % a.blkk != 0) return hipErrorInvalidValue;
     a.n_bh = B * a.H;
     const int has_pre = pre_kind(a.pre_q);
-    const int64_t total = (int64_t)B * a.H * (a.nq_blk + a.nk_blk + a.nv_tile);
+    int64_t total = (int64_t)B * a.H * (a.nq_blk + a.nk_blk + a.nv_tile);
+    a.n_sets = 0;
+    // Tables of 16 MiB and more, 128 channels: the blocks that read the same table rows share an XCD's L2.  A row of both tables
+    // is twice a row of Q or K, and four blocks (two batches) read it.  This launch, us, blocks in the order of heads -> in sets:
+    // [2,4352,30,128] 98.9 -> 88.0, [1,4608,24,128] 42.8 -> 36.8, e4m3 [1,9216,40,128] 181.7 -> 165.7, [2,2000,19,128] (19 MB) 34.4 ->
+    // 31.1; but e4m3 [2,1001,30,128] (15 MB) 31.8 -> 32.7, [1,700,32,128] 13.4 -> 14.6: the divisions of the mapping are on every
+    // workgroup's way (as a branch of the one kernel half a microsecond of small calls too, so it is a kernel of its own), and
+    // small tables come from the memory-side cache fast enough.  At 64 channels, workgroups of half the
+    // work, that is 1.5 us at any size ([2,4352,24,64] 35.3 -> 36.5).
+    const int64_t table_row = (int64_t)(D / 2) * (a.pre_q.tables_bf16 ? 4 : 8);
+    if (D == 128 && a.pre_q.cos != nullptr && (int64_t)a.Nq * a.H * table_row * (a.pre_q.batch_rows == 0 ? 1 : B) >= 16 << 20) {
+        // (a run is 128 rows: a block of 128, or several smaller ones)
+        a.batches = a.pre_q.batch_rows == 0 ? B : 1;
+        a.q_per = a.q8 != nullptr ? 128 / a.blkq : 0;
+        a.k_per = a.k8 != nullptr ? 128 / a.blkk : 0;
+        a.members = a.batches * (a.q_per + a.k_per);
+        const int64_t runs = max(a.q_per ? (a.nq_blk + a.q_per - 1) / a.q_per : 0, a.k_per ? (a.nk_blk + a.k_per - 1) / a.k_per : 0);
+        const int64_t n = set_grid(runs * (a.n_bh / a.batches), a.members);
+        total = n + (int64_t)B * a.H * a.nv_tile;
+        a.n_sets = (int)min(n, (int64_t)0x7FFFFFFF);
+    }
     if (total <= 0 || total > 0x7FFFFFFF) return hipErrorInvalidValue;
     dim3 grid((unsigned)total);
-#define SAGE_LAUNCH_QUANT(DD, PP)                                                                                              \
-    do {                                                                                                                       \
-        if (f != nullptr) hipLaunchKernelGGL((quant_kernel<DD, PP, true>), grid, dim3((quant_threads<DD, PP>())), 0, st, a, *f); \
-        else hipLaunchKernelGGL((quant_kernel<DD, PP, false>), grid, dim3((quant_threads<DD, PP>())), 0, st, a, FinalArgs{});    \
+#define SAGE_LAUNCH_QUANT(DD, PP, SETS)                                                                                              \
+    do {                                                                                                                             \
+        if (f != nullptr) hipLaunchKernelGGL((quant_kernel<DD, PP, true, SETS>), grid, dim3((quant_threads<DD, PP>())), 0, st, a, *f); \
+        else hipLaunchKernelGGL((quant_kernel<DD, PP, false, SETS>), grid, dim3((quant_threads<DD, PP>())), 0, st, a, FinalArgs{});    \
     } while (0)
-    if (D == 128 && has_pre == 2) SAGE_LAUNCH_QUANT(128, 2);
-    else if (D == 128 && has_pre) SAGE_LAUNCH_QUANT(128, 1);
-    else if (D == 128) SAGE_LAUNCH_QUANT(128, 0);
-    else if (D == 64 && has_pre == 2) SAGE_LAUNCH_QUANT(64, 2);
-    else if (D == 64 && has_pre) SAGE_LAUNCH_QUANT(64, 1);
-    else if (D == 64) SAGE_LAUNCH_QUANT(64, 0);
-    else if (D == 256 && !has_pre) SAGE_LAUNCH_QUANT(256, 0);
+    if (a.n_sets > 0 && has_pre == 2) SAGE_LAUNCH_QUANT(128, 2, true);
+    else if (a.n_sets > 0) SAGE_LAUNCH_QUANT(128, 1, true);
+    else if (D == 128 && has_pre == 2) SAGE_LAUNCH_QUANT(128, 2, false);
+    else if (D == 128 && has_pre) SAGE_LAUNCH_QUANT(128, 1, false);
+    else if (D == 128) SAGE_LAUNCH_QUANT(128, 0, false);
+    else if (D == 64 && has_pre == 2) SAGE_LAUNCH_QUANT(64, 2, false);
+    else if (D == 64 && has_pre) SAGE_LAUNCH_QUANT(64, 1, false);
+    else if (D == 64) SAGE_LAUNCH_QUANT(64, 0, false);
+    else if (D == 256 && !has_pre) SAGE_LAUNCH_QUANT(256, 0, false);
     else return hipErrorInvalidValue;
 #undef SAGE_LAUNCH_QUANT
     return hipGetLastError();
