@@ -423,6 +423,22 @@ int mi355_sage_sdpa_bwd_bf16(
     int causal, int real_N_q, int real_N_kv, void* stream,
     void* workspace, size_t workspace_bytes);
 
+/* The same for callers with F32 activations: dO, dQ, dK and dV are F32 (strides and offsets in elements, rows 16-byte
+ * aligned), Q, K, V and O bf16.  The call rounds dO to bf16 (nearest even) into dO_bf16, a buffer of dO's strides and offset in
+ * bf16 elements that it may leave anything else in, and the gradients hold the values the call above gives for it. */
+int mi355_sage_sdpa_bwd_f32_grads(
+    const void* Q, const void* K, const void* V, const void* O, const void* dO, void* dO_bf16, const void* Stats,
+    void* dQ, void* dK, void* dV,
+    int B, int H, int N_q, int N_kv, int D, float scale,
+    const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides,
+    const int64_t* o_strides, const int64_t* do_strides, const int64_t* dq_strides,
+    const int64_t* dk_strides, const int64_t* dv_strides,
+    int64_t q_offset_elems, int64_t k_offset_elems, int64_t v_offset_elems, int64_t o_offset_elems,
+    int64_t do_offset_elems, int64_t stats_offset_elems, int64_t dq_offset_elems,
+    int64_t dk_offset_elems, int64_t dv_offset_elems,
+    int causal, int real_N_q, int real_N_kv, void* stream,
+    void* workspace, size_t workspace_bytes);
+
 /* F32 <-> bf16 (round to nearest even) of `count` tensors (1 to 4) in one launch: the casts at the boundary of
  * callers with F32 activations (serenitymojo/ops/attention_flash.mojo:457-475, :478-535).  n: elements;
  * to_bf16 != 0: src F32, dst bf16, else the other way; bases 16-byte aligned. */

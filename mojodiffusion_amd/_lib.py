@@ -36,6 +36,8 @@ SIGNATURES = {
     "mi355_sage_bwd_workspace_bytes": (ctypes.c_size_t, [_int] * 5),
     "mi355_sage_sdpa_bwd_bf16": (_int, [_vp] * 9 + [_int] * 5 + [ctypes.c_float] + [_i64p] * 8 + [_i64] * 9
                                  + [_int, _int, _int, _vp, _vp, ctypes.c_size_t]),
+    "mi355_sage_sdpa_bwd_f32_grads": (_int, [_vp] * 10 + [_int] * 5 + [ctypes.c_float] + [_i64p] * 8 + [_i64] * 9
+                                      + [_int, _int, _int, _vp, _vp, ctypes.c_size_t]),
     "mi355_sage_pad_q": (_i64, [_i64]),
     "mi355_sage_pad_kv": (_i64, [_i64]),
     "mi355_sage_v_slot": (_int, [_int, _int]),
@@ -79,7 +81,7 @@ NORM_FULL_ROW = 4
 
 # entry points the native host path calls, in the order of its Api struct (csrc/sage_torch.cpp)
 _HOST_ENTRIES = ("workspace_bytes", "bwd_workspace_bytes", "sdpa_bf16", "sdpa_bf16_train_fwd", "sdpa_bf16_keymask", "sdpa_bf16_mask_any",
-                 "sdpa_bf16_norm_rope", "sdpa_bf16_norm_rope_train_fwd", "sdpa_bwd_bf16", "cast")
+                 "sdpa_bf16_norm_rope", "sdpa_bf16_norm_rope_train_fwd", "sdpa_bwd_bf16", "sdpa_bwd_f32_grads", "cast")
 
 _lib = None
 _host = None

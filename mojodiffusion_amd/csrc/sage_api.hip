@@ -43,12 +43,12 @@ bool dims_ok(int D) { return D == 64 || D == 128 || D == 256; }
 bool bwd_dims_ok(int D) { return D == 64 || D == 128; }
 
 // Row starts must be 16-byte aligned and the head dim contiguous.
-int check_view(const char* name, const void* p, const int64_t* s, int64_t off) {
+int check_view(const char* name, const void* p, const int64_t* s, int64_t off, int esz = 2) {
     if (s[3] != 1) {
         SAGE_LOG("%s: innermost stride %lld != 1", name, (long long)s[3]);
         return MI355_SAGE_EUNSUPPORTED;
     }
-    const uintptr_t a = reinterpret_cast<uintptr_t>(p) + (uintptr_t)(off * 2);
+    const uintptr_t a = reinterpret_cast<uintptr_t>(p) + (uintptr_t)(off * esz);
     if ((a & 15) || (s[0] & 7) || (s[1] & 7) || (s[2] & 7)) {
         SAGE_LOG("%s: rows are not 16-byte aligned", name);
         return MI355_SAGE_EUNSUPPORTED;
@@ -918,7 +918,7 @@ size_t mi355_sage_bwd_workspace_bytes(int B, int H, int N_q, int N_kv, int D) {
     return bwd_carve(B, H, N_q, D).total;
 }
 
-int mi355_sage_sdpa_bwd_bf16(const void* Q, const void* K, const void* V, const void* O, const void* dO,
+static int bwd_impl(bool f32, const void* Q, const void* K, const void* V, const void* O, const void* dO, void* dO_bf16,
                              const void* Stats, void* dQ, void* dK, void* dV,
                              int B, int H, int N_q, int N_kv, int D, float scale,
                              const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides,
@@ -930,17 +930,19 @@ int mi355_sage_sdpa_bwd_bf16(const void* Q, const void* K, const void* V, const 
                              void* workspace, size_t workspace_bytes) {
     // same order as serenitymojo/ops/cshim/cudnn_sdpa_bwd.cpp:348-352
     if (!Q || !K || !V || !O || !dO || !Stats) return MI355_SAGE_EINVAL;
-    if (!dQ || !dK || !dV) return MI355_SAGE_EINVAL;
+    if (!dQ || !dK || !dV || (f32 && !dO_bf16)) return MI355_SAGE_EINVAL;
     if (B <= 0 || H <= 0 || N_q <= 0 || N_kv <= 0 || D <= 0) return MI355_SAGE_EINVAL;
     if (!q_strides || !k_strides || !v_strides || !o_strides || !do_strides || !dq_strides || !dk_strides || !dv_strides)
         return MI355_SAGE_EINVAL;
     if (causal) { SAGE_LOG("causal attention is not supported"); return MI355_SAGE_EUNSUPPORTED; }
     if (!bwd_dims_ok(D)) { SAGE_LOG("backward: head dim %d is not supported (64 or 128)", D); return MI355_SAGE_EUNSUPPORTED; }
+    const int esz = f32 ? 4 : 2;
     int rc;
     if ((rc = check_view("Q", Q, q_strides, q_off)) || (rc = check_view("K", K, k_strides, k_off)) ||
         (rc = check_view("V", V, v_strides, v_off)) || (rc = check_view("O", O, o_strides, o_off)) ||
-        (rc = check_view("dO", dO, do_strides, do_off)) || (rc = check_view("dQ", dQ, dq_strides, dq_off)) ||
-        (rc = check_view("dK", dK, dk_strides, dk_off)) || (rc = check_view("dV", dV, dv_strides, dv_off)))
+        (rc = check_view("dO", dO, do_strides, do_off, esz)) || (rc = check_view("dQ", dQ, dq_strides, dq_off, esz)) ||
+        (rc = check_view("dK", dK, dk_strides, dk_off, esz)) || (rc = check_view("dV", dV, dv_strides, dv_off, esz)) ||
+        (f32 && (rc = check_view("dO_bf16", dO_bf16, do_strides, do_off))))
         return rc;
     // the tile copies address a head's rows with 32-bit byte offsets
     auto span_ok = [&](const char* name, int N, const int64_t* s) {
@@ -969,11 +971,14 @@ int mi355_sage_sdpa_bwd_bf16(const void* Q, const void* K, const void* V, const 
     a.k = make_view(K, k_strides, k_off);
     a.v = make_view(V, v_strides, v_off);
     a.o = make_view(O, o_strides, o_off);
-    a.dout = make_view(dO, do_strides, do_off);
+    a.dout = make_view(f32 ? dO_bf16 : dO, do_strides, do_off);
+    a.dout32 = f32 ? static_cast<const float*>(dO) + do_off : nullptr;
+    a.out32 = f32;
     a.stats = static_cast<const float*>(Stats) + stats_off;
-    a.dq = static_cast<uint16_t*>(dQ) + dq_off; a.dq_sb = dq_strides[0]; a.dq_sh = dq_strides[1]; a.dq_sn = dq_strides[2];
-    a.dk = static_cast<uint16_t*>(dK) + dk_off; a.dk_sb = dk_strides[0]; a.dk_sh = dk_strides[1]; a.dk_sn = dk_strides[2];
-    a.dv = static_cast<uint16_t*>(dV) + dv_off; a.dv_sb = dv_strides[0]; a.dv_sh = dv_strides[1]; a.dv_sn = dv_strides[2];
+    auto out = [&](void* p, int64_t off) { return reinterpret_cast<uint16_t*>(static_cast<uint8_t*>(p) + off * esz); };
+    a.dq = out(dQ, dq_off); a.dq_sb = dq_strides[0]; a.dq_sh = dq_strides[1]; a.dq_sn = dq_strides[2];
+    a.dk = out(dK, dk_off); a.dk_sb = dk_strides[0]; a.dk_sh = dk_strides[1]; a.dk_sn = dk_strides[2];
+    a.dv = out(dV, dv_off); a.dv_sb = dv_strides[0]; a.dv_sh = dv_strides[1]; a.dv_sn = dv_strides[2];
     a.B = B; a.H = H; a.Nq = N_q; a.Nkv = N_kv; a.D = D;
     a.valid_q = real_N_q > 0 && real_N_q < N_q ? real_N_q : N_q;          // cudnn_sdpa_bwd.cpp:362-363
     a.valid_kv = real_N_kv > 0 && real_N_kv < N_kv ? real_N_kv : N_kv;
@@ -985,5 +990,26 @@ int mi355_sage_sdpa_bwd_bf16(const void* Q, const void* K, const void* V, const 
     SAGE_HIP(launch_bwd(a, st));
     return 0;
 }
+
+#define SAGE_BWD_PARAMS                                                                                                          \
+    int B, int H, int N_q, int N_kv, int D, float scale, const int64_t *q_strides, const int64_t *k_strides,                     \
+        const int64_t *v_strides, const int64_t *o_strides, const int64_t *do_strides, const int64_t *dq_strides,                \
+        const int64_t *dk_strides, const int64_t *dv_strides, int64_t q_off, int64_t k_off, int64_t v_off, int64_t o_off,        \
+        int64_t do_off, int64_t stats_off, int64_t dq_off, int64_t dk_off, int64_t dv_off, int causal, int real_N_q,             \
+        int real_N_kv, void *stream, void *workspace, size_t workspace_bytes
+#define SAGE_BWD_ARGS                                                                                                            \
+    B, H, N_q, N_kv, D, scale, q_strides, k_strides, v_strides, o_strides, do_strides, dq_strides, dk_strides, dv_strides,       \
+        q_off, k_off, v_off, o_off, do_off, stats_off, dq_off, dk_off, dv_off, causal, real_N_q, real_N_kv, stream, workspace,   \
+        workspace_bytes
+int mi355_sage_sdpa_bwd_bf16(const void* Q, const void* K, const void* V, const void* O, const void* dO, const void* Stats, void* dQ,
+                             void* dK, void* dV, SAGE_BWD_PARAMS) {
+    return bwd_impl(false, Q, K, V, O, dO, nullptr, Stats, dQ, dK, dV, SAGE_BWD_ARGS);
+}
+int mi355_sage_sdpa_bwd_f32_grads(const void* Q, const void* K, const void* V, const void* O, const void* dO, void* dO_bf16,
+                                  const void* Stats, void* dQ, void* dK, void* dV, SAGE_BWD_PARAMS) {
+    return bwd_impl(true, Q, K, V, O, dO, dO_bf16, Stats, dQ, dK, dV, SAGE_BWD_ARGS);
+}
+#undef SAGE_BWD_PARAMS
+#undef SAGE_BWD_ARGS
 
 }  // extern "C"

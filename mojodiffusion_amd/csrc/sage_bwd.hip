@@ -8,7 +8,10 @@
 //
 // Two launches:
 //   1. bwd_prep_kernel     -Delta and Stats * log2(e) per query row (padding rows: +inf, so their
-//                          probabilities vanish); and a vector c close to the mean key.
+//                          probabilities vanish); and a vector c close to the mean key.  F32 callers: dO is
+//                          rounded here, and launch 2 stores F32, instead of a launch for each of the two casts:
+//                          the autograd call, us, [1,2304,12,64] 122.8 -> 115.0, [1,2304,12,128] 222 -> 207,
+//                          [2,1248,30,128] 370 -> 338, [1,4608,24,128] 1206 -> 1155.  Same values.
 //   2. bwd_fused_kernel    one grid of two kinds of 8-wave workgroups (4-wave at head dim 64), the longer kind first:
 //        dQ     owner = 256 (128) query rows, loop over key tiles, as scale * (dS K - rowsum(dS) c)
 //               = scale * dS (K - c)                                          (bwd_pass_body<D,0>)
@@ -128,12 +131,24 @@ template <int D>
 __device__ __forceinline__ void row_put(uint8_t* os, int l32, int half, int d, int g, u32x2 w) {
     *reinterpret_cast<u32x2*>(os + nat_off<D / 8>(l32, d * 4 + g) + half * 8) = w;
 }
-// ... and from there to the rows below n of the caller's tensor, 16 bytes per lane
+// ... and from there to the rows below n of the caller's tensor (`at`: elements up to this head), 16 bytes per lane; with
+// `f32` the same values as F32, 16 bytes to a lane of 4 channels.
 template <int D>
-__device__ __forceinline__ void rows_out(const uint8_t* os, uint16_t* head, int64_t sn, int row0, int n, int lane) {
+__device__ __forceinline__ void rows_out(const uint8_t* os, uint16_t* p, int64_t at, int64_t sn, int row0, int n, int lane, int f32) {
     constexpr int CPR = D / 8, RPI = 64 / CPR;
     asm volatile("" : "+v"(lane));      // (the row numbers of rows_in are formed again, not kept across the loop in between)
-    uint16_t* op = head + (lane % CPR) * 8;
+    if (f32) {
+        float* op = reinterpret_cast<float*>(p) + at + (lane % (2 * CPR)) * 4;
+#pragma unroll
+        for (int i = 0; i < 64 / RPI; i++) {
+            const int r = i * (RPI / 2) + lane / (2 * CPR);
+            const u32x2 w = *reinterpret_cast<const u32x2*>(os + nat_off<CPR>(r, lane % (2 * CPR) >> 1) + (lane & 1) * 8);
+            if (row0 + r < n)
+                *reinterpret_cast<u32x4*>(op + (int64_t)(row0 + r) * sn) = u32x4{w.x << 16, w.x & 0xFFFF0000u, w.y << 16, w.y & 0xFFFF0000u};
+        }
+        return;
+    }
+    uint16_t* op = p + at + (lane % CPR) * 8;
 #pragma unroll
     for (int i = 0; i < 32 / RPI; i++) {
         const int r = i * RPI + lane / CPR;
@@ -165,7 +180,23 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(BwdArgs a) {
         for (int i = 0; i < 64 / RPP; i++) {
             const int64_t row = min(r * 64 + i * RPP + tid / CPR, a.valid_q - 1);
             wo[i] = *reinterpret_cast<const u32x4*>(po + row * a.o.sn);
-            wg[i] = *reinterpret_cast<const u32x4*>(pg + row * a.dout.sn);
+            if (a.dout32 == nullptr) wg[i] = *reinterpret_cast<const u32x4*>(pg + row * a.dout.sn);
+        }
+        if (a.dout32 != nullptr) {                  // (the rounded rows also go where launch 2 reads them)
+            const float* pf = a.dout32 + b * a.dout.sb + h * a.dout.sh + col;
+            v4f f[64 / RPP][2];
+#pragma unroll
+            for (int i = 0; i < 64 / RPP; i++)
+#pragma unroll
+                for (int e = 0; e < 2; e++)
+                    f[i][e] = *reinterpret_cast<const v4f*>(pf + (int64_t)min(r * 64 + i * RPP + tid / CPR, a.valid_q - 1) * a.dout.sn + e * 4);
+#pragma unroll
+            for (int i = 0; i < 64 / RPP; i++) {
+                wg[i] = u32x4{pack_bf16(f[i][0][0], f[i][0][1]), pack_bf16(f[i][0][2], f[i][0][3]), pack_bf16(f[i][1][0], f[i][1][1]),
+                              pack_bf16(f[i][1][2], f[i][1][3])};
+                const int row = r * 64 + i * RPP + tid / CPR;
+                if (row < a.valid_q) *reinterpret_cast<u32x4*>(const_cast<uint16_t*>(pg) + (int64_t)row * a.dout.sn) = wg[i];
+            }
         }
 #pragma unroll
         for (int i = 0; i < 64 / RPP; i++) {
@@ -520,7 +551,8 @@ __device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, uint8_t* smem, i
             const u32x2 w = {pack_bf16(y[0] * a.scale, y[1] * a.scale), pack_bf16(y[2] * a.scale, y[3] * a.scale)};
             row_put<D>(os, l32, half, d, g, live ? w : u32x2{0u, 0u});
         }
-    rows_out<D>(os, PASS == 0 ? a.dq + b * a.dq_sb + h * a.dq_sh : a.dk + b * a.dk_sb + h * a.dk_sh, PASS == 0 ? a.dq_sn : a.dk_sn, x0, Nx, lane);
+    rows_out<D>(os, PASS == 0 ? a.dq : a.dk, PASS == 0 ? b * a.dq_sb + h * a.dq_sh : b * a.dk_sb + h * a.dk_sh, PASS == 0 ? a.dq_sn : a.dk_sn, x0, Nx,
+                lane, a.out32);
     if constexpr (PASS == 1) {
 #pragma unroll
         for (int d = 0; d < DB; d++)
@@ -529,7 +561,7 @@ __device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, uint8_t* smem, i
                 const u32x2 u = {pack_bf16(acc2[d][g * 4], acc2[d][g * 4 + 1]), pack_bf16(acc2[d][g * 4 + 2], acc2[d][g * 4 + 3])};
                 row_put<D>(os, l32, half, d, g, live ? u : u32x2{0u, 0u});
             }
-        rows_out<D>(os, a.dv + b * a.dv_sb + h * a.dv_sh, a.dv_sn, x0, Nx, lane);
+        rows_out<D>(os, a.dv, b * a.dv_sb + h * a.dv_sh, a.dv_sn, x0, Nx, lane, a.out32);
     }
 }
 
@@ -752,8 +784,8 @@ __device__ __forceinline__ void dkdv_role(const BwdArgs& a, uint8_t* smem, int b
                              pack_bf16(acc[d][g * 4 + 2] * mul, acc[d][g * 4 + 3] * mul)};
             row_put<D>(os, l32, half, d, g, live ? w : u32x2{0u, 0u});
         }
-    if constexpr (ROLE == 0) rows_out<D>(os, a.dv + b * a.dv_sb + h * a.dv_sh, a.dv_sn, x0, a.Nkv, lane);
-    else rows_out<D>(os, a.dk + b * a.dk_sb + h * a.dk_sh, a.dk_sn, x0, a.Nkv, lane);
+    if constexpr (ROLE == 0) rows_out<D>(os, a.dv, b * a.dv_sb + h * a.dv_sh, a.dv_sn, x0, a.Nkv, lane, a.out32);
+    else rows_out<D>(os, a.dk, b * a.dk_sb + h * a.dk_sh, a.dk_sn, x0, a.Nkv, lane, a.out32);
 }
 
 template <int D>

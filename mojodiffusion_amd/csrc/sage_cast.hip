@@ -1,5 +1,5 @@
 // sage_cast.hip — F32 <-> bf16 of up to four tensors in one launch (gfx950): callers with F32 activations
-// cast q, k and v at the boundary and the gradients on the way out, and a launch per tensor costs more than
+// cast q, k and v at the boundary and O on the way out (dO and the gradients: sage_bwd.hip), and a launch per tensor costs more than
 // the copy itself at a trainer's sizes ([1,2304,12,64]: 4.5 us each for 10.6 MB).  Bound by memory: 16-byte
 // loads and stores, eight elements per thread.
 #include "sage_internal.h"

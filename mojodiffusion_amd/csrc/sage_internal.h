@@ -222,6 +222,8 @@ int attn_split_faults(int reset);            // workgroups that gave up on the c
 struct BwdArgs {
     View q, k, v, o, dout;
     const float* stats;                          // [B,H,Nq] contiguous, natural log
+    const float* dout32;                         // F32 dO of dout's strides, which launch 1 rounds into dout's rows; null: dout holds dO
+    int out32;                                   // dq, dk, dv are F32 (holding the same bf16 values)
     uint16_t *dq, *dk, *dv;
     int64_t dq_sb, dq_sh, dq_sn, dk_sb, dk_sh, dk_sn, dv_sb, dv_sh, dv_sn;
     int B, H, Nq, Nkv, D;

@@ -32,6 +32,7 @@ struct Api {
     decltype(&mi355_sage_sdpa_bf16_norm_rope) norm_rope;
     decltype(&mi355_sage_sdpa_bf16_norm_rope_train_fwd) norm_rope_train;
     decltype(&mi355_sage_sdpa_bwd_bf16) bwd;
+    decltype(&mi355_sage_sdpa_bwd_f32_grads) bwd_f32;
     decltype(&mi355_sage_cast) cast;
 } api;
 constexpr int kApiEntries = sizeof(Api) / sizeof(void*);
@@ -124,23 +125,33 @@ int forward(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, doubl
 }
 
 // What the backward kernels read: shapes, types and devices of the saved set and the upstream gradient.
-bool bwd_set_ok(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& o, const at::Tensor& d, const at::Tensor& st) {
+bool bwd_set_ok(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& o, const at::Tensor& d, const at::Tensor& st,
+                bool f32_ok) {
     if (!shapes_ok(q, k, v, false) || q.scalar_type() != at::kBFloat16) return false;
     for (const at::Tensor* t : {&o, &d})
-        if (t->scalar_type() != at::kBFloat16 || !device_bhsd(*t) || t->sizes() != q.sizes() || t->device() != q.device()) return false;
+        if (!device_bhsd(*t) || t->sizes() != q.sizes() || t->device() != q.device()) return false;
+    if (o.scalar_type() != at::kBFloat16 || (d.scalar_type() != at::kBFloat16 && !(f32_ok && d.scalar_type() == at::kFloat))) return false;
     return st.scalar_type() == at::kFloat && st.is_cuda() && st.is_contiguous() && st.device() == q.device() &&
            st.numel() == q.size(0) * q.size(1) * q.size(2);
 }
 
+// Gradients of d_out's type, BF16 or F32.
 int backward(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& o, const at::Tensor& d_out,
              const at::Tensor& stats, double scale, int real_q, int real_kv, at::Tensor (&g)[3]) {
     const int B = q.size(0), Sq = q.size(1), H = q.size(2), D = q.size(3), Skv = k.size(1);
     const size_t need = api.bwd_workspace_bytes(B, H, Sq, Skv, D);
     if (need == 0) return MI355_SAGE_EUNSUPPORTED;
     void* st = stream_of(q);
-    g[0] = like(q, at::kBFloat16); g[1] = like(k, at::kBFloat16); g[2] = like(v, at::kBFloat16);
+    const at::ScalarType type = d_out.scalar_type();
+    g[0] = like(q, type); g[1] = like(k, type); g[2] = like(v, type);
     const at::Tensor ws = workspace(at_least(need), q.device(), st);
     const Strides qs = bshd(q), ks = bshd(k);
+    if (type == at::kFloat) {
+        const at::Tensor d16 = like(d_out, at::kBFloat16);
+        return api.bwd_f32(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), d_out.data_ptr(), d16.data_ptr(), stats.data_ptr(),
+                           g[0].data_ptr(), g[1].data_ptr(), g[2].data_ptr(), B, H, Sq, Skv, D, (float)scale, qs.s, ks.s, ks.s, qs.s, qs.s, qs.s,
+                           ks.s, ks.s, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, real_q, real_kv, st, ws.data_ptr(), (size_t)ws.numel());
+    }
     return api.bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), d_out.data_ptr(), stats.data_ptr(), g[0].data_ptr(),
                    g[1].data_ptr(), g[2].data_ptr(), B, H, Sq, Skv, D, (float)scale, qs.s, ks.s, ks.s, qs.s, qs.s, qs.s, ks.s, ks.s, 0, 0,
                    0, 0, 0, 0, 0, 0, 0, 0, real_q, real_kv, st, ws.data_ptr(), (size_t)ws.numel());
@@ -173,27 +184,17 @@ struct SdpaNode : torch::autograd::Function<SdpaNode> {
         const double scale = ctx->saved_data["scale"].toDouble();
         const at::Tensor& g = grads[0];
         const at::Tensor& q = saved[0];
-        at::Tensor d = g.is_contiguous() && aligned16(g) ? g : g.clone(at::MemoryFormat::Contiguous), out[3], res[3];
-        if (d.scalar_type() == at::kFloat) {
-            at::Tensor d32 = d;
-            const at::Tensor* src[1] = {&d32};
-            TORCH_CHECK(cast(1, src, &d, true) == 0, "record_sdpa: cast failed");
-        } else {
-            d = d.to(at::kBFloat16);
-        }
+        at::Tensor d = g.is_contiguous() && aligned16(g) ? g : g.clone(at::MemoryFormat::Contiguous), out[3];
+        if (d.scalar_type() != at::kFloat) d = d.to(at::kBFloat16);
         // (saved-tensor hooks may hand back anything)
         for (const at::Tensor& t : saved) TORCH_CHECK(plain(t), "sdpa_flash_backward_raw: a saved tensor came back without device memory");
-        TORCH_CHECK(bwd_set_ok(q, saved[1], saved[2], saved[3], d, saved[4]),
+        TORCH_CHECK(bwd_set_ok(q, saved[1], saved[2], saved[3], d, saved[4], true),
                     "sdpa_flash_backward_raw: a saved tensor came back with another shape, type, layout or device");
         const int rc = ::backward(q, saved[1], saved[2], saved[3], d, saved[4], scale, q.size(1), saved[1].size(1), out);
         TORCH_CHECK(rc == 0, "sdpa_flash_backward_raw: shim rc=", rc);
-        if (g.scalar_type() == at::kFloat) {
-            const at::Tensor* src[3] = {&out[0], &out[1], &out[2]};
-            TORCH_CHECK(cast(3, src, res, false) == 0, "record_sdpa: cast failed");
-        } else {
-            for (int i = 0; i < 3; i++) res[i] = out[i].to(g.scalar_type());
-        }
-        return {res[0], res[1], res[2], at::Tensor(), at::Tensor()};
+        if (g.scalar_type() != out[0].scalar_type())
+            for (at::Tensor& t : out) t = t.to(g.scalar_type());
+        return {out[0], out[1], out[2], at::Tensor(), at::Tensor()};
     }
 };
 
@@ -363,7 +364,7 @@ PyObject* py_bwd(PyObject* const* a, Py_ssize_t n) {
     if (intercepted() || n != 9 || !tensor_arg(a[0], q) || !tensor_arg(a[1], k) || !tensor_arg(a[2], v) || !tensor_arg(a[3], o) || !tensor_arg(a[4], d) ||
         !tensor_arg(a[5], st) || !double_arg(a[6], scale) || !int_arg(a[7], rq) || !int_arg(a[8], rk))
         Py_RETURN_NONE;
-    if (!bwd_set_ok(*q, *k, *v, *o, *d, *st)) Py_RETURN_NONE;
+    if (!bwd_set_ok(*q, *k, *v, *o, *d, *st, false)) Py_RETURN_NONE;
     at::Tensor g[3];
     if (without_gil([&] { return backward(*q, *k, *v, *o, *d, *st, scale, rq, rk, g); }) != 0) Py_RETURN_NONE;
     PyObject* t = PyTuple_New(3);
