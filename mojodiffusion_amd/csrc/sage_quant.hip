@@ -394,10 +394,12 @@ struct KGroupSmem {
 // D is the number of channels this call covers, starting at channel col0 of a head of DFULL
 // channels (the statistics are per channel, so a 256-channel head is done as two windows of 128).
 // Result in gsum, gmn, gmx of the threads tid < D (channel col0 + leaf_channel(tid)).
-template <int D, int PRE, int DFULL = D>
+// IN_LDS: the group's rows are at `rows` in LDS, those that do not count as zeros.
+template <int D, int PRE, int DFULL = D, bool IN_LDS = false>
 __device__ __forceinline__ void kstats_group(
     int g, int h, int b, int tid, const uint16_t* __restrict__ k, int64_t sb, int64_t sh, int64_t sn,
-    int N, int H, const KeyMask& km, KGroupSmem<D>& sm, const PreOp& pre, int col0, double& gsum, float& gmn, float& gmx) {
+    int N, int H, const KeyMask& km, KGroupSmem<D>& sm, const PreOp& pre, int col0, double& gsum, float& gmn, float& gmx,
+    const u32x4* rows = nullptr) {
     static_assert(!PRE || DFULL == D, "the fused pre-ops need the whole row in one call");
     constexpr int CPR = D / 8;
     const int leaf = tid / CPR, col = (tid % CPR) * 8;
@@ -409,7 +411,8 @@ __device__ __forceinline__ void kstats_group(
     u32x4 w[kLeaf];
     // every token of this leaf counts (no ragged end, no masked range inside it)
     const bool all_kept = s0 + kLeaf <= N && !(s0 < km.hi && s0 + kLeaf > km.lo);
-    if (__all(all_kept)) {
+    if constexpr (IN_LDS) {
+    } else if (__all(all_kept)) {
 #pragma unroll
         for (int i = 0; i < kLeaf; i++) w[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)(s0 + i) * sn);
     } else {
@@ -441,10 +444,9 @@ __device__ __forceinline__ void kstats_group(
         }
     }
     static_assert(kLeaf % 2 == 0, "tokens are taken in pairs");
-#pragma unroll
-    for (int i = 0; i < kLeaf; i++) {
+    auto token = [&](int i, bool odd, const u32x4& raw) {
         float x[8];
-        unpack8(w[i], x);
+        unpack8(raw, x);
         const bool kept = key_kept(s0 + i, N, km);
         if constexpr (PRE) {
             pre_apply<D, PRE>(pre, col, kept, inv[i], gain, tab[i % AHEAD], x);
@@ -457,7 +459,7 @@ __device__ __forceinline__ void kstats_group(
             // (the common case, two tokens per three-operand instruction; written as instructions because the
             // compiler puts a canonicalising v_max in front of every operand of fminf / fmaxf that comes out of
             // bit operations — six instructions per element instead of one)
-            if (i & 1) {
+            if (odd) {
 #pragma unroll
                 for (int e = 0; e < 8; e++) {
                     asm("v_min3_f32 %0, %0, %1, %2" : "+v"(mn[e]) : "v"(xprev[e]), "v"(x[e]));
@@ -471,6 +473,19 @@ __device__ __forceinline__ void kstats_group(
 #pragma unroll
             for (int e = 0; e < 8; e++) { mn[e] = fminf(mn[e], x[e]); mx[e] = fmaxf(mx[e], x[e]); }
         }
+    };
+    if constexpr (IN_LDS) {
+#pragma unroll 1
+        for (int i0 = 0; i0 < kLeaf; i0 += 4) {                // (registers for four rows, not sixteen)
+            u32x4 raw[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) raw[i] = rows[(leaf * kLeaf + i0 + i) * CPR + tid % CPR];
+#pragma unroll
+            for (int i = 0; i < 4; i++) token(i0 + i, i & 1, raw[i]);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < kLeaf; i++) token(i, i & 1, w[i]);
     }
 #pragma unroll
     for (int e = 0; e < 8; e++) {
@@ -493,14 +508,14 @@ __device__ __forceinline__ void kstats_group(
     }
 }
 
-template <int D, int PRE, int DFULL = D>
+template <int D, int PRE, int DFULL = D, bool IN_LDS = false>
 __device__ __forceinline__ void kstats_group_body(
     int g, int h, int b, int tid, const uint16_t* __restrict__ k, int64_t sb, int64_t sh, int64_t sn,
     int N, int H, int ngroups, const KeyMask& km, double* __restrict__ part_sum, float* __restrict__ part_mm,
-    KGroupSmem<D>& sm, const PreOp& pre, int col0 = 0) {
+    KGroupSmem<D>& sm, const PreOp& pre, int col0 = 0, const u32x4* rows = nullptr) {
     double gsum;
     float gmn, gmx;
-    kstats_group<D, PRE, DFULL>(g, h, b, tid, k, sb, sh, sn, N, H, km, sm, pre, col0, gsum, gmn, gmx);
+    kstats_group<D, PRE, DFULL, IN_LDS>(g, h, b, tid, k, sb, sh, sn, N, H, km, sm, pre, col0, gsum, gmn, gmx, rows);
     if (tid < D && g >= 0) {
         const int64_t o = (((int64_t)b * H + h) * ngroups + g) * DFULL + col0 + leaf_channel<D>(tid);
         part_sum[o] = gsum;
@@ -735,6 +750,56 @@ __global__ __launch_bounds__(256) void prep_kernel(PrepArgs a) {
     }
 }
 
+// The K statistics behind the pre-ops where there are no more groups than compute units.  A wave per SIMD norms and rotates
+// sixteen rows one after the other there, and that chain is the launch.  Here a group's 256 rows go to four times as many
+// threads, four rows each, and through LDS to those that add them up, in the same order.  The call, us: [1,8 heads,768,64] 25.1 ->
+// 21.4, [2,12,2000,64] 53.8 -> 49.1, [1,19,1153,128] 47.2 -> 44.0, [2,16,2048,128] (256 groups) 92.8 -> 89.8; but past one
+// workgroup per unit [1,30,2304,128] (270) 121.9 -> 125.0, [1,24,4608,128] 240 -> 245.
+template <int D, int PRE>
+__global__ __launch_bounds__(64 * (D / 8)) void prep_rows_kernel(PrepArgs a) {
+    constexpr int CPR = D / 8, NR = 4, PASS = kGroup / NR, AHEAD = PRE == 2 ? 2 : NR;
+    __shared__ __attribute__((aligned(16))) KGroupSmem<D> sm;
+    __shared__ __attribute__((aligned(16))) u32x4 rows[kGroup * CPR];
+    const int bh = blockIdx.x % a.n_bh, g = blockIdx.x / a.n_bh;
+    const int b = bh / a.H, h = bh % a.H;
+    const int tid = threadIdx.x, col = (tid % CPR) * 8, first = g * kGroup + tid / CPR;
+    const uint16_t* src = a.k.p + b * a.k.sb + h * a.k.sh + col;
+    u32x4 w[NR];
+    RopeTab<PRE> tab[AHEAD];
+    const RopeAt rope = rope_at<D>(a.pre_k, b, h, a.H, col);
+    auto clamped = [&](int i) { return min(first + i * PASS, a.Nkv - 1); };
+#pragma unroll
+    for (int i = 0; i < NR; i++) {
+        w[i] = u32x4{0u, 0u, 0u, 0u};
+        if (key_kept(first + i * PASS, a.Nkv, a.km)) w[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)(first + i * PASS) * a.k.sn);
+    }
+#pragma unroll
+    for (int i = 0; i < AHEAD; i++) rope_load<PRE>(rope, clamped(i), tab[i]);
+    float inv[NR], gain[8];
+    pre_gains(a.pre_k, h, D, col, gain);
+    if (a.pre_k.row_inv == nullptr) {
+        row_inverses<D, NR>(a.pre_k.eps, w, inv);
+    } else {
+#pragma unroll
+        for (int i = 0; i < NR; i++) inv[i] = a.pre_k.row_inv[(int64_t)b * a.pre_k.row_n + clamped(i)];
+    }
+#pragma unroll
+    for (int i = 0; i < NR; i++) {
+        float x[8];
+        unpack8(w[i], x);
+        pre_apply<D, PRE>(a.pre_k, col, key_kept(first + i * PASS, a.Nkv, a.km), inv[i], gain, tab[i % AHEAD], x);
+        if (i + AHEAD < NR) rope_load<PRE>(rope, clamped(i + AHEAD), tab[i % AHEAD]);
+        u32x4 y;                                           // (bf16 values: nothing below their upper halves)
+#pragma unroll
+        for (int e = 0; e < 4; e++) y[e] = __builtin_amdgcn_perm(__float_as_uint(x[2 * e + 1]), __float_as_uint(x[2 * e]), 0x07060302u);
+        rows[(i * PASS + tid / CPR) * CPR + tid % CPR] = y;
+    }
+    __syncthreads();
+    // (16 leaves; the other waves only meet the barrier inside)
+    kstats_group_body<D, 0, D, true>(tid < 16 * CPR ? g : -1, h, b, tid, a.k.p, a.k.sb, a.k.sh, a.k.sn, a.Nkv, a.H, a.ngroups, a.km, a.kpart_sum,
+                                     a.kpart_mm, sm, a.pre_k, 0, rows);
+}
+
 // ---------------------------------------------------------------------------
 // Launch 0: whole-row RMSNorm statistic.  One workgroup of 256 threads per token, exactly the
 // reference's reduction (serenitymojo/ops/norm.mojo:56-72): thread t adds the squares of
@@ -794,6 +859,16 @@ hipError_t launch_prep(const PrepArgs& a_in, int B, int D, hipStream_t st) {
     if (total == 0) return hipSuccess;
     if (total > 0x7FFFFFFF) return hipErrorInvalidValue;
     dim3 grid((unsigned)total), block(256);
+    // (more groups than compute units: prep_kernel's smaller workgroups fill the chip by themselves)
+    const int64_t groups = (int64_t)B * a.H * a.ngroups;
+    if (D <= 128 && has_pre && a.kpart_sum != nullptr && a.nv_units == 0 && groups <= compute_units()) {
+        const dim3 each((unsigned)groups), threads(8 * D);
+        if (D == 128 && has_pre == 2) hipLaunchKernelGGL((prep_rows_kernel<128, 2>), each, threads, 0, st, a);
+        else if (D == 128) hipLaunchKernelGGL((prep_rows_kernel<128, 1>), each, threads, 0, st, a);
+        else if (has_pre == 2) hipLaunchKernelGGL((prep_rows_kernel<64, 2>), each, threads, 0, st, a);
+        else hipLaunchKernelGGL((prep_rows_kernel<64, 1>), each, threads, 0, st, a);
+        return hipGetLastError();
+    }
     if (D == 128 && has_pre == 2) hipLaunchKernelGGL((prep_kernel<128, 2>), grid, block, 0, st, a);
     else if (D == 128 && has_pre) hipLaunchKernelGGL((prep_kernel<128, 1>), grid, block, 0, st, a);
     else if (D == 128) hipLaunchKernelGGL((prep_kernel<128, 0>), grid, block, 0, st, a);
