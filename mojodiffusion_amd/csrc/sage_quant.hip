@@ -1264,10 +1264,11 @@ static int64_t short_workgroups(const QuantArgs& a) { return (int64_t)a.n_bh * (
 // per compute unit).  Measured over 4 to 60 heads, stage of three launches -> one, us: 11.5-15 -> 7.5-9.5 up
 // to 256 keys, 13-15 -> 9-12.8 at 512 keys of 128 channels, 12-13.4 -> 8.4-10.7 at 1024 keys of 64; a second
 // pass costs 4 us and a second generation of workgroups 7, which is what the two launches less are worth.
-// Half as many keys with the pre-ops in front: a workgroup then norms and rotates every key of its head, a longer chain than
-// the launches saved.  The call, us, one launch -> two: [1,8 heads,768,64] 29.1 -> 25.5, [1,16,1024,64] 34.3 -> 30.4,
-// [1,24,333,128] 35.8 -> 32.1, [1,8,512,128] 32.4 -> 28.6, e4m3 [1,12,512,128] 28.3 -> 26.5; but [1,8,512,64] 24.2 -> 24.6,
-// [2,30,200,128] 31.6 -> 33.8, e4m3 [2,8,400,64] 22.6 -> 24.0.
+// With the pre-ops in front a workgroup norms and rotates every key of its head, a longer chain than the launch saved.  fp16
+// P.V takes two launches then, the first of which is prep_rows_kernel; the call, us, one launch -> two: [1,8 heads,128,64] 21.7 -> 18.5,
+// [1,24,512,64] 26.6 -> 22.6, [1,8,1000,64] 31.9 -> 24, [2,30,200,128] 31.9 -> 30.6, [1,24,333,128] 35.8 -> 30.2, [2,30,500,64] level.
+// With e4m3, whose first launch has the V maxima in it as well, half as many keys: [1,12,512,128] 28.3 -> 26.5, [1,8,1000,64]
+// 29.1 -> 25.8; but [1,30,256,128] 25.4 -> 26.7, [2,8,400,64] 22.6 -> 24.0.
 static int64_t short_rule(const QuantArgs& a, int D, bool pre_ops = false) {
     const int groups = (a.Nkv + kGroup - 1) / kGroup, most = D == 64 ? 4 : D == 128 ? 2 : 1;
     const int64_t wgs = short_workgroups(a);
@@ -1276,6 +1277,7 @@ static int64_t short_rule(const QuantArgs& a, int D, bool pre_ops = false) {
 int64_t quant_short_workgroups(const QuantArgs& a_in, int B, int D) {
     QuantArgs a = a_in;
     short_units(a, B, a.q8 != nullptr);
+    if (a.pre_k.gain != nullptr && a.v8 == nullptr) return 0;
     return short_rule(a, D, a.pre_k.gain != nullptr);
 }
 int64_t quant_short_workgroups(int B, int H, int Nq, int Nkv, int D, int blkq, int blkk, bool with_q) {
