@@ -592,12 +592,12 @@ __device__ __forceinline__ void quant_v_f16_body(
 // ---------------------------------------------------------------------------
 // V channel maxima of one group of 256 tokens (e4m3 variant; max is order-free).
 // ---------------------------------------------------------------------------
-template <int D>
+template <int D, int NT = 256>
 __device__ __forceinline__ void v_absmax_group_body(
     int g, int h, int b, const uint16_t* __restrict__ v, int64_t sb, int64_t sh, int64_t sn,
     int N, int H, int ngroups, const KeyMask& km, float* __restrict__ part, float (*red)[D + D / 8]) {
     constexpr int CPR = D / 8;
-    constexpr int ROWS = 256 / CPR;                        // rows covered per step
+    constexpr int ROWS = NT / CPR;                        // rows covered per step
     const int tid = threadIdx.x;
     const int col = (tid % CPR) * 8, r = tid / CPR;
     const uint16_t* src = v + b * sb + h * sh + col;
@@ -750,18 +750,27 @@ __global__ __launch_bounds__(256) void prep_kernel(PrepArgs a) {
     }
 }
 
-// The K statistics behind the pre-ops where there are no more groups than compute units.  A wave per SIMD norms and rotates
+// The K statistics behind the pre-ops, and with e4m3 the V channel maxima, where there are no more K groups than compute units.  A wave per SIMD norms and rotates
 // sixteen rows one after the other there, and that chain is the launch.  Here a group's 256 rows go to four times as many
 // threads, four rows each, and through LDS to those that add them up, in the same order.  The call, us: [1,8 heads,768,64] 25.1 ->
 // 21.4, [2,12,2000,64] 53.8 -> 49.1, [1,19,1153,128] 47.2 -> 44.0, [2,16,2048,128] (256 groups) 92.8 -> 89.8; but past one
-// workgroup per unit [1,30,2304,128] (270) 121.9 -> 125.0, [1,24,4608,128] 240 -> 245.
+// workgroup per unit [1,30,2304,128] (270) 121.9 -> 125.0, [1,24,4608,128] 240 -> 245.  e4m3 [1,8,1000,64] 25.8 -> 22.4, [1,24,2304,64]
+// 67.6 -> 60.3, [1,19,1153,128] 47.7 -> 44.9; but [1,32,2000,128] (256 and as many of V) 93.1 -> 94.1.
 template <int D, int PRE>
 __global__ __launch_bounds__(64 * (D / 8)) void prep_rows_kernel(PrepArgs a) {
     constexpr int CPR = D / 8, NR = 4, PASS = kGroup / NR, AHEAD = PRE == 2 ? 2 : NR;
-    __shared__ __attribute__((aligned(16))) KGroupSmem<D> sm;
+    union Smem {
+        float red[64][D + D / 8];
+        KGroupSmem<D> kg;
+    };
+    __shared__ __attribute__((aligned(16))) Smem sm;
     __shared__ __attribute__((aligned(16))) u32x4 rows[kGroup * CPR];
     const int bh = blockIdx.x % a.n_bh, g = blockIdx.x / a.n_bh;
     const int b = bh / a.H, h = bh % a.H;
+    if (g >= a.ngroups) {                                  // (behind the K groups, which are the longer ones)
+        v_absmax_group_body<D, 64 * CPR>(g - a.ngroups, h, b, a.v.p, a.v.sb, a.v.sh, a.v.sn, a.Nkv, a.H, a.ngroups, a.km, a.vpart, sm.red);
+        return;
+    }
     const int tid = threadIdx.x, col = (tid % CPR) * 8, first = g * kGroup + tid / CPR;
     const uint16_t* src = a.k.p + b * a.k.sb + h * a.k.sh + col;
     u32x4 w[NR];
@@ -797,7 +806,7 @@ __global__ __launch_bounds__(64 * (D / 8)) void prep_rows_kernel(PrepArgs a) {
     __syncthreads();
     // (16 leaves; the other waves only meet the barrier inside)
     kstats_group_body<D, 0, D, true>(tid < 16 * CPR ? g : -1, h, b, tid, a.k.p, a.k.sb, a.k.sh, a.k.sn, a.Nkv, a.H, a.ngroups, a.km, a.kpart_sum,
-                                     a.kpart_mm, sm, a.pre_k, 0, rows);
+                                     a.kpart_mm, sm.kg, a.pre_k, 0, rows);
 }
 
 // ---------------------------------------------------------------------------
@@ -859,10 +868,11 @@ hipError_t launch_prep(const PrepArgs& a_in, int B, int D, hipStream_t st) {
     if (total == 0) return hipSuccess;
     if (total > 0x7FFFFFFF) return hipErrorInvalidValue;
     dim3 grid((unsigned)total), block(256);
-    // (more groups than compute units: prep_kernel's smaller workgroups fill the chip by themselves)
-    const int64_t groups = (int64_t)B * a.H * a.ngroups;
-    if (D <= 128 && has_pre && a.kpart_sum != nullptr && a.nv_units == 0 && groups <= compute_units()) {
-        const dim3 each((unsigned)groups), threads(8 * D);
+    // (more groups than compute units: prep_kernel's smaller workgroups fill the chip by themselves.  A workgroup of 128 channels
+    // has a unit to itself, and its V blocks count; of 64 two share one)
+    const int64_t groups = (int64_t)B * a.H * a.ngroups, blocks = groups + (int64_t)B * a.H * a.nv_units;
+    if (D <= 128 && has_pre && a.kpart_sum != nullptr && a.vmode != 0 && (D == 64 ? groups : blocks) <= compute_units()) {
+        const dim3 each((unsigned)blocks), threads(8 * D);
         if (D == 128 && has_pre == 2) hipLaunchKernelGGL((prep_rows_kernel<128, 2>), each, threads, 0, st, a);
         else if (D == 128) hipLaunchKernelGGL((prep_rows_kernel<128, 1>), each, threads, 0, st, a);
         else if (has_pre == 2) hipLaunchKernelGGL((prep_rows_kernel<64, 2>), each, threads, 0, st, a);
@@ -1109,7 +1119,7 @@ hipError_t launch_quant(const QuantArgs& a_in, const FinalArgs* f, int B, int D,
 // ---------------------------------------------------------------------------
 constexpr int kShortThreads = 512;
 
-template <int D, int PRE>
+template <int D>
 __global__ __launch_bounds__(kShortThreads) void quant_short_kernel(QuantArgs a, FinalArgs f) {
     constexpr int DK = D > 128 ? 128 : D;                 // channels per K statistics call
     constexpr int NWIN = D / DK;                          // windows of DK channels
@@ -1142,8 +1152,8 @@ __global__ __launch_bounds__(kShortThreads) void quant_short_kernel(QuantArgs a,
         // The block's rows are requested ahead of the statistics where it has the size the one-shot call gives it.
         constexpr int CPR = D / 8, RPC = 256 / CPR;           // rows per chunk of the half's threads
         u32x4 rows[128 / RPC];
-        const int ahead = PRE == 0 && D <= 128 ? (is_k ? (a.blkk == 64 ? 64 : 0) : (a.blkq == 128 ? 128 : 0)) : 0;
-        if constexpr (PRE == 0 && D <= 128) {
+        const int ahead = D <= 128 ? (is_k ? (a.blkk == 64 ? 64 : 0) : (a.blkq == 128 ? 128 : 0)) : 0;
+        if constexpr (D <= 128) {
             const View& x = is_k ? a.k : a.q;
             const int n = is_k ? a.Nkv : a.Nq;
             const uint16_t* src = x.p + b * x.sb + h * x.sh + (utid % CPR) * 8;
@@ -1163,7 +1173,7 @@ __global__ __launch_bounds__(kShortThreads) void quant_short_kernel(QuantArgs a,
                     double gsum;
                     float gmn, gmx;
                     const int g = g0 + sub;
-                    kstats_group<DK, PRE, D>(g < f.ngroups ? g : -1, h, b, t, a.k.p, a.k.sb, a.k.sh, a.k.sn, a.Nkv, a.H, a.km,
+                    kstats_group<DK, 0, D>(g < f.ngroups ? g : -1, h, b, t, a.k.p, a.k.sb, a.k.sh, a.k.sn, a.Nkv, a.H, a.km,
                                              sm.kg[sub], a.pre_k, w * DK, gsum, gmn, gmx);
                     if (f.ngroups == 1) {                   // (nothing to exchange)
                         if (tid < DK) { sum += gsum; mn = fminf(mn, gmn); mx = fmaxf(mx, gmx); }
@@ -1197,11 +1207,11 @@ __global__ __launch_bounds__(kShortThreads) void quant_short_kernel(QuantArgs a,
             }
         }
         __syncthreads();
-#define SAGE_K(BLK, HAVE) quant_i8_block<D, BLK, true, PRE, 256, HAVE>(blk, h, b, utid, a.k.p, a.k.sb, a.k.sh, a.k.sn, a.Nkv, a.H, a.nkv_pad, a.km, \
+#define SAGE_K(BLK, HAVE) quant_i8_block<D, BLK, true, 0, 256, HAVE>(blk, h, b, utid, a.k.p, a.k.sb, a.k.sh, a.k.sn, a.Nkv, a.H, a.nkv_pad, a.km, \
                                                        s_mean, s_kmul, 0.0f, a.k8, a.kscale, nullptr, sm.red[unit], a.pre_k, rows)
-#define SAGE_Q(BLK, HAVE) quant_i8_block<D, BLK, false, PRE, 256, HAVE>(blk, h, b, utid, a.q.p, a.q.sb, a.q.sh, a.q.sn, a.Nq, a.H, a.nq_pad, none, \
+#define SAGE_Q(BLK, HAVE) quant_i8_block<D, BLK, false, 0, 256, HAVE>(blk, h, b, utid, a.q.p, a.q.sb, a.q.sh, a.q.sn, a.Nq, a.H, a.nq_pad, none, \
                                                         s_mean, s_qmul, a.cmul, a.q8, a.qscale, a.rowdot, sm.red[unit], a.pre_q, rows)
-        constexpr bool HAVE = PRE == 0 && D <= 128;
+        constexpr bool HAVE = D <= 128;
         if (is_k) {
             if (a.blkk == 128) SAGE_K(128, false);
             else if (a.blkk == 64) SAGE_K(64, HAVE);
@@ -1264,21 +1274,20 @@ static int64_t short_workgroups(const QuantArgs& a) { return (int64_t)a.n_bh * (
 // per compute unit).  Measured over 4 to 60 heads, stage of three launches -> one, us: 11.5-15 -> 7.5-9.5 up
 // to 256 keys, 13-15 -> 9-12.8 at 512 keys of 128 channels, 12-13.4 -> 8.4-10.7 at 1024 keys of 64; a second
 // pass costs 4 us and a second generation of workgroups 7, which is what the two launches less are worth.
-// With the pre-ops in front a workgroup norms and rotates every key of its head, a longer chain than the launch saved.  fp16
-// P.V takes two launches then, the first of which is prep_rows_kernel; the call, us, one launch -> two: [1,8 heads,128,64] 21.7 -> 18.5,
-// [1,24,512,64] 26.6 -> 22.6, [1,8,1000,64] 31.9 -> 24, [2,30,200,128] 31.9 -> 30.6, [1,24,333,128] 35.8 -> 30.2, [2,30,500,64] level.
-// With e4m3, whose first launch has the V maxima in it as well, half as many keys: [1,12,512,128] 28.3 -> 26.5, [1,8,1000,64]
-// 29.1 -> 25.8; but [1,30,256,128] 25.4 -> 26.7, [2,8,400,64] 22.6 -> 24.0.
-static int64_t short_rule(const QuantArgs& a, int D, bool pre_ops = false) {
+// Never with the pre-ops in front: a workgroup would norm and rotate every key of its head, a longer chain than the launch
+// saved.  The call, us, one launch -> two, the first of them prep_rows_kernel: [1,8 heads,128,64] 21.7 -> 18.5, [1,24,512,64] 26.6 ->
+// 22.6, [2,30,200,128] 31.9 -> 30.6, [1,24,333,128] 35.8 -> 30.2, [2,30,500,64] level; e4m3 [1,8,300,64] 22.5 -> 20.0, [1,24,512,64]
+// 34.9 -> 20.9, [2,30,200,128] 39.2 -> 30.5, [1,19,150,128] 24.9 -> 24.4.
+static int64_t short_rule(const QuantArgs& a, int D) {
     const int groups = (a.Nkv + kGroup - 1) / kGroup, most = D == 64 ? 4 : D == 128 ? 2 : 1;
     const int64_t wgs = short_workgroups(a);
-    return groups <= (pre_ops ? most / 2 : most) && wgs <= 512 ? wgs : 0;
+    return groups <= most && wgs <= 512 ? wgs : 0;
 }
 int64_t quant_short_workgroups(const QuantArgs& a_in, int B, int D) {
     QuantArgs a = a_in;
     short_units(a, B, a.q8 != nullptr);
-    if (a.pre_k.gain != nullptr && a.v8 == nullptr) return 0;
-    return short_rule(a, D, a.pre_k.gain != nullptr);
+    if (a.pre_k.gain != nullptr) return 0;
+    return short_rule(a, D);
 }
 int64_t quant_short_workgroups(int B, int H, int Nq, int Nkv, int D, int blkq, int blkk, bool with_q) {
     QuantArgs a{};
@@ -1296,14 +1305,10 @@ hipError_t launch_quant_short(const QuantArgs& a_in, const FinalArgs& f_in, int 
     const int64_t total = short_workgroups(a);
     if (total <= 0 || total > 0x7FFFFFFF || (a.nv_tile & 1)) return hipErrorInvalidValue;
     const dim3 grid((unsigned)total), block(kShortThreads);
-    const int has_pre = pre_kind(a.pre_q);
-    if (D == 128 && has_pre == 2) hipLaunchKernelGGL((quant_short_kernel<128, 2>), grid, block, 0, st, a, f_in);
-    else if (D == 128 && has_pre) hipLaunchKernelGGL((quant_short_kernel<128, 1>), grid, block, 0, st, a, f_in);
-    else if (D == 128) hipLaunchKernelGGL((quant_short_kernel<128, 0>), grid, block, 0, st, a, f_in);
-    else if (D == 64 && has_pre == 2) hipLaunchKernelGGL((quant_short_kernel<64, 2>), grid, block, 0, st, a, f_in);
-    else if (D == 64 && has_pre) hipLaunchKernelGGL((quant_short_kernel<64, 1>), grid, block, 0, st, a, f_in);
-    else if (D == 64) hipLaunchKernelGGL((quant_short_kernel<64, 0>), grid, block, 0, st, a, f_in);
-    else if (D == 256 && !has_pre) hipLaunchKernelGGL((quant_short_kernel<256, 0>), grid, block, 0, st, a, f_in);
+    if (a.pre_q.gain != nullptr || a.pre_k.gain != nullptr) return hipErrorInvalidValue;
+    if (D == 128) hipLaunchKernelGGL(quant_short_kernel<128>, grid, block, 0, st, a, f_in);
+    else if (D == 64) hipLaunchKernelGGL(quant_short_kernel<64>, grid, block, 0, st, a, f_in);
+    else if (D == 256) hipLaunchKernelGGL(quant_short_kernel<256>, grid, block, 0, st, a, f_in);
     else return hipErrorInvalidValue;
     return hipGetLastError();
 }

@@ -1,5 +1,5 @@
-"""RMSNorm + RoPE in front of short self-attention, on either side of the length from which the quantizers take two launches
-instead of one: bits of the same call on rows normed and rotated before."""
+"""RMSNorm + RoPE in front of short self-attention, whose quantizers take two launches where those of plain rows take one: bits of
+the same call on rows normed and rotated before."""
 import numpy as np
 import pytest
 
