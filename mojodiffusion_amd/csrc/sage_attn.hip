@@ -258,8 +258,9 @@ __global__ __launch_bounds__(WAVES * 64, D <= 128 ? 2 : 1) void sage_attn_kernel
     const int ush = blkk == 32 ? 0 : (blkk == 64 ? 1 : 2);      // log2(32-key blocks per scale block)
     // (staged per 32-key block, KS_OFF entries in: the main loop fetches the eight entries of one trip
     // with two 16-byte reads, the six of a trip over three slots with three of 8, and its first entry then sits
-    // on such a boundary)
-    for (int i = tid; i < (int)(nkv_pad / 32); i += THREADS) lds_ks[KS_OFF + i] = ksc[i >> ush];
+    // on such a boundary; those of the keys that count, however far the caller's cache goes on)
+    const int n_ks = (kv_valid_all + kPadKV - 1) / kPadKV * (kPadKV / 32);
+    for (int i = tid; i < n_ks; i += THREADS) lds_ks[KS_OFF + i] = ksc[i >> ush];
     auto kscale_of = [&](int u32blk) -> float { return lds_ks[KS_OFF + u32blk]; };
 
     // tile indices below are relative to the segment's first tile
@@ -1136,8 +1137,9 @@ static hipError_t launch_attn_dv(const AttnArgs& a, bool two_runs, hipStream_t s
     const int64_t first = two_runs ? 2 * a.main_items : 0;
     const int64_t total = two_runs || four ? (int64_t)n_qtiles * a.B * a.H - first : a.main_items;
     if (total <= 0 || first + total > 0x7FFFFFFF || first + total > (int64_t)n_qtiles * a.B * a.H) return hipErrorInvalidValue;
-    if (two_runs && (D > 128 || a.short_kw > 0 || a.split_wgs > 0 || a.nkv_pad > kTwoRunKeys || (VARIANT == 1 && a.amask != nullptr))) return hipErrorInvalidValue;
-    if (four && (a.amask != nullptr || a.two_runs || a.short_kw > 0 || a.split_wgs > 0 || a.nkv_pad > kTwoRunKeys)) return hipErrorInvalidValue;
+    const bool few_keys = pad_to(a.kv_valid, kPadKV) <= kTwoRunKeys;
+    if (two_runs && (D > 128 || a.short_kw > 0 || a.split_wgs > 0 || !few_keys || (VARIANT == 1 && a.amask != nullptr))) return hipErrorInvalidValue;
+    if (four && (a.amask != nullptr || a.two_runs || a.short_kw > 0 || a.split_wgs > 0 || !few_keys)) return hipErrorInvalidValue;
     const int split = (D <= 128 && VARIANT == 0 && !a.causal) ? a.split_wgs : 0;
     int* flags = nullptr;
     float* part = nullptr;
