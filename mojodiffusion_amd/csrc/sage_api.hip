@@ -823,10 +823,9 @@ int mi355_sage_attn_fwd_q16(const void* Q, const int64_t* q_strides, int64_t q_o
     int rc;
     if ((rc = check_kv_len(N_kv, blkk, D))) return rc;
     if ((rc = check_view("Q", Q, q_strides, q_off)) || (rc = check_view("O", O, o_strides, o_off))) return rc;
-    // (shapes that qualify for the split schedule keep the encoded-Q form here, whatever the plan)
     AttnArgs a{};
     const AttnPlan plan = attn_plan(B, H, N_q, kv_valid, D, variant, false);
-    if (plan.main_items > 0 && attn_split_workgroups(B, H, N_q, kv_valid, D, variant) > 0) return MI355_SAGE_EUNSUPPORTED;
+    if (attn_q8_only(plan, B, H, N_q, kv_valid, D, variant)) return MI355_SAGE_EUNSUPPORTED;
     a.main_items = plan.main_items; a.short_kw = plan.short_kw; a.two_runs = plan.two_runs; a.four_waves = plan.four_waves;
     const View q = make_view(Q, q_strides, q_off);
     a.q_src = q.p; a.qsb = q.sb; a.qsh = q.sh; a.qsn = q.sn; a.qmul = static_cast<const float*>(qmul); a.blkq = blkq;

@@ -812,61 +812,75 @@ Choice best_small(const FormCost* c, int64_t rows, int64_t bh, int D, int varian
     if (D <= 128) offer(c[RUNS8].of(wgs(32), (steps + 7) / 8, units), AttnPlan{0, 8, 0});
     return best;
 }
-}  // namespace
 
-// short_or_main: what the figures for all lengths say of those two alone.
-static AttnPlan plan_by_shape(int units, int B, int H, int Nq, int kv_valid, int D, int variant, bool causal, bool bias, int split, bool short_or_main = false) {
-    const int v = variant == 0 ? 0 : 1, d = D == 64 ? 0 : D == 128 ? 1 : 2;
-    const int64_t bh = (int64_t)B * H, tiles = (kv_valid + kTileKV - 1) / kTileKV;
-    const int rows = D > 128 ? 128 : 256;
-    const int64_t items = bh * ((Nq + rows - 1) / rows), whole = items / units * units;
-    const FormCost* by_length = D == 64 && v == 0 && tiles > 48 ? kCost64Long : kCostLong[d][v];
-    const int blkq = variant == 0 ? 128 : 32;
-    const int64_t alone = quant_short_workgroups(B, H, Nq, kv_valid, D, blkq, 64, false);
-    const int64_t with_q = alone > 0 ? quant_short_workgroups(B, H, Nq, kv_valid, D, blkq, 64, true) : 0;
-    const float q_cost = std::max(Nq > 2 * kv_valid ? kQCost[d][v][0] : 0.0f, alone > 0 && (with_q == 0 || with_q > units) ? kQCost[d][v][1] : 0.0f);
-    auto choose = [&](const FormCost* c, float q_main, float launch, bool two_runs) -> Choice {
-        // (past a round of row tiles the two-run form does what the main kernel's whole rounds leave: that is ahead of
-        // it doing everything, or level)
-        Choice best = best_small(c, Nq, bh, D, variant, kv_valid, units, two_runs && (causal || whole == 0 || whole == items));
-        const float main = c[MAIN].of(items, tiles, units) + q_main;
-        if (main <= best.t) best = Choice{main, AttnPlan{items, 0, 0}};
-        if (!causal && whole > 0 && whole < items) {
-            const Choice rest = best_small(c, rows, items - whole, D, variant, kv_valid, units, two_runs);
-            const float t = c[MAIN].of(whole, tiles, units) + q_main + launch + rest.t;
-            if (t < best.t) best = Choice{t, AttnPlan{whole, rest.p.short_kw, 0, rest.p.two_runs}};
-        }
-        return best;
-    };
-    if (!causal && split > 0 && D <= 128 &&
-        kSplitCost[d][0] + kSplitCost[d][1] * (float)(items * tiles) / 256.0f < choose(by_length, q_cost, 0.0f, false).t)
-        return AttnPlan{items, 0, split};
-    if (short_or_main) return choose(by_length, q_cost, 0.0f, false).p;
-    if (const int runs = fused_runs(units, B, H, Nq, kv_valid, D, variant)) return AttnPlan{0, runs, 0};
-    // (figures that were fitted to differences have not got what a second launch costs)
-    const float launch = d == 0 && v == 0 ? 0.0f : 3.0f;
-    const bool two_runs = D <= 128 && pad_to(kv_valid, kPadKV) <= kTwoRunKeys && !(bias && v == 1);
-    if (D <= 128 && bias && v == 0) return choose(kCostBias[d], 0.0f, 3.0f, two_runs).p;
-    if (D <= 128 && !bias && tiles <= 48) {
-        const Choice best = choose(kCost[d][v], 0.0f, launch, two_runs);
-        // Four waves: past a round of row tiles, but for the few that a second launch takes better (16 in 256).
-        const bool over = items > units && (tiles <= 4 || (items - whole) * 16 > units || items == whole);
-        const float four = kCostFour[d][v].of(bh * ((Nq + 127) / 128), tiles, 2 * units);
-        return over && four < best.t ? AttnPlan{items, 0, 0, false, true} : best.p;
+struct Problem {
+    int units, B, H, Nq, kv, D, variant;
+    bool causal, bias;
+    int64_t bh() const { return (int64_t)B * H; }
+    int64_t tiles() const { return (kv + kTileKV - 1) / kTileKV; }
+    int64_t items() const { const int rows = D > 128 ? 128 : 256; return bh() * ((Nq + rows - 1) / rows); }
+    int v() const { return variant == 0 ? 0 : 1; }
+    int d() const { return D == 64 ? 0 : D == 128 ? 1 : 2; }
+};
+
+Choice choose(const Problem& s, const FormCost* c, float q_main, float launch, bool two_runs) {
+    const int64_t items = s.items(), whole = items / s.units * s.units;
+    // (past a round of row tiles the two-run form does what the main kernel's whole rounds leave: that is ahead of
+    // it doing everything, or level)
+    Choice best = best_small(c, s.Nq, s.bh(), s.D, s.variant, s.kv, s.units, two_runs && (s.causal || whole == 0 || whole == items));
+    const float main = c[MAIN].of(items, s.tiles(), s.units) + q_main;
+    if (main <= best.t) best = Choice{main, AttnPlan{items, 0, 0}};
+    if (!s.causal && whole > 0 && whole < items) {
+        const Choice rest = best_small(c, s.D > 128 ? 128 : 256, items - whole, s.D, s.variant, s.kv, s.units, two_runs);
+        const float t = c[MAIN].of(whole, s.tiles(), s.units) + q_main + launch + rest.t;
+        if (t < best.t) best = Choice{t, AttnPlan{whole, rest.p.short_kw, 0, rest.p.two_runs}};
     }
-    return choose(by_length, q_cost, 0.0f, two_runs).p;
+    return best;
 }
 
-// 0: by shape; -1: never; 4, 8: always, that many key runs (4 at 256 channels)
+float q_cost(const Problem& s) {
+    const int blkq = s.variant == 0 ? 128 : 32;
+    const int64_t alone = quant_short_workgroups(s.B, s.H, s.Nq, s.kv, s.D, blkq, 64, false);
+    const int64_t with_q = alone > 0 ? quant_short_workgroups(s.B, s.H, s.Nq, s.kv, s.D, blkq, 64, true) : 0;
+    return std::max(s.Nq > 2 * s.kv ? kQCost[s.d()][s.v()][0] : 0.0f, alone > 0 && (with_q == 0 || with_q > s.units) ? kQCost[s.d()][s.v()][1] : 0.0f);
+}
+
+const FormCost* by_length(const Problem& s) { return s.D == 64 && s.v() == 0 && s.tiles() > 48 ? kCost64Long : kCostLong[s.d()][s.v()]; }
+
+// What the split schedule is compared with: main kernel and short form by the figures for all lengths.
+Choice main_or_short(const Problem& s) { return choose(s, by_length(s), q_cost(s), 0.0f, false); }
+bool split_ahead(const Problem& s, int split, const Choice& other) {
+    return !s.causal && split > 0 && s.D <= 128 && kSplitCost[s.d()][0] + kSplitCost[s.d()][1] * (float)(s.items() * s.tiles()) / 256.0f < other.t;
+}
+}  // namespace
+
+static AttnPlan plan_by_shape(const Problem& s, int split) {
+    if (split > 0 && split_ahead(s, split, main_or_short(s))) return AttnPlan{s.items(), 0, split};
+    if (const int runs = fused_runs(s.units, s.B, s.H, s.Nq, s.kv, s.D, s.variant)) return AttnPlan{0, runs, 0};
+    // (figures that were fitted to differences have not got what a second launch costs)
+    const float launch = s.d() == 0 && s.v() == 0 ? 0.0f : 3.0f;
+    const bool two_runs = s.D <= 128 && pad_to(s.kv, kPadKV) <= kTwoRunKeys && !(s.bias && s.v() == 1);
+    if (s.D <= 128 && s.bias && s.v() == 0) return choose(s, kCostBias[s.d()], 0.0f, 3.0f, two_runs).p;
+    if (s.D <= 128 && !s.bias && s.tiles() <= 48) {
+        const Choice best = choose(s, kCost[s.d()][s.v()], 0.0f, launch, two_runs);
+        // Four waves: past a round of row tiles, but for the few that a second launch takes better (16 in 256).
+        const int64_t items = s.items(), whole = items / s.units * s.units;
+        const bool over = items > s.units && (s.tiles() <= 4 || (items - whole) * 16 > s.units || items == whole);
+        const float four = kCostFour[s.d()][s.v()].of(s.bh() * ((s.Nq + 127) / 128), s.tiles(), 2 * s.units);
+        return over && four < best.t ? AttnPlan{items, 0, 0, false, true} : best.p;
+    }
+    return choose(s, by_length(s), q_cost(s), 0.0f, two_runs).p;
+}
+
 void attn_short_override(int mode) { g_short_mode.store(mode); }
 
 int attn_short_rule(int B, int H, int Nq, int kv_valid, int D, int variant) {
-    const AttnPlan p = plan_by_shape(256, B, H, Nq, kv_valid, D, variant, false, false, 0, true);
+    const AttnPlan p = main_or_short(Problem{256, B, H, Nq, kv_valid, D, variant, false, false}).p;
     return p.main_items == 0 ? p.short_kw : 0;
 }
 
 int64_t attn_main_items_on(int units, int B, int H, int Nq, int kv_valid, int D, int variant) {
-    return plan_by_shape(units, B, H, Nq, kv_valid, D, variant, false, false, 0).main_items;
+    return plan_by_shape(Problem{units, B, H, Nq, kv_valid, D, variant, false, false}, 0).main_items;
 }
 
 // Asked of the device once.  (256 where there is none to ask.)
@@ -892,7 +906,16 @@ AttnPlan attn_plan(int B, int H, int Nq, int kv_valid, int D, int variant, bool 
     const int split = causal ? 0 : attn_split_workgroups(B, H, Nq, kv_valid, D, variant);
     if (mode < 0 || attn_split_override_mode() != 0)      // (a schedule of the main kernel was asked for)
         return AttnPlan{(int64_t)B * H * ((Nq + rows - 1) / rows), 0, split};
-    return plan_by_shape(compute_units(), B, H, Nq, kv_valid, D, variant, causal, bias, split);
+    return plan_by_shape(Problem{compute_units(), B, H, Nq, kv_valid, D, variant, causal, bias}, split);
+}
+
+bool attn_q8_only(const AttnPlan& p, int B, int H, int Nq, int kv_valid, int D, int variant) {
+    const int split = attn_split_workgroups(B, H, Nq, kv_valid, D, variant);
+    if (split <= 0) return false;
+    if (g_short_mode.load() != 0 || attn_split_override_mode() != 0) return p.main_items > 0;
+    const Problem s{compute_units(), B, H, Nq, kv_valid, D, variant, false, false};
+    const Choice other = main_or_short(s);
+    return split_ahead(s, split, other) || other.p.main_items > 0;
 }
 
 }  // namespace sage

@@ -1,5 +1,5 @@
 """GPU tests of the attention stage's entry points where the choice of form meets their own arguments: key caches far longer
-than the keys that count."""
+than the keys that count, and shapes around those that mi355_sage_attn_fwd_q16 leaves to the encoded-Q form."""
 import pytest
 
 from mojodiffusion_amd import _lib
@@ -56,3 +56,22 @@ def test_cache_past_the_keys_that_two_runs_and_four_waves_stage(variant, D, mode
                 assert torch.isfinite(a.float()).all() and torch.equal(a, b), mask
     finally:
         L.mi355_sage_set_attn_short(0)
+
+
+@pytest.mark.parametrize("B,H,Sq,Skv,D,taken", [(3, 64, 257, 1770, 64, True), (4, 40, 311, 1084, 64, True), (3, 64, 285, 872, 64, True),
+                                                (1, 33, 2048, 2048, 128, False)])
+def test_shapes_that_the_stage_with_q_in_the_kernel_takes(B, H, Sq, Skv, D, taken):
+    """Considered by the split schedule: taken where the short form is ahead of it and of the main kernel by the figures for
+    all lengths, with the bits of the stage on encoded Q."""
+    import numpy as np
+    import gpu_harness as G
+    if _lib.lib().mi355_sage_attn_split_rule(B, H, Sq, Skv, D, 0) == 0:
+        pytest.skip("not a shape of the split schedule on this device")
+    rng = np.random.default_rng(Sq)
+    q, k, v = ((rng.standard_normal((B, n, H, D)).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16) for n in (Sq, Skv, Skv))
+    g, gv = G.quant_qk(q, k, D ** -0.5, 128, 64, True)["dev"], G.quant_v(v, 0)["dev"]
+    rc, got = G.attn_fwd_q16(q, g["qmul"], 128, g["k8"], g["kscale"], 64, gv["vq"], None, 0, Skv)
+    assert rc == (0 if taken else -2)
+    if taken:
+        want, _ = G.attn_fwd(g["q8"], g["qscale"], 128, g["k8"], g["kscale"], 64, gv["vq"], None, 0, Sq, Skv)
+        np.testing.assert_array_equal(got, want)
