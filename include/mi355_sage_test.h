@@ -39,12 +39,15 @@ int mi355_sage_attn_split_rule(int B, int H, int N_q, int N_kv, int D, int varia
  * a mode outside these. */
 int mi355_sage_set_attn_short(int mode);
 
-/* Key runs the short form would use for this shape where the choice is between it and the 256-row workgroups alone, 0 for
- * the latter. */
-int mi355_sage_attn_short_rule(int B, int H, int N_q, int N_kv, int D, int variant);
+/* The forms that a one-shot call of this shape takes (default blocks, no pre-ops) on the current device and under the
+ * current switches, six numbers: row tiles of the main kernel; key runs of the short form, which does the rest (or
+ * everything), 0 without it; 1: the two-run form does the rest (or everything); 1: the main kernel's row tiles in
+ * workgroups of four waves; workgroups of the split schedule, 0 without it; 1: the short form quantizes K and V
+ * itself (one launch).  causal and bias: whether the call has that mask.  Returns 0, or -1 for a bad shape. */
+int mi355_sage_attn_plan(int B, int H, int N_q, int N_kv, int D, int variant, int causal, int bias, int64_t* out);
 
 /* Row tiles (256 rows of a head; 128 at head dim 256) the main kernel would do for this shape on the current
- * device and under the current switches; the short form does the others. */
+ * device and under the current switches; the short or the two-run form does the others. */
 int64_t mi355_sage_attn_main_items(int B, int H, int N_q, int N_kv, int D, int variant);
 
 /* The same by the shape alone, on a device of that many compute units and without the split schedule. */

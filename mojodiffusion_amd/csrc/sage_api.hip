@@ -860,9 +860,12 @@ int mi355_sage_set_attn_short(int mode) {
     return MI355_SAGE_OK;
 }
 
-int mi355_sage_attn_short_rule(int B, int H, int N_q, int N_kv, int D, int variant) {
-    if (B <= 0 || H <= 0 || N_q <= 0 || N_kv <= 0) return 0;
-    return attn_short_rule(B, H, N_q, N_kv, D, variant);
+int mi355_sage_attn_plan(int B, int H, int N_q, int N_kv, int D, int variant, int causal, int bias, int64_t* out) {
+    if (B <= 0 || H <= 0 || N_q <= 0 || N_kv <= 0 || !dims_ok(D) || !out) return MI355_SAGE_EINVAL;
+    const AttnPlan p = attn_plan(B, H, N_q, N_kv, D, variant, causal != 0, bias != 0);
+    out[0] = p.main_items; out[1] = p.short_kw; out[2] = p.two_runs; out[3] = p.four_waves; out[4] = p.split_wgs;
+    out[5] = attn_fused_rule(p, B, H, N_q, N_kv, D, variant, default_blkq(variant), 64);
+    return MI355_SAGE_OK;
 }
 
 int64_t mi355_sage_attn_main_items(int B, int H, int N_q, int N_kv, int D, int variant) {

@@ -874,11 +874,6 @@ static AttnPlan plan_by_shape(const Problem& s, int split) {
 
 void attn_short_override(int mode) { g_short_mode.store(mode); }
 
-int attn_short_rule(int B, int H, int Nq, int kv_valid, int D, int variant) {
-    const AttnPlan p = main_or_short(Problem{256, B, H, Nq, kv_valid, D, variant, false, false}).p;
-    return p.main_items == 0 ? p.short_kw : 0;
-}
-
 int64_t attn_main_items_on(int units, int B, int H, int Nq, int kv_valid, int D, int variant) {
     return plan_by_shape(Problem{units, B, H, Nq, kv_valid, D, variant, false, false}, 0).main_items;
 }

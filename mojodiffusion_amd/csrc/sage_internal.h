@@ -199,7 +199,6 @@ struct FuseArgs {
 };
 hipError_t launch_attn_fused(const AttnArgs& a, const FuseArgs& f, hipStream_t st);
 bool attn_fused_rule(const AttnPlan& p, int B, int H, int Nq, int kv_valid, int D, int variant, int blkq, int blkk);
-int attn_short_rule(int B, int H, int Nq, int kv_valid, int D, int variant);     // short_kw where the short form does everything by shape, else 0
 // Shapes that mi355_sage_attn_fwd_q16 leaves to the encoded-Q form: the split schedule considers them, and it or the main
 // kernel is ahead of the short form by the figures for all lengths — whatever form the plan p gives them in the end.
 bool attn_q8_only(const AttnPlan& p, int B, int H, int Nq, int kv_valid, int D, int variant);

@@ -73,19 +73,37 @@ def test_split_schedule_is_a_function_of_the_shape():
         assert L.mi355_sage_set_attn_split(bad) == -1
 
 
+def attn_plan(B, H, Sq, Skv, D, variant, causal=0, bias=0):
+    """The form a call takes: "main", "short4", "short8", "one launch", "two runs", "four waves", "split", or "main + .."."""
+    out = (ctypes.c_int64 * 6)()
+    assert _lib.lib().mi355_sage_attn_plan(B, H, Sq, Skv, D, variant, causal, bias, out) == 0
+    main, short, two, four, split, one = out
+    if one or split or four:
+        return "one launch" if one else "split" if split else "four waves"
+    rest = "two runs" if two else "short%d" % short if short else ""
+    return ("main + " + rest if rest else "main") if main else rest
+
+
 def test_form_of_the_attention_kernel_by_shape():
-    """The short form (the keys split over a workgroup's waves) is for problems that do not fill the chip, whatever the
-    length: timed on an MI355X, it is behind the 256-row workgroups from about 75 (128 channels, fp16) to 190 (64
-    channels, e4m3) of them on, and ahead below half of that."""
-    rule = _lib.lib().mi355_sage_attn_short_rule
+    """The forms that split the keys are for problems that do not fill the chip, whatever the length; what they
+    measured against the others stands beside the rule."""
     for B, H, S, D, variant in [(1, 12, 16384, 64, 1), (1, 4, 16384, 64, 1), (2, 24, 16384, 64, 1), (1, 30, 12288, 64, 1), (1, 4, 12288, 128, 1),
-                                (1, 8, 12288, 64, 0), (1, 12, 8192, 64, 0), (1, 8, 10240, 128, 0), (1, 24, 4608, 128, 0), (1, 40, 2304, 64, 0)]:
-        assert rule(B, H, S, S, D, variant) == 0, (B, H, S, D, variant)
-    for B, H, S, D, variant in [(1, 4, 2048, 64, 1), (1, 4, 2048, 128, 0), (1, 2, 8192, 64, 1), (1, 1, 8192, 128, 1), (1, 8, 1024, 64, 0), (1, 30, 256, 128, 0)]:
-        assert rule(B, H, S, S, D, variant) in (4, 8), (B, H, S, D, variant)
-    # where Q stays in the main kernel's prologue: many queries on few keys, or K and V take one launch but not with Q
-    assert rule(1, 24, 510, 139, 128, 0) == rule(1, 40, 256, 292, 128, 0) == rule(2, 32, 71, 45, 256, 1) == rule(2, 30, 128, 26, 256, 1) == 4
-    assert rule(1, 24, 64, 64, 128, 0) == rule(1, 24, 64, 49, 128, 0) == 0
+                                (1, 12, 8192, 64, 0), (1, 8, 10240, 128, 0), (1, 24, 4608, 128, 0)]:
+        assert attn_plan(B, H, S, S, D, variant) in ("main", "main + short4", "main + short8", "main + two runs"), (B, H, S, D, variant)
+    for B, H, S, D, variant in [(1, 4, 2048, 64, 1), (1, 4, 2048, 128, 0), (1, 2, 8192, 64, 1), (1, 1, 8192, 128, 1), (1, 8, 1024, 64, 0)]:
+        assert attn_plan(B, H, S, S, D, variant) in ("short4", "short8"), (B, H, S, D, variant)
+    for B, H, S, D, variant in [(1, 19, 1127, 128, 0), (1, 16, 1091, 128, 0), (2, 16, 615, 128, 1), (1, 19, 1127, 64, 0)]:
+        assert attn_plan(B, H, S, S, D, variant) == "two runs", (B, H, S, D, variant)
+    assert attn_plan(1, 24, 1153, 1153, 128, 0, bias=1) == "two runs" and attn_plan(1, 24, 1153, 1153, 128, 1, bias=1) != "two runs"
+    assert attn_plan(1, 40, 3792, 341, 128, 0) == attn_plan(2, 30, 6224, 63, 64, 0) == attn_plan(2, 40, 775, 775, 64, 0) == "four waves"
+    # one launch: up to 256 keys of 128 channels, 512 of 64, a compute unit for every 64 rows at least, fp16 P.V
+    assert attn_plan(1, 30, 256, 256, 128, 0) == attn_plan(1, 24, 64, 64, 128, 0) == attn_plan(1, 8, 512, 512, 64, 0) == "one launch"
+    assert "one launch" not in (attn_plan(1, 30, 257, 257, 128, 0), attn_plan(1, 30, 256, 256, 128, 1), attn_plan(3, 30, 256, 256, 128, 0), attn_plan(1, 8, 513, 513, 64, 0))
+    # 256 channels: the main kernel and the short form
+    assert attn_plan(1, 18, 1153, 1153, 256, 0) == "main" and attn_plan(2, 32, 71, 45, 256, 1) == "short4"
+    # causal calls are one launch of the attention kernel
+    assert "+" not in attn_plan(1, 24, 4608, 4608, 128, 0, causal=1)
+    assert _lib.lib().mi355_sage_attn_plan(1, 24, 64, 64, 96, 0, 0, 0, (ctypes.c_int64 * 6)()) == -1
 
 
 def test_forms_scale_with_the_compute_units():

@@ -107,7 +107,14 @@ def test_full_rounds_by_the_main_kernel_and_the_rest_by_the_short_form(variant, 
 def test_short_form_rule():
     """By shape: small problems take it, problems that fill the chip with 256-row workgroups do not; a
     forced schedule of those workgroups keeps it out."""
-    rule = _lib.lib().mi355_sage_attn_short_rule
-    assert rule(1, 30, 256, 256, 128, 0) == 8 and rule(1, 8, 1024, 1024, 64, 0) == 8 and rule(1, 1, 1, 1, 128, 1) > 0
-    assert rule(1, 24, 4608, 4608, 128, 0) == 0 and rule(1, 24, 16896, 16896, 128, 1) == 0 and rule(2, 30, 1248, 1248, 128, 0) == 0
-    assert _lib.lib().mi355_sage_set_attn_short(5) == -1
+    from test_abi_exports import attn_plan
+    L = _lib.lib()
+    assert attn_plan(1, 30, 256, 256, 128, 0) == "one launch" and attn_plan(1, 8, 1024, 1024, 64, 0) == "short8"
+    assert attn_plan(1, 1, 1, 1, 128, 1) in ("short4", "short8")
+    assert not any("short" in attn_plan(*x) for x in ((1, 24, 4608, 4608, 128, 0), (2, 30, 1248, 1248, 128, 0)))
+    assert L.mi355_sage_set_attn_split(-1) == 0
+    try:
+        assert attn_plan(1, 30, 256, 256, 128, 0) == attn_plan(1, 8, 1024, 1024, 64, 0) == "main"
+    finally:
+        L.mi355_sage_set_attn_split(0)
+    assert L.mi355_sage_set_attn_short(5) == -1
