@@ -18,6 +18,8 @@
  *     Ideogram-4 arm uses it (serenitymojo/models/dit/ideogram4_dit.mojo:29-49) — 256;
  *     attention is full and non-causal; trailing keys (real_N_kv) or one range of keys
  *     (_keymask) can be masked; N_q may differ from N_kv;
+ *   - O and Stats of the one-shot forward calls may lie over Q, K or V (which are then all read before
+ *     anything is written), not over a bias; nothing else a call writes may overlap what it reads;
  *   - return 0 on success; -1 for a null pointer, a non-positive dimension or
  *     null strides (serenitymojo/ops/cshim/cudnn_sdpa.cpp:391-393); -2 for an
  *     unsupported configuration; -3 for a workspace that is too small; a

@@ -295,6 +295,17 @@ struct MaskArgs {
     bool any_row_start = false;        // rows of the bias may start at any even byte address
 };
 
+// The bytes from a view's first element to its last, for whether two may share memory.
+struct Bytes { uintptr_t lo, hi; };
+Bytes view_bytes(const void* p, const int64_t* s, int64_t off, int B, int H, int N, int D) {
+    int64_t lo = off, hi = off + D;
+    const int64_t last[3] = {(B - 1) * s[0], (H - 1) * s[1], (N - 1) * s[2]};
+    for (int64_t x : last) (x < 0 ? lo : hi) += x;
+    const uintptr_t base = reinterpret_cast<uintptr_t>(p);
+    return Bytes{base + (uintptr_t)(lo * 2), base + (uintptr_t)(hi * 2)};
+}
+bool meet(const Bytes& a, const Bytes& b) { return a.lo < b.hi && b.lo < a.hi; }
+
 int sdpa_impl(const void* Q, const void* K, const void* V, void* O, void* Stats,
               int B, int H, int N_q, int N_kv, int D, float scale,
               const int64_t* qs, const int64_t* ks, const int64_t* vs, const int64_t* os,
@@ -377,9 +388,21 @@ int sdpa_impl(const void* Q, const void* K, const void* V, void* O, void* Stats,
         const int64_t wgs = one_launch(true);
         q_in_encoders = wgs > 0 && wgs <= units;
     }
+    // Outputs that lie over Q, K or V: all three are read by the quantizers' launches then, before the attention kernel
+    // writes anything.
+    bool over_q = false, over_kv = false;
+    {
+        const Bytes q = view_bytes(Q, qs, q_off, B, H, N_q, D), k = view_bytes(K, ks, k_off, B, H, N_kv, D), v = view_bytes(V, vs, v_off, B, H, N_kv, D);
+        const uintptr_t st0 = reinterpret_cast<uintptr_t>(Stats) + (uintptr_t)(stats_off * 4);
+        const Bytes outs[2] = {view_bytes(O, os, o_off, B, H, N_q, D), Stats ? Bytes{st0, st0 + (uintptr_t)((int64_t)B * H * N_q * 4)} : Bytes{0, 0}};
+        for (const Bytes& x : outs) {
+            over_q = over_q || meet(x, q);
+            over_kv = over_kv || meet(x, k) || meet(x, v);
+        }
+    }
     const bool q_in_kernel = Stats == nullptr && mask.add == nullptr && pre.q.gain == nullptr && (D <= 128 || plan.main_items == 0) &&
-                             plan.split_wgs == 0 && !q_in_encoders;
-    if (pre.q.gain == nullptr && attn_fused_rule(plan, B, H, N_q, kv, D, variant, blkq, blkk)) {
+                             plan.split_wgs == 0 && !q_in_encoders && !over_q;
+    if (pre.q.gain == nullptr && !over_q && !over_kv && attn_fused_rule(plan, B, H, N_q, kv, D, variant, blkq, blkk)) {
         const View q = make_view(Q, qs, q_off);
         AttnArgs a{};
         a.blkq = blkq; a.blkk = blkk; a.variant = variant; a.km = km;
