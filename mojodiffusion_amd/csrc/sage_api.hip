@@ -389,14 +389,16 @@ int sdpa_impl(const void* Q, const void* K, const void* V, void* O, void* Stats,
         q_in_encoders = wgs > 0 && wgs <= units;
     }
     // Outputs that lie over Q, K or V: all three are read by the quantizers' launches then, before the attention kernel
-    // writes anything.
+    // writes anything.  (O in Q's own rows needs that in the short form only: elsewhere a workgroup that encodes Q has whole
+    // scale blocks, which it reads before it writes.)
     bool over_q = false, over_kv = false;
     {
         const Bytes q = view_bytes(Q, qs, q_off, B, H, N_q, D), k = view_bytes(K, ks, k_off, B, H, N_kv, D), v = view_bytes(V, vs, v_off, B, H, N_kv, D);
         const uintptr_t st0 = reinterpret_cast<uintptr_t>(Stats) + (uintptr_t)(stats_off * 4);
         const Bytes outs[2] = {view_bytes(O, os, o_off, B, H, N_q, D), Stats ? Bytes{st0, st0 + (uintptr_t)((int64_t)B * H * N_q * 4)} : Bytes{0, 0}};
         for (const Bytes& x : outs) {
-            over_q = over_q || meet(x, q);
+            const bool own_rows = &x == outs && plan.short_kw == 0 && x.lo == q.lo && os[0] == qs[0] && os[1] == qs[1] && os[2] == qs[2];
+            over_q = over_q || (meet(x, q) && !own_rows);
             over_kv = over_kv || meet(x, k) || meet(x, v);
         }
     }
