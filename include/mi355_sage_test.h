@@ -43,8 +43,9 @@ int mi355_sage_set_attn_short(int mode);
  * current switches, six numbers: row tiles of the main kernel; key runs of the short form, which does the rest (or
  * everything), 0 without it; 1: the two-run form does the rest (or everything); 1: the main kernel's row tiles in
  * workgroups of four waves; workgroups of the split schedule, 0 without it; 1: the short form quantizes K and V
- * itself (one launch).  causal and bias: whether the call has that mask.  Returns 0, or -1 for a bad shape. */
-int mi355_sage_attn_plan(int B, int H, int N_q, int N_kv, int D, int variant, int causal, int bias, int64_t* out);
+ * itself (one launch).  causal and bias: whether the call has that mask; masked: keys of a
+ * masked range.  Returns 0, or -1 for a bad shape. */
+int mi355_sage_attn_plan(int B, int H, int N_q, int N_kv, int D, int variant, int causal, int bias, int masked, int64_t* out);
 
 /* Row tiles (256 rows of a head; 128 at head dim 256) the main kernel would do for this shape on the current
  * device and under the current switches; the short or the two-run form does the others. */

@@ -65,7 +65,7 @@ SIGNATURES = {
     "mi355_sage_attn_split_rule": (_int, [_int] * 6),
     "mi355_sage_set_attn_split": (_int, [_int]),
     "mi355_sage_set_attn_short": (_int, [_int]),
-    "mi355_sage_attn_plan": (_int, [_int] * 8 + [_i64p]),
+    "mi355_sage_attn_plan": (_int, [_int] * 9 + [_i64p]),
     "mi355_sage_attn_main_items": (_i64, [_int] * 6),
     "mi355_sage_attn_main_items_on": (_i64, [_int] * 7),
     "mi355_sage_set_attn_split_wait": (_int, [_int]),

@@ -364,7 +364,7 @@ int sdpa_impl(const void* Q, const void* K, const void* V, void* O, void* Stats,
     }
     // (one decision for carving and launching; slots the caller's workspace was not sized for — a
     // forced schedule of the test switch — come from the library's per-stream buffer)
-    const AttnPlan plan = attn_plan(B, H, N_q, kv, D, variant, causal != 0, mask.add != nullptr);
+    const AttnPlan plan = attn_plan(B, H, N_q, kv, D, variant, causal != 0, mask.add != nullptr, km.hi - km.lo);
     // The plain forward leaves Q to the attention kernel, which encodes its own rows (same codes and
     // scales): the quantize stage then neither reads Q nor writes its codes.
     // Not where the encoders have room for it and a prologue is on the path of the whole call — the main kernel does
@@ -826,7 +826,7 @@ int mi355_sage_attn_fwd(const void* q8, const void* qscale, int blkq, const void
     a.stats = static_cast<float*>(stats);
     // Same scheduling, hence the same bits, as the one-shot calls: shapes that are split over a
     // fixed number of workgroups need hand-over slots, kept per (device, stream) by the library.
-    const AttnPlan plan = attn_plan(B, H, N_q, kv_valid, D, variant, false);
+    const AttnPlan plan = attn_plan(B, H, N_q, kv_valid, D, variant, false, false, a.km.hi - a.km.lo);
     a.main_items = plan.main_items; a.short_kw = plan.short_kw; a.split_wgs = plan.split_wgs; a.two_runs = plan.two_runs; a.four_waves = plan.four_waves;
     std::lock_guard<std::mutex> together(launch_mutex(static_cast<hipStream_t>(stream)));
     const size_t split_bytes = attn_split_bytes(a.split_wgs, D);
@@ -849,7 +849,8 @@ int mi355_sage_attn_fwd_q16(const void* Q, const int64_t* q_strides, int64_t q_o
     if ((rc = check_kv_len(N_kv, blkk, D))) return rc;
     if ((rc = check_view("Q", Q, q_strides, q_off)) || (rc = check_view("O", O, o_strides, o_off))) return rc;
     AttnArgs a{};
-    const AttnPlan plan = attn_plan(B, H, N_q, kv_valid, D, variant, false);
+    const bool keys = clip_mask(kv_valid, mask_lo, mask_hi, &a.km) > 0;
+    const AttnPlan plan = attn_plan(B, H, N_q, kv_valid, D, variant, false, false, a.km.hi - a.km.lo);
     if (attn_q8_only(plan, B, H, N_q, kv_valid, D, variant)) return MI355_SAGE_EUNSUPPORTED;
     a.main_items = plan.main_items; a.short_kw = plan.short_kw; a.two_runs = plan.two_runs; a.four_waves = plan.four_waves;
     const View q = make_view(Q, q_strides, q_off);
@@ -857,7 +858,7 @@ int mi355_sage_attn_fwd_q16(const void* Q, const int64_t* q_strides, int64_t q_o
     a.k8 = static_cast<const int8_t*>(k8); a.kscale = static_cast<const float*>(kscale); a.blkk = blkk;
     a.vq = vq; a.vscale = static_cast<const float*>(vscale);
     a.variant = variant;
-    if (clip_mask(kv_valid, mask_lo, mask_hi, &a.km) <= 0) return MI355_SAGE_EINVAL;
+    if (!keys) return MI355_SAGE_EINVAL;
     a.B = B; a.H = H; a.Nq = N_q; a.Nkv = N_kv; a.kv_valid = kv_valid; a.D = D;
     a.nq_pad = pad_to(N_q, kTileQ); a.nkv_pad = pad_to(N_kv, kPadKV);
     a.o = static_cast<uint16_t*>(O) + o_off; a.osb = o_strides[0]; a.osh = o_strides[1]; a.osn = o_strides[2];
@@ -885,9 +886,9 @@ int mi355_sage_set_attn_short(int mode) {
     return MI355_SAGE_OK;
 }
 
-int mi355_sage_attn_plan(int B, int H, int N_q, int N_kv, int D, int variant, int causal, int bias, int64_t* out) {
-    if (B <= 0 || H <= 0 || N_q <= 0 || N_kv <= 0 || !dims_ok(D) || !out) return MI355_SAGE_EINVAL;
-    const AttnPlan p = attn_plan(B, H, N_q, N_kv, D, variant, causal != 0, bias != 0);
+int mi355_sage_attn_plan(int B, int H, int N_q, int N_kv, int D, int variant, int causal, int bias, int masked, int64_t* out) {
+    if (B <= 0 || H <= 0 || N_q <= 0 || N_kv <= 0 || masked < 0 || masked >= N_kv || !dims_ok(D) || !out) return MI355_SAGE_EINVAL;
+    const AttnPlan p = attn_plan(B, H, N_q, N_kv, D, variant, causal != 0, bias != 0, masked);
     out[0] = p.main_items; out[1] = p.short_kw; out[2] = p.two_runs; out[3] = p.four_waves; out[4] = p.split_wgs;
     out[5] = attn_fused_rule(p, B, H, N_q, N_kv, D, variant, default_blkq(variant), 64);
     return MI355_SAGE_OK;

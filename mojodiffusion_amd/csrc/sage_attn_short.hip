@@ -778,6 +778,20 @@ static const FormCost kCostBias[2][FORMS] = {
     {{0.00f, 7.38f, 1.37f, 19.88f, 0.04f}, {4.24f, 3.73f, 0.78f, 11.53f, 0.00f}, {8.78f, 0.70f, 0.52f, 5.33f, 0.71f}, {7.37f, 1.30f, 0.00f, 2.40f, 1.24f}},
     {{0.00f, 14.94f, 1.53f, 14.28f, 0.06f}, {11.61f, 3.82f, 0.90f, 9.82f, 0.00f}, {10.61f, 5.30f, 0.78f, 3.42f, 0.85f}, {10.33f, 5.25f, 0.32f, 1.00f, 1.35f}},
 };
+// fp16 P.V with a masked key range (438 one-shot calls at 64 channels, 158 at 128, of 130 to 3072 tokens and up to a round of row
+// tiles; steps: of the keys that count; taken up to 40 key tiles), and causal (218 and 555, with and without Stats).  A range costs the main kernel and the
+// two-run form 2 to 6 us that the short form does not know: the steps around it go through their general bodies.  By the figures
+// of plain calls the two-run form or the main kernel was taken where the short one is ahead: us, so -> by these, [2,1439,4,128] 35.1 -> 29.3,
+// [1,940,30,64] 31.3 -> 28.9, causal [2,1303,12,64] 34.6 -> 30.4.  Over those calls the choice costs 0.4, 0.1, 0.5 and 0.1 % on average
+// over the best single form (the worst 13 %), by the plain figures 3.9, 0.6, 2.3 and 0.7 %.
+static const FormCost kCostRange[2][FORMS] = {
+    {{3.23f, 5.60f, 0.61f, 7.13f, 0.00f}, {1.02f, 6.46f, 0.29f, 5.39f, 0.00f}, {3.07f, 0.67f, 0.27f, 1.66f, 0.32f}, {1.04f, 2.46f, 0.00f, 0.00f, 0.53f}},
+    {{4.96f, 3.84f, 0.79f, 4.61f, 0.00f}, {0.36f, 8.41f, 0.41f, 2.37f, 0.02f}, {0.72f, 4.72f, 0.72f, 0.00f, 0.37f}, {0.26f, 4.24f, 0.69f, 0.00f, 0.36f}},
+};
+static const FormCost kCostCausal[2][FORMS] = {
+    {{1.36f, 5.53f, 0.50f, 1.86f, 0.00f}, {4.58f, 2.83f, 0.07f, 0.84f, 0.16f}, {4.98f, 0.35f, 0.10f, 0.91f, 0.27f}, {2.72f, 0.97f, 0.00f, 1.15f, 0.24f}},
+    {{7.41f, 2.10f, 0.62f, 5.27f, 0.00f}, {6.15f, 4.04f, 0.15f, 2.70f, 0.13f}, {5.09f, 4.20f, 0.10f, 0.77f, 0.51f}, {3.79f, 3.85f, 0.00f, 1.20f, 0.40f}},
+};
 // All lengths, by launches and calls of up to 32 768 keys of earlier forms of the kernels (the two-run form against the
 // main kernel's figures here): longer key sequences, 256 channels, and what the split schedule is compared with.
 static const FormCost kCostLong[3][2][FORMS] = {        // [64, 128, 256 channels]
@@ -802,12 +816,12 @@ static const float kQCost[3][2][2] = {{{0.0f, 0.0f}, {0.8f, 0.0f}}, {{1.4f, 1.4f
 namespace {
 struct Choice { float t; AttnPlan p; };
 // `rows` query rows of each of bh heads by the form that is predicted fastest, the main kernel's left out
-Choice best_small(const FormCost* c, int64_t rows, int64_t bh, int D, int variant, int64_t kv, int units, bool two_runs) {
+Choice best_small(const FormCost* c, int64_t rows, int64_t bh, int D, int variant, int64_t kv, int units, bool two_runs, float range = 0.0f) {
     const int64_t tiles = (kv + kTileKV - 1) / kTileKV, steps = variant == 0 ? (kv + 31) / 32 : tiles;
     auto wgs = [&](int per) { return bh * ((rows + per - 1) / per); };
     Choice best{1e30f, AttnPlan{0, 4, 0}};
     auto offer = [&](float t, const AttnPlan& p) { if (t < best.t) best = Choice{t, p}; };
-    if (two_runs) offer(c[TWO_RUNS].of(wgs(128), variant == 0 ? tiles : (tiles + 1) / 2 * 2, units), AttnPlan{0, 0, 0, true});
+    if (two_runs) offer(c[TWO_RUNS].of(wgs(128), variant == 0 ? tiles : (tiles + 1) / 2 * 2, units) + range, AttnPlan{0, 0, 0, true});
     offer(c[RUNS4].of(wgs(D > 128 ? 32 : 64), (steps + 3) / 4, units), AttnPlan{0, 4, 0});
     if (D <= 128) offer(c[RUNS8].of(wgs(32), (steps + 7) / 8, units), AttnPlan{0, 8, 0});
     return best;
@@ -816,6 +830,7 @@ Choice best_small(const FormCost* c, int64_t rows, int64_t bh, int D, int varian
 struct Problem {
     int units, B, H, Nq, kv, D, variant;
     bool causal, bias;
+    int masked;                 // keys of the masked range
     int64_t bh() const { return (int64_t)B * H; }
     int64_t tiles() const { return (kv + kTileKV - 1) / kTileKV; }
     int64_t items() const { const int rows = D > 128 ? 128 : 256; return bh() * ((Nq + rows - 1) / rows); }
@@ -831,8 +846,10 @@ Choice choose(const Problem& s, const FormCost* c, float q_main, float launch, b
     const float main = c[MAIN].of(items, s.tiles(), s.units) + q_main;
     if (main <= best.t) best = Choice{main, AttnPlan{items, 0, 0}};
     if (!s.causal && whole > 0 && whole < items) {
-        const Choice rest = best_small(c, s.D > 128 ? 128 : 256, items - whole, s.D, s.variant, s.kv, s.units, two_runs);
-        const float t = c[MAIN].of(whole, s.tiles(), s.units) + q_main + launch + rest.t;
+        // (a masked range: 3 us of the two-run form that the short form does not know, and the main kernel has either way)
+        const float range = s.masked > 0 ? 3.0f : 0.0f;
+        const Choice rest = best_small(c, s.D > 128 ? 128 : 256, items - whole, s.D, s.variant, s.kv, s.units, two_runs, range);
+        const float t = c[MAIN].of(whole, s.tiles(), s.units) + q_main + launch + rest.t - (rest.p.two_runs ? range : 0.0f);
         if (t < best.t) best = Choice{t, AttnPlan{whole, rest.p.short_kw, 0, rest.p.two_runs}};
     }
     return best;
@@ -861,6 +878,11 @@ static AttnPlan plan_by_shape(const Problem& s, int split) {
     const float launch = s.d() == 0 && s.v() == 0 ? 0.0f : 3.0f;
     const bool two_runs = s.D <= 128 && pad_to(s.kv, kPadKV) <= kTwoRunKeys && !(s.bias && s.v() == 1);
     if (s.D <= 128 && s.bias && s.v() == 0) return choose(s, kCostBias[s.d()], 0.0f, 3.0f, two_runs).p;
+    if (s.D <= 128 && !s.bias && s.v() == 0 && s.items() <= s.units && (s.causal || s.masked > 0) && s.tiles() > 2 && s.tiles() <= 40) {
+        Problem counted = s;
+        counted.kv -= s.masked;
+        return choose(counted, (s.causal ? kCostCausal : kCostRange)[s.d()], 0.0f, 0.0f, two_runs).p;
+    }
     if (s.D <= 128 && !s.bias && s.tiles() <= 48) {
         const Choice best = choose(s, kCost[s.d()][s.v()], 0.0f, launch, two_runs);
         // Four waves: past a round of row tiles, but for the few that a second launch takes better (16 in 256).
@@ -875,7 +897,7 @@ static AttnPlan plan_by_shape(const Problem& s, int split) {
 void attn_short_override(int mode) { g_short_mode.store(mode); }
 
 int64_t attn_main_items_on(int units, int B, int H, int Nq, int kv_valid, int D, int variant) {
-    return plan_by_shape(Problem{units, B, H, Nq, kv_valid, D, variant, false, false}, 0).main_items;
+    return plan_by_shape(Problem{units, B, H, Nq, kv_valid, D, variant, false, false, 0}, 0).main_items;
 }
 
 // Asked of the device once.  (256 where there is none to ask.)
@@ -891,7 +913,7 @@ int compute_units() {
     return n;
 }
 
-AttnPlan attn_plan(int B, int H, int Nq, int kv_valid, int D, int variant, bool causal, bool bias) {
+AttnPlan attn_plan(int B, int H, int Nq, int kv_valid, int D, int variant, bool causal, bool bias, int masked) {
     const int mode = g_short_mode.load(), rows = D > 128 ? 128 : 256;
     const bool two_runs_fit = D <= 128 && pad_to(kv_valid, kPadKV) <= kTwoRunKeys && !(bias && variant != 0);
     if (mode == 2 && two_runs_fit) return AttnPlan{0, 0, 0, true};
@@ -901,14 +923,14 @@ AttnPlan attn_plan(int B, int H, int Nq, int kv_valid, int D, int variant, bool 
     const int split = causal ? 0 : attn_split_workgroups(B, H, Nq, kv_valid, D, variant);
     if (mode < 0 || attn_split_override_mode() != 0)      // (a schedule of the main kernel was asked for)
         return AttnPlan{(int64_t)B * H * ((Nq + rows - 1) / rows), 0, split};
-    return plan_by_shape(Problem{compute_units(), B, H, Nq, kv_valid, D, variant, causal, bias}, split);
+    return plan_by_shape(Problem{compute_units(), B, H, Nq, kv_valid, D, variant, causal, bias, masked}, split);
 }
 
 bool attn_q8_only(const AttnPlan& p, int B, int H, int Nq, int kv_valid, int D, int variant) {
     const int split = attn_split_workgroups(B, H, Nq, kv_valid, D, variant);
     if (split <= 0) return false;
     if (g_short_mode.load() != 0 || attn_split_override_mode() != 0) return p.main_items > 0;
-    const Problem s{compute_units(), B, H, Nq, kv_valid, D, variant, false, false};
+    const Problem s{compute_units(), B, H, Nq, kv_valid, D, variant, false, false, 0};
     const Choice other = main_or_short(s);
     return split_ahead(s, split, other) || other.p.main_items > 0;
 }

@@ -185,7 +185,8 @@ struct AttnPlan {
     bool two_runs = false;   // the two-run form: the main kernel's loop, 128 rows per workgroup, two key runs over its waves
     bool four_waves = false; // the main kernel's items (then all of them) in workgroups of four waves, two to a compute unit
 };
-AttnPlan attn_plan(int B, int H, int Nq, int kv_valid, int D, int variant, bool causal, bool bias = false);
+// masked: keys of the masked range
+AttnPlan attn_plan(int B, int H, int Nq, int kv_valid, int D, int variant, bool causal, bool bias = false, int masked = 0);
 int compute_units();        // of the current device
 int64_t attn_main_items_on(int units, int B, int H, int Nq, int kv_valid, int D, int variant);       // the plan by shape on that many compute units
 hipError_t launch_attn_short(const AttnArgs& a, hipStream_t st);

@@ -73,10 +73,10 @@ def test_split_schedule_is_a_function_of_the_shape():
         assert L.mi355_sage_set_attn_split(bad) == -1
 
 
-def attn_plan(B, H, Sq, Skv, D, variant, causal=0, bias=0):
+def attn_plan(B, H, Sq, Skv, D, variant, causal=0, bias=0, masked=0):
     """The form a call takes: "main", "short4", "short8", "one launch", "two runs", "four waves", "split", or "main + .."."""
     out = (ctypes.c_int64 * 6)()
-    assert _lib.lib().mi355_sage_attn_plan(B, H, Sq, Skv, D, variant, causal, bias, out) == 0
+    assert _lib.lib().mi355_sage_attn_plan(B, H, Sq, Skv, D, variant, causal, bias, masked, out) == 0
     main, short, two, four, split, one = out
     if one or split or four:
         return "one launch" if one else "split" if split else "four waves"
@@ -103,7 +103,11 @@ def test_form_of_the_attention_kernel_by_shape():
     assert attn_plan(1, 18, 1153, 1153, 256, 0) == "main" and attn_plan(2, 32, 71, 45, 256, 1) == "short4"
     # causal calls are one launch of the attention kernel
     assert "+" not in attn_plan(1, 24, 4608, 4608, 128, 0, causal=1)
-    assert _lib.lib().mi355_sage_attn_plan(1, 24, 64, 64, 96, 0, 0, 0, (ctypes.c_int64 * 6)()) == -1
+    # two runs: behind the short form under a masked range or causal
+    for shape, masked in (((2, 4, 1439, 1439, 128, 0), 454), ((1, 30, 940, 940, 64, 0), 203)):
+        assert attn_plan(*shape) == "two runs" and "short" in attn_plan(*shape, masked=masked), shape
+    assert "short" in attn_plan(2, 12, 1303, 1303, 64, 0, causal=1) and "short" not in attn_plan(2, 12, 1303, 1303, 64, 0)
+    assert _lib.lib().mi355_sage_attn_plan(1, 24, 64, 64, 96, 0, 0, 0, 0, (ctypes.c_int64 * 6)()) == -1
 
 
 def test_forms_scale_with_the_compute_units():
