@@ -103,7 +103,8 @@ def test_form_of_the_attention_kernel_by_shape():
     assert attn_plan(1, 18, 1153, 1153, 256, 0) == "main" and attn_plan(2, 32, 71, 45, 256, 1) == "short4"
     # causal calls are one launch of the attention kernel
     assert "+" not in attn_plan(1, 24, 4608, 4608, 128, 0, causal=1)
-    # two runs: behind the short form under a masked range or causal
+    # two runs: not of two key tiles, and behind the short form under a masked range or causal
+    assert attn_plan(1, 30, 926, 89, 128, 1) == attn_plan(2, 24, 570, 44, 128, 0) == "main"
     for shape, masked in (((2, 4, 1439, 1439, 128, 0), 454), ((1, 30, 940, 940, 64, 0), 203)):
         assert attn_plan(*shape) == "two runs" and "short" in attn_plan(*shape, masked=masked), shape
     assert "short" in attn_plan(2, 12, 1303, 1303, 64, 0, causal=1) and "short" not in attn_plan(2, 12, 1303, 1303, 64, 0)
