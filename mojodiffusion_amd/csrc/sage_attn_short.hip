@@ -886,10 +886,15 @@ static AttnPlan plan_by_shape(const Problem& s, int split) {
     }
     if (s.D <= 128 && !s.bias && s.tiles() <= 48) {
         const Choice best = choose(s, kCost[s.d()][s.v()], 0.0f, launch, two_runs);
-        // Four waves: past a round of row tiles, but for the few that a second launch takes better (16 in 256).
-        const int64_t items = s.items(), whole = items / s.units * s.units;
-        const bool over = items > s.units && (s.tiles() <= 4 || (items - whole) * 16 > s.units || items == whole);
-        const float four = kCostFour[s.d()][s.v()].of(s.bh() * ((s.Nq + 127) / 128), s.tiles(), 2 * s.units);
+        // Four waves: past a round of row tiles, but for the few that a second launch takes better (16 in 256).  Plain calls at 64
+        // channels with fp16 P.V and 20 key tiles or more take it only where its own last round gives at most one workgroup to
+        // a unit: that round is the shorter one then, 0.75 to 0.95 of the main kernel's time in 33 calls of 2 to 4 rounds; past it
+        // 1.00 to 1.08 in 40 ([1,2602,40,64] 100.4 us against 96.1).  Not so with a range or causal ([2,1921,30,64] 62.9 against 74.1).
+        const int64_t items = s.items(), whole = items / s.units * s.units, wgs = s.bh() * ((s.Nq + 127) / 128);
+        const int64_t last = (wgs - 1) % (2 * s.units) + 1;
+        const bool over = items > s.units && (s.tiles() <= 4 || (items - whole) * 16 > s.units || items == whole) &&
+                          !(s.D == 64 && s.v() == 0 && !s.causal && s.masked == 0 && s.tiles() >= 20 && last > s.units);
+        const float four = kCostFour[s.d()][s.v()].of(wgs, s.tiles(), 2 * s.units);
         return over && four < best.t ? AttnPlan{items, 0, 0, false, true} : best.p;
     }
     return choose(s, by_length(s), q_cost(s), 0.0f, two_runs).p;

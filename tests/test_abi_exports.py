@@ -108,6 +108,9 @@ def test_form_of_the_attention_kernel_by_shape():
     for shape, masked in (((2, 4, 1439, 1439, 128, 0), 454), ((1, 30, 940, 940, 64, 0), 203)):
         assert attn_plan(*shape) == "two runs" and "short" in attn_plan(*shape, masked=masked), shape
     assert "short" in attn_plan(2, 12, 1303, 1303, 64, 0, causal=1) and "short" not in attn_plan(2, 12, 1303, 1303, 64, 0)
+    # four waves: where their own last round is the shorter one
+    assert attn_plan(1, 40, 2602, 2602, 64, 0) == attn_plan(2, 30, 1921, 1921, 64, 0) == "main"
+    assert attn_plan(2, 24, 1912, 1912, 64, 0) == attn_plan(2, 30, 1921, 1921, 64, 0, causal=1) == "four waves"
     assert _lib.lib().mi355_sage_attn_plan(1, 24, 64, 64, 96, 0, 0, 0, 0, (ctypes.c_int64 * 6)()) == -1
 
 
