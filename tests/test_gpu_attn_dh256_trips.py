@@ -45,3 +45,25 @@ def test_key_counts_around_the_trips(oracle, variant, tiles):
 @pytest.mark.parametrize("lo,hi", [(1, 70), (60, 500), (257, 259), (320, 704), (500, 1270), (1, 1279)])
 def test_masked_range_around_the_trips(oracle, variant, lo, hi):
     _check(oracle, variant, 1280, 1280, lo, hi, seed=lo)
+
+
+@pytest.mark.parametrize("variant", [0, 1])
+@pytest.mark.parametrize("Sq,Skv", [(130, 130), (700, 700), (300, 1025), (1025, 300)])
+def test_causal_end(oracle, variant, Sq, Skv):
+    """Against the checker given the mask as a bias.  (e4m3: a probability next to a rounding boundary may lie 2^-3 of itself off the
+    checker's, and in the first rows a key's probability is most of the row's: 2^-3 * 0.8 of |v - o| < 5, which leaves the cosine to
+    hold the rest.)"""
+    import gpu_harness as G
+    from mojodiffusion_amd.workloads import bf16_bits_to_f32
+    from test_gpu_attn_causal import _bias, _causal_call
+    rng = np.random.default_rng(Sq + Skv)
+    q, k, v = (f32_to_bf16_bits(rng.standard_normal((1, n, 2, D)).astype(np.float32)) for n in (Sq, Skv, Skv))
+    lib = _lib.lib()
+    assert lib.mi355_sage_set_attn_short(-1) == 0
+    try:
+        got, _ = _causal_call(q, k, v, float(D ** -0.5), variant, 128 if variant == 0 else 32)
+    finally:
+        lib.mi355_sage_set_attn_short(0)
+    _, want = oracle.sdpa_bf16(q, k, v, float(D ** -0.5), variant=variant, blkq=128 if variant == 0 else 32, blkk=64, addmask=_bias(1, 2, Sq, Skv))
+    cos, mx = G.cos_maxabs(bf16_bits_to_f32(got), want)
+    assert mx <= (2e-2 if variant == 0 else 0.5) and cos >= 0.9999, (cos, mx)

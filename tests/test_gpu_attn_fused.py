@@ -34,6 +34,8 @@ def test_bits_of_the_separate_launches(D, Skv, H, Sq, runs):
     k += 3.0 * torch.randn((1, 1, H, D), generator=g, device="cuda").to(torch.bfloat16)
     bias = torch.randn((1, H, Sq, Skv), generator=g, device="cuda").to(torch.bfloat16)
     scale = D ** -0.5
+    from test_abi_exports import attn_plan
+    assert attn_plan(1, H, Sq, Skv, D, 0) == attn_plan(1, H, Sq, Skv, D, 0, bias=1) == "one launch"
 
     def call():
         fwd = A.sdpa_flash_train_fwd_rect(q, k, v, scale)

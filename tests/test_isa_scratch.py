@@ -1,8 +1,7 @@
 """CPU-side check of the code generated for gfx950: no kernel keeps registers in scratch memory.
 
 A spill in a loop costs its traffic, and scratch accesses share the vector-memory counter by which the kernels wait for
-their tile copies.  Two instantiations are known to: the split schedule under an additive bias, and the one-launch quantize
-stage with a half-split rotation."""
+their tile copies.  One instantiation is known to: the split schedule under an additive bias."""
 import os
 import re
 import shutil
@@ -14,7 +13,7 @@ from mojodiffusion_amd import _lib
 
 READELF = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "llvm-readelf")
 OBJDUMP = os.path.join(os.path.dirname(READELF), "llvm-objdump")
-KNOWN = {"_ZN4sage16sage_attn_kernelILi128ELi0ELb0ELb1ELb1E": 20, "_ZN4sage18quant_short_kernelILi128ELi2EE": 12}       # prefix: bytes per lane
+KNOWN = {"_ZN4sage16sage_attn_kernelILi128ELi0ELb0ELb1ELb1E": 20}       # prefix: bytes per lane
 
 
 @pytest.mark.skipif(not (os.path.exists(READELF) and os.path.exists(OBJDUMP)), reason="no LLVM tools")
