@@ -15,7 +15,7 @@
 // wave's own copy counters; the loop has no barrier.  (Fragments loaded from L2 straight into registers —
 // no LDS at all — were built first: a fragment is 64 separate 16-byte pieces, an address cycle each, and
 // the first step alone took 6.4 us at [1,256,30,128].)  Per key tile a compute unit moves 8 times the main
-// kernel's operand bytes per query row, which is why attn_short_rule stops where the main kernel's
+// kernel's operand bytes per query row, which is why the choice of form (below) leaves it where the main kernel's
 // workgroups start to fill the chip.
 #include "sage_attn_common.h"
 #include "sage_grid.h"
@@ -734,7 +734,7 @@ hipError_t launch_attn_short(const AttnArgs& a, hipStream_t st) {
 // short form with 64 rows in four runs or 32 in eight.  What splits the keys is for grids that do not fill the chip: a
 // step takes a wave about as long with the chip half empty.  One-shot, us, without the two-run form -> with it: [1,1127,19,128] 39.0 ->
 // 32.5, [1,1091,16,128] 36.4 -> 29.2, e4m3 [2,615,16,128] 34.1 -> 31.1, [1,1127,19,64] 30.6 -> 25.7, with a bias
-// [1,1153,24,128] 55.0 -> 45.0.  Past about 128 row tiles its workgroups take a second round and the main kernel is ahead
+// [1,1153,24,128] 60.2 -> 48.9.  Past about 128 row tiles its workgroups take a second round and the main kernel is ahead
 // ([1,1322,30,128] 47 against 58); below 40 to 60 the short form is (eight runs: [1,256,30,128] 16.6 against 18.4).
 //
 // The same with workgroups of four waves, 128 rows and half of a compute unit's LDS: two share a unit, one's rows in and

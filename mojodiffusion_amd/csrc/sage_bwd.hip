@@ -304,7 +304,7 @@ __device__ __forceinline__ void bwd_pass_body(const BwdArgs& a, uint8_t* smem, i
     const int ntiles = xt * XROWS < valid_x ? (valid_y + 63) / 64 : 0;
 
     // per-lane pieces of the copy addresses: run i of this wave covers physical chunks
-    // (i*8 + wave)*64 + lane of a tile
+    // (i*NW + wave)*64 + lane of a tile
     int nat_row[RPW], nat_col[RPW];
 #pragma unroll
     for (int i = 0; i < RPW; i++) {
