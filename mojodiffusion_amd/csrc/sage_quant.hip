@@ -1077,10 +1077,16 @@ hipError_t launch_quant(const QuantArgs& a_in, const FinalArgs* f, int B, int D,
     // workgroup's way (as a branch of the one kernel half a microsecond of small calls too, so it is a kernel of its own), and
     // small tables come from the memory-side cache fast enough.  At 64 channels, workgroups of half the
     // work, that is 1.5 us at any size ([2,4352,24,64] 35.3 -> 36.5).
+    // In Q blocks of 32 rows (e4m3 P.V) a set of one batch is six workgroups, half of them short.  With half-split tables nothing is gained
+    // (the call, sets against none, 1.00 to 1.02 on average over 63 draws of either batch count, [1,1117,40,128] 73.1 -> 76.0); with
+    // interleaved ones and one batch it is level up to 32 MiB and 2 % ahead past it.
     const int64_t table_row = (int64_t)(D / 2) * (a.pre_q.tables_bf16 ? 4 : 8);
-    if (D == 128 && a.pre_q.cos != nullptr && (int64_t)a.Nq * a.H * table_row * (a.pre_q.batch_rows == 0 ? 1 : B) >= 16 << 20) {
+    const int batches = a.pre_q.batch_rows == 0 ? B : 1;
+    const bool small = a.q8 != nullptr && a.blkq < 128;
+    const int64_t from = batches == 1 && small ? 32 << 20 : 16 << 20;
+    if (D == 128 && a.pre_q.cos != nullptr && !(small && has_pre == 2) && (int64_t)a.Nq * a.H * table_row * (a.pre_q.batch_rows == 0 ? 1 : B) >= from) {
         // (a run is 128 rows: a block of 128, or several smaller ones)
-        a.batches = a.pre_q.batch_rows == 0 ? B : 1;
+        a.batches = batches;
         a.q_per = a.q8 != nullptr ? 128 / a.blkq : 0;
         a.k_per = a.k8 != nullptr ? 128 / a.blkk : 0;
         a.members = a.batches * (a.q_per + a.k_per);

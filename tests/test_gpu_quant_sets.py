@@ -1,4 +1,4 @@
-"""Encoders with rotation tables of 16 MiB and more deal their blocks in sets that read the same table rows: the same bits as
+"""Encoders with interleaved rotation tables of 16 MiB and more (32 for one batch in Q blocks below 128 rows) deal their blocks in sets that read the same table rows: the same bits as
 fewer heads at a time, whose tables are smaller and whose blocks go in the order of the heads."""
 import numpy as np
 import pytest
@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("B,S,blkq,blkk,per_batch,bf16", [(1, 1801, 128, 64, False, False), (2, 1801, 128, 64, False, False), (2, 897, 128, 64, True, False),
-                                                          (3, 1700, 32, 64, False, False), (1, 3500, 64, 128, False, True)])
+                                                          (3, 1700, 32, 64, False, False), (1, 6700, 64, 128, False, True)])
 def test_blocks_in_sets_give_the_same_bits(B, S, blkq, blkk, per_batch, bf16):
     D, Hh, part = 128, 20, 4
     rng = np.random.default_rng(S)
@@ -20,7 +20,7 @@ def test_blocks_in_sets_give_the_same_bits(B, S, blkq, blkk, per_batch, bf16):
     cos, sin = _tables(rng, batches * S * Hh, D)
     if bf16:
         cos, sin = f32_to_bf16_bits(cos), f32_to_bf16_bits(sin)
-    assert cos.nbytes + sin.nbytes >= 16 << 20
+    assert cos.nbytes + sin.nbytes >= (32 if B == 1 and blkq < 128 else 16) << 20
     run = lambda x, y, c, s, h: _gpu_quant(x, y, D ** -0.5, blkq, blkk, True, gq, gk, 1e-6, c, s, S * h if per_batch else 0)
     got = run(q, k, cos, sin, Hh)
     by_head = [t.reshape(batches, S, Hh, D // 2) for t in (cos, sin)]
