@@ -792,6 +792,19 @@ static const FormCost kCostCausal[2][FORMS] = {
     {{1.36f, 5.53f, 0.50f, 1.86f, 0.00f}, {4.58f, 2.83f, 0.07f, 0.84f, 0.16f}, {4.98f, 0.35f, 0.10f, 0.91f, 0.27f}, {2.72f, 0.97f, 0.00f, 1.15f, 0.24f}},
     {{7.41f, 2.10f, 0.62f, 5.27f, 0.00f}, {6.15f, 4.04f, 0.15f, 2.70f, 0.13f}, {5.09f, 4.20f, 0.10f, 0.77f, 0.51f}, {3.79f, 3.85f, 0.00f, 1.20f, 0.40f}},
 };
+// 256 channels with a masked range (160 one-shot calls in fp16, 147 in e4m3, of 33 to 2000 tokens and up to a round of row tiles) or
+// a bias (80 and 75, up to 4000 keys).  The main kernel takes the steps around a range, and all steps under a bias, in its general
+// bodies; by the figures of plain calls, below, it was taken where the short form is ahead: us, so -> by these, keymask [1,457,16,256]
+// with 7 keys masked 36.0 -> 30.7, e4m3 [3,61,4,256] with one 27.4 -> 24.3, e4m3 bias [1,78 x 38,24,256] 25.9 -> 23.6.  The choice costs
+// 0.1, 0.4, 0.0 and 0.0 % on average over the better form (the worst 24, the next 6 %), by the plain figures 6.9, 3.4, 10.2 and 2.3 %.
+static const FormCost kCost256Range[2][FORMS] = {
+    {{0.00f, 8.20f, 1.14f, 8.12f, 0.00f}, kNoForm, {0.00f, 7.09f, 0.85f, 0.00f, 0.74f}, kNoForm},
+    {{0.00f, 11.99f, 1.46f, 10.95f, 0.00f}, kNoForm, {0.00f, 7.40f, 1.87f, 0.33f, 0.00f}, kNoForm},
+};
+static const FormCost kCost256Bias[2][FORMS] = {
+    {{0.00f, 4.31f, 2.12f, 4.74f, 0.21f}, kNoForm, {0.00f, 4.17f, 1.72f, 0.77f, 0.22f}, kNoForm},
+    {{0.00f, 9.07f, 1.51f, 7.38f, 0.00f}, kNoForm, {0.00f, 6.44f, 1.86f, 0.25f, 0.54f}, kNoForm},
+};
 // All lengths, by launches and calls of up to 32 768 keys of earlier forms of the kernels (the two-run form against the
 // main kernel's figures here): longer key sequences, 256 channels, and what the split schedule is compared with.
 static const FormCost kCostLong[3][2][FORMS] = {        // [64, 128, 256 channels]
@@ -883,6 +896,11 @@ static AttnPlan plan_by_shape(const Problem& s, int split) {
         Problem counted = s;
         counted.kv -= s.masked;
         return choose(counted, (s.causal ? kCostCausal : kCostRange)[s.d()], 0.0f, 0.0f, two_runs).p;
+    }
+    if (s.D == 256 && !s.causal && (s.bias || s.masked > 0) && s.items() <= s.units && s.tiles() <= 64) {
+        Problem counted = s;
+        counted.kv -= s.masked;
+        return choose(counted, (s.bias ? kCost256Bias : kCost256Range)[s.v()], 0.0f, 0.0f, false).p;
     }
     if (s.D <= 128 && !s.bias && s.tiles() <= 48) {
         const Choice best = choose(s, kCost[s.d()][s.v()], 0.0f, launch, two_runs);
