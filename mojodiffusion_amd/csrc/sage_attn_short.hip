@@ -805,6 +805,13 @@ static const FormCost kCost256Bias[2][FORMS] = {
     {{0.00f, 4.31f, 2.12f, 4.74f, 0.21f}, kNoForm, {0.00f, 4.17f, 1.72f, 0.77f, 0.22f}, kNoForm},
     {{0.00f, 9.07f, 1.51f, 7.38f, 0.00f}, kNoForm, {0.00f, 6.44f, 1.86f, 0.25f, 0.54f}, kNoForm},
 };
+// e4m3 at 256 channels, plain (with and without Stats) and causal: 134 and 165 such calls.  Below 64 tokens they had gone to the main kernel by its
+// figures alone, refitted for longer calls: [1,40,30,256] 25.0 us, 23.6 so.  The choice costs 0.1 and 0.5 % over the better form, by
+// those figures 0.8 and 1.7 %.
+static const FormCost kCost256E4m3[2][FORMS] = {       // [plain, causal]
+    {{0.00f, 8.33f, 0.99f, 3.53f, 0.07f}, kNoForm, {0.00f, 6.10f, 1.58f, 0.57f, 0.00f}, kNoForm},
+    {{0.00f, 9.09f, 0.33f, 21.58f, 0.23f}, kNoForm, {0.00f, 6.93f, 0.54f, 4.78f, 0.00f}, kNoForm},
+};
 // All lengths, by launches and calls of up to 32 768 keys of earlier forms of the kernels (the two-run form against the
 // main kernel's figures here): longer key sequences, 256 channels, and what the split schedule is compared with.
 static const FormCost kCostLong[3][2][FORMS] = {        // [64, 128, 256 channels]
@@ -897,10 +904,11 @@ static AttnPlan plan_by_shape(const Problem& s, int split) {
         counted.kv -= s.masked;
         return choose(counted, (s.causal ? kCostCausal : kCostRange)[s.d()], 0.0f, 0.0f, two_runs).p;
     }
-    if (s.D == 256 && !s.causal && (s.bias || s.masked > 0) && s.items() <= s.units && s.tiles() <= 64) {
+    if (s.D == 256 && s.items() <= s.units && s.tiles() <= 64) {
         Problem counted = s;
         counted.kv -= s.masked;
-        return choose(counted, (s.bias ? kCost256Bias : kCost256Range)[s.v()], 0.0f, 0.0f, false).p;
+        const FormCost* c = s.bias ? kCost256Bias[s.v()] : s.masked > 0 ? kCost256Range[s.v()] : s.v() == 1 ? kCost256E4m3[s.causal] : nullptr;
+        if (c != nullptr) return choose(counted, c, 0.0f, 0.0f, false).p;
     }
     if (s.D <= 128 && !s.bias && s.tiles() <= 48) {
         const Choice best = choose(s, kCost[s.d()][s.v()], 0.0f, launch, two_runs);

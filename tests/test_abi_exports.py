@@ -103,7 +103,9 @@ def test_form_of_the_attention_kernel_by_shape():
     assert attn_plan(1, 18, 1153, 1153, 256, 0) == "main" and attn_plan(2, 32, 71, 45, 256, 1) == "short4"
     # ... the latter for small calls with a masked range or a bias, which the main kernel takes in its general bodies
     assert attn_plan(1, 16, 457, 457, 256, 0, masked=7) == attn_plan(3, 4, 61, 61, 256, 1, masked=1) == attn_plan(1, 24, 78, 38, 256, 1, bias=1) == "short4"
-    assert attn_plan(1, 16, 457, 457, 256, 0) == attn_plan(1, 24, 78, 38, 256, 1) == attn_plan(1, 18, 1153, 1153, 256, 0, bias=1) == "main"
+    assert attn_plan(1, 16, 457, 457, 256, 0) == attn_plan(1, 18, 1153, 1153, 256, 0, bias=1) == "main"
+    # ... and for e4m3 calls of few tokens, causal or not
+    assert attn_plan(1, 30, 40, 40, 256, 1) == attn_plan(2, 2, 52, 17, 256, 1, causal=1) == "short4" and attn_plan(1, 18, 1153, 1153, 256, 1) == "main"
     # causal calls are one launch of the attention kernel
     assert "+" not in attn_plan(1, 24, 4608, 4608, 128, 0, causal=1)
     # two runs: not of two key tiles, and behind the short form under a masked range or causal
