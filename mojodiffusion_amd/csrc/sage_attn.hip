@@ -1304,8 +1304,8 @@ size_t attn_split_bytes(int workgroups, int D) {
 hipError_t launch_attn(const AttnArgs& a, hipStream_t st) {
     if (a.nkv_pad > max_keys(a.D)) return hipErrorInvalidValue;      // K scales would not fit the LDS staging
     auto main = [&](bool two_runs) -> hipError_t {
-        // (256 channels first: in front of the code object its kernels stand where they do whatever the others' sizes are;
-        // moved by those, the same instructions took 29.0 instead of 28.6 us at [1,1153,18,256])
+        // (256 channels first: in front of the code object its kernels stand where they do whatever the others' sizes are.
+        // The same instructions at four places of the code object took 28.6 to 29.0 us at [1,1153,18,256], 28.8 here.)
         if (a.D == 256) return a.variant == 0 ? launch_attn_dv<256, 0>(a, two_runs, st) : launch_attn_dv<256, 1>(a, two_runs, st);
         if (a.D == 128) return a.variant == 0 ? launch_attn_dv<128, 0>(a, two_runs, st) : launch_attn_dv<128, 1>(a, two_runs, st);
         if (a.D == 64) return a.variant == 0 ? launch_attn_dv<64, 0>(a, two_runs, st) : launch_attn_dv<64, 1>(a, two_runs, st);
