@@ -858,11 +858,13 @@ struct Problem {
     int d() const { return D == 64 ? 0 : D == 128 ? 1 : 2; }
 };
 
-Choice choose(const Problem& s, const FormCost* c, float q_main, float launch, bool two_runs) {
+// alone: whether the forms without the main kernel may do everything
+Choice choose(const Problem& s, const FormCost* c, float q_main, float launch, bool two_runs, bool alone = true) {
     const int64_t items = s.items(), whole = items / s.units * s.units;
     // (past a round of row tiles the two-run form does what the main kernel's whole rounds leave: that is ahead of
     // it doing everything, or level)
-    Choice best = best_small(c, s.Nq, s.bh(), s.D, s.variant, s.kv, s.units, two_runs && (s.causal || whole == 0 || whole == items));
+    Choice best = alone ? best_small(c, s.Nq, s.bh(), s.D, s.variant, s.kv, s.units, two_runs && (s.causal || whole == 0 || whole == items))
+                        : Choice{1e30f, AttnPlan{items, 0, 0}};
     const float main = c[MAIN].of(items, s.tiles(), s.units) + q_main;
     if (main <= best.t) best = Choice{main, AttnPlan{items, 0, 0}};
     if (!s.causal && whole > 0 && whole < items) {
@@ -898,7 +900,10 @@ static AttnPlan plan_by_shape(const Problem& s, int split) {
     const float launch = s.d() == 0 && s.v() == 0 ? 0.0f : 3.0f;
     // (two key tiles or fewer leave a run nothing to gain, e4m3 [1,926 x 89,30,128] 21.2 us by the main kernel, 23.0 so)
     const bool two_runs = s.D <= 128 && s.tiles() > 2 && pad_to(s.kv, kPadKV) <= kTwoRunKeys && !(s.bias && s.v() == 1);
-    if (s.D <= 128 && s.bias && s.v() == 0) return choose(s, kCostBias[s.d()], 0.0f, 3.0f, two_runs).p;
+    // (under a bias at 128 channels the short form alone is not ahead past a round: 1.07 to 2 times the main kernel's time in 53 such
+    // calls.  A last row tile of a head that is hardly filled takes the main kernel less than the figures say: us, by the short
+    // form -> so, [3,316 x 244,64,128] 53.7 -> 48.7, [3,855 x 52,64,128] 71.5 -> 48.3)
+    if (s.D <= 128 && s.bias && s.v() == 0) return choose(s, kCostBias[s.d()], 0.0f, 3.0f, two_runs, s.D == 64 || s.items() <= s.units).p;
     if (s.D <= 128 && !s.bias && s.v() == 0 && s.items() <= s.units && (s.causal || s.masked > 0) && s.tiles() > 2 && s.tiles() <= 40) {
         Problem counted = s;
         counted.kv -= s.masked;

@@ -108,6 +108,8 @@ def test_form_of_the_attention_kernel_by_shape():
     assert attn_plan(1, 30, 40, 40, 256, 1) == attn_plan(2, 2, 52, 17, 256, 1, causal=1) == "short4" and attn_plan(1, 18, 1153, 1153, 256, 1) == "main"
     # causal calls are one launch of the attention kernel
     assert "+" not in attn_plan(1, 24, 4608, 4608, 128, 0, causal=1)
+    # under a bias at 128 channels the short form does no more than what is left of the main kernel's rounds
+    assert all("main" in attn_plan(3, 64, Sq, Skv, 128, 0, bias=1) for Sq, Skv in ((316, 244), (286, 188), (268, 193)))
     # two runs: not of two key tiles, and behind the short form under a masked range or causal
     assert attn_plan(1, 30, 926, 89, 128, 1) == attn_plan(2, 24, 570, 44, 128, 0) == "main"
     for shape, masked in (((2, 4, 1439, 1439, 128, 0), 454), ((1, 30, 940, 940, 64, 0), 203)):
