@@ -69,6 +69,8 @@ SIGNATURES = {
     "mi355_sage_attn_main_items": (_i64, [_int] * 6),
     "mi355_sage_attn_main_items_on": (_i64, [_int] * 7),
     "mi355_sage_set_attn_split_wait": (_int, [_int]),
+    "mi355_sage_quant_once": (_int, [_vp] * 3 + [_int] * 5 + [ctypes.c_float, _i64p, _i64p, _i64p] + [_int] * 4
+                              + [_vp, _vp, ctypes.c_float, _vp, _vp, _int] + [_vp] * 10 + [ctypes.c_size_t, _int, _vp]),
     "mi355_sage_version": (ctypes.c_char_p, []),
 }
 

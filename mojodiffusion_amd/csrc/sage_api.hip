@@ -4,7 +4,10 @@
 #include "../../include/mi355_sage_test.h"
 #include "sage_internal.h"
 
+#include <atomic>
+#include <chrono>
 #include <cstdio>
+#include <cstdlib>
 #include <mutex>
 #include <vector>
 
@@ -233,7 +236,28 @@ struct QuantOut {
     double* kpart_sum; float* kpart_mm;
     float* rowdot;
     float *rowinv_q, *rowinv_k;       // whole-row RMSNorm statistics (only with that pre-op)
+    uint64_t* flags;                  // room for the hand-over of the one-launch stage, null: the launches
+    size_t flag_bytes;
+    int once_polls;                   // tests: that form, with so many looks at a flag (< 0: and no flag raised); 0: by the rule
 };
+
+// A number for the flags of one call: no two calls of a process share one (a bijection of the counter), and memory that other
+// work has filled does not hold it but for a chance of 2^-64 a word.
+uint64_t call_tag() {
+    static std::atomic<uint64_t> n{(uint64_t)std::chrono::steady_clock::now().time_since_epoch().count() << 20};
+    uint64_t z = n.fetch_add(1, std::memory_order_relaxed) * 0x9E3779B97F4A7C15ull;
+    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+    return z ^ (z >> 31);
+}
+
+// Looks (of about a microsecond) at another workgroup's flag before a workgroup computes what it waits for itself.
+constexpr int kOncePolls = 1024;
+
+bool capturing(hipStream_t st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
+}
 
 // K statistics + Q / K encoders (+ the V passes when vq is given): launches 1-3, or one launch.
 int quantize(const View& q, const View& k, const View* v, int B, int H, int Nq, int Nkv, int D, float scale,
@@ -265,8 +289,19 @@ int quantize(const View& q, const View& k, const View* v, int B, int H, int Nq, 
     if (v_fp8) { a.v = *v; a.v8 = static_cast<uint8_t*>(vq); }
     else if (v != nullptr) { a.v = *v; a.v16 = static_cast<uint16_t*>(vq); }
     a.pre_q = pre.q; a.pre_k = pre.k;
-    if (v != nullptr && quant_short_workgroups(a, B, D) > 0) {
+    const bool forced = o.once_polls != 0;
+    if (!forced && v != nullptr && quant_short_workgroups(a, B, D) > 0) {
         SAGE_HIP(launch_quant_short(a, f, B, D, st));
+        return 0;
+    }
+    if (forced || (v != nullptr && o.flags != nullptr && quant_once_rule(a, f, B) &&
+                   (size_t)quant_once_flag_words(B, H, Nkv, v_fp8) * sizeof(uint64_t) <= o.flag_bytes && !capturing(st))) {
+        OnceArgs w{};
+        w.q = a; w.f = f;
+        w.flags = o.flags; w.tag = call_tag();
+        w.polls = forced ? abs(o.once_polls) : kOncePolls;
+        w.raise = o.once_polls >= 0;
+        SAGE_HIP(launch_quant_once(w, B, D, st));
         return 0;
     }
 
@@ -434,6 +469,8 @@ int sdpa_impl(const void* Q, const void* K, const void* V, void* O, void* Stats,
     o.kpart_mm = reinterpret_cast<float*>(ws + c.kpart_mm);
     o.rowinv_q = reinterpret_cast<float*>(ws + c.rowinv_q);
     o.rowinv_k = reinterpret_cast<float*>(ws + c.rowinv_k);
+    // (the flags lie where the whole-row statistics would)
+    if (!pre.full_row) { o.flags = reinterpret_cast<uint64_t*>(ws + c.rowinv_q); o.flag_bytes = c.split - c.rowinv_q; }
     // Stats needs <q, kmean> per row: K smoothing lowers every score of a row by it
     float* qshift = (Stats && (k_flags & MI355_SAGE_K_SMOOTH)) ? reinterpret_cast<float*>(ws + c.qshift) : nullptr;
     o.rowdot = qshift;
@@ -721,12 +758,12 @@ int mi355_sage_sdpa_bf16_norm_rope_train_fwd(const void* Q, const void* K, const
                      default_blkq(variant), 64, kDefaultFlags, workspace, workspace_bytes, pre);
 }
 
-int mi355_sage_quant_qkv_bf16(const void* Q, const void* K, const void* V, int B, int H, int N_q, int N_kv, int D,
+static int quant_qkv_entry(const void* Q, const void* K, const void* V, int B, int H, int N_q, int N_kv, int D,
                               float scale, const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides,
                               int64_t q_off, int64_t k_off, int64_t v_off,
                               int variant, int blkq, int blkk, int k_flags, int mask_lo, int mask_hi,
                               void* q8, void* qscale, void* k8, void* kscale, void* kmean, void* qmul, void* kmul,
-                              void* vq, void* vscale, void* scratch, size_t scratch_bytes, void* stream) {
+                              void* vq, void* vscale, void* scratch, size_t scratch_bytes, void* stream, const Pre& pre, int once_polls) {
     if (!Q || !K || !V || !k8 || !kscale || !kmean || !qmul || !kmul || !vq || !scratch) return MI355_SAGE_EINVAL;
     if ((q8 == nullptr) != (qscale == nullptr)) return MI355_SAGE_EINVAL;      // both NULL: Q is left to mi355_sage_attn_fwd_q16
     if (B <= 0 || H <= 0 || N_q <= 0 || N_kv <= 0 || D <= 0) return MI355_SAGE_EINVAL;
@@ -752,10 +789,40 @@ int mi355_sage_quant_qkv_bf16(const void* Q, const void* K, const void* V, int B
     o.kpart_mm = reinterpret_cast<float*>(scr + sc.kpart_mm);
     o.rowinv_q = reinterpret_cast<float*>(scr + sc.rowinv_q);
     o.rowinv_k = reinterpret_cast<float*>(scr + sc.rowinv_k);
+    if (once_polls != 0) {
+        const bool v_fp8 = variant != MI355_SAGE_PV_FP16;
+        if (D > 128 || blkk != 64 || !(k_flags & 3) || pre.full_row || (pre.q.cos != nullptr && N_q != N_kv)) return MI355_SAGE_EUNSUPPORTED;
+        o.flags = reinterpret_cast<uint64_t*>(scr + sc.total);
+        if (scratch_bytes < sc.total + (size_t)quant_once_flag_words(B, H, N_kv, v_fp8) * sizeof(uint64_t)) return MI355_SAGE_EWORKSPACE;
+        o.once_polls = once_polls;
+    }
     const View v = make_view(V, v_strides, v_off);
     return quantize(make_view(Q, q_strides, q_off), make_view(K, k_strides, k_off), &v, B, H, N_q, N_kv, D, scale,
                     blkq, blkk, k_flags, km, kept, o, variant, vq, static_cast<float*>(vscale),
-                    reinterpret_cast<float*>(scr + sc.vpart), Pre{}, static_cast<hipStream_t>(stream));
+                    reinterpret_cast<float*>(scr + sc.vpart), pre, static_cast<hipStream_t>(stream));
+}
+
+int mi355_sage_quant_qkv_bf16(const void* Q, const void* K, const void* V, int B, int H, int N_q, int N_kv, int D,
+                              float scale, const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides,
+                              int64_t q_off, int64_t k_off, int64_t v_off,
+                              int variant, int blkq, int blkk, int k_flags, int mask_lo, int mask_hi,
+                              void* q8, void* qscale, void* k8, void* kscale, void* kmean, void* qmul, void* kmul,
+                              void* vq, void* vscale, void* scratch, size_t scratch_bytes, void* stream) {
+    return quant_qkv_entry(Q, K, V, B, H, N_q, N_kv, D, scale, q_strides, k_strides, v_strides, q_off, k_off, v_off, variant, blkq, blkk, k_flags,
+                           mask_lo, mask_hi, q8, qscale, k8, kscale, kmean, qmul, kmul, vq, vscale, scratch, scratch_bytes, stream, Pre{}, 0);
+}
+
+int mi355_sage_quant_once(const void* Q, const void* K, const void* V, int B, int H, int N_q, int N_kv, int D, float scale,
+                          const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides, int variant, int blkq,
+                          int mask_lo, int mask_hi, const void* q_gain, const void* k_gain, float eps, const void* rope_cos,
+                          const void* rope_sin, int rope_layout, void* q8, void* qscale, void* k8, void* kscale, void* kmean, void* qmul,
+                          void* kmul, void* vq, void* vscale, void* scratch, size_t scratch_bytes, int polls, void* stream) {
+    if (polls == 0) return MI355_SAGE_EINVAL;
+    Pre pre;
+    int rc;
+    if ((rc = make_pre(q_gain, k_gain, eps, rope_cos, rope_sin, 0, rope_layout, &pre))) return rc;
+    return quant_qkv_entry(Q, K, V, B, H, N_q, N_kv, D, scale, q_strides, k_strides, v_strides, 0, 0, 0, variant, blkq, 64, kDefaultFlags,
+                           mask_lo, mask_hi, q8, qscale, k8, kscale, kmean, qmul, kmul, vq, vscale, scratch, scratch_bytes, stream, pre, polls);
 }
 
 int mi355_sage_quant_v_f16(const void* V, int B, int H, int N_kv, int D, const int64_t* v_strides,

@@ -112,6 +112,22 @@ int64_t quant_short_workgroups(const QuantArgs& a, int B, int D);     // 0: not 
 int64_t quant_short_workgroups(int B, int H, int Nq, int Nkv, int D, int blkq, int blkk, bool with_q);      // the same by the shape
 hipError_t launch_quant_short(const QuantArgs& a, const FinalArgs& f, int B, int D, hipStream_t st);
 
+// All of it as one launch whose workgroups hand their statistics to each other (K blocks of 64 keys, K statistics wanted, no
+// whole-row norm, not under capture).
+struct OnceArgs {
+    QuantArgs q;
+    FinalArgs f;                     // all K outputs, and V's with e4m3
+    uint64_t* flags;                 // quant_once_flag_words of them, whatever they hold
+    uint64_t tag;                    // a number no other call uses
+    int polls;                       // looks at a flag before a workgroup computes what it waits for itself
+    int raise;                       // 0: no flag is raised (tests)
+    int nk, nv, nkb, heads, flag_words;      // filled by the launcher
+    int k_apart, v_in;               // likewise: K's blocks are encoded by workgroups of their own / V (fp16) goes with K's groups
+};
+int64_t quant_once_flag_words(int B, int H, int Nkv, bool v_fp8);
+bool quant_once_rule(const QuantArgs& a, const FinalArgs& f, int B);
+hipError_t launch_quant_once(const OnceArgs& a, int B, int D, hipStream_t st);
+
 // ---- attention kernel (sage_attn.hip) --------------------------------------
 // rint(x / sc) for |x / sc| <= ~127 without paying a full IEEE divide per element: x * (1/sc)
 // is within 2^-15 of the correctly rounded quotient (both below 128), so whenever it lies at

@@ -1,5 +1,6 @@
-// sage_quant.hip — HBM-bound kernels of the quantized-SDPA path (gfx950), three launches (one for short
-// key sequences, quant_short_kernel; two for the next longer ones, quant_adds_up):
+// sage_quant.hip — HBM-bound kernels of the quantized-SDPA path (gfx950), one launch for short key sequences
+// (quant_short_kernel) and, in one-shot calls, for those of up to 8192 keys (quant_once_kernel); three otherwise, two for up to ten groups of
+// 256 keys (quant_adds_up):
 //
 //   prep_kernel         per (b,h), workgroup roles:  V repack to tiled fp16  |  V channel
 //                       maxima per 256-token group (e4m3 variant)  |  K channel sums (fp64),
@@ -13,6 +14,7 @@
 // round-half-to-even) and every reduction either has a fixed order (the fp64 sums) or is
 // order-free (max / min), so codes, scales and statistics are reproducible bit for bit.
 // All kernels read bf16 rows with 16-byte loads (8 channels per lane).
+#include "sage_attn_common.h"
 #include "sage_grid.h"
 #include "sage_quant_common.h"
 
@@ -241,7 +243,7 @@ __device__ __forceinline__ void quant_i8_block(
     float v[NCH][8];
     float amax = 0.0f;
     float inv[NCH], gain[8];
-    constexpr int AHEAD = 2;                   // (four take the kernel from three waves per SIMD to two)
+    constexpr int AHEAD = HAVE && PRE == 2 ? 1 : 2;      // (four take the kernel from three waves per SIMD to two)
     RopeTab<PRE> tab[AHEAD];
     auto clamped = [&](int i) { return min(r0 + (i * NT + tid) / CPR, N - 1); };
     RopeAt rope{};
@@ -538,6 +540,29 @@ __device__ __forceinline__ int v_tile_chunk(int slot, int chunk) {
     return D == 256 ? (chunk ^ (((slot >> 3) & 7) << 2)) : D == 128 ? (chunk ^ (((slot >> 3) & 7) << 1)) : (chunk ^ ((slot >> 3) & 7));
 }
 
+// A tile in LDS -> memory, channel-major.
+template <int D, int NT>
+__device__ __forceinline__ void store_v_f16_tile(int tid, const uint16_t* tile, uint16_t* dst) {
+    // work item = (channel pair, 8 consecutive slots): eight dword reads, two 16-byte stores
+    const uint32_t* tile32 = reinterpret_cast<const uint32_t*>(tile);
+#pragma unroll
+    for (int i = 0; i < (D / 2) * 8 / NT; i++) {
+        const int c = i * NT + tid;
+        const int dp = c >> 3, s0 = (c & 7) * 8;            // channels 2*dp, 2*dp+1
+        uint32_t w[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++)
+            w[e] = tile32[(s0 + e) * (D / 2) + v_tile_chunk<D>(s0 + e, dp >> 2) * 4 + (dp & 3)];
+        u32x4 lo, hi;
+        lo.x = __builtin_amdgcn_perm(w[1], w[0], 0x05040100u); hi.x = __builtin_amdgcn_perm(w[1], w[0], 0x07060302u);
+        lo.y = __builtin_amdgcn_perm(w[3], w[2], 0x05040100u); hi.y = __builtin_amdgcn_perm(w[3], w[2], 0x07060302u);
+        lo.z = __builtin_amdgcn_perm(w[5], w[4], 0x05040100u); hi.z = __builtin_amdgcn_perm(w[5], w[4], 0x07060302u);
+        lo.w = __builtin_amdgcn_perm(w[7], w[6], 0x05040100u); hi.w = __builtin_amdgcn_perm(w[7], w[6], 0x07060302u);
+        *reinterpret_cast<u32x4*>(dst + (2 * dp) * 64 + s0) = lo;
+        *reinterpret_cast<u32x4*>(dst + (2 * dp + 1) * 64 + s0) = hi;
+    }
+}
+
 template <int D, int NT = 256>
 __device__ __forceinline__ void quant_v_f16_body(
     int t, int h, int b, int tid, const uint16_t* __restrict__ v, int64_t sb, int64_t sh, int64_t sn,
@@ -568,25 +593,7 @@ __device__ __forceinline__ void quant_v_f16_body(
         *reinterpret_cast<u32x4*>(&tile[slot * D + v_tile_chunk<D>(slot, chunk) * 8]) = o;
     }
     __syncthreads();
-    uint16_t* dst = out + ((((int64_t)b * H + h) * (n_pad / 64)) + t) * (int64_t)(D * 64);
-    // work item = (channel pair, 8 consecutive slots): eight dword reads, two 16-byte stores
-    const uint32_t* tile32 = reinterpret_cast<const uint32_t*>(tile);
-#pragma unroll
-    for (int i = 0; i < (D / 2) * 8 / NT; i++) {
-        const int c = i * NT + tid;
-        const int dp = c >> 3, s0 = (c & 7) * 8;            // channels 2*dp, 2*dp+1
-        uint32_t w[8];
-#pragma unroll
-        for (int e = 0; e < 8; e++)
-            w[e] = tile32[(s0 + e) * (D / 2) + v_tile_chunk<D>(s0 + e, dp >> 2) * 4 + (dp & 3)];
-        u32x4 lo, hi;
-        lo.x = __builtin_amdgcn_perm(w[1], w[0], 0x05040100u); hi.x = __builtin_amdgcn_perm(w[1], w[0], 0x07060302u);
-        lo.y = __builtin_amdgcn_perm(w[3], w[2], 0x05040100u); hi.y = __builtin_amdgcn_perm(w[3], w[2], 0x07060302u);
-        lo.z = __builtin_amdgcn_perm(w[5], w[4], 0x05040100u); hi.z = __builtin_amdgcn_perm(w[5], w[4], 0x07060302u);
-        lo.w = __builtin_amdgcn_perm(w[7], w[6], 0x05040100u); hi.w = __builtin_amdgcn_perm(w[7], w[6], 0x07060302u);
-        *reinterpret_cast<u32x4*>(dst + (2 * dp) * 64 + s0) = lo;
-        *reinterpret_cast<u32x4*>(dst + (2 * dp + 1) * 64 + s0) = hi;
-    }
+    store_v_f16_tile<D, NT>(tid, tile, out + ((((int64_t)b * H + h) * (n_pad / 64)) + t) * (int64_t)(D * 64));
 }
 
 // ---------------------------------------------------------------------------
@@ -634,45 +641,31 @@ __device__ __forceinline__ void v_absmax_group_body(
 // and reaches 448 exactly where the quotient's magnitude is 448 (1 + 2^-23) at most, which the
 // scale guarantees.  A wave that sees a non-finite input, or a scale outside the range where none
 // of this can underflow, or with an all-ones significand, takes the plain formula.
-template <int D, int NT>
-__device__ __forceinline__ void quant_v_fp8_body(
-    int t, int h, int b, int tid, const uint16_t* __restrict__ v, int64_t sb, int64_t sh, int64_t sn,
-    int N, int H, int64_t n_pad, const KeyMask& km, const float* __restrict__ vscale,
-    uint8_t* __restrict__ out, uint8_t* tile) {
-    constexpr int CPR = D / 8;
-    constexpr int LD = D + 16;                             // padded row (bytes)
-    constexpr int NCH = 64 * CPR / NT;
-    static_assert(NT % CPR == 0, "a thread keeps one column group for all its chunks");
-    const int64_t bh = (int64_t)b * H + h;
-    const uint16_t* src = v + b * sb + h * sh;
-    const int col = (tid % CPR) * 8;
-    u32x4 w[NCH];
-#pragma unroll
-    for (int i = 0; i < NCH; i++) {
-        const int row = t * 64 + (i * NT + tid) / CPR;
-        w[i] = u32x4{0u, 0u, 0u, 0u};
-        if (key_kept(row, N, km)) w[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)row * sn + col);
-    }
+struct VScale8 {
     float sc[8], y[8];
-    load8(vscale + col, sc);
-    bool plain = false;
+    bool odd;                                              // a scale that the short way does not take
+    __device__ __forceinline__ explicit VScale8(const float* vscale) {
+        load8(vscale, sc);
+        odd = false;
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
-        y[e] = 1.0f / sc[e];
-        plain = plain || !(sc[e] >= 0x1p-60f && sc[e] <= 0x1p60f) || (__float_as_uint(sc[e]) & 0x7FFFFFu) == 0x7FFFFFu;
+        for (int e = 0; e < 8; e++) {
+            y[e] = 1.0f / sc[e];
+            odd = odd || !(sc[e] >= 0x1p-60f && sc[e] <= 0x1p60f) || (__float_as_uint(sc[e]) & 0x7FFFFFu) == 0x7FFFFFu;
+        }
     }
-    uint32_t mag = 0u;
+    // whether some lane of the wave needs the plain formula for these chunks
+    template <int N> __device__ __forceinline__ bool plain_for(const u32x4 (&w)[N]) const {
+        uint32_t mag = 0u;
 #pragma unroll
-    for (int i = 0; i < NCH; i++)
+        for (int i = 0; i < N; i++)
 #pragma unroll
-        for (int e = 0; e < 4; e++) mag = bf16_mag_max(mag, w[i][e]);
-    plain = __any(plain || !bf16_mag_finite(mag));
-#pragma unroll
-    for (int i = 0; i < NCH; i++) {
-        const int key = (i * NT + tid) / CPR;
+            for (int e = 0; e < 4; e++) mag = bf16_mag_max(mag, w[i][e]);
+        return __any(odd || !bf16_mag_finite(mag));
+    }
+    __device__ __forceinline__ void codes(const u32x4& w, bool plain, uint32_t (&pk)[2]) const {
         float x[8];
-        unpack8(w[i], x);
-        uint32_t pk[2] = {0u, 0u};
+        unpack8(w, x);
+        pk[0] = pk[1] = 0u;
         if (__builtin_expect(plain, 0)) {
 #pragma unroll
             for (int e = 0; e < 8; e++) pk[e >> 2] |= f32_to_e4m3(x[e] / sc[e]) << ((e & 3) * 8);
@@ -692,11 +685,12 @@ __device__ __forceinline__ void quant_v_fp8_body(
                 pk[j] = (uint32_t)p2;
             }
         }
-        *reinterpret_cast<u32x2*>(&tile[v_slot_fp8(key) * LD + col]) = u32x2{pk[0], pk[1]};
     }
-    __syncthreads();
-    uint8_t* dst = out + ((bh * (n_pad / 64)) + t) * (int64_t)(D * 64);
-    // output chunk = (channel d, 16 consecutive slots)
+};
+// Codes of a tile in LDS (row = slot, LD bytes) -> the tile in memory: 16 consecutive slots of a channel at a time.
+template <int D, int NT>
+__device__ __forceinline__ void store_v_fp8_tile(int tid, const uint8_t* tile, uint8_t* dst) {
+    constexpr int LD = D + 16;
 #pragma unroll
     for (int i = 0; i < D * 4 / NT; i++) {
         const int c = i * NT + tid;
@@ -706,6 +700,39 @@ __device__ __forceinline__ void quant_v_fp8_body(
         for (int e = 0; e < 16; e++) pk[e >> 2] |= (uint32_t)tile[(s0 + e) * LD + d] << ((e & 3) * 8);
         *reinterpret_cast<u32x4*>(dst + d * 64 + s0) = u32x4{pk[0], pk[1], pk[2], pk[3]};
     }
+}
+
+template <int D, int NT>
+__device__ __forceinline__ void quant_v_fp8_body(
+    int t, int h, int b, int tid, const uint16_t* __restrict__ v, int64_t sb, int64_t sh, int64_t sn,
+    int N, int H, int64_t n_pad, const KeyMask& km, const float* __restrict__ vscale,
+    uint8_t* __restrict__ out, uint8_t* tile) {
+    constexpr int CPR = D / 8;
+    constexpr int LD = D + 16;                             // padded row (bytes)
+    constexpr int NCH = 64 * CPR / NT;
+    static_assert(NT % CPR == 0, "a thread keeps one column group for all its chunks");
+    const int64_t bh = (int64_t)b * H + h;
+    const uint16_t* src = v + b * sb + h * sh;
+    const int col = (tid % CPR) * 8;
+    u32x4 w[NCH];
+#pragma unroll
+    for (int i = 0; i < NCH; i++) {
+        const int row = t * 64 + (i * NT + tid) / CPR;
+        w[i] = u32x4{0u, 0u, 0u, 0u};
+        if (key_kept(row, N, km)) w[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)row * sn + col);
+    }
+    const VScale8 vs(vscale + col);
+    const bool plain = vs.plain_for(w);
+#pragma unroll
+    for (int i = 0; i < NCH; i++) {
+        const int key = (i * NT + tid) / CPR;
+        uint32_t pk[2];
+        vs.codes(w[i], plain, pk);
+        *reinterpret_cast<u32x2*>(&tile[v_slot_fp8(key) * LD + col]) = u32x2{pk[0], pk[1]};
+    }
+    __syncthreads();
+    uint8_t* dst = out + ((bh * (n_pad / 64)) + t) * (int64_t)(D * 64);
+    store_v_fp8_tile<D, NT>(tid, tile, dst);
 }
 
 // ---------------------------------------------------------------------------
@@ -1316,6 +1343,566 @@ hipError_t launch_quant_short(const QuantArgs& a_in, const FinalArgs& f_in, int 
     else if (D == 64) hipLaunchKernelGGL(quant_short_kernel<64>, grid, block, 0, st, a, f_in);
     else if (D == 256) hipLaunchKernelGGL(quant_short_kernel<256>, grid, block, 0, st, a, f_in);
     else return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// The whole stage as one launch with the statistics handed over between workgroups.  A workgroup takes a group of 256 keys,
+// keeps its rows in registers, publishes the group's sums, minima and maxima, waits for those of the head's other groups and
+// encodes: K (and, for e4m3, V) is read once instead of twice, and two launches' starts and ends go.
+//
+// The hand-over.  Results and flags are written and read by relaxed atomics of agent scope only: these go past the L2s of the
+// XCDs, which are not coherent with each other inside a kernel, and need none of the write-backs and invalidations that a
+// fence of that scope is.  A flag is raised when the wave's stores are complete (vmcnt) behind a barrier of the workgroup.
+// Flags hold a number that no other call of the process uses, so memory may hold anything before; a call under capture, whose
+// replays would all use one number, takes the launches.
+// The wait is bounded.  A workgroup that sees a flag missing after `polls` computes all groups of its head itself, the same values
+// into the same places: nothing depends on which workgroups are resident together, only the time does.  To have them
+// resident, heads come in chunks (OnceArgs::heads), their K groups first: a group waits for workgroups in front of it and a few
+// behind it.
+// Every workgroup adds up the group results of its head itself, in group order.
+// What a K workgroup's time goes to at [1,1153,24,128] (one per compute unit), us: rows 1.6, sums and handing over 3, waiting 1.7, adding up 0.9,
+// encoding 3.4 (vector work), next to 3 of the launch's start and end; bandwidth comes first from about 400 groups on.  (Statistics
+// published once per head by the last group's workgroup: 6 us instead of 1.8 of waiting and adding up at 18 groups.  At 256 channels a
+// workgroup has a compute unit to itself: [2,2688,32,256] 503 -> 790 us; not built.)
+// ---------------------------------------------------------------------------
+
+template <typename T> __device__ __forceinline__ T agent_load(const T* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+template <typename T> __device__ __forceinline__ void agent_store(T* p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// (stores of this wave have reached the place agent-scope loads read)
+__device__ __forceinline__ void stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+template <int D> struct OnceShape {
+    static constexpr int CH = 4, CPR = D / CH, NT = 16 * CPR;       // channels per thread, threads per leaf and group
+    static constexpr int WPB = 4 * CPR / 64;                                      // waves per scale block of 64 keys
+    static constexpr int LD = D + D / 8;
+    static constexpr int VT = D == 128 ? 2 : 1;                                   // fp16 V tiles per workgroup
+    static constexpr int CPR8 = D / 8, RP = NT / CPR8;                            // rows per pass in chunks of eight channels
+};
+template <int D, int PRE> union OnceSmem {
+    using S = OnceShape<D>;
+    struct { double sum[16][S::LD]; float mn[16][S::LD], mx[16][S::LD]; } leaf;
+    u32x4 rows[PRE ? kGroup * S::CPR8 : 1];
+    float vred[S::RP][S::LD];
+    uint8_t tile8[4][64 * (D + 16)];
+    uint16_t tile16[4][64 * D];
+    float red[16];
+};
+template <int D> struct OnceHead { float mean[D], kmul[D], qmul[D]; };             // mean: also V's scales
+
+// flags[0 .. n) hold tag, within `polls` looks.  One wave calls it.
+__device__ __forceinline__ bool flags_up(const uint64_t* flags, int n, uint64_t tag, int polls, int lane) {
+    for (int p = 0; p < polls; p++) {
+        bool up = true;
+        for (int i = lane; i < n; i += 64) up = up && agent_load(flags + i) == tag;
+        if (__all(up)) return true;
+        __builtin_amdgcn_s_sleep(2);
+    }
+    return false;
+}
+
+// One group of keys in registers: a leaf of CH channels per thread.
+template <int D, int PRE>
+struct OnceGroup {
+    using S = OnceShape<D>;
+    static constexpr int CH = S::CH, W = CH / 2;
+    uint32_t w[kLeaf][W];
+    bool all_kept;                                  // every token of the wave's leaves counts
+    __device__ static __forceinline__ int leaf(int tid) { return tid / S::CPR; }
+    __device__ static __forceinline__ int col(int tid) { return tid % S::CPR * CH; }
+
+    // (what was computed from the rows is computed again behind this, not kept in registers)
+    __device__ __forceinline__ void pin() {
+#pragma unroll
+        for (int i = 0; i < kLeaf; i++)
+#pragma unroll
+            for (int e = 0; e < W; e++) asm volatile("" : "+v"(w[i][e]));
+    }
+
+    // Rows of group g; what does not count is zero.  (With the pre-ops: meets two barriers.)
+    __device__ __forceinline__ void load(const QuantArgs& a, int g, int h, int b, int tid, OnceSmem<D, PRE>& sm) {
+        asm volatile("" : "+v"(tid));               // (row addresses are formed where they are used, not held from one call to the next)
+        const int s0 = g * kGroup + leaf(tid) * kLeaf, N = a.Nkv;
+        all_kept = __all(s0 + kLeaf <= N && !(s0 < a.km.hi && s0 + kLeaf > a.km.lo));
+        if constexpr (PRE) {
+            constexpr int CPR8 = S::CPR8, NR = 2, AHEAD = PRE == 2 ? 1 : 2;
+            const int c8 = tid % CPR8 * 8;
+            const uint16_t* src = a.k.p + b * a.k.sb + h * a.k.sh + c8;
+            const RopeAt rope = rope_at<D>(a.pre_k, b, h, a.H, c8);
+            float gain[8];
+            pre_gains(a.pre_k, h, D, c8, gain);
+#pragma unroll 1
+            for (int r0 = 0; r0 < kGroup; r0 += NR * S::RP) {          // (registers for four rows at a time)
+                const int first = g * kGroup + r0 + tid / CPR8;
+                auto clamped = [&](int i) { return min(first + i * S::RP, N - 1); };
+                u32x4 raw[NR];
+                RopeTab<PRE> tab[AHEAD];
+#pragma unroll
+                for (int i = 0; i < NR; i++) raw[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)clamped(i) * a.k.sn);
+#pragma unroll
+                for (int i = 0; i < AHEAD; i++) rope_load<PRE>(rope, clamped(i), tab[i]);
+                float inv[NR];
+                row_inverses<D, NR>(a.pre_k.eps, raw, inv);
+#pragma unroll
+                for (int i = 0; i < NR; i++) {
+                    float x[8];
+                    unpack8(raw[i], x);
+                    pre_apply<D, PRE>(a.pre_k, c8, key_kept(first + i * S::RP, N, a.km), inv[i], gain, tab[i % AHEAD], x);
+                    if (i + AHEAD < NR) rope_load<PRE>(rope, clamped(i + AHEAD), tab[i % AHEAD]);
+                    u32x4 y;                                           // (bf16 values: nothing below their upper halves)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) y[e] = __builtin_amdgcn_perm(__float_as_uint(x[2 * e + 1]), __float_as_uint(x[2 * e]), 0x07060302u);
+                    sm.rows[(r0 + i * S::RP) * CPR8 + tid] = y;
+                }
+            }
+            __syncthreads();
+            const uint32_t* r32 = reinterpret_cast<const uint32_t*>(sm.rows);
+#pragma unroll
+            for (int i = 0; i < kLeaf; i++) {
+                const u32x2 v = *reinterpret_cast<const u32x2*>(r32 + ((leaf(tid) * kLeaf + i) * D + col(tid)) / 2);
+                w[i][0] = v.x; w[i][1] = v.y;
+            }
+            __syncthreads();                                       // (the leaves' results go where the rows are)
+        } else {
+            const uint16_t* src = a.k.p + b * a.k.sb + h * a.k.sh + col(tid);
+#pragma unroll
+            for (int i = 0; i < kLeaf; i++) {
+                const uint16_t* p = src + (int64_t)min(s0 + i, N - 1) * a.k.sn;
+                if constexpr (CH == 8) {
+                    const u32x4 v = *reinterpret_cast<const u32x4*>(p);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) w[i][e] = v[e];
+                } else {
+                    const u32x2 v = *reinterpret_cast<const u32x2*>(p);
+                    w[i][0] = v.x; w[i][1] = v.y;
+                }
+            }
+            if (!all_kept) {
+#pragma unroll
+                for (int i = 0; i < kLeaf; i++)
+                    if (!key_kept(s0 + i, N, a.km)) {
+#pragma unroll
+                        for (int e = 0; e < W; e++) w[i][e] = 0u;
+                    }
+            }
+        }
+    }
+
+    // The group's sums, minima and maxima to memory: the tree of kstats_group.  (Meets two barriers; stores complete behind them.)
+    __device__ __forceinline__ void publish(const QuantArgs& a, const FinalArgs& f, int64_t bh, int g, int tid, OnceSmem<D, PRE>& sm) const {
+        asm volatile("" : "+v"(tid));
+        const int s0 = g * kGroup + leaf(tid) * kLeaf, c = col(tid);
+        double acc[CH];
+        float mn[CH], mx[CH];
+#pragma unroll
+        for (int e = 0; e < CH; e++) { acc[e] = 0.0; mn[e] = INFINITY; mx[e] = -INFINITY; }
+#pragma unroll
+        for (int i = 0; i < kLeaf; i += 2) {
+            __builtin_amdgcn_sched_barrier(0);                     // (or all sixteen tokens are converted first)
+            float x[2][CH];
+#pragma unroll
+            for (int r = 0; r < 2; r++)
+#pragma unroll
+                for (int e = 0; e < W; e++) { x[r][2 * e] = bf16_lo(w[i + r][e]); x[r][2 * e + 1] = bf16_hi(w[i + r][e]); }
+            // (tokens that do not count are +0.0, which leaves a double sum unchanged)
+#pragma unroll
+            for (int r = 0; r < 2; r++)
+#pragma unroll
+                for (int e = 0; e < CH; e++) acc[e] += (double)x[r][e];
+            if (!all_kept) {
+                // (a NaN takes no part in a minimum or maximum)
+#pragma unroll
+                for (int r = 0; r < 2; r++)
+                    if (!key_kept(s0 + i + r, a.Nkv, a.km))
+#pragma unroll
+                        for (int e = 0; e < CH; e++) x[r][e] = __builtin_nanf("");
+            }
+            // (as instructions: see kstats_group)
+#pragma unroll
+            for (int e = 0; e < CH; e++) {
+                asm("v_min3_f32 %0, %0, %1, %2" : "+v"(mn[e]) : "v"(x[0][e]), "v"(x[1][e]));
+                asm("v_max3_f32 %0, %0, %1, %2" : "+v"(mx[e]) : "v"(x[0][e]), "v"(x[1][e]));
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < CH; e++) {
+            const int at = ((c + e) & 7) * S::CPR8 + (c >> 3);      // (as in KGroupSmem)
+            sm.leaf.sum[leaf(tid)][at] = acc[e];
+            sm.leaf.mn[leaf(tid)][at] = mn[e];
+            sm.leaf.mx[leaf(tid)][at] = mx[e];
+        }
+        __syncthreads();
+        if (tid < D) {
+            double sum = 0.0;
+#pragma unroll
+            for (int u = 0; u < 16; u++) sum += sm.leaf.sum[u][tid];
+            agent_store(const_cast<double*>(f.kpart_sum) + (bh * f.ngroups + g) * D + leaf_channel<D>(tid), sum);
+        } else if (tid < 2 * D) {
+            const int t = tid - D;
+            float lo = INFINITY, hi = -INFINITY;
+#pragma unroll
+            for (int u = 0; u < 16; u++) {
+                lo = fminf(lo, sm.leaf.mn[u][t]);
+                hi = fmaxf(hi, sm.leaf.mx[u][t]);
+            }
+            agent_store(reinterpret_cast<uint64_t*>(const_cast<float*>(f.kpart_mm)) + (bh * f.ngroups + g) * D + leaf_channel<D>(t),
+                        (uint64_t)__float_as_uint(lo) | (uint64_t)__float_as_uint(hi) << 32);
+        }
+        stores_done();
+        __syncthreads();
+    }
+
+    // Codes and scales of the group's blocks of 64 keys.  (Meets a barrier.)
+    __device__ __forceinline__ void encode(const QuantArgs& a, int64_t bh, int g, int tid, OnceSmem<D, PRE>& sm, const OnceHead<D>& hd) {
+        asm volatile("" : "+v"(tid));
+        const int s0 = g * kGroup + leaf(tid) * kLeaf, c = col(tid), wave = tid >> 6;
+        float mu[CH], mul[CH];
+#pragma unroll
+        for (int e = 0; e < CH; e++) { mu[e] = hd.mean[c + e]; mul[e] = hd.kmul[c + e]; }
+        pin();
+        auto value = [&](int i, int e) -> float {
+            const float x = e & 1 ? bf16_hi(w[i][e >> 1]) : bf16_lo(w[i][e >> 1]);
+            const float d = x - mu[e];
+            return d * mul[e];
+        };
+        float am = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kLeaf; i++)
+            if (all_kept || key_kept(s0 + i, a.Nkv, a.km)) {
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int e = 0; e < CH; e += 2) am = fmaxf(fmaxf(am, fabsf(value(i, e))), fabsf(value(i, e + 1)));
+            }
+        pin();
+        am = wave_max(am);
+        if constexpr (S::WPB == 2) {
+            if ((tid & 63) == 0) sm.red[wave] = am;
+            __syncthreads();
+            am = fmaxf(am, sm.red[wave ^ 1]);
+        }
+        const float sc = am > 0.0f ? am / 127.0f : 1.0f;
+        const bool there = s0 < a.nkv_pad;                          // (whole leaves)
+        if (there && (tid & (64 * S::WPB - 1)) == 0) a.kscale[bh * (a.nkv_pad / 64) + (s0 >> 6)] = sc;
+        const bool fast = sc >= 0x1p-100f && sc <= 0x1p100f;
+        const float rinv = 1.0f / sc;
+        int8_t* out = a.k8 + (bh * a.nkv_pad + s0) * D + c;
+        constexpr int TOK = 8 / CH;                                 // tokens per call of the encoder
+#pragma unroll
+        for (int i = 0; i < kLeaf; i += TOK) {
+            __builtin_amdgcn_sched_barrier(0);
+            float x[8];
+#pragma unroll
+            for (int r = 0; r < TOK; r++) {
+                const bool kept = all_kept || key_kept(s0 + i + r, a.Nkv, a.km);
+#pragma unroll
+                for (int e = 0; e < CH; e++) {
+                    x[r * CH + e] = value(i + r, e);
+                    if (!kept) x[r * CH + e] = 0.0f;
+                }
+            }
+            const u32x2 o = encode8_i8(x, sc, rinv, fast);
+            if (there) {
+                if constexpr (CH == 8) {
+                    *reinterpret_cast<u32x2*>(out + i * D) = o;
+                } else {
+                    *reinterpret_cast<uint32_t*>(out + i * D) = o.x;
+                    *reinterpret_cast<uint32_t*>(out + (i + 1) * D) = o.y;
+                }
+            }
+        }
+    }
+};
+
+// The head's K statistics into hd, for a workgroup of NT threads; `leave`: and into memory, for later launches.
+// Returns false where it computed the groups itself: what the caller held in registers is then to be loaded again.
+template <int D, int PRE>
+__device__ __forceinline__ bool once_k_head(const OnceArgs& a, int64_t bh, int h, int b, int tid, bool leave, OnceSmem<D, PRE>& sm, OnceHead<D>& hd, int& s_ok) {
+    const FinalArgs& f = a.f;
+    if (tid < 64) {
+        const bool up = flags_up(a.flags + bh * a.flag_words, f.ngroups, a.tag, a.polls, tid);
+        if (tid == 0) s_ok = up;
+    }
+    __syncthreads();
+    const bool ok = s_ok != 0;
+    if (__builtin_expect(!ok, 0)) {
+        for (int g = 0; g < f.ngroups; g++) {
+            OnceGroup<D, PRE> grp;
+            grp.load(a.q, g, h, b, tid, sm);
+            grp.publish(a.q, f, bh, g, tid, sm);
+        }
+    }
+    if (tid < D) {
+        constexpr int NB = 12;
+        const double* p = f.kpart_sum + bh * f.ngroups * D + tid;
+        const uint64_t* mm = reinterpret_cast<const uint64_t*>(f.kpart_mm) + bh * f.ngroups * D + tid;
+        double sum = 0.0;
+        float mn = INFINITY, mx = -INFINITY, mean, s;
+        for (int g0 = 0; g0 < f.ngroups; g0 += NB) {
+            double v[NB];
+            uint64_t lh[NB];
+#pragma unroll
+            for (int j = 0; j < NB; j++) {
+                const int g = min(g0 + j, f.ngroups - 1);
+                v[j] = agent_load(p + g * D);
+                lh[j] = agent_load(mm + g * D);
+            }
+#pragma unroll
+            for (int j = 0; j < NB; j++)
+                if (g0 + j < f.ngroups) {
+                    sum += v[j];
+                    mn = fminf(mn, __uint_as_float((uint32_t)lh[j]));
+                    mx = fmaxf(mx, __uint_as_float((uint32_t)(lh[j] >> 32)));
+                }
+        }
+        k_final(sum, mn, mx, f.kept, f.flags, mean, s);
+        const float kmul = 1.0f / s, qmul = f.cmul * s;
+        if (leave) {
+            const int64_t i = bh * D + tid;
+            f.kmean[i] = mean; f.kmul[i] = kmul; f.qmul[i] = qmul;
+        }
+        hd.mean[tid] = mean; hd.kmul[tid] = kmul; hd.qmul[tid] = qmul;
+    }
+    __syncthreads();
+    return ok;
+}
+
+// A group of 256 values of V: channel maxima, then e4m3 tiles.  The same hand-over.
+template <int D> struct OnceV {
+    using S = OnceShape<D>;
+    static constexpr int NCH = kGroup / S::RP;
+    u32x4 w[NCH];
+    __device__ __forceinline__ void pin() {
+#pragma unroll
+        for (int i = 0; i < NCH; i++) asm volatile("" : "+v"(w[i]));
+    }
+    __device__ __forceinline__ void load(const QuantArgs& a, int g, int h, int b, int tid) {
+        asm volatile("" : "+v"(tid));               // (as in OnceGroup)
+        const uint16_t* src = a.v.p + b * a.v.sb + h * a.v.sh + tid % S::CPR8 * 8;
+#pragma unroll
+        for (int i = 0; i < NCH; i++) {
+            const int row = g * kGroup + i * S::RP + tid / S::CPR8;
+            w[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)min(row, a.Nkv - 1) * a.v.sn);
+        }
+        if (g * kGroup + kGroup > a.Nkv || a.km.hi > a.km.lo) {
+#pragma unroll
+            for (int i = 0; i < NCH; i++)
+                if (!key_kept(g * kGroup + i * S::RP + tid / S::CPR8, a.Nkv, a.km)) w[i] = u32x4{0u, 0u, 0u, 0u};
+        }
+    }
+    __device__ __forceinline__ void publish(const FinalArgs& f, int64_t bh, int g, int tid, float (*red)[S::LD]) const {
+        float m[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < NCH; i++) {
+            float x[8];
+            unpack8(w[i], x);
+#pragma unroll
+            for (int e = 0; e < 8; e++) m[e] = fmaxf(m[e], fabsf(x[e]));
+        }
+#pragma unroll
+        for (int e = 0; e < 8; e++) red[tid / S::CPR8][e * S::CPR8 + tid % S::CPR8] = m[e];      // (as in KGroupSmem)
+        __syncthreads();
+        if (tid < D) {
+            float mm = 0.0f;
+#pragma unroll
+            for (int i = 0; i < S::RP; i++) mm = fmaxf(mm, red[i][tid]);
+            agent_store(const_cast<float*>(f.vpart) + (bh * f.ngroups + g) * D + leaf_channel<D>(tid), mm);
+        }
+        stores_done();
+        __syncthreads();
+    }
+};
+
+// The fp16 tiles of a group of 256 values of V whose rows are in registers.  (Meets a barrier.)
+template <int D>
+__device__ __forceinline__ void once_v_f16(const QuantArgs& a, int64_t bh, int g, int tid, const OnceV<D>& v, uint16_t (*tile)[64 * D]) {
+    using S = OnceShape<D>;
+#pragma unroll
+    for (int i = 0; i < OnceV<D>::NCH; i++) {
+        const int key = i * S::RP + tid / S::CPR8, slot = v_slot_f16(key & 63);
+        float x[8];
+        unpack8(v.w[i], x);
+        const u32x4 o = {f16_pair_sat(x[0], x[1]), f16_pair_sat(x[2], x[3]), f16_pair_sat(x[4], x[5]), f16_pair_sat(x[6], x[7])};
+        *reinterpret_cast<u32x4*>(&tile[key >> 6][slot * D + v_tile_chunk<D>(slot, tid % S::CPR8) * 8]) = o;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+        if ((g * 4 + j) * 64 < a.nkv_pad)
+            store_v_f16_tile<D, S::NT>(tid, tile[j], a.v16 + (bh * (a.nkv_pad / 64) + g * 4 + j) * (int64_t)(D * 64));
+}
+
+template <int D, int PRE>
+__global__ __launch_bounds__((OnceShape<D>::NT), 4) void quant_once_kernel(OnceArgs o) {
+    using S = OnceShape<D>;
+    constexpr int NT = S::NT;
+    __shared__ __attribute__((aligned(16))) OnceSmem<D, PRE> sm;
+    __shared__ __attribute__((aligned(16))) OnceHead<D> hd;
+    __shared__ int s_ok;
+    const QuantArgs& a = o.q;
+    const FinalArgs& f = o.f;
+    // heads in chunks; inside one, K groups, V, Q blocks, and consecutive workgroups take the same rows of consecutive heads
+    const int per = o.nk + o.nv + o.nkb + a.nq_blk, chunk = (int)blockIdx.x / (o.heads * per), in = (int)blockIdx.x - chunk * o.heads * per;
+    const int heads = min(o.heads, a.n_bh - chunk * o.heads);
+    const int unit = in / heads, bh = chunk * o.heads + in % heads;
+    const int b = bh / a.H, h = bh % a.H, tid = threadIdx.x;
+    uint64_t* flags = o.flags + (int64_t)bh * o.flag_words;
+    if (unit < o.nk) {
+        OnceGroup<D, PRE> grp;
+        grp.load(a, unit, h, b, tid, sm);
+        grp.publish(a, f, bh, unit, tid, sm);
+        if (tid == 0 && o.raise) agent_store(flags + unit, o.tag);
+        if (o.k_apart) return;
+        if (o.v_in) {
+            OnceV<D> v;
+            grp.pin();
+            v.load(a, unit, h, b, tid);
+            once_v_f16<D>(a, bh, unit, tid, v, sm.tile16);
+            __syncthreads();
+        }
+        if (!once_k_head<D, PRE>(o, bh, h, b, tid, unit == 0, sm, hd, s_ok)) grp.load(a, unit, h, b, tid, sm);
+        grp.encode(a, bh, unit, tid, sm, hd);
+    } else if (unit < o.nk + o.nv) {
+        const int t = unit - o.nk;
+        if (a.v16 != nullptr) {
+            constexpr int UT = NT / S::VT;
+            quant_v_f16_body<D, UT>(t * S::VT + tid / UT, h, b, tid % UT, a.v.p, a.v.sb, a.v.sh, a.v.sn, a.Nkv, a.H, a.nkv_pad, a.km, a.v16, sm.tile16[tid / UT]);
+            return;
+        }
+        flags += f.ngroups;
+        OnceV<D> v;
+        v.load(a, t, h, b, tid);
+        v.publish(f, bh, t, tid, sm.vred);
+        if (tid == 0 && o.raise) agent_store(flags + t, o.tag);
+        if (tid < 64) {
+            const bool up = flags_up(flags, f.ngroups, o.tag, o.polls, tid);
+            if (tid == 0) s_ok = up;
+        }
+        __syncthreads();
+        if (__builtin_expect(s_ok == 0, 0)) {
+            for (int g = 0; g < f.ngroups; g++) {
+                OnceV<D> x;
+                x.load(a, g, h, b, tid);
+                x.publish(f, bh, g, tid, sm.vred);
+            }
+            v.load(a, t, h, b, tid);
+        }
+        if (tid < D) {
+            constexpr int NB = 16;
+            const float* p = f.vpart + (int64_t)bh * f.ngroups * D + tid;
+            float amax = 0.0f;
+            for (int g0 = 0; g0 < f.ngroups; g0 += NB) {
+                float x[NB];
+#pragma unroll
+                for (int j = 0; j < NB; j++) x[j] = agent_load(p + min(g0 + j, f.ngroups - 1) * D);
+#pragma unroll
+                for (int j = 0; j < NB; j++) amax = fmaxf(amax, x[j]);
+            }
+            const float sc = amax > 0.0f ? amax / 448.0f : 1.0f;
+            if (t == 0) f.vscale[(int64_t)bh * D + tid] = sc;
+            hd.mean[tid] = sc;
+        }
+        __syncthreads();
+        const int col = tid % S::CPR8 * 8;
+        v.pin();
+        const VScale8 vs(&hd.mean[col]);
+        const bool plain = vs.plain_for(v.w);
+#pragma unroll
+        for (int i = 0; i < OnceV<D>::NCH; i++) {
+            const int key = i * S::RP + tid / S::CPR8;               // in the group
+            uint32_t pk[2];
+            vs.codes(v.w[i], plain, pk);
+            *reinterpret_cast<u32x2*>(&sm.tile8[key >> 6][v_slot_fp8(key & 63) * (D + 16) + col]) = u32x2{pk[0], pk[1]};
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int tile = t * 4 + j;
+            if (tile * 64 < a.nkv_pad) store_v_fp8_tile<D, NT>(tid, sm.tile8[j], a.v8 + ((int64_t)bh * (a.nkv_pad / 64) + tile) * (int64_t)(D * 64));
+        }
+    } else {
+        const int r = unit - o.nk - o.nv - o.nkb;
+        const KeyMask none{0, 0};
+        // (the block's rows are requested ahead of the wait)
+        if (unit < o.nk + o.nv + o.nkb) {
+            constexpr int NCH = 64 * S::CPR8 / NT;
+            const int blk = unit - o.nk - o.nv;
+            u32x4 rows[NCH];
+            auto load = [&] {
+                const uint16_t* src = a.k.p + b * a.k.sb + h * a.k.sh + tid % S::CPR8 * 8;
+#pragma unroll
+                for (int i = 0; i < NCH; i++) rows[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)min(blk * 64 + i * S::RP + tid / S::CPR8, a.Nkv - 1) * a.k.sn);
+            };
+            load();
+            if (!once_k_head<D, PRE>(o, bh, h, b, tid, blk == 0, sm, hd, s_ok)) load();
+            quant_i8_block<D, 64, true, PRE, NT, true>(blk, h, b, tid, a.k.p, a.k.sb, a.k.sh, a.k.sn, a.Nkv, a.H, a.nkv_pad, a.km, hd.mean, hd.kmul,
+                                                       0.0f, a.k8, a.kscale, nullptr, sm.red, a.pre_k, rows);
+            return;
+        }
+#define SAGE_Q(BLK)                                                                                                                                  do {                                                                                                                                                 constexpr int NCH = BLK * S::CPR8 / NT;                                                                                                          u32x4 rows[NCH];                                                                                                                                 auto load = [&] {                                                                                                                                    const uint16_t* src = a.q.p + b * a.q.sb + h * a.q.sh + tid % S::CPR8 * 8;                                                                       _Pragma("unroll") for (int i = 0; i < NCH; i++) {                                                                                                    const int row = r * BLK + i * S::RP + tid / S::CPR8;                                                                                             rows[i] = u32x4{0u, 0u, 0u, 0u};                                                                                                                 if (row < a.Nq) rows[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)row * a.q.sn);                                                      }                                                                                                                                            };                                                                                                                                               load();                                                                                                                                          if (!once_k_head<D, PRE>(o, bh, h, b, tid, false, sm, hd, s_ok)) load();                                                                            quant_i8_block<D, BLK, false, PRE, NT, true>(r, h, b, tid, a.q.p, a.q.sb, a.q.sh, a.q.sn, a.Nq, a.H, a.nq_pad, none, hd.mean, hd.qmul,                                                        a.cmul, a.q8, a.qscale, a.rowdot, sm.red, a.pre_q, rows);                                       } while (0)
+        if (a.blkq == 128) SAGE_Q(128);
+        else if (a.blkq == 64) SAGE_Q(64);
+        else SAGE_Q(32);
+#undef SAGE_Q
+    }
+}
+
+// Where the stage is one launch by hand-over.  Not where quant_short_kernel takes it (a workgroup there computes its head's
+// statistics in one pass and waits for nobody: [1,19 heads,512,128] 22.1 against 22.7 us), not past 32 groups to a head, which every workgroup
+// adds up.  Without the pre-ops all groups resident at once: [2,30,4416,128] (1080 groups) 492 -> 594 us with V in them, [2,40,2176,64]
+// (720) level.  Behind the pre-ops the second norm and rotation of K is what it saves, at any number.  The call, us, launches ->
+// hand-over: [1,4608,24,128] 232.5 -> 228.4, [1,24,364,128] train 57.7 -> 54.2, [1,12,2304,64] F32 125.2 -> 119.9, e4m3 [1,585,30,128] 33.0 ->
+// 31.0, [1,2915,30,64] 101.7 -> 95.1, [1,4544,24,128] 207.8 -> 204.3, norm + RoPE [1,2207,30,128] 126.9 -> 114.9, [2,4352,30,128] 529 -> 506; but
+// e4m3 [1,5184,30,128] with norm + RoPE (630 groups and as many of V) 355 -> 359, [1,5824,24,128] 320 -> 334.
+bool quant_once_rule(const QuantArgs& a, const FinalArgs& f, int B) {
+    const int64_t groups = (int64_t)f.ngroups * B * a.H;
+    return f.D <= 128 && f.ngroups <= 32 && a.blkk == 64 && (f.flags & 3) != 0 && a.pre_k.row_inv == nullptr &&
+           (a.pre_k.gain != nullptr && a.v8 == nullptr ? groups <= 4096 : groups <= 512);
+}
+
+int64_t quant_once_flag_words(int B, int H, int Nkv, bool v_fp8) {
+    const int64_t groups = (Nkv + kGroup - 1) / kGroup;
+    return (int64_t)B * H * groups * (v_fp8 ? 2 : 1);
+}
+
+hipError_t launch_quant_once(const OnceArgs& o_in, int B, int D, hipStream_t st) {
+    OnceArgs o = o_in;
+    QuantArgs& a = o.q;
+    const int pre = pre_kind(a.pre_k);
+    const bool v_fp8 = a.v8 != nullptr;
+    if (a.k8 == nullptr || (a.v8 == nullptr && a.v16 == nullptr) || a.blkk != 64 || a.pre_k.row_inv != nullptr || o.f.kpart_sum == nullptr ||
+        (a.q8 != nullptr && a.nq_pad % a.blkq != 0) || o.flags == nullptr || o.polls <= 0 || pre_kind(a.pre_q) != pre)
+        return hipErrorInvalidValue;
+    a.n_bh = B * a.H;
+    a.nq_blk = a.q8 != nullptr ? (int)(a.nq_pad / a.blkq) : 0;
+    o.nk = o.f.ngroups;
+    o.nv = v_fp8 ? o.f.ngroups : (int)(a.nkv_pad / 64) / (D == 128 ? 2 : 1);
+    o.flag_words = (int)(quant_once_flag_words(1, 1, a.Nkv, v_fp8));
+    // K's blocks by workgroups of their own, which start on them when the statistics are there, where the groups leave compute units
+    // without one (a group's encoding is 3.5 us of vector work in one workgroup, a block's 1); not behind the pre-ops, which they would do
+    // again, nor with e4m3, whose V groups are as long.  The call, us, with the groups -> apart: [1,1024,8,64] 19.0 -> 16.9,
+    // [2,24 heads,364,128] 55.2 -> 54.2, [2,24,1024,64] 36.4 -> 34.7; but 120 groups of 128 channels, [1,1153,24,128] bias, 49.8 -> 51.5.
+    const int64_t groups = (int64_t)o.nk * a.n_bh;
+    o.k_apart = !pre && !v_fp8 && groups * D <= 100 * 128;
+    o.nkb = o.k_apart ? (int)(a.nkv_pad / 64) : 0;
+    // fp16 V by K's workgroups, while the other groups' statistics are on their way, where they take more than one round of the
+    // compute units: [2,1248,30,128] 276.9 -> 270.4 (300 groups), norm + RoPE [2,4352,30,128] 516 -> 506 (1020); but
+    // [1,8,4224,128] (136) level, [2,24,1024,64] (192) 36.4 -> 39.1.
+    o.v_in = !o.k_apart && !v_fp8 && groups > compute_units();
+    if (o.v_in) o.nv = 0;
+    // (two workgroups to a compute unit are resident for certain)
+    o.heads = max(1, min(a.n_bh, 2 * compute_units() / (o.nk * (v_fp8 ? 2 : 1))));
+    const int64_t total = (int64_t)a.n_bh * (o.nk + o.nv + o.nkb + a.nq_blk);
+    if (total <= 0 || total > 0x7FFFFFFF) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)total);
+#define SAGE_ONCE(DD, PP) hipLaunchKernelGGL((quant_once_kernel<DD, PP>), grid, dim3(OnceShape<DD>::NT), 0, st, o)
+    if (D == 128 && pre == 2) SAGE_ONCE(128, 2);
+    else if (D == 128 && pre) SAGE_ONCE(128, 1);
+    else if (D == 128) SAGE_ONCE(128, 0);
+    else if (D == 64 && pre == 2) SAGE_ONCE(64, 2);
+    else if (D == 64 && pre) SAGE_ONCE(64, 1);
+    else if (D == 64) SAGE_ONCE(64, 0);
+    else return hipErrorInvalidValue;
+#undef SAGE_ONCE
     return hipGetLastError();
 }
 
