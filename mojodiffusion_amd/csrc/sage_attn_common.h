@@ -145,6 +145,52 @@ __device__ __forceinline__ u32x2 encode8_i8(const float (&x)[8], float sc, float
     return u32x2{wd[0], wd[1]};
 }
 
+// The same in two parts, for loops over several chunks: the common case, which says whether some lane of the wave comes close to a
+// tie, and the true quotient, in a loop over the chunks that did (redo_chunks).  Inside the unrolled loop the true quotient's eight divides
+// are two kilobytes of code to jump over per chunk.
+__device__ __forceinline__ u32x2 encode8_common(const float (&x)[8], float rinv, bool& near) {
+    float kRound = 12582912.0f, rv = rinv;
+    asm volatile("" : "+v"(rv), "+v"(kRound));
+    uint32_t tb[8], wd[2];
+    float dm = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+        const float t0 = fmaf(x[e], rv, kRound), t1 = fmaf(x[e + 1], rv, kRound);
+        const float d0 = fmaf(x[e], rv, -(t0 - kRound)), d1 = fmaf(x[e + 1], rv, -(t1 - kRound));
+        dm = fmaxf(fmaxf(dm, fabsf(d0)), fabsf(d1));
+        tb[e] = __float_as_uint(t0);
+        tb[e + 1] = __float_as_uint(t1);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const uint32_t lo = __builtin_amdgcn_perm(tb[4 * j + 1], tb[4 * j], 0x0c0c0400u);
+        const uint32_t hi = __builtin_amdgcn_perm(tb[4 * j + 3], tb[4 * j + 2], 0x0c0c0400u);
+        wd[j] = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+    }
+    near = __any(!(dm <= 0.5f - 0x1p-16f));
+    return u32x2{wd[0], wd[1]};
+}
+__device__ __forceinline__ u32x2 encode8_quotient(const float (&x)[8], float sc, float rinv, bool fast) {
+    uint32_t wd[2] = {0u, 0u};
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        float r = rint_quotient(x[e], sc, rinv, fast);
+        r = r > 127.0f ? 127.0f : r;
+        r = r < -127.0f ? -127.0f : r;
+        wd[e >> 2] |= ((uint32_t)((int)r) & 0xFFu) << ((e & 3) * 8);
+    }
+    return u32x2{wd[0], wd[1]};
+}
+// redo(i) for the set bits of a wave's mask.
+template <typename F> __device__ __forceinline__ void redo_chunks(uint32_t mask, F redo) {
+    mask = __builtin_amdgcn_readfirstlane(mask);
+#pragma unroll 1
+    while (__builtin_expect(mask != 0u, 0)) {
+        redo(__builtin_ctz(mask));
+        mask &= mask - 1u;
+    }
+}
+
 // ---- additive bias: 32 rows x 32 keys of a wave ------------------------------------------------------
 // Loaded 16 bytes per lane, whole rows next to each other (a lane's own four keys of its own row, the layout
 // the scores have, are 64 separate pieces per instruction: 4 to 8 of them per step took longer than the

@@ -1362,7 +1362,9 @@ hipError_t launch_quant_short(const QuantArgs& a_in, const FinalArgs& f_in, int 
 // behind it.
 // Every workgroup adds up the group results of its head itself, in group order.
 // What a K workgroup's time goes to at [1,1153,24,128] (one per compute unit), us: rows 1.6, sums and handing over 3, waiting 1.7, adding up 0.9,
-// encoding 3.4 (vector work), next to 3 of the launch's start and end; bandwidth comes first from about 400 groups on.  (Statistics
+// encoding 2.6, next to 3 of the launch's start and end; bandwidth comes first from about 400 groups on.  (Encoding was 3.4 with a pass over
+// the rows for the blocks' largest values, which a leaf's extremes say without one, and the true quotient inside the unrolled loop:
+// e4m3 [1,256 x 1971,24,64] 22.0 -> 21.3 us, [1,2432,12,128] 51.8 -> 50.6, bias [1,1153,24,128] 49.9 -> 49.5.)  (Statistics
 // published once per head by the last group's workgroup: 6 us instead of 1.8 of waiting and adding up at 18 groups.  At 256 channels a
 // workgroup has a compute unit to itself: [2,2688,32,256] 503 -> 790 us; not built.)
 // ---------------------------------------------------------------------------
@@ -1407,6 +1409,7 @@ struct OnceGroup {
     using S = OnceShape<D>;
     static constexpr int CH = S::CH, W = CH / 2;
     uint32_t w[kLeaf][W];
+    uint32_t ext[CH];                               // smallest and largest value of this thread's leaf per channel, as the bf16 they are (publish)
     bool all_kept;                                  // every token of the wave's leaves counts
     __device__ static __forceinline__ int leaf(int tid) { return tid / S::CPR; }
     __device__ static __forceinline__ int col(int tid) { return tid % S::CPR * CH; }
@@ -1489,7 +1492,7 @@ struct OnceGroup {
     }
 
     // The group's sums, minima and maxima to memory: the tree of kstats_group.  (Meets two barriers; stores complete behind them.)
-    __device__ __forceinline__ void publish(const QuantArgs& a, const FinalArgs& f, int64_t bh, int g, int tid, OnceSmem<D, PRE>& sm) const {
+    __device__ __forceinline__ void publish(const QuantArgs& a, const FinalArgs& f, int64_t bh, int g, int tid, OnceSmem<D, PRE>& sm) {
         asm volatile("" : "+v"(tid));
         const int s0 = g * kGroup + leaf(tid) * kLeaf, c = col(tid);
         double acc[CH];
@@ -1530,6 +1533,7 @@ struct OnceGroup {
             sm.leaf.sum[leaf(tid)][at] = acc[e];
             sm.leaf.mn[leaf(tid)][at] = mn[e];
             sm.leaf.mx[leaf(tid)][at] = mx[e];
+            ext[e] = __builtin_amdgcn_perm(__float_as_uint(mx[e]), __float_as_uint(mn[e]), 0x07060302u);
         }
         __syncthreads();
         if (tid < D) {
@@ -1559,20 +1563,29 @@ struct OnceGroup {
         float mu[CH], mul[CH];
 #pragma unroll
         for (int e = 0; e < CH; e++) { mu[e] = hd.mean[c + e]; mul[e] = hd.kmul[c + e]; }
-        pin();
-        auto value = [&](int i, int e) -> float {
-            const float x = e & 1 ? bf16_hi(w[i][e >> 1]) : bf16_lo(w[i][e >> 1]);
-            const float d = x - mu[e];
-            return d * mul[e];
-        };
         float am = 0.0f;
+        if constexpr (PRE) {
+            // (the extremes, kept that long, are one register too many here)
 #pragma unroll
-        for (int i = 0; i < kLeaf; i++)
-            if (all_kept || key_kept(s0 + i, a.Nkv, a.km)) {
-                __builtin_amdgcn_sched_barrier(0);
+            for (int i = 0; i < kLeaf; i++)
+                if (all_kept || key_kept(s0 + i, a.Nkv, a.km)) {
 #pragma unroll
-                for (int e = 0; e < CH; e += 2) am = fmaxf(fmaxf(am, fabsf(value(i, e))), fabsf(value(i, e + 1)));
+                    for (int e = 0; e < CH; e++) {
+                        const float d = (e & 1 ? bf16_hi(w[i][e >> 1]) : bf16_lo(w[i][e >> 1])) - mu[e];
+                        am = fmaxf(am, fabsf(d * mul[e]));
+                    }
+                }
+        } else {
+            // (rounding is monotone: a leaf's largest |(k - mean) mul| in a channel is that of its largest or its smallest k)
+#pragma unroll
+            for (int e = 0; e < CH; e++) {
+                const float mn = bf16_lo(ext[e]), mx = bf16_hi(ext[e]);
+                if (mn <= mx) {                                     // (not: a leaf without a key that counts, or NaNs alone)
+                    const float hi = mx - mu[e], lo = mn - mu[e];
+                    am = fmaxf(fmaxf(am, fabsf(hi * mul[e])), fabsf(lo * mul[e]));
+                }
             }
+        }
         pin();
         am = wave_max(am);
         if constexpr (S::WPB == 2) {
@@ -1586,30 +1599,52 @@ struct OnceGroup {
         const bool fast = sc >= 0x1p-100f && sc <= 0x1p100f;
         const float rinv = 1.0f / sc;
         int8_t* out = a.k8 + (bh * a.nkv_pad + s0) * D + c;
-        constexpr int TOK = 8 / CH;                                 // tokens per call of the encoder
+        // two tokens of four channels as one chunk of eight values
+        auto chunk = [&](int i, const uint32_t (&w0)[W], const uint32_t (&w1)[W], float (&x)[8]) {
 #pragma unroll
-        for (int i = 0; i < kLeaf; i += TOK) {
-            __builtin_amdgcn_sched_barrier(0);
-            float x[8];
-#pragma unroll
-            for (int r = 0; r < TOK; r++) {
+            for (int r = 0; r < 2; r++) {
                 const bool kept = all_kept || key_kept(s0 + i + r, a.Nkv, a.km);
 #pragma unroll
                 for (int e = 0; e < CH; e++) {
-                    x[r * CH + e] = value(i + r, e);
+                    const uint32_t u = r ? w1[e >> 1] : w0[e >> 1];
+                    const float d = (e & 1 ? bf16_hi(u) : bf16_lo(u)) - mu[e];
+                    x[r * CH + e] = d * mul[e];
                     if (!kept) x[r * CH + e] = 0.0f;
                 }
             }
-            const u32x2 o = encode8_i8(x, sc, rinv, fast);
-            if (there) {
-                if constexpr (CH == 8) {
-                    *reinterpret_cast<u32x2*>(out + i * D) = o;
-                } else {
-                    *reinterpret_cast<uint32_t*>(out + i * D) = o.x;
-                    *reinterpret_cast<uint32_t*>(out + (i + 1) * D) = o.y;
+        };
+        auto put = [&](int i, const u32x2& o) {
+            if (!there) return;
+            *reinterpret_cast<uint32_t*>(out + i * D) = o.x;
+            *reinterpret_cast<uint32_t*>(out + (i + 1) * D) = o.y;
+        };
+        uint32_t redo = fast ? 0u : (1u << (kLeaf / 2)) - 1u;
+#pragma unroll
+        for (int i = 0; i < kLeaf; i += 2) {
+            __builtin_amdgcn_sched_barrier(0);
+            float x[8];
+            bool near;
+            chunk(i, w[i], w[i + 1], x);
+            put(i, encode8_common(x, rinv, near));
+            redo |= near ? 1u << (i / 2) : 0u;
+        }
+        redo_chunks(redo, [&](int j) {
+            uint32_t w0[W], w1[W];
+#pragma unroll
+            for (int e = 0; e < W; e++) {
+                w0[e] = w[0][e];
+                w1[e] = w[1][e];
+#pragma unroll
+                for (int i = 2; i < kLeaf; i += 2) {
+                    w0[e] = j == i / 2 ? w[i][e] : w0[e];
+                    w1[e] = j == i / 2 ? w[i + 1][e] : w1[e];
+                    asm volatile("" : "+v"(w0[e]), "+v"(w1[e]));    // (or the rows go to memory, to be indexed there)
                 }
             }
-        }
+            float x[8];
+            chunk(j * 2, w0, w1, x);
+            put(j * 2, encode8_quotient(x, sc, rinv, fast));
+        });
     }
 };
 
@@ -1878,7 +1913,7 @@ hipError_t launch_quant_once(const OnceArgs& o_in, int B, int D, hipStream_t st)
     o.nv = v_fp8 ? o.f.ngroups : (int)(a.nkv_pad / 64) / (D == 128 ? 2 : 1);
     o.flag_words = (int)(quant_once_flag_words(1, 1, a.Nkv, v_fp8));
     // K's blocks by workgroups of their own, which start on them when the statistics are there, where the groups leave compute units
-    // without one (a group's encoding is 3.5 us of vector work in one workgroup, a block's 1); not behind the pre-ops, which they would do
+    // without one (a group's encoding is 2.6 us in one workgroup, a block's 1); not behind the pre-ops, which they would do
     // again, nor with e4m3, whose V groups are as long.  The call, us, with the groups -> apart: [1,1024,8,64] 19.0 -> 16.9,
     // [2,24 heads,364,128] 55.2 -> 54.2, [2,24,1024,64] 36.4 -> 34.7; but 120 groups of 128 channels, [1,1153,24,128] bias, 49.8 -> 51.5.
     const int64_t groups = (int64_t)o.nk * a.n_bh;
