@@ -289,12 +289,8 @@ int quantize(const View& q, const View& k, const View* v, int B, int H, int Nq, 
     if (v_fp8) { a.v = *v; a.v8 = static_cast<uint8_t*>(vq); }
     else if (v != nullptr) { a.v = *v; a.v16 = static_cast<uint16_t*>(vq); }
     a.pre_q = pre.q; a.pre_k = pre.k;
-    const bool forced = o.once_polls != 0;
-    if (!forced && v != nullptr && quant_short_workgroups(a, B, D) > 0) {
-        SAGE_HIP(launch_quant_short(a, f, B, D, st));
-        return 0;
-    }
-    if (forced || (v != nullptr && o.flags != nullptr && quant_once_rule(a, f, B) &&
+    const bool forced = o.once_polls != 0, short_form = v != nullptr && quant_short_workgroups(a, B, D) > 0;
+    if (forced || (v != nullptr && o.flags != nullptr && quant_once_rule(a, f, B, short_form) &&
                    (size_t)quant_once_flag_words(B, H, Nkv, v_fp8) * sizeof(uint64_t) <= o.flag_bytes && !capturing(st))) {
         OnceArgs w{};
         w.q = a; w.f = f;
@@ -302,6 +298,10 @@ int quantize(const View& q, const View& k, const View* v, int B, int H, int Nq, 
         w.polls = forced ? abs(o.once_polls) : kOncePolls;
         w.raise = o.once_polls >= 0;
         SAGE_HIP(launch_quant_once(w, B, D, st));
+        return 0;
+    }
+    if (!forced && short_form) {
+        SAGE_HIP(launch_quant_short(a, f, B, D, st));
         return 0;
     }
 

@@ -125,7 +125,7 @@ struct OnceArgs {
     int k_apart, v_in;               // likewise: K's blocks are encoded by workgroups of their own / V (fp16) goes with K's groups
 };
 int64_t quant_once_flag_words(int B, int H, int Nkv, bool v_fp8);
-bool quant_once_rule(const QuantArgs& a, const FinalArgs& f, int B);
+bool quant_once_rule(const QuantArgs& a, const FinalArgs& f, int B, bool short_form);     // short_form: quant_short_kernel takes the call
 hipError_t launch_quant_once(const OnceArgs& a, int B, int D, hipStream_t st);
 
 // ---- attention kernel (sage_attn.hip) --------------------------------------

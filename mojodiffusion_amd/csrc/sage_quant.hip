@@ -1881,15 +1881,18 @@ __global__ __launch_bounds__((OnceShape<D>::NT), 4) void quant_once_kernel(OnceA
     }
 }
 
-// Where the stage is one launch by hand-over.  Not where quant_short_kernel takes it (a workgroup there computes its head's
-// statistics in one pass and waits for nobody: [1,19 heads,512,128] 22.1 against 22.7 us), not past 32 groups to a head, which every workgroup
-// adds up.  Without the pre-ops all groups resident at once: [2,30,4416,128] (1080 groups) 492 -> 594 us with V in them, [2,40,2176,64]
+// Where the stage is one launch by hand-over.  Not past 32 groups to a head, which every workgroup adds up.  Of the calls that
+// quant_short_kernel takes (a workgroup there computes its head's statistics itself and waits for nobody), those with fp16 V of two and more groups,
+// three at 64 channels, up to 56 groups of 128 channels in all.  The call, us, short -> hand-over, K's blocks apart: [1,8 heads,600,64] 16.8 ->
+// 15.0, [1,1024,8,64] 16.6 -> 15.7, with Stats [1,8,1000,64] 18.8 -> 17.1, [1,333,8,128] 18.2 -> 17.3, bias [1,16,500,128] 20.8 -> 19.7; but
+// [1,512,30,128] (60 groups) 24.1 -> 24.4, [1,257,30,128] 20.7 -> 21.1, e4m3 [1,320,30,128] 19.8 -> 21.8.  Without the pre-ops all groups resident at once: [2,30,4416,128] (1080 groups) 492 -> 594 us with V in them, [2,40,2176,64]
 // (720) level.  Behind the pre-ops the second norm and rotation of K is what it saves, at any number.  The call, us, launches ->
 // hand-over: [1,4608,24,128] 232.5 -> 228.4, [1,24,364,128] train 57.7 -> 54.2, [1,12,2304,64] F32 125.2 -> 119.9, e4m3 [1,585,30,128] 33.0 ->
 // 31.0, [1,2915,30,64] 101.7 -> 95.1, [1,4544,24,128] 207.8 -> 204.3, norm + RoPE [1,2207,30,128] 126.9 -> 114.9, [2,4352,30,128] 529 -> 506; but
 // e4m3 [1,5184,30,128] with norm + RoPE (630 groups and as many of V) 355 -> 359, [1,5824,24,128] 320 -> 334.
-bool quant_once_rule(const QuantArgs& a, const FinalArgs& f, int B) {
+bool quant_once_rule(const QuantArgs& a, const FinalArgs& f, int B, bool short_form) {
     const int64_t groups = (int64_t)f.ngroups * B * a.H;
+    if (short_form && (a.v8 != nullptr || f.ngroups < (f.D == 64 ? 3 : 2) || groups * f.D > 56 * 128)) return false;
     return f.D <= 128 && f.ngroups <= 32 && a.blkk == 64 && (f.flags & 3) != 0 && a.pre_k.row_inv == nullptr &&
            (a.pre_k.gain != nullptr && a.v8 == nullptr ? groups <= 4096 : groups <= 512);
 }
