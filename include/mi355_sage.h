@@ -313,8 +313,9 @@ int mi355_sage_quant_qk_norm_rope_bf16(
     void* q8, void* qscale, void* k8, void* kscale, void* kmean, void* qmul, void* kmul,
     void* scratch, size_t scratch_bytes, void* stream);
 
-/* Q, K and V as the one-shot calls quantize them: three launches (V channel maxima ride with the K
- * statistics, V repack or e4m3 V encode with the Q / K encoders), one for short key sequences: same outputs, bit for bit, as
+/* Q, K and V together, in launches of which one-shot calls under capture, at 256 channels or of more than 8192 keys are made too: three
+ * (V channel maxima ride with the K statistics, V repack or e4m3 V encode with the Q / K encoders), two or one for shorter key
+ * sequences.  (The other one-shot calls hand statistics over inside one launch.)  Same outputs, bit for bit, as
  * mi355_sage_quant_qk_bf16 followed by mi355_sage_quant_v_f16 / _fp8, which take five.  vq is v16
  * or v8 by `variant`; vscale is written for MI355_SAGE_PV_FP8 only (may be NULL otherwise).
  * q8 == qscale == NULL: Q is not encoded here (mi355_sage_attn_fwd_q16 does it); qmul is still written.

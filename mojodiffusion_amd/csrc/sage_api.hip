@@ -256,7 +256,11 @@ constexpr int kOncePolls = 1024;
 
 bool capturing(hipStream_t st) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cs) != hipSuccess) {
+        (void)hipGetLastError();               // (or the launches that follow would report it as theirs)
+        return true;
+    }
+    return cs != hipStreamCaptureStatusNone;
 }
 
 // K statistics + Q / K encoders (+ the V passes when vq is given): launches 1-3, or one launch.

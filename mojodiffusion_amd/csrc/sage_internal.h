@@ -46,7 +46,7 @@ struct KeyMask {
     int lo, hi;
 };
 
-// ---- quantize kernels (sage_quant.hip): three launches --------------------------------
+// ---- quantize kernels (sage_quant.hip): up to three launches, or one --------------------------------
 // Launch 1: passes over V and K whose results the later launches need.
 struct PrepArgs {
     View k, v;

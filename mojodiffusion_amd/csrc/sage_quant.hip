@@ -1890,11 +1890,16 @@ __global__ __launch_bounds__((OnceShape<D>::NT), 4) void quant_once_kernel(OnceA
 // hand-over: [1,4608,24,128] 232.5 -> 228.4, [1,24,364,128] train 57.7 -> 54.2, [1,12,2304,64] F32 125.2 -> 119.9, e4m3 [1,585,30,128] 33.0 ->
 // 31.0, [1,2915,30,64] 101.7 -> 95.1, [1,4544,24,128] 207.8 -> 204.3, norm + RoPE [1,2207,30,128] 126.9 -> 114.9, [2,4352,30,128] 529 -> 506; but
 // e4m3 [1,5184,30,128] with norm + RoPE (630 groups and as many of V) 355 -> 359, [1,5824,24,128] 320 -> 334.
+// Behind the pre-ops, too, prep_rows_kernel has a group's norms done by four times as many threads, which is shorter for few keys and groups:
+// e4m3 [1,256,16,64] 17.9 -> 19.8 us, [1,1000,4,64] 21.0 -> 22.0, [1,128,16,128] 22.1 -> 22.7, fp16 [1,256,16,64] 19.0 -> 19.8, [1,500,40,64] 25.6 ->
+// 26.1; but fp16 of 128 channels gains at any length, [1,64,16,128] 24.3 -> 23.0, [1,300,16,128] 28.7 -> 25.8, [1,1000,40,128] 55.3 -> 46.9.
 bool quant_once_rule(const QuantArgs& a, const FinalArgs& f, int B, bool short_form) {
     const int64_t groups = (int64_t)f.ngroups * B * a.H;
-    if (short_form && (a.v8 != nullptr || f.ngroups < (f.D == 64 ? 3 : 2) || groups * f.D > 56 * 128)) return false;
+    const bool v_fp8 = a.v8 != nullptr;
+    if (a.pre_k.gain != nullptr && (f.D == 64 ? (v_fp8 ? groups < 72 : f.ngroups < 4) : v_fp8 && f.ngroups < 2)) return false;
+    if (short_form && (v_fp8 || f.ngroups < (f.D == 64 ? 3 : 2) || groups * f.D > 56 * 128)) return false;
     return f.D <= 128 && f.ngroups <= 32 && a.blkk == 64 && (f.flags & 3) != 0 && a.pre_k.row_inv == nullptr &&
-           (a.pre_k.gain != nullptr && a.v8 == nullptr ? groups <= 4096 : groups <= 512);
+           (a.pre_k.gain != nullptr && !v_fp8 ? groups <= 4096 : groups <= 512);
 }
 
 int64_t quant_once_flag_words(int B, int H, int Nkv, bool v_fp8) {
