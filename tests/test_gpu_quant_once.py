@@ -93,3 +93,23 @@ def test_one_shot_calls_that_share_a_workspace():
         A.sdpa_nomask(*qkv[0], 128 ** -0.5)
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(first, captured))
+
+
+@pytest.mark.parametrize("D,variant,Hh,S", [(128, 0, 2, 700), (64, 0, 70, 700), (64, 1, 3, 600), (128, 0, 29, 2305)])
+def test_non_finite_values_as_the_launches_take_them(D, variant, Hh, S):
+    """Infinities and NaNs in single tokens, NaNs alone in a leaf's channel, and values whose distance to the mean is the largest there is."""
+    rng = np.random.default_rng(S)
+    q, k, v = (f32_to_bf16_bits(rng.standard_normal((1, S, Hh, D), dtype=np.float32)) for _ in range(3))
+    k[0, 5, 0, 3] = 0x7F80
+    k[0, 300, 1, 7] = 0xFF80
+    k[0, 270, 0, 9] = 0x7FC0
+    k[0, 272:288, 1, 11] = 0x7FC0
+    k[0, 40, 1, 13], k[0, 41, 1, 13] = 0x7F7F, 0xFF7F
+    v[0, 17, 0, 2], v[0, 18, 1, 2] = 0x7F80, 0x7FC0
+    blkq = 128 if variant == 0 else 32
+    want = H.quant_qkv(q, k, v, D ** -0.5, variant, blkq, 64)
+    got = _once(q, k, v, D ** -0.5, variant, blkq, (0, 0), None, 1024)
+    for name in ("kscale", "k8", "qscale", "q8", "vq"):
+        np.testing.assert_array_equal(np.ascontiguousarray(got[name]).view(np.uint8), np.ascontiguousarray(want[name]).view(np.uint8), err_msg=name)
+    for name in ("kmean", "kmul", "qmul"):
+        np.testing.assert_array_equal(got[name], want[name], err_msg=name)          # (NaNs where there are NaNs)
