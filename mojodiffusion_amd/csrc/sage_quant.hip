@@ -1410,6 +1410,7 @@ struct OnceGroup {
     static constexpr int CH = S::CH, W = CH / 2;
     uint32_t w[kLeaf][W];
     uint32_t ext[CH];                               // smallest and largest value of this thread's leaf per channel, as the bf16 they are (publish)
+    bool ext_known;                                 // ... which they are in all of the wave's leaves
     bool all_kept;                                  // every token of the wave's leaves counts
     __device__ static __forceinline__ int leaf(int tid) { return tid / S::CPR; }
     __device__ static __forceinline__ int col(int tid) { return tid % S::CPR * CH; }
@@ -1513,12 +1514,20 @@ struct OnceGroup {
 #pragma unroll
                 for (int e = 0; e < CH; e++) acc[e] += (double)x[r][e];
             if (!all_kept) {
-                // (a NaN takes no part in a minimum or maximum)
+                // (a quiet NaN takes no part in a minimum or maximum; nor does one that signals in a leaf that is cut, as in kstats_group.
+                // The pre-ops leave none)
+                const bool whole = s0 + kLeaf <= a.Nkv && !(s0 < a.km.hi && s0 + kLeaf > a.km.lo);
 #pragma unroll
-                for (int r = 0; r < 2; r++)
-                    if (!key_kept(s0 + i + r, a.Nkv, a.km))
+                for (int r = 0; r < 2; r++) {
+                    const bool kept = key_kept(s0 + i + r, a.Nkv, a.km);
+                    if constexpr (!PRE) {
+#pragma unroll
+                        for (int e = 0; e < CH; e++) x[r][e] = whole ? x[r][e] : __builtin_canonicalizef(x[r][e]);
+                    }
+                    if (!kept)
 #pragma unroll
                         for (int e = 0; e < CH; e++) x[r][e] = __builtin_nanf("");
+                }
             }
             // (as instructions: see kstats_group)
 #pragma unroll
@@ -1526,6 +1535,13 @@ struct OnceGroup {
                 asm("v_min3_f32 %0, %0, %1, %2" : "+v"(mn[e]) : "v"(x[0][e]), "v"(x[1][e]));
                 asm("v_max3_f32 %0, %0, %1, %2" : "+v"(mx[e]) : "v"(x[0][e]), "v"(x[1][e]));
             }
+        }
+        // (where a leaf's values do not add up to a number, one of them may be a NaN that signals: min3 and max3 put it in the extreme's place)
+        if constexpr (!PRE) {
+            bool odd = false;
+#pragma unroll
+            for (int e = 0; e < CH; e++) odd = odd || acc[e] != acc[e];
+            ext_known = !__any(odd);
         }
 #pragma unroll
         for (int e = 0; e < CH; e++) {
@@ -1557,7 +1573,7 @@ struct OnceGroup {
     }
 
     // Codes and scales of the group's blocks of 64 keys.  (Meets a barrier.)
-    __device__ __forceinline__ void encode(const QuantArgs& a, int64_t bh, int g, int tid, OnceSmem<D, PRE>& sm, const OnceHead<D>& hd) {
+    __device__ __forceinline__ void encode(const QuantArgs& a, int64_t bh, int g, int h, int b, int tid, OnceSmem<D, PRE>& sm, const OnceHead<D>& hd) {
         asm volatile("" : "+v"(tid));
         const int s0 = g * kGroup + leaf(tid) * kLeaf, c = col(tid), wave = tid >> 6;
         float mu[CH], mul[CH];
@@ -1575,12 +1591,24 @@ struct OnceGroup {
                         am = fmaxf(am, fabsf(d * mul[e]));
                     }
                 }
+        } else if (__builtin_expect(!ext_known, 0)) {
+            const uint16_t* src = a.k.p + b * a.k.sb + h * a.k.sh + c;
+#pragma unroll 1
+            for (int i = 0; i < kLeaf; i++) {
+                if (!key_kept(s0 + i, a.Nkv, a.km)) continue;
+                const u32x2 v = *reinterpret_cast<const u32x2*>(src + (int64_t)(s0 + i) * a.k.sn);
+#pragma unroll
+                for (int e = 0; e < CH; e++) {
+                    const float d = (e & 1 ? bf16_hi(v[e >> 1]) : bf16_lo(v[e >> 1])) - mu[e];
+                    am = fmaxf(am, fabsf(d * mul[e]));
+                }
+            }
         } else {
             // (rounding is monotone: a leaf's largest |(k - mean) mul| in a channel is that of its largest or its smallest k)
 #pragma unroll
             for (int e = 0; e < CH; e++) {
                 const float mn = bf16_lo(ext[e]), mx = bf16_hi(ext[e]);
-                if (mn <= mx) {                                     // (not: a leaf without a key that counts, or NaNs alone)
+                if (mn <= mx) {                                     // (not: a leaf without a key that counts)
                     const float hi = mx - mu[e], lo = mn - mu[e];
                     am = fmaxf(fmaxf(am, fabsf(hi * mul[e])), fabsf(lo * mul[e]));
                 }
@@ -1795,7 +1823,7 @@ __global__ __launch_bounds__((OnceShape<D>::NT), 4) void quant_once_kernel(OnceA
             __syncthreads();
         }
         if (!once_k_head<D, PRE>(o, bh, h, b, tid, unit == 0, sm, hd, s_ok)) grp.load(a, unit, h, b, tid, sm);
-        grp.encode(a, bh, unit, tid, sm, hd);
+        grp.encode(a, bh, unit, h, b, tid, sm, hd);
     } else if (unit < o.nk + o.nv) {
         const int t = unit - o.nk;
         if (a.v16 != nullptr) {
