@@ -1471,15 +1471,8 @@ struct OnceGroup {
             const uint16_t* src = a.k.p + b * a.k.sb + h * a.k.sh + col(tid);
 #pragma unroll
             for (int i = 0; i < kLeaf; i++) {
-                const uint16_t* p = src + (int64_t)min(s0 + i, N - 1) * a.k.sn;
-                if constexpr (CH == 8) {
-                    const u32x4 v = *reinterpret_cast<const u32x4*>(p);
-#pragma unroll
-                    for (int e = 0; e < 4; e++) w[i][e] = v[e];
-                } else {
-                    const u32x2 v = *reinterpret_cast<const u32x2*>(p);
-                    w[i][0] = v.x; w[i][1] = v.y;
-                }
+                const u32x2 v = *reinterpret_cast<const u32x2*>(src + (int64_t)min(s0 + i, N - 1) * a.k.sn);
+                w[i][0] = v.x; w[i][1] = v.y;
             }
             if (!all_kept) {
 #pragma unroll
@@ -1814,7 +1807,7 @@ __global__ __launch_bounds__((OnceShape<D>::NT), 4) void quant_once_kernel(OnceA
         grp.load(a, unit, h, b, tid, sm);
         grp.publish(a, f, bh, unit, tid, sm);
         if (tid == 0 && o.raise) agent_store(flags + unit, o.tag);
-        if (o.k_apart) return;
+        if (PRE == 0 && o.k_apart) return;
         if (o.v_in) {
             OnceV<D> v;
             grp.pin();
@@ -1886,20 +1879,22 @@ __global__ __launch_bounds__((OnceShape<D>::NT), 4) void quant_once_kernel(OnceA
         const int r = unit - o.nk - o.nv - o.nkb;
         const KeyMask none{0, 0};
         // (the block's rows are requested ahead of the wait)
-        if (unit < o.nk + o.nv + o.nkb) {
-            constexpr int NCH = 64 * S::CPR8 / NT;
-            const int blk = unit - o.nk - o.nv;
-            u32x4 rows[NCH];
-            auto load = [&] {
-                const uint16_t* src = a.k.p + b * a.k.sb + h * a.k.sh + tid % S::CPR8 * 8;
+        if constexpr (PRE == 0) {
+            if (unit < o.nk + o.nv + o.nkb) {
+                constexpr int NCH = 64 * S::CPR8 / NT;
+                const int blk = unit - o.nk - o.nv;
+                u32x4 rows[NCH];
+                auto load = [&] {
+                    const uint16_t* src = a.k.p + b * a.k.sb + h * a.k.sh + tid % S::CPR8 * 8;
 #pragma unroll
-                for (int i = 0; i < NCH; i++) rows[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)min(blk * 64 + i * S::RP + tid / S::CPR8, a.Nkv - 1) * a.k.sn);
-            };
-            load();
-            if (!once_k_head<D, PRE>(o, bh, h, b, tid, blk == 0, sm, hd, s_ok)) load();
-            quant_i8_block<D, 64, true, PRE, NT, true>(blk, h, b, tid, a.k.p, a.k.sb, a.k.sh, a.k.sn, a.Nkv, a.H, a.nkv_pad, a.km, hd.mean, hd.kmul,
-                                                       0.0f, a.k8, a.kscale, nullptr, sm.red, a.pre_k, rows);
-            return;
+                    for (int i = 0; i < NCH; i++) rows[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)min(blk * 64 + i * S::RP + tid / S::CPR8, a.Nkv - 1) * a.k.sn);
+                };
+                load();
+                if (!once_k_head<D, PRE>(o, bh, h, b, tid, blk == 0, sm, hd, s_ok)) load();
+                quant_i8_block<D, 64, true, PRE, NT, true>(blk, h, b, tid, a.k.p, a.k.sb, a.k.sh, a.k.sn, a.Nkv, a.H, a.nkv_pad, a.km, hd.mean, hd.kmul,
+                                                           0.0f, a.k8, a.kscale, nullptr, sm.red, a.pre_k, rows);
+                return;
+            }
         }
 #define SAGE_Q(BLK)                                                                                                                                  do {                                                                                                                                                 constexpr int NCH = BLK * S::CPR8 / NT;                                                                                                          u32x4 rows[NCH];                                                                                                                                 auto load = [&] {                                                                                                                                    const uint16_t* src = a.q.p + b * a.q.sb + h * a.q.sh + tid % S::CPR8 * 8;                                                                       _Pragma("unroll") for (int i = 0; i < NCH; i++) {                                                                                                    const int row = r * BLK + i * S::RP + tid / S::CPR8;                                                                                             rows[i] = u32x4{0u, 0u, 0u, 0u};                                                                                                                 if (row < a.Nq) rows[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)row * a.q.sn);                                                      }                                                                                                                                            };                                                                                                                                               load();                                                                                                                                          if (!once_k_head<D, PRE>(o, bh, h, b, tid, false, sm, hd, s_ok)) load();                                                                            quant_i8_block<D, BLK, false, PRE, NT, true>(r, h, b, tid, a.q.p, a.q.sb, a.q.sh, a.q.sn, a.Nq, a.H, a.nq_pad, none, hd.mean, hd.qmul,                                                        a.cmul, a.q8, a.qscale, a.rowdot, sm.red, a.pre_q, rows);                                       } while (0)
         if (a.blkq == 128) SAGE_Q(128);
