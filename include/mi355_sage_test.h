@@ -58,13 +58,18 @@ int64_t mi355_sage_attn_main_items_on(int units, int B, int H, int N_q, int N_kv
 /* The quantize stage as the one launch whose workgroups hand their statistics to each other, whatever the shape (head
  * dims 64 and 128, K blocks of 64 keys, both K flags): outputs as mi355_sage_quant_qkv_bf16's, bit for bit, with the pre-ops of
  * mi355_sage_quant_qk_norm_rope_bf16 where q_gain is given.  scratch: mi355_sage_quant_scratch_bytes and 16 bytes
- * more per head and group of 256 keys, with any contents.  polls > 0: looks at a flag before a workgroup computes the groups it
- * waits for itself; polls < 0: no workgroup raises its flag, and every one computes them after -polls looks. */
+ * more per head and group of 256 keys, with any contents: behind mi355_sage_quant_scratch_bytes lie the flags, 8 bytes each, by head those of K's
+ * groups and, with e4m3, of V's.  polls > 0: looks at the flags before a workgroup computes the groups that are missing
+ * itself; polls < 0: no workgroup raises a flag, and every one computes all groups after -polls looks. */
 int mi355_sage_quant_once(const void* Q, const void* K, const void* V, int B, int H, int N_q, int N_kv, int D, float scale,
                           const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides, int variant, int blkq,
                           int mask_lo, int mask_hi, const void* q_gain, const void* k_gain, float eps, const void* rope_cos,
                           const void* rope_sin, int rope_layout, void* q8, void* qscale, void* k8, void* kscale, void* kmean, void* qmul,
                           void* kmul, void* vq, void* vscale, void* scratch, size_t scratch_bytes, int polls, void* stream);
+
+/* Groups that workgroups of that launch, in any call on the current device, computed after they had waited for them, since the last
+ * reset (< 0: a HIP error).  Asked after the caller's own synchronisation. */
+int mi355_sage_quant_once_helps(int reset);
 
 #ifdef __cplusplus
 }

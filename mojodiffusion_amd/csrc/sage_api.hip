@@ -251,8 +251,10 @@ uint64_t call_tag() {
     return z ^ (z >> 31);
 }
 
-// Looks (of about a microsecond) at another workgroup's flag before a workgroup computes what it waits for itself.
-constexpr int kOncePolls = 1024;
+// Looks (0.27 us each) at the other workgroups' flags before a workgroup computes what is missing itself: twice what any takes on a device with
+// nothing else on it (16 without the pre-ops, 32 and a few with them: [1,8192,30,128] with norm + RoPE has 61 groups computed twice at 32, none
+// at 64), and less than computing a head's groups takes (14 us for five, 60 for 18).  Behind another stream's kernel: see quant_once_kernel.
+constexpr int kOncePolls = 64;
 
 bool capturing(hipStream_t st) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -938,6 +940,7 @@ int mi355_sage_attn_fwd_q16(const void* Q, const int64_t* q_strides, int64_t q_o
 }
 
 int mi355_sage_attn_split_faults(int reset) { return attn_split_faults(reset); }
+int mi355_sage_quant_once_helps(int reset) { return quant_once_helps(reset); }
 
 // (declared in include/mi355_sage_test.h: switches for the library's own tests)
 int mi355_sage_attn_split_rule(int B, int H, int N_q, int N_kv, int D, int variant) {

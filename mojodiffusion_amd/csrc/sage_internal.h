@@ -119,7 +119,7 @@ struct OnceArgs {
     FinalArgs f;                     // all K outputs, and V's with e4m3
     uint64_t* flags;                 // quant_once_flag_words of them, whatever they hold
     uint64_t tag;                    // a number no other call uses
-    int polls;                       // looks at a flag before a workgroup computes what it waits for itself
+    int polls;                       // looks at the flags before a workgroup computes what is missing itself
     int raise;                       // 0: no flag is raised (tests)
     int nk, nv, nkb, heads, flag_words;      // filled by the launcher
     int k_apart, v_in;               // likewise: K's blocks are encoded by workgroups of their own / V (fp16) goes with K's groups
@@ -127,6 +127,7 @@ struct OnceArgs {
 int64_t quant_once_flag_words(int B, int H, int Nkv, bool v_fp8);
 bool quant_once_rule(const QuantArgs& a, const FinalArgs& f, int B, bool short_form);     // short_form: quant_short_kernel takes the call
 hipError_t launch_quant_once(const OnceArgs& a, int B, int D, hipStream_t st);
+int quant_once_helps(int reset);     // groups computed by workgroups that had waited for them, since the last reset (< 0: an error)
 
 // ---- attention kernel (sage_attn.hip) --------------------------------------
 // rint(x / sc) for |x / sc| <= ~127 without paying a full IEEE divide per element: x * (1/sc)

@@ -1356,10 +1356,16 @@ hipError_t launch_quant_short(const QuantArgs& a_in, const FinalArgs& f_in, int 
 // fence of that scope is.  A flag is raised when the wave's stores are complete (vmcnt) behind a barrier of the workgroup.
 // Flags hold a number that no other call of the process uses, so memory may hold anything before; a call under capture, whose
 // replays would all use one number, takes the launches.
-// The wait is bounded.  A workgroup that sees a flag missing after `polls` computes all groups of its head itself, the same values
-// into the same places: nothing depends on which workgroups are resident together, only the time does.  To have them
-// resident, heads come in chunks (OnceArgs::heads), their K groups first: a group waits for workgroups in front of it and a few
+// The wait is bounded.  A workgroup that sees a flag missing after `polls` looks computes the missing groups of its head itself, the same values
+// into the same places, and raises their flags: nothing depends on which workgroups are resident together, only the time does.  To have
+// them resident, heads come in chunks (OnceArgs::heads), their K groups first: a group waits for workgroups in front of it and a few
 // behind it.
+// Where another stream's kernel holds the chip they are not, and who waits keeps a compute unit from whoever it waits for: hence a bound of few looks.  Beside
+// back-to-back e4m3 [1,16896,24,128] calls of another stream, us a call and ms for twelve of the other's, by launches / with 1024 looks and all groups
+// computed by whoever gave up / now: [1,4608,24,128] 778 and 28.2 / 912 and 30.7 / 702 and 28.3; [2,2048,32,128] 550 and 26.9 / 840 and 28.8 / 608
+// and 26.6; [1,2304,12,64] 398 / 212 / 216.  The same calls on two streams at once, us a call: [1,1153,24,128] 30.5 / 28.8 / 28.8,
+// [2,2048,32,128] 134 / 126 / 124, but [1,4608,24,128] 195 / 216 to 271 / 214: the launches' small workgroups find room beside those of the
+// attention kernel, a group's does not (one stream: 229 / 221 / 221).
 // Every workgroup adds up the group results of its head itself, in group order.
 // What a K workgroup's time goes to at [1,1153,24,128] (one per compute unit), us: rows 1.6, sums and handing over 3, waiting 1.7, adding up 0.9,
 // encoding 2.6, next to 3 of the launch's start and end; bandwidth comes first from about 400 groups on.  (Encoding was 3.4 with a pass over
@@ -1401,6 +1407,31 @@ __device__ __forceinline__ bool flags_up(const uint64_t* flags, int n, uint64_t 
         __builtin_amdgcn_s_sleep(2);
     }
     return false;
+}
+
+// Groups that workgroups computed after they had waited for them, since the last reset (mi355_sage_quant_once_helps).
+static __device__ unsigned int g_once_helps;
+
+// The groups 0 .. n - 1 whose flag is missing, by this workgroup, from `from` on in a ring: group(g) leaves its results in memory, complete
+// behind a barrier.  Their flags are raised for whoever else waits.  (ok: in LDS, read by all before.)
+template <typename F>
+__device__ __forceinline__ void help_missing(uint64_t* flags, int n, int from, uint64_t tag, bool raise, int tid, int& ok, F group) {
+    int g = from;
+#pragma unroll 1
+    do {
+        __syncthreads();
+        asm volatile("" : "+s"(tag));               // (or vector registers hold it from one group to the next)
+        if (tid == 0) ok = agent_load(flags + g) == tag;
+        __syncthreads();
+        if (ok == 0) {
+            group(g);
+            if (tid == 0) {
+                atomicAdd(&g_once_helps, 1u);
+                if (raise) agent_store(flags + g, tag);
+            }
+        }
+        g = g + 1 == n ? 0 : g + 1;
+    } while (g != from);
 }
 
 // One group of keys in registers: a leaf of CH channels per thread.
@@ -1485,9 +1516,18 @@ struct OnceGroup {
         }
     }
 
+    // The rows once more, without what publish keeps of them.
+    __device__ __forceinline__ void reload(const QuantArgs& a, int g, int h, int b, int tid, OnceSmem<D, PRE>& sm) {
+        load(a, g, h, b, tid, sm);
+        ext_known = false;
+#pragma unroll
+        for (int e = 0; e < CH; e++) ext[e] = 0u;
+    }
+
     // The group's sums, minima and maxima to memory: the tree of kstats_group.  (Meets two barriers; stores complete behind them.)
     __device__ __forceinline__ void publish(const QuantArgs& a, const FinalArgs& f, int64_t bh, int g, int tid, OnceSmem<D, PRE>& sm) {
         asm volatile("" : "+v"(tid));
+        __builtin_assume(tid >= 0);                                // (or its sign is a register of its own)
         const int s0 = g * kGroup + leaf(tid) * kLeaf, c = col(tid);
         double acc[CH];
         float mn[CH], mx[CH];
@@ -1672,7 +1712,7 @@ struct OnceGroup {
 // The head's K statistics into hd, for a workgroup of NT threads; `leave`: and into memory, for later launches.
 // Returns false where it computed the groups itself: what the caller held in registers is then to be loaded again.
 template <int D, int PRE>
-__device__ __forceinline__ bool once_k_head(const OnceArgs& a, int64_t bh, int h, int b, int tid, bool leave, OnceSmem<D, PRE>& sm, OnceHead<D>& hd, int& s_ok) {
+__device__ __forceinline__ bool once_k_head(const OnceArgs& a, int64_t bh, int h, int b, int from, int tid, bool leave, OnceSmem<D, PRE>& sm, OnceHead<D>& hd, int& s_ok) {
     const FinalArgs& f = a.f;
     if (tid < 64) {
         const bool up = flags_up(a.flags + bh * a.flag_words, f.ngroups, a.tag, a.polls, tid);
@@ -1681,11 +1721,11 @@ __device__ __forceinline__ bool once_k_head(const OnceArgs& a, int64_t bh, int h
     __syncthreads();
     const bool ok = s_ok != 0;
     if (__builtin_expect(!ok, 0)) {
-        for (int g = 0; g < f.ngroups; g++) {
+        help_missing(a.flags + bh * a.flag_words, f.ngroups, (int)((unsigned)from % (unsigned)f.ngroups), a.tag, a.raise, tid, s_ok, [&](int g) {
             OnceGroup<D, PRE> grp;
             grp.load(a.q, g, h, b, tid, sm);
             grp.publish(a.q, f, bh, g, tid, sm);
-        }
+        });
     }
     if (tid < D) {
         constexpr int NB = 12;
@@ -1815,7 +1855,7 @@ __global__ __launch_bounds__((OnceShape<D>::NT), 4) void quant_once_kernel(OnceA
             once_v_f16<D>(a, bh, unit, tid, v, sm.tile16);
             __syncthreads();
         }
-        if (!once_k_head<D, PRE>(o, bh, h, b, tid, unit == 0, sm, hd, s_ok)) grp.load(a, unit, h, b, tid, sm);
+        if (!once_k_head<D, PRE>(o, bh, h, b, unit, tid, unit == 0, sm, hd, s_ok)) grp.reload(a, unit, h, b, tid, sm);
         grp.encode(a, bh, unit, h, b, tid, sm, hd);
     } else if (unit < o.nk + o.nv) {
         const int t = unit - o.nk;
@@ -1835,11 +1875,11 @@ __global__ __launch_bounds__((OnceShape<D>::NT), 4) void quant_once_kernel(OnceA
         }
         __syncthreads();
         if (__builtin_expect(s_ok == 0, 0)) {
-            for (int g = 0; g < f.ngroups; g++) {
+            help_missing(flags, f.ngroups, t, o.tag, o.raise, tid, s_ok, [&](int g) {
                 OnceV<D> x;
                 x.load(a, g, h, b, tid);
                 x.publish(f, bh, g, tid, sm.vred);
-            }
+            });
             v.load(a, t, h, b, tid);
         }
         if (tid < D) {
@@ -1890,13 +1930,13 @@ __global__ __launch_bounds__((OnceShape<D>::NT), 4) void quant_once_kernel(OnceA
                     for (int i = 0; i < NCH; i++) rows[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)min(blk * 64 + i * S::RP + tid / S::CPR8, a.Nkv - 1) * a.k.sn);
                 };
                 load();
-                if (!once_k_head<D, PRE>(o, bh, h, b, tid, blk == 0, sm, hd, s_ok)) load();
+                if (!once_k_head<D, PRE>(o, bh, h, b, blk, tid, blk == 0, sm, hd, s_ok)) load();
                 quant_i8_block<D, 64, true, PRE, NT, true>(blk, h, b, tid, a.k.p, a.k.sb, a.k.sh, a.k.sn, a.Nkv, a.H, a.nkv_pad, a.km, hd.mean, hd.kmul,
                                                            0.0f, a.k8, a.kscale, nullptr, sm.red, a.pre_k, rows);
                 return;
             }
         }
-#define SAGE_Q(BLK)                                                                                                                                  do {                                                                                                                                                 constexpr int NCH = BLK * S::CPR8 / NT;                                                                                                          u32x4 rows[NCH];                                                                                                                                 auto load = [&] {                                                                                                                                    const uint16_t* src = a.q.p + b * a.q.sb + h * a.q.sh + tid % S::CPR8 * 8;                                                                       _Pragma("unroll") for (int i = 0; i < NCH; i++) {                                                                                                    const int row = r * BLK + i * S::RP + tid / S::CPR8;                                                                                             rows[i] = u32x4{0u, 0u, 0u, 0u};                                                                                                                 if (row < a.Nq) rows[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)row * a.q.sn);                                                      }                                                                                                                                            };                                                                                                                                               load();                                                                                                                                          if (!once_k_head<D, PRE>(o, bh, h, b, tid, false, sm, hd, s_ok)) load();                                                                            quant_i8_block<D, BLK, false, PRE, NT, true>(r, h, b, tid, a.q.p, a.q.sb, a.q.sh, a.q.sn, a.Nq, a.H, a.nq_pad, none, hd.mean, hd.qmul,                                                        a.cmul, a.q8, a.qscale, a.rowdot, sm.red, a.pre_q, rows);                                       } while (0)
+#define SAGE_Q(BLK)                                                                                                                                  do {                                                                                                                                                 constexpr int NCH = BLK * S::CPR8 / NT;                                                                                                          u32x4 rows[NCH];                                                                                                                                 auto load = [&] {                                                                                                                                    const uint16_t* src = a.q.p + b * a.q.sb + h * a.q.sh + tid % S::CPR8 * 8;                                                                       _Pragma("unroll") for (int i = 0; i < NCH; i++) {                                                                                                    const int row = r * BLK + i * S::RP + tid / S::CPR8;                                                                                             rows[i] = u32x4{0u, 0u, 0u, 0u};                                                                                                                 if (row < a.Nq) rows[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)row * a.q.sn);                                                      }                                                                                                                                            };                                                                                                                                               load();                                                                                                                                          if (!once_k_head<D, PRE>(o, bh, h, b, r, tid, false, sm, hd, s_ok)) load();                                                                            quant_i8_block<D, BLK, false, PRE, NT, true>(r, h, b, tid, a.q.p, a.q.sb, a.q.sh, a.q.sn, a.Nq, a.H, a.nq_pad, none, hd.mean, hd.qmul,                                                        a.cmul, a.q8, a.qscale, a.rowdot, sm.red, a.pre_q, rows);                                       } while (0)
         if (a.blkq == 128) SAGE_Q(128);
         else if (a.blkq == 64) SAGE_Q(64);
         else SAGE_Q(32);
@@ -1955,7 +1995,7 @@ hipError_t launch_quant_once(const OnceArgs& o_in, int B, int D, hipStream_t st)
     // [1,8,4224,128] (136) level, [2,24,1024,64] (192) 36.4 -> 39.1.
     o.v_in = !o.k_apart && !v_fp8 && groups > compute_units();
     if (o.v_in) o.nv = 0;
-    // (two workgroups to a compute unit are resident for certain)
+    // (two workgroups to a compute unit are resident together where nothing else runs on the device; elsewhere the bound on the wait counts)
     o.heads = max(1, min(a.n_bh, 2 * compute_units() / (o.nk * (v_fp8 ? 2 : 1))));
     const int64_t total = (int64_t)a.n_bh * (o.nk + o.nv + o.nkb + a.nq_blk);
     if (total <= 0 || total > 0x7FFFFFFF) return hipErrorInvalidValue;
@@ -1970,6 +2010,16 @@ hipError_t launch_quant_once(const OnceArgs& o_in, int B, int D, hipStream_t st)
     else return hipErrorInvalidValue;
 #undef SAGE_ONCE
     return hipGetLastError();
+}
+
+int quant_once_helps(int reset) {
+    unsigned n = 0;
+    hipError_t e = hipMemcpyFromSymbol(&n, HIP_SYMBOL(g_once_helps), sizeof(n));
+    if (e == hipSuccess && reset) {
+        const unsigned zero = 0;
+        e = hipMemcpyToSymbol(HIP_SYMBOL(g_once_helps), &zero, sizeof(zero));
+    }
+    return e == hipSuccess ? (int)n : -(int)e;
 }
 
 }  // namespace sage
