@@ -1,6 +1,6 @@
 """The waits of the one-launch quantize stage: each run by itself leaves the bits of the launches, in buffers that hold something else
 before — handed over with no group computed twice, with a single look before a workgroup computes what is missing, and where no flag is
-ever raised — and calls of all kinds on two streams at once give the bits they give alone."""
+ever raised — and calls of all kinds on two streams at once, and under capture, give the bits they give alone."""
 import numpy as np
 import pytest
 
@@ -123,6 +123,20 @@ def test_each_run_by_itself(D, variant, B, Hh, Sq, Skv, mask, pre):
         assert helps == 0 if polls > 1 else helps < s.helps_without_flags()
 
 
+@pytest.mark.parametrize("D,variant,Hh,S,pre", [(128, 0, 3, 700, 0), (64, 0, 3, 1100, 1), (64, 1, 3, 600, 0), (128, 1, 3, 600, 1)])
+def test_non_finite_values_behind_the_pre_ops(D, variant, Hh, S, pre):
+    rng, q, k, v = _inputs(1, Hh, S, S, D)
+    k[0, 5, 0, 3], k[0, 300, 1, 7], k[0, 270, 0, 9], k[0, 17, 2, 1] = 0x7F80, 0xFF80, 0x7FC0, 0x7F81
+    k[0, 40, 1, 13], k[0, 41, 1, 13] = 0x7F7F, 0xFF7F
+    q[0, 9, 0, 4], q[0, 130, 1, 4], q[0, 131, 2, 4] = 0x7F80, 0x7FC0, 0xFF81
+    v[0, 17, 0, 2], v[0, 18, 1, 2], v[0, 19, 2, 2] = 0x7F80, 0x7FC0, 0x7F81
+    blkq = 128 if variant == 0 else 32
+    want, p = _by_launches(rng, q, k, v, variant, blkq, (0, 0), pre)
+    s = Stage(q, k, v, variant, blkq, (0, 0), p)
+    for polls in (1024, -1):
+        _same(s.run(polls, 0x5A)[0], want, variant, bits=False)
+
+
 def _calls():
     """One-shot calls of the forms the stage has, as functions of no arguments that return their output."""
     import torch
@@ -140,6 +154,23 @@ def _calls():
         tables = [torch.rand((S * Hh, D // 2), generator=g, device="cuda") for _ in range(2)]
         calls.append(lambda x=x, gains=gains, tables=tables, D=D, variant=variant: A.qk_norm_rope_sdpa_nomask(*x, *gains, 1e-6, *tables, D ** -0.5, variant))
     return calls
+
+
+def test_one_workspace_for_calls_of_all_kinds():
+    """In turn on one stream, whose flags and group results lie over each other's workspace, eager and in a graph's replays."""
+    import torch
+    calls = _calls()
+    g = torch.cuda.CUDAGraph()
+    first = [f().clone() for f in calls]
+    with torch.cuda.graph(g):
+        captured = [f() for f in calls]
+    for turn in range(6):
+        outs = [f() for f in (calls if turn % 2 else calls[::-1])]
+        for o, want in zip(outs if turn % 2 else outs[::-1], first):
+            assert torch.equal(o, want)
+        g.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(o, want) for o, want in zip(captured, first))
 
 
 def test_calls_on_two_streams_at_once():
