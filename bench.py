@@ -191,10 +191,10 @@ def clock_probe(args, L, w, qd, kd, vd, o, st, stream):
 def run_workload(L, torch, w, qd, kd, vd, steps, warmup, n_events):
     """One workload through the one-shot call (wall clock over back-to-back steps) and through the
     stage entry points with HIP events on the launch stream, each stage as the one-shot call runs it:
-    the quantize stage (three launches, mi355_sage_quant_qkv_bf16) and the attention kernel.  Where the
+    the quantize stage (one launch by hand-over, mi355_sage_quant_once, where the call makes that; otherwise the
+    launches of mi355_sage_quant_qkv_bf16, which calls under capture make too) and the attention kernel.  Where the
     one-shot call leaves the Q encode to the attention kernel (every shape but those of the split
-    schedule), so do the stages timed here: mi355_sage_quant_qkv_bf16 without Q outputs and
-    mi355_sage_attn_fwd_q16."""
+    schedule), so do the stages timed here: the quantize stage without Q outputs and mi355_sage_attn_fwd_q16."""
     from mojodiffusion_amd import _lib
     dev = qd.device
     B, S, H, D = w.B, w.S, w.H, w.D
@@ -237,14 +237,16 @@ def run_workload(L, torch, w, qd, kd, vd, steps, warmup, n_events):
     ks = torch.empty((B, H, nkp // w.blkk), dtype=torch.float32, device=dev)
     km, qm, kmu, vsc = (torch.empty((B, H, D), dtype=torch.float32, device=dev) for _ in range(4))
     vq = torch.empty((B, H, nkp // 64, D, 64), dtype=torch.int16 if w.variant == 0 else torch.uint8, device=dev)
-    scr = torch.empty(max(L.mi355_sage_quant_scratch_bytes(B, H, S, D), 8), dtype=torch.uint8, device=dev)
+    # (and the hand-over's flags: 16 bytes per head and group of 256 keys)
+    scr = torch.empty(L.mi355_sage_quant_scratch_bytes(B, H, S, D) + 16 * B * H * ((S + 255) // 256), dtype=torch.uint8, device=dev)
 
-    def stage_quant(with_q):
-        return L.mi355_sage_quant_qkv_bf16(qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), B, H, S, S, D, w.scale, st, st, st,
-                                           0, 0, 0, w.variant, w.blkq, w.blkk, K_FLAGS, 0, 0,
-                                           q8.data_ptr() if with_q else None, qs.data_ptr() if with_q else None,
-                                           k8.data_ptr(), ks.data_ptr(), km.data_ptr(), qm.data_ptr(), kmu.data_ptr(),
-                                           vq.data_ptr(), vsc.data_ptr(), scr.data_ptr(), scr.numel(), stream)
+    def stage_quant(with_q, once=False):
+        outs = (q8.data_ptr() if with_q else None, qs.data_ptr() if with_q else None, k8.data_ptr(), ks.data_ptr(), km.data_ptr(),
+                qm.data_ptr(), kmu.data_ptr(), vq.data_ptr(), vsc.data_ptr(), scr.data_ptr(), scr.numel())
+        x = (qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), B, H, S, S, D, w.scale, st, st, st)
+        if once:                              # (64 looks: the one-shot call's own)
+            return L.mi355_sage_quant_once(*x, w.variant, w.blkq, 0, 0, None, None, 0.0, None, None, 0, *outs, 64, stream)
+        return L.mi355_sage_quant_qkv_bf16(*x, 0, 0, 0, w.variant, w.blkq, w.blkk, K_FLAGS, 0, 0, *outs, stream)
 
     def attn_q8():
         return L.mi355_sage_attn_fwd(q8.data_ptr(), qs.data_ptr(), w.blkq, k8.data_ptr(), ks.data_ptr(), w.blkk,
@@ -276,10 +278,11 @@ def run_workload(L, torch, w, qd, kd, vd, steps, warmup, n_events):
         ts = sorted(a.elapsed_time(b) for a, b in evs)
         return sum(ts) / len(ts), ts[len(ts) // 2], ts[0]
 
-    qt_avg, qt_med, qt_min = time_stage(lambda: stage_quant(not q_in_kernel), n_events)
+    once = L.mi355_sage_quant_once_takes(B, H, S, S, D, w.variant, w.blkq, w.blkk, K_FLAGS, not q_in_kernel) == 1
+    qt_avg, qt_med, qt_min = time_stage(lambda: stage_quant(not q_in_kernel, once), n_events)
     at_avg, at_med, at_min = time_stage(stage_attn, n_events)
     return dict(step=step, ms_per_step=ms_per_step, ramp_steps=ramp_steps, quant=(qt_avg, qt_med, qt_min),
-                attn=(at_avg, at_med, at_min), q_in_kernel=q_in_kernel, keep=(o, ws, q8, k8, qs, ks, km, qm, kmu, vsc, vq, scr))
+                attn=(at_avg, at_med, at_min), q_in_kernel=q_in_kernel, once=once, keep=(o, ws, q8, k8, qs, ks, km, qm, kmu, vsc, vq, scr))
 
 
 def main():
@@ -407,8 +410,7 @@ def main():
             "ops_per_step": w.ops,
             "pct_of_peak": round(100.0 * tops / peak, 2),
             "peak_tops_used": peak,
-            # HIP-event pairs on the launch stream around the quantize stage as the step runs it (three
-            # launches through mi355_sage_quant_qkv_bf16) and around the attention launch
+            # HIP-event pairs on the launch stream around the quantize stage as the step runs it and around the attention launch
             "stage_ms": {"quantize": round(qt_avg, 5), "attn": round(at_avg, 5)},
             "q_encoded_by": "attention kernel (prologue)" if fused else "quantize stage",
             "graph_replay_ms": None if graph_ms is None else round(graph_ms, 5),
@@ -430,10 +432,10 @@ def main():
             "avg_ms": round(at_avg, 5), "median_ms": round(at_med, 5), "min_ms": round(at_min, 5),
             "algorithmic_ops_per_launch": w.ops,
         },
-        # the HBM-bound part of the step: prep_kernel, stats_final_kernel, quant_kernel together
+        # the HBM-bound part of the step
         "roofline_quantize": {
-            "kernels": "prep_kernel + stats_final_kernel + quant_kernel (one event pair around the three launches)%s" % (
-                "; K and V only" if fused else ""),
+            "kernels": ("quant_once_kernel (one launch)" if r["once"] else
+                        "prep_kernel + stats_final_kernel + quant_kernel (one event pair around the launches)") + ("; K and V only" if fused else ""),
             "bound": "hbm",
             "achieved": round(quant_gbs, 1),
             "peak": PEAK_HBM_GBS,

@@ -70,6 +70,8 @@ int mi355_sage_quant_once(const void* Q, const void* K, const void* V, int B, in
 /* Groups that workgroups of that launch, in any call on the current device, computed after they had waited for them, since the last
  * reset (< 0: a HIP error).  Asked after the caller's own synchronisation. */
 int mi355_sage_quant_once_helps(int reset);
+/* 1 where a one-shot call of that shape without pre-ops, not under capture, makes its quantize stage that launch (with_q: Q's codes in it). */
+int mi355_sage_quant_once_takes(int B, int H, int N_q, int N_kv, int D, int variant, int blkq, int blkk, int k_flags, int with_q);
 
 #ifdef __cplusplus
 }

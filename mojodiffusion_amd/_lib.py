@@ -72,6 +72,7 @@ SIGNATURES = {
     "mi355_sage_quant_once": (_int, [_vp] * 3 + [_int] * 5 + [ctypes.c_float, _i64p, _i64p, _i64p] + [_int] * 4
                               + [_vp, _vp, ctypes.c_float, _vp, _vp, _int] + [_vp] * 10 + [ctypes.c_size_t, _int, _vp]),
     "mi355_sage_quant_once_helps": (_int, [_int]),
+    "mi355_sage_quant_once_takes": (_int, [_int] * 10),
     "mi355_sage_version": (ctypes.c_char_p, []),
 }
 

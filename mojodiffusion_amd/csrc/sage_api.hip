@@ -296,7 +296,8 @@ int quantize(const View& q, const View& k, const View* v, int B, int H, int Nq, 
     else if (v != nullptr) { a.v = *v; a.v16 = static_cast<uint16_t*>(vq); }
     a.pre_q = pre.q; a.pre_k = pre.k;
     const bool forced = o.once_polls != 0, short_form = v != nullptr && quant_short_workgroups(a, B, D) > 0;
-    if (forced || (v != nullptr && o.flags != nullptr && quant_once_rule(a, f, B, short_form) &&
+    if (forced || (v != nullptr && o.flags != nullptr &&
+                   quant_once_rule(B, H, Nkv, D, blkk, k_flags, v_fp8, a.pre_k.gain != nullptr, pre.full_row, short_form) &&
                    (size_t)quant_once_flag_words(B, H, Nkv, v_fp8) * sizeof(uint64_t) <= o.flag_bytes && !capturing(st))) {
         OnceArgs w{};
         w.q = a; w.f = f;
@@ -941,6 +942,13 @@ int mi355_sage_attn_fwd_q16(const void* Q, const int64_t* q_strides, int64_t q_o
 
 int mi355_sage_attn_split_faults(int reset) { return attn_split_faults(reset); }
 int mi355_sage_quant_once_helps(int reset) { return quant_once_helps(reset); }
+int mi355_sage_quant_once_takes(int B, int H, int N_q, int N_kv, int D, int variant, int blkq, int blkk, int k_flags, int with_q) {
+    if (B <= 0 || H <= 0 || N_q <= 0 || N_kv <= 0 || !dims_ok(D) || !blk_ok(blkq) || !blk_ok(blkk)) return MI355_SAGE_EINVAL;
+    const bool v_fp8 = variant != MI355_SAGE_PV_FP16;
+    const Carve c = carve(B, H, N_q, N_kv, D, variant);
+    return quant_once_rule(B, H, N_kv, D, blkk, k_flags, v_fp8, false, false, quant_short_workgroups(B, H, N_q, N_kv, D, blkq, blkk, with_q != 0) > 0) &&
+           (size_t)quant_once_flag_words(B, H, N_kv, v_fp8) * sizeof(uint64_t) <= c.split - c.rowinv_q;
+}
 
 // (declared in include/mi355_sage_test.h: switches for the library's own tests)
 int mi355_sage_attn_split_rule(int B, int H, int N_q, int N_kv, int D, int variant) {

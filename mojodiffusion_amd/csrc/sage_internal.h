@@ -74,10 +74,10 @@ struct FinalArgs {
     int64_t total;                   // B*H*D
     int D, ngroups, kept, flags;     // kept = number of keys that count; flags: bit 0 smoothing, bit 1 balancing
     float cmul;                      // fp32(scale*log2(e))
-    const double* kpart_sum;         // null: no K statistics (mean 0, factor 1)
-    const float* kpart_mm;
+    double* kpart_sum;               // null: no K statistics (mean 0, factor 1).  (The one-launch stage writes the three.)
+    float* kpart_mm;
     float *kmean, *qmul, *kmul;      // [B,H,D] each; kmean null: K outputs are skipped
-    const float* vpart;
+    float* vpart;
     float* vscale;                   // null: V output is skipped
 };
 hipError_t launch_stats_final(const FinalArgs& a, hipStream_t st);
@@ -125,7 +125,8 @@ struct OnceArgs {
     int k_apart, v_in;               // likewise: K's blocks are encoded by workgroups of their own / V (fp16) goes with K's groups
 };
 int64_t quant_once_flag_words(int B, int H, int Nkv, bool v_fp8);
-bool quant_once_rule(const QuantArgs& a, const FinalArgs& f, int B, bool short_form);     // short_form: quant_short_kernel takes the call
+// (pre: the fused pre-ops; full_row: with a norm of whole rows; short_form: quant_short_kernel takes the call)
+bool quant_once_rule(int B, int H, int Nkv, int D, int blkk, int k_flags, bool v_fp8, bool pre, bool full_row, bool short_form);
 hipError_t launch_quant_once(const OnceArgs& a, int B, int D, hipStream_t st);
 int quant_once_helps(int reset);     // groups computed by workgroups that had waited for them, since the last reset (< 0: an error)
 

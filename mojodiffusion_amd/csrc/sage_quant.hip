@@ -1589,7 +1589,7 @@ struct OnceGroup {
             double sum = 0.0;
 #pragma unroll
             for (int u = 0; u < 16; u++) sum += sm.leaf.sum[u][tid];
-            agent_store(const_cast<double*>(f.kpart_sum) + (bh * f.ngroups + g) * D + leaf_channel<D>(tid), sum);
+            agent_store(f.kpart_sum + (bh * f.ngroups + g) * D + leaf_channel<D>(tid), sum);
         } else if (tid < 2 * D) {
             const int t = tid - D;
             float lo = INFINITY, hi = -INFINITY;
@@ -1598,7 +1598,7 @@ struct OnceGroup {
                 lo = fminf(lo, sm.leaf.mn[u][t]);
                 hi = fmaxf(hi, sm.leaf.mx[u][t]);
             }
-            agent_store(reinterpret_cast<uint64_t*>(const_cast<float*>(f.kpart_mm)) + (bh * f.ngroups + g) * D + leaf_channel<D>(t),
+            agent_store(reinterpret_cast<uint64_t*>(f.kpart_mm) + (bh * f.ngroups + g) * D + leaf_channel<D>(t),
                         (uint64_t)__float_as_uint(lo) | (uint64_t)__float_as_uint(hi) << 32);
         }
         stores_done();
@@ -1801,7 +1801,7 @@ template <int D> struct OnceV {
             float mm = 0.0f;
 #pragma unroll
             for (int i = 0; i < S::RP; i++) mm = fmaxf(mm, red[i][tid]);
-            agent_store(const_cast<float*>(f.vpart) + (bh * f.ngroups + g) * D + leaf_channel<D>(tid), mm);
+            agent_store(f.vpart + (bh * f.ngroups + g) * D + leaf_channel<D>(tid), mm);
         }
         stores_done();
         __syncthreads();
@@ -1825,6 +1825,28 @@ __device__ __forceinline__ void once_v_f16(const QuantArgs& a, int64_t bh, int g
     for (int j = 0; j < 4; j++)
         if ((g * 4 + j) * 64 < a.nkv_pad)
             store_v_f16_tile<D, S::NT>(tid, tile[j], a.v16 + (bh * (a.nkv_pad / 64) + g * 4 + j) * (int64_t)(D * 64));
+}
+
+// Block r of BLK queries, whose rows are requested ahead of the wait.
+template <int D, int PRE, int BLK>
+__device__ __forceinline__ void once_q_block(const OnceArgs& o, int64_t bh, int h, int b, int r, int tid, OnceSmem<D, PRE>& sm, OnceHead<D>& hd, int& s_ok) {
+    using S = OnceShape<D>;
+    constexpr int NCH = BLK * S::CPR8 / S::NT;
+    const QuantArgs& a = o.q;
+    u32x4 rows[NCH];
+    auto load = [&] {
+        const uint16_t* src = a.q.p + b * a.q.sb + h * a.q.sh + tid % S::CPR8 * 8;
+#pragma unroll
+        for (int i = 0; i < NCH; i++) {
+            const int row = r * BLK + i * S::RP + tid / S::CPR8;
+            rows[i] = u32x4{0u, 0u, 0u, 0u};
+            if (row < a.Nq) rows[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)row * a.q.sn);
+        }
+    };
+    load();
+    if (!once_k_head<D, PRE>(o, bh, h, b, r, tid, false, sm, hd, s_ok)) load();
+    quant_i8_block<D, BLK, false, PRE, S::NT, true>(r, h, b, tid, a.q.p, a.q.sb, a.q.sh, a.q.sn, a.Nq, a.H, a.nq_pad, KeyMask{0, 0}, hd.mean, hd.qmul,
+                                                    a.cmul, a.q8, a.qscale, a.rowdot, sm.red, a.pre_q, rows);
 }
 
 template <int D, int PRE>
@@ -1917,10 +1939,8 @@ __global__ __launch_bounds__((OnceShape<D>::NT), 4) void quant_once_kernel(OnceA
         }
     } else {
         const int r = unit - o.nk - o.nv - o.nkb;
-        const KeyMask none{0, 0};
-        // (the block's rows are requested ahead of the wait)
         if constexpr (PRE == 0) {
-            if (unit < o.nk + o.nv + o.nkb) {
+            if (unit < o.nk + o.nv + o.nkb) {              // (rows ahead of the wait, as in once_q_block)
                 constexpr int NCH = 64 * S::CPR8 / NT;
                 const int blk = unit - o.nk - o.nv;
                 u32x4 rows[NCH];
@@ -1936,11 +1956,9 @@ __global__ __launch_bounds__((OnceShape<D>::NT), 4) void quant_once_kernel(OnceA
                 return;
             }
         }
-#define SAGE_Q(BLK)                                                                                                                                  do {                                                                                                                                                 constexpr int NCH = BLK * S::CPR8 / NT;                                                                                                          u32x4 rows[NCH];                                                                                                                                 auto load = [&] {                                                                                                                                    const uint16_t* src = a.q.p + b * a.q.sb + h * a.q.sh + tid % S::CPR8 * 8;                                                                       _Pragma("unroll") for (int i = 0; i < NCH; i++) {                                                                                                    const int row = r * BLK + i * S::RP + tid / S::CPR8;                                                                                             rows[i] = u32x4{0u, 0u, 0u, 0u};                                                                                                                 if (row < a.Nq) rows[i] = *reinterpret_cast<const u32x4*>(src + (int64_t)row * a.q.sn);                                                      }                                                                                                                                            };                                                                                                                                               load();                                                                                                                                          if (!once_k_head<D, PRE>(o, bh, h, b, r, tid, false, sm, hd, s_ok)) load();                                                                            quant_i8_block<D, BLK, false, PRE, NT, true>(r, h, b, tid, a.q.p, a.q.sb, a.q.sh, a.q.sn, a.Nq, a.H, a.nq_pad, none, hd.mean, hd.qmul,                                                        a.cmul, a.q8, a.qscale, a.rowdot, sm.red, a.pre_q, rows);                                       } while (0)
-        if (a.blkq == 128) SAGE_Q(128);
-        else if (a.blkq == 64) SAGE_Q(64);
-        else SAGE_Q(32);
-#undef SAGE_Q
+        if (a.blkq == 128) once_q_block<D, PRE, 128>(o, bh, h, b, r, tid, sm, hd, s_ok);
+        else if (a.blkq == 64) once_q_block<D, PRE, 64>(o, bh, h, b, r, tid, sm, hd, s_ok);
+        else once_q_block<D, PRE, 32>(o, bh, h, b, r, tid, sm, hd, s_ok);
     }
 }
 
@@ -1956,13 +1974,12 @@ __global__ __launch_bounds__((OnceShape<D>::NT), 4) void quant_once_kernel(OnceA
 // Behind the pre-ops, too, prep_rows_kernel has a group's norms done by four times as many threads, which is shorter for few keys and groups:
 // e4m3 [1,256,16,64] 17.9 -> 19.8 us, [1,1000,4,64] 21.0 -> 22.0, [1,128,16,128] 22.1 -> 22.7, fp16 [1,256,16,64] 19.0 -> 19.8, [1,500,40,64] 25.6 ->
 // 26.1; but fp16 of 128 channels gains at any length, [1,64,16,128] 24.3 -> 23.0, [1,300,16,128] 28.7 -> 25.8, [1,1000,40,128] 55.3 -> 46.9.
-bool quant_once_rule(const QuantArgs& a, const FinalArgs& f, int B, bool short_form) {
-    const int64_t groups = (int64_t)f.ngroups * B * a.H;
-    const bool v_fp8 = a.v8 != nullptr;
-    if (a.pre_k.gain != nullptr && (f.D == 64 ? (v_fp8 ? groups < 72 : f.ngroups < 4) : v_fp8 && f.ngroups < 2)) return false;
-    if (short_form && (v_fp8 || f.ngroups < (f.D == 64 ? 3 : 2) || groups * f.D > 56 * 128)) return false;
-    return f.D <= 128 && f.ngroups <= 32 && a.blkk == 64 && (f.flags & 3) != 0 && a.pre_k.row_inv == nullptr &&
-           (a.pre_k.gain != nullptr && !v_fp8 ? groups <= 4096 : groups <= 512);
+bool quant_once_rule(int B, int H, int Nkv, int D, int blkk, int k_flags, bool v_fp8, bool pre, bool full_row, bool short_form) {
+    const int ngroups = (Nkv + kGroup - 1) / kGroup;
+    const int64_t groups = (int64_t)ngroups * B * H;
+    if (pre && (D == 64 ? (v_fp8 ? groups < 72 : ngroups < 4) : v_fp8 && ngroups < 2)) return false;
+    if (short_form && (v_fp8 || ngroups < (D == 64 ? 3 : 2) || groups * D > 56 * 128)) return false;
+    return D <= 128 && ngroups <= 32 && blkk == 64 && (k_flags & 3) != 0 && !full_row && (pre && !v_fp8 ? groups <= 4096 : groups <= 512);
 }
 
 int64_t quant_once_flag_words(int B, int H, int Nkv, bool v_fp8) {
