@@ -241,8 +241,8 @@ struct QuantOut {
     int once_polls;                   // tests: that form, with so many looks at a flag (< 0: and no flag raised); 0: by the rule
 };
 
-// A number for the flags of one call: no two calls of a process share one (a bijection of the counter), and memory that other
-// work has filled does not hold it but for a chance of 2^-64 a word.
+// A number for the flags of one call: no two calls of a process share one (SplitMix64's finalizer, a bijection of the counter), and memory that
+// other work has filled does not hold it but for a chance of 2^-64 a word.
 uint64_t call_tag() {
     static std::atomic<uint64_t> n{(uint64_t)std::chrono::steady_clock::now().time_since_epoch().count() << 20};
     uint64_t z = n.fetch_add(1, std::memory_order_relaxed) * 0x9E3779B97F4A7C15ull;
@@ -411,14 +411,14 @@ int sdpa_impl(const void* Q, const void* K, const void* V, void* O, void* Stats,
     // scales): the quantize stage then neither reads Q nor writes its codes.
     // Not where the encoders have room for it and a prologue is on the path of the whole call — the main kernel does
     // everything in one round that leaves compute units without a workgroup (us with Q in the kernel -> in the
-    // encoders: [1,700,24,128] 36.7 -> 34.3, [1,1153,24,128] 46.6 -> 43.8; but [1,2304,24,128], two rounds, 72.9 ->
-    // 75.4) — nor, with e4m3 P.V, whose scale blocks are single waves' and whose prologue costs more, where the short form
-    // does all or part of it ([1,256,30,128] 18.9 -> 16.8, [1,1153,24,128] 49.8 -> 46.6, [1,3072,30,128] 153.2 -> 151.1) or the
-    // main kernel fills at most five eighths of the chip ([2,320,32,128], 128 of them, 33.2 -> 31.4; but 240, [1,1497,40,128], 62.9 -> 66.7,
-    // 256, [2,1995,16,128], 73.9 -> 78.0, 960, [2,2822,40,128], 308.6 -> 315.9), up to 8192 tokens of 128 channels, 4096 of 64
-    // (level at 16896).  Many queries on few keys keep it ([1,3840 x 333,32,128] fp16
-    // 50.1 -> 52.0, e4m3 57.5 -> 64.0), and so does a K that takes one launch alone and three, or more than a
-    // workgroup per compute unit, with Q ([1,2048 x 512,32,64] 23.7 -> 30.4, e4m3 [1,512,24,128] 21.5 -> 25.6).
+    // encoders, with the stage in one launch by hand-over wherever the call makes it that: [1,700,24,128] 28.5 -> 26.5, [1,1153,24,128] 38.0 -> 34.4,
+    // [1,2000,12,128] 42.2 -> 40.2; level at two rounds, [1,2304,24,128] 67.0; [1,4608,24,128] 206.8 -> 209.3) — nor, with e4m3 P.V, whose scale blocks
+    // are single waves' and whose prologue costs more, where the short form does all or part of it ([1,256,30,128] 15.7 -> 14.6; the line was drawn where the stage was
+    // two launches, [1,1153,24,128] 49.8 -> 46.6, and that call is now 35.4 -> 37.0) or the main kernel fills at most five eighths of the chip
+    // (128 of them, [2,320,32,128], 31.1 -> 30.7, where the last of these rules speaks against it; but 240, [1,1497,40,128], 53.3 -> 60.3, 256, [2,1995,16,128], 63.6 -> 71.3, 960, [2,2822,40,128],
+    // 285.9 -> 290.1), up to 8192 tokens of 128 channels, 4096 of 64.  Many queries on few keys keep it ([1,3840 x 333,32,128] fp16
+    // 43.4 -> 47.3, e4m3 44.0 -> 60.0), and so does a K that takes quant_short_kernel alone and the launches, or more than a
+    // workgroup per compute unit, with Q ([1,2048 x 512,32,64] 21.5 -> 26.5, e4m3 [1,512,24,128] 20.4 -> 24.3).
     auto one_launch = [&](bool with_q) { return quant_short_workgroups(B, H, N_q, kv, D, blkq, blkk, with_q); };
     const int units = compute_units();
     // (row tiles of the main kernel's loop in one round or less; of both its forms together where it takes more)

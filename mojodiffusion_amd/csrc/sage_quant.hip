@@ -1962,18 +1962,22 @@ __global__ __launch_bounds__((OnceShape<D>::NT), 4) void quant_once_kernel(OnceA
     }
 }
 
-// Where the stage is one launch by hand-over.  Not past 32 groups to a head, which every workgroup adds up.  Of the calls that
-// quant_short_kernel takes (a workgroup there computes its head's statistics itself and waits for nobody), those with fp16 V of two and more groups,
-// three at 64 channels, up to 56 groups of 128 channels in all.  The call, us, short -> hand-over, K's blocks apart: [1,8 heads,600,64] 16.8 ->
-// 15.0, [1,1024,8,64] 16.6 -> 15.7, with Stats [1,8,1000,64] 18.8 -> 17.1, [1,333,8,128] 18.2 -> 17.3, bias [1,16,500,128] 20.8 -> 19.7; but
-// [1,512,30,128] (60 groups) 24.1 -> 24.4, [1,257,30,128] 20.7 -> 21.1, e4m3 [1,320,30,128] 19.8 -> 21.8.  Without the pre-ops all groups resident at once: [2,30,4416,128] (1080 groups) 492 -> 594 us with V in them, [2,40,2176,64]
-// (720) level.  Behind the pre-ops the second norm and rotation of K is what it saves, at any number.  The call, us, launches ->
-// hand-over: [1,4608,24,128] 232.5 -> 228.4, [1,24,364,128] train 57.7 -> 54.2, [1,12,2304,64] F32 125.2 -> 119.9, e4m3 [1,585,30,128] 33.0 ->
-// 31.0, [1,2915,30,64] 101.7 -> 95.1, [1,4544,24,128] 207.8 -> 204.3, norm + RoPE [1,2207,30,128] 126.9 -> 114.9, [2,4352,30,128] 529 -> 506; but
-// e4m3 [1,5184,30,128] with norm + RoPE (630 groups and as many of V) 355 -> 359, [1,5824,24,128] 320 -> 334.
-// Behind the pre-ops, too, prep_rows_kernel has a group's norms done by four times as many threads, which is shorter for few keys and groups:
-// e4m3 [1,256,16,64] 17.9 -> 19.8 us, [1,1000,4,64] 21.0 -> 22.0, [1,128,16,128] 22.1 -> 22.7, fp16 [1,256,16,64] 19.0 -> 19.8, [1,500,40,64] 25.6 ->
-// 26.1; but fp16 of 128 channels gains at any length, [1,64,16,128] 24.3 -> 23.0, [1,300,16,128] 28.7 -> 25.8, [1,1000,40,128] 55.3 -> 46.9.
+// Where the stage is one launch by hand-over: both sides of each line, us a call on one card, by the launches or quant_short_kernel -> by hand-over.
+// Up to 32 groups of a head, all of which every workgroup adds up: [1,8192,8,128] 208.1 -> 203.2, e4m3 171.9 -> 164.4.  Past that it still gains, less and
+// less ([1,9216,12,128] 392.9 -> 383.7, [1,12288,8,128] 448.5 -> 441.8, 64 channels 315.4 -> 318.6): the line is on the safe side.
+// Without the pre-ops, and with e4m3, up to 512 groups in all, which are resident at once: [1,5376,24,128] (504) 273.4 -> 264.8, e4m3 234.4 -> 226.2; e4m3, whose V
+// groups are as many again, loses by some numbers past that ([1,5632,24,128] 270.6 -> 283.9, [2,3072,24,128] 195.7 -> 201.8, [2,4416,30,128] 448 -> 489, but
+// [2,2176,40,128] 177.8 -> 168.2; with norm + RoPE [1,5184,30,128] 363.1 -> 367.6, [1,9216,30,128] 941 -> 978), fp16 by the most ([2,3072,24,128]
+// 216.2 -> 209.2, [2,4416,30,128] (1080) 512.6 -> 518.4).
+// Behind the pre-ops the second norm and rotation of K is what it saves: fp16 [1,2304,30,128] 119.0 -> 106.7, [2,4352,30,128] 517.0 -> 495.1, level at the 4096
+// groups of [4,8192,32,128] (3223 -> 3227).  But prep_rows_kernel has a group's norms done by four times as many threads, which is shorter for few keys and groups
+// of 64 channels: fp16 under four groups of a head ([1,256,40,64] 19.9 -> 20.9, [1,500,40,64] 24.9 -> 25.7; [1,1000,16,64] 26.3 -> 25.7), e4m3 under 72
+// in all ([1,256,40,64] 18.5 -> 20.1, [1,500,16,64] 19.6 -> 20.5, [1,1000,16,64] (64) 24.8 level; [1,2304,8,64] (72) 40.1 -> 38.1, [1,500,40,64] (80) 26.0 -> 24.8)
+// and, of 128, e4m3 with one group ([1,256,16,128] 22.2 -> 22.5; [1,500,16,128] 25.2 -> 24.5; fp16 [1,256,16,128] 25.3 -> 23.2).
+// Of the calls that quant_short_kernel takes (a workgroup there computes its head's statistics itself and waits for nobody), those with fp16 V of two and more
+// groups, three at 64 channels, up to 56 groups of 128 channels in all: [1,333,8,128] 18.0 -> 17.3, [1,500,16,128] 20.0 -> 19.3, [1,500,28,128] (56) 24.5 -> 24.4,
+// [1,500,30,128] (60) 24.6 -> 24.7; [1,600,8,64] 16.4 -> 14.8, [1,1024,8,64] 16.6 -> 15.9, [1,500,16,64] 14.1 -> 14.0, [1,500,40,64] 19.9 -> 20.2; e4m3 [1,333,8,128]
+// 16.1 -> 17.1, [1,500,16,64] 13.9 -> 15.8, though not with many heads ([1,500,40,64] 24.2 -> 21.5, [1,900,30,64] 31.2 -> 25.7), where no line is drawn yet.
 bool quant_once_rule(int B, int H, int Nkv, int D, int blkk, int k_flags, bool v_fp8, bool pre, bool full_row, bool short_form) {
     const int ngroups = (Nkv + kGroup - 1) / kGroup;
     const int64_t groups = (int64_t)ngroups * B * H;
